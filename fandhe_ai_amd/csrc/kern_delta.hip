@@ -15,7 +15,7 @@ namespace fa {
 namespace k {
 using namespace fa::dev;
 
-int g_delta_form = 0;        // tuning: 1 keeps the token-by-token kernel for prompts
+int g_delta_form = 0;        // tuning: 1 keeps the token-by-token kernel for prompts, 2 the split scan for every pass, 3 for none
 
 namespace {
 
@@ -918,6 +918,129 @@ __global__ void __launch_bounds__(512)
         }
 }
 
+// Wavefronts that share the rows of a state's 16 columns in delta_scan_split_kernel.
+constexpr int scan_waves(int kt) { return kt >= 16 ? 8 : kt >= 4 ? 4 : kt; }
+
+// The same for few states.  A sequence's chunks follow one another, so with no more than two column tiles per compute unit the
+// time is a chunk's latency, and one wavefront per tile leaves matrix cores idle: here a block takes one tile and its wavefronts
+// KT / waves row tiles of the state each.  A chunk is: every wavefront's share of W S_0 and exp(G) Q S_0 over its own rows, the
+// shares exchanged through LDS (one barrier), the writes U whole in every wavefront, every wavefront's own rows of the state; the
+// first two also form a half of the read-outs each.  A wavefront alone reads its rows' fragments: they go from memory to
+// registers, a chunk ahead.  Measured, 32 heads 128 x 128: 2048 tokens of one sequence 330 -> 120 us (of two 335 -> 270); with
+// four sequences (1024 tiles, four per compute unit) the exchanges cost more than the idle cores: 10 % slower than the form above.
+template <int KT, Recurrence KIND>
+__global__ void __launch_bounds__(scan_waves(KT) * 64)
+    delta_scan_split_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, const float *__restrict__ frags, const float *__restrict__ chunk_decay,
+                            float *__restrict__ o, uint32_t vt, uint32_t n_frags) {
+    constexpr int NW = scan_waves(KT), KW = KT / NW, SHARED = shared_frags(KIND, KT), FQ = frag_q(KIND, KT), FK = frag_k(KIND, KT), FP = frag_p(KIND, KT);
+    constexpr bool CHANNEL = KIND == Recurrence::kChannelDelta, LIGHTNING = KIND == Recurrence::kLightning;
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lr = lane % 16, g = lane / 16;
+    __shared__ v4f part[2][NW][4][64];               // shares of W S_0 (two row tiles) and of the read-outs
+    // the column tiles of a head, which read the same fragments, on one XCD
+    const uint32_t b = blockIdx.y, h = blockIdx.x / 8 / vt * 8 + blockIdx.x % 8, nt = blockIdx.x / 8 % vt;
+    const uint32_t row0 = rr.row_start[b], n = rr.row_start[b + 1] - row0;
+    if (n < kChunkFrom || h >= sh.heads) return;
+    const uint32_t dim = sh.dim, vp = sh.vdim_p(), col = nt * 16 + lr, slot0 = slot_base(rr, b), vdim = sh.vdim;
+    float *state = io.state + ((uint64_t)rr.state_slot[b] * sh.heads + h) * dim * vp;
+    const bool fresh = rr.pos[row0] == 0;
+    v4f S[KW];
+#pragma unroll
+    for (int kt = 0; kt < KW; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t d = (wave * KW + kt) * 16 + 4 * g + e;
+            S[kt][e] = !fresh && d < dim && col < vdim ? state[(uint64_t)d * vp + col] : 0.0f;
+        }
+    struct Fragments {
+        v4f w[KW][2], q[KW][2], k[KW][2], d[KW], p[3], v[2];
+        float decay;
+    };
+    const bool first = wave == 0, second = NW == 1 || wave == 1;     // read-outs of the chunk's first, second 16 tokens
+    auto read = [&](uint32_t c, Fragments &f) {
+        const v4f *src = (const v4f *)(frags + ((uint64_t)(slot0 + c) * sh.heads + h) * n_frags * 256) + lane;
+#pragma unroll
+        for (int kt = 0; kt < KW; ++kt)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if constexpr (!LIGHTNING) f.w[kt][t] = src[(t * KT + wave * KW + kt) * 64];
+                f.q[kt][t] = src[(FQ + t * KT + wave * KW + kt) * 64];
+            }
+        f.v[0] = src[(SHARED + nt * 2) * 64];
+        f.v[1] = src[(SHARED + nt * 2 + 1) * 64];
+#pragma unroll
+        for (int kt = 0; kt < KW; ++kt) {
+            f.k[kt][0] = src[(FK + (wave * KW + kt) * 2) * 64];
+            f.k[kt][1] = src[(FK + (wave * KW + kt) * 2 + 1) * 64];
+            if constexpr (CHANNEL) f.d[kt] = (src - lane + (FP + 3) * 64)[(wave * KW + kt) * 4 + g];
+        }
+        if constexpr (!CHANNEL) f.decay = chunk_decay[(uint64_t)(slot0 + c) * sh.heads + h];
+        if (first) f.p[0] = src[FP * 64];
+        if (second) {
+            f.p[1] = src[(FP + 1) * 64];
+            f.p[2] = src[(FP + 2) * 64];
+        }
+    };
+    const uint32_t chunks = (n + kChunk - 1) / kChunk;
+    const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
+    auto chunk = [&](uint32_t c, const Fragments &f, Fragments &next) {
+        read(c + 1 < chunks ? c + 1 : c, next);
+        __builtin_amdgcn_sched_barrier(0);           // asked for ahead of everything else
+        v4f x[4] = {zero, zero, zero, zero};
+#pragma unroll
+        for (int kt = 0; kt < KW; ++kt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    if constexpr (!LIGHTNING) x[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[kt][t][e], S[kt][e], x[t], 0, 0, 0);
+                    x[2 + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.q[kt][t][e], S[kt][e], x[2 + t], 0, 0, 0);
+                }
+        v4f(*p)[4][64] = part[c & 1];
+#pragma unroll
+        for (int i = LIGHTNING ? 2 : 0; i < 4; ++i) p[wave][i][lane] = x[i];
+        __syncthreads();                             // the other buffer is rewritten behind the next one
+        auto sum = [&](int i, v4f s) {
+#pragma unroll
+            for (int w = 0; w < NW; ++w) s += p[w][i][lane];
+            return s;
+        };
+        const v4f u[2] = {LIGHTNING ? f.v[0] : sum(0, f.v[0]), LIGHTNING ? f.v[1] : sum(1, f.v[1])};
+#pragma unroll
+        for (int kt = 0; kt < KW; ++kt) {            // row 16 kt + 4 g + e of the state is element e here
+            if constexpr (CHANNEL) S[kt] *= f.d[kt];
+            else S[kt] *= f.decay;
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int kt = 0; kt < KW; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[kt][t][e], u[t][e], S[kt], 0, 0, 0);
+        auto store = [&](int t, const v4f &r) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t at = c * kChunk + t * 16 + 4 * g + e;
+                if (at < n && col < vdim) o[((uint64_t)(row0 + at) * sh.heads + h) * vdim + col] = r[e];
+            }
+        };
+        if (first) store(0, mfma4(f.p[0], u[0], sum(2, zero)));
+        if (second) store(1, mfma4(f.p[2], u[1], mfma4(f.p[1], u[0], sum(3, zero))));
+    };
+    Fragments even, odd;
+    read(0, even);
+    for (uint32_t c = 0; c < chunks; c += 2) {
+        chunk(c, even, odd);
+        if (c + 1 < chunks) chunk(c + 1, odd, even);
+    }
+#pragma unroll
+    for (int kt = 0; kt < KW; ++kt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t d = (wave * KW + kt) * 16 + 4 * g + e;
+            if (d < dim && col < vdim) state[(uint64_t)d * vp + col] = S[kt][e];
+        }
+}
+
 // Four read-outs, or one: weight, gate, scale, rounding.
 template <typename T, typename P>
 __device__ __forceinline__ void store_gated(const DeltaShape &sh, P v, const T *gate, T *out) {
@@ -1028,16 +1151,21 @@ void launch_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr
         configure(&lightning_chunk_kernel<T, KT>);
         lightning_chunk_kernel<T, KT><<<dim3(p.slots, sh.heads), 256, lds, s>>>(sh, io, rr, frags, decay, p.frags);
     }
-    // wavefronts of a block share a head's fragments; fewer per block where there are few blocks
-    uint32_t waves = 1;
-    while (waves < 8 && waves < p.vt && (uint64_t)rr.batch * sh.heads * ((p.vt + waves - 1) / waves) > 256) waves *= 2;
-    const size_t scan_lds = scan_buffers(KT) * (shared_frags(KIND, KT) + 2 * (size_t)waves) * 1024;
-    if constexpr (KT >= 2) {
-        static bool scan_configured = false;
-        if (!scan_configured) allow_lds(&delta_scan_kernel<KT, KIND>, 160 * 1024);
-        scan_configured = true;
+    // the line between the two scans: up to two column tiles per compute unit of 256 (measured: see delta_scan_split_kernel)
+    if (g_delta_form == 2 || (g_delta_form != 3 && (uint64_t)p.vt * sh.heads * rr.batch <= 512)) {
+        delta_scan_split_kernel<KT, KIND><<<dim3((sh.heads + 7) / 8 * 8 * p.vt, rr.batch), scan_waves(KT) * 64, 0, s>>>(sh, io, rr, frags, decay, io.raw, p.vt, p.frags);
+    } else {
+        // wavefronts of a block share a head's fragments; fewer per block where there are few blocks
+        uint32_t waves = 1;
+        while (waves < 8 && waves < p.vt && (uint64_t)rr.batch * sh.heads * ((p.vt + waves - 1) / waves) > 256) waves *= 2;
+        const size_t scan_lds = scan_buffers(KT) * (shared_frags(KIND, KT) + 2 * (size_t)waves) * 1024;
+        if constexpr (KT >= 2) {
+            static bool scan_configured = false;
+            if (!scan_configured) allow_lds(&delta_scan_kernel<KT, KIND>, 160 * 1024);
+            scan_configured = true;
+        }
+        delta_scan_kernel<KT, KIND><<<dim3((p.vt + waves - 1) / waves, sh.heads, rr.batch), waves * 64, scan_lds, s>>>(sh, io, rr, frags, decay, io.raw, p.vt, p.frags);
     }
-    delta_scan_kernel<KT, KIND><<<dim3((p.vt + waves - 1) / waves, sh.heads, rr.batch), waves * 64, scan_lds, s>>>(sh, io, rr, frags, decay, io.raw, p.vt, p.frags);
     if (sh.norm_all) return;                         // the whole pass's rows at the end
     if (sh.vdim <= 128 && ((sh.vdim | io.ld_gate | io.ld_out) & 3) == 0) delta_gate_halves_kernel<T><<<rr.rows, 256, 0, s>>>(sh, io, rr);
     else delta_gate_kernel<T><<<rr.rows, 256, 0, s>>>(sh, io, rr, io.raw);
