@@ -427,7 +427,7 @@ fa_status enqueue_prefill_chunk(fa_context *ctx, fa_decoder *d, PrefillBuffers &
             const k::QkvRopeTargets qt{t.cos_sin.as<float>(), t.slots.as<uint32_t>(), t.q_bf.as<uint16_t>(), (uint16_t *)L.k_pool->ptr,
                                        (uint16_t *)L.v_pool->ptr, c.n_heads, c.n_kv_heads, c.head_dim, pool_rows};
             k::gemm_w8a8_qkv_rope_mfma(t.xq.as<int8_t>(), (const int8_t *)L.wqkv->codes->ptr, t.sx.as<float>(),
-                                       (const float *)L.wqkv->scales->ptr, M, L.wqkv->k_pad, qt, s);
+                                       (const float *)L.wqkv->scales->ptr, M, L.wqkv->k_pad, qt, cus, s);
         } else {
             gemm(L.wqkv, t.qkv.as<float>(), nullptr);
             k::rope_append(t.qkv.as<float>(), t.cos_sin.as<float>(), t.slots.as<uint32_t>(), t.q_bf.as<uint16_t>(),

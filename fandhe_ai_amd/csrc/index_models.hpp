@@ -18,15 +18,17 @@ namespace fa {
 namespace ixm {
 
 // ------------------------------------------------------------------ large-tile GEMM (gemm_mfma_big_kernel)
-// Block tile 256 rows x NTB * 16 columns, NWAVES = 2 WM wavefronts (WM along m, 2 along n).  One stage is 128 bytes
-// of k: 16 A tiles and NTB B tiles of 2 KiB, each moved as two 1 KiB slices by direct global -> LDS loads that
-// write 16 bytes per lane at slice base + lane * 16.
+// Block tile MTB * 16 rows (256 unless stated) x NTB * 16 columns, NWAVES = 2 WM wavefronts (WM along m, 2 along n).  One
+// stage is 128 bytes of k: MTB A tiles and NTB B tiles of 2 KiB, each moved as two 1 KiB slices by direct global -> LDS
+// loads that write 16 bytes per lane at slice base + lane * 16.
 constexpr int kBigTk = 128, kBigTile = 2048, kBigRows = 256;
 constexpr int kBigStagesA = 3, kBigStagesB = 2;
+// Stages of B: three where they fit the 160 KiB beside three of A.
+FA_HD int big_stages_b(int mtb, int ntb) { return (3 * mtb + 3 * ntb) * kBigTile <= 160 * 1024 ? 3 : kBigStagesB; }
 
-template <int NTB>
+template <int NTB, int MTB = 16>
 struct BigLds {
-    static constexpr int a_stage = 16 * kBigTile, b_stage = NTB * kBigTile;
+    static constexpr int a_stage = MTB * kBigTile, b_stage = NTB * kBigTile;
     static constexpr int b_base = kBigStagesA * a_stage;
     static constexpr int bytes = b_base + kBigStagesB * b_stage;
 };
@@ -52,6 +54,20 @@ FA_HD void big_block_tile(uint32_t bid, uint32_t m_blocks, uint32_t n_blocks, ui
 // A tile (of 16 rows) that wavefront `wave` moves with its load pair i, and the tile-local row of lane `lane`.
 template <int NWAVES>
 FA_HD int big_a_tile(int wave, int i) { return wave + NWAVES * i; }
+// ... and tile and slice of its load instruction idx: pairs of slices, and where the tiles do not go round (12 tiles, 8
+// wavefronts) the last NWAVES / 2 tiles by slices.
+template <int MTB, int NWAVES>
+FA_HD void big_a_load(int wave, int idx, int *tile, int *h) {
+    if (idx / 2 < MTB / NWAVES) {
+        *tile = big_a_tile<NWAVES>(wave, idx / 2);
+        *h = idx % 2;
+    } else {
+        *tile = MTB / NWAVES * NWAVES + wave / 2;
+        *h = wave % 2;
+    }
+}
+template <int MTB, int NWAVES>
+FA_HD int big_a_loads() { return 2 * MTB / NWAVES; }
 FA_HD int big_a_row(int lane) { return lane / 4; }
 // Byte offset inside the row's 128 stage bytes that lane `lane` fetches with load x (0 or 1) of a pair, r = lane / 4,
 // p = lane % 4 its slot in the row's four slots of slice x.  e4m3: the 16-byte piece q = 2 ((p - r / 2) mod 4) + x.
@@ -68,8 +84,8 @@ FA_HD int big_a_src_byte(int lane, int x) {
     return j * 32 + x * 16;
 }
 // LDS byte offset of the slice that load (tile, h) of stage slot `slot` fills (the lane's 16 bytes go to + lane * 16).
-template <int NTB>
-FA_HD int big_a_lds_slice(int slot, int tile, int h) { return slot * BigLds<NTB>::a_stage + tile * kBigTile + h * 1024; }
+template <int NTB, int MTB = 16>
+FA_HD int big_a_lds_slice(int slot, int tile, int h) { return slot * BigLds<NTB, MTB>::a_stage + tile * kBigTile + h * 1024; }
 // Byte offsets, inside an A tile of a stage, of the two 16-byte operand reads of lane `lane`: e4m3 reads k bytes
 // 32 g .. 32 g + 15 (sub 0) and 32 g + 16 .. + 31 (sub 1) of row r; int8 reads k bytes 64 sub + 16 g .. + 15
 // (k-step `sub` of the stage), g = lane / 16, r = lane % 16.
@@ -88,9 +104,9 @@ FA_HD int big_b_tile(int wave, int i) { return (wave + NWAVES * i) % NTB; }
 // hold 32 bytes per lane (slice h = its half h), int8 stages are two adjacent 1 KiB tiles of 16 bytes per lane.
 template <bool FP8>
 FA_HD int big_b_src_byte(int lane, int h) { return FP8 ? lane * 32 + h * 16 : h * 1024 + lane * 16; }
-template <int NTB>
+template <int NTB, int MTB = 16>
 FA_HD int big_b_lds_slice(int slot, int tile, int h) {
-    return BigLds<NTB>::b_base + slot * BigLds<NTB>::b_stage + tile * kBigTile + h * 1024;
+    return BigLds<NTB, MTB>::b_base + slot * BigLds<NTB, MTB>::b_stage + tile * kBigTile + h * 1024;
 }
 // First byte, inside a stage's B region, of the fragment (tile j of wavefront column wn, slice h) of lane `lane`.
 template <int NTB>
@@ -108,11 +124,18 @@ FA_HD uint32_t big_swiglu_tile(uint32_t nb, int local, uint32_t f_tiles) {
     return (j < NTB / 4 ? 0 : f_tiles) + prod_tile;
 }
 
+// RoPE form on 128 columns (one head of 128 dims per block): wavefront column wn has the head's tiles 2 wn, 2 wn + 1 and
+// 2 wn + 4, 2 wn + 5, so that both dims of a rotate-half pair sit in one lane, accumulator tiles j and j + 2.
+FA_HD uint32_t big_rope_tile(uint32_t nb, int local) {
+    const int wn = local / 4, j = local % 4;
+    return nb * 8 + (uint32_t)(j / 2 * 4 + wn * 2 + j % 2);
+}
+
 // Output element e (0 .. 3) of accumulator tile (i, j) of wavefront (wm, wn) in lane `lane`, block-local: the matrix
 // instructions take the weight fragment first, so a lane holds row lane % 16 and columns 4 (lane / 16) + e.
-template <int NTB, int WM>
+template <int NTB, int WM, int MTB = 16>
 FA_HD void big_out_elem(int wm, int wn, int i, int j, int e, int lane, int *row, int *col) {
-    *row = (wm * (16 / WM) + i) * 16 + lane % 16;
+    *row = (wm * (MTB / WM) + i) * 16 + lane % 16;
     *col = (wn * (NTB / 2) + j) * 16 + 4 * (lane / 16) + e;
 }
 

@@ -7,6 +7,7 @@
 // tiles are double-buffered in LDS; every LDS read is a conflict-free 16-byte
 // read at lane * 16.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 #include <utility>
 
@@ -25,9 +26,10 @@ int g_gemm_pair = 0;          // tuning, 256 x 128 tiles of the large-tile kerne
                               // only where the tiles alone would cover half the device
 int g_gemm_swiglu = 0;        // tuning, prompt passes: bit 0 keeps SwiGLU out of the gate | up GEMM's epilogue, bit 1 RoPE
                               // and the K / V append out of the q | k | v GEMM's
-int g_gemm_waves = 0;
+int g_gemm_waves = 0;         // tuning: 4 = four wavefronts per large-tile block instead of eight, 16 = sixteen
 int g_gemm_split_fill = 0;    // tuning: blocks per compute unit a split-k launch aims for (default 2)
-int g_gemm_ntb = 0;           // tuning: 14 or 16 fixes the column tiles per large-tile block         // tuning: 4 = four wavefronts per large-tile block instead of eight
+int g_gemm_ntb = 0;           // tuning: 8, 14 or 16 fixes the column tiles per large-tile block
+int g_gemm_mtb = 0;           // tuning: 8, 12 or 16 fixes its row tiles
 
 namespace {
 
@@ -36,14 +38,17 @@ struct EpiI8 {
     int32_t *acc_out;
     void *out;
     int out_bf16;
-    // Large-tile kernel, k split over split_s = 2 or 4 blocks (split_partial != null): blocks b, b + 8, ... of a launch
-    // (one XCD) own one output tile and a share of k each; all leave their raw sums in split_partial, wait for their
-    // stores and take a ticket from the tile's counter, and the one that draws the last ticket adds the others' sums
-    // (int32: exact in any order) and runs the epilogue.  split_local: the exchange stays in the XCD's L2.
-    int32_t *split_partial = nullptr;
-    uint32_t *split_counters = nullptr;
-    int split_local = 0;
-    uint32_t split_s = 2;
+};
+// Large-tile kernel on tiles of 128 columns, k split over split_s = 2 or 4 blocks: blocks b, b + 8, ... of a launch (one XCD) own
+// one output tile and a share of k each; all leave their raw sums in split_partial, wait for their stores and take a ticket from
+// the tile's counter, and the one that draws the last ticket adds the others' sums (int32: exact in any order) and runs the
+// epilogue.  split_local: the exchange stays in the XCD's L2.  (A type of its own: the sums added to the accumulators make the
+// compiler spill on the wide tiles.)
+struct EpiI8Split : EpiI8 {
+    int32_t *split_partial;
+    uint32_t *split_counters;
+    int split_local;
+    uint32_t split_s;
 };
 // int8, large-tile kernel only: the weight is gate | up (f columns each) and the kernel leaves silu(gate) * up, f32 [m, f]
 struct EpiI8Swiglu {
@@ -328,6 +333,14 @@ __device__ __forceinline__ void drain_row(T (&r)[8]) {
                  : "+a"(r[0]), "+a"(r[1]), "+a"(r[2]), "+a"(r[3]), "+a"(r[4]), "+a"(r[5]), "+a"(r[6]), "+a"(r[7]));
 }
 
+// Keeps a tile in the accumulation registers up to this point: the forms of an epilogue all begin with the same conversion, which
+// the compiler would otherwise form for all tiles ahead of the branch between them, in registers that are not there.  (int32 sums in
+// blocks of eight wavefronts; elsewhere it makes the compiler move tiles inside the main loop.)
+template <typename T>
+__device__ __forceinline__ void hold_acc(T &c) {
+    asm volatile("" : "+a"(c));
+}
+
 // LDS fragment reads and the waits for them, as assembly, for the large-tile kernel's main loop.  A read's result
 // may only be touched after an lds_wait that names it: the wait takes the registers as in/out operands, so every
 // use the compiler sees comes after it.  addr is an LDS byte address, OFF an immediate offset below 65536.
@@ -346,6 +359,12 @@ template <int N>
 __device__ __forceinline__ void lds_wait_all_a(v4i (&a)[2][2], v4i (&b)[2]) {
     asm volatile("s_waitcnt lgkmcnt(%6)"
                  : "+v"(a[0][0]), "+v"(a[0][1]), "+v"(a[1][0]), "+v"(a[1][1]), "+v"(b[0]), "+v"(b[1])
+                 : "n"(N));
+}
+template <int N>
+__device__ __forceinline__ void lds_wait_all_a(v4i (&a)[3][2], v4i (&b)[2]) {
+    asm volatile("s_waitcnt lgkmcnt(%8)"
+                 : "+v"(a[0][0]), "+v"(a[0][1]), "+v"(a[1][0]), "+v"(a[1][1]), "+v"(a[2][0]), "+v"(a[2][1]), "+v"(b[0]), "+v"(b[1])
                  : "n"(N));
 }
 template <int N>
@@ -385,7 +404,7 @@ __device__ __forceinline__ void static_for(F &&f) {
 // hardware deals consecutive block ids round-robin over the 8 XCDs) are
 // consecutive tiles, m fastest: they share one B panel and walk k together,
 // which keeps the panel in that XCD's L2.
-template <bool FP8, int NTB, int WM, typename Epi>
+template <bool FP8, int NTB, int WM, typename Epi, int MTB>
 __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(WM / 2, WM / 2)))
     gemm_mfma_big_kernel(const uint8_t *__restrict__ aq, const uint8_t *__restrict__ w_tiles, uint32_t m, uint32_t n,
                          uint32_t n_tiles, uint32_t k_steps, uint32_t m_blocks, uint32_t n_blocks, Epi ep) {
@@ -395,40 +414,39 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     constexpr int TK = 128, TILE = 2048;             // bytes of k per stage; bytes per operand tile and stage
     constexpr int WNT = NTB / 2;                     // column tiles per wavefront
     constexpr int NWAVES = 2 * WM;                   // WM wavefronts along m, 2 along n
-    constexpr int AI = 16 / WM;                      // row tiles per wavefront
-    constexpr int TPW = 16 / NWAVES;                 // operand tiles each wavefront moves per stage
-    constexpr int A_STAGE = 16 * TILE, B_STAGE = NTB * TILE;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [3][A_STAGE] then [2][B_STAGE]
+    constexpr int AI = MTB / WM;                     // row tiles per wavefront
+    constexpr int ROWS = MTB * 16;                   // rows per block
+    constexpr int TPWB = (NTB + NWAVES - 1) / NWAVES;        // weight tiles each wavefront moves per stage
+    static_assert(MTB % WM == 0 && 2 * MTB % NWAVES == 0, "whole row tiles per wavefront, whole load instructions");
+    constexpr int A_STAGE = MTB * TILE, B_STAGE = NTB * TILE;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [3][A_STAGE] then [2 or 3][B_STAGE]
 
     constexpr bool SWI = std::is_same<Epi, EpiI8Swiglu>::value, ROPE = std::is_same<Epi, EpiI8QkvRope>::value;
     constexpr bool BF16 = IsBf16<Epi>::value;
     static_assert(!BF16 || !FP8, "bf16 operands take the int8 layout");
     static_assert(!SWI || (!FP8 && NTB % 4 == 0), "the SwiGLU form pairs gate and up tiles inside a wavefront");
-    static_assert(!ROPE || (!FP8 && NTB == 16), "the RoPE form: a head of 128 dims is the eight column tiles of one wavefront");
+    static_assert(!ROPE || (!FP8 && (NTB == 16 || NTB == 8)), "the RoPE form: a head of 128 dims per wavefront, or per block");
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int wm = wave / 2, wn = wave % 2;
     uint32_t mb, nb;
     uint32_t tile_id = blockIdx.x, half = 0, ks_lo = 0, ks_n = k_steps;
-    [[maybe_unused]] bool split = false;
-    if constexpr (std::is_same<Epi, EpiI8>::value) {
-        if (ep.split_partial) {
-            split = true;
-            ixm::ksplit_block(blockIdx.x, ep.split_s, &tile_id, &half);      // partners b, b + 8, ...: one XCD
-            if (tile_id >= m_blocks * n_blocks) return;               // the same for all partners
-            uint32_t ks_hi;
-            ixm::ksplit_k_range(k_steps, half, ep.split_s, &ks_lo, &ks_hi);
-            ks_n = ks_hi - ks_lo;
-        }
+    constexpr bool SPLIT = std::is_same<Epi, EpiI8Split>::value;
+    if constexpr (SPLIT) {
+        ixm::ksplit_block(blockIdx.x, ep.split_s, &tile_id, &half);          // partners b, b + 8, ...: one XCD
+        if (tile_id >= m_blocks * n_blocks) return;                   // the same for all partners
+        uint32_t ks_hi;
+        ixm::ksplit_k_range(k_steps, half, ep.split_s, &ks_lo, &ks_hi);
+        ks_n = ks_hi - ks_lo;
     }
     constexpr bool GROUPED = IsBf16<Epi>::grouped;
     [[maybe_unused]] const uint32_t *list = nullptr;
     if constexpr (GROUPED) {
         // consecutive tiles of a group, rows fastest, to one XCD: block ids go round the XCDs
-        const uint32_t total = __builtin_amdgcn_readfirstlane(group_tiles(ep.rg, 256)) * n_blocks, chunk = (total + 7) / 8;
+        const uint32_t total = __builtin_amdgcn_readfirstlane(group_tiles(ep.rg, ROWS)) * n_blocks, chunk = (total + 7) / 8;
         uint32_t group;
         tile_id = blockIdx.x % 8 * chunk + blockIdx.x / 8;
-        if (blockIdx.x / 8 >= chunk || !group_tile(ep.rg, tile_id, 256, n_blocks, &group, &mb, &nb)) return;
+        if (blockIdx.x / 8 >= chunk || !group_tile(ep.rg, tile_id, ROWS, n_blocks, &group, &mb, &nb)) return;
         group = __builtin_amdgcn_readfirstlane(group);
         mb = __builtin_amdgcn_readfirstlane(mb);
         nb = __builtin_amdgcn_readfirstlane(nb);
@@ -438,7 +456,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     } else {
         ixm::big_block_tile(tile_id, m_blocks, n_blocks, &mb, &nb);
     }
-    const uint32_t m0 = mb * 256, nt0 = nb * NTB;
+    const uint32_t m0 = mb * ROWS, nt0 = nb * NTB;
     const uint64_t k_bytes = (uint64_t)k_steps * TK;
 
     // Global -> LDS without passing through registers: one load instruction moves 16 bytes per lane to
@@ -458,44 +476,51 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     // their slots have to differ by an odd number, or the read runs at half rate).
     constexpr int B_H = FP8 ? 16 : 1024;             // byte offset of slice h in a stage's weight tile in memory
     static_assert(ixm::big_b_src_byte<FP8>(0, 1) == B_H && ixm::kBigTk == TK && ixm::kBigTile == TILE, "index model out of step");
-    const uint8_t *a_src[TPW][2];
-    const uint8_t *b_src[TPW];
+    constexpr int NLDA = ixm::big_a_loads<MTB, NWAVES>(), NLDB = 2 * TPWB;      // load instructions per wavefront and stage
+    const uint8_t *a_src[NLDA];
+    const uint8_t *b_src[TPWB];
     // (the index expressions live in index_models.hpp, where a host program checks them for every instantiation)
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
-        uint32_t row = m0 + ixm::big_a_tile<NWAVES>(wave, i) * 16 + ixm::big_a_row(lane);
+    for (int idx = 0; idx < NLDA; ++idx) {
+        int tile, h;
+        ixm::big_a_load<MTB, NWAVES>(wave, idx, &tile, &h);
+        uint32_t row = m0 + tile * 16 + ixm::big_a_row(lane);
         row = row < m ? row : m - 1;
         if constexpr (GROUPED) row = list[row] / ep.rg.a_div;
+        a_src[idx] = aq + (uint64_t)row * k_bytes + (uint64_t)ks_lo * TK + ixm::big_a_src_byte<FP8>(lane, h);
+    }
 #pragma unroll
-        for (int x = 0; x < 2; ++x) a_src[i][x] = aq + (uint64_t)row * k_bytes + (uint64_t)ks_lo * TK + ixm::big_a_src_byte<FP8>(lane, x);
+    for (int i = 0; i < TPWB; ++i) {
         // a block of NTB = 14 has no tiles 14, 15: the wavefronts that would move them repeat tiles
         // 0, 1 instead (same bytes to the same place, served by the L1), which keeps the main loop
         // free of branches
         uint32_t t = nt0 + ixm::big_b_tile<NTB, NWAVES>(wave, i);
         if constexpr (SWI) t = ixm::big_swiglu_tile<NTB>(nb, ixm::big_b_tile<NTB, NWAVES>(wave, i), ep.f / 16);
+        if constexpr (ROPE && NTB == 8) t = ixm::big_rope_tile(nb, ixm::big_b_tile<NTB, NWAVES>(wave, i));
         t = t < n_tiles ? t : n_tiles - 1;
         b_src[i] = w_tiles + ((uint64_t)t * k_steps + ks_lo) * TILE + ixm::big_b_src_byte<FP8>(lane, 0);
     }
     // byte offsets of this lane's two A operand reads inside a tile
     const int a_off[2] = {ixm::big_a_frag_off<FP8>(lane, 0), ixm::big_a_frag_off<FP8>(lane, 1)};
-    // LDS holds three stages of A and two of B: A runs two stages ahead of the multiplies, B one, so that
-    // requests stay in flight across the wait at the top of a stage (with both operands one stage ahead
-    // the path from L2 runs dry there; a third stage of both does not fit).
-    constexpr int NSA = 3, NSB = 2;
+    // LDS holds three stages of A and, on the wide tiles, two of B: A runs two stages ahead of the multiplies, B one, so
+    // that requests stay in flight across the wait at the top of a stage (with both operands one stage ahead the path from
+    // L2 runs dry there; a third stage of both does not fit).  The small tiles' stages are shorter than the way from L2
+    // (about 1900 cycles under load, which their stages took with B one stage ahead): there B has three too.
+    constexpr int NSA = 3, NSB = ixm::big_stages_b(MTB, NTB);
     // Load instruction `idx` of a stage: tile wave + NWAVES (idx / 2), slice idx % 2.  They are spread over
     // the multiply groups of the stage before, which keeps a steady stream of requests going to the L2
     // instead of one burst per stage.
     typedef __attribute__((address_space(1))) const void *gptr;
     typedef __attribute__((address_space(3))) void *lptr;
     auto issue_a = [&](uint32_t ks, int slot, int idx) {
-        const int i = idx / 2, h = idx % 2;
-        __builtin_amdgcn_global_load_lds((gptr)(a_src[i][h] + (uint64_t)ks * TK),
-                                         (lptr)(lds + ixm::big_a_lds_slice<NTB>(slot, ixm::big_a_tile<NWAVES>(wave, i), h)), 16, 0, 0);
+        int tile, h;
+        ixm::big_a_load<MTB, NWAVES>(wave, idx, &tile, &h);
+        __builtin_amdgcn_global_load_lds((gptr)(a_src[idx] + (uint64_t)ks * TK), (lptr)(lds + ixm::big_a_lds_slice<NTB, MTB>(slot, tile, h)), 16, 0, 0);
     };
     auto issue_b = [&](uint32_t ks, int slot, int idx) {
         const int i = idx / 2, h = idx % 2;
         __builtin_amdgcn_global_load_lds((gptr)(b_src[i] + (uint64_t)ks * TILE + h * B_H),
-                                         (lptr)(lds + ixm::big_b_lds_slice<NTB>(slot, ixm::big_b_tile<NTB, NWAVES>(wave, i), h)), 16, 0, 0);
+                                         (lptr)(lds + ixm::big_b_lds_slice<NTB, MTB>(slot, ixm::big_b_tile<NTB, NWAVES>(wave, i), h)), 16, 0, 0);
     };
 
     typedef typename std::conditional<FP8 || BF16, v4f, v4i>::type acc_t;
@@ -515,22 +540,27 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     }
 
     // Per stage a wavefront issues its B loads of stage ks + 1 first and its A loads of stage ks + 2 after
-    // them, so the wait at the top of stage ks + 1 can leave exactly those 2 TPW A loads outstanding.  Past
+    // them, so the wait at the top of stage ks + 1 can leave exactly those NLDA loads outstanding (three stages of B: both
+    // operands' loads of stage ks + 2).  Past
     // the end the loads are repeated from the last stage into slots nobody reads again, which keeps the
     // count of outstanding loads the same in every pass.
-    constexpr int NLD = 2 * TPW;                     // A load instructions per wavefront and stage
     const uint32_t last = ks_n - 1;                  // stages are counted from the block's first one
 #pragma unroll
-    for (int idx = 0; idx < NLD; ++idx) issue_a(0, 0, idx);
+    for (int idx = 0; idx < NLDA; ++idx) issue_a(0, 0, idx);
 #pragma unroll
-    for (int idx = 0; idx < NLD; ++idx) issue_b(0, 0, idx);
+    for (int idx = 0; idx < NLDB; ++idx) issue_b(0, 0, idx);
 #pragma unroll
-    for (int idx = 0; idx < NLD; ++idx) issue_a(last < 1 ? last : 1, 1, idx);
+    for (int idx = 0; idx < NLDA; ++idx) issue_a(last < 1 ? last : 1, 1, idx);
+    if constexpr (NSB == 3) {
+#pragma unroll
+        for (int idx = 0; idx < NLDB; ++idx) issue_b(last < 1 ? last : 1, 1, idx);
+    }
+    constexpr int AHEAD = NSB == 3 ? NLDA + NLDB : NLDA;      // loads of the stage after next that a wait leaves in flight
     // The barrier that opens stage ks + 1 sits before the last multiply group of stage ks, and the first
     // fragments of stage ks + 1 (all of A, the first of B) are read under that group: with the barrier
     // at the top of a stage every wavefront of the block would wait there for its first fragments at
     // the same time, with the matrix cores idle.  Per stage:
-    //   groups 0 .. WNT - 2: loads of B (stage ks + 1) and A (stage ks + 2), B fragment j + 1, multiplies j
+    //   groups 0 .. WNT - 2: loads of B (stage ks + 1, or + 2) and A (stage ks + 2), B fragment j + 1, multiplies j
     //   group WNT - 1: own reads of stage ks complete and own loads of stage ks + 1 landed, barrier,
     //                  multiplies interleaved with the A fragment reads of stage ks + 1, then its first B
     // The loads overwrite the buffers of stage ks - 1; they are issued after the barrier that opened
@@ -544,7 +574,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     const uint32_t lb_lane = lds0 + NSA * A_STAGE + ixm::big_b_frag_off<NTB>(wn, 0, 0, lane);
     uint32_t la[2] = {la_lane[0], la_lane[1]};        // A fragment (i, sub) at la[sub] + i * TILE
     uint32_t lb = lb_lane;                            // B fragment j, slice h at lb + j * TILE + h * 1024
-    __builtin_amdgcn_s_waitcnt(0x0F70 | NLD);         // stage 0 of this wavefront has landed (A of stage 1 may not)
+    __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);         // stage 0 of this wavefront has landed (A of stage 1 may not)
     __builtin_amdgcn_s_barrier();                     // a bare barrier: __syncthreads would add a fence on top
     // B fragments go through three registers sets: group 0 of a stage multiplies from set 2, group j >= 1 from set
     // (j - 1) % 2.  Fragment j + 1 is read under the multiplies of group j, and fragment 0 of the next stage is read
@@ -562,19 +592,19 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     lds_read16<1024>(b[2][1], lb);
     uint32_t ks = 0;
     do {                                              // ks_n >= 1: the launcher sees to it
-        const int buf = ks % NSB;
+        const int buf = ks % 2;
         const uint32_t ks_b = ks + 1 < last ? ks + 1 : last, ks_a = ks + 2 < last ? ks + 2 : last;
         const int slot_a2 = slot_a == 0 ? 2 : slot_a - 1;             // (slot_a + 2) % 3
         static_for<WNT>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
             {
-                // 2 NLD load instructions over the first multiply groups, B before A
-                constexpr int PER = (2 * NLD + WNT - 3) / (WNT - 2);
+                // the load instructions over the first multiply groups, B before A
+                constexpr int PER = (NLDA + NLDB + WNT - 3) / (WNT - 2);
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     const int idx = j * PER + q;
-                    if (idx < NLD) issue_b(ks_b, buf ^ 1, idx);
-                    else if (idx < 2 * NLD) issue_a(ks_a, slot_a2, idx - NLD);
+                    if (idx < NLDB) issue_b(NSB == 3 ? ks_a : ks_b, NSB == 3 ? slot_a2 : buf ^ 1, idx);
+                    else if (idx < NLDB + NLDA) issue_a(ks_a, slot_a2, idx - NLDB);
                 }
             }
             constexpr int cur = j == 0 ? 2 : (j - 1) % 2, nxt = j % 2;   // sets of group j and of group j + 1
@@ -585,15 +615,15 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
                 if constexpr (j == 0) lds_wait_all_a<2>(a, b[cur]);
                 else lds_wait<2>(b[cur][0], b[cur][1]);
             } else {
-                // lgkmcnt(0), vmcnt(NLD): every read of stage ks by this wavefront is complete and its
-                // loads of stage ks + 1 have landed (the A loads of stage ks + 2 may be outstanding)
-                __builtin_amdgcn_s_waitcnt(0x0070 | NLD);
+                // lgkmcnt(0), vmcnt(AHEAD): every read of stage ks by this wavefront is complete and its
+                // loads of stage ks + 1 have landed (those of stage ks + 2 may be outstanding)
+                __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
                 lds_wait<0>(b[cur][0], b[cur][1]);    // no instruction: ties the fragment to the wait above
                 __builtin_amdgcn_s_barrier();         // stage ks + 1 visible to all; stage ks no longer read
                 slot_a = slot_a == 2 ? 0 : slot_a + 1;
                 la[0] = la_lane[0] + slot_a * A_STAGE;
                 la[1] = la_lane[1] + slot_a * A_STAGE;
-                lb = lb_lane + (buf ^ 1) * B_STAGE;
+                lb = lb_lane + (NSB == 3 ? slot_a : buf ^ 1) * B_STAGE;
                 lds_read16<0>(b[2][0], lb);           // fragment 0 of the next stage (set 2 was last used by group 0)
                 lds_read16<1024>(b[2][1], lb);
             }
@@ -635,52 +665,50 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     for (int i = 0; i < AI; ++i) drain_row(acc[i]);
     __builtin_amdgcn_s_waitcnt(0x0F70);               // the repeated loads of the tail have landed too
 
-    if constexpr (std::is_same<Epi, EpiI8>::value) {
-        if (split) {
-            // raw sums of this half of k: word (i, j, e) of thread t at [(i * WNT + j) * 4 + e][t], 2 KiB per store
-            constexpr int WORDS = AI * WNT * 4;
-            const uint32_t S = ep.split_s;
-            int32_t *mine = ep.split_partial + ((uint64_t)tile_id * S + half) * ((uint64_t)WORDS * 128 * WM);
-            const bool local = ep.split_local != 0;
+    if constexpr (SPLIT) {
+        // raw sums of this half of k: word (i, j, e) of thread t at [(i * WNT + j) * 4 + e][t], 2 KiB per store
+        constexpr int WORDS = AI * WNT * 4;
+        const uint32_t S = ep.split_s;
+        int32_t *mine = ep.split_partial + ((uint64_t)tile_id * S + half) * ((uint64_t)WORDS * 128 * WM);
+        const bool local = ep.split_local != 0;
+#pragma unroll
+        for (int i = 0; i < AI; ++i)
+#pragma unroll
+            for (int j = 0; j < WNT; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    int32_t *p = mine + ((i * WNT + j) * 4 + e) * (128 * WM) + tid;
+                    if (local) __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    else __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+        __builtin_amdgcn_s_waitcnt(0);            // this thread's stores are acknowledged
+        __syncthreads();                          // ... and everybody's; nobody reads the stages any more
+        uint32_t *slot = (uint32_t *)lds;
+        if (tid == 0) {
+            uint32_t *ctr = ep.split_counters + tile_id;
+            const uint32_t t = local ? __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+                                     : __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (t == S - 1) {                     // all are in: the counter returns to zero for the next launch
+                if (local) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                else __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            *slot = t;
+        }
+        __syncthreads();
+        if (*slot != S - 1) return;               // a partner finishes the tile
+        for (uint32_t r = 0; r < S; ++r) {
+            if (r == half) continue;
+            const int32_t *other = ep.split_partial + ((uint64_t)tile_id * S + r) * ((uint64_t)WORDS * 128 * WM);
 #pragma unroll
             for (int i = 0; i < AI; ++i)
 #pragma unroll
                 for (int j = 0; j < WNT; ++j)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        int32_t *p = mine + ((i * WNT + j) * 4 + e) * (128 * WM) + tid;
-                        if (local) __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        else __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        const int32_t *p = other + ((i * WNT + j) * 4 + e) * (128 * WM) + tid;
+                        acc[i][j][e] += local ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+                                              : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     }
-            __builtin_amdgcn_s_waitcnt(0);            // this thread's stores are acknowledged
-            __syncthreads();                          // ... and everybody's; nobody reads the stages any more
-            uint32_t *slot = (uint32_t *)lds;
-            if (tid == 0) {
-                uint32_t *ctr = ep.split_counters + tile_id;
-                const uint32_t t = local ? __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                         : __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (t == S - 1) {                     // all are in: the counter returns to zero for the next launch
-                    if (local) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    else __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                *slot = t;
-            }
-            __syncthreads();
-            if (*slot != S - 1) return;               // a partner finishes the tile
-            for (uint32_t r = 0; r < S; ++r) {
-                if (r == half) continue;
-                const int32_t *other = ep.split_partial + ((uint64_t)tile_id * S + r) * ((uint64_t)WORDS * 128 * WM);
-#pragma unroll
-                for (int i = 0; i < AI; ++i)
-#pragma unroll
-                    for (int j = 0; j < WNT; ++j)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int32_t *p = other + ((i * WNT + j) * 4 + e) * (128 * WM) + tid;
-                            acc[i][j][e] += local ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                                  : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        }
-            }
         }
     }
 
@@ -690,7 +718,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     // without passing through LDS, the activation scale is one value per lane and row tile, and the channel scales
     // of a tile are one 16-byte load.  Two bf16 roundings are one v_cvt_pk_bf16_f32.
     int row_l0, col_l0;                               // block-local row of this lane in row tile 0, first column in tile 0
-    ixm::big_out_elem<NTB, WM>(wm, wn, 0, 0, 0, lane, &row_l0, &col_l0);
+    ixm::big_out_elem<NTB, WM, MTB>(wm, wn, 0, 0, 0, lane, &row_l0, &col_l0);
     const int g = lane / 16;
     if constexpr (BF16) {
         constexpr int MODE = IsBf16<Epi>::mode, STEP = is_glu(MODE) ? 2 : 1;      // gate, up: neighbouring tiles
@@ -708,15 +736,18 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
         }
         return;
     } else if constexpr (ROPE) {
-        // The eight column tiles of this wavefront are head hd = 2 nb + wn of q | k | v; tiles j and j + 4 hold dims d
-        // and d + 64 of the rotate-half pairs (four consecutive d per lane).  The arithmetic is rope_append's: dequantize,
-        // x0 c - x1 s and x1 c + x0 s with explicit roundings, one rounding to bf16.
-        const uint32_t hd = nb * 2 + wn, heads = ep.heads, kv = ep.kv_heads;
+        // 256 columns: the eight column tiles of this wavefront are head hd = 2 nb + wn of q | k | v; tiles j and j + 4 hold
+        // dims d and d + 64 of the rotate-half pairs (four consecutive d per lane).  128 columns: half of head nb, tiles j and
+        // j + 2.  The arithmetic is rope_append's: dequantize, x0 c - x1 s and x1 c + x0 s with explicit roundings, one
+        // rounding to bf16.
+        constexpr int HT = WNT / 2;
+        const uint32_t hd = NTB == 16 ? nb * 2 + wn : nb, heads = ep.heads, kv = ep.kv_heads;
         const uint64_t eq = (uint64_t)heads * 128, ekv = (uint64_t)kv * 128;
-        const uint32_t c0 = hd * 128 + 4 * g;                              // this lane's first column in tile 0
-        v4f sw0[4], sw1[4];
+        const uint32_t d0 = (NTB == 16 ? 0 : wn * HT * 16) + 4 * g;        // this lane's first dim in tile 0
+        const uint32_t c0 = hd * 128 + d0;
+        v4f sw0[HT], sw1[HT];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < HT; ++j) {
             sw0[j] = *(const v4f *)(ep.sw + c0 + j * 16);
             sw1[j] = *(const v4f *)(ep.sw + c0 + 64 + j * 16);
         }
@@ -737,17 +768,17 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
             }
             const bool rotate = hd < heads + kv;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < HT; ++j) {
                 v4f cs = v4f{0.f, 0.f, 0.f, 0.f}, sn = cs;
                 if (rotate) {
-                    cs = *(const v4f *)(ep.cos_sin + (uint64_t)rc * 128 + j * 16 + 4 * g);
-                    sn = *(const v4f *)(ep.cos_sin + (uint64_t)rc * 128 + 64 + j * 16 + 4 * g);
+                    cs = *(const v4f *)(ep.cos_sin + (uint64_t)rc * 128 + d0 + j * 16);
+                    sn = *(const v4f *)(ep.cos_sin + (uint64_t)rc * 128 + 64 + d0 + j * 16);
                 }
                 float y0[4], y1[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     float x0 = __fmul_rn((float)acc[i][j][e], __fmul_rn(sxr, sw0[j][e]));
-                    float x1 = __fmul_rn((float)acc[i][j + 4][e], __fmul_rn(sxr, sw1[j][e]));
+                    float x1 = __fmul_rn((float)acc[i][j + HT][e], __fmul_rn(sxr, sw1[j][e]));
                     if (rotate) {
                         const float r0 = __fsub_rn(__fmul_rn(x0, cs[e]), __fmul_rn(x1, sn[e]));
                         const float r1 = __fadd_rn(__fmul_rn(x1, cs[e]), __fmul_rn(x0, sn[e]));
@@ -758,8 +789,8 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
                     y1[e] = x1;
                 }
                 if (row_ok && dst) {
-                    *(v2u *)(dst + j * 16 + 4 * g) = v2u{f32x2_to_bf16x2(y0[0], y0[1]), f32x2_to_bf16x2(y0[2], y0[3])};
-                    *(v2u *)(dst + 64 + j * 16 + 4 * g) = v2u{f32x2_to_bf16x2(y1[0], y1[1]), f32x2_to_bf16x2(y1[2], y1[3])};
+                    *(v2u *)(dst + d0 + j * 16) = v2u{f32x2_to_bf16x2(y0[0], y0[1]), f32x2_to_bf16x2(y0[2], y0[3])};
+                    *(v2u *)(dst + 64 + d0 + j * 16) = v2u{f32x2_to_bf16x2(y1[0], y1[1]), f32x2_to_bf16x2(y1[2], y1[3])};
                 }
             }
         }
@@ -796,16 +827,14 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
         }
         return;
     } else {
-    bool extras = false, raw_out = false;
+    bool raw_out = false;
     const bool out_bf16 = ep.out_bf16 != 0;
     bool f8_rows = false;
     const float *bias = nullptr, *residual = nullptr;
     if constexpr (FP8) {
         f8_rows = ep.sx != nullptr;
-        extras = f8_rows && ep.bias != nullptr;
-        if (extras) bias = ep.bias;
+        if (f8_rows) bias = ep.bias;
     } else {
-        extras = ep.acc_out != nullptr || ep.bias != nullptr || ep.residual != nullptr;
         raw_out = ep.acc_out != nullptr;
         bias = ep.bias;
         residual = ep.residual;
@@ -813,13 +842,12 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     const uint32_t col0 = (nt0 + wn * WNT) * 16;      // first column of this wavefront
     const bool full_cols = nt0 + wn * WNT + WNT <= n_tiles && col0 + WNT * 16 <= n;
     const bool row_scales = !FP8 || f8_rows;
-    if (!raw_out && full_cols && n % 8 == 0) {
-        // bias and residual are added in the order of the general form below: (product + bias), then residual + that
-        v4f swc[WNT], bc[WNT];
+    // One row's tiles after another; the combinations that the linears of this library come with (the rest takes the form below).
+    auto whole_rows = [&](auto has_bias, auto has_residual, auto to_bf16) {
+        v4f swc[WNT];
+        if (row_scales) {
 #pragma unroll
-        for (int j = 0; j < WNT; ++j) {
-            if (row_scales) swc[j] = *(const v4f *)(ep.sw + col0 + j * 16 + 4 * g);
-            if (bias) bc[j] = *(const v4f *)(bias + col0 + j * 16 + 4 * g);
+            for (int j = 0; j < WNT; ++j) swc[j] = *(const v4f *)(ep.sw + col0 + j * 16 + 4 * g);
         }
 #pragma unroll
         for (int i = 0; i < AI; ++i) {
@@ -827,27 +855,28 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
             const bool row_ok = row < m;
             const float sxr = row_scales ? ep.sx[row_ok ? row : m - 1] : 0.0f;
             const uint64_t o0 = (uint64_t)(row_ok ? row : m - 1) * n + nt0 * 16 + col_l0;
-            uint8_t *orow = (uint8_t *)ep.out + o0 * (out_bf16 ? 2 : 4);
-            v4f res[WNT];
-            if (residual) {
+            uint8_t *orow = (uint8_t *)ep.out + o0 * (to_bf16 ? 2 : 4);
+            v4f add[WNT];                             // the bias (read for every row: no room for it beside the scales) or the residual
+            if constexpr (has_bias || has_residual) {
+                const float *src = has_bias ? bias + col0 + 4 * g : residual + o0;
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) res[j] = *(const v4f *)(residual + o0 + j * 16);
+                for (int j = 0; j < WNT; ++j) add[j] = *(const v4f *)(src + j * 16);
             }
             v2u pk[WNT];                              // bf16 output: the four columns of tile j, packed
 #pragma unroll
             for (int j = 0; j < WNT; ++j) {
+                if constexpr (!FP8 && WM == 4) hold_acc(acc[i][j]);
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     if constexpr (FP8) v[e] = __fmul_rn(acc[i][j][e], f8_rows ? __fmul_rn(sxr, swc[j][e]) : fscale);
                     else v[e] = __fmul_rn((float)acc[i][j][e], __fmul_rn(sxr, swc[j][e]));
-                    if (bias) v[e] = __fadd_rn(v[e], bc[j][e]);
-                    if (residual) v[e] = __fadd_rn(res[j][e], v[e]);
+                    if constexpr (has_bias || has_residual) v[e] = __fadd_rn(v[e], add[j][e]);
                 }
-                if (out_bf16) pk[j] = v2u{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])};
+                if constexpr (to_bf16) pk[j] = v2u{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])};
                 else if (row_ok) *(v4f *)(orow + j * 64) = v4f{v[0], v[1], v[2], v[3]};
             }
-            if (out_bf16) {
+            if constexpr (to_bf16) {
                 // Two tiles at a time, the lanes of column groups g = 1, 3 trade their four columns of the first tile
                 // for the four columns that groups g - 1 hold of the second (v_permlane16_swap: rows of sixteen lanes
                 // 1, 3 of one register against rows 0, 2 of the other).  Then g = 0, 2 hold columns 0 .. 7 and 8 .. 15
@@ -862,141 +891,221 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
                 if (WNT % 2 == 1 && row_ok) *(v2u *)(orow + (WNT - 1) * 32) = pk[WNT - 1];
             }
         }
+    };
+    if (!raw_out && full_cols && n % 8 == 0 && !(bias && residual) && !(residual && out_bf16)) {
+        constexpr std::true_type yes{};
+        constexpr std::false_type no{};
+        if (residual) {
+            if constexpr (!FP8) whole_rows(no, yes, no);
+        } else if (bias) {
+            if (out_bf16) whole_rows(yes, no, yes);
+            else whole_rows(yes, no, no);
+        } else {
+            if (out_bf16) whole_rows(no, no, yes);
+            else whole_rows(no, no, no);
+        }
         return;
     }
+    // Every other form: rows of any length (their vectors are aligned to an element only), blocks that the last column cuts,
+    // raw accumulators.  Four columns at a time where all four are there.
+    typedef float __attribute__((ext_vector_type(4), aligned(4))) v4f_any;
+    typedef int32_t __attribute__((ext_vector_type(4), aligned(4))) v4i_any;
+    typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) v2u_any;
 #pragma unroll
     for (int j = 0; j < WNT; ++j) {
+        const uint32_t t = nt0 + wn * WNT + j, col = t * 16 + 4 * g;
+        if (t >= n_tiles || col >= n) continue;
+        uint32_t pitch = n;                           // formed anew for every tile: row offsets kept over all tiles would cost
+        asm volatile("" : "+s"(pitch));               // registers that the accumulators need
+        const bool whole = col + 4 <= n;
+        float swc[4], bc[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const uint32_t col = (nt0 + wn * WNT + j) * 16 + 4 * g + e;
-            const bool col_ok = col < n && nt0 + wn * WNT + j < n_tiles;
-            float swc = 0.0f;
-            if (row_scales) swc = col_ok ? ep.sw[col] : 0.0f;
+            const uint32_t c = col + e < n ? col + e : n - 1;
+            swc[e] = row_scales ? ep.sw[c] : 0.0f;
+            bc[e] = bias ? bias[c] : 0.0f;
+        }
 #pragma unroll
-            for (int i = 0; i < AI; ++i) {
-                const uint32_t row = m0 + row_l0 + i * 16;
-                if (col_ok && row < m) {
-                    const uint64_t o = (uint64_t)row * n + col;
-                    float v;
-                    if constexpr (FP8) {
-                        v = __fmul_rn(acc[i][j][e], f8_rows ? __fmul_rn(ep.sx[row], swc) : fscale);
-                        if (extras) v = __fadd_rn(v, ep.bias[col]);
-                    } else {
-                        v = __fmul_rn((float)acc[i][j][e], __fmul_rn(ep.sx[row], swc));
-                        if (extras) {                  // uniform: raw accumulators, bias, residual
-                            if (ep.acc_out) ep.acc_out[o] = acc[i][j][e];
-                            if (ep.bias) v = __fadd_rn(v, ep.bias[col]);
-                            if (ep.residual) v = __fadd_rn(ep.residual[o], v);
-                        }
+        for (int i = 0; i < AI; ++i) {
+            const uint32_t row = m0 + row_l0 + i * 16;
+            if (row >= m) continue;
+            const uint64_t o = (uint64_t)row * pitch + col;
+            const float sxr = row_scales ? ep.sx[row] : 0.0f;
+            if constexpr (!FP8 && WM == 4) hold_acc(acc[i][j]);
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (FP8) v[e] = __fmul_rn(acc[i][j][e], f8_rows ? __fmul_rn(sxr, swc[e]) : fscale);
+                else v[e] = __fmul_rn((float)acc[i][j][e], __fmul_rn(sxr, swc[e]));
+                if (bias) v[e] = __fadd_rn(v[e], bc[e]);
+            }
+            if (whole) {
+                if constexpr (!FP8) {
+                    if (raw_out) *(v4i_any *)(ep.acc_out + o) = acc[i][j];
+                    if (residual) {
+                        const v4f_any r = *(const v4f_any *)(residual + o);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = __fadd_rn(r[e], v[e]);
                     }
-                    if (out_bf16)
-                        ((uint16_t *)ep.out)[o] = f32_to_bf16(v);
-                    else
-                        ((float *)ep.out)[o] = v;
+                }
+                if (out_bf16) *(v2u_any *)((uint16_t *)ep.out + o) = v2u_any{f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3])};
+                else *(v4f_any *)((float *)ep.out + o) = v4f_any{v[0], v[1], v[2], v[3]};
+            } else {
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    if (col + e >= n) continue;
+                    if constexpr (!FP8) {
+                        if (raw_out) ep.acc_out[o + e] = acc[i][j][e];
+                        if (residual) v[e] = __fadd_rn(residual[o + e], v[e]);
+                    }
+                    if (out_bf16) ((uint16_t *)ep.out)[o + e] = f32_to_bf16(v[e]);
+                    else ((float *)ep.out)[o + e] = v[e];
                 }
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
     }                                                 // !SWI
 }
 
-// Column tiles per block for the large-tile kernel: the width that leaves the fewest idle block slots
-// in the last round over the compute units (0: the matrix is too small for it).
-inline int pick_big_ntb(uint64_t m, uint64_t n_tiles, int num_cus) {
-    if (m < 256 || n_tiles < 14) return 0;
-    if (g_gemm_ntb == 14 || g_gemm_ntb == 16) return g_gemm_ntb;
-    uint64_t mb = (m + 255) / 256;
-    // a few hundred rows against a narrow weight: too few large tiles to keep the compute units' L2 ports
-    // busy (each pulls operands at a fixed rate), the 128 x 128 kernel spreads the same bytes over more of them
-    if (mb * ((n_tiles + 13) / 14) * 2 <= (uint64_t)num_cus) return 0;
-    int best = 0;
-    double best_cost = 0;
-    for (int ntb : {16, 14}) {
-        uint64_t blocks = mb * ((n_tiles + ntb - 1) / ntb);
-        uint64_t rounds = (blocks + num_cus - 1) / num_cus;
-        double cost = (double)rounds * ntb;           // time ~ rounds x tile width
-        if (best == 0 || cost < best_cost) {
-            best = ntb;
-            best_cost = cost;
+// Row and column tiles per block for the large-tile kernel (ntb 0: not for it), and over how many blocks k is divided.
+struct BigTile {
+    int mtb = 16, ntb = 0;
+    uint32_t share = 1;
+    double cost = 0;
+};
+// Bits of the widths a caller's epilogue has
+enum { kWide16 = 1, kWide14 = 2, kWide8 = 4 };
+
+// What a tile costs, us: `fixed` and `per_2k` per 2 KiB of k when all compute units hold one (measured, int8 on N(0,1) data, k of
+// 2, 4 and 14 KiB; e4m3 the same to 5 %, bf16 has the same bytes and instruction time).
+struct BigShape {
+    int mtb, ntb;
+    double fixed, per_2k;
+};
+constexpr double kShareCost = 1.5;           // us per sharing block of 128 x 128: partial sums left and added
+constexpr BigShape kBigShapes[] = {{16, 16, 14.5, 23.7}, {16, 14, 12.3, 21.6}, {12, 16, 10.4, 18.6}, {12, 14, 10.3, 16.6},
+                                   {16, 8, 9.5, 13.4},   {8, 16, 9.8, 13.1},   {12, 8, 7.6, 10.6},   {8, 8, 6.0, 7.5}};
+
+// The tile with the lowest cost: whole rounds over the compute units, and a last one that costs less the emptier it is (0.6 of a
+// full one at the least: measured 0.65 at 0.3, 0.8 at 0.6: the blocks in it have the L2s, and the power, to themselves).
+// tiles_of(rows): row blocks of that many rows.  max_share: blocks that may share a tile of 128 columns, a part of k each (8 stages
+// at the least).
+template <typename F>
+BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, uint32_t max_share) {
+    BigTile best;
+    auto has = [&](const BigShape &b) { return (widths & (b.ntb == 16 ? kWide16 : b.ntb == 14 ? kWide14 : kWide8)) != 0; };
+    auto wanted = [](const BigShape &b) { return (!g_gemm_ntb || g_gemm_ntb == b.ntb) && (!g_gemm_mtb || g_gemm_mtb == b.mtb); };
+    bool knobs = false;                               // the tuning keys name a tile that is there
+    for (const BigShape &b : kBigShapes) knobs = knobs || (has(b) && wanted(b));
+    for (const BigShape &b : kBigShapes) {
+        if (!has(b) || (knobs && !wanted(b))) continue;
+        const double tiles = (double)tiles_of(b.mtb * 16) * (double)((n_tiles + b.ntb - 1) / b.ntb);
+        for (uint32_t share = 1; share <= max_share; share *= 2) {
+            if (share > 1 && (b.ntb != 8 || k_steps / share < 8)) break;
+            const double blocks = tiles * share, rounds = std::floor(blocks / num_cus), rest = blocks / num_cus - rounds;
+            const double one = b.fixed + b.per_2k * (double)((k_steps + share - 1) / share) / 16.0 + (share > 1 ? kShareCost * share * b.mtb * b.ntb / 64.0 : 0.0);
+            const double cost = one * (rounds + (rest > 0 ? 0.6 + 0.4 * rest : 0.0));
+            if (best.ntb == 0 || cost < best.cost) best = BigTile{b.mtb, b.ntb, share, cost};
         }
     }
     return best;
 }
-
-template <bool FP8, int NTB, int WM, typename Epi>
-void launch_big_wm(const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps,
-                const Epi &e, hipStream_t s) {
-    const size_t smem = (3 * 16 + 2 * (size_t)NTB) * 2048;          // three stages of A, two of B
-    static bool configured = false;
-    if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_big_kernel<FP8, NTB, WM, Epi>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        configured = true;
-    }
-    uint32_t mb = (uint32_t)((m + 255) / 256), nb = (uint32_t)((n_tiles + NTB - 1) / NTB);
-    gemm_mfma_big_kernel<FP8, NTB, WM, Epi><<<mb * nb, 128 * WM, smem, s>>>(aq, w_tiles, (uint32_t)m, (uint32_t)n, (uint32_t)n_tiles,
-                                                                  (uint32_t)k_steps, mb, nb, e);
+BigTile pick_big(uint64_t m, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, uint32_t max_share = 1) {
+    return pick_big_rows([m](int rows) { return (m + rows - 1) / rows; }, n_tiles, k_steps, num_cus, widths, max_share);
 }
 
-template <bool FP8, int NTB, typename Epi>
-void launch_big(const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps,
-                const Epi &e, hipStream_t s) {
-    if (g_gemm_waves == 4)
-        launch_big_wm<FP8, NTB, 2, Epi>(aq, w_tiles, m, n, n_tiles, k_steps, e, s);
-    else if (g_gemm_waves == 16)
-        launch_big_wm<FP8, NTB, 8, Epi>(aq, w_tiles, m, n, n_tiles, k_steps, e, s);
-    else
-        launch_big_wm<FP8, NTB, 4, Epi>(aq, w_tiles, m, n, n_tiles, k_steps, e, s);
+// One of a kernel's forms with its LDS (above the default limit)
+template <typename F>
+void allow_lds(F f, size_t bytes) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(f), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+
+template <bool FP8, int NTB, int WM, int MTB, typename Epi>
+void launch_big_tile(const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, uint32_t n_blocks,
+                     unsigned grid, const Epi &e, hipStream_t s) {
+    constexpr size_t smem = (3 * MTB + ixm::big_stages_b(MTB, NTB) * NTB) * 2048;
+    static bool configured = false;
+    if (!configured) allow_lds(&gemm_mfma_big_kernel<FP8, NTB, WM, Epi, MTB>, smem);
+    configured = true;
+    const uint32_t mb = (uint32_t)((m + MTB * 16 - 1) / (MTB * 16));
+    gemm_mfma_big_kernel<FP8, NTB, WM, Epi, MTB><<<grid ? grid : mb * n_blocks, 128 * WM, smem, s>>>(aq, w_tiles, (uint32_t)m, (uint32_t)n, (uint32_t)n_tiles,
+                                                                                                  (uint32_t)k_steps, mb, n_blocks, e);
+}
+// ... with eight wavefronts on the tile that was picked; WIDTHS: the widths instantiated
+template <bool FP8, int WIDTHS, typename Epi>
+void launch_big(const BigTile &t, const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, const Epi &e, hipStream_t s,
+                unsigned grid = 0) {
+    const uint32_t nb = (uint32_t)((n_tiles + t.ntb - 1) / t.ntb);
+    auto rows = [&](auto ntb) {
+        constexpr int NTB = decltype(ntb)::value;
+        if (NTB != 14 && t.mtb == 8) launch_big_tile<FP8, NTB, 4, NTB != 14 ? 8 : 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, grid, e, s);
+        else if (t.mtb == 12) launch_big_tile<FP8, NTB, 4, 12>(aq, w_tiles, m, n, n_tiles, k_steps, nb, grid, e, s);
+        else launch_big_tile<FP8, NTB, 4, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, grid, e, s);
+    };
+    if constexpr ((WIDTHS & kWide8) != 0) {
+        if (t.ntb == 8) return rows(std::integral_constant<int, 8>{});
+    }
+    if constexpr ((WIDTHS & kWide14) != 0) {
+        if (t.ntb == 14) return rows(std::integral_constant<int, 14>{});
+    }
+    if constexpr ((WIDTHS & kWide16) != 0) rows(std::integral_constant<int, 16>{});
+}
+// The quantized GEMMs' other wavefront counts (tuning): 256 rows
+template <bool FP8, typename Epi>
+bool launch_big_waves(const BigTile &t, const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, const Epi &e, hipStream_t s) {
+    const uint32_t nb = (uint32_t)((n_tiles + t.ntb - 1) / t.ntb);
+    if (t.mtb != 16 || t.ntb == 8) return false;
+    if (g_gemm_waves == 4) {
+        if (t.ntb == 14) launch_big_tile<FP8, 14, 2, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
+        else launch_big_tile<FP8, 16, 2, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
+        return true;
+    }
+    if (g_gemm_waves == 16) {
+        if (t.ntb == 14) launch_big_tile<FP8, 14, 8, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
+        else launch_big_tile<FP8, 16, 8, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
+        return true;
+    }
+    return false;
 }
 
 }  // namespace
 
-// How an int8 GEMM is launched.  ntb != 0: the large-tile kernel with that many column tiles per block,
-// ntb == 0: the 128 x 128 kernel; splits > 1 (128 x 128 kernel only): k is divided over that many blocks
-// per output tile, which leave int32 partial sums in a workspace that a second kernel adds (exactly) before
-// the epilogue.  A matrix with few output tiles (a prompt of a few hundred rows against a 4096-column
-// weight) occupies only a fraction of the compute units otherwise, and each of them pulls operands at a
-// fixed rate.  (The same split on the large-tile kernel measured no faster.)
+// Where the large-tile kernel takes a quantized GEMM.  Weights of fewer than 1024 columns stay with the 128 x 128 kernel, as callers of
+// the plan query expect; it is the slower one there too (300 x 1024 -> 520, us: int8 12.5 against 7.0, e4m3 24 against 7).
+static bool big_applies(uint64_t n_tiles, uint64_t k_pad) { return !g_gemm_small_tiles && k_pad % 128 == 0 && k_pad != 0 && n_tiles >= 64; }
+
+// How an int8 GEMM is launched.  tile.ntb != 0: the large-tile kernel, k over tile.share blocks of one XCD that meet in a workspace
+// (two or four where the tiles alone leave compute units idle); ntb == 0: the 128 x 128 kernel (k not a multiple of 128); splits > 1
+// there: k is divided over that many blocks per output tile, which leave int32 partial sums that a second kernel adds (exactly)
+// before the epilogue.
 struct W8a8Plan {
-    int ntb;
-    uint32_t splits;
-    uint32_t share = 1;    // large-tile kernel on 256 x 128 tiles: same-XCD blocks that share a tile, a part of k each
+    BigTile tile;
+    uint32_t splits = 1;
 };
 
 static W8a8Plan plan_w8a8(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, bool may_share = true) {
     const uint64_t n_tiles = n_pad / 16;
+    if (big_applies(n_tiles, k_pad))
+        return {pick_big(m, n_tiles, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8, may_share && g_gemm_pair != 1 ? 4 : 1), 1};
     const uint64_t fill = (uint64_t)num_cus * (g_gemm_split_fill > 0 ? g_gemm_split_fill : 2);
-    const bool big_ok = !(g_gemm_small_tiles || k_pad % 128 || k_pad == 0) && n_tiles >= 14;
-    if (big_ok && m >= 256) {
-        if (int ntb = pick_big_ntb(m, n_tiles, num_cus)) return {ntb, 1};
-        // Too few 256 x 224 tiles for the device, but 256 x 128 tiles for at least half of it (about a thousand rows
-        // against a 4096- or 6144-column weight): the large-tile kernel on the narrower tile keeps its rate per compute
-        // unit, where the 128 x 128 kernel with its k split and second pass ran at a third of it (1024 rows, us: q | k | v
-        // 65 + 18 -> 40, o 65 + 18 -> 37)
-        const uint64_t blocks8 = ((m + 255) / 256) * ((n_tiles + 7) / 8), k_steps = k_pad / 128;
-        // ... and when those tiles cover a quarter to a half of it, two blocks share a tile, half of k each (one prompt
-        // of 1024 tokens through 32 layers: 14.0 -> 12.4 ms; 600 / 767 rows, us incl. the row quantizer: 4096 -> 4096
-        // 46 / 53 -> 41 / 41, 14336 -> 4096 105 / 133 -> 93 / 95), at least sixteen stages of k per block.  Four blocks a
-        // tile measured slower than every other form (14336 -> 4096 at 257 .. 512 rows: 82 - 87 us against 55 - 78 us).
-        if (g_gemm_ntb == 0 && blocks8 * 2 >= (uint64_t)num_cus)
-            return {8, 1, (may_share && g_gemm_pair != 1 && blocks8 * 2 <= (uint64_t)num_cus && k_steps >= 32) ? 2u : 1u};
-        if (may_share && g_gemm_ntb == 0 && g_gemm_pair != 1 && g_gemm_pair != 2) {
-            if (blocks8 * 4 >= (uint64_t)num_cus && blocks8 * 2 <= (uint64_t)num_cus && k_steps >= 32) return {8, 1, 2};
-        }
-    }
     const uint64_t blocks = ((n_tiles + NT - 1) / NT) * ((m + BM - 1) / BM);
-    if (blocks == 0 || blocks * 2 > fill) return {0, 1};
+    if (blocks == 0 || blocks * 2 > fill) return {};
     uint64_t s = std::min<uint64_t>(std::min<uint64_t>(16, fill / blocks), (k_pad / 64) / 4);
-    return {0, (uint32_t)std::max<uint64_t>(s, 1)};
+    return {BigTile{}, (uint32_t)std::max<uint64_t>(s, 1)};
+}
+static uint64_t big_tiles(const BigTile &t, uint64_t m, uint64_t n_pad) { return (m + t.mtb * 16 - 1) / (t.mtb * 16) * ((n_pad / 16 + t.ntb - 1) / t.ntb); }
+static uint64_t share_bytes(const BigTile &t, uint64_t m, uint64_t n_pad) {
+    return t.share > 1 ? big_tiles(t, m, n_pad) * t.share * ((uint64_t)t.mtb * t.ntb * 256 * 4) : 0;
 }
 
 GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus) {
     GemmPlan out{0, 4, 1};
     if (fp8) {
-        out.big_ntb = (g_gemm_small_tiles || k_pad == 0) ? 0 : pick_big_ntb(m, n_pad / 16, num_cus);
+        out.big_ntb = !big_applies(n_pad / 16, k_pad) ? 0 : pick_big(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8).ntb;
     } else {
         const W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus);
-        out.big_ntb = p.ntb;
+        out.big_ntb = p.tile.ntb;
         out.splits = p.splits;
     }
     if (out.big_ntb) out.waves = g_gemm_waves == 4 ? 4 : g_gemm_waves == 16 ? 16 : 8;
@@ -1005,7 +1114,7 @@ GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num
 
 uint64_t gemm_w8a8_workspace_bytes(uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad, int num_cus) {
     const W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus);
-    if (p.share > 1) return ((m + 255) / 256) * ((n_pad / 16 + 7) / 8) * p.share * (uint64_t)(256 * 128 * 4);
+    if (p.tile.ntb) return share_bytes(p.tile, m, n_pad);
     return p.splits > 1 ? (uint64_t)p.splits * m * n * 4 : 0;
 }
 
@@ -1013,28 +1122,15 @@ void gemm_w8a8_mfma(const int8_t *aq, const int8_t *w_tiles, uint64_t m, uint64_
                     const EpilogueI8 &ep, int num_cus, hipStream_t s, void *workspace, uint64_t workspace_bytes,
                     const SplitKArea *sk) {
     if (m == 0 || n == 0) return;
-    EpiI8 e{ep.sx, ep.sw, ep.bias, ep.residual, ep.acc_out, ep.out, ep.out_bf16};
+    const EpiI8 e{ep.sx, ep.sw, ep.bias, ep.residual, ep.acc_out, ep.out, ep.out_bf16};
     W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus);
-    if (p.share > 1) {
-        const uint64_t tiles = ((m + 255) / 256) * ((n_pad / 16 + 7) / 8), need = tiles * p.share * (uint64_t)(256 * 128 * 4);
-        if (sk && sk->counters && tiles <= sk->n_counters && workspace && workspace_bytes >= need && g_gemm_waves != 4 && g_gemm_waves != 16) {
-            e.split_partial = (int32_t *)workspace;
-            e.split_counters = sk->counters;
+    if (p.tile.share > 1) {
+        const uint64_t tiles = big_tiles(p.tile, m, n_pad);
+        if (sk && sk->counters && tiles <= sk->n_counters && workspace && workspace_bytes >= share_bytes(p.tile, m, n_pad) && g_gemm_waves != 4 && g_gemm_waves != 16) {
             // (the scope knob of the split-k decode linears forces either form here as well: 2 agent scope, 3 the XCD's L2)
-            e.split_local = g_skinny_ksplit == 2 ? 0 : g_skinny_ksplit == 3 ? 1 : sk->xcd_local;
-            e.split_s = p.share;
-            constexpr int NTB = 8;
-            const size_t smem = (3 * 16 + 2 * (size_t)NTB) * 2048;
-            static bool configured = false;
-            if (!configured) {
-                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_big_kernel<false, NTB, 4, EpiI8>),
-                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-                configured = true;
-            }
-            const uint32_t mb = (uint32_t)((m + 255) / 256), nb = (uint32_t)((n_pad / 16 + NTB - 1) / NTB);
-            const unsigned grid = 8u * p.share * (unsigned)((tiles + 7) / 8);   // whole groups on every XCD; surplus groups return at once
-            gemm_mfma_big_kernel<false, NTB, 4, EpiI8><<<grid, 512, smem, s>>>((const uint8_t *)aq, (const uint8_t *)w_tiles, (uint32_t)m,
-                                                                           (uint32_t)n, (uint32_t)(n_pad / 16), (uint32_t)(k_pad / 128), mb, nb, e);
+            const EpiI8Split es{e, (int32_t *)workspace, sk->counters, g_skinny_ksplit == 2 ? 0 : g_skinny_ksplit == 3 ? 1 : sk->xcd_local, p.tile.share};
+            const unsigned grid = 8u * p.tile.share * (unsigned)((tiles + 7) / 8);   // whole groups on every XCD; surplus groups return at once
+            launch_big<false, kWide8>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, es, s, grid);
             return;
         }
         p = plan_w8a8(m, n_pad, k_pad, num_cus, false);      // no counters or no room: the plan without shared tiles
@@ -1042,12 +1138,9 @@ void gemm_w8a8_mfma(const int8_t *aq, const int8_t *w_tiles, uint64_t m, uint64_
     if (p.splits > 1 && (!workspace || workspace_bytes < (uint64_t)p.splits * m * n * 4))
         p.splits = 1;                                 // no room for partial sums: one block per tile
     int32_t *partial = p.splits > 1 ? (int32_t *)workspace : nullptr;
-    if (p.ntb == 16) {
-        launch_big<false, 16, EpiI8>((const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
-    } else if (p.ntb == 8) {
-        launch_big<false, 8, EpiI8>((const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
-    } else if (p.ntb) {
-        launch_big<false, 14, EpiI8>((const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
+    if (p.tile.ntb) {
+        if (!launch_big_waves<false>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, e, s))
+            launch_big<false, kWide16 | kWide14 | kWide8>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
     } else {
         dim3 grid((unsigned)((n_pad / 16 + NT - 1) / NT), (unsigned)((m + BM - 1) / BM), p.splits);
         gemm_mfma_kernel<false, EpiI8><<<grid, 256, 0, s>>>((const uint8_t *)aq, (const uint8_t *)w_tiles, (uint32_t)m,
@@ -1072,34 +1165,12 @@ bool gemm_w8a8_swiglu_applies(uint64_t m, uint64_t f, uint64_t n_pad, uint64_t k
     return !(g_gemm_swiglu & 1) && !g_gemm_small_tiles && m >= 65 && f != 0 && f % 128 == 0 && n_pad == 2 * f && k_pad != 0 &&
            k_pad % 128 == 0;
 }
-namespace {
-template <int NTB>
-void launch_swiglu(const int8_t *aq, const int8_t *w_tiles, const EpiI8Swiglu &e, uint64_t m, uint64_t f, uint64_t k_pad, hipStream_t s) {
-    const size_t smem = (3 * 16 + 2 * (size_t)NTB) * 2048;
-    static bool configured = false;
-    if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_big_kernel<false, NTB, 4, EpiI8Swiglu>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        configured = true;
-    }
-    const uint32_t mb = (uint32_t)((m + 255) / 256), nb = (uint32_t)(f / (8 * NTB));      // NTB / 2 product tiles per block
-    gemm_mfma_big_kernel<false, NTB, 4, EpiI8Swiglu><<<mb * nb, 512, smem, s>>>((const uint8_t *)aq, (const uint8_t *)w_tiles, (uint32_t)m,
-                                                                              (uint32_t)(2 * f), (uint32_t)(2 * f / 16),
-                                                                              (uint32_t)(k_pad / 128), mb, nb, e);
-}
-}  // namespace
 void gemm_w8a8_swiglu_mfma(const int8_t *aq, const int8_t *w_tiles, const float *sx, const float *sw, uint64_t m, uint64_t f,
                            uint64_t k_pad, float *out, int num_cus, hipStream_t s) {
     if (m == 0 || f == 0) return;
     const EpiI8Swiglu e{sx, sw, out, (uint32_t)f};
-    // 256 x 256 tiles (eight gate and eight up column tiles), or 256 x 128 where the wide tiles would cover at most half the
-    // device (up to 256 rows at d_ffn 14336: 112 wide tiles, 224 narrow ones; one prompt of 200 tokens through 32 layers
-    // 5.56 -> 5.21 ms).  With more rows three rounds of narrow tiles measured no better than two of wide ones.
-    const uint64_t mb = (m + 255) / 256;
-    if (g_gemm_ntb == 8 || (g_gemm_ntb == 0 && mb * (f / 128) * 2 <= (uint64_t)num_cus))
-        launch_swiglu<8>(aq, w_tiles, e, m, f, k_pad, s);
-    else
-        launch_swiglu<16>(aq, w_tiles, e, m, f, k_pad, s);
+    const BigTile t = pick_big(m, 2 * f / 16, k_pad / 128, num_cus, kWide16 | kWide8);
+    launch_big<false, kWide16 | kWide8>(t, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, 2 * f, 2 * f / 16, k_pad / 128, e, s);
 }
 
 // q | k | v projection of a prompt pass with RoPE, the bf16 rounding and the K / V append in the epilogue (heads of 128 dims:
@@ -1107,27 +1178,16 @@ void gemm_w8a8_swiglu_mfma(const int8_t *aq, const int8_t *w_tiles, const float 
 // large-tile kernel too.
 bool gemm_w8a8_qkv_rope_applies(uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad, uint32_t heads, uint32_t kv_heads,
                                 uint32_t head_dim, int num_cus) {
-    if ((g_gemm_swiglu & 2) || g_gemm_small_tiles || head_dim != 128 || m < 256 || k_pad == 0 || k_pad % 128) return false;
-    if (n != (uint64_t)(heads + 2 * kv_heads) * 128 || n_pad != n || (heads + 2 * kv_heads) % 2) return false;
-    return pick_big_ntb(m, n_pad / 16, num_cus) != 0;
+    if ((g_gemm_swiglu & 2) || g_gemm_small_tiles || head_dim != 128 || m < 65 || k_pad == 0 || k_pad % 128) return false;
+    return n == (uint64_t)(heads + 2 * kv_heads) * 128 && n_pad == n;
 }
 void gemm_w8a8_qkv_rope_mfma(const int8_t *aq, const int8_t *w_tiles, const float *sx, const float *sw, uint64_t m, uint64_t k_pad,
-                             const QkvRopeTargets &t, hipStream_t s) {
+                             const QkvRopeTargets &t, int num_cus, hipStream_t s) {
     if (m == 0) return;
     const EpiI8QkvRope e{sx, sw, t.cos_sin, t.slots, t.q_out, t.k_pool, t.v_pool, t.heads, t.kv_heads, t.pool_rows};
-    constexpr int NTB = 16;
-    const size_t smem = (3 * 16 + 2 * (size_t)NTB) * 2048;
-    static bool configured = false;
-    if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_big_kernel<false, NTB, 4, EpiI8QkvRope>),
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        configured = true;
-    }
     const uint64_t n = (uint64_t)(t.heads + 2 * t.kv_heads) * 128;
-    const uint32_t mb = (uint32_t)((m + 255) / 256), nb = (uint32_t)(n / 256);
-    gemm_mfma_big_kernel<false, NTB, 4, EpiI8QkvRope><<<mb * nb, 512, smem, s>>>((const uint8_t *)aq, (const uint8_t *)w_tiles,
-                                                                               (uint32_t)m, (uint32_t)n, (uint32_t)(n / 16),
-                                                                               (uint32_t)(k_pad / 128), mb, nb, e);
+    const BigTile tile = pick_big(m, n / 16, k_pad / 128, num_cus, (t.heads + 2 * t.kv_heads) % 2 == 0 ? kWide16 | kWide8 : kWide8);
+    launch_big<false, kWide16 | kWide8>(tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n / 16, k_pad / 128, e, s);
 }
 
 static void launch_e4m3(const uint8_t *aq, const uint8_t *w_tiles, const EpiF8 &e, uint64_t m, uint64_t n, uint64_t n_pad,
@@ -1148,11 +1208,9 @@ void gemm_e4m3_rows_mfma(const uint8_t *aq, const uint8_t *w_tiles, const float 
 
 static void launch_e4m3(const uint8_t *aq, const uint8_t *w_tiles, const EpiF8 &e, uint64_t m, uint64_t n, uint64_t n_pad,
                         uint64_t k_pad, int num_cus, hipStream_t s) {
-    if (int ntb = (g_gemm_small_tiles || k_pad == 0) ? 0 : pick_big_ntb(m, n_pad / 16, num_cus)) {
-        if (ntb == 16)
-            launch_big<true, 16, EpiF8>(aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
-        else
-            launch_big<true, 14, EpiF8>(aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
+    if (big_applies(n_pad / 16, k_pad)) {
+        const BigTile t = pick_big(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8);
+        if (!launch_big_waves<true>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s)) launch_big<true, kWide16 | kWide14 | kWide8>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
         return;
     }
     dim3 grid((unsigned)((n_pad / 16 + NT - 1) / NT), (unsigned)((m + BM - 1) / BM));
@@ -1162,52 +1220,49 @@ static void launch_e4m3(const uint8_t *aq, const uint8_t *w_tiles, const EpiF8 &
 
 namespace {
 template <int MODE>
-void launch_big_bf16(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int ntb, hipStream_t s) {
-    const EpiBf16<MODE> e{ep};
-    if constexpr (!is_glu(MODE)) {
-        if (ntb == 14) return launch_big_wm<false, 14, 4>((const uint8_t *)a, (const uint8_t *)w.w, m, w.n, w.n_tiles, w.k_tiles / 2, e, s);
-    }
-    launch_big_wm<false, 16, 4>((const uint8_t *)a, (const uint8_t *)w.w, m, w.n, w.n_tiles, w.k_tiles / 2, e, s);
+void launch_big_bf16(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+    constexpr int WIDTHS = is_glu(MODE) ? kWide16 | kWide8 : kWide16 | kWide14 | kWide8;
+    launch_big<false, WIDTHS>(pick_big(m, w.n_tiles, w.k_tiles / 2, num_cus, WIDTHS), (const uint8_t *)a, (const uint8_t *)w.w, m, w.n, w.n_tiles,
+                              w.k_tiles / 2, EpiBf16<MODE>{ep}, s);
 }
 }  // namespace
 
-bool gemm_bf16_big_applies(uint64_t lda, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus) {
-    return w.batches == 1 && lda == (uint64_t)w.k_tiles * 32 && w.k_tiles % 2 == 0 && pick_big_ntb(m, w.n_tiles, num_cus) != 0;
+bool gemm_bf16_big_applies(uint64_t lda, uint64_t m, const LinearWeight &w) {
+    return w.batches == 1 && lda == (uint64_t)w.k_tiles * 32 && w.k_tiles % 2 == 0 && m > 64;
 }
 
 void gemm_bf16_big(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
-    const int ntb = pick_big_ntb(m, w.n_tiles, num_cus);
     switch (ep.mode) {
-        case LinearEpilogue::kResidual: return launch_big_bf16<LinearEpilogue::kResidual>(a, m, w, ep, ntb, s);
-        case LinearEpilogue::kGlu: return launch_big_bf16<LinearEpilogue::kGlu>(a, m, w, ep, ntb, s);
-        case LinearEpilogue::kSiluGlu: return launch_big_bf16<LinearEpilogue::kSiluGlu>(a, m, w, ep, ntb, s);
-        case LinearEpilogue::kXielu: return launch_big_bf16<LinearEpilogue::kXielu>(a, m, w, ep, ntb, s);
-        case LinearEpilogue::kSoftcap: return launch_big_bf16<LinearEpilogue::kSoftcap>(a, m, w, ep, ntb, s);
-        default: return launch_big_bf16<LinearEpilogue::kStore>(a, m, w, ep, ntb, s);
+        case LinearEpilogue::kResidual: return launch_big_bf16<LinearEpilogue::kResidual>(a, m, w, ep, num_cus, s);
+        case LinearEpilogue::kGlu: return launch_big_bf16<LinearEpilogue::kGlu>(a, m, w, ep, num_cus, s);
+        case LinearEpilogue::kSiluGlu: return launch_big_bf16<LinearEpilogue::kSiluGlu>(a, m, w, ep, num_cus, s);
+        case LinearEpilogue::kXielu: return launch_big_bf16<LinearEpilogue::kXielu>(a, m, w, ep, num_cus, s);
+        case LinearEpilogue::kSoftcap: return launch_big_bf16<LinearEpilogue::kSoftcap>(a, m, w, ep, num_cus, s);
+        default: return launch_big_bf16<LinearEpilogue::kStore>(a, m, w, ep, num_cus, s);
     }
 }
 
 namespace {
 template <int MODE>
-void launch_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, hipStream_t s) {
-    constexpr int NTB = 16, WM = 4;
-    typedef EpiBf16Grouped<MODE> Epi;
-    const size_t smem = (3 * 16 + 2 * (size_t)NTB) * 2048;
-    static bool configured = false;
-    if (!configured) {
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_mfma_big_kernel<false, NTB, WM, Epi>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-        configured = true;
-    }
-    const uint32_t nb = (w.n_tiles + NTB - 1) / NTB, tiles = rg.entries / 256 + (rg.groups < rg.entries ? rg.groups : rg.entries);
-    gemm_mfma_big_kernel<false, NTB, WM, Epi><<<(tiles * nb + 7) / 8 * 8, 128 * WM, smem, s>>>((const uint8_t *)a, (const uint8_t *)w.w, 0, w.n, w.n_tiles,
-                                                                                              w.k_tiles / 2, 0, nb, Epi{ep, rg});
+void launch_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+    auto rows = [&](auto mtb) {
+        constexpr int MTB = decltype(mtb)::value;
+        const uint32_t nb = (w.n_tiles + 15) / 16, tiles = rg.entries / (MTB * 16) + (rg.groups < rg.entries ? rg.groups : rg.entries);
+        launch_big_tile<false, 16, 4, MTB>((const uint8_t *)a, (const uint8_t *)w.w, 0, w.n, w.n_tiles, w.k_tiles / 2, nb, (tiles * nb + 7) / 8 * 8, EpiBf16Grouped<MODE>{ep, rg}, s);
+    };
+    // how the rows spread over the groups is known on the device only: half a tile per group is taken to be padding
+    const double likely = rg.likely ? rg.likely : rg.entries, groups = rg.groups;
+    const BigTile t = pick_big_rows([&](int r) { return likely / r + 0.5 * groups; }, w.n_tiles, w.k_tiles / 2, num_cus, kWide16, 1);
+    if (t.mtb == 8) rows(std::integral_constant<int, 8>{});
+    else if (t.mtb == 12) rows(std::integral_constant<int, 12>{});
+    else rows(std::integral_constant<int, 16>{});
 }
 }  // namespace
 
-void gemm_bf16_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, hipStream_t s) {
-    if (ep.mode == LinearEpilogue::kSquaredRelu) launch_big_grouped<LinearEpilogue::kSquaredRelu>(a, w, rg, ep, s);
-    else if (ep.mode == LinearEpilogue::kSiluGlu) launch_big_grouped<LinearEpilogue::kSiluGlu>(a, w, rg, ep, s);
-    else launch_big_grouped<LinearEpilogue::kStore>(a, w, rg, ep, s);
+void gemm_bf16_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+    if (ep.mode == LinearEpilogue::kSquaredRelu) launch_big_grouped<LinearEpilogue::kSquaredRelu>(a, w, rg, ep, num_cus, s);
+    else if (ep.mode == LinearEpilogue::kSiluGlu) launch_big_grouped<LinearEpilogue::kSiluGlu>(a, w, rg, ep, num_cus, s);
+    else launch_big_grouped<LinearEpilogue::kStore>(a, w, rg, ep, num_cus, s);
 }
 
 }  // namespace k

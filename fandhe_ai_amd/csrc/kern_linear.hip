@@ -353,7 +353,7 @@ void launch_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, 
 #undef FA_ROWS
         return;
     }
-    if (MODE != LinearEpilogue::kHeadGate && g_linear_form != 2 && gemm_bf16_big_applies(lda, m, w, ep, num_cus)) return gemm_bf16_big(a, m, w, ep, num_cus, s);
+    if (MODE != LinearEpilogue::kHeadGate && g_linear_form != 2 && gemm_bf16_big_applies(lda, m, w)) return gemm_bf16_big(a, m, w, ep, num_cus, s);
     const dim3 grid((w.n_tiles + 7) / 8, (unsigned)((m + 127) / 128), w.batches);
     linear_tile_kernel<MODE><<<grid, 256, 0, s>>>(a, lda, a_batch, wt, (uint32_t)m, w.n, w.n_tiles, w.k_tiles, ep, RowGroups{});
 }
@@ -383,7 +383,7 @@ void launch_grouped_bf16(const uint16_t *a, uint64_t lda, const LinearWeight &w,
 #undef FA_ROWS
         return;
     }
-    if (form == 6 || (form != 5 && mean >= 112 && lda == (uint64_t)w.k_tiles * 32 && w.n_tiles >= 14)) return gemm_bf16_big_grouped(a, w, rg, ep, s);
+    if (form == 6 || (form != 5 && mean >= 112 && lda == (uint64_t)w.k_tiles * 32 && w.n_tiles >= 14)) return gemm_bf16_big_grouped(a, w, rg, ep, num_cus, s);
     const uint32_t tiles = rg.entries / 128 + std::min(rg.groups, rg.entries);
     linear_tile_kernel<MODE, true><<<tiles * ((w.n_tiles + 7) / 8), 256, 0, s>>>(a, lda, 0, wt, 0, w.n, w.n_tiles, w.k_tiles, ep, rg);
 }

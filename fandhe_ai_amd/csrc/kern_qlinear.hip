@@ -2107,6 +2107,11 @@ void linear_w8a8_skinny(const int8_t *xq_tiled, const int8_t *w_tiles, uint64_t 
         launch_w8a8_rows<2, kEpiPlain>(m, waves, grid, s, xq_tiled, w_tiles, (uint32_t)m, (uint32_t)n, n_tiles, k_tiles, e);
 }
 
+// Rows up to which the weight-stationary kernels are the faster ones against the large-tile GEMM on small tiles: a prompt pass of
+// four layers at 100 / 130 / 200 / 300 / 512 tokens, us, on them / on the GEMM: width 4096 529 / 613 / 695 / 846 / 1090 against 609 /
+// 640 / 678 / 794 / 940; width 2048 397 / 446 / 502 / 593 / 730 against 448 / 443 / 468 / 535 / 620.
+constexpr uint64_t kRowsMost = 160;
+
 // The split-k form of the weight-stationary kernel (w8a8_wstat_ksplit_kernel): deep, narrow weights (k from 8192 up to
 // what four members x eight wavefronts x eight k-tiles hold, about one column tile per compute unit), more rows than
 // the decode kernels take, and a quarter of the activations (m x k / 4 bytes per block) within what a compute unit
@@ -2121,12 +2126,10 @@ inline bool rows_ksplit_plan(uint64_t m, uint32_t n_tiles, uint32_t k_tiles, int
     if (!sk || !sk->counters || g_rows_kernel == 1 || g_rows_kernel == 2 || g_skinny_ksplit == 1) return false;
     // (k up to what the kernel without the split holds as well, so that a caller without a workspace still has a form)
     if (m <= 64 || n_tiles == 0 || k_tiles < 128 || k_tiles > 224) return false;
-    // measured against the tiled GEMM with its k split and the kernel without the split (us incl. the row quantizer, 65 / 128 /
-    // 200 / 300 / 512 rows): 14336 -> 4096 27.7 / 31.6 / 45.4 / 57.8 / 79.3 against 37.6 / 41.8 / 49.3 / 67.7 / 90.7 and 32.7 /
-    // 36.6 / 53.8 / 69.1 / 102; 11008 -> 4096 26.0 / 29.7 / 43.8 / 53.9 / 71.6 against 34.6 / 39.9 / 43.5 / 56.0 / 76.3; at
-    // 8192 -> 4096 the kernel without the split is the faster one while its rule admits it and the three are level above
+    // against the kernel without the split, us incl. the row quantizer at 65 / 128 rows: 14336 -> 4096 27.7 / 31.6 against 32.7 /
+    // 36.6; 8192 -> 4096 the kernel without the split is the faster one.  Against the large-tile GEMM: kRowsMost.
     if (g_rows_kernel != 3 && k_tiles < 160) return false;
-    if (g_rows_kernel != 3 && (m > 512 || (uint64_t)n_tiles > 2 * (uint64_t)num_cus)) return false;
+    if (g_rows_kernel != 3 && (m > kRowsMost || (uint64_t)n_tiles > 2 * (uint64_t)num_cus)) return false;
     const uint32_t n_groups = (n_tiles + 3) / 4;
     if (n_groups > sk->n_counters) return false;
     p->n_groups = n_groups;
@@ -2149,10 +2152,8 @@ bool linear_w8a8_rows_applies(uint64_t m, uint64_t n_pad, uint64_t k_pad, int nu
     if (rows_ksplit_plan(m, (uint32_t)n_tiles, (uint32_t)k_tiles, num_cus, sk, &kp)) return true;
     if (m <= 64 || n_tiles == 0 || k_tiles == 0 || k_tiles > 224) return false;
     if (g_rows_kernel == 2) return true;
-    // measured against the tiled GEMM with its k split (both with their row quantizer, us): 4096 -> 4096 at 65 / 128 / 300 /
-    // 512 rows 13.9 / 14.8 / 25.7 / 37.1 against 24.3 / 27.5 / 33.2 / 41.1; 14336 -> 4096 at 128 rows 36.9 against 41.5, at 200
-    // rows 54.9 against 48.7: what it costs is the m x k bytes of activations every block pulls from L2
-    return n_tiles <= 2 * (uint64_t)num_cus && m * k_pad <= (2ull << 20);
+    // what it costs is the m x k bytes of activations every block pulls from L2
+    return m <= kRowsMost && n_tiles <= 2 * (uint64_t)num_cus && m * k_pad <= (2ull << 20);
 }
 
 uint64_t linear_w8a8_rows_workspace_bytes(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, const SplitKArea *sk) {

@@ -203,7 +203,7 @@ void linear_w8a8_qkv_rope_rows(const int8_t *xq_tiled, const int8_t *w_tiles, co
 bool gemm_w8a8_qkv_rope_applies(uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad, uint32_t heads, uint32_t kv_heads,
                                 uint32_t head_dim, int num_cus);
 void gemm_w8a8_qkv_rope_mfma(const int8_t *aq, const int8_t *w_tiles, const float *sx, const float *sw, uint64_t m, uint64_t k_pad,
-                             const QkvRopeTargets &t, hipStream_t s);
+                             const QkvRopeTargets &t, int num_cus, hipStream_t s);
 // a: bf16 [m, k] row-major (k == k_pad required), m <= 32.
 void linear_w8a16_skinny(const uint16_t *a, const int8_t *w_tiles, const float *sw, uint64_t m,
                          uint64_t n, uint64_t n_pad, uint64_t k_pad, void *out, int out_bf16,
@@ -367,9 +367,9 @@ struct RowGroups {
 void linear_grouped_bf16(const uint16_t *a, uint64_t lda, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, int num_cus,
                          hipStream_t s);
 void linear_grouped_f32(const float *a, uint64_t lda, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, hipStream_t s);
-void gemm_bf16_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, hipStream_t s);
+void gemm_bf16_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, int num_cus, hipStream_t s);
 // The large-tile form (kern_gemm_mfma.hip): m >= 256, one batch entry, lda == 32 * k_tiles.
-bool gemm_bf16_big_applies(uint64_t lda, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus);
+bool gemm_bf16_big_applies(uint64_t lda, uint64_t m, const LinearWeight &w);
 void gemm_bf16_big(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s);
 // Packs `rows` source rows of `cols` values (bf16 bits or f32; element (r, c) at src[r * row_stride + c * col_stride]) into
 // columns dst_row(r) of a weight: dst_row(r) = n0 + (r / group) * pitch + r % group, from its input k0 on.

@@ -65,3 +65,57 @@ def test_scan_forms(kind, dim, vdim, form, tune):
         assert lc.error(got, want) < F32_TOL, (b, n)
         at += n
     dec.close()
+
+
+def rows_of_gemm(m):
+    """Rows around the edges of 128, 192 and 256 row tiles, and some in the middle."""
+    return np.unique(np.r_[0:4, np.arange(126, m, 64), np.arange(128, m, 64), m - 2:m]) % m
+
+
+@pytest.mark.parametrize("m,k,n", [(161, 1024, 1040), (300, 1152, 1763), (385, 2176, 2048), (517, 1024, 4100), (129, 4096, 1031)])
+@pytest.mark.parametrize("mtb,ntb", [(8, 8), (12, 8), (16, 8), (8, 16), (12, 16), (16, 16), (12, 14), (16, 14), (0, 0)])
+def test_int8_gemm_on_every_tile(mtb, ntb, m, k, n, tune):
+    """Every tile of the large-tile GEMM: raw sums and outputs exact against the oracle with a bias, f32 and bf16, rows and columns
+    that cut the last tiles, rows whose vectors are not aligned, an odd number of k stages, k shared by blocks (the plan's own choice)."""
+    import fandhe_ai_amd as fa
+    import oracle_lib as o
+    be = ops()
+    rng = o.Rng(m + n)
+    x, w, bias = rng.randn((m, k)), rng.randn((k, n), std=0.05), rng.randn((n,))
+    o.set_threads(8)
+    wq, ws = o.quantize_cols_i8(w)
+    want_acc, want = o.linear_w8a8(x, wq, ws, bias)
+    o.set_threads(1)
+    qw, dx, db = be.import_quantized_weight(wq, ws), be.upload(x), fa.DeviceBufferView(be.upload(bias), 0, (n,))
+    tune(21, 1)                                            # no weight-stationary kernel
+    tune(37, mtb)
+    tune(7, ntb)
+    out, acc = be.linear_w8a8(dx, qw, bias=db, want_acc=True)
+    assert np.array_equal(be.download_owned(acc), want_acc)
+    assert np.array_equal(be.download_owned(out), want)
+    for _ in range(2):                                     # the counters of shared tiles are back at zero
+        assert np.array_equal(be.download_owned(be.linear_w8a8(dx, qw, bias=db)), want)
+    got = be.download_owned(be.linear_w8a8(dx, qw, bias=db, out_dtype=fa.capi.BF16))
+    assert np.array_equal(got.astype(np.uint32) << 16, lc.bf16_round(want).view(np.uint32))
+
+
+@pytest.mark.parametrize("m,k,n", [(161, 1024, 1040), (300, 1152, 1763), (385, 2176, 2048), (65, 1024, 28673)])
+@pytest.mark.parametrize("mtb,ntb", [(8, 8), (12, 8), (16, 8), (8, 16), (12, 16), (16, 16), (12, 14), (16, 14)])
+def test_fp8_gemm_on_every_tile(mtb, ntb, m, k, n, tune):
+    """The same for e4m3: products of e4m3 numbers are exact in f32, so any order of the sum is within k roundings of the exact one."""
+    import fandhe_ai_amd as fa
+    import oracle_lib as o
+    be = ops()
+    rng = np.random.default_rng(m * n)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    aq, sa = be.quantize_tensor_e4m3(be.upload(x))
+    qw = be.quantize_weight(fa.DeviceBufferView(be.upload(w), 0, (k, n)), fa.capi.QW_E4M3_TENSOR)
+    codes, sw = qw.export()
+    tune(37, mtb)
+    tune(7, ntb)
+    got = be.download_owned(be.gemm_e4m3(aq, sa, qw, fa.capi.F32))
+    rows = rows_of_gemm(m)
+    a64, w64 = o.from_e4m3(be.download(aq)[rows]).astype(np.float64), o.from_e4m3(codes).astype(np.float64)
+    scale = float(be.download(sa)[0]) * float(sw[0])
+    bound = (np.abs(a64) @ np.abs(w64)) * scale * (k + 2) * 2.0 ** -24
+    assert np.all(np.abs(got[rows] - a64 @ w64 * scale) <= bound)
