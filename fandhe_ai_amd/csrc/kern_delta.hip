@@ -58,13 +58,21 @@ __device__ __forceinline__ float conv_silu(const T *__restrict__ y, uint32_t ld,
 // ------------------------------------------------------------------ token by token
 // One block per (sequence, head); the state sits in registers (thread: four neighbouring columns of up to RPT rows) from
 // the first token of the pass to the last.  CG = column groups of four, a power of two.
-// FAST (single tokens, at most four taps, no more than 2 NT channels): the inputs of the convolution are requested ahead of
+// FAST (single tokens, at most four taps, no more than NQ NT channels): the inputs of the convolution are requested ahead of
 // the state, so that the convolution runs while the state travels.
+// A single token of a few sequences is a chain of latencies: dependent loads, barriers, and the instructions themselves,
+// which come from memory at every launch (about half a microsecond per KiB of code that runs through once).  So a block is
+// a thousand threads with up to eight rows each where few blocks leave the CUs to them (16 K values at four rows), every
+// wavefront forms the norms and k . q for itself, and the wavefronts meet three times: 4 sequences of 16 heads 128 x 128 13.4 us
+// on 256 threads with eight meetings, 11.5 so (32 sequences: 256 threads still, 35.5 us, 27 at the rate of a copy).
+constexpr int step_channels(int nt, int rpt) { return nt == 1024 && rpt <= 8 ? 1 : 2; }
+
 template <typename T, int NT, int RPT, bool FAST, Recurrence KIND>
 __global__ void __launch_bounds__(NT)
     delta_step_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, uint32_t cg_log2, int write_ring, uint32_t max_tokens) {
-    constexpr int NW = NT / 64;
-    extern __shared__ float lds[];                   // q [dim], k [dim], v [vdim_p], partial sums [2][RG][CG * 4], decays [dim]
+    constexpr int NW = NT / 64, NQ = step_channels(NT, RPT);
+    // q [dim], k [dim], v [CG * 4], decays [dim] or shares of S^T k and S^T q [2][parts][CG * 4], their sums [2][CG * 4]
+    extern __shared__ float lds[];
     constexpr bool CHANNEL = KIND == Recurrence::kChannelDelta, LIGHTNING = KIND == Recurrence::kLightning;
     __shared__ float smem[NW];
     const uint32_t b = blockIdx.x, h = blockIdx.y;
@@ -72,19 +80,21 @@ __global__ void __launch_bounds__(NT)
     if (n_tok == 0 || n_tok > max_tokens) return;
     const uint32_t dim = sh.dim, vdim = sh.vdim, vp = sh.vdim_p(), channels = sh.qkv();
     const uint32_t share = sh.heads / sh.kv_heads, hk = h / share;
-    const uint32_t CG = 1u << cg_log2, RG = NT >> cg_log2, cg = threadIdx.x & (CG - 1), rg = threadIdx.x >> cg_log2;
-    const uint32_t dim_a = (dim + 3) / 4 * 4;        // keeps v and the partial sums 16-byte aligned
-    float *lq = lds, *lk = lds + dim_a, *lv = lk + dim_a, *part = lv + CG * 4, *lg = part + 2 * NT * 4;
+    const uint32_t CG = 1u << cg_log2, RG = NT >> cg_log2, cg = threadIdx.x & (CG - 1), rg = threadIdx.x >> cg_log2, lane = threadIdx.x % 64;
+    // a wavefront's row groups are added inside it; parts: what is left to add
+    const uint32_t wide = CG < 64 ? 64 : CG, parts = NT / wide, own_part = threadIdx.x / wide;
+    const uint32_t dim_a = (dim + 3) / 4 * 4;        // keeps v and the shares 16-byte aligned
+    float *lq = lds, *lk = lds + dim_a, *lv = lk + dim_a, *part = lv + CG * 4, *total = part + 2 * parts * CG * 4, *lg = total + 2 * CG * 4;
     const T *y = (const T *)io.y;
     T *ring = (T *)io.ring + (uint64_t)rr.state_slot[b] * sh.taps * channels;
     float *state = io.state + ((uint64_t)rr.state_slot[b] * sh.heads + h) * dim * vp;
     const bool col_ok = cg * 4 < vp;
     const uint32_t p0 = (uint32_t)rr.pos[row0];
     auto channel = [&](uint32_t i) { return i < dim ? hk * dim + i : i < 2 * dim ? (sh.kv_heads + hk) * dim + (i - dim) : 2 * sh.kv_heads * dim + h * vdim + (i - 2 * dim); };
-    float xin[2][4], win[2][4];
+    float xin[NQ][4], win[NQ][4];
     if constexpr (FAST) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < NQ; ++q) {
             const uint32_t i = threadIdx.x + q * NT;
 #pragma unroll
             for (uint32_t back = 0; back < 4; ++back) {
@@ -118,9 +128,8 @@ __global__ void __launch_bounds__(NT)
         const uint64_t row = row0 + t;
         const uint32_t p = p0 + t;
         // q, k, v of this head behind the convolution
-        float sq = 0.0f, sk = 0.0f;
-#pragma unroll FAST ? 2 : 1
-        for (uint32_t q = 0; q < (FAST ? 2u : 0x40000000u); ++q) {
+#pragma unroll FAST ? NQ : 1
+        for (uint32_t q = 0; q < (FAST ? (uint32_t)NQ : 0x40000000u); ++q) {
             const uint32_t i = threadIdx.x + q * NT;
             if (i >= 2 * dim + CG * 4) break;
             float v = 0.0f;
@@ -137,8 +146,6 @@ __global__ void __launch_bounds__(NT)
                 if (write_ring && (i >= 2 * dim || h % share == 0)) ring[(uint64_t)(p % sh.taps) * channels + c] = y[row * io.ld_y + c];
             }
             (i < dim ? lq[i] : i < 2 * dim ? lk[i - dim] : lv[i - 2 * dim]) = v;
-            if (i < dim) sq = fmaf(v, v, sq);
-            else if (i < 2 * dim) sk = fmaf(v, v, sk);
         }
         if constexpr (CHANNEL) {
             if (threadIdx.x < dim) {
@@ -146,39 +153,58 @@ __global__ void __launch_bounds__(NT)
                 lg[threadIdx.x] = expf(log_decay(a_log, decay_in + decay_bias));
             }
         }
-        float rq = 1.0f, rk = 1.0f, beta = 1.0f, g = 1.0f;
+        float beta = 1.0f, g = 1.0f;
         if constexpr (LIGHTNING) {
             g = io.decay[h];
-            __syncthreads();
         } else {
-            rq = 1.0f / sqrtf(block_sum<float, NW, true>(sq, smem) + 1e-6f) / sqrtf((float)dim);
-            rk = 1.0f / sqrtf(block_sum<float, NW, true>(sk, smem) + 1e-6f);
             beta = sigmoid_f32(io.beta[row * io.ld_beta + h]);
             if constexpr (!CHANNEL) g = expf(log_decay(a_log, io.decay[row * io.ld_decay + h] + dt_bias));
         }
+        __syncthreads();
+        float sq = 0.0f, sk = 0.0f, kq = 0.0f;       // the same in every wavefront
+        for (uint32_t d = lane; d < dim; d += 64) {
+            const float kd = lk[d], qd = lq[d];
+            sq = fmaf(qd, qd, sq);
+            sk = fmaf(kd, kd, sk);
+            kq = fmaf(kd, qd, kq);
+        }
+        float rq = 1.0f, rk = 1.0f;
+        kq = wave_sum_dpp(kq);
+        if constexpr (!LIGHTNING) {
+            rq = 1.0f / sqrtf(wave_sum_dpp(sq) + 1e-6f) / sqrtf((float)dim);
+            rk = 1.0f / sqrtf(wave_sum_dpp(sk) + 1e-6f);
+            kq *= rq * rk;
+        }
         // S <- g S; S^T k and S^T q of it in one pass
         v4f dk = v4f{0.f, 0.f, 0.f, 0.f}, dq = dk;
-        float kq = 0.0f;
 #pragma unroll
         for (int i = 0; i < RPT; ++i) {
             const uint32_t d = rg + i * RG;
             if (d >= dim) continue;
-            const float kd = lk[d] * rk, qd = lq[d] * rq;
             S[i] *= CHANNEL ? lg[d] : g;
-            if constexpr (!LIGHTNING) dk += S[i] * kd;
-            dq += S[i] * qd;
-            kq = fmaf(kd, qd, kq);
+            if constexpr (!LIGHTNING) dk += S[i] * (lk[d] * rk);
+            dq += S[i] * (lq[d] * rq);
         }
-        if constexpr (!LIGHTNING) ((v4f *)part)[threadIdx.x] = dk;
-        ((v4f *)part)[NT + threadIdx.x] = dq;
-        // every column group of a row group holds the same share of k . q
-        kq = block_sum<float, NW, true>(cg == 0 ? kq : 0.0f, smem);
-        dk = dq = v4f{0.f, 0.f, 0.f, 0.f};
-        for (uint32_t q = 0; q < RG; ++q) {
-            if constexpr (!LIGHTNING) dk += ((const v4f *)part)[(q << cg_log2) + cg];
-            dq += ((const v4f *)part)[NT + (q << cg_log2) + cg];
+        for (uint32_t off = CG; off < 64; off <<= 1)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (!LIGHTNING) dk[e] += __shfl_xor(dk[e], (int)off, 64);
+                dq[e] += __shfl_xor(dq[e], (int)off, 64);
+            }
+        if (CG >= 64 || lane < CG) {
+            if constexpr (!LIGHTNING) ((v4f *)part)[own_part * CG + cg] = dk;
+            ((v4f *)part)[(parts + own_part) * CG + cg] = dq;
         }
-        const v4f u = LIGHTNING ? *(const v4f *)(lv + cg * 4) : (*(const v4f *)(lv + cg * 4) - dk) * beta;
+        __syncthreads();
+        if (threadIdx.x < 2 * CG) {                  // (2 CG <= NT)
+            v4f x = v4f{0.f, 0.f, 0.f, 0.f};
+            if (!LIGHTNING || threadIdx.x >= CG)
+                for (uint32_t q = 0; q < parts; ++q) x += ((const v4f *)part)[(threadIdx.x / CG * parts + q) * CG + cg];
+            ((v4f *)total)[threadIdx.x] = x;
+        }
+        __syncthreads();
+        dq = ((const v4f *)total)[CG + cg];
+        const v4f u = LIGHTNING ? *(const v4f *)(lv + cg * 4) : (*(const v4f *)(lv + cg * 4) - ((const v4f *)total)[cg]) * beta;
 #pragma unroll
         for (int i = 0; i < RPT; ++i) {
             const uint32_t d = rg + i * RG;
@@ -192,16 +218,18 @@ __global__ void __launch_bounds__(NT)
                 for (int e = 0; e < 4; ++e)
                     if (cg * 4 + e < vdim) io.raw[(row * sh.heads + h) * vdim + cg * 4 + e] = o[e];
             }
-            __syncthreads();
+            if (t + 1 < n_tok) __syncthreads();
             continue;
         }
+        // up to 64 column groups are a wavefront's lanes (each as often as it has row groups)
         float so = 0.0f;
-        if (rg == 0) {
+        if (CG <= 64 ? lane < CG : rg == 0) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (cg * 4 + e < vdim) so = fmaf(o[e], o[e], so);
         }
-        const float ro = 1.0f / sqrtf(block_sum<float, NW, true>(so, smem) / (float)vdim + sh.eps);
+        so = CG <= 64 ? wave_sum_dpp(so) : block_sum<float, NW, true>(so, smem);
+        const float ro = 1.0f / sqrtf(so / (float)vdim + sh.eps);
         if (rg == 0) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -212,7 +240,7 @@ __global__ void __launch_bounds__(NT)
                 }
             }
         }
-        __syncthreads();                             // q, k, v and the partial sums are overwritten by the next token
+        if (t + 1 < n_tok) __syncthreads();          // q, k, v and the sums are overwritten by the next token
     }
 }
 
@@ -1196,18 +1224,28 @@ __global__ void __launch_bounds__(256) delta_ring_kernel(DeltaShape sh, DeltaIo 
 
 template <typename T, int NT, Recurrence KIND>
 void launch_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, uint32_t cg_log2, int write_ring, uint32_t max_tokens, hipStream_t s) {
-    const uint32_t rg = NT >> cg_log2, rpt = (sh.dim + rg - 1) / rg;
-    const size_t lds = (3 * ((sh.dim + 3) / 4 * 4) + (4u << cg_log2) + 2 * NT * 4) * 4;
+    const uint32_t CG = 1u << cg_log2, rg = NT >> cg_log2, parts = NT / std::max(CG, 64u);
+    const size_t lds = (3 * ((sh.dim + 3) / 4 * 4) + 4 * CG + 2 * (parts + 1) * 4 * CG) * 4;
     const dim3 grid(rr.batch, sh.heads);
-    // FAST's channels fit two per thread by the caller's check
 #define FA_STEP(R_)                                                                                                   \
     fast ? delta_step_kernel<T, NT, R_, true, KIND><<<grid, NT, lds, s>>>(sh, io, rr, cg_log2, write_ring, max_tokens)       \
          : delta_step_kernel<T, NT, R_, false, KIND><<<grid, NT, lds, s>>>(sh, io, rr, cg_log2, write_ring, max_tokens)
-    const bool fast = max_tokens == 1 && sh.taps <= 4 && 2 * sh.dim + (4u << cg_log2) <= 2 * NT;
-    if (rpt <= 8) FA_STEP(8);
-    else if (rpt <= 16) FA_STEP(16);
-    else if (rpt <= 32) FA_STEP(32);
-    else FA_STEP(64);
+    const uint32_t in = 2 * sh.dim + 4 * CG;
+    const bool fast = max_tokens == 1 && sh.taps <= 4 && in <= 2 * NT;
+    // (FAST's few rows come with one channel per thread)
+    const uint32_t rpt = fast && NT == 1024 && in > NT ? std::max(16u, (sh.dim + rg - 1) / rg) : (sh.dim + rg - 1) / rg;
+    if constexpr (NT == 1024) {
+        if (rpt <= 4) FA_STEP(4);
+        else if (rpt <= 8) FA_STEP(8);
+        else if (rpt <= 16) FA_STEP(16);
+        else if (rpt <= 32) FA_STEP(32);
+        else FA_STEP(64);
+    } else {
+        if (rpt <= 4) FA_STEP(4);
+        else if (rpt <= 16) FA_STEP(16);
+        else if (rpt <= 32) FA_STEP(32);
+        else FA_STEP(64);
+    }
 #undef FA_STEP
 }
 
@@ -1219,8 +1257,12 @@ void mixer_kind(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, u
     const bool chunks = max_new >= kChunkFrom && g_delta_form != 1;
     const uint32_t longest = chunks ? kChunkFrom - 1 : max_new;      // sequences of a pass go to one of the two forms by length
     if (!chunks || rr.batch > 1) {
-        if (cg_log2 <= 6) launch_step<T, 256, KIND>(sh, io, rr, cg_log2, write_ring, longest, s);
-        else launch_step<T, 1024, KIND>(sh, io, rr, cg_log2, write_ring, longest, s);
+        // A thousand threads where every block has a CU to itself and eight rows per thread hold the state (or where 256
+        // threads have too few columns); from two blocks per CU on the small ones stand in each other's waits.  A turn of 16
+        // steps, heads of 128 x 128, 256 and 1024 threads: 64 blocks 6100 and 6014 us, 256 6640 and 6590, 512 7402 and 7580,
+        // 1024 9341 and 9723.
+        if (cg_log2 > 6 || ((uint64_t)rr.batch * sh.heads <= 256 && ((uint64_t)sh.dim << cg_log2) <= 8 * 1024)) launch_step<T, 1024, KIND>(sh, io, rr, cg_log2, write_ring, longest, s);
+        else launch_step<T, 256, KIND>(sh, io, rr, cg_log2, write_ring, longest, s);
     }
     if (chunks) run_chunks<T, KIND>(sh, io, rr, s);
     if (!write_ring && sh.taps) delta_ring_kernel<T><<<dim3(rr.batch, (sh.qkv() + 255) / 256), 256, 0, s>>>(sh, io, rr);

@@ -67,6 +67,29 @@ def test_scan_forms(kind, dim, vdim, form, tune):
     dec.close()
 
 
+@pytest.mark.parametrize("dim,vdim,batch", [(9, 7, 3), (128, 128, 3), (256, 127, 3), (256, 132, 3), (130, 260, 3), (256, 300, 3),
+                                            (20, 1000, 3), (128, 128, 100), (40, 72, 160)])
+@pytest.mark.parametrize("kind", sorted(RECURRENCES))
+def test_single_tokens(kind, dim, vdim, batch):
+    """Steps behind prompts shorter and longer than the convolution: four rows of a state per thread, eight, and 64; 256
+    threads and 1024; more columns than 64 groups; more inputs than threads; as many blocks as CUs and more."""
+    cfg = RECURRENCES[kind](dim, vdim)
+    w = lc.weights(cfg, 5)
+    steps = 3
+    dec = lc.make_decoder(ops(), cfg, w, max_tokens=4096, max_batch=batch)
+    lens = [1 + i % 7 for i in range(batch)]
+    toks = [lc.tokens(cfg, n + steps, 40 + i % 3) for i, n in enumerate(lens)]
+    table = np.full((batch, dec.cfg.max_blocks_per_seq), 0xFFFFFFFF, dtype=np.uint32)
+    table[:, 0] = np.arange(batch)
+    dec.set_sequences(table, [0] * batch)
+    dec.forward([t[:n] for t, n in zip(toks, lens)], [list(range(n)) for n in lens])
+    got = [dec.forward([t[n + i:n + i + 1] for t, n in zip(toks, lens)], [[0]] * batch) for i in range(steps)]
+    for b in list(range(min(batch, 3))) + [batch - 1]:
+        want = oracle.forward(cfg, w, toks[b])[lens[b]:]
+        assert lc.error(np.stack([g[b] for g in got]), want) < F32_TOL, b
+    dec.close()
+
+
 def rows_of_gemm(m):
     """Rows around the edges of 128, 192 and 256 row tiles, and some in the middle."""
     return np.unique(np.r_[0:4, np.arange(126, m, 64), np.arange(128, m, 64), m - 2:m]) % m
