@@ -58,12 +58,13 @@ __device__ __forceinline__ void hold(v8bf (&r)[N]) {
 // 2^x without the detour for subnormal results (weights that small count as zero)
 __device__ __forceinline__ float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// Maximum over the four lanes with equal lane % 16, in every one of them.
+// Maximum over the four lanes with equal lane % 16, in every one of them; NaN if any is.  (maximum needs no instruction to
+// quiet its operands first, fmaxf needs two.)
 __device__ __forceinline__ float column_max(float v) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);      // rows of 16: 0 0 2 2 and 1 1 3 3
-    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    v = __builtin_elementwise_maximum(__uint_as_float(r[0]), __uint_as_float(r[1]));
     const auto q = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(q[0]), __uint_as_float(q[1]));
+    return __builtin_elementwise_maximum(__uint_as_float(q[0]), __uint_as_float(q[1]));
 }
 
 // One online-softmax step of a column (query row): scores of eight keys per lane, lanes with equal lane % 16 share the

@@ -1,6 +1,7 @@
 // Paged KV cache kernels: row scatter (append), a generic attention kernel
 // that keeps the reference's per-row summation order, and the decode fast
 // path (bf16, head_dim 128, 16-token pages, one query token, grouped-query).
+#include "attention_tiles.hpp"
 #include "device_utils.hpp"
 #include "index_models.hpp"
 #include "kernels.hpp"
@@ -906,18 +907,22 @@ __global__ void __launch_bounds__(1024) decode_stream_merge_quantize_kernel(Stre
 // ------------------------------------------------------- prefill, block form
 // Causal attention of many new tokens per row, one block of NW wavefronts per (row, kv head, tile of
 // 32 NW / group new tokens).  The block walks the cached positions once, 32 at a time: the K and V rows
-// of a step are staged in LDS (two stages; the loads of the next three steps are in flight while this
-// one is multiplied) and shared by the wavefronts, so K / V leave the L2 once per tile.  Every
+// of a step are staged in LDS (two stages, K a step ahead of V; the rows of a step are requested three steps
+// ahead) and shared by the wavefronts, so K / V leave the L2 once per tile.  Every
 // wavefront owns 32 columns (new token x head of the group, column = token * group + head):
 //   S^T = K Q^T on v_mfma_f32_16x16x32_bf16 as in the decode kernel (lane (g, c): positions 4g .. 4g+3
 //   of a 16-position tile for column c), two position tiles per step;
 //   O^T += V^T P^T on the same instruction with k = the 32 positions of the step: the operand slot
 //   8g + i of a lane is position 4g + i of the first tile (i < 4) or of the second (i >= 4), which is
-//   where the scores of that lane already are; V^T is read from the staged rows 4 bytes (two dims of
-//   one position) at a time and split into an even and an odd operand by byte permutes.  Every f32
-//   weight is fed as three bf16 terms that add up to it exactly, as in the decode kernel.
-// The running maximum is per column; accumulators are rescaled only on steps where some column's maximum
-// grew.  A step wholly past the causal limit of all the columns of a wavefront is skipped by it.  The
+//   where the scores of that lane already are; V^T is read from the staged rows by transposing reads.
+//   Every f32 weight is fed as three bf16 terms that add up to it exactly, as in the decode kernel.
+// Bound by a wavefront's own chain (scores, maximum, weights, products) on two wavefronts per SIMD, then by the issue of
+// vector instructions (about 250 a step beside 64 products).  So the next step's scores are multiplied while this step's
+// weights are formed, the maximum crosses lanes by swaps, and the accumulators are rescaled only where a maximum has grown by
+// 2^8 or more: with 32 columns some maximum grows in most steps.  4 x 2048 tokens, 32 / 8 heads: 413 us with all that in
+// turn, exchanges through LDS and V^T by byte permutes, 367 so; 2545 tokens in five sequences, 16 / 4 heads 39 and 34;
+// 300 tokens of one 17.8 and 15.5.  Error against 64 bits (900 tokens, unit scores): 2.2e-8 r.m.s. (2.3e-8 before).
+// A step wholly past the causal limit of all the columns of a wavefront is skipped by it.  The
 // result is normalised and written by the block itself (no partial results, no merge pass).
 struct FlashParams {
     const uint16_t *q, *k_pool, *v_pool;
@@ -933,6 +938,34 @@ struct FlashParams {
     float *part_o, *part_ml;
 };
 constexpr int kFlashNQ = 2, kFlashKeys = 32;
+
+// Weights of eight scores as three bf16 terms that add up to each exactly; returns their sum.
+__device__ __forceinline__ float weights_3(const v4f (&sc)[2], float to_log2, float ref, v8bf (&w)[3]) {
+    float sum = 0.0f;
+    v4u ph, pm, pl;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float e[2];
+        uint32_t hi[2], mid[2], lo[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            // one rounding; whatever the reference was rounded to is the same for the whole column.  Masked: exp2(-inf) = 0
+            e[h] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i / 2][2 * (i % 2) + h], to_log2, -ref));
+            hi[h] = __float_as_uint(e[h]) & 0xffff0000u;
+            const float r1 = e[h] - __uint_as_float(hi[h]);
+            mid[h] = __float_as_uint(r1) & 0xffff0000u;
+            lo[h] = __float_as_uint(r1 - __uint_as_float(mid[h]));
+        }
+        sum += e[0] + e[1];
+        ph[i] = __builtin_amdgcn_perm(hi[1], hi[0], 0x07060302u);
+        pm[i] = __builtin_amdgcn_perm(mid[1], mid[0], 0x07060302u);
+        pl[i] = __builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u);
+    }
+    w[0] = __builtin_bit_cast(v8bf, ph);
+    w[1] = __builtin_bit_cast(v8bf, pm);
+    w[2] = __builtin_bit_cast(v8bf, pl);
+    return sum;
+}
 
 // NQ: column tiles of 16 per wavefront (2: 32 columns; 1: 16 columns, half the multiplies per step and twice the blocks,
 // for prompts that leave most compute units without a block).
@@ -989,7 +1022,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             v4u t4 = *(const v4u *)(qrow + 32 * s);
-            if (!valid[qi]) t4 = v4u{0, 0, 0, 0};
+            if (!valid[qi] || p.scale == 0.0f) t4 = v4u{0, 0, 0, 0};
+            if (p.scale < 0.0f) t4 ^= 0x80008000u;
             qb[qi][s] = __builtin_bit_cast(v8bf, t4);
         }
         const uint32_t l = base + t + 1;
@@ -1023,34 +1057,49 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         if (id >= p.num_blocks) id = 0;
         return ((uint64_t)id * kPage + (it * kFlashKeys + ps * kRows + r_st) % kPage) * p.e_kv + (uint64_t)kvh * kDh + 8 * c16;
     };
-    v4u k_a[kPasses], v_a[kPasses], k_b[kPasses], v_b[kPasses];  // rows of step it + 1 (a) and it + 2 (b)
-    uint32_t id_c[kPasses];                                      // page ids of step it + 3
+    v4u k_a[kPasses], v_a[kPasses];                              // K rows of step it + 2, V rows of step it + 1
+    uint32_t id_k[kPasses], id_v[kPasses];                       // page ids of the steps that are requested next: it + 3, it + 2
+    auto put = [&](uint16_t *rows, const v4u (&x)[kPasses]) {
+#pragma unroll
+        for (int ps = 0; ps < kPasses; ++ps) *(v4u *)(&rows[(ps * kRows + r_st) * kVPitch + 8 * c16]) = x[ps];
+    };
+    auto no_rows_past = [&](uint32_t it, v4u (&x)[kPasses]) {     // the pool may hold anything past the sequence end
+#pragma unroll
+        for (int ps = 0; ps < kPasses; ++ps)
+            if (it * kFlashKeys + ps * kRows + r_st >= ctx) x[ps] = v4u{0, 0, 0, 0};
+    };
 #pragma unroll
     for (int ps = 0; ps < kPasses; ++ps) {
-        k_a[ps] = v_a[ps] = k_b[ps] = v_b[ps] = v4u{0, 0, 0, 0};
-        id_c[ps] = 0;
+        k_a[ps] = v_a[ps] = v4u{0, 0, 0, 0};
+        id_k[ps] = id_v[ps] = 0;
     }
     if (n_it > it_lo) {
+        v4u k0[kPasses], k1[kPasses], v0[kPasses];
 #pragma unroll
         for (int ps = 0; ps < kPasses; ++ps) {
-            const uint32_t id0 = load_id(it_lo, ps), id1 = load_id(it_lo + 1, ps), id2 = load_id(it_lo + 2, ps);
-            id_c[ps] = load_id(it_lo + 3, ps);
-            const uint64_t off0 = row_off(it_lo, ps, id0), off1 = row_off(it_lo + 1, ps, id1), off2 = row_off(it_lo + 2, ps, id2);
-            v4u k0 = *(const v4u *)(p.k_pool + off0), v0 = *(const v4u *)(p.v_pool + off0);
-            k_a[ps] = *(const v4u *)(p.k_pool + off1);
+            const uint32_t id0 = load_id(it_lo, ps), id1 = load_id(it_lo + 1, ps);
+            id_v[ps] = load_id(it_lo + 2, ps);
+            id_k[ps] = load_id(it_lo + 3, ps);
+            const uint64_t off0 = row_off(it_lo, ps, id0), off1 = row_off(it_lo + 1, ps, id1);
+            k0[ps] = *(const v4u *)(p.k_pool + off0);
+            v0[ps] = *(const v4u *)(p.v_pool + off0);
+            k1[ps] = *(const v4u *)(p.k_pool + off1);
             v_a[ps] = *(const v4u *)(p.v_pool + off1);
-            k_b[ps] = *(const v4u *)(p.k_pool + off2);
-            v_b[ps] = *(const v4u *)(p.v_pool + off2);
-            const uint32_t row = ps * kRows + r_st;
-            if (it_lo * kFlashKeys + row >= ctx) v0 = v4u{0, 0, 0, 0};   // the pool may hold anything past the sequence end
-            *(v4u *)(&k_s[0][row * kVPitch + 8 * c16]) = k0;
-            *(v4u *)(&v_s[0][row * kVPitch + 8 * c16]) = v0;
+            k_a[ps] = *(const v4u *)(p.k_pool + row_off(it_lo + 2, ps, id_v[ps]));
         }
+        no_rows_past(it_lo, v0);
+        put(k_s[0], k0);
+        put(k_s[1], k1);
+        put(v_s[0], v0);
     }
     __syncthreads();
 
+    // m_run, the columns' reference in powers of two, follows the running maximum when that has grown by more than 2^kSlack:
+    // a weight may be that much above one, and the accumulators are rescaled in the first steps only
+    constexpr float kSlack = 8.0f;
+    const float to_log2 = p.scale == 0.0f ? kLog2e : fabsf(p.scale) * kLog2e;
     float m_run[NQ], l_run[NQ];
-    v4f o[NQ][8];
+    v4f o[NQ][8], sc[NQ][2];
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
         m_run[qi] = -INFINITY;
@@ -1058,147 +1107,102 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int t = 0; t < 8; ++t) o[qi][t] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    constexpr float kLog2e = 1.4426950408889634f;
+    auto scores = [&](int st, v4f (&x)[NQ][2]) {      // of a step: two tiles of 16 positions
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+            for (int qi = 0; qi < NQ; ++qi) x[qi][kt] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const v8bf ka = *(const v8bf *)(&k_s[st][(kt * 16 + c) * kVPitch + 32 * s + 8 * g]);
+#pragma unroll
+                for (int qi = 0; qi < NQ; ++qi) x[qi][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[qi][s], x[qi][kt], 0, 0, 0);
+            }
+        }
+    };
+    if (it_lo < n_it) scores(0, sc);
+    __syncthreads();                                  // the first K stage is written again in the first step
 
     for (uint32_t it = it_lo; it < n_it; ++it) {
         const int st = (it - it_lo) & 1;
-        // requests of this step: the rows of step it + 3 (their page id was requested one step ago) and the
-        // page id of step it + 4
         v4u k_n[kPasses], v_n[kPasses];
 #pragma unroll
         for (int ps = 0; ps < kPasses; ++ps) {
-            const uint32_t id_use = id_c[ps];
-            id_c[ps] = load_id(it + 4, ps);
-            const uint64_t off_n = row_off(it + 3, ps, id_use);
-            k_n[ps] = *(const v4u *)(p.k_pool + off_n);
-            v_n[ps] = *(const v4u *)(p.v_pool + off_n);
+            k_n[ps] = *(const v4u *)(p.k_pool + row_off(it + 3, ps, id_k[ps]));
+            v_n[ps] = *(const v4u *)(p.v_pool + row_off(it + 2, ps, id_v[ps]));
+            id_v[ps] = id_k[ps];
+            id_k[ps] = load_id(it + 4, ps);
         }
         const uint32_t key0 = it * kFlashKeys;
         if (key0 < wmax) {
-            // ---- scores of the step: two tiles of 16 positions
-            float sc[NQ][8];
-#pragma unroll
-            for (int kt = 0; kt < 2; ++kt) {
-                v4u ka[4];
-#pragma unroll
-                for (int s = 0; s < 4; ++s) ka[s] = *(const v4u *)(&k_s[st][(kt * 16 + c) * kVPitch + 32 * s + 8 * g]);
-#pragma unroll
-                for (int qi = 0; qi < NQ; ++qi) {
-                    v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int s = 0; s < 4; ++s)
-                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, ka[s]), qb[qi][s], acc, 0, 0, 0);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) sc[qi][kt * 4 + j] = acc[j] * p.scale;
-                }
-            }
             if (key0 + kFlashKeys > wmin) {
 #pragma unroll
                 for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
                     for (int i = 0; i < 8; ++i) {
                         const uint32_t tok = key0 + (i / 4) * 16 + 4 * g + (i % 4);
-                        sc[qi][i] = tok < lim[qi] ? sc[qi][i] : -INFINITY;
+                        sc[qi][i / 4][i % 4] = tok < lim[qi] ? sc[qi][i / 4][i % 4] : -INFINITY;
                     }
             }
-            // ---- running maximum per column (lanes with equal c hold one column)
-            float m_new[NQ], m_use[NQ];
+            float mx[NQ];
             bool grew = false;
 #pragma unroll
             for (int qi = 0; qi < NQ; ++qi) {
-                float m = sc[qi][0];
+                const v4f x = sc[qi][0], y = sc[qi][1];
+                float m = x[0];
 #pragma unroll
-                for (int i = 1; i < 8; ++i) m = fmaxf(m, sc[qi][i]);
-                m = fmaxf(m, __shfl_xor(m, 16, 64));
-                m = fmaxf(m, __shfl_xor(m, 32, 64));
-                m_new[qi] = fmaxf(m_run[qi], m);
-                grew = grew || m_new[qi] > m_run[qi];
-                // every score of a column can be masked so far: its maximum stays -inf and the exponentials
-                // are taken against 0
-                m_use[qi] = m_new[qi] == -INFINITY ? 0.0f : m_new[qi];
+                for (int e = 1; e < 4; ++e) m = __builtin_elementwise_maximum(m, x[e]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m = __builtin_elementwise_maximum(m, y[e]);
+                mx[qi] = column_max(m) * to_log2;
+                grew = grew || mx[qi] > m_run[qi] + kSlack;
             }
-            if (__ballot(grew) != 0) {
+            if (__any(grew)) {
 #pragma unroll
                 for (int qi = 0; qi < NQ; ++qi) {
-                    const float alpha = __builtin_amdgcn_exp2f((m_run[qi] - m_use[qi]) * kLog2e);   // first step: exp2(-inf) = 0
+                    const float m_new = fmaxf(m_run[qi], mx[qi]), ref = m_new == -INFINITY ? 0.0f : m_new;
+                    const float alpha = __builtin_amdgcn_exp2f(m_run[qi] - ref);    // first step: exp2(-inf) = 0
+                    m_run[qi] = m_new;
                     l_run[qi] *= alpha;
 #pragma unroll
                     for (int t = 0; t < 8; ++t) o[qi][t] = o[qi][t] * alpha;
                 }
             }
-            // each f32 weight as three bf16 operands by repeated truncation: hi + mid + lo == weight exactly
-            v8bf p_hi[NQ], p_mid[NQ], p_lo[NQ];
+            // the next step's scores are multiplied while this one's weights are formed
+            v4f sn[NQ][2];
+            scores(st ^ 1, sn);
+            v8bf vt[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) vt[t] = transposed_keys(v_s[st] + 16 * t, kVPitch, lane);
 #pragma unroll
             for (int qi = 0; qi < NQ; ++qi) {
-                m_run[qi] = m_new[qi];
-                float sum = 0.0f;
-                v4u ph, pm, pl;
+                // every score of a column can be masked so far: its reference is -inf and the exponentials are taken against 0
+                const float ref = m_run[qi] == -INFINITY ? 0.0f : m_run[qi];
+                v8bf w[3];
+                l_run[qi] += weights_3(sc[qi], to_log2, ref, w);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float e[2];
-                    uint32_t hi[2], mid[2], lo[2];
+                for (int u = 2; u >= 0; --u)          // smallest terms first
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        // the difference is exact for scores near the maximum, which carry the weight;
-                        // masked scores: exp2(-inf) = 0
-                        e[h] = __builtin_amdgcn_exp2f((sc[qi][2 * i + h] - m_use[qi]) * kLog2e);
-                        hi[h] = __float_as_uint(e[h]) & 0xffff0000u;
-                        const float r1 = e[h] - __uint_as_float(hi[h]);
-                        mid[h] = __float_as_uint(r1) & 0xffff0000u;
-                        lo[h] = __float_as_uint(r1 - __uint_as_float(mid[h]));
-                    }
-                    sum += e[0] + e[1];
-                    ph[i] = __builtin_amdgcn_perm(hi[1], hi[0], 0x07060302u);
-                    pm[i] = __builtin_amdgcn_perm(mid[1], mid[0], 0x07060302u);
-                    pl[i] = __builtin_amdgcn_perm(lo[1], lo[0], 0x07060302u);
-                }
-                l_run[qi] += sum;
-                p_hi[qi] = __builtin_bit_cast(v8bf, ph);
-                p_mid[qi] = __builtin_bit_cast(v8bf, pm);
-                p_lo[qi] = __builtin_bit_cast(v8bf, pl);
+                    for (int t = 0; t < 8; ++t) o[qi][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vt[t], w[u], o[qi][t], 0, 0, 0);
             }
-            // ---- O^T += V^T P^T
 #pragma unroll
-            for (int bp = 0; bp < 4; ++bp) {
-                uint32_t w[8];
+            for (int qi = 0; qi < NQ; ++qi)
 #pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    w[i] = *(const uint32_t *)(&v_s[st][((i / 4) * 16 + 4 * g + (i % 4)) * kVPitch + 32 * bp + 2 * c]);
-                v4u ae, ao;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    ae[i] = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x05040100u);
-                    ao[i] = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], 0x07060302u);
-                }
-                const v8bf a_even = __builtin_bit_cast(v8bf, ae), a_odd = __builtin_bit_cast(v8bf, ao);
-#pragma unroll
-                for (int qi = 0; qi < NQ; ++qi) {
-                    // smallest terms first
-                    o[qi][2 * bp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_even, p_lo[qi], o[qi][2 * bp], 0, 0, 0);
-                    o[qi][2 * bp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_odd, p_lo[qi], o[qi][2 * bp + 1], 0, 0, 0);
-                    o[qi][2 * bp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_even, p_mid[qi], o[qi][2 * bp], 0, 0, 0);
-                    o[qi][2 * bp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_odd, p_mid[qi], o[qi][2 * bp + 1], 0, 0, 0);
-                    o[qi][2 * bp] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_even, p_hi[qi], o[qi][2 * bp], 0, 0, 0);
-                    o[qi][2 * bp + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_odd, p_hi[qi], o[qi][2 * bp + 1], 0, 0, 0);
-                }
-            }
+                for (int kt = 0; kt < 2; ++kt) sc[qi][kt] = sn[qi][kt];
         }
-        // rows of step it + 1 go to the other stage (its readers passed the barrier of the last step)
+        // K two steps and V one step ahead go to stages whose readers passed the barrier of the last step
+        no_rows_past(it + 1, v_a);
+        put(k_s[st], k_a);
+        put(v_s[st ^ 1], v_a);
 #pragma unroll
         for (int ps = 0; ps < kPasses; ++ps) {
-            const uint32_t row = ps * kRows + r_st;
-            if ((it + 1) * kFlashKeys + row >= ctx) v_a[ps] = v4u{0, 0, 0, 0};
-            *(v4u *)(&k_s[st ^ 1][row * kVPitch + 8 * c16]) = k_a[ps];
-            *(v4u *)(&v_s[st ^ 1][row * kVPitch + 8 * c16]) = v_a[ps];
-            k_a[ps] = k_b[ps];
-            v_a[ps] = v_b[ps];
-            k_b[ps] = k_n[ps];
-            v_b[ps] = v_n[ps];
+            k_a[ps] = k_n[ps];
+            v_a[ps] = v_n[ps];
         }
         __syncthreads();
     }
 
-    // lane (g, c) holds, for column c: dims 32 bp + 8 g + {0..7} = {o[2bp][0], o[2bp+1][0], o[2bp][1], ...}
+    // lane (g, c) holds, for column c, dims 16 t + 4 g + {0..3}
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
         float l = l_run[qi];
@@ -1209,12 +1213,9 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
         if (p.nsplit > 1) {
             const uint32_t cols = NW * NQ * 16, col = (uint32_t)wave * (NQ * 16) + qi * 16 + c;
             const uint64_t slot = (uint64_t)blockIdx.x * p.nsplit + blockIdx.y;
-            float *po = p.part_o + (slot * cols + col) * kDh + 8 * g;
+            float *po = p.part_o + (slot * cols + col) * kDh + 4 * g;
 #pragma unroll
-            for (int bp = 0; bp < 4; ++bp) {
-                *(v4f *)(po + 32 * bp) = v4f{o[qi][2 * bp][0], o[qi][2 * bp + 1][0], o[qi][2 * bp][1], o[qi][2 * bp + 1][1]};
-                *(v4f *)(po + 32 * bp + 4) = v4f{o[qi][2 * bp][2], o[qi][2 * bp + 1][2], o[qi][2 * bp][3], o[qi][2 * bp + 1][3]};
-            }
+            for (int t = 0; t < 8; ++t) *(v4f *)(po + 16 * t) = o[qi][t];
             if (g == 0) {
                 const float nanv = __uint_as_float(0x7fc00000u);
                 p.part_ml[slot * (2 * cols) + col] = nan_out ? nanv : m_run[qi];
@@ -1223,25 +1224,16 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             continue;
         }
 #pragma unroll
-        for (int bp = 0; bp < 4; ++bp) {
-            float r8[8];
+        for (int t = 0; t < 8; ++t) {
+            v4f r;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float acc = o[qi][2 * bp + (e & 1)][e / 2];
-                float res = l > 0.0f ? __fdiv_rn(acc, l) : 0.0f;
-                r8[e] = nan_out ? __uint_as_float(0x7fc00000u) : res;
+            for (int e = 0; e < 4; ++e) {
+                const float res = l > 0.0f ? __fdiv_rn(o[qi][t][e], l) : 0.0f;
+                r[e] = nan_out ? __uint_as_float(0x7fc00000u) : res;
             }
-            const uint64_t oi = out_row[qi] + 32 * bp + 8 * g;
-            if (p.out_bf16) {
-                v4u pk;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    pk[e] = (uint32_t)f32_to_bf16(r8[2 * e]) | ((uint32_t)f32_to_bf16(r8[2 * e + 1]) << 16);
-                *(v4u *)((uint16_t *)p.out + oi) = pk;
-            } else {
-                *(v4f *)((float *)p.out + oi) = v4f{r8[0], r8[1], r8[2], r8[3]};
-                *(v4f *)((float *)p.out + oi + 4) = v4f{r8[4], r8[5], r8[6], r8[7]};
-            }
+            const uint64_t oi = out_row[qi] + 16 * t + 4 * g;
+            if (p.out_bf16) *(v2u *)((uint16_t *)p.out + oi) = v2u{f32x2_to_bf16x2(r[0], r[1]), f32x2_to_bf16x2(r[2], r[3])};
+            else *(v4f *)((float *)p.out + oi) = r;
         }
     }
 }
@@ -1282,7 +1274,7 @@ __global__ void __launch_bounds__(1024) flash_split_merge_kernel(FlashParams p) 
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const float w = z0 + u < p.nsplit ? expf(m[u] - m_use) : 0.0f;           // a share that saw nothing: exp(-inf) = 0
+            const float w = z0 + u < p.nsplit ? exp2f(m[u] - m_use) : 0.0f;           // a share that saw nothing: exp(-inf) = 0
             den = __builtin_fmaf(w, l[u], den);
             acc = __builtin_fmaf(w, o[u], acc);
         }
