@@ -21,7 +21,7 @@ extern int g_skinny_ntw, g_skinny_waves, g_skinny_astat, g_gemm_small_tiles, g_g
 int g_decode_waves = 0;
 int g_prefill_generic = 0;
 extern int g_layered_rows;
-extern int g_prefill_rows, g_prefill_fused_rows, g_decode_partials_only, g_prefill_block_form, g_prefill_block_waves, g_prefill_block_split, g_prefill_block_cols;
+extern int g_prefill_rows, g_prefill_fused_rows, g_decode_partials_only, g_prefill_block_form, g_prefill_block_split, g_prefill_block_cols;
 }  // namespace fa
 
 namespace {
@@ -89,7 +89,7 @@ fa_status fa_set_tuning(int32_t key, int32_t value) {
         case 8: fa::g_prefill_generic = value; return FA_OK;
         case 9: k::g_gemm_split_fill = value; return FA_OK;
         case 10: fa::g_prefill_block_form = value; return FA_OK;
-        case 11: fa::g_prefill_block_waves = value; return FA_OK;
+        case 11: return FA_OK;            // blocks have four wavefronts
         case 12: fa::g_prefill_block_split = value; return FA_OK;
         case 13: k::g_gemm_f32_form = value; return FA_OK;
         case 14: k::g_weight_prefetch = value; return FA_OK;

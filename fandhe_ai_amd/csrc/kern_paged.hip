@@ -905,10 +905,9 @@ __global__ void __launch_bounds__(1024) decode_stream_merge_quantize_kernel(Stre
 }
 
 // ------------------------------------------------------- prefill, block form
-// Causal attention of many new tokens per row, one block of NW wavefronts per (row, kv head, tile of
-// 32 NW / group new tokens).  The block walks the cached positions once, 32 at a time: the K and V rows
-// of a step are staged in LDS (two stages, K a step ahead of V; the rows of a step are requested three steps
-// ahead) and shared by the wavefronts, so K / V leave the L2 once per tile.  Every
+// Causal attention of many new tokens per row, one block of four wavefronts per (row, kv head, tile of
+// 128 / group new tokens; NQ = 1: 64 / group).  The block walks the cached positions once, 32 at a time: the K and V rows
+// of a step are staged in LDS (three stages, filled by loads that write LDS themselves) and shared by the wavefronts, so K / V leave the L2 once per tile.  Every
 // wavefront owns 32 columns (new token x head of the group, column = token * group + head):
 //   S^T = K Q^T on v_mfma_f32_16x16x32_bf16 as in the decode kernel (lane (g, c): positions 4g .. 4g+3
 //   of a 16-position tile for column c), two position tiles per step;
@@ -918,10 +917,12 @@ __global__ void __launch_bounds__(1024) decode_stream_merge_quantize_kernel(Stre
 //   Every f32 weight is fed as three bf16 terms that add up to it exactly, as in the decode kernel.
 // Bound by a wavefront's own chain (scores, maximum, weights, products) on two wavefronts per SIMD, then by the issue of
 // vector instructions (about 250 a step beside 64 products).  So the next step's scores are multiplied while this step's
-// weights are formed, the maximum crosses lanes by swaps, and the accumulators are rescaled only where a maximum has grown by
-// 2^8 or more: with 32 columns some maximum grows in most steps.  4 x 2048 tokens, 32 / 8 heads: 413 us with all that in
-// turn, exchanges through LDS and V^T by byte permutes, 367 so; 2545 tokens in five sequences, 16 / 4 heads 39 and 34;
-// 300 tokens of one 17.8 and 15.5.  Error against 64 bits (900 tokens, unit scores): 2.2e-8 r.m.s. (2.3e-8 before).
+// weights are formed, the maximum crosses lanes by swaps, the accumulators are rescaled only where a maximum has grown by
+// 2^8 or more (with 32 columns some maximum grows in most steps), and staging takes no vector instruction.  4 x 2048 tokens,
+// 32 / 8 heads, in a prompt pass: 413 us with all that in turn, exchanges through LDS and V^T by byte permutes, 367 with rows
+// staged through registers by blocks of eight wavefronts, 303 so; 2545 tokens in five sequences, 16 / 4 heads 39, 34 and 24;
+// 300 tokens of one 17.8, 15.5 and 12.9.  Eight wavefronts per block meet in every step and so want the same unit at the same
+// time: 277 us alone, against 248 in two blocks of four.  Error against 64 bits (900 tokens, unit scores): 2.2e-8 r.m.s. (2.3e-8 before).
 // A step wholly past the causal limit of all the columns of a wavefront is skipped by it.  The
 // result is normalised and written by the block itself (no partial results, no merge pass).
 struct FlashParams {
@@ -937,7 +938,7 @@ struct FlashParams {
     uint32_t nsplit;
     float *part_o, *part_ml;
 };
-constexpr int kFlashNQ = 2, kFlashKeys = 32;
+constexpr int kFlashNW = 4, kFlashNQ = 2, kFlashKeys = 32;
 
 // Weights of eight scores as three bf16 terms that add up to each exactly; returns their sum.
 __device__ __forceinline__ float weights_3(const v4f (&sc)[2], float to_log2, float ref, v8bf (&w)[3]) {
@@ -969,11 +970,15 @@ __device__ __forceinline__ float weights_3(const v4f (&sc)[2], float to_log2, fl
 
 // NQ: column tiles of 16 per wavefront (2: 32 columns; 1: 16 columns, half the multiplies per step and twice the blocks,
 // for prompts that leave most compute units without a block).
-template <int NW, int NQ = kFlashNQ>
-__global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_flash_kernel(FlashParams p) {
-    constexpr int kRows = NW * 4, kPasses = kFlashKeys / kRows;   // staging: rows per pass of the block, passes per step
-    __shared__ __attribute__((aligned(16))) uint16_t k_s[2][kFlashKeys * kVPitch];
-    __shared__ __attribute__((aligned(16))) uint16_t v_s[2][kFlashKeys * kVPitch];
+template <int NQ>
+__global__ void __launch_bounds__(kFlashNW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_flash_kernel(FlashParams p) {
+    constexpr int NW = kFlashNW, kRows = NW * 4, kPasses = kFlashKeys / kRows;   // rows that one load of every wavefront brings, loads per step
+    // Three stages.  A row's 16-byte piece
+    // j sits at j ^ (row % 16): sixteen rows of a piece, and sixteen pieces of a row, are in banks of their own.
+    __shared__ __attribute__((aligned(16))) uint16_t k_s0[kFlashKeys * kDh], k_s1[kFlashKeys * kDh], k_s2[kFlashKeys * kDh];
+    __shared__ __attribute__((aligned(16))) uint16_t v_s0[kFlashKeys * kDh], v_s1[kFlashKeys * kDh], v_s2[kFlashKeys * kDh];
+    auto k_stage = [&](auto i) { return decltype(i)::value == 0 ? k_s0 : decltype(i)::value == 1 ? k_s1 : k_s2; };
+    auto v_stage = [&](auto i) { return decltype(i)::value == 0 ? v_s0 : decltype(i)::value == 1 ? v_s1 : v_s2; };
     __shared__ uint32_t s_bad;
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -1044,55 +1049,49 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
     wmax = __builtin_amdgcn_readfirstlane(wmax);
     wmin = __builtin_amdgcn_readfirstlane(wmin);
 
-    // staging: thread (row r of the step, 16-byte piece c16).  Page ids are requested four steps and K / V
-    // rows three steps ahead of the step that multiplies them, so neither the id -> row dependence nor the
-    // row loads themselves are waited for; steps past the walk repeat its last page (never used).
-    const uint32_t r_st = tid / 16, c16 = tid % 16;           // pass ps stages row r_st + ps * kRows
+    // Staging: rows go from memory to LDS by themselves, K requested three steps ahead, V two (page ids four).  A
+    // wavefront brings four rows of one page at a time: the page is a scalar, a lane's place in it the same in every step.
+    // Steps past the walk repeat its last page (never used).
+    typedef __attribute__((address_space(4))) const uint32_t *ids_t;
+    typedef __attribute__((address_space(3))) void *lptr;
+    const ids_t ids = (ids_t)(uintptr_t)tab;
+    const uint32_t row_in = (uint32_t)wave * 4 % kPage + lane / 16;
+    const uint32_t lane_off = (row_in * p.e_kv + kvh * kDh + ((uint32_t)lane % 16 ^ row_in) * 8) * 2;
+    const uint64_t page_bytes = (uint64_t)kPage * p.e_kv * 2;
     auto load_id = [&](uint32_t it, int ps) -> uint32_t {
-        uint32_t pg = (it * kFlashKeys + ps * kRows + r_st) / kPage;
+        uint32_t pg = (it * kFlashKeys + ps * kRows + wave * 4) / kPage;
         if (pg >= npages) pg = npages - 1;
-        return tab[pg];
+        return ids[pg];
     };
-    auto row_off = [&](uint32_t it, int ps, uint32_t id) -> uint64_t {
-        if (id >= p.num_blocks) id = 0;
-        return ((uint64_t)id * kPage + (it * kFlashKeys + ps * kRows + r_st) % kPage) * p.e_kv + (uint64_t)kvh * kDh + 8 * c16;
-    };
-    v4u k_a[kPasses], v_a[kPasses];                              // K rows of step it + 2, V rows of step it + 1
-    uint32_t id_k[kPasses], id_v[kPasses];                       // page ids of the steps that are requested next: it + 3, it + 2
-    auto put = [&](uint16_t *rows, const v4u (&x)[kPasses]) {
-#pragma unroll
-        for (int ps = 0; ps < kPasses; ++ps) *(v4u *)(&rows[(ps * kRows + r_st) * kVPitch + 8 * c16]) = x[ps];
-    };
-    auto no_rows_past = [&](uint32_t it, v4u (&x)[kPasses]) {     // the pool may hold anything past the sequence end
-#pragma unroll
-        for (int ps = 0; ps < kPasses; ++ps)
-            if (it * kFlashKeys + ps * kRows + r_st >= ctx) x[ps] = v4u{0, 0, 0, 0};
-    };
-#pragma unroll
-    for (int ps = 0; ps < kPasses; ++ps) {
-        k_a[ps] = v_a[ps] = v4u{0, 0, 0, 0};
-        id_k[ps] = id_v[ps] = 0;
-    }
-    if (n_it > it_lo) {
-        v4u k0[kPasses], k1[kPasses], v0[kPasses];
+    uint32_t id_k[kPasses], id_v[kPasses];                       // of the steps that are requested next
+    // (written out: the compiler waits for every load on the way before it reads a stage that was requested in the same trip
+    // of the loop; here arrive() is the wait)
+    auto request = [&](const uint16_t *pool, const uint32_t (&id)[kPasses], uint16_t *rows) {
 #pragma unroll
         for (int ps = 0; ps < kPasses; ++ps) {
-            const uint32_t id0 = load_id(it_lo, ps), id1 = load_id(it_lo + 1, ps);
-            id_v[ps] = load_id(it_lo + 2, ps);
-            id_k[ps] = load_id(it_lo + 3, ps);
-            const uint64_t off0 = row_off(it_lo, ps, id0), off1 = row_off(it_lo + 1, ps, id1);
-            k0[ps] = *(const v4u *)(p.k_pool + off0);
-            v0[ps] = *(const v4u *)(p.v_pool + off0);
-            k1[ps] = *(const v4u *)(p.k_pool + off1);
-            v_a[ps] = *(const v4u *)(p.v_pool + off1);
-            k_a[ps] = *(const v4u *)(p.k_pool + row_off(it_lo + 2, ps, id_v[ps]));
+            const uint64_t page = (uint64_t)(uintptr_t)pool + (id[ps] < p.num_blocks ? id[ps] : 0) * page_bytes;
+            const uint32_t to = (uint32_t)(uintptr_t)(lptr)(rows + (ps * kRows + wave * 4) * kDh);
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(page), "s"(to) : "memory");
         }
-        no_rows_past(it_lo, v0);
-        put(k_s[0], k0);
-        put(k_s[1], k1);
-        put(v_s[0], v0);
+    };
+    // all but the last N requests of every wavefront are there
+    auto arrive = [&](auto n) { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(decltype(n)::value * kPasses) : "memory"); };
+    if (n_it > it_lo) {
+        auto ids_of = [&](uint32_t it, uint32_t (&id)[kPasses]) {
+#pragma unroll
+            for (int ps = 0; ps < kPasses; ++ps) id[ps] = load_id(it, ps);
+        };
+        ids_of(it_lo, id_k);
+        ids_of(it_lo + 1, id_v);
+        request(p.k_pool, id_k, k_s0);
+        request(p.k_pool, id_v, k_s1);
+        request(p.v_pool, id_k, v_s0);
+        request(p.v_pool, id_v, v_s1);
+        ids_of(it_lo + 2, id_v);
+        request(p.k_pool, id_v, k_s2);
+        ids_of(it_lo + 3, id_k);
+        arrive(std::integral_constant<int, 2>{});                // K of two steps, V of one
     }
-    __syncthreads();
 
     // m_run, the columns' reference in powers of two, follows the running maximum when that has grown by more than 2^kSlack:
     // a weight may be that much above one, and the accumulators are rescaled in the first steps only
@@ -1107,33 +1106,49 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
         for (int t = 0; t < 8; ++t) o[qi][t] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    auto scores = [&](int st, v4f (&x)[NQ][2]) {      // of a step: two tiles of 16 positions
+    const uint32_t v_row = 4 * g + c / 4, v_piece = (c % 4 / 2) ^ v_row;
+    auto transposed = [&](const uint16_t *vs, int t) {            // transposed_keys on the staged order of pieces
+        typedef __attribute__((address_space(3))) v4s *sptr;
+        const uint16_t *x = vs + v_row * kDh + (v_piece ^ (2 * t)) * 8 + c % 2 * 4;
+        const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((sptr)x), hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((sptr)(x + 16 * kDh));
+        return __builtin_bit_cast(v8bf, v8s{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]});
+    };
+    auto scores = [&](const uint16_t *ks, v4f (&x)[NQ][2]) {      // of a step: two tiles of 16 positions
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) {
 #pragma unroll
             for (int qi = 0; qi < NQ; ++qi) x[qi][kt] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const v8bf ka = *(const v8bf *)(&k_s[st][(kt * 16 + c) * kVPitch + 32 * s + 8 * g]);
+                const v8bf ka = *(const v8bf *)(ks + (kt * 16 + c) * kDh + ((4 * s + g) ^ c) * 8);
 #pragma unroll
                 for (int qi = 0; qi < NQ; ++qi) x[qi][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qb[qi][s], x[qi][kt], 0, 0, 0);
             }
         }
     };
-    if (it_lo < n_it) scores(0, sc);
-    __syncthreads();                                  // the first K stage is written again in the first step
+    if (it_lo < n_it) {
+        scores(k_s0, sc);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");     // the first step requests into that stage
+    }
 
-    for (uint32_t it = it_lo; it < n_it; ++it) {
-        const int st = (it - it_lo) & 1;
-        v4u k_n[kPasses], v_n[kPasses];
+    auto step = [&](uint32_t it, auto i0) {
+        constexpr int S = decltype(i0)::value;
+        using int_1 = std::integral_constant<int, (S + 1) % 3>;
+        using int_2 = std::integral_constant<int, (S + 2) % 3>;
+        uint16_t *vs = v_stage(i0);
+        request(p.k_pool, id_k, k_stage(i0));                     // of step it + 3; the stages were last read in step it - 1
+        request(p.v_pool, id_v, v_stage(int_2{}));                // of step it + 2
 #pragma unroll
         for (int ps = 0; ps < kPasses; ++ps) {
-            k_n[ps] = *(const v4u *)(p.k_pool + row_off(it + 3, ps, id_k[ps]));
-            v_n[ps] = *(const v4u *)(p.v_pool + row_off(it + 2, ps, id_v[ps]));
             id_v[ps] = id_k[ps];
             id_k[ps] = load_id(it + 4, ps);
         }
         const uint32_t key0 = it * kFlashKeys;
+        if (key0 + kFlashKeys > ctx) {                            // the pool may hold anything past the sequence end
+            for (uint32_t e = tid * 8; e < kFlashKeys * kDh; e += NW * 64 * 8)
+                if (key0 + e / kDh >= ctx) *(v4u *)(vs + e) = v4u{0, 0, 0, 0};
+            __syncthreads();
+        }
         if (key0 < wmax) {
             if (key0 + kFlashKeys > wmin) {
 #pragma unroll
@@ -1170,10 +1185,10 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
             }
             // the next step's scores are multiplied while this one's weights are formed
             v4f sn[NQ][2];
-            scores(st ^ 1, sn);
+            scores(k_stage(int_1{}), sn);
             v8bf vt[8];
 #pragma unroll
-            for (int t = 0; t < 8; ++t) vt[t] = transposed_keys(v_s[st] + 16 * t, kVPitch, lane);
+            for (int t = 0; t < 8; ++t) vt[t] = transposed(vs, t);
 #pragma unroll
             for (int qi = 0; qi < NQ; ++qi) {
                 // every score of a column can be masked so far: its reference is -inf and the exponentials are taken against 0
@@ -1190,17 +1205,14 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
                 for (int kt = 0; kt < 2; ++kt) sc[qi][kt] = sn[qi][kt];
         }
-        // K two steps and V one step ahead go to stages whose readers passed the barrier of the last step
-        no_rows_past(it + 1, v_a);
-        put(k_s[st], k_a);
-        put(v_s[st ^ 1], v_a);
-#pragma unroll
-        for (int ps = 0; ps < kPasses; ++ps) {
-            k_a[ps] = k_n[ps];
-            v_a[ps] = v_n[ps];
-        }
-        __syncthreads();
+        arrive(std::integral_constant<int, 2>{});
+    };
+    for (uint32_t it = it_lo; it < n_it; it += 3) {
+        step(it, std::integral_constant<int, 0>{});
+        if (it + 1 < n_it) step(it + 1, std::integral_constant<int, 1>{});
+        if (it + 2 < n_it) step(it + 2, std::integral_constant<int, 2>{});
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");              // requests past the walk still write the block's LDS
 
     // lane (g, c) holds, for column c, dims 16 t + 4 g + {0..3}
 #pragma unroll
@@ -1241,9 +1253,8 @@ __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2,
 // Adds the shares of a split walk: one block per (tile block, eight columns), thread (column, dim).  The shares
 // of a column are read eight at a time, all loads of a batch before the first use (a chain of L2 round trips
 // otherwise); slots past the last share repeat it with weight zero.
-template <int NW>
 __global__ void __launch_bounds__(1024) flash_split_merge_kernel(FlashParams p) {
-    constexpr uint32_t kCols = NW * kFlashNQ * 16;
+    constexpr uint32_t kCols = kFlashNW * kFlashNQ * 16;
     const uint32_t per_tile = p.batch * p.num_kv_heads;
     const uint32_t tile = p.tiles - 1 - blockIdx.x / per_tile;
     const uint32_t b = (blockIdx.x % per_tile) / p.num_kv_heads, kvh = blockIdx.x % p.num_kv_heads;
@@ -1330,7 +1341,6 @@ void paged_attention_generic(const void *q, const void *k_pool, const void *v_po
 }  // namespace k
 int g_decode_partials_only = 0;   // profiling: launch only the streaming kernel (the output is not written)
 int g_prefill_block_form = 0;     // 0: by shape, 1: never, 2: whenever the group size allows
-int g_prefill_block_waves = 0;    // wavefronts per block of the block form: 4 or 8, anything else by shape
 int g_prefill_block_split = 0;    // upper bound of the blocks that share one tile's walk (0: by shape)
 int g_prefill_block_cols = 0;     // columns per wavefront of the block form: 0 by shape, 1: 16 whenever allowed, 2: always 32
 namespace k {
@@ -1475,7 +1485,7 @@ static uint32_t prefill_seqs_per_row(const PagedShape &ps) {           // virtua
 
 // shares of a split walk that one launch may leave in the workspace (four-wavefront blocks, 128 columns each)
 static uint64_t flash_split_slots() { return 2ull * compute_units(); }
-constexpr uint64_t kFlashSplitCols = 4 * kFlashNQ * 16;
+constexpr uint64_t kFlashSplitCols = kFlashNW * kFlashNQ * 16;
 
 uint64_t paged_prefill_workspace_bytes(const PagedShape &ps, uint32_t waves_per_cu) {
     uint64_t items = ((uint64_t)stream_ranges(ps, waves_per_cu) + (uint64_t)ps.batch * prefill_seqs_per_row(ps)) *
@@ -1492,46 +1502,38 @@ uint64_t paged_prefill_workspace_bytes(const PagedShape &ps, uint32_t waves_per_
 // (32 / 8 heads): they only need to be right where the two forms are far apart, which is where it matters.
 struct BlockFormPlan {
     bool use;
-    int waves;
     uint32_t nsplit;                    // blocks sharing a tile's walk (1: none)
 };
 static BlockFormPlan plan_block_form(const PagedShape &ps) {
     const uint32_t group = ps.num_heads / ps.num_kv_heads;
-    if (group == 0 || group > 16 || g_prefill_block_form == 1) return {false, 0, 1};
+    if (group == 0 || group > 16 || g_prefill_block_form == 1) return {false, 1};
     const uint32_t cus = compute_units();
     const uint32_t bound = ps.max_blocks_per_seq * kPage;
     uint32_t ctx = ps.ctx_hint != 0 && ps.ctx_hint < bound ? ps.ctx_hint : bound;
     if (ctx < ps.l_new) ctx = ps.l_new;
     const double cached = (double)(ctx - ps.l_new), l_new = (double)ps.l_new;
     const uint64_t rows = (uint64_t)ps.batch * ps.num_kv_heads;
-    int waves = g_prefill_block_waves == 8 ? 8 : g_prefill_block_waves == 4 ? 4 : 0;
-    if (waves == 0) {
-        // eight wavefronts halve the K / V traffic of a block pair; they pay once the device is oversubscribed
-        const uint32_t tq8 = 256 / group;
-        waves = rows * ((ps.l_new + tq8 - 1) / tq8) >= 2ull * cus && ps.l_new >= 1024 ? 8 : 4;
-    }
-    const uint32_t tq = (uint32_t)waves * kFlashNQ * 16 / group, tiles = (ps.l_new + tq - 1) / tq;
+    const uint32_t tq = kFlashNW * kFlashNQ * 16 / group, tiles = (ps.l_new + tq - 1) / tq;
     const double steps_longest = (cached + l_new) / kFlashKeys;
     // few blocks against a long walk over what was cached before (the walks of all tiles are then about equally
     // long): several blocks share a tile's walk (at least eight steps each, at most as many shares as the
     // workspace holds) and a merge pass adds them
     uint32_t nsplit = 1;
     const uint64_t blocks = rows * tiles;
-    if (waves == 4 && blocks < cus && cached >= 2.0 * l_new) {
+    if (blocks < cus && cached >= 2.0 * l_new) {
         uint64_t want = flash_split_slots() / blocks, by_steps = (uint64_t)(steps_longest / 8.0);
         if (g_prefill_block_split > 0) want = (uint64_t)g_prefill_block_split < want ? (uint64_t)g_prefill_block_split : want;
         nsplit = (uint32_t)(want < by_steps ? want : by_steps);
         if (nsplit < 1) nsplit = 1;
     }
-    if (g_prefill_block_form == 2) return {true, waves, nsplit};
+    if (g_prefill_block_form == 2) return {true, nsplit};
     const double steps_all = (double)blocks * (cached + (tiles > 1 ? 0.5 * l_new : l_new)) / kFlashKeys;
-    const double per_cu = waves == 8 ? 2.05 : 1.05;                       // us per step at two wavefronts per SIMD
-    const double a = steps_longest / nsplit * 1.4 + (nsplit > 1 ? 9.0 : 0.0), b = steps_all / cus * per_cu;
+    const double a = steps_longest / nsplit * 1.4 + (nsplit > 1 ? 9.0 : 0.0), b = steps_all / cus * 1.05;       // us per step at two wavefronts per SIMD
     const double t_block = (a > b ? a : b) + 8.0;
     const uint32_t tpt = 16 / group, tpv = ps.l_new > tpt ? 2 * tpt : tpt;
     const double bytes = (double)rows * ((ps.l_new + tpv - 1) / tpv) * (cached + 0.5 * l_new) * (2.0 * kDh * 2);
     const double t_stream = 35.0 + bytes / 4.9e6 + 0.035 * l_new * ps.batch;
-    return {t_block <= t_stream, waves, nsplit};
+    return {t_block <= t_stream, nsplit};
 }
 
 void paged_attention_prefill_bf16(const uint16_t *q, const uint16_t *k_pool, const uint16_t *v_pool,
@@ -1556,32 +1558,30 @@ void paged_attention_prefill_bf16(const uint16_t *q, const uint16_t *k_pool, con
         fp.group = ps.num_heads / ps.num_kv_heads;
         fp.max_blocks_per_seq = ps.max_blocks_per_seq;
         fp.l_new = ps.l_new;
-        fp.tq = (uint32_t)plan.waves * kFlashNQ * 16 / fp.group;
+        fp.tq = kFlashNW * kFlashNQ * 16 / fp.group;
         fp.tiles = (ps.l_new + fp.tq - 1) / fp.tq;
         fp.scale = ps.scale;
         // A short prompt leaves compute units without a block, and a block's time is its walk: with 16 columns per
-        // wavefront instead of 32 a step costs half the multiplies and there are twice the blocks (a 300-token prompt:
-        // 80 -> 152 blocks; measured through 32 layers: 300 tokens 6.80 -> 6.59 ms, 1024 tokens 16.24 -> 15.72 ms).  Only
-        // the unsplit four-wavefront form, and only while the wide blocks would not fill the device more than once.
-        const bool narrow = g_prefill_block_cols != 2 && plan.waves == 4 && plan.nsplit == 1 && fp.group <= 16 && 16 % fp.group == 0 &&
+        // wavefront instead of 32 a step costs half the multiplies and there are twice the blocks.  The line is two wide blocks
+        // per compute unit, what is resident: 32 / 8 heads, 300 tokens (80 blocks) 19 and 13 us, 4 x 512 and 2048 (512) 35.4 and
+        // 34.5, 92 and 84, 3000 (752) 157 and 156, 8 x 512 (1024) 56 and 61.  Only the unsplit form.
+        const bool narrow = g_prefill_block_cols != 2 && plan.nsplit == 1 && fp.group <= 16 && 16 % fp.group == 0 &&
                             (g_prefill_block_cols == 1 ||
-                             (uint64_t)ps.batch * ps.num_kv_heads * fp.tiles <= (uint64_t)compute_units());
+                             (uint64_t)ps.batch * ps.num_kv_heads * fp.tiles <= 2 * (uint64_t)compute_units());
         if (narrow) {
-            fp.tq = (uint32_t)plan.waves * 16 / fp.group;
+            fp.tq = kFlashNW * 16 / fp.group;
             fp.tiles = (ps.l_new + fp.tq - 1) / fp.tq;
         }
         const uint64_t blocks = (uint64_t)ps.batch * ps.num_kv_heads * fp.tiles;
         fp.nsplit = plan.nsplit;
         fp.part_o = (float *)workspace;
         fp.part_ml = fp.part_o + blocks * fp.nsplit * kFlashSplitCols * kDh;
-        if (plan.waves == 8) {
-            prefill_flash_kernel<8><<<(unsigned)blocks, 512, 0, s>>>(fp);
-        } else if (narrow) {
-            prefill_flash_kernel<4, 1><<<(unsigned)blocks, 256, 0, s>>>(fp);
+        if (narrow) {
+            prefill_flash_kernel<1><<<(unsigned)blocks, kFlashNW * 64, 0, s>>>(fp);
         } else {
-            prefill_flash_kernel<4><<<dim3((unsigned)blocks, fp.nsplit), 256, 0, s>>>(fp);
+            prefill_flash_kernel<kFlashNQ><<<dim3((unsigned)blocks, fp.nsplit), kFlashNW * 64, 0, s>>>(fp);
             if (fp.nsplit > 1)
-                flash_split_merge_kernel<4><<<dim3((unsigned)blocks, (unsigned)((fp.tq * fp.group + 7) / 8)), 1024, 0, s>>>(fp);
+                flash_split_merge_kernel<<<dim3((unsigned)blocks, (unsigned)((fp.tq * fp.group + 7) / 8)), 1024, 0, s>>>(fp);
         }
         return;
     }

@@ -61,14 +61,14 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  * key 5: activation-stationary decode linears: 1 never, 2 whenever the shape allows, 3 by shape but 33 to 64 rows stay
  *        on the block-per-tile kernels;
  * key 6: wavefronts per block of the large-tile prefill GEMMs (4 or 16; default 8);
- * key 7: column tiles of 16 per block of the large-tile prefill GEMMs (14 or 16);
+ * key 7: column tiles of 16 per block of the large-tile prefill GEMMs (8, 14 or 16);
  * key 8: nonzero sends attention with more than one new token per row to the generic
  *        kernel (the reference's summation order) instead of the streamed one;
  * key 9: blocks per compute unit that a split-k launch of the 128 x 128 int8 GEMM aims
  *        for (default 2);
  * key 10: form of the attention with more than one new token per row: 1 always the
  *        streamed form, 2 always the block form, 0 by shape;
- * key 11: wavefronts per block of that block form (4 or 8; 0 by shape);
+ * key 11: without effect;
  * key 12: upper bound of the blocks that share the cache walk of one tile of new tokens
  *        in the block form (1: never split; 0 by shape);
  * key 13: kernel of the order-fixed f32 GEMM (gemm_device / linear_forward_device): 1 the few-rows vector
@@ -116,12 +116,14 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  * key 29: bf16 linears: 2: never the large-tile kernel, 3: never four column tiles per block; experts' linears: 4: weights
  *        streamed past the rows, 5: 128 x 128 tiles, 6: large tiles, whatever the number of rows;
  * key 30: latent attention: 1: the plain kernel, 2: the absorbed form for every pass, 3: the expanded form wherever it
- *        can run; key 31: gated delta rule: 1: token by token for prompts too;
+ *        can run; key 31: gated delta rule: 1: token by token for prompts too, 2: a state's rows always
+ *        over a block's wavefronts, 3: never;
  * key 32: blocks per compute unit the key split of the absorbed form aims at;
  * key 33: grouped-query attention: 1: the plain kernel, 2: the few-rows kernel for every sequence, 3: the many-rows kernel
  *        for every sequence; key 34: blocks per compute unit its key split aims at;
  * key 35: routing of experts: 1: always in the residual update's launch, 2: always in a launch of its own.
- * key 36: minimal gated recurrence: threads across the channels of a block of the scan, 8 or 16. */
+ * key 36: minimal gated recurrence: threads across the channels of a block of the scan, 8 or 16;
+ * key 37: row tiles of 16 per block of the large-tile prefill GEMMs (8, 12 or 16; with key 7). */
 fa_status fa_set_tuning(int32_t key, int32_t value);
 
 /* What the context found when it was created: xcd_local = 1 when workgroups b and b + 8 of a launch were seen to
