@@ -159,7 +159,7 @@ class DeviceBuffer:
         self._ops, self._h, self.shape, self.dtype = ops, handle, tuple(int(s) for s in shape), dtype
 
     def numel(self):
-        return int(np.prod(self.shape, dtype=np.uint64)) if self.shape else 1
+        return math.prod(self.shape)
 
     def device(self):
         return self._ops.device()
@@ -304,14 +304,12 @@ class RocmBackendOps:
 
     def alloc_zeroed(self, shape, dtype=capi.F32):
         h = capi.buf_p()
-        check(lib.fa_alloc_zeroed(self._ctx, dtype, int(np.prod(shape, dtype=np.uint64)) if len(shape) else 1,
-                                  C.byref(h)))
+        check(lib.fa_alloc_zeroed(self._ctx, dtype, math.prod(map(int, shape)), C.byref(h)))
         return self._wrap(h, shape, dtype)
 
     def alloc_uninit(self, shape, dtype=capi.F32):
         h = capi.buf_p()
-        check(lib.fa_alloc_uninit(self._ctx, dtype, int(np.prod(shape, dtype=np.uint64)) if len(shape) else 1,
-                                  C.byref(h)))
+        check(lib.fa_alloc_uninit(self._ctx, dtype, math.prod(map(int, shape)), C.byref(h)))
         return self._wrap(h, shape, dtype)
 
     def upload(self, tensor, dtype=None):

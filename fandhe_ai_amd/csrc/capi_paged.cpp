@@ -169,9 +169,7 @@ fa_status fa_paged_kv_append(fa_context *ctx, const fa_buffer *k_new, const fa_b
     if (rows == 0) return FA_OK;
     if (ctx->capturing) return fail(FA_ERR_CAPTURE_IN_PROGRESS, "paged_kv_append with host tables during graph capture");
     if (fa_status s = ensure_table_stage(ctx, rows * 4)) return s;
-    hipError_t e = hipMemcpyAsync(ctx->table_stage, slot_mapping, rows * 4, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);      // the host array is consumed on return
-    if (e != hipSuccess) return hip_fail(ctx, e, "slot_mapping upload", FA_ERR_TRANSFER_FAILED);
+    if (fa_status s = queue_upload(ctx, ctx->table_stage, slot_mapping, rows * 4, "slot_mapping upload")) return s;
     k::paged_kv_append(k_new->ptr, v_new->ptr, k_pool->ptr, v_pool->ptr, (const uint32_t *)ctx->table_stage, rows,
                        layout->embed_dim, layout->num_blocks * layout->block_size, (int)dtype_size(k_new->dtype),
                        ctx->stream);
@@ -222,11 +220,8 @@ fa_status fa_paged_attention_forward(fa_context *ctx, const fa_buffer *q, const 
     uint64_t tb = n_tables * 4, lb = n_seq * 4;
     uint64_t lens_off = (tb + 255) / 256 * 256;
     if (fa_status s = ensure_table_stage(ctx, lens_off + lb)) return s;
-    hipError_t e = hipMemcpyAsync(ctx->table_stage, block_tables, tb, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync((char *)ctx->table_stage + lens_off, seq_lens, lb, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) return hip_fail(ctx, e, "block table upload", FA_ERR_TRANSFER_FAILED);
+    if (fa_status s = queue_upload(ctx, ctx->table_stage, block_tables, tb, "block table upload")) return s;
+    if (fa_status s = queue_upload(ctx, (char *)ctx->table_stage + lens_off, seq_lens, lb, "sequence lengths upload")) return s;
     uint32_t longest = 0;
     for (uint64_t i = 0; i < n_seq; ++i) longest = seq_lens[i] > longest ? seq_lens[i] : longest;
     return launch_attention(ctx, q, k_pool, v_pool, (const uint32_t *)ctx->table_stage,

@@ -695,8 +695,8 @@ fa_status fa_decoder_set_sequences(fa_context *ctx, fa_decoder *d, uint32_t batc
                 return fail(FA_ERR_INVALID_ARGUMENT, "paged_kv: row " + std::to_string(b) + " entry " +
                                                          std::to_string(i) + " is not a valid block id");
     }
-    if (fa_status s = fa_upload_into(ctx, block_tables, (uint64_t)batch * c.max_blocks_per_seq, d->tables, 0)) return s;
-    if (fa_status s = fa_upload_into(ctx, seq_lens, batch, d->seq_lens, 0)) return s;
+    if (fa_status s = queue_upload(ctx, d->tables->ptr, block_tables, (uint64_t)batch * c.max_blocks_per_seq * 4, "decoder_set_sequences")) return s;
+    if (fa_status s = queue_upload(ctx, d->seq_lens->ptr, seq_lens, (uint64_t)batch * 4, "decoder_set_sequences")) return s;
     d->batch = batch;
     try {
         d->host_tables.assign(block_tables, block_tables + (uint64_t)batch * c.max_blocks_per_seq);
@@ -717,7 +717,7 @@ fa_status fa_decoder_set_tokens(fa_context *ctx, fa_decoder *d, const int32_t *t
     for (uint32_t b = 0; b < d->batch; ++b)
         if (tokens[b] < 0 || (uint32_t)tokens[b] >= d->cfg.vocab)
             return fail(FA_ERR_INVALID_ARGUMENT, "decoder_set_tokens: token id outside the vocabulary");
-    return fa_upload_into(ctx, tokens, d->batch, d->tokens, 0);
+    return queue_upload(ctx, d->tokens->ptr, tokens, (uint64_t)d->batch * 4, "decoder_set_tokens");
 }
 
 // The position every row writes in a decode step must have a page (validate_paged_kv_append rejects a row
@@ -930,15 +930,9 @@ static fa_status prefill_impl(fa_context *ctx, fa_decoder *d, const int32_t *tok
         const uint32_t lc = std::min(lc_max, l_new - t0);
         for (uint32_t b = 0; b < B; ++b)
             for (uint32_t i = 0; i < lc; ++i) stage[(uint64_t)b * lc + i] = tokens[(uint64_t)b * l_new + t0 + i];
-        // the staging vector is reused by the next chunk: the copy must have consumed it before this call goes on
-        hipError_t e = hipMemcpyAsync(t.tok.ptr, stage.data(), (uint64_t)B * lc * 4, hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        if (e != hipSuccess) return hip_fail(ctx, e, "prompt token upload", FA_ERR_TRANSFER_FAILED);
-        if (padded) {
-            e = hipMemcpyAsync(t.row_lens.ptr, row_lens, (uint64_t)B * 4, hipMemcpyHostToDevice, ctx->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-            if (e != hipSuccess) return hip_fail(ctx, e, "prompt lengths upload", FA_ERR_TRANSFER_FAILED);
-        }
+        if (fa_status s = queue_upload(ctx, t.tok.ptr, stage.data(), (uint64_t)B * lc * 4, "prompt token upload")) return s;
+        if (padded)
+            if (fa_status s = queue_upload(ctx, t.row_lens.ptr, row_lens, (uint64_t)B * 4, "prompt lengths upload")) return s;
         if (fa_status s = enqueue_prefill_chunk(ctx, d, t, lc, t0 + lc == l_new, verify, padded)) return s;
         for (uint32_t b = 0; b < B; ++b) d->host_lens[b] += padded ? row_lens[b] : lc;
     }
@@ -983,7 +977,7 @@ fa_status fa_decoder_rewind(fa_context *ctx, fa_decoder *d, const uint32_t *seq_
         for (uint32_t b = 0; b < d->batch; ++b)
             if (seq_lens[b] != d->host_lens[b])
                 return fail(FA_ERR_UNSUPPORTED, "decoder_rewind: a recurrent state cannot be cut back");
-    if (fa_status s = fa_upload_into(ctx, seq_lens, d->batch, d->seq_lens, 0)) return s;
+    if (fa_status s = queue_upload(ctx, d->seq_lens->ptr, seq_lens, (uint64_t)d->batch * 4, "decoder_rewind")) return s;
     std::copy(seq_lens, seq_lens + d->batch, d->host_lens.begin());
     return FA_OK;
 }

@@ -117,6 +117,11 @@ __global__ void fill_u32_kernel(uint32_t *p, uint32_t v, uint64_t n) {
     for (; i < n; i += stride) p[i] = v;
 }
 
+__global__ void copy_words_kernel(const uint32_t *from, uint32_t *to, uint64_t n) {
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) to[i] = __builtin_nontemporal_load(from + i);
+}
+
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
     x += 0x9E3779B97F4A7C15ull;
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -209,6 +214,10 @@ void convert_bf16_to_f32(const uint16_t *in, float *out, uint64_t n, hipStream_t
 void fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s) {
     if (n == 0) return;
     fill_u32_kernel<<<grid_for(n, 256), 256, 0, s>>>(p, v, n);
+}
+void copy_words(const uint32_t *from, uint32_t *to, uint64_t n, hipStream_t s) {
+    if (n == 0) return;
+    copy_words_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(from, to, n);
 }
 void fill_normal(void *out, int out_bf16, uint64_t n, uint64_t seed, float mean, float std, hipStream_t s) {
     if (n == 0) return;

@@ -677,11 +677,7 @@ ExpandPlan plan_expand(const LayeredState &L, const std::vector<uint32_t> &lens,
 
 uint64_t pass_rows() { return g_layered_rows >= 64 ? (uint64_t)g_layered_rows : 8192; }
 
-fa_status upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes) {
-    hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    return e == hipSuccess ? FA_OK : hip_fail(ctx, e, "upload of a pass", FA_ERR_TRANSFER_FAILED);
-}
+fa_status upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes) { return queue_upload(ctx, dst, src, bytes, "upload of a pass"); }
 
 }  // namespace
 
@@ -709,7 +705,7 @@ fa_status layered_sequences_set(fa_context *ctx, fa_decoder *d) {
     if (!L.slots_set) return FA_OK;
     std::vector<uint32_t> iota(d->batch);
     for (uint32_t b = 0; b < d->batch; ++b) iota[b] = b;
-    return fa_upload_into(ctx, iota.data(), d->batch, L.state_slots, 0);
+    return queue_upload(ctx, L.state_slots->ptr, iota.data(), (uint64_t)d->batch * 4, "decoder_set_sequences");
 }
 
 fa_status layered_prepare_step(fa_context *ctx, fa_decoder *d) {
@@ -1461,7 +1457,7 @@ fa_status fa_decoder_set_state_slots(fa_context *ctx, fa_decoder *d, const uint3
         for (uint32_t o = 0; o < b; ++o)
             if (slots[o] == slots[b]) return fail(FA_ERR_INVALID_ARGUMENT, "decoder_set_state_slots: two rows share a slot");
     }
-    if (fa_status s = fa_upload_into(ctx, slots, d->batch, d->layered->state_slots, 0)) return s;
+    if (fa_status s = queue_upload(ctx, d->layered->state_slots->ptr, slots, (uint64_t)d->batch * 4, "decoder_set_state_slots")) return s;
     d->layered->slots_set = true;
     return FA_OK;
 }

@@ -162,6 +162,58 @@ fa_status after_launch(fa_context *ctx, const char *kernel) {
     return FA_OK;
 }
 
+// --------------------------------------------------------------- uploads
+// A wait per upload costs a decode step about 20 us of an idle device (its lengths and tokens).  A copy out of pinned
+// memory by a kernel of our own takes 3 us of the stream and nothing else; only one that is too large for the ring waits.
+static bool ring_ready(fa_context *ctx) {
+    fa_upload_ring &r = ctx->ring;
+    if (r.host || r.off) return r.host != nullptr;
+    void *h = nullptr, *d = nullptr;
+    bool ok = hipHostMalloc(&h, 2 * r.kHalf, hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess;
+    ok = ok && hipHostGetDevicePointer(&d, h, 0) == hipSuccess;
+    for (hipEvent_t &e : r.queued) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        for (hipEvent_t &e : r.queued) {
+            if (e) (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+        if (h) (void)hipHostFree(h);
+        r.off = true;
+        return false;
+    }
+    r.host = (char *)h;
+    r.device = (char *)d;
+    return true;
+}
+
+fa_status queue_upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes, const char *what) {
+    if (bytes == 0) return FA_OK;
+    if (ctx->capturing) return fail(FA_ERR_CAPTURE_IN_PROGRESS, std::string(what) + " is not allowed during graph capture");
+    fa_upload_ring &r = ctx->ring;
+    std::lock_guard<std::mutex> g(r.mu);
+    if (bytes > r.kHalf || bytes % 4 != 0 || (uintptr_t)dst % 4 != 0 || !ring_ready(ctx)) {
+        hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
+        return e == hipSuccess ? FA_OK : hip_fail(ctx, e, what, FA_ERR_TRANSFER_FAILED);
+    }
+    if (r.used + bytes > r.kHalf) {
+        hipError_t e = hipEventRecord(r.queued[r.half], ctx->stream);
+        if (e != hipSuccess) return hip_fail(ctx, e, what, FA_ERR_TRANSFER_FAILED);
+        r.busy[r.half] = true;
+        r.half ^= 1;
+        if (r.busy[r.half]) e = hipEventSynchronize(r.queued[r.half]);
+        if (e != hipSuccess) return hip_fail(ctx, e, what, FA_ERR_TRANSFER_FAILED);
+        r.busy[r.half] = false;
+        r.used = 0;
+    }
+    const uint64_t at = r.half * r.kHalf + r.used;
+    std::memcpy(r.host + at, src, bytes);
+    r.used += (bytes + 63) / 64 * 64;
+    k::copy_words((const uint32_t *)(r.device + at), (uint32_t *)dst, bytes / 4, ctx->stream);
+    return after_launch(ctx, what);
+}
+
 // ------------------------------------------------------------- allocation
 fa_status pool_alloc(fa_context *ctx, uint64_t bytes, void **ptr, uint64_t *class_bytes) {
     uint64_t cls;
@@ -487,6 +539,9 @@ fa_status fa_context_destroy(fa_context *ctx) {
     if (ctx->workspace) (void)hipFree(ctx->workspace);
     if (ctx->splitk.partial) (void)hipFree(ctx->splitk.partial);
     if (ctx->splitk.fault) (void)hipHostFree(ctx->splitk.fault);
+    for (hipEvent_t e : ctx->ring.queued)
+        if (e) (void)hipEventDestroy(e);
+    if (ctx->ring.host) (void)hipHostFree(ctx->ring.host);
     for (void *w : ctx->retired_workspaces) (void)hipFree(w);
     for (auto &b : ctx->capture_owned) (void)hipFree(b.ptr);   // a capture that was never ended
     for (void *p : ctx->deferred_frees) (void)hipFree(p);

@@ -66,6 +66,19 @@ struct fa_owned_block {
     uint64_t bytes, cls;
 };
 
+// Pinned memory through which small tables and tokens go to the device without a wait: two halves, each taken from front to
+// back; before a half is used again the copies that were queued out of it are waited for.
+struct fa_upload_ring {
+    static constexpr uint64_t kHalf = 128 * 1024;
+    std::mutex mu;
+    char *host = nullptr, *device = nullptr;
+    hipEvent_t queued[2] = {nullptr, nullptr};
+    bool busy[2] = {false, false};
+    int half = 0;
+    uint64_t used = 0;
+    bool off = false;                                // no pinned memory to be had: every upload waits
+};
+
 struct fa_context {
     uint32_t magic;
     int device;
@@ -98,6 +111,7 @@ struct fa_context {
     // graphs recorded on this context that are still alive; a context is not destroyed while one of them holds
     // device blocks of its pool
     uint64_t live_graphs = 0;
+    fa_upload_ring ring;
 };
 
 struct fa_buffer {
@@ -148,6 +162,9 @@ fa_status check_buf_typed(const fa_context *ctx, const fa_buffer *b, fa_dtype t,
 fa_status hip_fail(fa_context *ctx, hipError_t e, const char *what, fa_status as);
 // Checks hipGetLastError after a launch.
 fa_status after_launch(fa_context *ctx, const char *kernel);
+// Host memory to memory that only work queued on the context's stream reads: the source is consumed on return, the copy is
+// queued.  (Buffers that a caller may read elsewhere are filled by fa_upload and fa_upload_into, which wait for the copy.)
+fa_status queue_upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes, const char *what);
 
 // Pool-backed raw allocation used by buffers and by internal scratch.
 fa_status pool_alloc(fa_context *ctx, uint64_t bytes, void **ptr, uint64_t *class_bytes);

@@ -170,3 +170,28 @@ def test_prefill_block_form_scales_and_growing_maxima(l_new, lens, split, cols, 
     # longest keys; values of unit size are weighed
     tol = max(2e-5, 2 * 128 * 2.0 ** -24 * 1300 * abs(scale))
     assert np.abs(got - want).max() < tol, np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("max_blocks", [7, 600, 1500], ids=["small tables", "two calls to a half", "larger than a half"])
+def test_tables_queued_one_call_behind_the_other(max_blocks):
+    """Calls whose tables differ, with nothing waited for between them and the host's arrays overwritten behind each: every call
+    reads the tables that it was given, also where the pinned memory they pass through is used over and over."""
+    import test_gpu_paged as paged
+    o, fa, be = paged.o, paged._fa(), paged.ops()
+    batch, heads, kv_heads, num_blocks, dh = 27, 4, 2, 64, 128
+    rng = o.Rng(max_blocks)
+    pool = lambda: be.upload(o.to_bf16(rng.randn((num_blocks, 16, kv_heads * dh))))
+    kp, vp, q = pool(), pool(), be.upload(o.to_bf16(rng.randn((batch, 1, heads * dh))))
+    args = fa.PagedAttentionArgs(fa.PagedKvLayout.new(num_blocks, 16, kv_heads * dh), batch, 1, heads, max_blocks, fa.default_scale(dh), kv_heads)
+    perm = np.random.default_rng(max_blocks)
+    cases, got = [], []
+    tables, lens = np.empty((batch, max_blocks), np.uint32), np.empty(batch, np.uint32)
+    for _ in range(12):
+        tables[:] = perm.integers(0, num_blocks, tables.shape)
+        lens[:] = perm.integers(1, 7 * 16, batch)
+        cases.append((tables.copy(), lens.copy()))
+        got.append(be.paged_attention_forward(q, kp, vp, tables, lens, args, out_dtype=fa.capi.F32))
+        tables[:], lens[:] = 0, 1
+    for (t, n), g in zip(cases, got):
+        want = be.download_owned(be.paged_attention_forward_device(q, kp, vp, be.upload(t), be.upload(n), args, out_dtype=fa.capi.F32))
+        assert np.abs(be.download_owned(g) - want).max() < 2e-6      # the splits of a walk may differ: f32 sums of unit values
