@@ -95,19 +95,28 @@ void free_all(fa_context *ctx, fa_decoder *d) {
     }
 }
 
-// Whether the step about to be enqueued (the host lengths already count its token) sees only short contexts: its
-// attention then takes the one-launch form, and the recorded graphs of the two kinds are kept apart.
-// With at most one block (sequence x kv head) per compute unit: a scheduler's batch of up to a few dozen short
-// conversations, whose few pages the streamed form would cut into ranges of a dozen, leaving partial results and a
-// merge launch (measured through 32 layers at 4 .. 32 rows and contexts up to 1000: 2 - 14 % of the step; from 36 rows
-// on, with more blocks than compute units and their unequal lengths, the streamed form is the faster one).
-bool step_is_short(const fa_decoder *d) {
+// Whether the attention of the step about to be enqueued (the host lengths already count its token) finishes in one launch;
+// the recorded graphs of the two kinds are kept apart.
+// With at most one block per compute unit (sequences x kv heads; left-over units take shares of the sequences) the one-launch
+// form saves the partial results and the merge, and its time is the longest share; the streamed form cuts all pages into equal
+// ranges, whatever the lengths.  So the line is how far the longest share exceeds an even one.  Step through 8 layers, 32 / 8
+// heads, one launch and streamed, us: one sequence of 700 588 and 603, 6000 661 and 807; four of 4000 696 and 817; sixteen of
+// 3000 (share 1500, even 1500) 901 and 938, of 100 .. 1500 (730, 400) 766 and 791, of 200 .. 3000 (1450, 800) 871 and 843;
+// thirty-two of 2500 1116 and 1164; 16 / 4 heads, sixty of 100 .. 2000 (1980, 980) 794 and 734.  With so few sequences that
+// units are left over, the streamed form's many small ranges cost it more: one of 8000 (1000, 250) 696 and 893.
+bool step_attends_at_once(const fa_decoder *d) {
     if (k::g_decode_one == 1) return false;
-    uint32_t longest = 0;
-    for (uint32_t b = 0; b < d->batch && b < d->host_lens.size(); ++b) longest = std::max(longest, d->host_lens[b]);
-    if (d->batch == 0 || longest > k::kDecodeOneMaxCtx) return false;
-    const uint64_t blocks = (uint64_t)d->batch * d->cfg.n_kv_heads;
-    return k::g_decode_one == 2 || blocks <= (uint64_t)d->ctx->props.multiProcessorCount;
+    uint64_t longest = 0, all = 0;
+    for (uint32_t b = 0; b < d->batch && b < d->host_lens.size(); ++b) {
+        longest = std::max<uint64_t>(longest, d->host_lens[b]);
+        all += d->host_lens[b];
+    }
+    if (d->batch == 0) return false;
+    if (k::g_decode_one >= 2) return k::g_decode_one == 3 || longest <= 1024;
+    const uint64_t cus = (uint64_t)d->ctx->props.multiProcessorCount, items = (uint64_t)d->batch * d->cfg.n_kv_heads;
+    if (items > cus) return false;
+    const uint64_t shares = k::decode_one_shares(items, &d->ctx->splitk, (int)cus), even = all * d->cfg.n_kv_heads / cus;
+    return longest / shares <= even + (shares == k::kDecodeOneShares ? 1024 : 512);
 }
 
 // The kernels of one step, enqueued on the context's stream.  stop_after (test aid, -1 in normal use) ends the
@@ -131,7 +140,8 @@ fa_status enqueue_step(fa_context *ctx, fa_decoder *d, int stop_after = -1) {
     k::gather_rows_f32((const float *)d->embed->ptr, V, D, (const int32_t *)d->tokens->ptr, (float *)d->h->ptr, B, s);
     int stage = 0;
     auto stop_here = [&]() { return stop_after >= 0 && stage++ == stop_after; };
-    const bool short_ctx = step_is_short(d);
+    const bool at_once = step_attends_at_once(d);
+    const uint32_t shares = k::decode_one_shares((uint64_t)B * c.n_kv_heads, &ctx->splitk, cus);
     if (stop_here()) return after_launch(ctx, "decoder step (partial)");
 
     k::PagedShape ps;
@@ -191,10 +201,9 @@ fa_status enqueue_step(fa_context *ctx, fa_decoder *d, int stop_after = -1) {
         // inside their own launch (k::RowPrologue): the row stage then launches nothing and its outputs (codes,
         // scales) appear with the linear's stage, written by one block of it.
         const bool fuse_qkv = k::qkv_rope_fuses_norm(B, L.wqkv->k_pad);
-        // Short sequences: the attention finishes in one launch (a block per sequence and kv head; no
-        // partial results, no merge launch) and leaves its output and the heads' maxima for the o projection, which
+        // The attention finishes in one launch (a block per share of a sequence and kv head; no merge launch) and leaves its output and the heads' maxima for the o projection, which
         // does the per-token quantizer itself when there is one row (a launch of its own otherwise).
-        const bool one_form = short_ctx && c.n_heads <= 32 && F >= EQ && EQ % 64 == 0;
+        const bool one_form = at_once && c.n_heads <= 32 && F >= EQ && EQ % 64 == 0;
         const bool one_attn = one_form && k::plain_fuses_pmax_quantizer(B, L.wo->n_pad, L.wo->k_pad, cus);
         if (!fuse_qkv)
             k::rmsnorm_quantize_i8((const float *)d->h->ptr, (const float *)L.attn_norm->ptr, c.rms_eps, nullptr,
@@ -213,14 +222,14 @@ fa_status enqueue_step(fa_context *ctx, fa_decoder *d, int stop_after = -1) {
             k::paged_attention_decode_one_bf16((const uint16_t *)d->q_bf->ptr, (const uint16_t *)L.k_pool->ptr,
                                                (const uint16_t *)L.v_pool->ptr, (const uint32_t *)d->tables->ptr,
                                                (const uint32_t *)d->seq_lens->ptr, ps, (float *)d->act->ptr,
-                                               (float *)d->pmax->ptr, s);
+                                               (float *)d->pmax->ptr, s, shares, &ctx->splitk);
         } else if (one_form) {
             // the same launch for more rows than the o projection quantizes for itself: the quantizer from the heads'
             // maxima is a launch of its own (the output is f32 values already rounded to bf16, the operator's output type)
             k::paged_attention_decode_one_bf16((const uint16_t *)d->q_bf->ptr, (const uint16_t *)L.k_pool->ptr,
                                                (const uint16_t *)L.v_pool->ptr, (const uint32_t *)d->tables->ptr,
                                                (const uint32_t *)d->seq_lens->ptr, ps, (float *)d->act->ptr,
-                                               (float *)d->pmax->ptr, s);
+                                               (float *)d->pmax->ptr, s, shares, &ctx->splitk);
             k::quantize_rows_from_pmax(d->act->ptr, false, (const float *)d->pmax->ptr, c.n_heads, (int8_t *)d->xq->ptr,
                                        (float *)d->sx->ptr, B, m_pad, EQ, s);
         } else if (c.n_heads <= 32) {
@@ -769,9 +778,9 @@ fa_status fa_decoder_step(fa_context *ctx, fa_decoder *d, int32_t use_graph) {
         return es;
     }
     if (d->graph_waves != g_decode_waves) drop_graphs(d);
-    // a graph per batch size and kind of step (bit 31: the short-context form, decided on the lengths after this step)
+    // a graph per batch size and kind of step (bit 31: the one-launch attention, decided on the lengths after this step)
     advance(1);
-    const uint32_t key = d->batch | (!d->layered && step_is_short(d) ? 0x80000000u : 0u);
+    const uint32_t key = d->batch | (!d->layered && step_attends_at_once(d) ? 0x80000000u : 0u);
     advance(-1);
     auto it = d->graphs.find(key);
     if (it == d->graphs.end()) {

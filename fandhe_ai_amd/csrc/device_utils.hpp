@@ -235,5 +235,39 @@ __device__ __forceinline__ void prefetch_weights(const PF &pf, uint32_t j) {
     asm volatile("" ::"v"(acc[0] ^ acc[1] ^ acc[2] ^ acc[3]));      // the loads are the point; keep them
 }
 
+// Blocks that meet in memory: partial results are stored, the stores awaited, and a ticket drawn from the group's counter; who
+// draws the last one goes on with everybody's.  LOCAL: the members run on one XCD and share its L2.
+template <bool LOCAL, typename T>
+__device__ __forceinline__ void meet_store(T *p, T v) {
+    if constexpr (LOCAL)
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <bool LOCAL, typename T>
+__device__ __forceinline__ T meet_load(const T *p) {
+    if constexpr (LOCAL)
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    else
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Ticket of this block in its group (0 .. S - 1), the same value in every thread.  `slot` is one LDS word that
+// nobody else uses between the two barriers.  Call with all of the block's partial stores issued.
+template <bool LOCAL>
+__device__ __forceinline__ uint32_t meet_ticket(uint32_t *counter, uint32_t *slot) {
+    __builtin_amdgcn_s_waitcnt(0);                   // this thread's partial stores are acknowledged by L2 / memory
+    __syncthreads();                                 // ... and so are everybody's
+    if (threadIdx.x == 0) {
+        uint32_t t;
+        if constexpr (LOCAL)
+            t = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        else
+            t = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *slot = t;
+    }
+    __syncthreads();
+    return *slot;
+}
+
 }  // namespace dev
 }  // namespace fa

@@ -169,6 +169,11 @@ struct StreamParams {
     // ONE form only (decode_stream_kernel<..., ONE = true>): the finished attention output, f32 values already rounded
     // to bf16 (the operator's output type), [batch][num_heads][128], and the absmax of every head's slice
     float *one_out = nullptr, *one_pmax = nullptr;
+    // ... and where up to `shares` blocks of a sequence and kv head meet: [block][256 threads][8] sums, [block][2][16] maxima
+    // and denominators, a counter per sequence and kv head
+    uint32_t shares = 1;
+    float *one_part = nullptr, *one_part_ml = nullptr;
+    uint32_t *one_counters = nullptr;
 };
 
 // Length of (virtual) sequence vs: all cached positions up to the last new token of its tile.  A row whose
@@ -199,9 +204,11 @@ __device__ __forceinline__ uint32_t range_pages(const StreamParams &p, uint32_t 
 
 // ONE (decode only): one block per (sequence, kv head) instead of one wavefront per (range, kv head).  The four
 // wavefronts of the block take a quarter of the sequence's pages each, their results meet in LDS, and the first
-// wavefront normalises and stores the finished output (p.one_out, p.one_pmax): no partial results in memory, no
-// merge launch.  For a few short sequences (a compute unit per kv head streams a whole sequence); the arithmetic of
-// the meeting is that of the merge kernels.
+// wavefront normalises and stores the finished output (p.one_out, p.one_pmax): no merge launch.  What bounds it is what one
+// compute unit can have in flight (about 25 bytes a nanosecond), so sequences of more than sixteen pages are cut into up to
+// p.shares blocks while compute units are left: each leaves its sums, and the one that draws the last ticket adds them in the
+// order of the shares.  Eight kv heads of one sequence, 700 tokens: 18.9 us in 8 blocks, 13.4 in 24; the streamed form 9.6 and
+// 10.0 for its merge.  The arithmetic of both meetings is that of the merge kernels.
 template <int SP, int KD, int VD, int WPE, bool PF, int TT = 1, bool ONE = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) decode_stream_kernel(StreamParams p) {
     static_assert(PF || TT == 1, "several token tiles per wavefront exist only in the prefill form");
@@ -210,10 +217,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
     __shared__ __attribute__((aligned(16))) uint16_t v_s[4][kPage * kVPitch];
     __shared__ float one_o[ONE ? 4 : 1][ONE ? 64 : 1][ONE ? 33 : 1];       // [wavefront][lane][its 32 dims], padded
     __shared__ float one_ml[ONE ? 4 : 1][2][16], one_amax[ONE ? 4 : 1][16];
+    __shared__ uint32_t one_ticket;
+    constexpr uint32_t kOneShares = kDecodeOneShares, kOneSharePages = kDecodeOneSharePages;
     const int lane = threadIdx.x % 64;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int g = lane / 16, c = lane % 16;
-    const uint32_t item_id = ONE ? blockIdx.x : blockIdx.x * 4 + wave;
+    const uint32_t item_id = ONE ? blockIdx.x % (p.batch * p.num_kv_heads) : blockIdx.x * 4 + wave;
     const uint32_t kvh = item_id % p.num_kv_heads, r = item_id / p.num_kv_heads;   // ONE: r is the sequence
     if (r >= (ONE ? p.batch : p.n_ranges)) return;
     const uint32_t max_ctx = p.max_blocks_per_seq * kPage;
@@ -501,7 +510,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
         const uint32_t len_b = p.seq_lens[r];
         const uint32_t len_c = len_b > max_ctx ? max_ctx : len_b;
         const uint32_t npg = (len_c + kPage - 1) / kPage;
-        const uint32_t lo = (uint32_t)((uint64_t)npg * (uint32_t)wave / 4), hi = (uint32_t)((uint64_t)npg * ((uint32_t)wave + 1) / 4);
+        const uint32_t items = p.batch * p.num_kv_heads, share = blockIdx.x / items, fill = (npg + kOneSharePages - 1) / kOneSharePages;
+        const uint32_t shares = fill < 2 ? 1 : fill < p.shares ? fill : p.shares;
+        if (share >= shares) return;
+        const uint32_t part = share * 4 + wave, parts = shares * 4;
+        const uint32_t lo = (uint32_t)((uint64_t)npg * part / parts), hi = (uint32_t)((uint64_t)npg * (part + 1) / parts);
         if (hi > lo) {
             segment(r, lo, hi, len_b);
         } else {                                                       // no pages for this wavefront: weight zero
@@ -530,6 +543,45 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
             den = __builtin_fmaf(wt, one_ml[w][1][c], den);
 #pragma unroll
             for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(wt, one_o[w][lane][8 * wave + e], acc[e]);
+        }
+        if (shares > 1) {
+            const uint64_t first = (uint64_t)item_id * p.shares;
+            float *sums = p.one_part + first * 2048 + threadIdx.x * 8, *ml = p.one_part_ml + first * 32 + c;
+            if ((uint32_t)c < p.group) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) meet_store<false>(sums + share * 2048 + e, acc[e]);
+                if (wave == 0 && g == 0) {
+                    meet_store<false>(ml + share * 32, mx);
+                    meet_store<false>(ml + share * 32 + 16, den);
+                }
+            }
+            if (meet_ticket<false>(p.one_counters + item_id, &one_ticket) != shares - 1) return;
+            if (threadIdx.x == 0) meet_store<false>(p.one_counters + item_id, 0u);
+            // in the order of the shares, whoever came last; shares that are not there repeat the last with weight zero
+            float m[kOneShares], l[kOneShares], o[kOneShares][8];
+            if ((uint32_t)c < p.group) {
+#pragma unroll
+                for (uint32_t t = 0; t < kOneShares; ++t) {
+                    const uint32_t at = t < shares ? t : shares - 1;
+                    m[t] = meet_load<false>(ml + at * 32);
+                    l[t] = meet_load<false>(ml + at * 32 + 16);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[t][e] = meet_load<false>(sums + at * 2048 + e);
+                }
+                mx = -INFINITY;
+#pragma unroll
+                for (uint32_t t = 0; t < kOneShares; ++t) mx = (m[t] != m[t] || mx != mx) ? __uint_as_float(0x7fc00000u) : fmaxf(mx, m[t]);
+                den = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
+#pragma unroll
+                for (uint32_t t = 0; t < kOneShares; ++t) {
+                    const float wt = t < shares ? expf(m[t] - mx) : 0.0f;
+                    den = __builtin_fmaf(wt, l[t], den);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(wt, o[t][e], acc[e]);
+                }
+            }
         }
         float amax = 0.0f, v[8];
 #pragma unroll
@@ -1430,14 +1482,17 @@ void paged_attention_decode_bf16(const uint16_t *q, const uint16_t *k_pool, cons
     decode_stream_merge_kernel<<<grid2, 256, 0, s>>>(sp, out, out_bf16, pmax);
 }
 
-// Decode attention of a few short sequences with the finished output in one launch (decode_stream_kernel's ONE
-// form): out_f32 [batch][num_heads][128] holds the output values rounded to bf16, pmax [batch][num_heads] the absmax
-// of every head's slice, which is what a per-token quantizer in front of the next projection needs.  A compute unit
-// per (sequence, kv head) streams the whole sequence, so this is for contexts of at most kDecodeOneMaxCtx tokens;
-// longer ones go through paged_attention_decode_bf16.
+// Decode attention with the finished output in one launch (decode_stream_kernel's ONE form): out_f32
+// [batch][num_heads][128] holds the output values rounded to bf16, pmax [batch][num_heads] the absmax of every head's
+// slice, which is what a per-token quantizer in front of the next projection needs.
 int g_decode_one = 0;
+uint32_t decode_one_shares(uint64_t items, const SplitKArea *sk, int num_cus) {
+    if (items == 0 || !sk || !sk->partial || !sk->counters || items > sk->n_counters) return 1;
+    const uint64_t room = std::min<uint64_t>((uint64_t)num_cus, sk->partial_bytes / ((2048 + 32) * sizeof(float)));
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kDecodeOneShares, room / items));
+}
 void paged_attention_decode_one_bf16(const uint16_t *q, const uint16_t *k_pool, const uint16_t *v_pool, const uint32_t *tables,
-                                     const uint32_t *seq_lens, const PagedShape &ps, float *out_f32, float *pmax, hipStream_t s) {
+                                     const uint32_t *seq_lens, const PagedShape &ps, float *out_f32, float *pmax, hipStream_t s, uint32_t shares, const SplitKArea *sk) {
     if (ps.batch == 0) return;
     StreamParams sp;
     sp.q = q;
@@ -1462,7 +1517,14 @@ void paged_attention_decode_one_bf16(const uint16_t *q, const uint16_t *k_pool, 
     sp.n_vseq = ps.batch;
     sp.one_out = out_f32;
     sp.one_pmax = pmax;
-    decode_stream_kernel<4, 4, 2, 2, false, 1, true><<<ps.batch * ps.num_kv_heads, 256, 0, s>>>(sp);
+    const uint64_t items = (uint64_t)ps.batch * ps.num_kv_heads;
+    sp.shares = shares;
+    if (shares > 1) {
+        sp.one_part = (float *)sk->partial;
+        sp.one_part_ml = sp.one_part + items * shares * 2048;
+        sp.one_counters = sk->counters;
+    }
+    decode_stream_kernel<4, 4, 2, 2, false, 1, true><<<(unsigned)(items * shares), 256, 0, s>>>(sp);
 }
 
 // Prefill (l_new > 1) on the same streaming kernel: groups of kPrefillTT token tiles of 16 / group new tokens

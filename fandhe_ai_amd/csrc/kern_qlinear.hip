@@ -1185,21 +1185,8 @@ __global__ void __launch_bounds__(512)
 // x + 8 (S q + r), r = 0 .. S - 1: they share one L2.  LOCAL = true relies on that (probed once per context by
 // the caller): stores, ticket and loads are ordinary L2 accesses.  LOCAL = false uses agent-scope accesses that
 // are coherent between XCDs wherever the blocks run.  The ticket is relaxed; what orders it behind the stores is
-// the wait for their acknowledgement, not a fence (an agent-scope release writes back a whole L2).
-template <bool LOCAL, typename T>
-__device__ __forceinline__ void meet_store(T *p, T v) {
-    if constexpr (LOCAL)
-        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else
-        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <bool LOCAL, typename T>
-__device__ __forceinline__ T meet_load(const T *p) {
-    if constexpr (LOCAL)
-        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    else
-        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+// the wait for their acknowledgement, not a fence (an agent-scope release writes back a whole L2).  (meet_store, meet_load,
+// meet_ticket: device_utils.hpp)
 // Four consecutive words of a partial tile set, requested with the cache policy of meet_load (a wider relaxed atomic
 // load does not exist; the words were written by one 16-byte store whose acknowledgement the writer awaited before its
 // ticket).  The request is an assembly statement, so the compiler neither waits for it nor knows that `v` is in
@@ -1215,24 +1202,6 @@ __device__ __forceinline__ void unseen_wait_all(v4i (&x)[4][4]) {
                    "+v"(x[1][3]), "+v"(x[2][0]), "+v"(x[2][1]), "+v"(x[2][2]), "+v"(x[2][3]), "+v"(x[3][0]), "+v"(x[3][1]),
                    "+v"(x[3][2]), "+v"(x[3][3]));
 }
-// Ticket of this block in its group (0 .. S - 1), the same value in every thread.  `slot` is one LDS word that
-// nobody else uses between the two barriers.  Call with all of the block's partial stores issued.
-template <bool LOCAL>
-__device__ __forceinline__ uint32_t meet_ticket(uint32_t *counter, uint32_t *slot) {
-    __builtin_amdgcn_s_waitcnt(0);                   // this thread's partial stores are acknowledged by L2 / memory
-    __syncthreads();                                 // ... and so are everybody's
-    if (threadIdx.x == 0) {
-        uint32_t t;
-        if constexpr (LOCAL)
-            t = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        else
-            t = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *slot = t;
-    }
-    __syncthreads();
-    return *slot;
-}
-
 // LOCAL only: the members of a group must share an XCD, or the partial tiles above were exchanged through two
 // different L2s.  Every member notes the XCD it runs on before it takes its ticket; the last arriver compares and
 // reports a mismatch in host memory (the context then refuses further work: the launch's results are wrong).

@@ -89,10 +89,10 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  *        size; 0: the linears that follow do that row work themselves where that measured faster (norm + quantizer: one
  *        or two rows, quantizer from partial maxima: one row); 2: wherever the kernels can (four / two rows); takes
  *        effect when a step is recorded;
- * key 20: 1 keeps the streamed attention with its merge launch for every decode step; 0: a step whose contexts are
- *        at most 1024 tokens runs the attention as one launch (a block per sequence and kv head) while there is at
- *        most one such block per compute unit (with one or two sequences the o projection then does the quantizer);
- *        2: whenever the contexts are that short (takes effect when a step is recorded);
+ * key 20: 1 keeps the streamed attention with its merge launch for every decode step; 0: the attention runs as one
+ *        launch while there is at most one (sequence, kv head) per compute unit and no share of a sequence is much longer
+ *        than an even one (with one or two sequences the o projection then does the quantizer); 2: whenever the contexts
+ *        are at most 1024 tokens; 3: always (takes effect when a step is recorded);
  * key 21: the int8 linears of 65 to a few hundred rows (fa_linear_w8a8, prompt passes of the decoder): 0 the
  *        weight-stationary kernel where the shape rule picks it (a weight with at most about two column tiles per
  *        compute unit, m x k at most 2 MiB; k of 8192 .. 14336: the form that splits k over four blocks of an XCD,

@@ -195,3 +195,39 @@ def test_tables_queued_one_call_behind_the_other(max_blocks):
     for (t, n), g in zip(cases, got):
         want = be.download_owned(be.paged_attention_forward_device(q, kp, vp, be.upload(t), be.upload(n), args, out_dtype=fa.capi.F32))
         assert np.abs(be.download_owned(g) - want).max() < 2e-6      # the splits of a walk may differ: f32 sums of unit values
+
+
+@pytest.mark.parametrize("ctxs", [[255], [256], [257, 15], [513, 1792, 40], [1793], [2047, 2500], [300, 3999, 16, 1]], ids=str)
+def test_attention_shares_of_one_launch(ctxs, tune):
+    """A step whose sequences are one share, two, some and as many as there may be (sixteen pages fill one), beside sequences
+    that have fewer: codes and scales of the attention output against the streamed form, up to the last bits of the f32 sums."""
+    import ctypes as C
+    import test_gpu_decoder as td
+    import fandhe_ai_amd as fa
+    be, lib = ops(), fa.capi.lib
+    shape = dict(n_layers=2, d_model=2048, n_heads=16, n_kv_heads=4, d_ffn=3072, vocab=3000)
+    m = td.build_model(seed=90 + sum(ctxs), steps=5, batch=len(ctxs), ctxs=ctxs, **shape)
+    got = {}
+    for form in (3, 1):
+        tune(20, form)
+        dec = td.GpuDecoder(be, m)
+        dec.set_state(m.seq_lens, m.tokens)
+        for _ in range(2):                            # the counters are as they were found
+            fa.check(lib.fa_decoder_debug_step_until(be._ctx, dec.h, 4))
+            dec.set_state(m.seq_lens, m.tokens)
+        xq, sx = C.c_void_p(), C.c_void_p()
+        fa.check(lib.fa_decoder_debug_buffer(dec.h, 1, C.byref(xq)))
+        fa.check(lib.fa_decoder_debug_buffer(dec.h, 2, C.byref(sx)))
+        codes, scales = np.empty(16 * shape["d_model"], np.int8), np.empty(len(ctxs), np.float32)
+        fa.check(lib.fa_download(be._ctx, xq, 0, codes.ctypes.data, codes.size))
+        fa.check(lib.fa_download(be._ctx, sx, 0, scales.ctypes.data, len(ctxs)))
+        got[form] = codes.astype(np.int32), scales
+        if form == 3:                                 # eager and replayed, against the oracle
+            lens, tokens = m.seq_lens.copy(), m.tokens.copy()
+            for step in range(3):
+                tokens = td._check_small(m, dec, lens, tokens, step > 0, "shares:%s:%d" % (ctxs, step))
+                dec.set_state(lens, tokens)
+        dec.close()
+    (ca, sa), (cb, sb) = got[3], got[1]
+    assert np.all(sb > 0) and np.allclose(sa, sb, rtol=1e-6, atol=0)
+    assert np.abs(ca - cb).max() <= 1 and (ca != cb).mean() < 2e-3 and np.any(ca != 0)
