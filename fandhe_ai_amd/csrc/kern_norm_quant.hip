@@ -9,7 +9,7 @@ namespace fa {
 namespace k {
 using namespace fa::dev;
 
-int g_rows_wide = 0;        // tuning: 1 keeps the 256-thread row kernels for every row count
+int g_rows_wide = 0;        // tuning: 1 keeps the kernels of sixteen neighbouring elements per thread for every row count
 
 namespace {
 
@@ -139,10 +139,9 @@ __global__ void __launch_bounds__(kBlock)
         for (uint64_t c = threadIdx.x; c < k_pad / 16; c += kBlock) {
             uint32_t words[4] = {0, 0, 0, 0};
             if (c < k / 16) {
-                float v[16];
-                load16<IN_BF16>(x, base + c * 16, v);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) words[e / 4] |= ((uint32_t)quant_i8(v[e], scale) & 0xffu) << (8 * (e % 4));
+                float v[4][4];
+                load16<IN_BF16>(x, base + c * 16, *reinterpret_cast<float(*)[16]>(&v));
+                quant_i8_words(v, scale, words);
             }
             if (xq_tiled)
                 *(v4u *)(xq_tiled + tiled_chunk_offset(r, c, k_tiles)) = v4u{words[0], words[1], words[2], words[3]};
@@ -246,21 +245,17 @@ __global__ void __launch_bounds__(kBlock)
         uint64_t c = threadIdx.x + (uint64_t)i * kBlock;
         if (c >= n_chunks) continue;
         uint32_t words[4];
+        quant_i8_words(xv[i], scale, words);
+        if (out_f32)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            uint32_t word = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) word |= ((uint32_t)quant_i8(xv[i][v][e], scale) & 0xffu) << (8 * e);
-            words[v] = word;
-            if (out_f32) *(v4f *)(out_f32 + r * hidden + c * 16 + v * 4) = xv[i][v];
-        }
+            for (int v = 0; v < 4; ++v) *(v4f *)(out_f32 + r * hidden + c * 16 + v * 4) = xv[i][v];
         int8_t *dst = ROW ? xq_tiled + r * hidden + c * 16 : xq_tiled + tiled_chunk_offset(r, c, k_tiles);
         *(v4u *)dst = v4u{words[0], words[1], words[2], words[3]};
     }
 }
 
-// The same for few rows (a decode step: 32 rows on 32 compute units), where the kernel's time is its chain of
-// dependent steps and not its bytes: a block of THREADS threads per row, thread t owning the four-element groups
+// The same with neighbouring threads on neighbouring groups: for few rows (a decode step: 32 rows on 32 compute units), where
+// the kernel's time is its chain of dependent steps, and for many (wide_form): a block of THREADS threads per row, thread t owning the four-element groups
 // t, t + THREADS, ... (VPT of them), so that at 4096 columns a thread converts, squares, scales and divides four
 // elements instead of sixteen and the row's bytes are requested by sixteen wavefronts at once.  Same arithmetic
 // per element; the f64 sum of squares is split over more threads (only its order differs, as above).
@@ -314,16 +309,15 @@ __global__ void __launch_bounds__(THREADS)
     amax = block_max<NW, true, true>(amax, smem_f);
     const float scale = __fdiv_rn(amax, 127.0f);
     if (threadIdx.x == 0) sx[r] = scale;
+    uint32_t words[VPT];
+    quant_i8_words(xv, scale, words);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const uint64_t j = threadIdx.x + (uint64_t)i * THREADS;
         if (j >= n_vec) continue;
-        uint32_t word = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) word |= ((uint32_t)quant_i8(xv[i][e], scale) & 0xffu) << (8 * e);
         if (out_f32) *(v4f *)(out_f32 + r * hidden + j * 4) = xv[i];
         int8_t *dst = ROW ? xq + r * hidden + j * 4 : xq + tiled_chunk_offset(r, j / 4, k_tiles) + (j % 4) * 4;
-        *(uint32_t *)dst = word;
+        *(uint32_t *)dst = words[i];
     }
 }
 
@@ -404,15 +398,14 @@ __global__ void __launch_bounds__(THREADS)
     amax = block_max<NW, true, true>(amax, smem);
     const float scale = __fdiv_rn(amax, 127.0f);
     if (threadIdx.x == 0) sx[r] = scale;
+    uint32_t words[VPT];
+    quant_i8_words(xv, scale, words);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
         const uint64_t j = threadIdx.x + (uint64_t)i * THREADS;
         if (j >= n_vec) continue;
-        uint32_t word = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) word |= ((uint32_t)quant_i8(xv[i][e], scale) & 0xffu) << (8 * e);
-        if (xq_tiled) *(uint32_t *)(xq_tiled + tiled_chunk_offset(r, j / 4, k_tiles) + (j % 4) * 4) = word;
-        if (xq_row) *(uint32_t *)(xq_row + r * k + j * 4) = word;
+        if (xq_tiled) *(uint32_t *)(xq_tiled + tiled_chunk_offset(r, j / 4, k_tiles) + (j % 4) * 4) = words[i];
+        if (xq_row) *(uint32_t *)(xq_row + r * k + j * 4) = words[i];
     }
 }
 
@@ -432,7 +425,8 @@ __global__ void __launch_bounds__(ONE ? 1024 : kBlock)
     const uint64_t r = blockIdx.x;
     const float *gate = gu + r * (PROD ? 1 : 2) * f, *up = gate + f;
     // the product of chunk c: silu(gate) * up, or the stored product
-    auto products = [&](uint64_t c, float (&p)[16]) {
+    auto products = [&](uint64_t c, float (&quads)[4][4]) {
+        float(&p)[16] = *reinterpret_cast<float(*)[16]>(&quads);
         if constexpr (PROD) {
             load16<false>(gate, c * 16, p);
         } else {
@@ -444,22 +438,22 @@ __global__ void __launch_bounds__(ONE ? 1024 : kBlock)
         }
     };
     float amax = 0.0f;
-    float prod[16];
+    float prod[4][4];
     if constexpr (ONE) {
         const uint64_t c = threadIdx.x;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) prod[e] = 0.0f;
+        for (int e = 0; e < 16; ++e) prod[e / 4][e % 4] = 0.0f;
         if (c < f / 16) {
             products(c, prod);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(prod[e]));
+            for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(prod[e / 4][e % 4]));
         }
     } else {
         for (uint64_t c = threadIdx.x; c < f / 16; c += THREADS) {
-            float pr[16];
+            float pr[4][4];
             products(c, pr);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(pr[e]));
+            for (int e = 0; e < 16; ++e) amax = fmaxf(amax, fabsf(pr[e / 4][e % 4]));
         }
     }
     amax = block_max<THREADS / 64>(amax, smem);
@@ -468,18 +462,16 @@ __global__ void __launch_bounds__(ONE ? 1024 : kBlock)
     if constexpr (ONE) {
         const uint64_t c = threadIdx.x;
         if (c < f / 16) {
-            uint32_t words[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 16; ++e) words[e / 4] |= ((uint32_t)quant_i8(prod[e], scale) & 0xffu) << (8 * (e % 4));
+            uint32_t words[4];
+            quant_i8_words(prod, scale, words);
             *(v4u *)(xq_row + (tiled ? tiled_chunk_offset(r, c, f / 64) : r * f + c * 16)) = v4u{words[0], words[1], words[2], words[3]};
         }
     } else {
         for (uint64_t c = threadIdx.x; c < f / 16; c += THREADS) {
-            float pr[16];
+            float pr[4][4];
             products(c, pr);
-            uint32_t words[4] = {0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 16; ++e) words[e / 4] |= ((uint32_t)quant_i8(pr[e], scale) & 0xffu) << (8 * (e % 4));
+            uint32_t words[4];
+            quant_i8_words(pr, scale, words);
             *(v4u *)(xq_row + (tiled ? tiled_chunk_offset(r, c, f / 64) : r * f + c * 16)) = v4u{words[0], words[1], words[2], words[3]};
         }
     }
@@ -501,18 +493,18 @@ __global__ void __launch_bounds__(kBlock)
         return;
     }
     // the group's values are requested before the partial maxima are reduced: one memory round trip, not two
-    float xv[4];
+    float xv[1][4];
     const uint64_t jj = j < n_vec ? j : n_vec - 1;
     if constexpr (IN_BF16) {
         const v2u t = *(const v2u *)((const uint16_t *)x + r * k + jj * 4);
-        xv[0] = bf16_lo(t[0]);
-        xv[1] = bf16_hi(t[0]);
-        xv[2] = bf16_lo(t[1]);
-        xv[3] = bf16_hi(t[1]);
+        xv[0][0] = bf16_lo(t[0]);
+        xv[0][1] = bf16_hi(t[0]);
+        xv[0][2] = bf16_lo(t[1]);
+        xv[0][3] = bf16_hi(t[1]);
     } else {
         const v4f t = *(const v4f *)((const float *)x + r * k + jj * 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) xv[e] = t[e];
+        for (int e = 0; e < 4; ++e) xv[0][e] = t[e];
     }
     float amax = 0.0f;
     for (uint32_t i = threadIdx.x; i < parts; i += kBlock) amax = fmaxf(amax, pmax[r * parts + i]);
@@ -520,10 +512,9 @@ __global__ void __launch_bounds__(kBlock)
     const float scale = __fdiv_rn(amax, 127.0f);
     if (blockIdx.x == 0 && threadIdx.x == 0) sx[r] = scale;
     if (j >= n_vec) return;
-    uint32_t word = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) word |= ((uint32_t)quant_i8(xv[b], scale) & 0xffu) << (8 * b);
-    *(uint32_t *)(xq_tiled + tiled_chunk_offset(r, j / 4, k_tiles) + (j % 4) * 4) = word;
+    uint32_t word[1];
+    quant_i8_words(xv, scale, word);
+    *(uint32_t *)(xq_tiled + tiled_chunk_offset(r, j / 4, k_tiles) + (j % 4) * 4) = word[0];
 }
 
 // absmax over a tensor: block maxima merged with an integer max on the bit
@@ -622,28 +613,46 @@ void rmsnorm_f32(const float *x, const float *w, float *out, uint64_t rows, uint
     rmsnorm_kernel<<<(unsigned)rows, kBlock, 0, s>>>(x, w, out, hidden, inv_n, eps);
 }
 
+// The row kernels that keep a row in registers: threads per row and four-element groups per thread.  Up to one block per compute
+// unit a row's chain is all there is: a thousand threads.  From there on rows queue, and what counts is how many are under way
+// and that every load is a whole line: 256 threads (RMSNorm and quantizer of 8192 x 4096, us: 128 threads 31.9, 256 29.4, 512
+// 36.2, 1024 66; with sixteen neighbouring elements per thread 39.9; of 2545 x 2048 8.8, 8.6, 10.4, 17.9; 11.4), up to two
+// blocks per unit 512 (300 x 4096: 256 threads 6.3, 512 5.6, 1024 6.2; sixteen neighbours 6.5).  false: rows too wide for it.
+template <typename F>
+static bool wide_form(uint64_t rows, uint64_t width, F &&go) {
+    using std::integral_constant;
+    if (g_rows_wide == 1 || width > 16384) return false;
+    if (rows <= 256 && width > 1024) {
+        if (width <= 4096) go(integral_constant<int, 1024>{}, integral_constant<int, 1>{});
+        else if (width <= 8192) go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
+        else go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
+    } else if (rows > 512 ? width > 8192 : width > 1024) {
+        if (width <= 2048) go(integral_constant<int, 512>{}, integral_constant<int, 1>{});
+        else if (width <= 4096) go(integral_constant<int, 512>{}, integral_constant<int, 2>{});
+        else if (width <= 8192) go(integral_constant<int, 512>{}, integral_constant<int, 4>{});
+        else go(integral_constant<int, 512>{}, integral_constant<int, 8>{});
+    } else {
+        if (width <= 1024) go(integral_constant<int, 256>{}, integral_constant<int, 1>{});
+        else if (width <= 2048) go(integral_constant<int, 256>{}, integral_constant<int, 2>{});
+        else if (width <= 4096) go(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+        else go(integral_constant<int, 256>{}, integral_constant<int, 8>{});
+    }
+    return true;
+}
+
 void quantize_rows_i8(const void *x, bool in_bf16, int8_t *xq_rowmajor, int8_t *xq_tiled, float *sx, uint64_t m,
                       uint64_t m_pad, uint64_t k, uint64_t k_pad, hipStream_t s) {
     uint64_t rows = xq_tiled ? m_pad : m;
     if (rows == 0 || k_pad == 0) return;
-    if (g_rows_wide != 1 && rows <= 256 && k == k_pad && k % 64 == 0 && k <= 16384) {
-        auto go = [&](auto threads, auto vpt) {
+    if (k == k_pad && k % 64 == 0 &&
+        wide_form(rows, k, [&](auto threads, auto vpt) {
             constexpr int T = decltype(threads)::value, V = decltype(vpt)::value;
             if (in_bf16)
                 quantize_rows_wide_kernel<T, V, true><<<(unsigned)rows, T, 0, s>>>(x, xq_rowmajor, xq_tiled, sx, m, k);
             else
                 quantize_rows_wide_kernel<T, V, false><<<(unsigned)rows, T, 0, s>>>(x, xq_rowmajor, xq_tiled, sx, m, k);
-        };
-        if (k <= 1024)
-            go(std::integral_constant<int, 256>{}, std::integral_constant<int, 1>{});
-        else if (k <= 4096)
-            go(std::integral_constant<int, 1024>{}, std::integral_constant<int, 1>{});
-        else if (k <= 8192)
-            go(std::integral_constant<int, 1024>{}, std::integral_constant<int, 2>{});
-        else
-            go(std::integral_constant<int, 1024>{}, std::integral_constant<int, 4>{});
+        }))
         return;
-    }
     if (in_bf16)
         quantize_rows_kernel<true><<<(unsigned)rows, kBlock, 0, s>>>(x, xq_rowmajor, xq_tiled, sx, m, k, k_pad);
     else
@@ -651,21 +660,14 @@ void quantize_rows_i8(const void *x, bool in_bf16, int8_t *xq_rowmajor, int8_t *
 }
 
 namespace {
-// Few rows (at most one block per compute unit): the wide form.  Returns false when the shape is not its case.
 template <bool ROW>
 bool launch_rmsnorm_quantize_wide(const float *x, const float *w, float eps, float inv_n, float *out_f32, int8_t *xq, float *sx,
                                   uint64_t m, uint64_t hidden, uint32_t rows, unsigned grid, const WeightPrefetch &pf,
                                   hipStream_t s) {
-    if (g_rows_wide == 1 || rows > 256 || hidden > 16384 || hidden % 16 != 0) return false;
-    if (hidden <= 1024)
-        rmsnorm_quantize_wide_kernel<256, 1, ROW><<<grid, 256, 0, s>>>(x, w, eps, inv_n, out_f32, xq, sx, m, hidden, rows, pf);
-    else if (hidden <= 4096)
-        rmsnorm_quantize_wide_kernel<1024, 1, ROW><<<grid, 1024, 0, s>>>(x, w, eps, inv_n, out_f32, xq, sx, m, hidden, rows, pf);
-    else if (hidden <= 8192)
-        rmsnorm_quantize_wide_kernel<1024, 2, ROW><<<grid, 1024, 0, s>>>(x, w, eps, inv_n, out_f32, xq, sx, m, hidden, rows, pf);
-    else
-        rmsnorm_quantize_wide_kernel<1024, 4, ROW><<<grid, 1024, 0, s>>>(x, w, eps, inv_n, out_f32, xq, sx, m, hidden, rows, pf);
-    return true;
+    return hidden % 16 == 0 && wide_form(rows, hidden, [&](auto threads, auto vpt) {
+        constexpr int T = decltype(threads)::value, V = decltype(vpt)::value;
+        rmsnorm_quantize_wide_kernel<T, V, ROW><<<grid, T, 0, s>>>(x, w, eps, inv_n, out_f32, xq, sx, m, hidden, rows, pf);
+    });
 }
 }  // namespace
 

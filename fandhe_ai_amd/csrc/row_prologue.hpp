@@ -91,14 +91,12 @@ __device__ __forceinline__ void prologue_rmsnorm_quantize(const RowPrologue &p, 
         for (int i = 1; i < 16; ++i) amax = fmaxf(amax, smem_f[i]);
         const float scale = __fdiv_rn(amax, 127.0f);
         if (tid == 0) sx[r] = scale;
+        uint32_t words[2];
+        quant_i8_words(xv[r], scale, words);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const uint32_t j = tid + h * kPrologueThreads;
-            if (j >= n_vec) continue;
-            uint32_t word = 0;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) word |= ((uint32_t)quant_i8(xv[r][h][e], scale) & 0xffu) << (8 * e);
-            *(uint32_t *)(codes + (uint64_t)r * k + j * 4) = word;
+            if (j < n_vec) *(uint32_t *)(codes + (uint64_t)r * k + j * 4) = words[h];
         }
         __syncthreads();                                // smem_f free again; codes of the row visible
     }
@@ -143,13 +141,16 @@ __device__ __forceinline__ void prologue_quantize_from_pmax(const RowPrologue &p
         const float scale = __fdiv_rn(amax, 127.0f);
         if (tid == 0) sx[r] = scale;
 #pragma unroll
-        for (int u = 0; u < kPmaxVecs; ++u) {
-            const uint32_t j = tid + u * kPrologueThreads;
-            if (j >= n_vec) continue;
-            uint32_t word = 0;
+        for (int u = 0; u < kPmaxVecs; u += 2) {
+            if ((uint32_t)u * kPrologueThreads >= n_vec) break;      // uniform
+            const v4f pair[2] = {t.xv[r][u], t.xv[r][u + 1]};
+            uint32_t words[2];
+            quant_i8_words(pair, scale, words);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) word |= ((uint32_t)quant_i8(t.xv[r][u][e], scale) & 0xffu) << (8 * e);
-            *(uint32_t *)(codes + (uint64_t)r * k + j * 4) = word;
+            for (int h = 0; h < 2; ++h) {
+                const uint32_t j = tid + (u + h) * kPrologueThreads;
+                if (j < n_vec) *(uint32_t *)(codes + (uint64_t)r * k + j * 4) = words[h];
+            }
         }
         __syncthreads();
     }

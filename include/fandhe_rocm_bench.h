@@ -83,8 +83,8 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  *        tiles meeting in memory (agent-scope accesses), 3 whenever the shape allows it with the partial tiles
  *        meeting in the XCD's L2, 4 by shape but meeting in memory;
  * key 17: blocks per group of that form: 0 by shape, 2 or 4;
- * key 18: 1 keeps the 256-thread form of the row kernels (norm, quantizer, norm + quantizer) for every row count
- *        instead of the up-to-1024-thread form used for at most 256 rows;
+ * key 18: 1 keeps the row kernels (norm, quantizer, norm + quantizer) of sixteen neighbouring elements per thread for every
+ *        row count and width;
  * key 19: 1 keeps the norm + quantizer and quantizer kernels of a decode step as launches of their own for every batch
  *        size; 0: the linears that follow do that row work themselves where that measured faster (norm + quantizer: one
  *        or two rows, quantizer from partial maxima: one row); 2: wherever the kernels can (four / two rows); takes

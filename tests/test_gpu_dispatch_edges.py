@@ -231,3 +231,32 @@ def test_attention_shares_of_one_launch(ctxs, tune):
     (ca, sa), (cb, sb) = got[3], got[1]
     assert np.all(sb > 0) and np.allclose(sa, sb, rtol=1e-6, atol=0)
     assert np.abs(ca - cb).max() <= 1 and (ca != cb).mean() < 2e-3 and np.any(ca != 0)
+
+
+@pytest.mark.parametrize("rows,k", [(256, 1088), (257, 1024), (257, 2112), (512, 4160), (513, 1024), (513, 2112), (600, 4096), (600, 8256),
+                                    (300, 16384), (513, 16384), (300, 16448)])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_row_quantizer_codes(rows, k, bf16):
+    """Threads per row and groups per thread on both sides of their lines; values in the middle of two codes and next to it, rows
+    of zeros, of subnormals, with an infinity or a NaN: the codes of the division, a byte each."""
+    import test_gpu_paged as paged
+    o, fa, be = paged.o, paged._fa(), paged.ops()
+    rng = np.random.default_rng(rows + k)
+    x = rng.standard_normal((rows, k)).astype(np.float32)
+    grid = (rng.integers(-254, 255, (rows, k)) / 2).astype(np.float32)
+    x[0::5] = grid[0::5]
+    x[0::5, 0] = 127.0                                # scale 1: halves are ties
+    x[1::5] = grid[1::5] * np.float32(0.37) * (1 + rng.integers(-2, 3, x[1::5].shape).astype(np.float32) * np.float32(2.0 ** -23))
+    x[1::5, 1] = np.float32(127 * 0.37)
+    x[7], x[12], x[17] = 0.0, x[12] * np.float32(1e-41), x[17] * np.float32(1e37)
+    if bf16:
+        x = o.from_bf16(o.to_bf16(x))
+    x[22, 5], x[27, 9], x[32, 3] = np.inf, np.nan, -np.inf
+    xq, sx = be.quantize_rows_i8(be.upload(o.to_bf16(x) if bf16 else x))
+    with np.errstate(all="ignore"):
+        scale = (np.fmax.reduce(np.abs(x), axis=1) / np.float32(127)).astype(np.float32)
+        q = np.rint(x / scale[:, None])
+        q = np.where(np.isnan(q), -127, np.clip(q, -127, 127))
+    q[scale == 0] = 0
+    assert np.array_equal(be.download_owned(sx), scale, equal_nan=True)
+    assert np.array_equal(be.download_owned(xq).reshape(rows, k), q.astype(np.int8))
