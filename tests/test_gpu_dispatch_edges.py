@@ -260,3 +260,21 @@ def test_row_quantizer_codes(rows, k, bf16):
     q[scale == 0] = 0
     assert np.array_equal(be.download_owned(sx), scale, equal_nan=True)
     assert np.array_equal(be.download_owned(xq).reshape(rows, k), q.astype(np.int8))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 4096), (2, 32764), (2, 32768), (1, 32772), (2, 65537), (1, 131076), (3, 7)])
+def test_argmax_around_eight_loads_per_thread(rows, cols):
+    """The first of equal maxima, wherever the thread that sees it stands; NaN passed over; a row of nothing else gives 0."""
+    import oracle_lib as o
+    rng = np.random.default_rng(cols)
+    be = ops()
+    for case in range(6):
+        x = np.round(rng.standard_normal((rows, cols)) * 2).astype(np.float32)
+        x[rng.random(x.shape) < 0.1] = np.nan
+        if case == 1:
+            x[:] = np.nan
+        if case == 2:
+            x[:] = -np.inf
+        if case == 3:
+            x[0, -1] = 99.0
+        assert np.array_equal(be.download_owned(be.argmax(be.upload(x))), o.argmax_rows(x)), case
