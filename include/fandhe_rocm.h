@@ -520,7 +520,7 @@ fa_status fa_decoder_read_row_sampling(fa_context *ctx, fa_decoder *dec, fa_row_
  * fa_decoder_step continues from there.  The per-row arithmetic is the decode
  * step's: a prompt token leaves the K / V rows it would leave if it were
  * decoded.  Rejected before anything is queued if a row has no pages for its
- * prompt.  Asynchronous apart from the upload of the token ids.  The activation
+ * prompt.  Asynchronous (the token ids are consumed on return).  The activation
  * buffers of a pass that are 32 MiB or larger stay with the decoder for its next
  * pass (grow only, released by fa_decoder_destroy; about 1.8 GB for 8192 rows at
  * d_model 4096 / d_ffn 14336); smaller ones come from the context's pool. */
