@@ -220,8 +220,8 @@ fa_status fa_paged_attention_forward(fa_context *ctx, const fa_buffer *q, const 
     uint64_t tb = n_tables * 4, lb = n_seq * 4;
     uint64_t lens_off = (tb + 255) / 256 * 256;
     if (fa_status s = ensure_table_stage(ctx, lens_off + lb)) return s;
-    if (fa_status s = queue_upload(ctx, ctx->table_stage, block_tables, tb, "block table upload")) return s;
-    if (fa_status s = queue_upload(ctx, (char *)ctx->table_stage + lens_off, seq_lens, lb, "sequence lengths upload")) return s;
+    const Upload parts[2] = {{ctx->table_stage, block_tables, tb}, {(char *)ctx->table_stage + lens_off, seq_lens, lb}};
+    if (fa_status s = queue_uploads(ctx, parts, 2, "block table upload")) return s;
     uint32_t longest = 0;
     for (uint64_t i = 0; i < n_seq; ++i) longest = seq_lens[i] > longest ? seq_lens[i] : longest;
     return launch_attention(ctx, q, k_pool, v_pool, (const uint32_t *)ctx->table_stage,

@@ -704,8 +704,8 @@ fa_status fa_decoder_set_sequences(fa_context *ctx, fa_decoder *d, uint32_t batc
                 return fail(FA_ERR_INVALID_ARGUMENT, "paged_kv: row " + std::to_string(b) + " entry " +
                                                          std::to_string(i) + " is not a valid block id");
     }
-    if (fa_status s = queue_upload(ctx, d->tables->ptr, block_tables, (uint64_t)batch * c.max_blocks_per_seq * 4, "decoder_set_sequences")) return s;
-    if (fa_status s = queue_upload(ctx, d->seq_lens->ptr, seq_lens, (uint64_t)batch * 4, "decoder_set_sequences")) return s;
+    const Upload parts[2] = {{d->tables->ptr, block_tables, (uint64_t)batch * c.max_blocks_per_seq * 4}, {d->seq_lens->ptr, seq_lens, (uint64_t)batch * 4}};
+    if (fa_status s = queue_uploads(ctx, parts, 2, "decoder_set_sequences")) return s;
     d->batch = batch;
     try {
         d->host_tables.assign(block_tables, block_tables + (uint64_t)batch * c.max_blocks_per_seq);
@@ -939,9 +939,8 @@ static fa_status prefill_impl(fa_context *ctx, fa_decoder *d, const int32_t *tok
         const uint32_t lc = std::min(lc_max, l_new - t0);
         for (uint32_t b = 0; b < B; ++b)
             for (uint32_t i = 0; i < lc; ++i) stage[(uint64_t)b * lc + i] = tokens[(uint64_t)b * l_new + t0 + i];
-        if (fa_status s = queue_upload(ctx, t.tok.ptr, stage.data(), (uint64_t)B * lc * 4, "prompt token upload")) return s;
-        if (padded)
-            if (fa_status s = queue_upload(ctx, t.row_lens.ptr, row_lens, (uint64_t)B * 4, "prompt lengths upload")) return s;
+        const Upload parts[2] = {{t.tok.ptr, stage.data(), (uint64_t)B * lc * 4}, {t.row_lens.ptr, row_lens, (uint64_t)B * 4}};
+        if (fa_status s = queue_uploads(ctx, parts, padded ? 2 : 1, "prompt token upload")) return s;
         if (fa_status s = enqueue_prefill_chunk(ctx, d, t, lc, t0 + lc == l_new, verify, padded)) return s;
         for (uint32_t b = 0; b < B; ++b) d->host_lens[b] += padded ? row_lens[b] : lc;
     }

@@ -133,9 +133,13 @@ __global__ void fill_u32_kernel(uint32_t *p, uint32_t v, uint64_t n) {
     for (; i < n; i += stride) p[i] = v;
 }
 
-__global__ void copy_words_kernel(const uint32_t *from, uint32_t *to, uint64_t n) {
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) to[i] = __builtin_nontemporal_load(from + i);
+struct WordRanges {
+    WordRange r[kWordRanges];
+};
+__global__ void copy_words_kernel(WordRanges w) {
+    const WordRange r = w.r[blockIdx.y];
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < r.n) r.to[i] = __builtin_nontemporal_load(r.from + i);
 }
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
@@ -231,9 +235,14 @@ void fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s) {
     if (n == 0) return;
     fill_u32_kernel<<<grid_for(n, 256), 256, 0, s>>>(p, v, n);
 }
-void copy_words(const uint32_t *from, uint32_t *to, uint64_t n, hipStream_t s) {
-    if (n == 0) return;
-    copy_words_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(from, to, n);
+void copy_words(const WordRange *ranges, int count, hipStream_t s) {
+    WordRanges w{};
+    uint32_t most = 0;
+    for (int i = 0; i < count; ++i) {
+        w.r[i] = ranges[i];
+        most = std::max(most, ranges[i].n);
+    }
+    if (most) copy_words_kernel<<<dim3((most + 255) / 256, (unsigned)count), 256, 0, s>>>(w);
 }
 void fill_normal(void *out, int out_bf16, uint64_t n, uint64_t seed, float mean, float std, hipStream_t s) {
     if (n == 0) return;

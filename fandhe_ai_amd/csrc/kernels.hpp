@@ -48,8 +48,14 @@ void convert_bf16_to_f32(const uint16_t *in, float *out, uint64_t n, hipStream_t
 void rope_f32(const float *x, const int32_t *pos, float *out, uint64_t rows, uint64_t heads,
               uint64_t head_dim, double theta, hipStream_t s);
 void fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s);
-// 32-bit words from memory of the host that the device can read
-void copy_words(const uint32_t *from, uint32_t *to, uint64_t n, hipStream_t s);
+// 32-bit words from memory of the host that the device can read: up to four ranges in one launch
+struct WordRange {
+    const uint32_t *from;
+    uint32_t *to;
+    uint32_t n;
+};
+constexpr int kWordRanges = 4;
+void copy_words(const WordRange *ranges, int count, hipStream_t s);
 // N(mean, std) from a counter-based hash of (seed, index); out is f32 or bf16
 void fill_normal(void *out, int out_bf16, uint64_t n, uint64_t seed, float mean, float std, hipStream_t s);
 

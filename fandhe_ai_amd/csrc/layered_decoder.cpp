@@ -814,8 +814,8 @@ fa_status layered_forward(fa_context *ctx, fa_decoder *d, const uint32_t *counts
                 if (fa_status s = upload(ctx, a.expand_meta, expand.meta.data(), expand.meta.size() * 4)) return s;
             }
             if (fa_status s = attention_workspace(ctx, L, a, rows, B, portions)) return s;
-            if (fa_status s = upload(ctx, a.row_start, starts.data(), (B + 1) * 4)) return s;
-            if (fa_status s = upload(ctx, a.tokens, stage.data(), (uint64_t)rows * 4)) return s;
+            const Upload parts[2] = {{a.row_start, starts.data(), (B + 1) * 4ull}, {a.tokens, stage.data(), (uint64_t)rows * 4}};
+            if (fa_status s = queue_uploads(ctx, parts, 2, "upload of a pass")) return s;
             prepare_rows(ctx, d, a, a.row_start, rows);
             const k::RaggedRows rr = ragged(d, a, a.row_start, rows);
             enqueue_embed(ctx, L, a, a.tokens, rr);

@@ -187,13 +187,21 @@ static bool ring_ready(fa_context *ctx) {
     return true;
 }
 
-fa_status queue_upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes, const char *what) {
+fa_status queue_uploads(fa_context *ctx, const Upload *parts, int count, const char *what) {
+    uint64_t bytes = 0;
+    bool words = true;
+    for (int i = 0; i < count; ++i) {
+        bytes += (parts[i].bytes + 63) / 64 * 64;
+        words = words && parts[i].bytes % 4 == 0 && (uintptr_t)parts[i].dst % 4 == 0;
+    }
     if (bytes == 0) return FA_OK;
     if (ctx->capturing) return fail(FA_ERR_CAPTURE_IN_PROGRESS, std::string(what) + " is not allowed during graph capture");
     fa_upload_ring &r = ctx->ring;
     std::lock_guard<std::mutex> g(r.mu);
-    if (bytes > r.kHalf || bytes % 4 != 0 || (uintptr_t)dst % 4 != 0 || !ring_ready(ctx)) {
-        hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream);
+    if (bytes > r.kHalf || !words || count > k::kWordRanges || !ring_ready(ctx)) {
+        hipError_t e = hipSuccess;
+        for (int i = 0; i < count && e == hipSuccess; ++i)
+            if (parts[i].bytes) e = hipMemcpyAsync(parts[i].dst, parts[i].src, parts[i].bytes, hipMemcpyHostToDevice, ctx->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
         return e == hipSuccess ? FA_OK : hip_fail(ctx, e, what, FA_ERR_TRANSFER_FAILED);
     }
@@ -207,10 +215,14 @@ fa_status queue_upload(fa_context *ctx, void *dst, const void *src, uint64_t byt
         r.busy[r.half] = false;
         r.used = 0;
     }
-    const uint64_t at = r.half * r.kHalf + r.used;
-    std::memcpy(r.host + at, src, bytes);
-    r.used += (bytes + 63) / 64 * 64;
-    k::copy_words((const uint32_t *)(r.device + at), (uint32_t *)dst, bytes / 4, ctx->stream);
+    k::WordRange ranges[k::kWordRanges];
+    for (int i = 0; i < count; ++i) {
+        const uint64_t at = r.half * r.kHalf + r.used;
+        if (parts[i].bytes) std::memcpy(r.host + at, parts[i].src, parts[i].bytes);
+        ranges[i] = k::WordRange{(const uint32_t *)(r.device + at), (uint32_t *)parts[i].dst, (uint32_t)(parts[i].bytes / 4)};
+        r.used += (parts[i].bytes + 63) / 64 * 64;
+    }
+    k::copy_words(ranges, count, ctx->stream);
     return after_launch(ctx, what);
 }
 

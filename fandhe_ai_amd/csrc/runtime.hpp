@@ -164,7 +164,16 @@ fa_status hip_fail(fa_context *ctx, hipError_t e, const char *what, fa_status as
 fa_status after_launch(fa_context *ctx, const char *kernel);
 // Host memory to memory that only work queued on the context's stream reads: the source is consumed on return, the copy is
 // queued.  (Buffers that a caller may read elsewhere are filled by fa_upload and fa_upload_into, which wait for the copy.)
-fa_status queue_upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes, const char *what);
+struct Upload {
+    void *dst;
+    const void *src;
+    uint64_t bytes;
+};
+fa_status queue_uploads(fa_context *ctx, const Upload *parts, int count, const char *what);      // at most four
+inline fa_status queue_upload(fa_context *ctx, void *dst, const void *src, uint64_t bytes, const char *what) {
+    const Upload part{dst, src, bytes};
+    return queue_uploads(ctx, &part, 1, what);
+}
 
 // Pool-backed raw allocation used by buffers and by internal scratch.
 fa_status pool_alloc(fa_context *ctx, uint64_t bytes, void **ptr, uint64_t *class_bytes);
