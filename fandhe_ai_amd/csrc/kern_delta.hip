@@ -56,41 +56,42 @@ __device__ __forceinline__ float conv_silu(const T *__restrict__ y, uint32_t ld,
 }
 
 // ------------------------------------------------------------------ token by token
-// One block per (sequence, head); the state sits in registers (thread: four neighbouring columns of up to RPT rows) from
-// the first token of the pass to the last.  CG = column groups of four, a power of two.
+// One block per (sequence, head), or per part of a wide state's columns (StepPlan); the state sits in registers (thread: four
+// neighbouring columns of up to RPT rows) from the first token of the pass to the last.  CG = column groups of four, a power of two.
 // FAST (single tokens, at most four taps, no more than NQ NT channels): the inputs of the convolution are requested ahead of
 // the state, so that the convolution runs while the state travels.
 // A single token of a few sequences is a chain of latencies: dependent loads, barriers, and the instructions themselves,
 // which come from memory at every launch (about half a microsecond per KiB of code that runs through once).  So a block is
-// a thousand threads with up to eight rows each where few blocks leave the CUs to them (16 K values at four rows), every
+// a thousand threads with up to eight rows each where few blocks leave the CUs to them (StepPlan), every
 // wavefront forms the norms and k . q for itself, and the wavefronts meet three times: 4 sequences of 16 heads 128 x 128 13.4 us
 // on 256 threads with eight meetings, 11.5 so (32 sequences: 256 threads still, 35.5 us, 27 at the rate of a copy).
-constexpr int step_channels(int nt, int rpt) { return nt == 1024 && rpt <= 8 ? 1 : 2; }
+constexpr int step_channels(int nt) { return nt == 1024 ? 1 : 2; }
 
 template <typename T, int NT, int RPT, bool FAST, Recurrence KIND>
 __global__ void __launch_bounds__(NT)
     delta_step_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, uint32_t cg_log2, int write_ring, uint32_t max_tokens) {
-    constexpr int NW = NT / 64, NQ = step_channels(NT, RPT);
+    constexpr int NQ = step_channels(NT);
     // q [dim], k [dim], v [CG * 4], decays [dim] or shares of S^T k and S^T q [2][parts][CG * 4], their sums [2][CG * 4]
     extern __shared__ float lds[];
     constexpr bool CHANNEL = KIND == Recurrence::kChannelDelta, LIGHTNING = KIND == Recurrence::kLightning;
-    __shared__ float smem[NW];
     const uint32_t b = blockIdx.x, h = blockIdx.y;
     const uint32_t row0 = rr.row_start[b], n_tok = rr.row_start[b + 1] - row0;
     if (n_tok == 0 || n_tok > max_tokens) return;
     const uint32_t dim = sh.dim, vdim = sh.vdim, vp = sh.vdim_p(), channels = sh.qkv();
     const uint32_t share = sh.heads / sh.kv_heads, hk = h / share;
     const uint32_t CG = 1u << cg_log2, RG = NT >> cg_log2, cg = threadIdx.x & (CG - 1), rg = threadIdx.x >> cg_log2, lane = threadIdx.x % 64;
+    const uint32_t col0 = blockIdx.z * CG * 4, cols = vdim - col0 < CG * 4 ? vdim - col0 : CG * 4, col = col0 + cg * 4;      // this block's, this thread's
     // a wavefront's row groups are added inside it; parts: what is left to add
-    const uint32_t wide = CG < 64 ? 64 : CG, parts = NT / wide, own_part = threadIdx.x / wide;
+    constexpr uint32_t parts = NT / 64;
+    const uint32_t own_part = threadIdx.x / 64;
     const uint32_t dim_a = (dim + 3) / 4 * 4;        // keeps v and the shares 16-byte aligned
     float *lq = lds, *lk = lds + dim_a, *lv = lk + dim_a, *part = lv + CG * 4, *total = part + 2 * parts * CG * 4, *lg = total + 2 * CG * 4;
     const T *y = (const T *)io.y;
     T *ring = (T *)io.ring + (uint64_t)rr.state_slot[b] * sh.taps * channels;
     float *state = io.state + ((uint64_t)rr.state_slot[b] * sh.heads + h) * dim * vp;
-    const bool col_ok = cg * 4 < vp;
+    const bool col_ok = col < vp;
     const uint32_t p0 = (uint32_t)rr.pos[row0];
-    auto channel = [&](uint32_t i) { return i < dim ? hk * dim + i : i < 2 * dim ? (sh.kv_heads + hk) * dim + (i - dim) : 2 * sh.kv_heads * dim + h * vdim + (i - 2 * dim); };
+    auto channel = [&](uint32_t i) { return i < dim ? hk * dim + i : i < 2 * dim ? (sh.kv_heads + hk) * dim + (i - dim) : 2 * sh.kv_heads * dim + h * vdim + col0 + (i - 2 * dim); };
     float xin[NQ][4], win[NQ][4];
     if constexpr (FAST) {
 #pragma unroll
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(NT)
 #pragma unroll
             for (uint32_t back = 0; back < 4; ++back) {
                 xin[q][back] = win[q][back] = 0.0f;
-                if (i < 2 * dim + vdim && (back < sh.taps || back == 0) && back <= p0) {
+                if (i < 2 * dim + cols && (back < sh.taps || back == 0) && back <= p0) {
                     const uint32_t c = channel(i);
                     xin[q][back] = load_as_f32(back == 0 ? y + (uint64_t)row0 * io.ld_y + c : ring + (uint64_t)((p0 - back) % sh.taps) * channels + c);
                     win[q][back] = sh.taps ? io.conv[(uint64_t)c * sh.taps + sh.taps - 1 - back] : 1.0f;
@@ -120,7 +121,7 @@ __global__ void __launch_bounds__(NT)
     for (int i = 0; i < RPT; ++i) {
         const uint32_t d = rg + i * RG;
         S[i] = v4f{0.f, 0.f, 0.f, 0.f};
-        if (p0 != 0 && col_ok && d < dim) S[i] = stream_load<true>((const v4f *)(state + (uint64_t)d * vp + cg * 4));
+        if (p0 != 0 && col_ok && d < dim) S[i] = stream_load<true>((const v4f *)(state + (uint64_t)d * vp + col));
     }
     __builtin_amdgcn_sched_barrier(0);
     const float a_log = LIGHTNING ? 0.0f : io.a_log[h], dt_bias = KIND == Recurrence::kDelta ? io.dt_bias[h] : 0.0f;
@@ -133,7 +134,7 @@ __global__ void __launch_bounds__(NT)
             const uint32_t i = threadIdx.x + q * NT;
             if (i >= 2 * dim + CG * 4) break;
             float v = 0.0f;
-            if (i < 2 * dim + vdim) {
+            if (i < 2 * dim + cols) {
                 const uint32_t c = channel(i);
                 if constexpr (FAST) {
                     float acc = 0.0f;
@@ -143,7 +144,7 @@ __global__ void __launch_bounds__(NT)
                 } else {
                     v = conv_silu(y, io.ld_y, ring, io.conv, sh.taps, channels, c, row0, t, p);
                 }
-                if (write_ring && (i >= 2 * dim || h % share == 0)) ring[(uint64_t)(p % sh.taps) * channels + c] = y[row * io.ld_y + c];
+                if (write_ring && (i >= 2 * dim || (h % share == 0 && col0 == 0))) ring[(uint64_t)(p % sh.taps) * channels + c] = y[row * io.ld_y + c];
             }
             (i < dim ? lq[i] : i < 2 * dim ? lk[i - dim] : lv[i - 2 * dim]) = v;
         }
@@ -191,7 +192,7 @@ __global__ void __launch_bounds__(NT)
                 if constexpr (!LIGHTNING) dk[e] += __shfl_xor(dk[e], (int)off, 64);
                 dq[e] += __shfl_xor(dq[e], (int)off, 64);
             }
-        if (CG >= 64 || lane < CG) {
+        if (lane < CG) {
             if constexpr (!LIGHTNING) ((v4f *)part)[own_part * CG + cg] = dk;
             ((v4f *)part)[(parts + own_part) * CG + cg] = dq;
         }
@@ -209,26 +210,26 @@ __global__ void __launch_bounds__(NT)
         for (int i = 0; i < RPT; ++i) {
             const uint32_t d = rg + i * RG;
             if (d < dim) S[i] += u * (lk[d] * rk);
-            if (t + 1 == n_tok && col_ok && d < dim) __builtin_nontemporal_store(S[i], (v4f *)(state + (uint64_t)d * vp + cg * 4));
+            if (t + 1 == n_tok && col_ok && d < dim) __builtin_nontemporal_store(S[i], (v4f *)(state + (uint64_t)d * vp + col));
         }
         const v4f o = dq + u * kq;
-        if (sh.norm_all) {                           // the norm runs over all heads: another launch's
+        if (sh.norm_all) {                           // the norm runs over more than this block's columns: another launch's
             if (rg == 0) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (cg * 4 + e < vdim) io.raw[(row * sh.heads + h) * vdim + cg * 4 + e] = o[e];
+                    if (col + e < vdim) io.raw[(row * sh.heads + h) * vdim + col + e] = o[e];
             }
             if (t + 1 < n_tok) __syncthreads();
             continue;
         }
-        // up to 64 column groups are a wavefront's lanes (each as often as it has row groups)
+        // the column groups are a wavefront's lanes (each as often as it has row groups)
         float so = 0.0f;
-        if (CG <= 64 ? lane < CG : rg == 0) {
+        if (lane < CG) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (cg * 4 + e < vdim) so = fmaf(o[e], o[e], so);
         }
-        so = CG <= 64 ? wave_sum_dpp(so) : block_sum<float, NW, true>(so, smem);
+        so = wave_sum_dpp(so);
         const float ro = 1.0f / sqrtf(so / (float)vdim + sh.eps);
         if (rg == 0) {
 #pragma unroll
@@ -1083,7 +1084,7 @@ __device__ __forceinline__ void store_gated(const DeltaShape &sh, P v, const T *
     }
 }
 
-// Read-outs of the chunk form: root mean square, weight, gate.  One wavefront per (row, head); two heads with 32 lanes each where
+// Read-outs of the chunk form, and of states in column parts: root mean square, weight, gate.  One wavefront per (row, head); two heads with 32 lanes each where
 // four values per lane make a head (HALVES).
 template <typename T>
 __global__ void __launch_bounds__(256) delta_gate_halves_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr) {
@@ -1101,10 +1102,10 @@ __global__ void __launch_bounds__(256) delta_gate_halves_kernel(DeltaShape sh, D
     }
 }
 template <typename T>
-__global__ void __launch_bounds__(256) delta_gate_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, const float *__restrict__ o) {
+__global__ void __launch_bounds__(256) delta_gate_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, const float *__restrict__ o, uint32_t from) {
     const uint32_t lane = threadIdx.x % 64, r = blockIdx.x, vdim = sh.vdim, b = rr.row_seq[r];
-    if (rr.row_start[b + 1] - rr.row_start[b] < kChunkFrom) return;          // done token by token
-    for (uint32_t h = threadIdx.x / 64; h < sh.heads; h += 4) {
+    if (rr.row_start[b + 1] - rr.row_start[b] < from) return;                // done token by token
+    for (uint32_t h = blockIdx.y * 4 + threadIdx.x / 64; h < sh.heads; h += gridDim.y * 4) {
         const float *x = o + ((uint64_t)r * sh.heads + h) * vdim;
         float sq = 0.0f;
         for (uint32_t c = lane; c < vdim; c += 64) sq = fmaf(x[c], x[c], sq);
@@ -1158,8 +1159,9 @@ void allow_lds(F f, size_t bytes) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void *>(f), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+// gate_from: sequences with fewer new tokens have their rows gated already
 template <typename T, int KT, Recurrence KIND>
-void launch_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, const ChunkPlan &p, hipStream_t s) {
+void launch_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, const ChunkPlan &p, uint32_t gate_from, hipStream_t s) {
     float *frags = io.scratch, *decay = frags + (uint64_t)p.slots * sh.heads * p.frags * 256;
     constexpr size_t rows = 32 * (KT * 16 + 4), lds = (rows * (KIND == Recurrence::kChannelDelta ? 3 : 2) + 32 * 68 + 2 * 32 * 36) * 4;
     static bool configured = false;
@@ -1196,18 +1198,18 @@ void launch_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr
     }
     if (sh.norm_all) return;                         // the whole pass's rows at the end
     if (sh.vdim <= 128 && ((sh.vdim | io.ld_gate | io.ld_out) & 3) == 0) delta_gate_halves_kernel<T><<<rr.rows, 256, 0, s>>>(sh, io, rr);
-    else delta_gate_kernel<T><<<rr.rows, 256, 0, s>>>(sh, io, rr, io.raw);
+    else delta_gate_kernel<T><<<rr.rows, 256, 0, s>>>(sh, io, rr, io.raw, gate_from);
 }
 
 template <typename T, Recurrence KIND>
-void run_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, hipStream_t s) {
+void run_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, uint32_t gate_from, hipStream_t s) {
     const ChunkPlan p = chunk_plan(sh, rr.rows, rr.batch);
     switch (p.kt) {
-        case 1: return launch_chunks<T, 1, KIND>(sh, io, rr, p, s);
-        case 2: return launch_chunks<T, 2, KIND>(sh, io, rr, p, s);
-        case 4: return launch_chunks<T, 4, KIND>(sh, io, rr, p, s);
-        case 8: return launch_chunks<T, 8, KIND>(sh, io, rr, p, s);
-        default: return launch_chunks<T, 16, KIND>(sh, io, rr, p, s);
+        case 1: return launch_chunks<T, 1, KIND>(sh, io, rr, p, gate_from, s);
+        case 2: return launch_chunks<T, 2, KIND>(sh, io, rr, p, gate_from, s);
+        case 4: return launch_chunks<T, 4, KIND>(sh, io, rr, p, gate_from, s);
+        case 8: return launch_chunks<T, 8, KIND>(sh, io, rr, p, gate_from, s);
+        default: return launch_chunks<T, 16, KIND>(sh, io, rr, p, gate_from, s);
     }
 }
 
@@ -1222,49 +1224,64 @@ __global__ void __launch_bounds__(256) delta_ring_kernel(DeltaShape sh, DeltaIo 
     for (uint32_t t = n - keep; t < n; ++t) ring[(uint64_t)((p0 + t) % sh.taps) * channels + c] = ((const T *)io.y)[(uint64_t)(row0 + t) * io.ld_y + c];
 }
 
+// How single tokens divide a state: column groups of four per block (log2), parts of its columns, threads.
+// A thousand threads where every block has a CU to itself; from two blocks per CU on the small ones stand in each other's waits.  A
+// turn of 16 steps, heads of 128 x 128, 256 and 1024 threads: 64 blocks 6100 and 6014 us, 256 6640 and 6590, 512 7402 and 7580, 1024
+// 9341 and 9723.
+// A thread holds a part's rows in registers, so a state of more than 32 K values (or more than 256 columns) is cut into parts of at
+// most 16 K.  (In one block it is 16 to 64 rows of four on a thousand threads, which have 128 registers each, or 64 on 256, and up to two
+// KiB per lane of it lie in scratch.)  Its read-outs are normed by a launch of their own.
+// A step of four layers, us, in one block and so: 16 heads of 256 x 256, 4 sequences 194 and 131, 32 sequences 460 and 412; of 140 x 200,
+// 16 sequences 206 and 199; 8 heads of 256 x 200 with decays per channel, 4 sequences 316 and 161.
+struct StepPlan {
+    uint32_t cg_log2, parts;
+    bool small;                              // 256 threads
+};
+StepPlan step_plan(const DeltaShape &sh, uint32_t batch) {
+    StepPlan p{0, 1, true};
+    while ((4u << p.cg_log2) < sh.vdim) ++p.cg_log2;
+    if (p.cg_log2 > 6 || ((uint64_t)sh.dim << p.cg_log2) > 8 * 1024) {
+        p.cg_log2 = sh.dim > 128 ? 4 : 5;
+        p.parts = (sh.vdim + (4u << p.cg_log2) - 1) / (4u << p.cg_log2);
+    }
+    p.small = (uint64_t)batch * sh.heads * p.parts > 256;
+    return p;
+}
+
 template <typename T, int NT, Recurrence KIND>
-void launch_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, uint32_t cg_log2, int write_ring, uint32_t max_tokens, hipStream_t s) {
-    const uint32_t CG = 1u << cg_log2, rg = NT >> cg_log2, parts = NT / std::max(CG, 64u);
-    const size_t lds = (3 * ((sh.dim + 3) / 4 * 4) + 4 * CG + 2 * (parts + 1) * 4 * CG) * 4;
-    const dim3 grid(rr.batch, sh.heads);
-#define FA_STEP(R_)                                                                                                   \
-    fast ? delta_step_kernel<T, NT, R_, true, KIND><<<grid, NT, lds, s>>>(sh, io, rr, cg_log2, write_ring, max_tokens)       \
-         : delta_step_kernel<T, NT, R_, false, KIND><<<grid, NT, lds, s>>>(sh, io, rr, cg_log2, write_ring, max_tokens)
-    const uint32_t in = 2 * sh.dim + 4 * CG;
-    const bool fast = max_tokens == 1 && sh.taps <= 4 && in <= 2 * NT;
-    // (FAST's few rows come with one channel per thread)
-    const uint32_t rpt = fast && NT == 1024 && in > NT ? std::max(16u, (sh.dim + rg - 1) / rg) : (sh.dim + rg - 1) / rg;
-    if constexpr (NT == 1024) {
+void launch_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, const StepPlan &p, int write_ring, uint32_t max_tokens, hipStream_t s) {
+    const uint32_t CG = 1u << p.cg_log2, rg = NT >> p.cg_log2, rpt = (sh.dim + rg - 1) / rg, in = 2 * sh.dim + 4 * CG;
+    const size_t lds = (3 * ((sh.dim + 3) / 4 * 4) + 4 * CG + 2 * (NT / 64 + 1) * 4 * CG) * 4;
+    const dim3 grid(rr.batch, sh.heads, p.parts);
+    DeltaShape part = sh;
+    if (p.parts > 1) part.norm_all = 1;
+    const bool fast = max_tokens == 1 && sh.taps <= 4 && in <= step_channels(NT) * NT;
+#define FA_STEP(R_)                                                                                                           \
+    fast ? delta_step_kernel<T, NT, R_, true, KIND><<<grid, NT, lds, s>>>(part, io, rr, p.cg_log2, write_ring, max_tokens)       \
+         : delta_step_kernel<T, NT, R_, false, KIND><<<grid, NT, lds, s>>>(part, io, rr, p.cg_log2, write_ring, max_tokens)
+    if constexpr (NT == 1024) {                      // dim x columns <= 32 K: at most eight rows
         if (rpt <= 4) FA_STEP(4);
-        else if (rpt <= 8) FA_STEP(8);
-        else if (rpt <= 16) FA_STEP(16);
-        else if (rpt <= 32) FA_STEP(32);
-        else FA_STEP(64);
-    } else {
+        else FA_STEP(8);
+    } else {                                         // ... and 32
         if (rpt <= 4) FA_STEP(4);
         else if (rpt <= 16) FA_STEP(16);
-        else if (rpt <= 32) FA_STEP(32);
-        else FA_STEP(64);
+        else FA_STEP(32);
     }
 #undef FA_STEP
 }
 
 template <typename T, Recurrence KIND>
 void mixer_kind(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, uint32_t max_new, hipStream_t s) {
-    uint32_t cg_log2 = 0;
-    while ((4u << cg_log2) < sh.vdim) ++cg_log2;
+    const StepPlan p = step_plan(sh, rr.batch);
     const int write_ring = max_new == 1 && sh.taps;
     const bool chunks = max_new >= kChunkFrom && g_delta_form != 1;
     const uint32_t longest = chunks ? kChunkFrom - 1 : max_new;      // sequences of a pass go to one of the two forms by length
     if (!chunks || rr.batch > 1) {
-        // A thousand threads where every block has a CU to itself and eight rows per thread hold the state (or where 256
-        // threads have too few columns); from two blocks per CU on the small ones stand in each other's waits.  A turn of 16
-        // steps, heads of 128 x 128, 256 and 1024 threads: 64 blocks 6100 and 6014 us, 256 6640 and 6590, 512 7402 and 7580,
-        // 1024 9341 and 9723.
-        if (cg_log2 > 6 || ((uint64_t)rr.batch * sh.heads <= 256 && ((uint64_t)sh.dim << cg_log2) <= 8 * 1024)) launch_step<T, 1024, KIND>(sh, io, rr, cg_log2, write_ring, longest, s);
-        else launch_step<T, 256, KIND>(sh, io, rr, cg_log2, write_ring, longest, s);
+        if (p.small) launch_step<T, 256, KIND>(sh, io, rr, p, write_ring, longest, s);
+        else launch_step<T, 1024, KIND>(sh, io, rr, p, write_ring, longest, s);
     }
-    if (chunks) run_chunks<T, KIND>(sh, io, rr, s);
+    if (chunks) run_chunks<T, KIND>(sh, io, rr, p.parts > 1 ? 0 : kChunkFrom, s);
+    else if (p.parts > 1 && !sh.norm_all) delta_gate_kernel<T><<<dim3(rr.rows, rr.rows <= 256 ? (sh.heads + 3) / 4 : 1), 256, 0, s>>>(sh, io, rr, io.raw, 0);
     if (!write_ring && sh.taps) delta_ring_kernel<T><<<dim3(rr.batch, (sh.qkv() + 255) / 256), 256, 0, s>>>(sh, io, rr);
     if (sh.norm_all) gate_all<T>(sh, io, rr.rows, s);
 }

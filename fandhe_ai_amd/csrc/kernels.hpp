@@ -578,7 +578,7 @@ struct DeltaIo {
     uint32_t ld_out;
     float out_scale;
     float *scratch;              // delta_scratch_bytes: chunk form only
-    float *raw;                  // [rows, heads x vdim] read-outs: chunk form and norm_all
+    float *raw;                  // [rows, heads x vdim] read-outs: chunk form, norm_all, single tokens of wide states
 };
 constexpr uint32_t kDeltaMaxDim = 256, kDeltaMaxVdim = 1024;
 uint64_t delta_scratch_bytes(const DeltaShape &sh, uint32_t rows, uint32_t batch);
