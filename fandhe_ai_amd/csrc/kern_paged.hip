@@ -1123,7 +1123,11 @@ __global__ void __launch_bounds__(kFlashNW * 64) __attribute__((amdgpu_waves_per
         for (int ps = 0; ps < kPasses; ++ps) {
             const uint64_t page = (uint64_t)(uintptr_t)pool + (id[ps] < p.num_blocks ? id[ps] : 0) * page_bytes;
             const uint32_t to = (uint32_t)(uintptr_t)(lptr)(rows + (ps * kRows + wave * 4) * kDh);
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(page), "s"(to) : "memory");
+            // (m0 is a reserved register: named, so that no value the compiler may have put there is expected behind this, and warned about)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_off), "s"(page), "s"(to) : "memory", "m0");
+#pragma clang diagnostic pop
         }
     };
     // all but the last N requests of every wavefront are there
