@@ -75,7 +75,8 @@ class RowSampling(C.Structure):
 
 class GemmPlan(C.Structure):
     """fa_gemm_plan: the kernel a prefill-shape GEMM is launched with."""
-    _fields_ = [("big_ntb", C.c_int32), ("waves", C.c_int32), ("splits", C.c_uint32)]
+    _fields_ = [("big_ntb", C.c_int32), ("waves", C.c_int32), ("splits", C.c_uint32), ("big_mtb", C.c_int32), ("share", C.c_uint32),
+                ("weight_stationary", C.c_int32)]
 
 
 class DecoderConfig(C.Structure):

@@ -129,10 +129,15 @@ fa_status fa_gemm_f32_form_query(uint64_t m, uint64_t n, uint64_t k, int32_t *fo
 fa_status fa_gemm_plan_query(const fa_context *ctx, uint64_t m, const fa_qweight *qw, fa_gemm_plan *out) {
     if (!ctx || ctx->magic != kCtxMagic || !out) return fail(FA_ERR_INVALID_ARGUMENT, "gemm_plan_query: bad argument");
     if (!qw || qw->magic != kQwMagic) return fail(FA_ERR_INVALID_ARGUMENT, "gemm_plan_query: not a quantized weight");
-    const k::GemmPlan p = k::gemm_plan(qw->kind != FA_QW_INT8_CHANNEL, m, qw->n_pad, qw->k_pad, ctx->props.multiProcessorCount);
+    const bool int8 = qw->kind == FA_QW_INT8_CHANNEL;
+    const int cus = ctx->props.multiProcessorCount;
+    const k::GemmPlan p = k::gemm_plan(!int8, m, qw->n_pad, qw->k_pad, cus, &ctx->splitk);
     out->big_ntb = p.big_ntb;
     out->waves = p.waves;
     out->splits = p.splits;
+    out->big_mtb = p.big_mtb;
+    out->share = p.share;
+    out->weight_stationary = int8 && m > 64 && qw->k == qw->k_pad && k::linear_w8a8_rows_applies(m, qw->n_pad, qw->k_pad, cus, &ctx->splitk);
     return FA_OK;
 }
 

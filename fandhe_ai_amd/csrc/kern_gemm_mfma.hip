@@ -1051,17 +1051,17 @@ void launch_big(const BigTile &t, const uint8_t *aq, const uint8_t *w_tiles, uin
     }
     if constexpr ((WIDTHS & kWide16) != 0) rows(std::integral_constant<int, 16>{});
 }
-// The quantized GEMMs' other wavefront counts (tuning): 256 rows
+// The quantized GEMMs' other wavefront counts (tuning): tiles of 256 rows and 224 or 256 columns
+int big_waves(const BigTile &t) { return t.mtb == 16 && t.ntb != 8 && (g_gemm_waves == 4 || g_gemm_waves == 16) ? g_gemm_waves : 8; }
 template <bool FP8, typename Epi>
 bool launch_big_waves(const BigTile &t, const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, const Epi &e, hipStream_t s) {
     const uint32_t nb = (uint32_t)((n_tiles + t.ntb - 1) / t.ntb);
-    if (t.mtb != 16 || t.ntb == 8) return false;
-    if (g_gemm_waves == 4) {
+    if (big_waves(t) == 4) {
         if (t.ntb == 14) launch_big_tile<FP8, 14, 2, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
         else launch_big_tile<FP8, 16, 2, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
         return true;
     }
-    if (g_gemm_waves == 16) {
+    if (big_waves(t) == 16) {
         if (t.ntb == 14) launch_big_tile<FP8, 14, 8, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
         else launch_big_tile<FP8, 16, 8, 16>(aq, w_tiles, m, n, n_tiles, k_steps, nb, 0, e, s);
         return true;
@@ -1099,16 +1099,25 @@ static uint64_t share_bytes(const BigTile &t, uint64_t m, uint64_t n_pad) {
     return t.share > 1 ? big_tiles(t, m, n_pad) * t.share * ((uint64_t)t.mtb * t.ntb * 256 * 4) : 0;
 }
 
-GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus) {
-    GemmPlan out{0, 4, 1};
-    if (fp8) {
-        out.big_ntb = !big_applies(n_pad / 16, k_pad) ? 0 : pick_big(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8).ntb;
-    } else {
-        const W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus);
+// ... with what the context has for blocks that share a tile (they come with eight wavefronts only)
+static W8a8Plan plan_w8a8(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, const SplitKArea *sk) {
+    const W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus);
+    if (p.tile.share == 1 || (sk && sk->counters && big_tiles(p.tile, m, n_pad) <= sk->n_counters && g_gemm_waves != 4 && g_gemm_waves != 16)) return p;
+    return plan_w8a8(m, n_pad, k_pad, num_cus, false);
+}
+
+GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, const SplitKArea *sk) {
+    GemmPlan out{0, 4, 1, 0, 1};
+    W8a8Plan p;
+    if (!fp8) p = plan_w8a8(m, n_pad, k_pad, num_cus, sk);
+    else if (big_applies(n_pad / 16, k_pad)) p.tile = pick_big(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8);
+    out.splits = p.splits;
+    if (p.tile.ntb) {
         out.big_ntb = p.tile.ntb;
-        out.splits = p.splits;
+        out.big_mtb = p.tile.mtb;
+        out.share = p.tile.share;
+        out.waves = big_waves(p.tile);
     }
-    if (out.big_ntb) out.waves = g_gemm_waves == 4 ? 4 : g_gemm_waves == 16 ? 16 : 8;
     return out;
 }
 
@@ -1123,17 +1132,17 @@ void gemm_w8a8_mfma(const int8_t *aq, const int8_t *w_tiles, uint64_t m, uint64_
                     const SplitKArea *sk) {
     if (m == 0 || n == 0) return;
     const EpiI8 e{ep.sx, ep.sw, ep.bias, ep.residual, ep.acc_out, ep.out, ep.out_bf16};
-    W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus);
+    W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus, sk);
     if (p.tile.share > 1) {
         const uint64_t tiles = big_tiles(p.tile, m, n_pad);
-        if (sk && sk->counters && tiles <= sk->n_counters && workspace && workspace_bytes >= share_bytes(p.tile, m, n_pad) && g_gemm_waves != 4 && g_gemm_waves != 16) {
+        if (workspace && workspace_bytes >= share_bytes(p.tile, m, n_pad)) {
             // (the scope knob of the split-k decode linears forces either form here as well: 2 agent scope, 3 the XCD's L2)
             const EpiI8Split es{e, (int32_t *)workspace, sk->counters, g_skinny_ksplit == 2 ? 0 : g_skinny_ksplit == 3 ? 1 : sk->xcd_local, p.tile.share};
             const unsigned grid = 8u * p.tile.share * (unsigned)((tiles + 7) / 8);   // whole groups on every XCD; surplus groups return at once
             launch_big<false, kWide8>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, es, s, grid);
             return;
         }
-        p = plan_w8a8(m, n_pad, k_pad, num_cus, false);      // no counters or no room: the plan without shared tiles
+        p = plan_w8a8(m, n_pad, k_pad, num_cus, false);      // no room: the plan without shared tiles
     }
     if (p.splits > 1 && (!workspace || workspace_bytes < (uint64_t)p.splits * m * n * 4))
         p.splits = 1;                                 // no room for partial sums: one block per tile

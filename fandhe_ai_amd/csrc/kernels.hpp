@@ -256,8 +256,10 @@ void gemm_w8a8_swiglu_mfma(const int8_t *aq, const int8_t *w_tiles, const float 
 struct GemmPlan {
     int big_ntb, waves;
     uint32_t splits;
+    int big_mtb;
+    uint32_t share;
 };
-GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus);
+GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, const SplitKArea *sk);
 // aq: e4m3 [m, k_pad] row-major; scales are device scalars.
 void gemm_e4m3_mfma(const uint8_t *aq, const uint8_t *w_tiles, const float *a_scale,
                     const float *w_scale, uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad,

@@ -134,11 +134,16 @@ fa_status fa_topology_query(const fa_context *ctx, int32_t *xcd_local, int32_t *
 /* Which kernel a prefill-shape GEMM of m rows against `qw` is launched with under the
  * current knobs (pure host function, nothing is queued).  big_ntb: column tiles of 16
  * per block of the large-tile kernel (gemm_mfma_big_kernel), 0 when the 128 x 128 kernel
- * (gemm_mfma_kernel) is used; waves: wavefronts per block; splits: blocks that share the
- * k range of one output tile (1: no split). */
+ * (gemm_mfma_kernel) is used; waves: wavefronts per block; splits: blocks of the 128 x 128
+ * kernel that share the k range of one output tile (1: no split); big_mtb: row tiles of 16 per
+ * block of the large-tile kernel; share: blocks of it that share a tile, a part of k each;
+ * weight_stationary: 1 when fa_linear_w8a8 takes the weight-stationary kernel instead. */
 typedef struct {
     int32_t big_ntb, waves;
     uint32_t splits;
+    int32_t big_mtb;
+    uint32_t share;
+    int32_t weight_stationary;
 } fa_gemm_plan;
 fa_status fa_gemm_plan_query(const fa_context *ctx, uint64_t m, const fa_qweight *qw, fa_gemm_plan *out);
 

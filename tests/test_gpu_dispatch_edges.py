@@ -173,6 +173,28 @@ def test_fp8_gemm_on_every_tile(mtb, ntb, m, k, n, tune):
     assert np.all(np.abs(got[rows] - a64 @ w64 * scale) <= bound)
 
 
+@pytest.mark.parametrize("mtb,ntb,waves", [(8, 16, 4), (12, 14, 16), (16, 8, 4), (16, 14, 4), (16, 16, 16), (8, 8, 4)])
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+def test_plan_names_the_wavefronts_that_are_launched(kind, mtb, ntb, waves, tune):
+    """Blocks of four and sixteen wavefronts exist on 256 rows x 224 and 256 columns; on other tiles the key changes nothing, other
+    than that such a call has no tile shared by several blocks."""
+    import fandhe_ai_amd as fa
+    import test_gpu_quantized as tq
+    be = ops()
+    m, k, n = 300, 8192, 2048
+    w = be.upload(np.ones((k, n), np.float32))
+    qw = be.quantize_weight(fa.DeviceBufferView(w, 0, (k, n)), fa.capi.QW_INT8_CHANNEL if kind == "int8" else fa.capi.QW_E4M3_TENSOR)
+    tune(37, mtb)
+    tune(7, ntb)
+    plan = tq._gemm_plan(fa, be, m, qw)
+    assert (plan.big_mtb, plan.big_ntb, plan.waves) == (mtb, ntb, 8)
+    assert (plan.share > 1) == (kind == "int8" and ntb == 8)
+    tune(6, waves)
+    plan = tq._gemm_plan(fa, be, m, qw)
+    assert (plan.big_mtb, plan.big_ntb, plan.share) == (mtb, ntb, 1)
+    assert plan.waves == (waves if mtb == 16 and ntb != 8 else 8)
+
+
 @pytest.mark.parametrize("scale", [-0.25, 0.0, 0.0883883476, 3.0])
 @pytest.mark.parametrize("split,cols", [(1, 2), (1, 1), (2, 2)])
 @pytest.mark.parametrize("l_new,lens", [(70, [70, 101, 400]), (33, [33, 64, 65])])

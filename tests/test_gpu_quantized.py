@@ -506,10 +506,13 @@ def test_int8_large_tile_kernel_tile_order_with_many_row_blocks(m, k, n):
     qw = be.import_quantized_weight(wq, sw)
     try:
         fa.check(lib.fa_set_tuning(7, 16))                # 256 x 256 tiles whatever the shape would pick
-        assert _gemm_plan(fa, be, m, qw).big_ntb == 16
+        fa.check(lib.fa_set_tuning(37, 16))
+        plan = _gemm_plan(fa, be, m, qw)
+        assert (plan.big_mtb, plan.big_ntb) == (16, 16)
         out, acc = be.gemm_w8a8(be.upload(aq), be.upload(sx), qw, fa.capi.F32, want_acc=True)
     finally:
         fa.check(lib.fa_set_tuning(7, 0))
+        fa.check(lib.fa_set_tuning(37, 0))
     got_acc, got = be.download_owned(acc), be.download_owned(out)
     rows = np.unique(np.r_[np.arange(0, m, 256), np.arange(255, m, 256), m - 1, 1000:1003])
     want_acc = o.gemm_i8_i32(np.ascontiguousarray(aq[rows]), wq)
@@ -620,6 +623,7 @@ def test_fp8_prefill_gemm_large_tile_kernel_rows_sampled_at_full_size():
         for ntb, waves in ((0, 0), (14, 0), (16, 0), (14, 4), (16, 16), (14, 16)):
             fa.check(lib.fa_set_tuning(7, ntb))
             fa.check(lib.fa_set_tuning(6, waves))
+            fa.check(lib.fa_set_tuning(37, 16 if waves else 0))      # those counts have tiles of 256 rows only
             plan = _gemm_plan(fa, be, m, qw)
             assert plan.big_ntb in (14, 16) and (ntb == 0 or plan.big_ntb == ntb), (ntb, plan.big_ntb)
             assert plan.waves == (waves or 8) and plan.splits == 1
@@ -638,6 +642,7 @@ def test_fp8_prefill_gemm_large_tile_kernel_rows_sampled_at_full_size():
     finally:
         fa.check(lib.fa_set_tuning(7, 0))
         fa.check(lib.fa_set_tuning(6, 0))
+        fa.check(lib.fa_set_tuning(37, 0))
     # whole-output checksum: sum over rows of the exact result is (sum_m a[m, :]) @ w; the f32 outputs
     # summed in f64 must agree within the per-element bound summed over the rows
     a_f = o.from_e4m3(want_aq).astype(np.float64)
@@ -784,14 +789,16 @@ def test_int8_large_tile_kernel_wavefront_variants_are_bit_exact():
         for ntb, waves in ((14, 4), (16, 4), (14, 16), (16, 16), (0, 0)):
             fa.check(lib.fa_set_tuning(7, ntb))
             fa.check(lib.fa_set_tuning(6, waves))
+            fa.check(lib.fa_set_tuning(37, 16 if waves else 0))      # those counts have tiles of 256 rows only
             plan = _gemm_plan(fa, be, m, qw)
-            assert plan.big_ntb in (14, 16) and plan.waves == (waves or 8)
+            assert plan.big_ntb in (14, 16) and plan.waves == (waves or 8) and (not waves or plan.big_mtb == 16)
             out, acc = be.gemm_w8a8(daq, dsx, qw, fa.capi.F32, want_acc=True)
             assert np.array_equal(be.download_owned(acc)[rows], want_acc), (ntb, waves)
             assert np.array_equal(be.download_owned(out)[rows], want), (ntb, waves)
     finally:
         fa.check(lib.fa_set_tuning(7, 0))
         fa.check(lib.fa_set_tuning(6, 0))
+        fa.check(lib.fa_set_tuning(37, 0))
 
 
 def _fp8_rows_bound_check(tag, got, qa, qb, sa, sb, bias=None):
