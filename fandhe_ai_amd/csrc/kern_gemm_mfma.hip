@@ -1071,9 +1071,10 @@ bool launch_big_waves(const BigTile &t, const uint8_t *aq, const uint8_t *w_tile
 
 }  // namespace
 
-// Where the large-tile kernel takes a quantized GEMM.  Weights of fewer than 1024 columns stay with the 128 x 128 kernel, as callers of
-// the plan query expect; it is the slower one there too (300 x 1024 -> 520, us: int8 12.5 against 7.0, e4m3 24 against 7).
-static bool big_applies(uint64_t n_tiles, uint64_t k_pad) { return !g_gemm_small_tiles && k_pad % 128 == 0 && k_pad != 0 && n_tiles >= 64; }
+// The large-tile kernel takes every quantized GEMM that it can hold, whose stages are 128 bytes of k.  The 128 x 128 kernel measured
+// slower for narrow weights too, us, 128 x 128 and large tiles: int8 with its quantizer 300 x 512 -> 16 11.9 and 7.3, 300 x 4096 -> 512 21.0
+// and 17.1, 8192 x 4096 -> 768 93.6 and 61; e4m3 300 x 1024 -> 512 23.6 and 6.3, 16384 x 4096 -> 1000 130 and 59.
+static bool big_applies(uint64_t n_tiles, uint64_t k_pad) { return !g_gemm_small_tiles && k_pad % 128 == 0 && k_pad != 0 && n_tiles != 0; }
 
 // How an int8 GEMM is launched.  tile.ntb != 0: the large-tile kernel, k over tile.share blocks of one XCD that meet in a workspace
 // (two or four where the tiles alone leave compute units idle); ntb == 0: the 128 x 128 kernel (k not a multiple of 128); splits > 1

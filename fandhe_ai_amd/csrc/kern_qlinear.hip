@@ -2076,10 +2076,21 @@ void linear_w8a8_skinny(const int8_t *xq_tiled, const int8_t *w_tiles, uint64_t 
         launch_w8a8_rows<2, kEpiPlain>(m, waves, grid, s, xq_tiled, w_tiles, (uint32_t)m, (uint32_t)n, n_tiles, k_tiles, e);
 }
 
-// Rows up to which the weight-stationary kernels are the faster ones against the large-tile GEMM on small tiles: a prompt pass of
-// four layers at 100 / 130 / 200 / 300 / 512 tokens, us, on them / on the GEMM: width 4096 529 / 613 / 695 / 846 / 1090 against 609 /
-// 640 / 678 / 794 / 940; width 2048 397 / 446 / 502 / 593 / 730 against 448 / 443 / 468 / 535 / 620.
-constexpr uint64_t kRowsMost = 160;
+// Rows up to which the weight-stationary kernels are the faster ones against the tiled GEMMs.
+// k a multiple of 128, against the large-tile GEMM: a prompt pass of four layers at 100 / 130 / 200 / 300 / 512 tokens, us, on them / on
+// the GEMM: width 4096 529 / 613 / 695 / 846 / 1090 against 609 / 640 / 678 / 794 / 940; width 2048 397 / 446 / 502 / 593 / 730 against 448
+// / 443 / 468 / 535 / 620.  The linears by themselves at 160 / 192 / 224 rows, with their quantizer: 4096 -> 768 14.8 / 15.6 / 18.1 against
+// 16.7 / 16.8 / 16.8, 3072 -> 4096 14.8 / 15.6 / 17.9 against 16.7 / 16.7 / 16.8; 2048 -> 768 13.8 / 14.2 / 16.5 against 13.9 / 13.9 / 14.0.
+// Other k, against the 128 x 128 kernel, which costs more the more columns there are: 1088 -> 256 at 161 / 200 / 240 / 320 rows 13.5 /
+// 16.0 / 16.3 / 19.2 against 15.3 / 15.2 / 15.4 / 15.6, 1088 -> 4096 14.0 / 16.6 / 17.0 / 20.0 against 17.8 / 18.7 / 19.3 / 21.9; 4160 ->
+// 1024 21.3 / 25.8 / 26.2 / 32.3 against 21.4 / 22.2 / 22.8 / 25.9, 4160 -> 4096 22.8 / 27.0 / 27.9 / 34.1 against 25.6 / 27.0 / 28.5 / 31.7;
+// with k over four blocks 10304 -> 512 at 130 / 160 / 200 / 300 rows 27.2 / 27.9 / 32.6 / 43.5 against 26.1 / 26.3 / 26.9 / 30.2, 10304 -> 4096
+// 33.2 / 34.1 / 39.0 / 51.8 against 34.4 / 35.7 / 37.9 / 48.6.
+inline uint64_t rows_most(uint64_t n_pad, uint64_t k_pad) {
+    if (k_pad % 128 == 0) return k_pad > 2048 && k_pad <= 4096 ? 192 : 160;
+    const uint64_t n = std::min<uint64_t>(n_pad, 4096);
+    return k_pad <= 4096 ? 192 + n / 32 : 144 + n / 48;
+}
 
 // The split-k form of the weight-stationary kernel (w8a8_wstat_ksplit_kernel): deep, narrow weights (k from 8192 up to
 // what four members x eight wavefronts x eight k-tiles hold, about one column tile per compute unit), more rows than
@@ -2096,9 +2107,9 @@ inline bool rows_ksplit_plan(uint64_t m, uint32_t n_tiles, uint32_t k_tiles, int
     // (k up to what the kernel without the split holds as well, so that a caller without a workspace still has a form)
     if (m <= 64 || n_tiles == 0 || k_tiles < 128 || k_tiles > 224) return false;
     // against the kernel without the split, us incl. the row quantizer at 65 / 128 rows: 14336 -> 4096 27.7 / 31.6 against 32.7 /
-    // 36.6; 8192 -> 4096 the kernel without the split is the faster one.  Against the large-tile GEMM: kRowsMost.
+    // 36.6; 8192 -> 4096 the kernel without the split is the faster one.  Against the tiled GEMMs: rows_most.
     if (g_rows_kernel != 3 && k_tiles < 160) return false;
-    if (g_rows_kernel != 3 && (m > kRowsMost || (uint64_t)n_tiles > 2 * (uint64_t)num_cus)) return false;
+    if (g_rows_kernel != 3 && (m > rows_most((uint64_t)n_tiles * 16, (uint64_t)k_tiles * 64) || (uint64_t)n_tiles > 2 * (uint64_t)num_cus)) return false;
     const uint32_t n_groups = (n_tiles + 3) / 4;
     if (n_groups > sk->n_counters) return false;
     p->n_groups = n_groups;
@@ -2122,7 +2133,7 @@ bool linear_w8a8_rows_applies(uint64_t m, uint64_t n_pad, uint64_t k_pad, int nu
     if (m <= 64 || n_tiles == 0 || k_tiles == 0 || k_tiles > 224) return false;
     if (g_rows_kernel == 2) return true;
     // what it costs is the m x k bytes of activations every block pulls from L2
-    return m <= kRowsMost && n_tiles <= 2 * (uint64_t)num_cus && m * k_pad <= (2ull << 20);
+    return m <= rows_most(n_pad, k_pad) && n_tiles <= 2 * (uint64_t)num_cus && m * k_pad <= (2ull << 20);
 }
 
 uint64_t linear_w8a8_rows_workspace_bytes(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, const SplitKArea *sk) {

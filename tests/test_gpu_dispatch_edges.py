@@ -195,6 +195,62 @@ def test_plan_names_the_wavefronts_that_are_launched(kind, mtb, ntb, waves, tune
     assert plan.waves == (waves if mtb == 16 and ntb != 8 else 8)
 
 
+@pytest.mark.parametrize("k,n,most", [(512, 16, 160), (1024, 520, 160), (2048, 768, 160), (2176, 1000, 192), (4096, 512, 192), (4096, 4096, 192),
+                                      (4224, 64, 160), (1088, 512, 208), (1088, 4112, 320), (4160, 1008, 165), (4160, 4096, 229), (8256, 80, 145), (10304, 80, 145), (10304, 2048, 186)])
+def test_rows_up_to_the_weight_stationary_line(k, n, most, tune):
+    """Linears of narrow and wide weights on both sides of the rows where the kernels change, k a multiple of 128 or not: the
+    large-tile GEMM behind the line wherever it can hold k, and the oracle's outputs bit for bit on every side."""
+    import fandhe_ai_amd as fa
+    import oracle_lib as o
+    import test_gpu_quantized as tq
+    be = ops()
+    rng = o.Rng(k + n)
+    x, w = rng.randn((most + 1, k)), rng.randn((k, n), std=0.05)
+    o.set_threads(8)
+    wq, ws = o.quantize_cols_i8(w)
+    _, want = o.linear_w8a8(x, wq, ws)
+    o.set_threads(1)
+    qw = be.import_quantized_weight(wq, ws)
+    for m in (most, most + 1):
+        plan = tq._gemm_plan(fa, be, m, qw)
+        assert plan.weight_stationary == (m <= most), m
+        assert (plan.big_ntb != 0) == (k % 128 == 0)
+        assert np.array_equal(be.download_owned(be.linear_w8a8(be.upload(np.ascontiguousarray(x[:m])), qw)), want[:m]), m
+
+
+@pytest.mark.parametrize("kind", ["int8", "e4m3"])
+@pytest.mark.parametrize("m,k,n", [(65, 128, 16), (193, 640, 100), (300, 1024, 520), (700, 2048, 1000), (4099, 256, 250)])
+def test_narrow_weights_on_large_tiles(m, k, n, kind):
+    """Weights of fewer columns than a tile has, and of a few tiles, many rows and few: sampled rows against exact sums (e4m3
+    products are exact in f32: within k roundings)."""
+    import fandhe_ai_amd as fa
+    import oracle_lib as o
+    import test_gpu_quantized as tq
+    be = ops()
+    rng = np.random.default_rng(m + n)
+    rows = rows_of_gemm(m)
+    if kind == "int8":
+        aq, wq = rng.integers(-127, 128, (m, k), dtype=np.int8), rng.integers(-127, 128, (k, n), dtype=np.int8)
+        sx, sw = rng.uniform(0.01, 0.05, m).astype(np.float32), rng.uniform(1e-4, 1e-3, n).astype(np.float32)
+        qw = be.import_quantized_weight(wq, sw)
+        assert tq._gemm_plan(fa, be, m, qw).big_ntb != 0
+        out, acc = be.gemm_w8a8(be.upload(aq), be.upload(sx), qw, fa.capi.F32, want_acc=True)
+        want = o.gemm_i8_i32(np.ascontiguousarray(aq[rows]), wq)
+        assert np.array_equal(be.download_owned(acc)[rows], want)
+        assert np.array_equal(be.download_owned(out)[rows], o.dequant_i32(want, np.ascontiguousarray(sx[rows]), sw))
+        return
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    aq, sa = be.quantize_tensor_e4m3(be.upload(x))
+    qw = be.quantize_weight(fa.DeviceBufferView(be.upload(w), 0, (k, n)), fa.capi.QW_E4M3_TENSOR)
+    assert tq._gemm_plan(fa, be, m, qw).big_ntb != 0
+    codes, sw = qw.export()
+    got = be.download_owned(be.gemm_e4m3(aq, sa, qw, fa.capi.F32))
+    a64, w64 = o.from_e4m3(be.download(aq)[rows]).astype(np.float64), o.from_e4m3(codes).astype(np.float64)
+    scale = float(be.download(sa)[0]) * float(sw[0])
+    bound = (np.abs(a64) @ np.abs(w64)) * scale * (k + 2) * 2.0 ** -24
+    assert np.all(np.abs(got[rows] - a64 @ w64 * scale) <= bound)
+
+
 @pytest.mark.parametrize("scale", [-0.25, 0.0, 0.0883883476, 3.0])
 @pytest.mark.parametrize("split,cols", [(1, 2), (1, 1), (2, 2)])
 @pytest.mark.parametrize("l_new,lens", [(70, [70, 101, 400]), (33, [33, 64, 65])])

@@ -824,8 +824,8 @@ def _fp8_rows_bound_check(tag, got, qa, qb, sa, sb, bias=None):
                                    (17, 200, 70), (300, 1024, 520), (1000, 1024, 9004)])
 def test_fp8_per_token_per_channel_linear(m, k, n):
     """fa_linear_e4m3: per-token e4m3 activations (row absmax / 448) against per-channel e4m3 weights (column
-    absmax / 448), dequantization fused.  Rows up to 64 take the weight-streaming kernel, 300 rows the 128 x 128
-    GEMM, 1000 x 9004 the large-tile GEMM; (17, 200, 70) has a k that is no multiple of the 128-wide tile."""
+    absmax / 448), dequantization fused.  Rows up to 64 take the weight-streaming kernel, more the large-tile GEMM, 300
+    also the 128 x 128 GEMM (key 4); (17, 200, 70) has a k that is no multiple of the 128-wide tile."""
     fa = _fa()
     be = ops()
     rng = np.random.default_rng(m * 7 + n)
@@ -846,11 +846,20 @@ def test_fp8_per_token_per_channel_linear(m, k, n):
     c2, s2 = qw2.export()
     assert np.array_equal(c2, want_wq) and np.array_equal(s2, want_sw)
     if m > 64:
-        plan = _gemm_plan(fa, be, m, qw)
-        assert (plan.big_ntb != 0) == (m == 1000)
+        assert _gemm_plan(fa, be, m, qw).big_ntb != 0
     dbias = fa.DeviceBufferView(be.upload(bias), 0, (n,))
     got = be.download_owned(be.linear_e4m3(dx, qw, out_dtype=fa.capi.F32))
     _fp8_rows_bound_check("%dx%dx%d" % (m, n, k), got, want_xq, want_wq, want_sx, want_sw)
+    if m == 300:
+        fa.check(fa.capi.lib.fa_set_tuning(4, 1))
+        try:
+            assert _gemm_plan(fa, be, m, qw).big_ntb == 0
+            assert np.array_equal(be.download_owned(be.linear_e4m3(dx, qw, out_dtype=fa.capi.F32)), got)      # the same order of the k sum
+            for b in (None, dbias):
+                small = be.download_owned(be.linear_e4m3(dx, qw, bias=b, out_dtype=fa.capi.F32))
+                _fp8_rows_bound_check("%dx%dx%d:128 tiles" % (m, n, k), small, want_xq, want_wq, want_sx, want_sw, None if b is None else bias)
+        finally:
+            fa.check(fa.capi.lib.fa_set_tuning(4, 0))
     got_b = be.download_owned(be.linear_e4m3(dx, qw, bias=dbias, out_dtype=fa.capi.F32))
     _fp8_rows_bound_check("%dx%dx%d+bias" % (m, n, k), got_b, want_xq, want_wq, want_sx, want_sw, bias)
     assert_bf16_rounding_of("linear_e4m3 bf16", be.download_owned(be.linear_e4m3(dx, qw, bias=dbias, out_dtype=fa.capi.BF16)),
