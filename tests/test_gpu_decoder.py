@@ -328,7 +328,8 @@ def test_prompt_prefill_matches_the_oracle_decoding_the_prompt_token_by_token(sh
 
 
 def test_prompt_pass_on_large_tiles_equals_the_pass_on_128_tiles_bit_for_bit():
-    """The projections of a prompt pass on the large-tile GEMM (forced: 256 x 224 tiles; its epilogue adds the
+    """The projections of a prompt pass on the large-tile GEMM (o and down forced to 224 columns, which the SwiGLU and
+    RoPE forms do not have: those on the tile that costs least; its epilogue adds the
     residual of the o and down projections from registers, four outputs of a row per lane, the gate | up projection
     takes SwiGLU into its epilogue and the q | k | v projection RoPE and the K / V append) against the same pass with
     SwiGLU left to the row quantizer and RoPE to its own pass, and against
@@ -346,9 +347,9 @@ def test_prompt_pass_on_large_tiles_equals_the_pass_on_128_tiles_bit_for_bit():
     try:
         # (every projection on the tiled GEMMs: at this width the weight-stationary kernel would take them, key 21 = 1)
         fa.check(lib.fa_set_tuning(21, 1))
-        # "big": large tiles, the gate | up GEMM with SwiGLU in its epilogue (256 x 256 tiles of eight gate and eight
-        # up column tiles, products written) and the q | k | v GEMM with RoPE, the bf16 rounding and the K / V append
-        # in its epilogue (a head per wavefront); "plain": large tiles, both left to their own passes (key 22 = 3);
+        # "big": large tiles, the gate | up GEMM with SwiGLU in its epilogue (gate and up column tiles side by side,
+        # products written) and the q | k | v GEMM with RoPE, the bf16 rounding and the K / V append
+        # in its epilogue; "plain": large tiles, both left to their own passes (key 22 = 3);
         # "small": the 128 x 128 kernel everywhere
         for form in ("big", "plain", "small"):
             fa.check(lib.fa_set_tuning(7, 0 if form == "small" else 14))

@@ -173,6 +173,97 @@ def test_fp8_gemm_on_every_tile(mtb, ntb, m, k, n, tune):
     assert np.all(np.abs(got[rows] - a64 @ w64 * scale) <= bound)
 
 
+TILES = [(8, 8), (12, 8), (16, 8), (8, 16), (12, 16), (16, 16), (12, 14), (16, 14)]
+STACKS = {"heads in pairs": dict(n_layers=2, d_model=512, n_heads=4, n_kv_heads=2, d_ffn=4096, vocab=700, batch=3, ctxs=[0, 9, 40]),
+          "an odd sum of heads": dict(n_layers=2, d_model=384, n_heads=3, n_kv_heads=1, d_ffn=1152, vocab=700, batch=3, ctxs=[0, 9, 40])}
+_prompts = {}
+
+
+def prompt_pass(stack, l_new):
+    """Logits, tokens and cache rows behind a prompt pass, as the tuning keys are."""
+    import test_gpu_decoder as td
+    if (stack, l_new) not in _prompts:
+        shape = STACKS[stack]
+        m = td.build_model(seed=77, steps=l_new + 2, **shape)
+        _prompts[stack, l_new] = m, td.o.Rng(6).randint(0, shape["vocab"], 3 * l_new).astype(np.int32).reshape(3, l_new)
+    m, prompt = _prompts[stack, l_new]
+    dec = td.GpuDecoder(ops(), m)
+    dec.prefill(prompt)
+    out = [dec.logits().copy(), dec.tokens().copy()] + [x.copy() for i in range(2) for x in dec.kv_pool(i)]
+    dec.close()
+    return out
+
+
+@pytest.mark.parametrize("l_new", [67, 100], ids=["201 rows", "300 rows"])
+@pytest.mark.parametrize("stack", sorted(STACKS))
+def test_prompt_pass_on_every_tile(stack, l_new, tune):
+    """The epilogues of a prompt pass - the residual of the o and down projections (k shared by blocks on the narrow tiles among
+    them), SwiGLU, RoPE with the K / V append on a head's 128 columns and on two heads' - on every tile of the large-tile GEMM: bit for
+    bit the pass on the 128 x 128 kernel with SwiGLU and RoPE in passes of their own."""
+    import fandhe_ai_amd as fa
+    import test_gpu_quantized as tq
+    be = ops()
+    tune(21, 1)                                            # no weight-stationary kernel
+    tune(4, 1)
+    tune(22, 3)
+    want = prompt_pass(stack, l_new)
+    assert np.all(np.isfinite(want[0])) and np.any(want[0] != 0)
+    tune(4, 0)
+    tune(22, 0)
+    ff, d = STACKS[stack]["d_ffn"], STACKS[stack]["d_model"]
+    down = be.quantize_weight(fa.DeviceBufferView(be.upload(np.ones((ff, d), np.float32)), 0, (ff, d)))
+    for mtb, ntb in TILES:
+        tune(37, mtb)
+        tune(7, ntb)
+        plan = tq._gemm_plan(fa, be, 3 * l_new, down)
+        assert (plan.big_mtb, plan.big_ntb) == (mtb, ntb) and (plan.share > 1) == (ntb == 8 and ff == 4096)
+        for x, y in zip(want, prompt_pass(stack, l_new)):
+            assert np.array_equal(x, y), (mtb, ntb)
+
+
+BF16_STACKS = {
+    "nugelix": lambda: lc.config([lc.latent(heads=4, dim=32, rot=16, vdim=32, q_rank=64, kv_rank=64, window=100, mlp=lc.glu(ff=320)),
+                                  lc.delta(heads=4, kv_heads=2, dim=32, vdim=64)], width=256),
+    "zoferax": lambda: lc.zoferax([lc.attention(heads=8, kv_heads=2, dim=32, vdim=32, mlp=lc.experts(5, 2, ff=256))], width=256),
+    "bubetar": lambda: lc.bubetar([lc.parallel(mlp=lc.dense(ff=320)), lc.parallel_2(mlp=lc.dense(ff=192))], width=256),
+    "lugipel": lambda: lc.lugipel([lc.sigmoid_attention(mlp=lc.dense(ff=320)), lc.mingru(256, mlp=lc.scored(3, 1, None, 2, ff=256))], width=256),
+}
+
+
+@pytest.mark.parametrize("name", sorted(BF16_STACKS))
+def test_bf16_linears_on_every_tile(name, tune):
+    """The bf16 linears of a pass of 390 rows, experts' rows in groups among them, on every tile that their epilogues have: the order
+    of the sums over k is the same on all of them, and so are the logits, bit for bit; near the oracle's and those of the 128 x 128
+    kernel, which sums in another order."""
+    cfg = BF16_STACKS[name]()
+    w, lens = lc.weights(cfg, 5), [260, 33, 97]
+    toks = [lc.tokens(cfg, n, 40 + n) for n in lens]
+    dec = lc.make_decoder(ops(), cfg, w, "bfloat16", max_tokens=1024, max_batch=3)
+    table = np.full((3, dec.cfg.max_blocks_per_seq), 0xFFFFFFFF, dtype=np.uint32)
+    table[:, :20] = np.arange(60).reshape(20, 3).T
+
+    def logits():
+        dec.set_sequences(table, [0] * 3)
+        return dec.forward(toks, [list(range(n)) for n in lens])
+
+    got = {}
+    for tile in TILES:
+        tune(37, tile[0])
+        tune(7, tile[1])
+        got[tile] = logits()
+        assert np.array_equal(got[tile], got[TILES[0]]), tile
+    tune(37, 0)
+    tune(7, 0)
+    assert np.array_equal(logits(), got[TILES[0]])
+    want = np.concatenate([oracle.forward(cfg, w, t) for t in toks])
+    tune(29, 5 if "experts" in str(cfg) else 2)
+    other = logits()
+    dec.close()
+    # the bf16 tests' bar for the worst row is 0.12; half of it for the middle one
+    near = lambda x: np.median(np.sqrt(np.mean((x - want) ** 2, axis=1))) / np.sqrt(np.mean(want ** 2))
+    assert near(got[TILES[0]]) < 0.06 and abs(near(other) - near(got[TILES[0]])) < 0.02, (near(got[TILES[0]]), near(other))
+
+
 @pytest.mark.parametrize("mtb,ntb,waves", [(8, 16, 4), (12, 14, 16), (16, 8, 4), (16, 14, 4), (16, 16, 16), (8, 8, 4)])
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
 def test_plan_names_the_wavefronts_that_are_launched(kind, mtb, ntb, waves, tune):
