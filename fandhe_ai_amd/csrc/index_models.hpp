@@ -29,8 +29,8 @@ FA_HD int big_stages_b(int mtb, int ntb) { return (3 * mtb + 3 * ntb) * kBigTile
 template <int NTB, int MTB = 16>
 struct BigLds {
     static constexpr int a_stage = MTB * kBigTile, b_stage = NTB * kBigTile;
-    static constexpr int b_base = kBigStagesA * a_stage;
-    static constexpr int bytes = b_base + kBigStagesB * b_stage;
+    static constexpr int b_base = kBigStagesA * a_stage, stages_b = big_stages_b(MTB, NTB);
+    static constexpr int bytes = b_base + stages_b * b_stage;
 };
 
 // Blocks of one XCD (the hardware deals consecutive ids round-robin over 8 XCDs) take consecutive tiles, m fastest.

@@ -1024,7 +1024,7 @@ void allow_lds(F f, size_t bytes) {
 template <bool FP8, int NTB, int WM, int MTB, typename Epi>
 void launch_big_tile(const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, uint32_t n_blocks,
                      unsigned grid, const Epi &e, hipStream_t s) {
-    constexpr size_t smem = (3 * MTB + ixm::big_stages_b(MTB, NTB) * NTB) * 2048;
+    constexpr size_t smem = ixm::BigLds<NTB, MTB>::bytes;
     static bool configured = false;
     if (!configured) allow_lds(&gemm_mfma_big_kernel<FP8, NTB, WM, Epi, MTB>, smem);
     configured = true;

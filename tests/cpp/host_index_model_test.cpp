@@ -2,7 +2,7 @@
 // themselves call).  No device: every block, wavefront, lane, load and stage of every instantiation is walked on
 // the host and checked for bounds, for agreement between where a stage's bytes are written and where the operand
 // reads expect them, and for every output being written exactly once.
-//   large-tile GEMM   : e4m3 / int8 x 14 / 16 column tiles x 4 / 8 / 16 wavefronts
+//   large-tile GEMM   : e4m3 / int8 (bf16 moves the same bytes) x 8 / 14 / 16 column tiles x 8 / 12 / 16 row tiles x 4 / 8 / 16 wavefronts
 //   streamed attention: ranges, segments and partial-result slots against the merge's expectation, ragged lengths
 //   split-k linears   : groups on one XCD, k ranges, workspace offsets
 #include <cstdio>
@@ -31,37 +31,45 @@ struct Tag {
     int row = -1, kbyte = -1;
 };
 
-template <bool FP8, int NTB, int WM>
+template <bool FP8, int NTB, int WM, int MTB = 16>
 static void gemm_case() {
-    constexpr int NWAVES = 2 * WM, TPW = 16 / NWAVES, AI = 16 / WM, WNT = NTB / 2;
-    using L = BigLds<NTB>;
+    constexpr int NWAVES = 2 * WM, NLDA = big_a_loads<MTB, NWAVES>(), TPWB = (NTB + NWAVES - 1) / NWAVES, AI = MTB / WM, WNT = NTB / 2, ROWS = MTB * 16;
+    using L = BigLds<NTB, MTB>;
+    constexpr int NSB = L::stages_b;
     static_assert(L::bytes <= 160 * 1024, "stages exceed the LDS of a compute unit");
-    // one stage's loads of every wavefront into slot `slot` (A) / `slot % 2` (B)
+    static_assert(L::bytes == L::b_base + NSB * L::b_stage && (NSB == 2 || NSB == 3), "all stages of B are counted");
+    static_assert(AI * WM == MTB && WNT * 2 == NTB, "whole tiles per wavefront");
+    static_assert((NSB == 3 ? NLDA + 2 * TPWB : NLDA) <= 15, "loads that a wait leaves in flight: four bits of its immediate");
+    // one stage's loads of every wavefront into slot `slot` (A) / `slot % NSB` (B)
     for (int slot = 0; slot < kBigStagesA; ++slot) {
         std::vector<Tag> lds(L::bytes);
         std::vector<int> writes(L::bytes, 0);
-        for (int wave = 0; wave < NWAVES; ++wave)
-            for (int i = 0; i < TPW; ++i)
+        for (int wave = 0; wave < NWAVES; ++wave) {
+            for (int idx = 0; idx < NLDA; ++idx)
+                for (int lane = 0; lane < 64; ++lane) {
+                    // A: lane fetches 16 bytes of row (tile * 16 + lane / 4) at big_a_src_byte, lands at slice + lane * 16
+                    int tile, h;
+                    big_a_load<MTB, NWAVES>(wave, idx, &tile, &h);
+                    CHECK(tile >= 0 && tile < MTB && (h == 0 || h == 1));
+                    const int row = tile * 16 + big_a_row(lane), src = big_a_src_byte<FP8>(lane, h);
+                    CHECK(row < ROWS && src >= 0 && src % 16 == 0 && src + 16 <= kBigTk);
+                    const int dst = big_a_lds_slice<NTB, MTB>(slot, tile, h) + lane * 16;
+                    CHECK(dst >= slot * L::a_stage && dst + 16 <= (slot + 1) * L::a_stage);
+                    for (int b = 0; b < 16; ++b) {
+                        lds[dst + b] = Tag{row, src + b};
+                        writes[dst + b] += 1;
+                    }
+                }
+            for (int i = 0; i < TPWB; ++i)
                 for (int h = 0; h < 2; ++h)
                     for (int lane = 0; lane < 64; ++lane) {
-                        // A: lane fetches 16 bytes of row (tile * 16 + lane / 4) at big_a_src_byte, lands at slice + lane * 16
-                        const int tile = big_a_tile<NWAVES>(wave, i);
-                        CHECK(tile >= 0 && tile < 16);
-                        const int row = tile * 16 + big_a_row(lane), src = big_a_src_byte<FP8>(lane, h);
-                        CHECK(row < kBigRows && src >= 0 && src % 16 == 0 && src + 16 <= kBigTk);
-                        const int dst = big_a_lds_slice<NTB>(slot, tile, h) + lane * 16;
-                        CHECK(dst >= slot * L::a_stage && dst + 16 <= (slot + 1) * L::a_stage);
-                        for (int b = 0; b < 16; ++b) {
-                            lds[dst + b] = Tag{row, src + b};
-                            writes[dst + b] += 1;
-                        }
                         // B: lane's 16 bytes of slice h of the stage's weight tile, lands at slice + lane * 16
                         const int bt = big_b_tile<NTB, NWAVES>(wave, i);
                         CHECK(bt >= 0 && bt < NTB);
                         const int bsrc = big_b_src_byte<FP8>(lane, h);
                         CHECK(bsrc >= 0 && bsrc + 16 <= kBigTile);
-                        const int bslot = slot % kBigStagesB;
-                        const int bdst = big_b_lds_slice<NTB>(bslot, bt, h) + lane * 16;
+                        const int bslot = slot % NSB;
+                        const int bdst = big_b_lds_slice<NTB, MTB>(bslot, bt, h) + lane * 16;
                         CHECK(bdst >= L::b_base + bslot * L::b_stage && bdst + 16 <= L::b_base + (bslot + 1) * L::b_stage);
                         for (int b = 0; b < 16; ++b) {
                             // a tile moved twice (14-tile blocks) must bring the same bytes to the same place
@@ -70,13 +78,14 @@ static void gemm_case() {
                             writes[bdst + b] += 1;
                         }
                     }
+        }
         // every byte of the stage's A region exactly once, every byte of its B region at least once
         for (int b = 0; b < L::a_stage; ++b) CHECK(writes[slot * L::a_stage + b] == 1);
-        for (int b = 0; b < L::b_stage; ++b) CHECK(writes[L::b_base + (slot % kBigStagesB) * L::b_stage + b] >= 1);
-        // every source byte of the stage reaches LDS: 256 rows x 128 bytes of A
+        for (int b = 0; b < L::b_stage; ++b) CHECK(writes[L::b_base + (slot % NSB) * L::b_stage + b] >= 1);
+        // every source byte of the stage reaches LDS: the block's rows x 128 bytes of A
         std::set<std::pair<int, int>> seen;
         for (int b = 0; b < L::a_stage; ++b) seen.insert({lds[slot * L::a_stage + b].row, lds[slot * L::a_stage + b].kbyte});
-        CHECK((int)seen.size() == kBigRows * kBigTk);
+        CHECK((int)seen.size() == ROWS * kBigTk);
 
         // operand reads.  A: lane (g, r) of row tile t wants row 16 t + r and, e4m3, k bytes 32 g + 16 sub .. + 15;
         // int8, k bytes 64 sub + 16 g .. + 15.  16-byte reads must also be bank-conflict free.
@@ -115,7 +124,7 @@ static void gemm_case() {
             for (int j = 0; j < WNT; ++j)
                 for (int h = 0; h < 2; ++h)
                     for (int lane = 0; lane < 64; ++lane) {
-                        const int bslot = slot % kBigStagesB;
+                        const int bslot = slot % NSB;
                         const int off = L::b_base + bslot * L::b_stage + big_b_frag_off<NTB>(wn, j, h, lane);
                         CHECK(off + 16 <= L::b_base + (bslot + 1) * L::b_stage);
                         for (int b = 0; b < 16; ++b) {
@@ -124,21 +133,21 @@ static void gemm_case() {
                         }
                     }
     }
-    // outputs: every element of the 256 x NTB * 16 tile exactly once, four consecutive columns per lane and tile
-    std::vector<int> hit(kBigRows * NTB * 16, 0);
+    // outputs: every element of the tile exactly once, four consecutive columns per lane and tile
+    std::vector<int> hit(ROWS * NTB * 16, 0);
     for (int wm = 0; wm < WM; ++wm)
         for (int wn = 0; wn < 2; ++wn)
             for (int i = 0; i < AI; ++i)
                 for (int j = 0; j < WNT; ++j)
                     for (int lane = 0; lane < 64; ++lane) {
                         int row0, col0;
-                        big_out_elem<NTB, WM>(wm, wn, i, j, 0, lane, &row0, &col0);
+                        big_out_elem<NTB, WM, MTB>(wm, wn, i, j, 0, lane, &row0, &col0);
                         CHECK(col0 % 4 == 0);                  // the 8 / 16-byte store is aligned
                         for (int e = 0; e < 4; ++e) {
                             int row, col;
-                            big_out_elem<NTB, WM>(wm, wn, i, j, e, lane, &row, &col);
+                            big_out_elem<NTB, WM, MTB>(wm, wn, i, j, e, lane, &row, &col);
                             CHECK(row == row0 && col == col0 + e);
-                            CHECK(row >= 0 && row < kBigRows && col >= 0 && col < NTB * 16);
+                            CHECK(row >= 0 && row < ROWS && col >= 0 && col < NTB * 16);
                             hit[row * NTB * 16 + col] += 1;
                         }
                     }
@@ -341,26 +350,62 @@ static void swiglu_tile_case(uint32_t f_tiles) {
     CHECK(seen.size() == 2 * (size_t)f_tiles);
 }
 
+// RoPE form on 128 columns: a block's eight column tiles are a head's, each taken once, and the rotate-half partners of
+// accumulator tile j (64 dims further) sit in accumulator tile j + 2 of the same wavefront column.
+static void rope_tile_case(uint32_t heads) {
+    std::set<uint32_t> seen;
+    for (uint32_t hd = 0; hd < heads; ++hd)
+        for (int wn = 0; wn < 2; ++wn)
+            for (int j = 0; j < 2; ++j) {
+                const uint32_t lo = big_rope_tile(hd, wn * 4 + j), hi = big_rope_tile(hd, wn * 4 + j + 2);
+                CHECK(lo == hd * 8 + (uint32_t)(wn * 2 + j));              // the dims the epilogue gives it: 16 (2 wn + j) ..
+                CHECK(hi == lo + 4);
+                CHECK(seen.insert(lo).second && seen.insert(hi).second);
+            }
+    CHECK(seen.size() == 8 * (size_t)heads);
+}
+
+// Stages in flight: slot of stage ks (A, and B with three stages: ks % 3; B with two: ks % 2).  While stage ks is multiplied,
+// A of ks + 2 and B of ks + 1 (two stages) or ks + 2 (three) are requested: into slots that hold neither ks nor what comes next.
+static void stage_ring_case(int nsb) {
+    for (int ks = 0; ks < 60; ++ks) {
+        const int slot_a = ks % 3, slot_a2 = slot_a == 0 ? 2 : slot_a - 1;
+        CHECK(slot_a2 == (ks + 2) % 3 && slot_a2 != slot_a && slot_a2 != (ks + 1) % 3);
+        const int ahead = nsb == 3 ? ks + 2 : ks + 1, to = nsb == 3 ? slot_a2 : (ks % 2) ^ 1;
+        CHECK(to == ahead % nsb && to != ks % nsb);
+        if (nsb == 3) CHECK(to != (ks + 1) % 3);
+    }
+}
+
+template <bool FP8>
+static void gemm_cases() {
+    gemm_case<FP8, 16, 4, 16>();
+    gemm_case<FP8, 16, 4, 12>();
+    gemm_case<FP8, 16, 4, 8>();
+    gemm_case<FP8, 14, 4, 16>();
+    gemm_case<FP8, 14, 4, 12>();
+    gemm_case<FP8, 8, 4, 16>();
+    gemm_case<FP8, 8, 4, 12>();
+    gemm_case<FP8, 8, 4, 8>();
+    gemm_case<FP8, 14, 2>();
+    gemm_case<FP8, 16, 2>();
+    gemm_case<FP8, 14, 8>();
+    gemm_case<FP8, 16, 8>();
+}
+
 int main() {
+    rope_tile_case(1);
+    rope_tile_case(13);
+    stage_ring_case(2);
+    stage_ring_case(3);
     swiglu_tile_case<16>(8);
     swiglu_tile_case<16>(896);
     swiglu_tile_case<8>(8);
     swiglu_tile_case<8>(896);
     rows_ksplit_cases();
     decode_a_cases();
-    gemm_case<true, 14, 4>();
-    gemm_case<true, 16, 4>();
-    gemm_case<false, 14, 4>();
-    gemm_case<false, 16, 4>();
-    gemm_case<false, 8, 4>();
-    gemm_case<true, 14, 2>();
-    gemm_case<true, 16, 2>();
-    gemm_case<false, 14, 2>();
-    gemm_case<false, 16, 2>();
-    gemm_case<true, 14, 8>();
-    gemm_case<true, 16, 8>();
-    gemm_case<false, 14, 8>();
-    gemm_case<false, 16, 8>();
+    gemm_cases<true>();
+    gemm_cases<false>();
     gemm_block_map();
     stream_cases();
     ksplit_cases();
