@@ -89,7 +89,6 @@ fa_status fa_set_tuning(int32_t key, int32_t value) {
         case 8: fa::g_prefill_generic = value; return FA_OK;
         case 9: k::g_gemm_split_fill = value; return FA_OK;
         case 10: fa::g_prefill_block_form = value; return FA_OK;
-        case 11: return FA_OK;            // blocks have four wavefronts
         case 12: fa::g_prefill_block_split = value; return FA_OK;
         case 13: k::g_gemm_f32_form = value; return FA_OK;
         case 14: k::g_weight_prefetch = value; return FA_OK;

@@ -68,7 +68,7 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  *        for (default 2);
  * key 10: form of the attention with more than one new token per row: 1 always the
  *        streamed form, 2 always the block form, 0 by shape;
- * key 11: without effect;
+ * (key 11 is not in use;)
  * key 12: upper bound of the blocks that share the cache walk of one tile of new tokens
  *        in the block form (1: never split; 0 by shape);
  * key 13: kernel of the order-fixed f32 GEMM (gemm_device / linear_forward_device): 1 the few-rows vector

@@ -42,6 +42,15 @@ def test_library_exports_every_declared_symbol():
     assert fa.capi.lib.fa_status_name(fa.capi.UNSUPPORTED) == b"Unsupported"
 
 
+def test_tuning_keys_are_the_documented_ones():
+    """A key that does nothing would look like a kernel form that is covered."""
+    import fandhe_ai_amd as fa
+    header = open(os.path.join(ROOT, "include", "fandhe_rocm_bench.h")).read()
+    documented = {int(k) for k in re.findall(r"\bkey (\d+):", header)}
+    accepted = {k for k in range(-1, 100) if fa.capi.lib.fa_set_tuning(k, 0) == 0}
+    assert accepted == documented, accepted ^ documented
+
+
 def test_validators_follow_the_reference_tables():
     # crates/tensor-core/src/paged_kv.rs:387-521 through the C ABI
     fa = _fa()

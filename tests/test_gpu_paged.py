@@ -248,7 +248,7 @@ PREFILL_CASES = [
     (32, 8, 16, [16, 17, 64]), (32, 8, 17, [17, 31, 200]), (32, 8, 37, [37, 38, 500]), (32, 8, 200, [200, 333, 777]),
     (8, 8, 19, [19, 40]), (8, 4, 9, [9, 100]), (16, 2, 11, [11, 64]), (16, 1, 6, [6, 90]), (6, 2, 13, [13, 70]),
     (5, 1, 7, [7, 40]),
-    # several tiles of the block form (256 / group new tokens per tile), ragged last tiles
+    # several tiles of the block form (128 / group or 64 / group new tokens per tile), ragged last tiles
     (32, 8, 300, [300, 1000]), (8, 8, 600, [600, 700]), (16, 2, 100, [100, 250]), (16, 1, 50, [50, 51, 333]),
     (4, 2, 129, [129, 640]),
 ]
@@ -280,18 +280,17 @@ def test_bf16_prefill_on_the_streaming_kernel_against_the_oracle(heads, kv_heads
         got = be.download_owned(be.paged_attention_forward(dq, dk, dv, tables, seq_lens, args, out_dtype=fa.capi.F32))
         assert_parity("PAGED_PREFILL_PARITY", f"H{heads}/{kv_heads}:L{l_new}:waves{waves}", got, want)
     fa.check(fa.capi.lib.fa_set_tuning(2, 0))
-    # the block form (one block per tile of 256 / group new tokens walks the cache once), forced for every
+    # the block form (one block per tile of new tokens walks the cache once), forced for every
     # group size it supports whatever the shape heuristics would choose
     fa.check(fa.capi.lib.fa_set_tuning(10, 2))
-    # tiles of 256 / group and of 128 / group new tokens; the smaller blocks also with the cache walk of a tile
-    # shared by several blocks (as many as the shape allows, or two) and a merge pass
-    # (cols: 32 columns per wavefront, key 23 = 2, or 16, key 23 = 1: half the multiplies per step, twice the blocks)
-    for block_waves, split, cols in ((8, 1, 2), (4, 1, 2), (4, 1, 1), (4, 0, 2), (4, 2, 2)):
-        fa.check(fa.capi.lib.fa_set_tuning(11, block_waves))
+    # tiles of 128 / group and of 64 / group new tokens (cols: 32 columns per wavefront, key 23 = 2, or 16, key 23 = 1:
+    # half the multiplies per step, twice the blocks); the larger ones also with the cache walk of a tile
+    # shared by several blocks (as many as the shape allows, two or three) and a merge pass
+    for split, cols in ((1, 2), (1, 1), (0, 2), (2, 2), (3, 2)):
         fa.check(fa.capi.lib.fa_set_tuning(12, split))
         fa.check(fa.capi.lib.fa_set_tuning(23, cols))
         blk = be.download_owned(be.paged_attention_forward(dq, dk, dv, tables, seq_lens, args, out_dtype=fa.capi.F32))
-        assert_parity("PAGED_PREFILL_PARITY", f"H{heads}/{kv_heads}:L{l_new}:block form, {block_waves} wavefronts, split {split}, cols {cols}", blk, want)
+        assert_parity("PAGED_PREFILL_PARITY", f"H{heads}/{kv_heads}:L{l_new}:block form, split {split}, cols {cols}", blk, want)
         blk_bf = be.download_owned(be.paged_attention_forward(dq, dk, dv, tables, seq_lens, args))
         assert_bf16_rounding_of("paged prefill bf16, block form", blk_bf, blk)
         blk_dev = be.download_owned(be.paged_attention_forward_device(dq, dk, dv, be.upload(tables), be.upload(seq_lens), args,
@@ -303,7 +302,6 @@ def test_bf16_prefill_on_the_streaming_kernel_against_the_oracle(heads, kv_heads
         for h in range(heads):
             gq = h // (heads // kv_heads)
             assert np.array_equal(blk_bf[0, 0, h * 128:(h + 1) * 128], vp[tables[0, 0], 0, gq * 128:(gq + 1) * 128])
-    fa.check(fa.capi.lib.fa_set_tuning(11, 0))
     fa.check(fa.capi.lib.fa_set_tuning(12, 0))
     fa.check(fa.capi.lib.fa_set_tuning(23, 0))
     # whatever the shape selects by itself (host tables: the longest row is known; device tables: the table width)
@@ -441,8 +439,7 @@ def test_block_form_prefill_flags_violations_per_column():
     bad_l[2] = l_new - 1                            # row 2: fewer positions than new tokens
     fa.check(fa.capi.lib.fa_set_tuning(10, 2))
     try:
-        for block_waves, split, cols in ((4, 1, 2), (4, 1, 1), (4, 0, 2), (8, 1, 2)):
-            fa.check(fa.capi.lib.fa_set_tuning(11, block_waves))
+        for split, cols in ((1, 2), (1, 1), (0, 2), (2, 2)):
             fa.check(fa.capi.lib.fa_set_tuning(12, split))
             fa.check(fa.capi.lib.fa_set_tuning(23, cols))
             got = be.download_owned(be.paged_attention_forward_device(
@@ -453,13 +450,12 @@ def test_block_form_prefill_flags_violations_per_column():
             assert np.all(np.isnan(got[1, 12:])) and np.all(np.isnan(got[2]))
     finally:
         fa.check(fa.capi.lib.fa_set_tuning(10, 0))
-        fa.check(fa.capi.lib.fa_set_tuning(11, 0))
         fa.check(fa.capi.lib.fa_set_tuning(12, 0))
         fa.check(fa.capi.lib.fa_set_tuning(23, 0))
 
 
 def test_bf16_prefill_properties_at_prompt_size():
-    """4 rows x 2048 new tokens, 32 / 8 heads (the prompt pass of the benchmark): both block sizes of the block
+    """4 rows x 2048 new tokens, 32 / 8 heads (the prompt pass of the benchmark): both column counts of the block
     form and the streamed form against each other and against one-token decode calls on sampled positions, plus
     the invariances that hold at any size."""
     fa = _fa()
@@ -478,21 +474,21 @@ def test_bf16_prefill_properties_at_prompt_size():
     lib = fa.capi.lib
     outs = {}
     try:
-        for name, form, waves in (("block8", 2, 8), ("block4", 2, 4), ("streamed", 1, 0), ("by shape", 0, 0)):
+        for name, form, cols in (("block", 2, 2), ("narrow", 2, 1), ("streamed", 1, 0), ("by shape", 0, 0)):
             fa.check(lib.fa_set_tuning(10, form))
-            fa.check(lib.fa_set_tuning(11, waves))
+            fa.check(lib.fa_set_tuning(23, cols))
             outs[name] = be.download_owned(be.paged_attention_forward(dq, dk, dv, tables, seq_lens, args, out_dtype=fa.capi.F32))
             assert np.all(np.isfinite(outs[name])), name
         fa.check(lib.fa_set_tuning(10, 0))
-        fa.check(lib.fa_set_tuning(11, 0))
-        for name in ("block8", "block4", "by shape"):
+        fa.check(lib.fa_set_tuning(23, 0))
+        for name in ("block", "narrow", "by shape"):
             assert_parity("PREFILL_FORMS", f"{name} vs streamed", outs[name], outs["streamed"])
-        # sampled positions against one-token decode calls over the same cache (tile edges of both block sizes)
+        # sampled positions against one-token decode calls over the same cache (tile edges of both column counts)
         for t in (0, 1, 31, 32, 63, 64, 1000, 2047):
             lens_t = (seq_lens - l_new + t + 1).astype(np.uint32)
             dec = be.download_owned(be.paged_attention_forward(be.upload(np.ascontiguousarray(q[:, t:t + 1, :])), dk, dv,
                                                                tables, lens_t, args1, out_dtype=fa.capi.F32))
-            for name in ("block8", "block4"):
+            for name in ("block", "narrow"):
                 assert_parity("PREFILL_VS_DECODE", f"{name}:t{t}", outs[name][:, t:t + 1, :], dec)
         # the oracle on the first 40 tokens of the row with the longest cache
         oargs = o.paged_args(num_blocks, 16, e_kv, 1, 40, heads, max_blocks, args.scale, kv_heads)
@@ -501,7 +497,7 @@ def test_bf16_prefill_properties_at_prompt_size():
                                           np.array([lens[1] - l_new + 40], np.uint32), oargs)
         o.set_threads(1)
         assert rc == 0
-        assert_parity("PAGED_PREFILL_PARITY", "row 1, tokens 0..39", outs["block8"][1:2, :40], want)
+        assert_parity("PAGED_PREFILL_PARITY", "row 1, tokens 0..39", outs["block"][1:2, :40], want)
         got = outs["by shape"]
         # every output is a convex combination of V rows of its kv head
         used = tables[tables != U32MAX]
@@ -525,7 +521,7 @@ def test_bf16_prefill_properties_at_prompt_size():
         assert np.allclose(got3, 1.5, rtol=1e-5, atol=0)
     finally:
         fa.check(lib.fa_set_tuning(10, 0))
-        fa.check(lib.fa_set_tuning(11, 0))
+        fa.check(lib.fa_set_tuning(23, 0))
 
 
 def test_bf16_prefill_few_new_tokens_over_a_long_cache_share_the_walk():
