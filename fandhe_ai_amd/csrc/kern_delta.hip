@@ -1181,8 +1181,8 @@ void launch_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr
         configure(&lightning_chunk_kernel<T, KT>);
         lightning_chunk_kernel<T, KT><<<dim3(p.slots, sh.heads), 256, lds, s>>>(sh, io, rr, frags, decay, p.frags);
     }
-    // the line between the two scans: up to two column tiles per compute unit of 256 (measured: see delta_scan_split_kernel)
-    if (g_delta_form == 2 || (g_delta_form != 3 && (uint64_t)p.vt * sh.heads * rr.batch <= 512)) {
+    // the line between the two scans: up to two column tiles per compute unit (measured: see delta_scan_split_kernel)
+    if (g_delta_form == 2 || (g_delta_form != 3 && (uint64_t)p.vt * sh.heads * rr.batch <= 2 * compute_units())) {
         delta_scan_split_kernel<KT, KIND><<<dim3((sh.heads + 7) / 8 * 8 * p.vt, rr.batch), scan_waves(KT) * 64, 0, s>>>(sh, io, rr, frags, decay, io.raw, p.vt, p.frags);
     } else {
         // wavefronts of a block share a head's fragments; fewer per block where there are few blocks
@@ -1244,7 +1244,7 @@ StepPlan step_plan(const DeltaShape &sh, uint32_t batch) {
         p.cg_log2 = sh.dim > 128 ? 4 : 5;
         p.parts = (sh.vdim + (4u << p.cg_log2) - 1) / (4u << p.cg_log2);
     }
-    p.small = (uint64_t)batch * sh.heads * p.parts > 256;
+    p.small = (uint64_t)batch * sh.heads * p.parts > compute_units();
     return p;
 }
 

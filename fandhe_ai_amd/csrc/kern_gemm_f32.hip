@@ -204,17 +204,6 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-int compute_units() {
-    static int cus = 0;
-    if (cus == 0) {
-        int dev = 0;
-        hipDeviceProp_t p;
-        if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&p, dev) == hipSuccess) cus = p.multiProcessorCount;
-        if (cus <= 0) cus = 256;
-    }
-    return cus;
-}
-
 }  // namespace
 
 int g_gemm_f32_form = 0;      // 0 by shape, 1 the few-rows kernel, 2 the matrix-core kernel
@@ -226,7 +215,7 @@ int gemm_f32_form(uint64_t m, uint64_t n, uint64_t k) {
     // Both forms run a chain of k steps per output; what differs is the clocks a step occupies its SIMD for (two
     // 64-clock matrix instructions per 64 x 64 tile against SR vector instructions of 4 clocks per 64 x SR
     // outputs) and how many rounds the launch needs to seat its wavefronts (one per SIMD at a time).
-    const uint64_t simds = 4ull * (uint64_t)compute_units();
+    const uint64_t simds = 4ull * compute_units();
     const uint64_t mfma_waves = tiles_m * tiles_n * 4, rows_waves = ((m + SR - 1) / SR) * ((n + 63) / 64);
     const uint64_t mfma_cost = ((mfma_waves + simds - 1) / simds) * 128, rows_cost = ((rows_waves + simds - 1) / simds) * 4 * SR;
     return rows_cost < mfma_cost ? 1 : 2;

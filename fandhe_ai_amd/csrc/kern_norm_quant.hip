@@ -622,11 +622,12 @@ template <typename F>
 static bool wide_form(uint64_t rows, uint64_t width, F &&go) {
     using std::integral_constant;
     if (g_rows_wide == 1 || width > 16384) return false;
-    if (rows <= 256 && width > 1024) {
+    const uint64_t cus = compute_units();
+    if (rows <= cus && width > 1024) {
         if (width <= 4096) go(integral_constant<int, 1024>{}, integral_constant<int, 1>{});
         else if (width <= 8192) go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
         else go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
-    } else if (rows > 512 ? width > 8192 : width > 1024) {
+    } else if (rows > 2 * cus ? width > 8192 : width > 1024) {
         if (width <= 2048) go(integral_constant<int, 512>{}, integral_constant<int, 1>{});
         else if (width <= 4096) go(integral_constant<int, 512>{}, integral_constant<int, 2>{});
         else if (width <= 8192) go(integral_constant<int, 512>{}, integral_constant<int, 4>{});

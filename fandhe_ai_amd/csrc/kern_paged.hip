@@ -1401,7 +1401,7 @@ int g_prefill_block_split = 0;    // upper bound of the blocks that share one ti
 int g_prefill_block_cols = 0;     // columns per wavefront of the block form: 0 by shape, 1: 16 whenever allowed, 2: always 32
 namespace k {
 
-static uint32_t compute_units() {
+uint32_t compute_units() {
     static int cus = 0;
     if (cus == 0) {
         int dev = 0, v = 0;

@@ -48,6 +48,8 @@ void convert_bf16_to_f32(const uint16_t *in, float *out, uint64_t n, hipStream_t
 void rope_f32(const float *x, const int32_t *pos, float *out, uint64_t rows, uint64_t heads,
               uint64_t head_dim, double theta, hipStream_t s);
 void fill_u32(uint32_t *p, uint32_t v, uint64_t n, hipStream_t s);
+// Compute units of the current device (kern_paged.hip)
+uint32_t compute_units();
 // 32-bit words from memory of the host that the device can read: up to four ranges in one launch
 struct WordRange {
     const uint32_t *from;
