@@ -9,13 +9,26 @@
 #include <cstdint>
 
 #if defined(__HIPCC__)
-#define FA_HD __host__ __device__ __forceinline__ constexpr
+#define FA_HD_CALL __host__ __device__ __forceinline__
 #else
-#define FA_HD inline constexpr
+#define FA_HD_CALL inline
 #endif
+#define FA_HD FA_HD_CALL constexpr
 
 namespace fa {
 namespace ixm {
+
+// ------------------------------------------------------------------ row quantizer
+// x / scale for an int8 code, inv the rounded 1 / scale: the product and one correction by its exact remainder.  It rounds to the
+// same integer as the rounded quotient does: the product alone can be off by an ulp or two, which matters next to the middle of two
+// codes (and values that were rounded to bf16 lie exactly there in three wavefronts of four); the corrected one is off only where
+// the quotient is within 2^-22 ulp of the middle of two floats, and next to a middle of two codes no quotient of floats is (walked
+// on the host for every mantissa of scale).  From kQuantLeastScale on no remainder that counts is subnormal.
+constexpr float kQuantLeastScale = 0x1p-100f;
+FA_HD_CALL float quant_quotient(float x, float scale, float inv) {
+    const float q = x * inv;
+    return __builtin_fmaf(__builtin_fmaf(-q, scale, x), inv, q);
+}
 
 // ------------------------------------------------------------------ large-tile GEMM (gemm_mfma_big_kernel)
 // Block tile MTB * 16 rows (256 unless stated) x NTB * 16 columns, NWAVES = 2 WM wavefronts (WM along m, 2 along n).  One

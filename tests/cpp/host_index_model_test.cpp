@@ -5,8 +5,11 @@
 //   large-tile GEMM   : e4m3 / int8 (bf16 moves the same bytes) x 8 / 14 / 16 column tiles x 8 / 12 / 16 row tiles x 4 / 8 / 16 wavefronts
 //   streamed attention: ranges, segments and partial-result slots against the merge's expectation, ragged lengths
 //   split-k linears   : groups on one XCD, k ranges, workspace offsets
+//   row quantizer     : codes at the middles of two codes
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <set>
 #include <vector>
@@ -393,7 +396,29 @@ static void gemm_cases() {
     gemm_case<FP8, 16, 8>();
 }
 
-int main() {
+// Row quantizer: codes around every middle of two codes are those of the division, for every 64th mantissa of the scale (with an
+// argument: for every one), at the least scale that takes this form and at the largest there is.
+static void quantizer_case(uint32_t step) {
+    for (float unit : {1.0f, kQuantLeastScale, 0x1p120f})
+        for (uint32_t m = unit == 1.0f ? 0 : 5; m < (1u << 23); m += unit == 1.0f ? step : 131071) {
+            const float scale = unit * (1.0f + (float)m * 0x1p-23f), inv = 1.0f / scale;
+            for (int k = 0; k < 127; ++k) {
+                const float at = (float)((k + 0.5) * (double)scale);
+                uint32_t bits;
+                std::memcpy(&bits, &at, 4);
+                for (int d = -3; d <= 3; ++d) {
+                    float x;
+                    const uint32_t b = bits + (uint32_t)d;
+                    std::memcpy(&x, &b, 4);
+                    const float q = quant_quotient(x, scale, inv), sum = q + 12582912.0f;
+                    CHECK(std::rint(x / scale) == sum - 12582912.0f && -std::rint(x / scale) == (quant_quotient(-x, scale, inv) + 12582912.0f) - 12582912.0f);
+                }
+            }
+        }
+}
+
+int main(int argc, char **) {
+    quantizer_case(argc > 1 ? 1 : 64);
     rope_tile_case(1);
     rope_tile_case(13);
     stage_ring_case(2);
