@@ -50,18 +50,20 @@ __global__ void __launch_bounds__(kArgmaxThreads)
         }
     };
     if (cols % 4 == 0) {                                          // rows start on 16-byte boundaries
-        // eight loads under way per thread: a block has a row's bytes to itself, and one at a time it waits for memory once per
-        // 16 KiB (32000 columns: 7.2 us so, 5.9 with eight)
+        // two loads under way per thread: a block has a row's bytes to itself, and one at a time it waits for memory once per 16 KiB;
+        // more of them cost short rows what they give long ones.  One, two, four, eight, us: a row of 4096 3.94, 3.96, 4.12, 4.42, of
+        // 32000 6.02, 5.75, 5.76, 5.92, of 151936 14.1, 13.1, 12.9, 12.8; 512 rows of 65536 23.4, 23.4, 24.9, 27.0
+        constexpr int U = 2;
         const uint64_t n = cols / 4;
-        for (uint64_t q0 = threadIdx.x; q0 < n; q0 += 8 * kArgmaxThreads) {
-            float4 v[8];
+        for (uint64_t q0 = threadIdx.x; q0 < n; q0 += U * kArgmaxThreads) {
+            float4 v[U];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < U; ++u) {
                 const uint64_t q = q0 + u * kArgmaxThreads;
                 v[u] = *(const float4 *)(row + 4 * (q < n ? q : n - 1));
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < U; ++u) {
                 const uint64_t q = q0 + u * kArgmaxThreads;
                 if (q >= n) break;
                 see(v[u].x, (uint32_t)(4 * q));
