@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "decoder.hpp"
+#include "index_models.hpp"
 #include "kernels.hpp"
 #include "runtime.hpp"
 #include "validate.hpp"
@@ -95,15 +96,8 @@ void free_all(fa_context *ctx, fa_decoder *d) {
     }
 }
 
-// Whether the attention of the step about to be enqueued (the host lengths already count its token) finishes in one launch;
-// the recorded graphs of the two kinds are kept apart.
-// With at most one block per compute unit (sequences x kv heads; left-over units take shares of the sequences) the one-launch
-// form saves the partial results and the merge, and its time is the longest share; the streamed form cuts all pages into equal
-// ranges, whatever the lengths.  So the line is how far the longest share exceeds an even one.  Step through 8 layers, 32 / 8
-// heads, one launch and streamed, us: one sequence of 700 588 and 603, 6000 661 and 807; four of 4000 696 and 817; sixteen of
-// 3000 (share 1500, even 1500) 901 and 938, of 100 .. 1500 (730, 400) 766 and 791, of 200 .. 3000 (1450, 800) 871 and 843;
-// thirty-two of 2500 1116 and 1164; 16 / 4 heads, sixty of 100 .. 2000 (1980, 980) 794 and 734.  With so few sequences that
-// units are left over, the streamed form's many small ranges cost it more: one of 8000 (1000, 250) 696 and 893.
+// Whether the attention of the step about to be enqueued (the host lengths already count its token) finishes in one launch
+// (ixm::decode_attends_at_once); the recorded graphs of the two kinds are kept apart.
 bool step_attends_at_once(const fa_decoder *d) {
     if (k::g_decode_one == 1) return false;
     uint64_t longest = 0, all = 0;
@@ -115,8 +109,8 @@ bool step_attends_at_once(const fa_decoder *d) {
     if (k::g_decode_one >= 2) return k::g_decode_one == 3 || longest <= 1024;
     const uint64_t cus = (uint64_t)d->ctx->props.multiProcessorCount, items = (uint64_t)d->batch * d->cfg.n_kv_heads;
     if (items > cus) return false;
-    const uint64_t shares = k::decode_one_shares(items, &d->ctx->splitk, (int)cus), even = all * d->cfg.n_kv_heads / cus;
-    return longest / shares <= even + (shares == k::kDecodeOneShares ? 1024 : 512);
+    const uint64_t shares = k::decode_one_shares(items, &d->ctx->splitk, (int)cus);
+    return ixm::decode_attends_at_once(longest / shares, all * d->cfg.n_kv_heads / cus, shares == k::kDecodeOneShares);
 }
 
 // The kernels of one step, enqueued on the context's stream.  stop_after (test aid, -1 in normal use) ends the

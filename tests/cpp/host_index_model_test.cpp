@@ -5,6 +5,7 @@
 //   large-tile GEMM   : e4m3 / int8 (bf16 moves the same bytes) x 8 / 14 / 16 column tiles x 8 / 12 / 16 row tiles x 4 / 8 / 16 wavefronts
 //   streamed attention: ranges, segments and partial-result slots against the merge's expectation, ragged lengths
 //   split-k linears   : groups on one XCD, k ranges, workspace offsets
+//   decode attention  : which form a step takes
 //   row quantizer     : codes at the middles of two codes
 #include <cmath>
 #include <cstdio>
@@ -417,7 +418,23 @@ static void quantizer_case(uint32_t step) {
         }
 }
 
+// The decode attention's form on both sides of its line, at lengths whose steps were measured (256 compute units).
+static void decode_form_cases() {
+    struct Case {
+        uint64_t batch, kv_heads, low, high;
+        bool once;
+    };
+    for (const Case &c : {Case{1, 8, 700, 700, true}, Case{1, 8, 8000, 8000, true}, Case{4, 8, 500, 8000, true}, Case{8, 8, 500, 8000, false}, Case{8, 8, 8000, 8000, true},
+                          Case{16, 8, 3000, 3000, true}, Case{16, 8, 6000, 6000, false}, Case{16, 8, 2000, 4096, false}, Case{24, 8, 1000, 1000, true},
+                          Case{24, 8, 3000, 3000, false}, Case{32, 8, 2000, 2000, true}, Case{32, 8, 3000, 3000, false}, Case{32, 8, 1024, 8192, false},
+                          Case{24, 4, 4096, 4096, false}, Case{48, 4, 1000, 1000, true}, Case{48, 4, 2000, 2000, false}, Case{64, 4, 1000, 1000, true}}) {
+        const uint64_t items = c.batch * c.kv_heads, room = 256 / items, shares = room < 1 ? 1 : room > 8 ? 8 : room;
+        CHECK(decode_attends_at_once(c.high / shares, (c.low + c.high) * c.batch / 2 * c.kv_heads / 256, shares == 8) == c.once);
+    }
+}
+
 int main(int argc, char **) {
+    decode_form_cases();
     quantizer_case(argc > 1 ? 1 : 64);
     rope_tile_case(1);
     rope_tile_case(13);
