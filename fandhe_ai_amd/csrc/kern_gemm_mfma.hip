@@ -990,9 +990,9 @@ constexpr BigShape kBigShapes[] = {{16, 16, 14.5, 23.7}, {16, 14, 12.3, 21.6}, {
 // The tile with the lowest cost: whole rounds over the compute units, and a last one that costs less the emptier it is (0.6 of a
 // full one at the least: measured 0.65 at 0.3, 0.8 at 0.6: the blocks in it have the L2s, and the power, to themselves).
 // tiles_of(rows): row blocks of that many rows.  max_share: blocks that may share a tile of 128 columns, a part of k each (8 stages
-// at the least).
+// at the least).  low: what tiles of fewer than 256 rows cost more than the table says.
 template <typename F>
-BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, uint32_t max_share) {
+BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, uint32_t max_share, double low = 1.0) {
     BigTile best;
     auto has = [&](const BigShape &b) { return (widths & (b.ntb == 16 ? kWide16 : b.ntb == 14 ? kWide14 : kWide8)) != 0; };
     auto wanted = [](const BigShape &b) { return (!g_gemm_ntb || g_gemm_ntb == b.ntb) && (!g_gemm_mtb || g_gemm_mtb == b.mtb); };
@@ -1005,7 +1005,7 @@ BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_
             if (share > 1 && (b.ntb != 8 || k_steps / share < 8)) break;
             const double blocks = tiles * share, rounds = std::floor(blocks / num_cus), rest = blocks / num_cus - rounds;
             const double one = b.fixed + b.per_2k * (double)((k_steps + share - 1) / share) / 16.0 + (share > 1 ? kShareCost * share * b.mtb * b.ntb / 64.0 : 0.0);
-            const double cost = one * (rounds + (rest > 0 ? 0.6 + 0.4 * rest : 0.0));
+            const double cost = one * (rounds + (rest > 0 ? 0.6 + 0.4 * rest : 0.0)) * (b.mtb < 16 ? low : 1.0);
             if (best.ntb == 0 || cost < best.cost) best = BigTile{b.mtb, b.ntb, share, cost};
         }
     }
@@ -1260,9 +1260,19 @@ void launch_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroup
         const uint32_t nb = (w.n_tiles + 15) / 16, tiles = rg.entries / (MTB * 16) + (rg.groups < rg.entries ? rg.groups : rg.entries);
         launch_big_tile<false, 16, 4, MTB>((const uint8_t *)a, (const uint8_t *)w.w, 0, w.n, w.n_tiles, w.k_tiles / 2, nb, (tiles * nb + 7) / 8 * 8, EpiBf16Grouped<MODE>{ep, rg}, s);
     };
-    // how the rows spread over the groups is known on the device only: half a tile per group is taken to be padding
-    const double likely = rg.likely ? rg.likely : rg.entries, groups = rg.groups;
-    const BigTile t = pick_big_rows([&](int r) { return likely / r + 0.5 * groups; }, w.n_tiles, w.k_tiles / 2, num_cus, kWide16, 1);
+    // How the rows spread over the groups is known on the device only: a group's tiles, rounded up, averaged over 0.85 to 1.15 of the
+    // mean.  Rows gathered through a list cost the lower tiles more than the table says: 1.1 times where the entries of a group share rows
+    // with other groups' (the way up), 1.18 where all are distinct.  16 experts, 4 a token, us on 128 / 192 / 256 rows: 2048 -> 3072 at 130
+    // rows a group 86 / 56 / 58, at 384 108 / 102 / 112, at 2048 497 / 444 / 398; 3072 -> 2048 at 225 61 / 78 / 87, at 450 106 / 150 / 98, at 650
+    // 163 / 158 / 169, at 2048 498 / 452 / 422; 5376 -> 4096 at 172 207 / 272 / 171, at 450 377 / 392 / 303, at 2048 1536 / 1493 / 1251.
+    // (Half a tile per group taken as padding, and the table's costs, chose 192 rows at 2048 and at 450 rows a group and 128 at 172.)
+    const double mean = (double)(rg.likely ? rg.likely : rg.entries) / rg.groups;
+    auto tiles = [&](int r) {
+        double sum = 0.0;
+        for (int d = -3; d <= 3; ++d) sum += std::ceil(mean * (1.0 + 0.05 * d) / r);
+        return sum / 7.0 * rg.groups;
+    };
+    const BigTile t = pick_big_rows(tiles, w.n_tiles, w.k_tiles / 2, num_cus, kWide16, 1, rg.a_div > 1 ? 1.1 : 1.18);
     if (t.mtb == 8) rows(std::integral_constant<int, 8>{});
     else if (t.mtb == 12) rows(std::integral_constant<int, 12>{});
     else rows(std::integral_constant<int, 16>{});
