@@ -110,7 +110,7 @@ bool step_attends_at_once(const fa_decoder *d) {
     const uint64_t cus = (uint64_t)d->ctx->props.multiProcessorCount, items = (uint64_t)d->batch * d->cfg.n_kv_heads;
     if (items > cus) return false;
     const uint64_t shares = k::decode_one_shares(items, &d->ctx->splitk, (int)cus);
-    return ixm::decode_attends_at_once(longest / shares, all * d->cfg.n_kv_heads / cus, shares == k::kDecodeOneShares);
+    return ixm::decode_attends_at_once(longest / shares, all * d->cfg.n_kv_heads / cus, shares, k::kDecodeOneShares);
 }
 
 // The kernels of one step, enqueued on the context's stream.  stop_after (test aid, -1 in normal use) ends the

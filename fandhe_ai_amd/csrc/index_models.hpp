@@ -19,20 +19,21 @@ namespace fa {
 namespace ixm {
 
 // ------------------------------------------------------------------ decode attention
-// Whether a decode step's attention runs as one launch: a block per sequence and kv head, or per share of one where compute units are
+// Whether a decode step's attention runs as one launch: a block per sequence and kv head, or up to `shares` where compute units are
 // left, `share` tokens in the longest; `even`: what an even division over the units would give each.  That form saves the partial
 // results and the merge, and its time is the longest share; the streamed form cuts all pages into equal ranges, whatever the lengths.
 // So what counts is how far the longest share exceeds an even one, and how long it is (a block alone keeps a unit's loads less busy
 // than the streamed form's wavefronts).  Step through 4 layers, streamed and one launch, us:
 //   32 / 8 heads, equal lengths, 16 sequences (two shares) of 3000 475 and 474, 6000 572 and 606; 24 (one) of 1000 445 and 429, 2000 501
 //   and 507; 32 of 1000 471 and 445, 2000 548 and 535, 3000 601 and 623, 4096 703 and 723;
-//   16 / 4 heads, 24 (two shares) of 2000 332 and 332, 4096 391 and 418; 32 of 2000 355 and 347, 4096 434 and 445; 48 of 1500 368 and 377;
+//   16 / 4 heads, 24 (two shares) of 2000 332 and 332, 4096 391 and 418; 32 of 2000 355 and 347, 3000 381 and 391, 4096 434 and 445; 48 of
+//   1500 368 and 377; 16 (four shares) of 4096 338 and 333, 8000 416 and 412;
 //   lengths apart, 32 / 8 heads: 16 of 100 .. 1000 395 and 379, 2000 .. 4096 487 and 510; 8 (four shares) of 1000 .. 4000 419 and 408.
-// With so few sequences that units are left over at `most` shares, the streamed form's many small ranges cost it more: one of 8000 465
+// (Two blocks to a sequence fill the units no better than one does, and have to meet.)  With so few sequences that units are left over at `most` shares, the streamed form's many small ranges cost it more: one of 8000 465
 // and 360, four of 500 .. 8000 449 and 400.
-FA_HD bool decode_attends_at_once(uint64_t share, uint64_t even, bool most) {
-    if (most) return share <= even + 1024;
-    return 8 * (share > even ? share - even : 0) + 3 * share <= 6400;
+FA_HD bool decode_attends_at_once(uint64_t share, uint64_t even, uint64_t shares, uint64_t most) {
+    if (shares == most) return share <= even + 1024;
+    return 8 * (share > even ? share - even : 0) + (shares == 2 ? 9 : 6) * share / 2 <= 6400;
 }
 
 // ------------------------------------------------------------------ row quantizer

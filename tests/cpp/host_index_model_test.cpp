@@ -425,11 +425,11 @@ static void decode_form_cases() {
         bool once;
     };
     for (const Case &c : {Case{1, 8, 700, 700, true}, Case{1, 8, 8000, 8000, true}, Case{4, 8, 500, 8000, true}, Case{8, 8, 500, 8000, false}, Case{8, 8, 8000, 8000, true},
-                          Case{16, 8, 3000, 3000, true}, Case{16, 8, 6000, 6000, false}, Case{16, 8, 2000, 4096, false}, Case{24, 8, 1000, 1000, true},
+                          Case{16, 8, 2000, 2000, true}, Case{16, 8, 6000, 6000, false}, Case{16, 8, 2000, 4096, false}, Case{24, 8, 1000, 1000, true},
                           Case{24, 8, 3000, 3000, false}, Case{32, 8, 2000, 2000, true}, Case{32, 8, 3000, 3000, false}, Case{32, 8, 1024, 8192, false},
-                          Case{24, 4, 4096, 4096, false}, Case{48, 4, 1000, 1000, true}, Case{48, 4, 2000, 2000, false}, Case{64, 4, 1000, 1000, true}}) {
+                          Case{24, 4, 4096, 4096, false}, Case{32, 4, 2000, 2000, true}, Case{32, 4, 4096, 4096, false}, Case{16, 4, 8000, 8000, true}, Case{48, 4, 1000, 1000, true}, Case{48, 4, 2000, 2000, false}, Case{64, 4, 1000, 1000, true}}) {
         const uint64_t items = c.batch * c.kv_heads, room = 256 / items, shares = room < 1 ? 1 : room > 8 ? 8 : room;
-        CHECK(decode_attends_at_once(c.high / shares, (c.low + c.high) * c.batch / 2 * c.kv_heads / 256, shares == 8) == c.once);
+        CHECK(decode_attends_at_once(c.high / shares, (c.low + c.high) * c.batch / 2 * c.kv_heads / 256, shares, 8) == c.once);
     }
 }
 
