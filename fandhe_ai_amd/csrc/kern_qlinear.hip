@@ -1187,20 +1187,15 @@ __global__ void __launch_bounds__(512)
 // are coherent between XCDs wherever the blocks run.  The ticket is relaxed; what orders it behind the stores is
 // the wait for their acknowledgement, not a fence (an agent-scope release writes back a whole L2).  (meet_store, meet_load,
 // meet_ticket: device_utils.hpp)
-// Four consecutive words of a partial tile set, requested with the cache policy of meet_load (a wider relaxed atomic
-// load does not exist; the words were written by one 16-byte store whose acknowledgement the writer awaited before its
-// ticket).  The request is an assembly statement, so the compiler neither waits for it nor knows that `v` is in
-// flight: `v` may only be touched after an unseen_wait_all that names it.
+// Four consecutive words of a partial tile set, with the cache policy of meet_load (a wider relaxed atomic load does not
+// exist; the words were written by one 16-byte store whose acknowledgement the writer awaited before its ticket).  A buffer
+// load, because its builtin takes the policy (1: sc0, 16: sc1) and leaves registers and waits to the compiler: as an
+// assembly statement whose wait stands elsewhere, nothing would keep the compiler from moving a register still in flight.
+// `word` counts from `base`; the resource has no bound of its own, so base + word must lie in the workspace (below 4 GiB).
 template <bool LOCAL>
-__device__ __forceinline__ void meet_request_b128(v4i &v, const int32_t *p) {
-    if constexpr (LOCAL) asm volatile("global_load_dwordx4 %0, %1, off sc0" : "=&v"(v) : "v"(p));
-    else asm volatile("global_load_dwordx4 %0, %1, off sc1" : "=&v"(v) : "v"(p));
-}
-__device__ __forceinline__ void unseen_wait_all(v4i (&x)[4][4]) {
-    asm volatile("s_waitcnt vmcnt(0)"
-                 : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[0][2]), "+v"(x[0][3]), "+v"(x[1][0]), "+v"(x[1][1]), "+v"(x[1][2]),
-                   "+v"(x[1][3]), "+v"(x[2][0]), "+v"(x[2][1]), "+v"(x[2][2]), "+v"(x[2][3]), "+v"(x[3][0]), "+v"(x[3][1]),
-                   "+v"(x[3][2]), "+v"(x[3][3]));
+__device__ __forceinline__ v4i meet_load_b128(const int32_t *base, uint32_t word) {
+    const __amdgpu_buffer_rsrc_t area = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
+    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(area, word * 4, 0, LOCAL ? 1 : 16));
 }
 // LOCAL only: the members of a group must share an XCD, or the partial tiles above were exchanged through two
 // different L2s.  Every member notes the XCD it runs on before it takes its ticket; the last arriver compares and
@@ -1471,7 +1466,7 @@ __global__ void __launch_bounds__(512)
             const uint32_t g = g0 + u < row_groups ? g0 + u : row_groups - 1;
 #pragma unroll
             for (int r = 0; r < S; ++r)
-                meet_request_b128<LOCAL>(part[u][r], partial + ixm::rows_ksplit_partial_base(group, r, S, row_groups, g, NACC) + (wave * 64 + lane) * 4);
+                part[u][r] = meet_load_b128<LOCAL>(partial, (uint32_t)ixm::rows_ksplit_partial_base(group, r, S, row_groups, g, NACC) + (wave * 64 + lane) * 4);
         }
         float p_sx[4][4], p_res[4][4];
 #pragma unroll
@@ -1484,7 +1479,7 @@ __global__ void __launch_bounds__(512)
                 p_res[u][e] = (ok && ep.residual) ? ep.residual[(uint64_t)(row0 + e) * n + col] : 0.0f;
             }
         }
-        unseen_wait_all(part);
+        __builtin_amdgcn_sched_barrier(0);                       // every load is under way before the first sum
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const uint32_t row0 = ((g0 + u) * MT + ti) * 16 + 4 * (lane / 16);
@@ -2116,6 +2111,7 @@ inline bool rows_ksplit_plan(uint64_t m, uint32_t n_tiles, uint32_t k_tiles, int
     p->blocks = 32u * ((n_groups + 7) / 8);                    // whole groups on every XCD; surplus groups return at once
     p->row_groups = (uint32_t)((m + 31) / 32);
     p->workspace_bytes = (uint64_t)n_groups * 4 * p->row_groups * (2 * 4 * 4 * 64 * 4);
+    if (p->workspace_bytes >> 32) return false;                // the partial sets are read by 32-bit byte offsets
     p->local = g_skinny_ksplit == 3 || ((g_skinny_ksplit == 0) && sk->xcd_local);
     return true;
 }

@@ -1,4 +1,4 @@
-"""Inline assembly names the special registers it writes among its clobbers: the compiler may keep values of its own in them."""
+"""What inline assembly has to tell the compiler: the special registers it writes, and no result that is still under way."""
 import glob
 import os
 import re
@@ -47,3 +47,13 @@ def test_special_registers_are_named_as_clobbers():
                 if w and w.group(1) in SPECIAL:
                     assert '"%s"' % w.group(1) in p[3], "%s: %s" % (os.path.basename(path), s.strip())
     assert seen > 10
+
+
+def test_loads_into_registers_are_waited_for_in_their_statement():
+    """The compiler takes an output as written when the statement ends and may move or reuse its register from there on.  (LDS
+    reads ahead of their waits are followed through the machine code of the one kernel that has them.)"""
+    for path in sorted(glob.glob(os.path.join(ROOT, "*.h*"))):
+        for s in statements(open(path).read()):
+            p = parts(s)
+            if p[1].strip() and re.search(r"\b(global|buffer|flat|scratch|s)_load", p[0]):
+                assert "s_waitcnt" in p[0][p[0].rindex("_load"):], "%s: %s" % (os.path.basename(path), s.strip())
