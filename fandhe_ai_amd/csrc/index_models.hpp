@@ -29,8 +29,8 @@ namespace ixm {
 //   16 / 4 heads, 24 (two shares) of 2000 332 and 332, 4096 391 and 418; 32 of 2000 355 and 347, 3000 381 and 391, 4096 434 and 445; 48 of
 //   1500 368 and 377; 16 (four shares) of 4096 338 and 333, 8000 416 and 412;
 //   lengths apart, 32 / 8 heads: 16 of 100 .. 1000 395 and 379, 2000 .. 4096 487 and 510; 8 (four shares) of 1000 .. 4000 419 and 408.
-// (Two blocks to a sequence fill the units no better than one does, and have to meet.)  With so few sequences that units are left over at `most` shares, the streamed form's many small ranges cost it more: one of 8000 465
-// and 360, four of 500 .. 8000 449 and 400.
+// (Two blocks to a sequence fill the units no better than one does, and have to meet.)  With so few sequences that units are left
+// over at `most` shares, the streamed form's many small ranges cost it more: one of 8000 465 and 360, four of 500 .. 8000 449 and 400.
 FA_HD bool decode_attends_at_once(uint64_t share, uint64_t even, uint64_t shares, uint64_t most) {
     if (shares == most) return share <= even + 1024;
     return 8 * (share > even ? share - even : 0) + (shares == 2 ? 9 : 6) * share / 2 <= 6400;

@@ -955,7 +955,7 @@ constexpr int scan_waves(int kt) { return kt >= 16 ? 8 : kt >= 4 ? 4 : kt; }
 // KT / waves row tiles of the state each.  A chunk is: every wavefront's share of W S_0 and exp(G) Q S_0 over its own rows, the
 // shares exchanged through LDS (one barrier), the writes U whole in every wavefront, every wavefront's own rows of the state; the
 // first two also form a half of the read-outs each.  A wavefront alone reads its rows' fragments: they go from memory to
-// registers, a chunk ahead.  Measured, 32 heads 128 x 128: 2048 tokens of one sequence 330 -> 120 us (of two 335 -> 270); with
+// registers, a chunk ahead.  Measured, 32 heads 128 x 128: 2048 tokens of one sequence 330 -> 130 us (of two 335 -> 270); with
 // four sequences (1024 tiles, four per compute unit) the exchanges cost more than the idle cores: 10 % slower than the form above.
 template <int KT, Recurrence KIND>
 __global__ void __launch_bounds__(scan_waves(KT) * 64)

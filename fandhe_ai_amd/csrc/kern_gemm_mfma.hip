@@ -22,8 +22,7 @@ using namespace fa::dev;
 
 int g_gemm_small_tiles = 0;   // tuning: nonzero keeps the 128 x 128 kernel for every shape
 extern int g_skinny_ksplit;   // kern_qlinear.hip
-int g_gemm_pair = 0;          // tuning, 256 x 128 tiles of the large-tile kernel: 1 keeps one block per tile, 2 shares a tile
-                              // only where the tiles alone would cover half the device
+int g_gemm_pair = 0;          // tuning, tiles of 128 columns of the large-tile kernel: 1 keeps one block per tile
 int g_gemm_swiglu = 0;        // tuning, prompt passes: bit 0 keeps SwiGLU out of the gate | up GEMM's epilogue, bit 1 RoPE
                               // and the K / V append out of the q | k | v GEMM's
 int g_gemm_waves = 0;         // tuning: 4 = four wavefronts per large-tile block instead of eight, 16 = sixteen
@@ -393,11 +392,11 @@ __device__ __forceinline__ void static_for(F &&f) {
 }
 
 // ------------------------------------------------------------ large tiles
-// Block tile 256 rows x NTB * 16 columns, four wavefronts in 2 x 2, one per
-// SIMD, each owning 128 rows x NTB / 2 column tiles of accumulators (up to 256
-// registers).  Per k-step a wavefront reads 8 A fragments once and streams its
-// B fragments past them, so the LDS traffic per matrix instruction is a quarter
-// of the 64 x 64 wavefront tile above, which is what lets the matrix cores run
+// Block tile MTB * 16 rows (128, 192 or 256) x NTB * 16 columns (128, 224 or 256), WM x 2
+// wavefronts (2 x 2, 4 x 2 or 8 x 2; eight unless tuned), each owning MTB / WM row tiles x
+// NTB / 2 column tiles of accumulators.  Per k-step a wavefront reads its A fragments once and
+// streams its B fragments past them: 12 fragments of 4 x 8 tiles of 256 x 256 feed 32
+// multiplies, where the 64 x 64 wavefront tile above reads 8 for 16, and the matrix cores run
 // instead of waiting on LDS.  Rows / tiles past the edge are loaded from a
 // clamped address (never stored), so the main loop has no predicated loads.
 // The block index is remapped so that the blocks that land on one XCD (the

@@ -95,18 +95,17 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  *        are at most 1024 tokens; 3: always (takes effect when a step is recorded);
  * key 21: the int8 linears of 65 to a few hundred rows (fa_linear_w8a8, prompt passes of the decoder): 0 the
  *        weight-stationary kernel where the shape rule picks it (a weight with at most about two column tiles per
- *        compute unit, m x k at most 2 MiB; k of 8192 .. 14336: the form that splits k over four blocks of an XCD,
- *        up to 512 rows) and the decode kernels for prompt passes of at most 64 rows, 1 the tiled GEMMs always, 2 the
+ *        compute unit, m x k at most 2 MiB, at most 160 to 320 rows by k and n: those for which the tiled GEMMs measured
+ *        slower; k of 10240 .. 14336: the form that splits k over four blocks of an XCD) and the decode kernels for prompt passes of at most 64 rows, 1 the tiled GEMMs always, 2 the
  *        weight-stationary kernel without the split whenever it can run, 3 the split form whenever it can run;
  * key 22: prompt passes on the large-tile GEMM, bits: 1 keeps SwiGLU out of the epilogue of the gate | up GEMM (the plain
  *        GEMM into [rows, 2 d_ffn] and the SwiGLU pass of the row quantizer), 2 keeps RoPE, the bf16 rounding and the K / V
  *        append out of the epilogue of the q | k | v GEMM (the plain GEMM and the RoPE + append pass); 0: both in the
  *        epilogues;
  * key 23: columns (new token x head) per wavefront of the block form of the prefill attention: 0 by shape (16 while
- *        blocks of 32 would not fill the device more than once, else 32), 1: 16 whenever the form allows, 2: 32;
- * key 24: the large-tile int8 GEMM on 256 x 128 tiles: 0: when those tiles cover at most half the device, two or four
- *        same-XCD blocks share a tile, a part of k each; 1: one block per tile; 2: shared tiles only where the tiles
- *        alone cover half the device (pairs);
+ *        blocks of 32 would leave compute units with fewer than two, else 32), 1: 16 whenever the form allows, 2: 32;
+ * key 24: the large-tile int8 GEMM on tiles of 128 columns: 0: where the tiles alone leave compute units idle, two or
+ *        four same-XCD blocks may share a tile, a part of k each; 1: one block per tile;
  * key 25: rows (sequences x tokens) per chunk of a prompt pass, from 256 up; anything smaller: the built-in 8192;
  * key 26: prompt passes of at most 64 rows: 0: q | k | v and gate | up on the decode step's fused kernels (RoPE and the
  *        K / V append, SwiGLU, in the epilogues), 1: plain projections and separate passes;
