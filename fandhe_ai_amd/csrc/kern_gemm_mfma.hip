@@ -342,7 +342,8 @@ __device__ __forceinline__ void hold_acc(T &c) {
 
 // LDS fragment reads and the waits for them, as assembly, for the large-tile kernel's main loop.  A read's result
 // may only be touched after an lds_wait that names it: the wait takes the registers as in/out operands, so every
-// use the compiler sees comes after it.  addr is an LDS byte address, OFF an immediate offset below 65536.
+// use the compiler sees comes after it.  It could still move a register under way; that it does not is checked in the
+// machine code of every instance (test_gemm_lds_reads_cpu.py).  addr is an LDS byte address, OFF an immediate offset below 65536.
 template <int OFF>
 __device__ __forceinline__ void lds_read16(v4i &dst, uint32_t addr) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));

@@ -617,7 +617,9 @@ void rmsnorm_f32(const float *x, const float *w, float *out, uint64_t rows, uint
 // unit a row's chain is all there is: a thousand threads.  From there on rows queue, and what counts is how many are under way
 // and that every load is a whole line: 256 threads (RMSNorm and quantizer of 8192 x 4096, us: 128 threads 31.9, 256 29.4, 512
 // 36.2, 1024 66; with sixteen neighbouring elements per thread 39.9; of 2545 x 2048 8.8, 8.6, 10.4, 17.9; 11.4), up to two
-// blocks per unit 512 (300 x 4096: 256 threads 6.3, 512 5.6, 1024 6.2; sixteen neighbours 6.5).  false: rows too wide for it.
+// blocks per unit 512 (300 x 4096: 256 threads 6.3, 512 5.6, 1024 6.2; sixteen neighbours 6.5; all with codes that were divided
+// next to ties, corrected by their remainder as now 26.6, 7.4 and 5.5 for 8192 x 4096, 2545 x 2048 and 300 x 4096).  false: rows
+// too wide for it.
 template <typename F>
 static bool wide_form(uint64_t rows, uint64_t width, F &&go) {
     using std::integral_constant;
