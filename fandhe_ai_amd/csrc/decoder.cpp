@@ -8,6 +8,7 @@
 #include <cmath>
 #include <exception>
 #include <new>
+#include <numeric>
 #include <string>
 #include <vector>
 
@@ -327,7 +328,8 @@ struct Temp {
     T *as() const { return (T *)ptr; }
 };
 
-// One pass of a prompt chunk (lc tokens per sequence, rows = batch * lc, row b * lc + t) through all layers
+// One pass of a prompt chunk (lc tokens per sequence, rows = batch * lc, row b * lc + t; padded: the prompts' own tokens one
+// prompt behind the other, lc the longest's) through all layers
 // on the prefill-shape GEMMs and the prefill form of the attention kernel.  The arithmetic per row is
 // that of the decode step (same quantizers, same dequantization, same RoPE and SwiGLU expressions), so
 // a prompt token leaves the same K / V rows in the cache as if it had been decoded.
@@ -335,30 +337,29 @@ struct PrefillBuffers {
     Temp tok, h, xq, sx, qkv, q_bf, attn, gu, slots, cos_sin, last_rows, splitk;
     // verification only: logits and greedy picks of every row
     Temp all_logits, all_picked;
-    // padded pass only: the true prompt length of every row
-    Temp row_lens;
+    // padded pass only: where every prompt's rows start, and behind the last one
+    Temp row_start;
     PrefillBuffers(fa_context *c, fa_decoder *d)
         : tok(c), h(c, &d->kept[0]), xq(c, &d->kept[1]), sx(c), qkv(c, &d->kept[2]), q_bf(c, &d->kept[3]), attn(c, &d->kept[4]),
           gu(c, &d->kept[5]), slots(c), cos_sin(c), last_rows(c), splitk(c, &d->kept[6]), all_logits(c, &d->kept[7]),
-          all_picked(c), row_lens(c) {}
+          all_picked(c), row_start(c) {}
 };
 
-fa_status enqueue_prefill_chunk(fa_context *ctx, fa_decoder *d, PrefillBuffers &t, uint32_t lc, bool last_chunk,
-                                bool every_row = false, bool padded = false) {
+fa_status enqueue_prefill_chunk(fa_context *ctx, fa_decoder *d, PrefillBuffers &t, uint32_t lc, uint64_t M, uint32_t ctx_max, bool last_chunk,
+                                bool every_row, bool padded) {
     const fa_decoder_config &c = d->cfg;
     const uint32_t B = d->batch;
-    const uint64_t M = (uint64_t)B * lc;
     const uint64_t D = c.d_model, F = c.d_ffn, V = c.vocab;
+    const uint32_t *row_start = padded ? t.row_start.as<uint32_t>() : nullptr;
     const uint64_t EKV = (uint64_t)c.n_kv_heads * c.head_dim;
     const int cus = ctx->props.multiProcessorCount;
     hipStream_t s = ctx->stream;
     const uint64_t pool_rows = (uint64_t)c.num_blocks * c.block_size;
 
-    k::prefill_prepare((const uint32_t *)d->tables->ptr, (const uint32_t *)d->seq_lens->ptr, t.slots.as<uint32_t>(),
-                       t.cos_sin.as<float>(), B, lc, c.block_size, c.max_blocks_per_seq, c.num_blocks, c.head_dim,
+    k::prefill_prepare((const uint32_t *)d->tables->ptr, (const uint32_t *)d->seq_lens->ptr, row_start, t.slots.as<uint32_t>(),
+                       t.cos_sin.as<float>(), (uint32_t)M, B, lc, c.block_size, c.max_blocks_per_seq, c.num_blocks, c.head_dim,
                        c.rope_theta, s);
-    k::advance_seq_lens((uint32_t *)d->seq_lens->ptr, t.last_rows.as<int32_t>(), B, lc,
-                        padded ? t.row_lens.as<uint32_t>() : nullptr, s);
+    k::advance_seq_lens((uint32_t *)d->seq_lens->ptr, t.last_rows.as<int32_t>(), row_start, B, lc, s);
     k::gather_rows_f32((const float *)d->embed->ptr, V, D, t.tok.as<int32_t>(), t.h.as<float>(), M, s);
 
     k::PagedShape ps;
@@ -372,7 +373,9 @@ fa_status enqueue_prefill_chunk(fa_context *ctx, fa_decoder *d, PrefillBuffers &
     ps.head_dim = c.head_dim;
     ps.max_blocks_per_seq = c.max_blocks_per_seq;
     ps.scale = 1.0f / std::sqrt((float)c.head_dim);
-    for (uint32_t b = 0; b < B; ++b) ps.ctx_hint = std::max(ps.ctx_hint, d->host_lens[b] + lc);
+    ps.ctx_hint = ctx_max;
+    ps.row_start = row_start;
+    ps.rows = M;
 
     // A pass of 65 to a few hundred rows runs its narrow projections on the weight-stationary kernel, which takes
     // activation tiles (the decode kernels' layout) instead of row-major codes: the quantizer in front of such a
@@ -469,7 +472,6 @@ fa_status enqueue_prefill_chunk(fa_context *ctx, fa_decoder *d, PrefillBuffers &
         k::swiglu_quantize_rows_i8(t.gu.as<float>(), t.xq.as<int8_t>(), t.sx.as<float>(), M, F, s, rows_form(L.wdown), swiglu_in_gemm);
         gemm(L.wdown, t.h.as<float>(), t.h.as<float>());
     }
-    if (padded) k::trim_seq_lens((uint32_t *)d->seq_lens->ptr, t.row_lens.as<uint32_t>(), B, lc, s);
     if (every_row) {
         // verification: the head over every row of the chunk (row b * lc + t is token t of sequence b)
         norm_quantize((const float *)d->final_norm->ptr, d->lm_head);
@@ -877,8 +879,9 @@ static fa_status prefill_impl(fa_context *ctx, fa_decoder *d, const int32_t *tok
     constexpr uint64_t kRowsChecked = 4096;
     if ((verify || padded) && (uint64_t)B * l_new > kRowsChecked)
         return fail(FA_ERR_INVALID_ARGUMENT, "decoder: at most 4096 rows (batch x tokens) per verification or padded prompt pass");
-    const uint32_t lc_max = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(l_new, kRows / B));
-    const uint64_t M = (uint64_t)B * lc_max;
+    const uint32_t lc_max = padded ? l_new : (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(l_new, kRows / B));
+    uint64_t M = (uint64_t)B * lc_max;                    // a padded pass is one chunk and leaves the padding out
+    if (padded) M = std::accumulate(row_lens, row_lens + B, (uint64_t)0);
     const uint64_t D = c.d_model, F = c.d_ffn, EQ = (uint64_t)c.n_heads * c.head_dim, EKV = (uint64_t)c.n_kv_heads * c.head_dim;
     const uint64_t kmax = std::max(std::max(D, F), EQ);
     PrefillBuffers t(ctx, d);
@@ -913,7 +916,7 @@ static fa_status prefill_impl(fa_context *ctx, fa_decoder *d, const int32_t *tok
         get(t.all_logits, M * c.vocab * 4);
         get(t.all_picked, M * 4);
     }
-    if (padded) get(t.row_lens, (uint64_t)B * 4);
+    if (padded) get(t.row_start, (uint64_t)(B + 1) * 4);
     if (st != FA_OK) return st;
     k::PagedShape ps{};
     ps.batch = B;
@@ -924,18 +927,27 @@ static fa_status prefill_impl(fa_context *ctx, fa_decoder *d, const int32_t *tok
     if (fa_status s = ensure_workspace(ctx, k::paged_prefill_workspace_bytes(ps, (uint32_t)g_decode_waves))) return s;
 
     std::vector<int32_t> stage;
+    std::vector<uint32_t> starts;
     try {
         stage.resize(M);
+        starts.resize(B + 1);
     } catch (const std::exception &) {
         return fail(FA_ERR_ALLOCATION_FAILED, "decoder_prefill: out of host memory");
     }
     for (uint32_t t0 = 0; t0 < l_new; t0 += lc_max) {
         const uint32_t lc = std::min(lc_max, l_new - t0);
-        for (uint32_t b = 0; b < B; ++b)
-            for (uint32_t i = 0; i < lc; ++i) stage[(uint64_t)b * lc + i] = tokens[(uint64_t)b * l_new + t0 + i];
-        const Upload parts[2] = {{t.tok.ptr, stage.data(), (uint64_t)B * lc * 4}, {t.row_lens.ptr, row_lens, (uint64_t)B * 4}};
+        uint32_t rows = 0, ctx_max = 0;
+        for (uint32_t b = 0; b < B; ++b) {
+            const uint32_t n = padded ? row_lens[b] : lc;
+            starts[b] = rows;
+            std::copy_n(tokens + (uint64_t)b * l_new + t0, n, stage.begin() + rows);
+            rows += n;
+            ctx_max = std::max(ctx_max, d->host_lens[b] + n);
+        }
+        starts[B] = rows;
+        const Upload parts[2] = {{t.tok.ptr, stage.data(), (uint64_t)rows * 4}, {t.row_start.ptr, starts.data(), (uint64_t)(B + 1) * 4}};
         if (fa_status s = queue_uploads(ctx, parts, padded ? 2 : 1, "prompt token upload")) return s;
-        if (fa_status s = enqueue_prefill_chunk(ctx, d, t, lc, t0 + lc == l_new, verify, padded)) return s;
+        if (fa_status s = enqueue_prefill_chunk(ctx, d, t, lc, rows, ctx_max, t0 + lc == l_new, verify, padded)) return s;
         for (uint32_t b = 0; b < B; ++b) d->host_lens[b] += padded ? row_lens[b] : lc;
     }
     if (verify) {

@@ -40,16 +40,36 @@ __global__ void __launch_bounds__(64)
     }
 }
 
-// Prompt chunk of l_chunk tokens per sequence: row r = b * l_chunk + t sits at position seq_lens[b] + t.
+// The last sequence b < batch with row_start[b] <= r: the one that row r of a pass belongs to
+__device__ __forceinline__ uint32_t sequence_of(const uint32_t *row_start, uint32_t batch, uint32_t r) {
+    uint32_t lo = 0, hi = batch;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (row_start[mid] <= r) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Prompt chunk of l_chunk tokens per sequence: row r = b * l_chunk + t sits at position seq_lens[b] + t.  With row_start, prompts
+// of different lengths behind one another: row r = row_start[b] + t.
 // Same cos / sin arithmetic as the decode step, so a prompt token and the same token decoded later rotate
 // identically.  seq_lens is advanced by a second launch, after every block of this one has read it.
 __global__ void __launch_bounds__(64)
     prefill_prepare_kernel(const uint32_t *__restrict__ tables, const uint32_t *__restrict__ seq_lens,
-                           uint32_t *__restrict__ slots, float *__restrict__ cos_sin, uint32_t l_chunk,
+                           const uint32_t *__restrict__ row_start, uint32_t *__restrict__ slots, float *__restrict__ cos_sin, uint32_t batch,
+                           uint32_t l_chunk,
                            uint32_t block_size, uint32_t max_blocks_per_seq, uint32_t num_blocks, uint32_t head_dim,
                            double theta) {
-    const uint32_t t = blockIdx.x, b = blockIdx.y;
-    const uint64_t r = (uint64_t)b * l_chunk + t;
+    const uint64_t r = blockIdx.x;
+    uint32_t b, t;
+    if (row_start) {
+        b = sequence_of(row_start, batch, blockIdx.x);
+        t = blockIdx.x - row_start[b];
+    } else {
+        b = blockIdx.x / l_chunk;
+        t = blockIdx.x % l_chunk;
+    }
     const uint32_t p = seq_lens[b] + t;
     const uint32_t half = head_dim / 2;
     for (uint32_t i = threadIdx.x; i < half; i += 64) {
@@ -69,23 +89,14 @@ __global__ void __launch_bounds__(64)
     }
 }
 
-// row_lens (optional): row b's prompt is only row_lens[b] <= l_chunk tokens long and the rest of its chunk
-// is padding; its last token is then row b * l_chunk + row_lens[b] - 1.  seq_lens advances by the whole chunk
-// either way (the attention of the pass places token t at seq_len - l_chunk + t); trim_lens_kernel takes the
-// padding off afterwards.
-__global__ void advance_lens_kernel(uint32_t *__restrict__ seq_lens, int32_t *__restrict__ last_rows, uint32_t batch,
-                                    uint32_t l_chunk, const uint32_t *__restrict__ row_lens) {
+__global__ void advance_lens_kernel(uint32_t *__restrict__ seq_lens, int32_t *__restrict__ last_rows, const uint32_t *__restrict__ row_start,
+                                    uint32_t batch, uint32_t l_chunk) {
     const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b < batch) {
-        seq_lens[b] += l_chunk;
-        last_rows[b] = (int32_t)(b * l_chunk + (row_lens ? row_lens[b] : l_chunk) - 1);
+        const uint32_t first = row_start ? row_start[b] : b * l_chunk, end = row_start ? row_start[b + 1] : first + l_chunk;
+        seq_lens[b] += end - first;
+        last_rows[b] = (int32_t)(end - 1);
     }
-}
-
-__global__ void trim_lens_kernel(uint32_t *__restrict__ seq_lens, const uint32_t *__restrict__ row_lens, uint32_t batch,
-                                 uint32_t l_chunk) {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < batch) seq_lens[b] -= l_chunk - row_lens[b];
 }
 
 // qkv [rows, (heads + 2 kv_heads) head_dim] f32 -> q rotated, bf16 [rows, heads head_dim]; K rotated and V
@@ -134,12 +145,7 @@ __global__ void __launch_bounds__(256)
                           uint32_t block_size, uint32_t max_blocks, uint32_t num_blocks) {
     const uint32_t r = blockIdx.x * 256 + threadIdx.x;
     if (r >= rows) return;
-    uint32_t lo = 0, hi = batch;                     // the last b with row_start[b] <= r
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) / 2;
-        if (row_start[mid] <= r) lo = mid;
-        else hi = mid;
-    }
+    const uint32_t lo = sequence_of(row_start, batch, r);
     const uint32_t p = seq_lens[lo] + (r - row_start[lo]);
     uint32_t slot = 0xffffffffu;
     if (p / block_size < max_blocks) {
@@ -186,23 +192,17 @@ void rotation_table(const int32_t *pos, float *cos_sin, uint32_t rows, uint32_t 
     rotation_table_kernel<<<rows, 64, 0, s>>>(pos, cos_sin, dims, freq);
 }
 
-void prefill_prepare(const uint32_t *tables, const uint32_t *seq_lens, uint32_t *slots, float *cos_sin, uint32_t batch,
-                     uint32_t l_chunk, uint32_t block_size, uint32_t max_blocks_per_seq, uint32_t num_blocks,
+void prefill_prepare(const uint32_t *tables, const uint32_t *seq_lens, const uint32_t *row_start, uint32_t *slots, float *cos_sin,
+                     uint32_t rows, uint32_t batch, uint32_t l_chunk, uint32_t block_size, uint32_t max_blocks_per_seq, uint32_t num_blocks,
                      uint32_t head_dim, double theta, hipStream_t s) {
-    if (batch == 0 || l_chunk == 0) return;
-    prefill_prepare_kernel<<<dim3(l_chunk, batch), 64, 0, s>>>(tables, seq_lens, slots, cos_sin, l_chunk, block_size,
-                                                              max_blocks_per_seq, num_blocks, head_dim, theta);
+    if (rows == 0) return;
+    prefill_prepare_kernel<<<rows, 64, 0, s>>>(tables, seq_lens, row_start, slots, cos_sin, batch, l_chunk, block_size, max_blocks_per_seq,
+                                               num_blocks, head_dim, theta);
 }
 
-void advance_seq_lens(uint32_t *seq_lens, int32_t *last_rows, uint32_t batch, uint32_t l_chunk, const uint32_t *row_lens,
-                      hipStream_t s) {
+void advance_seq_lens(uint32_t *seq_lens, int32_t *last_rows, const uint32_t *row_start, uint32_t batch, uint32_t l_chunk, hipStream_t s) {
     if (batch == 0) return;
-    advance_lens_kernel<<<(batch + 63) / 64, 64, 0, s>>>(seq_lens, last_rows, batch, l_chunk, row_lens);
-}
-
-void trim_seq_lens(uint32_t *seq_lens, const uint32_t *row_lens, uint32_t batch, uint32_t l_chunk, hipStream_t s) {
-    if (batch == 0) return;
-    trim_lens_kernel<<<(batch + 63) / 64, 64, 0, s>>>(seq_lens, row_lens, batch, l_chunk);
+    advance_lens_kernel<<<(batch + 63) / 64, 64, 0, s>>>(seq_lens, last_rows, row_start, batch, l_chunk);
 }
 
 void rope_append(const float *qkv, const float *cos_sin, const uint32_t *slots, uint16_t *q_out, uint16_t *k_pool,

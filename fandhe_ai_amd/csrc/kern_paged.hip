@@ -166,6 +166,7 @@ struct StreamParams {
     // per tpv new tokens.  One launch covers the new tokens [t0, t0 + qt * tpv) of every sequence.
     // Decode: l_new = tpt = tpv = qt = 1, t0 = 0.
     uint32_t l_new, tpt, tpv, qt, t0, n_vseq;
+    const uint32_t *row_start = nullptr;                    // prefill of sequences of different lengths (PagedShape::row_start)
     // ONE form only (decode_stream_kernel<..., ONE = true>): the finished attention output, f32 values already rounded
     // to bf16 (the operator's output type), [batch][num_heads][128], and the absmax of every head's slice
     float *one_out = nullptr, *one_pmax = nullptr;
@@ -176,6 +177,18 @@ struct StreamParams {
     uint32_t *one_counters = nullptr;
 };
 
+// The new tokens of sequence b: rows first .. first + n - 1 of the pass
+struct NewRows {
+    uint64_t first;
+    uint32_t n;
+};
+template <typename P>
+__device__ __forceinline__ NewRows new_rows(const P &p, uint32_t b) {
+    if (!p.row_start) return {(uint64_t)b * p.l_new, p.l_new};
+    const uint32_t lo = p.row_start[b], hi = p.row_start[b + 1];
+    return {lo, hi - lo};
+}
+
 // Length of (virtual) sequence vs: all cached positions up to the last new token of its tile.  A row whose
 // length is below l_new (possible only with unvalidated device tables) streams nothing.
 template <bool PF>
@@ -183,11 +196,11 @@ __device__ __forceinline__ uint32_t vseq_len(const StreamParams &p, uint32_t vs)
     if constexpr (!PF) {
         return p.seq_lens[vs];
     } else {
-        const uint32_t len = p.seq_lens[vs / p.qt];
-        if (len < p.l_new) return 0;
+        const uint32_t len = p.seq_lens[vs / p.qt], l_new = new_rows(p, vs / p.qt).n;
         uint32_t after = p.t0 + (vs % p.qt + 1) * p.tpv;
-        if (after > p.l_new) after = p.l_new;
-        return len - p.l_new + after;
+        if (len < l_new || after - p.tpv >= l_new) return 0;
+        if (after > l_new) after = l_new;
+        return len - l_new + after;
     }
 }
 template <bool PF>
@@ -269,13 +282,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
                 }
             } else {
                 const uint32_t tl = (uint32_t)c / p.group, hc = (uint32_t)c % p.group;
+                const NewRows nr = new_rows(p, b);
 #pragma unroll
                 for (int tt = 0; tt < TT; ++tt) {
                     const uint32_t t = p.t0 + (vq % p.qt) * p.tpv + tt * p.tpt + tl;
-                    const bool valid = tl < p.tpt && t < p.l_new;
+                    const bool valid = tl < p.tpt && t < nr.n;
                     const uint32_t tc = valid ? t : 0;
                     const uint16_t *qrow =
-                        p.q + (((uint64_t)b * p.l_new + tc) * p.num_heads + (uint64_t)kvh * p.group + hc) * kDh + 8 * g;
+                        p.q + ((nr.first + tc) * p.num_heads + (uint64_t)kvh * p.group + hc) * kDh + 8 * g;
 #pragma unroll
                     for (int s = 0; s < 4; ++s) {
                         v4u t4 = *(const v4u *)(qrow + 32 * s);
@@ -284,7 +298,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
                     }
                     // cached positions before the new tokens + new tokens up to and including t; never above
                     // ctx, which is already clamped to what the table can describe
-                    const uint32_t lim = p.seq_lens[b] - p.l_new + t + 1;
+                    const uint32_t lim = p.seq_lens[b] - nr.n + t + 1;
                     ctx_l[tt] = valid && lim < ctx ? lim : ctx;
                 }
             }
@@ -768,11 +782,12 @@ __global__ void __launch_bounds__(kPrefillMergeThreads)
     uint32_t r_lo, r_hi;
     ixm::stream_merge_ranges(pre, npg, per, &r_lo, &r_hi);   // nothing streamed: no partials
     const uint32_t seq = vq / p.qt, tiles = p.tpv / p.tpt, cols = p.tpt * p.group;
-    const bool violation = p.seq_lens[seq] < p.l_new;              // possible only with unvalidated device tables
+    const NewRows nr = new_rows(p, seq);
+    const bool violation = p.seq_lens[seq] < nr.n;                 // possible only with unvalidated device tables
     for (uint32_t ci = part; ci < tiles * cols; ci += kSlots) {
         const uint32_t tile = ci / cols, col = ci % cols;
         const uint32_t t = p.t0 + (vq % p.qt) * p.tpv + tile * p.tpt + col / p.group;
-        if (t >= p.l_new) continue;
+        if (t >= nr.n) continue;
         float mx = -INFINITY;
         for (uint32_t r = r_lo; r <= r_hi; ++r) {
             float m = p.part_ml[(((uint64_t)(r + vq) * p.num_kv_heads + kvh) * tiles + tile) * (2 * p.g_pad) + col];
@@ -789,7 +804,7 @@ __global__ void __launch_bounds__(kPrefillMergeThreads)
         }
         float res = npg == 0 ? 0.0f : __fdiv_rn(acc, den);
         if (violation) res = __uint_as_float(0x7fc00000u);
-        const uint64_t oi = (((uint64_t)seq * p.l_new + t) * p.num_heads + (uint64_t)kvh * p.group + col % p.group) * kDh + d;
+        const uint64_t oi = ((nr.first + t) * p.num_heads + (uint64_t)kvh * p.group + col % p.group) * kDh + d;
         if (out_bf16)
             ((uint16_t *)out)[oi] = f32_to_bf16(res);
         else
@@ -989,6 +1004,7 @@ struct FlashParams {
     // part_o [tile block][y][column][128] / part_ml [tile block][y][2][columns]; flash_split_merge_kernel adds them.
     uint32_t nsplit;
     float *part_o, *part_ml;
+    const uint32_t *row_start;          // sequences of different lengths (PagedShape::row_start); l_new is the longest's
 };
 constexpr int kFlashNW = 4, kFlashNQ = 2, kFlashKeys = 32;
 
@@ -1041,11 +1057,13 @@ __global__ void __launch_bounds__(kFlashNW * 64) __attribute__((amdgpu_waves_per
     const uint32_t b = (blockIdx.x % per_tile) / p.num_kv_heads, kvh = blockIdx.x % p.num_kv_heads;
     const uint32_t max_ctx = p.max_blocks_per_seq * kPage;
     const uint32_t len = p.seq_lens[b];
-    const bool violation = len < p.l_new || len > max_ctx;     // possible only with unvalidated device tables
-    const uint32_t ctx = len > max_ctx ? max_ctx : len;
-    const uint32_t base = violation ? 0 : len - p.l_new;       // cached positions before the new tokens
+    const NewRows nr = new_rows(p, b);
     const uint32_t t0 = tile * p.tq;
-    const uint32_t t_end = t0 + p.tq < p.l_new ? t0 + p.tq : p.l_new;
+    if (t0 >= nr.n) return;                                    // a tile that only longer sequences have
+    const bool violation = len < nr.n || len > max_ctx;     // possible only with unvalidated device tables
+    const uint32_t ctx = len > max_ctx ? max_ctx : len;
+    const uint32_t base = violation ? 0 : len - nr.n;       // cached positions before the new tokens
+    const uint32_t t_end = t0 + p.tq < nr.n ? t0 + p.tq : nr.n;
     uint32_t kmax = violation ? 0 : base + t_end;              // positions the last token of the tile sees
     if (kmax > ctx) kmax = ctx;
     const uint32_t npages = (kmax + kPage - 1) / kPage, n_all = (kmax + kFlashKeys - 1) / kFlashKeys;
@@ -1072,9 +1090,9 @@ __global__ void __launch_bounds__(kFlashNW * 64) __attribute__((amdgpu_waves_per
     for (int qi = 0; qi < NQ; ++qi) {
         const uint32_t col = (uint32_t)wave * (NQ * 16) + qi * 16 + c;
         const uint32_t t = t0 + col / p.group, hc = col % p.group;
-        valid[qi] = col < p.tq * p.group && t < p.l_new;        // a group that does not divide the columns leaves some idle
+        valid[qi] = col < p.tq * p.group && t < nr.n;        // a group that does not divide the columns leaves some idle
         const uint32_t tc = valid[qi] ? t : 0;
-        out_row[qi] = (((uint64_t)b * p.l_new + tc) * p.num_heads + (uint64_t)kvh * p.group + hc) * kDh;
+        out_row[qi] = ((nr.first + tc) * p.num_heads + (uint64_t)kvh * p.group + hc) * kDh;
         const uint16_t *qrow = p.q + out_row[qi] + 8 * g;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -1316,7 +1334,8 @@ __global__ void __launch_bounds__(1024) flash_split_merge_kernel(FlashParams p) 
     const uint32_t b = (blockIdx.x % per_tile) / p.num_kv_heads, kvh = blockIdx.x % p.num_kv_heads;
     const uint32_t d = threadIdx.x % 128, col = blockIdx.y * 8 + threadIdx.x / 128;
     const uint32_t t = tile * p.tq + col / p.group;
-    if (col >= p.tq * p.group || t >= p.l_new) return;
+    const NewRows nr = new_rows(p, b);
+    if (col >= p.tq * p.group || t >= nr.n) return;
     const float *ml = p.part_ml + (uint64_t)blockIdx.x * p.nsplit * (2 * kCols) + col;
     const float *po = p.part_o + ((uint64_t)blockIdx.x * p.nsplit * kCols + col) * kDh + d;
     const uint32_t last = p.nsplit - 1;
@@ -1348,7 +1367,7 @@ __global__ void __launch_bounds__(1024) flash_split_merge_kernel(FlashParams p) 
     }
     float res = den > 0.0f ? __fdiv_rn(acc, den) : 0.0f;
     if (mx != mx) res = mx;
-    const uint64_t oi = (((uint64_t)b * p.l_new + t) * p.num_heads + (uint64_t)kvh * p.group + col % p.group) * kDh + d;
+    const uint64_t oi = ((nr.first + t) * p.num_heads + (uint64_t)kvh * p.group + col % p.group) * kDh + d;
     if (p.out_bf16)
         ((uint16_t *)p.out)[oi] = f32_to_bf16(res);
     else
@@ -1570,6 +1589,11 @@ struct BlockFormPlan {
     bool use;
     uint32_t nsplit;                    // blocks sharing a tile's walk (1: none)
 };
+// Blocks with work: a sequence's last tile is half full on average where the lengths differ
+static uint64_t flash_blocks(const PagedShape &ps, uint32_t tq) {
+    if (!ps.row_start) return (uint64_t)ps.batch * ps.num_kv_heads * ((ps.l_new + tq - 1) / tq);
+    return (uint64_t)ps.num_kv_heads * (ps.rows / tq + (ps.batch + 1) / 2);
+}
 static BlockFormPlan plan_block_form(const PagedShape &ps) {
     const uint32_t group = ps.num_heads / ps.num_kv_heads;
     if (group == 0 || group > 16 || g_prefill_block_form == 1) return {false, 1};
@@ -1585,9 +1609,9 @@ static BlockFormPlan plan_block_form(const PagedShape &ps) {
     // long): several blocks share a tile's walk (at least eight steps each, at most as many shares as the
     // workspace holds) and a merge pass adds them
     uint32_t nsplit = 1;
-    const uint64_t blocks = rows * tiles;
+    const uint64_t blocks = flash_blocks(ps, tq);
     if (blocks < cus && cached >= 2.0 * l_new) {
-        uint64_t want = flash_split_slots() / blocks, by_steps = (uint64_t)(steps_longest / 8.0);
+        uint64_t want = flash_split_slots() / (rows * tiles), by_steps = (uint64_t)(steps_longest / 8.0);
         if (g_prefill_block_split > 0) want = (uint64_t)g_prefill_block_split < want ? (uint64_t)g_prefill_block_split : want;
         nsplit = (uint32_t)(want < by_steps ? want : by_steps);
         if (nsplit < 1) nsplit = 1;
@@ -1633,12 +1657,13 @@ void paged_attention_prefill_bf16(const uint16_t *q, const uint16_t *k_pool, con
         // 34.5, 92 and 84, 3000 (752) 157 and 156, 8 x 512 (1024) 56 and 61.  Only the unsplit form.
         const bool narrow = g_prefill_block_cols != 2 && plan.nsplit == 1 && fp.group <= 16 && 16 % fp.group == 0 &&
                             (g_prefill_block_cols == 1 ||
-                             (uint64_t)ps.batch * ps.num_kv_heads * fp.tiles <= 2 * (uint64_t)compute_units());
+                             flash_blocks(ps, fp.tq) <= 2 * (uint64_t)compute_units());
         if (narrow) {
             fp.tq = kFlashNW * 16 / fp.group;
             fp.tiles = (ps.l_new + fp.tq - 1) / fp.tq;
         }
         const uint64_t blocks = (uint64_t)ps.batch * ps.num_kv_heads * fp.tiles;
+        fp.row_start = ps.row_start;
         fp.nsplit = plan.nsplit;
         fp.part_o = (float *)workspace;
         fp.part_ml = fp.part_o + blocks * fp.nsplit * kFlashSplitCols * kDh;
@@ -1668,6 +1693,7 @@ void paged_attention_prefill_bf16(const uint16_t *q, const uint16_t *k_pool, con
     sp.min_pages = 4;
     sp.scale = ps.scale;
     sp.l_new = ps.l_new;
+    sp.row_start = ps.row_start;
     sp.tpt = 16 / sp.group;
     const uint32_t tt = prefill_tt(ps);
     sp.tpv = sp.tpt * tt;

@@ -283,6 +283,10 @@ struct PagedShape {
     // upper bound the host knows for the positions any row holds after this call's new tokens (0: unknown,
     // the table width is used); only steers the choice between the two prefill forms
     uint32_t ctx_hint = 0;
+    // prefill of sequences with different numbers of new tokens (device, [batch + 1], null: l_new each): those of sequence b are rows
+    // row_start[b] .. row_start[b + 1] - 1 of q and out, `rows` of them in all; l_new is the longest's
+    const uint32_t *row_start = nullptr;
+    uint64_t rows = 0;
 };
 // Row scatter; elem_bytes 2 or 4; slots bounds-checked against pool_rows.
 void paged_kv_append(const void *k_new, const void *v_new, void *k_pool, void *v_pool,
@@ -661,16 +665,13 @@ void decode_prepare(const uint32_t *tables, uint32_t *seq_lens, int32_t *pos, ui
                     uint32_t batch, uint32_t block_size, uint32_t max_blocks_per_seq, uint32_t num_blocks,
                     uint32_t head_dim, double theta, hipStream_t s);
 
-// Prompt chunks (several new tokens per sequence): row b * l_chunk + t is at position seq_lens[b] + t;
-// slots [batch * l_chunk] and the cos/sin table [batch * l_chunk, head_dim] as in decode_prepare.
-void prefill_prepare(const uint32_t *tables, const uint32_t *seq_lens, uint32_t *slots, float *cos_sin, uint32_t batch,
-                     uint32_t l_chunk, uint32_t block_size, uint32_t max_blocks_per_seq, uint32_t num_blocks,
+// Prompt chunks (several new tokens per sequence): row b * l_chunk + t is at position seq_lens[b] + t, with row_start
+// ([batch + 1], else null) row row_start[b] + t; slots [rows] and the cos/sin table [rows, head_dim] as in decode_prepare.
+void prefill_prepare(const uint32_t *tables, const uint32_t *seq_lens, const uint32_t *row_start, uint32_t *slots, float *cos_sin,
+                     uint32_t rows, uint32_t batch, uint32_t l_chunk, uint32_t block_size, uint32_t max_blocks_per_seq, uint32_t num_blocks,
                      uint32_t head_dim, double theta, hipStream_t s);
-// seq_lens[b] += l_chunk; last_rows[b] = row of the chunk's last token of sequence b
-void advance_seq_lens(uint32_t *seq_lens, int32_t *last_rows, uint32_t batch, uint32_t l_chunk, const uint32_t *row_lens,
-                      hipStream_t s);
-// After a padded prompt pass: seq_lens[b] -= l_chunk - row_lens[b].
-void trim_seq_lens(uint32_t *seq_lens, const uint32_t *row_lens, uint32_t batch, uint32_t l_chunk, hipStream_t s);
+// seq_lens[b] advances by the sequence's rows; last_rows[b] = row of the chunk's last token of sequence b
+void advance_seq_lens(uint32_t *seq_lens, int32_t *last_rows, const uint32_t *row_start, uint32_t batch, uint32_t l_chunk, hipStream_t s);
 // RoPE on the q and k heads of qkv [rows, (heads + 2 kv_heads) head_dim] (f32), one rounding to bf16;
 // q to q_out [rows, heads head_dim], K / V to pool row slots[r].
 void rope_append(const float *qkv, const float *cos_sin, const uint32_t *slots, uint16_t *q_out, uint16_t *k_pool,

@@ -530,9 +530,8 @@ fa_status fa_decoder_prefill(fa_context *ctx, fa_decoder *dec, const int32_t *to
  * [batch] is a host array with 1 <= row_lens[b] <= l_max, batch * l_max <= 4096.
  * Every row ends as if it had been ingested alone with fa_decoder_prefill: its
  * length advances by row_lens[b], the logits and the next token are those of
- * its own last prompt token.  The padding is computed and thrown away: its
- * cache rows land past the sequence's length (in pages the row owns, if any;
- * positions without a page are skipped) and are overwritten by later tokens.
+ * its own last prompt token.  The padding is left out: nothing is computed for
+ * it and no cache row is written past a prompt's own tokens.
  * What a scheduler uses when several requests join in the same iteration
  * (crates/autodiff/src/generate/scheduler.rs:521-562 admits them one by one). */
 fa_status fa_decoder_prefill_padded(fa_context *ctx, fa_decoder *dec, const int32_t *tokens, uint32_t l_max,

@@ -435,3 +435,60 @@ def test_padded_prompt_pass_leaves_every_row_as_its_own_prompt_pass_would():
     assert fa.capi.lib.fa_decoder_prefill_padded(ops()._ctx, dec._h, pad.ctypes.data_as(fa.capi.i32p), 5,
                                                  lens.ctypes.data_as(fa.capi.u32p)) == fa.capi.INVALID_ARGUMENT
     dec.close()
+
+
+@pytest.mark.parametrize("form", [{10: 2, 23: 1}, {10: 2, 23: 2}, {10: 2, 12: 4}, {10: 1}], ids=["narrow", "wide", "split", "streamed"])
+@pytest.mark.parametrize("cached,lens", [(0, (1, 33, 16, 32)), (16, (17, 1, 40)), (150, (2, 31, 5))])
+def test_padded_pass_without_its_padding(cached, lens, form):
+    """Prompts of lengths around the attention's tiles, also behind cached tokens, in every form of the prompt attention: the logits and
+    the cache rows of each are those of its own pass (the chained-step bar), and rows of the pages behind its tokens stay as they were."""
+    import fandhe_ai_amd as fa
+    pages = (cached + max(lens) + 15) // 16
+    dec = _decoder(max_blocks_per_seq=pages, num_blocks=pages * len(lens), max_batch=4)
+    rng = np.random.default_rng(cached + len(lens))
+    tables = rng.permutation(pages * len(lens)).astype(np.uint32).reshape(len(lens), pages)
+    before = [rng.integers(0, VOCAB, cached).astype(np.int32) for _ in lens]
+    prompts = [rng.integers(0, VOCAB, n).astype(np.int32) for n in lens]
+    pools = []
+    for i in range(L):
+        k, v = fa.capi.buf_p(), fa.capi.buf_p()
+        fa.check(fa.capi.lib.fa_decoder_kv_pools(dec._h, i, k, v))
+        pools += [k, v]
+
+    def contents():
+        out = np.empty((len(pools), pages * len(lens), 16, KV * (D // HEADS)), dtype=np.uint16)
+        for a, h in zip(out, pools):
+            fa.check(fa.capi.lib.fa_download(ops()._ctx, h, 0, a.ctypes.data, a.size))
+        return out
+
+    alone = []
+    for b, prompt in enumerate(prompts):
+        dec.set_sequences(tables[b:b + 1], np.zeros(1, np.uint32))
+        if cached:
+            dec.prefill(before[b][None])
+        dec.prefill(prompt[None])
+        alone.append(dec.logits()[0].copy())
+    want = contents()
+    try:
+        for key, value in form.items():
+            fa.check(fa.capi.lib.fa_set_tuning(key, value))
+        dec.set_sequences(tables, np.full(len(lens), cached, np.uint32))
+        dec.prefill_padded(prompts)
+        got = dec.logits()
+    finally:
+        for key in form:
+            fa.check(fa.capi.lib.fa_set_tuning(key, 0))
+    assert dec.seq_lens().tolist() == [cached + n for n in lens]
+    for b in range(len(lens)):
+        err = np.abs(got[b] - alone[b]) / float(alone[b].max() - alone[b].min())
+        assert np.isfinite(got[b]).all() and err.mean() < 2e-4 and err.max() < 2e-2, (b, err.mean(), err.max())
+    have = contents()
+    for b, n in enumerate(lens):
+        own = np.arange(cached + n)
+        rows = (slice(None), tables[b][own // 16], own % 16)
+        a, w = [(x[rows].astype(np.uint32) << 16).view(np.float32) for x in (have, want)]
+        assert np.abs(a - w).max() <= 2e-2 * np.abs(w).max()
+        rest = np.arange(cached + n, 16 * pages)
+        rows = (slice(None), tables[b][rest // 16], rest % 16)
+        assert np.array_equal(have[rows], want[rows])
+    dec.close()
