@@ -187,17 +187,25 @@ __device__ __forceinline__ void quant_i8_words(const V (&x)[N], float scale, uin
     }
 }
 
-// x * sigmoid(x) with the two-branch sigmoid of crates/tensor-core/src/scalar_op.rs:666-673 (and :355)
-__device__ __forceinline__ float silu_f32(float x) {
-    float s;
-    if (x >= 0.0f) {
-        s = __fdiv_rn(1.0f, 1.0f + expf(-x));
-    } else {
-        float e = expf(x);
-        s = __fdiv_rn(e, 1.0f + e);
-    }
-    return x * s;
+// e^-|x|, about one unit in the last place down to the subnormal range: 2^r 2^f with the product by log2(e) kept in two parts.  Needs
+// none of expf's selects for large arguments.
+__device__ __forceinline__ float exp_minus_abs(float x) {
+    constexpr float kHi = 1.44269502f, kLo = 1.92596303e-8f;          // log2(e)
+    const float a = __builtin_elementwise_maximum(-fabsf(x), -256.0f);    // 2^-369 is zero; a NaN stays one
+    const float t = a * kHi, lo = __builtin_fmaf(a, kLo, __builtin_fmaf(a, kHi, -t)), r = rintf(t);
+    return __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f((t - r) + lo), (int)r);
 }
+// 1 / (1 + e^-x) with the two-branch form of crates/tensor-core/src/scalar_op.rs:666-673: both branches take the same exponential,
+// e = e^-|x|, and divide 1 or e by 1 + e.  The denominator lies in [1, 2], so the quotient needs no scaling: an estimate and its
+// remainder's correction, rounded once (off the nearest value only where that is a tie to about 2^-24).
+__device__ __forceinline__ float sigmoid_f32(float x) {
+    const float e = exp_minus_abs(x), d = 1.0f + e, num = x >= 0.0f ? 1.0f : e;
+    const float y = __builtin_amdgcn_rcpf(d), q = num * y;
+    return __builtin_fmaf(__builtin_fmaf(-d, q, num), y, q);
+}
+// x * sigmoid(x) (crates/tensor-core/src/scalar_op.rs:355).  18 instructions: with expf in either branch and a scaled division it was
+// 46, and the SwiGLU epilogue of a 256 x 256 tile is 128 of them to a lane (see kern_gemm_mfma.hip).
+__device__ __forceinline__ float silu_f32(float x) { return x * sigmoid_f32(x); }
 
 // byte offset of the 16-byte chunk `chunk` (= k / 16) of activation row r in the 16-row x 64-k tile order
 // of the quantized activations

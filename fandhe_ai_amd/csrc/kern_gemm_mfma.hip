@@ -723,6 +723,39 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     if constexpr (BF16) {
         constexpr int MODE = IsBf16<Epi>::mode, STEP = is_glu(MODE) ? 2 : 1;      // gate, up: neighbouring tiles
         static_assert(STEP == 1 || WNT % 2 == 0, "a gate tile and its up tile belong to one wavefront");
+        if constexpr (MODE == LinearEpilogue::kResidual) {
+            // The stream is read and written in place, so the compiler keeps every read behind the writes before it: a memory round
+            // trip per tile.  Here four tiles are requested while the four before them are added.
+            const uint32_t col0 = (nt0 + wn * WNT) * 16;
+            if (nt0 + wn * WNT + WNT <= n_tiles && col0 + WNT * 16 <= n && ep.ep.ld_out % 4 == 0) {
+                float *base = (float *)ep.ep.out + col0 + 4 * g;
+                const float *scale = ep.ep.scale ? ep.ep.scale + col0 + 4 * g : nullptr;
+                constexpr int TILES = AI * WNT, STEP_T = 4;       // tiles requested together (all of a row's: spills)
+                v4f res[2][STEP_T];
+                auto place = [&](int q) {
+                    const uint32_t row = m0 + row_l0 + q / WNT * 16;
+                    return base + (uint64_t)(row < m ? row : m - 1) * ep.ep.ld_out + q % WNT * 16;
+                };
+                auto request = [&](int q0) {
+#pragma unroll
+                    for (int q = q0; q < q0 + STEP_T && q < TILES; ++q) res[q0 / STEP_T % 2][q - q0] = *(const v4f *)place(q);
+                };
+                request(0);
+#pragma unroll
+                for (int q0 = 0; q0 < TILES; q0 += STEP_T) {
+                    request(q0 + STEP_T);
+#pragma unroll
+                    for (int q = q0; q < q0 + STEP_T && q < TILES; ++q) {
+                        const v4f ls = scale ? *(const v4f *)(scale + q % WNT * 16) : v4f{1.0f, 1.0f, 1.0f, 1.0f};
+                        hold_acc(acc[q / WNT][q % WNT]);      // not copied out ahead of the branch
+                        const v4f r = res[q0 / STEP_T % 2][q - q0], y = acc[q / WNT][q % WNT];
+                        if (m0 + row_l0 + q / WNT * 16 < m)
+                            *(v4f *)place(q) = v4f{r[0] + ls[0] * y[0], r[1] + ls[1] * y[1], r[2] + ls[2] * y[2], r[3] + ls[3] * y[3]};
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < AI; ++i) {
             uint32_t row = m0 + row_l0 + i * 16;
@@ -731,6 +764,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
             for (int j = 0; j < WNT; j += STEP) {
                 const uint32_t t = nt0 + wn * WNT + j;
+                if constexpr (MODE == LinearEpilogue::kResidual) hold_acc(acc[i][j]);
                 if (t < n_tiles) epilogue_store4<MODE>(ep.ep, row, t / STEP * 16 + 4 * g, n, 0, acc[i][j], acc[i][j + STEP - 1]);
             }
         }
@@ -849,6 +883,14 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
             for (int j = 0; j < WNT; ++j) swc[j] = *(const v4f *)(ep.sw + col0 + j * 16 + 4 * g);
         }
+        [[maybe_unused]] v4f ahead[WNT];              // residual of the next row: out may be the same buffer, so the compiler would read it
+        [[maybe_unused]] auto request = [&](int i) {  // behind this row's stores
+            const uint32_t row = m0 + row_l0 + i * 16;
+            const float *src = residual + (uint64_t)(row < m ? row : m - 1) * n + nt0 * 16 + col_l0;
+#pragma unroll
+            for (int j = 0; j < WNT; ++j) ahead[j] = *(const v4f *)(src + j * 16);
+        };
+        if constexpr (has_residual) request(0);
 #pragma unroll
         for (int i = 0; i < AI; ++i) {
             const uint32_t row = m0 + row_l0 + i * 16;
@@ -857,10 +899,13 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
             const uint64_t o0 = (uint64_t)(row_ok ? row : m - 1) * n + nt0 * 16 + col_l0;
             uint8_t *orow = (uint8_t *)ep.out + o0 * (to_bf16 ? 2 : 4);
             v4f add[WNT];                             // the bias (read for every row: no room for it beside the scales) or the residual
-            if constexpr (has_bias || has_residual) {
-                const float *src = has_bias ? bias + col0 + 4 * g : residual + o0;
+            if constexpr (has_residual) {
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) add[j] = *(const v4f *)(src + j * 16);
+                for (int j = 0; j < WNT; ++j) add[j] = ahead[j];
+                if (i + 1 < AI) request(i + 1);
+            } else if constexpr (has_bias) {
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) add[j] = *(const v4f *)(bias + col0 + 4 * g + j * 16);
             }
             v2u pk[WNT];                              // bf16 output: the four columns of tile j, packed
 #pragma unroll

@@ -7,7 +7,7 @@
 namespace fa {
 namespace k {
 
-__device__ __forceinline__ float sigmoid_f32(float z) { return 1.0f / (1.0f + expf(-z)); }
+using dev::sigmoid_f32;
 
 // The value the epilogue makes of y (and, for gate | up, of the up column's y).
 template <int MODE>
