@@ -4,6 +4,7 @@
 // The matrix instruction takes the weight tile as its first operand, so lane l of an accumulator tile holds row
 // l % 16 of the output and its columns 4 (l / 16) .. + 3.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_utils.hpp"
 #include "kernels.hpp"
@@ -13,114 +14,187 @@ namespace fa {
 namespace k {
 using namespace fa::dev;
 
-int g_linear_form = 0;        // tuning: 2 keeps the large-tile kernel out, 3 four column tiles per block; grouped rows: 4 streamed
+int g_linear_form = 0;        // tuning: 2 keeps the large-tile kernel out; grouped rows: 4 streamed
                               // weights, 5 128 x 128 tiles, 6 large tiles whatever the rows
 
 namespace {
 
 // ------------------------------------------------------------------ up to 64 rows
-// A block owns NTW column tiles; its wavefronts take every NWAVES-th k tile, stream weights and activations through a
-// ring of D register slots, and meet in LDS in a fixed order.  row_of(i): the activation row behind row i of the block's
-// rows (i < m; others repeat row 0 and are never stored) and the output row.
-template <int MT, int NTW, int NWAVES, int MODE, typename RowOf>
+// A block owns NTW column tiles.  Its eight wavefronts take every eighth pair of k tiles, two pairs at a time under way: the weight
+// tiles in registers, the activation rows' 128 bytes of a pair in LDS, eight neighbouring lanes to a row (global_load_lds).  The
+// sums meet in LDS in a fixed order.  row_of(i): the activation row behind row i of the block's rows (i < m; others repeat the last
+// one and are never stored) and the output row.
+// What bounds it is the weights' way from memory, as long as the rows do not stand in it: the matrix instruction wants a lane to
+// hold 16 bytes of its own row, and loaded that way into registers four neighbouring lanes touch four cache lines, which the
+// address unit serves one per cycle (64 cycles an instruction instead of 16).  In microseconds, loaded so and staged, with 4, 16
+// and 32 rows: 2048 -> 2048 4.6, 6.0, 8.0 and 4.1, 4.7, 5.7; 2048 -> 6176 6.7, 9.3, 9.5 and 6.1, 6.6, 8.1; 8192 -> 2048 10.0,
+// 15.1, 21.1 and 9.1, 11.5, 15.3; 4096 -> 32000 47, 45, 50 and 42, 42, 47 (6.3 TB/s).  Three and four pairs under way: slower
+// (longer code, fewer blocks to a compute unit) in nearly all shapes.  What the epilogue reads from memory is requested ahead of
+// the weights (0.7 us of the residual form at 4.5).
+constexpr int kRowWaves = 8, kRowPairs = 2;          // wavefronts of a block; pairs of k tiles under way in each
+constexpr uint32_t row_stage_bytes(int mt) { return mt * 2048; }     // rows of one pair
+constexpr uint32_t row_lds_bytes(int mt, int ntw) {
+    const uint32_t stage = kRowWaves * kRowPairs * row_stage_bytes(mt), sums = kRowWaves * mt * ntw * 1024;
+    return stage > sums ? stage : sums;
+}
+typedef __attribute__((address_space(1))) const void *gptr;
+typedef __attribute__((address_space(3))) void *lptr;
+
+// This wavefront's loads but the N youngest have landed, those into LDS too.
+template <int N>
+__device__ __forceinline__ void loads_wait() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// The operand fragments of MT row tiles of a staged pair: k tile h of row tile i at at[h] + BASE + 2048 i.  Assembly, because the
+// compiler would wait for every load into LDS that is under way ahead of any read.
+template <int BASE>
+__device__ __forceinline__ void stage_read(v4i (&a)[1][2], const uint32_t (&at)[2]) {
+    asm volatile("ds_read_b128 %0, %2 offset:%4\n\tds_read_b128 %1, %3 offset:%4\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[0][1])
+                 : "v"(at[0]), "v"(at[1]), "n"(BASE)
+                 : "memory");
+}
+template <int BASE>
+__device__ __forceinline__ void stage_read(v4i (&a)[2][2], const uint32_t (&at)[2]) {
+    asm volatile("ds_read_b128 %0, %4 offset:%6\n\tds_read_b128 %1, %5 offset:%6\n\t"
+                 "ds_read_b128 %2, %4 offset:%7\n\tds_read_b128 %3, %5 offset:%7\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1])
+                 : "v"(at[0]), "v"(at[1]), "n"(BASE), "n"(BASE + 2048)
+                 : "memory");
+}
+template <int BASE>
+__device__ __forceinline__ void stage_read(v4i (&a)[4][2], const uint32_t (&at)[2]) {
+    asm volatile("ds_read_b128 %0, %8 offset:%10\n\tds_read_b128 %1, %9 offset:%10\n\t"
+                 "ds_read_b128 %2, %8 offset:%11\n\tds_read_b128 %3, %9 offset:%11\n\t"
+                 "ds_read_b128 %4, %8 offset:%12\n\tds_read_b128 %5, %9 offset:%12\n\t"
+                 "ds_read_b128 %6, %8 offset:%13\n\tds_read_b128 %7, %9 offset:%13\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[0][1]), "=&v"(a[1][0]), "=&v"(a[1][1]), "=&v"(a[2][0]), "=&v"(a[2][1]), "=&v"(a[3][0]), "=&v"(a[3][1])
+                 : "v"(at[0]), "v"(at[1]), "n"(BASE), "n"(BASE + 2048), "n"(BASE + 4096), "n"(BASE + 6144)
+                 : "memory");
+}
+
+template <int MT, int NTW, int MODE, typename RowOf>
 __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint64_t lda, const uint8_t *__restrict__ w_batch, uint32_t m,
-                                            uint32_t n, uint32_t n_tiles, uint32_t k_tiles, uint32_t batch, const LinearEpilogue &ep, v4f *red_all,
+                                            uint32_t n, uint32_t n_tiles, uint32_t k_tiles, uint32_t batch, const LinearEpilogue &ep, uint8_t *lds,
                                             RowOf row_of) {
     static_assert(!is_glu(MODE) || NTW % 2 == 0, "gate and up are neighbouring tiles");
-    constexpr int NT = MT * NTW, D = NTW == 4 || MT == 4 ? 4 : 8;
-    v4f(*red)[NT][64] = (v4f(*)[NT][64])red_all;
-    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    const uint32_t nt0 = blockIdx.x * NTW;
-    const uint8_t *wb = w_batch + lane * 16;
-    const uint8_t *a_row[MT];
+    constexpr int NT = MT * NTW, STEP = is_glu(MODE) ? 2 : 1, LOADS = 2 * (MT + NTW);
+    static_assert(NT <= kRowWaves * STEP, "a wavefront finishes one tile, or one gate and its up");
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const uint32_t nt0 = blockIdx.x * NTW, pairs = k_tiles / 2;
+    const uint32_t cnt = pairs > (uint32_t)wave ? (pairs - wave + kRowWaves - 1) / kRowWaves : 0;
+    // load x of a row tile: rows 8 x .. + 7, lane l brings piece (l % 8) ^ (l / 8) of row l / 8, so that the 16 lanes an LDS
+    // read serves together (eight rows of two neighbouring k groups) find theirs in different banks
+    const uint8_t *a_src[MT][2];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        uint32_t r = i * 16 + lane % 16;
-        r = r < m ? r : 0;                       // a row past the end repeats row 0 and is never stored
-        a_row[i] = (const uint8_t *)(a + (uint64_t)row_of(r).x * lda) + (lane / 16) * 16;
-    }
-    const uint32_t cnt = k_tiles > (uint32_t)wave ? (k_tiles - wave + NWAVES - 1) / NWAVES : 0;
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const uint32_t r = i * 16 + x * 8 + lane / 8;
+            a_src[i][x] = (const uint8_t *)(a + (uint64_t)row_of(r < m ? r : m - 1).x * lda) + ((lane % 8) ^ (lane / 8)) * 16;
+        }
+    const uint8_t *w_src[NTW];
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) w_src[j] = w_batch + (uint64_t)(nt0 + j < n_tiles ? nt0 + j : n_tiles - 1) * k_tiles * 1024 + lane * 16;
+    uint8_t *stage = lds + wave * (kRowPairs * row_stage_bytes(MT));
+    const uint32_t r16 = lane % 16, at0 = (uint32_t)(uintptr_t)(lptr)stage + (r16 / 8) * 1024 + (r16 % 8) * 128;
+    const uint32_t at[2] = {at0 + (((uint32_t)lane / 16) ^ (r16 % 8)) * 16, at0 + ((4 + (uint32_t)lane / 16) ^ (r16 % 8)) * 16};
+    // the tile this wavefront finishes
+    const uint32_t t = wave * STEP, row = t / NTW * 16 + r16, tile = nt0 + t % NTW;
+    const bool own = t < (uint32_t)NT && row < m && tile < n_tiles;
+    const uint32_t out_row = own ? row_of(row).y : 0, col = (is_glu(MODE) ? tile / 2 : tile) * 16 + 4 * (lane / 16);
+    const EpilogueAhead ahead = own ? epilogue_ahead<MODE>(ep, out_row, col, n, batch) : EpilogueAhead{};
+    __builtin_amdgcn_sched_barrier(0);
+
     v4f acc[MT][NTW];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NTW; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    v4i av[D][MT], bv[D][NTW];
-    auto load = [&](int s, uint32_t it) {
-        const uint32_t kt = wave + (it < cnt ? it : cnt - 1) * NWAVES;
+    v4i bv[kRowPairs][2][NTW];
+    auto load = [&](int s, uint32_t it) {            // past the end: the wavefront's last pair again, so that the number under way is the same
+        const uint32_t p = wave + (it < cnt ? it : cnt - 1) * kRowWaves;
 #pragma unroll
-        for (int j = 0; j < NTW; ++j) {
-            const uint32_t nt = nt0 + j < n_tiles ? nt0 + j : n_tiles - 1;
-            bv[s][j] = stream_load<true>((const v4i *)(wb + ((uint64_t)nt * k_tiles + kt) * 1024));
-        }
+        for (int j = 0; j < NTW; ++j)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) av[s][i] = *(const v4i *)(a_row[i] + (uint64_t)kt * 64);
-    };
-    auto mul = [&](int s) {
+            for (int h = 0; h < 2; ++h) bv[s][h][j] = stream_load<true>((const v4i *)(w_src[j] + (uint64_t)p * 2048 + h * 1024));
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 0; j < NTW; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, bv[s][j]),
-                                                                    __builtin_bit_cast(v8bf, av[s][i]), acc[i][j], 0, 0, 0);
+            for (int x = 0; x < 2; ++x)
+                __builtin_amdgcn_global_load_lds((gptr)(a_src[i][x] + (uint64_t)p * 128), (lptr)(stage + s * row_stage_bytes(MT) + i * 2048 + x * 1024), 16, 0, 0);
     };
+    auto mul = [&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        v4i av[MT][2];
+        stage_read<s * (int)row_stage_bytes(MT)>(av, at);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NTW; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, bv[s][h][j]), __builtin_bit_cast(v8bf, av[i][h]),
+                                                                        acc[i][j], 0, 0, 0);
+    };
+    static_assert(kRowPairs == 2, "two slots are written out below");
     if (cnt != 0) {
-#pragma unroll
-        for (int s = 0; s < D; ++s) load(s, (uint32_t)s);
-        uint32_t it0 = 0;
-        for (; it0 + D < cnt; it0 += D) {
-#pragma unroll
-            for (int s = 0; s < D; ++s) {
-                mul(s);
-                __builtin_amdgcn_sched_barrier(0);
-                load(s, it0 + D + s);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        load(0, 0);
+        load(1, 1);
+        uint32_t it = 0;
+        for (; it + 2 < cnt; it += 2) {
+            // the reads of a slot are complete (stage_read waits) before it is loaded again
+            loads_wait<LOADS>();
+            mul(std::integral_constant<int, 0>{});
+            __builtin_amdgcn_sched_barrier(0);
+            load(0, it + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            loads_wait<LOADS>();
+            mul(std::integral_constant<int, 1>{});
+            __builtin_amdgcn_sched_barrier(0);
+            load(1, it + 3);
+            __builtin_amdgcn_sched_barrier(0);
         }
-#pragma unroll
-        for (int s = 0; s < D; ++s)
-            if (it0 + s < cnt) mul(s);
+        loads_wait<LOADS>();
+        mul(std::integral_constant<int, 0>{});
+        loads_wait<0>();
+        if (it + 1 < cnt) mul(std::integral_constant<int, 1>{});
     }
+    v4f(*red)[NT][64] = (v4f(*)[NT][64])lds;
+    __syncthreads();                                 // nobody reads rows any more
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NTW; ++j) red[wave][i * NTW + j][lane] = acc[i][j];
     __syncthreads();
-    auto total = [&](int t) {
-        v4f r = red[0][t][lane];
+    if (!own) return;
+    auto total = [&](int u) {
+        v4f r = red[0][u][lane];
 #pragma unroll
-        for (int q = 1; q < NWAVES; ++q) r += red[q][t][lane];
+        for (int q = 1; q < kRowWaves; ++q) r += red[q][u][lane];
         return r;
     };
-    constexpr int STEP = is_glu(MODE) ? 2 : 1;
-    for (int t = wave * STEP; t < NT; t += NWAVES * STEP) {
-        const int i = t / NTW, j = t % NTW;
-        const uint32_t row = i * 16 + lane % 16;
-        if (row >= m || nt0 + j >= n_tiles) continue;
-        const v4f x = total(t);
-        const v4f up = STEP == 2 ? total(t + 1) : x;
-        const uint32_t tile = is_glu(MODE) ? (nt0 + j) / 2 : nt0 + j;
-        epilogue_store4<MODE>(ep, row_of(row).y, tile * 16 + 4 * (lane / 16), n, batch, x, up);
-    }
+    const v4f x = total(t);
+    epilogue_store4<MODE, true>(ep, out_row, col, n, batch, x, STEP == 2 ? total(t + 1) : x, ahead);
 }
 
-template <int MT, int NTW, int NWAVES, int MODE>
-__global__ void __launch_bounds__(NWAVES * 64)
+template <int MT, int NTW, int MODE>
+__global__ void __launch_bounds__(kRowWaves * 64)
     linear_rows_kernel(const uint16_t *__restrict__ a, uint64_t lda, uint64_t a_batch, const uint8_t *__restrict__ w, uint32_t m,
                        uint32_t n, uint32_t n_tiles, uint32_t k_tiles, LinearEpilogue ep) {
-    __shared__ v4f red[NWAVES * MT * NTW * 64];
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t batch = blockIdx.y;
-    linear_rows<MT, NTW, NWAVES, MODE>(a + batch * a_batch, lda, w + (uint64_t)batch * n_tiles * k_tiles * 1024, m, n, n_tiles, k_tiles, batch, ep, red,
-                                       [](uint32_t r) { return make_uint2(r, r); });
+    linear_rows<MT, NTW, MODE>(a + batch * a_batch, lda, w + (uint64_t)batch * n_tiles * k_tiles * 1024, m, n, n_tiles, k_tiles, batch, ep, lds,
+                               [](uint32_t r) { return make_uint2(r, r); });
 }
 
 // The rows of a group, up to 16 MT at a time (its weights then come from the caches again); groups without rows cost a
 // launch slot only.
-template <int MT, int NTW, int NWAVES, int MODE>
-__global__ void __launch_bounds__(NWAVES * 64)
+template <int MT, int NTW, int MODE>
+__global__ void __launch_bounds__(kRowWaves * 64)
     linear_rows_grouped_kernel(const uint16_t *__restrict__ a, uint64_t lda, const uint8_t *__restrict__ w, uint32_t n, uint32_t n_tiles,
                                uint32_t k_tiles, RowGroups rg, LinearEpilogue ep) {
-    __shared__ v4f red[NWAVES * MT * NTW * 64];
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t group = blockIdx.y;
     uint32_t m = rg.count[group];
     m = m < rg.pitch ? m : rg.pitch;
@@ -133,9 +207,9 @@ __global__ void __launch_bounds__(NWAVES * 64)
             return make_uint2(e / rg.a_div, e);
         };
         if (r0) __syncthreads();
-        if (MT == 1 || left <= 16) linear_rows<1, NTW, NWAVES, MODE>(a, lda, wg, left < 16 ? left : 16, n, n_tiles, k_tiles, 0, ep, red, row_of);
-        else if (MT == 2 || left <= 32) linear_rows<(MT < 2 ? MT : 2), NTW, NWAVES, MODE>(a, lda, wg, left < 32 ? left : 32, n, n_tiles, k_tiles, 0, ep, red, row_of);
-        else linear_rows<MT, NTW, NWAVES, MODE>(a, lda, wg, left < 16 * MT ? left : 16 * MT, n, n_tiles, k_tiles, 0, ep, red, row_of);
+        if (MT == 1 || left <= 16) linear_rows<1, NTW, MODE>(a, lda, wg, left < 16 ? left : 16, n, n_tiles, k_tiles, 0, ep, lds, row_of);
+        else if (MT == 2 || left <= 32) linear_rows<(MT < 2 ? MT : 2), NTW, MODE>(a, lda, wg, left < 32 ? left : 32, n, n_tiles, k_tiles, 0, ep, lds, row_of);
+        else linear_rows<MT, NTW, MODE>(a, lda, wg, left < 16 * MT ? left : 16 * MT, n, n_tiles, k_tiles, 0, ep, lds, row_of);
     }
 }
 
@@ -322,36 +396,52 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// LDS beyond 64 KiB has to be asked for once
+template <typename K>
+void allow_lds(K kernel, uint32_t bytes) {
+    if (bytes > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+}
+template <int MT, int NTW, int MODE>
+void launch_rows(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, hipStream_t s) {
+    constexpr uint32_t lds = row_lds_bytes(MT, NTW);
+    static const bool allowed = (allow_lds(&linear_rows_kernel<MT, NTW, MODE>, lds), true);
+    (void)allowed;
+    linear_rows_kernel<MT, NTW, MODE><<<dim3((w.n_tiles + NTW - 1) / NTW, w.batches), kRowWaves * 64, lds, s>>>(
+        a, lda, a_batch, (const uint8_t *)w.w, (uint32_t)m, w.n, w.n_tiles, w.k_tiles, ep);
+}
+template <int MT, int NTW, int MODE>
+void launch_rows_grouped(const uint16_t *a, uint64_t lda, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, hipStream_t s) {
+    constexpr uint32_t lds = row_lds_bytes(MT, NTW);
+    static const bool allowed = (allow_lds(&linear_rows_grouped_kernel<MT, NTW, MODE>, lds), true);
+    (void)allowed;
+    linear_rows_grouped_kernel<MT, NTW, MODE><<<dim3((w.n_tiles + NTW - 1) / NTW, rg.groups), kRowWaves * 64, lds, s>>>(
+        a, lda, (const uint8_t *)w.w, w.n, w.n_tiles, w.k_tiles, rg, ep);
+}
+
 template <int MODE>
 void launch_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
                  int num_cus, hipStream_t s) {
     const uint8_t *wt = (const uint8_t *)w.w;
     if (m <= 64) {
-        constexpr bool GLU = is_glu(MODE);
-        const int mt = (int)((m + 15) / 16);
-        // two tiles per block once one tile each would fill the device twice over; beyond 16 rows, where the registers allow
-        // one block per compute unit, as soon as one tile each does not fit it at once
-        const uint64_t tiles = (uint64_t)w.n_tiles * w.batches;
-        const bool two = GLU || tiles >= 2 * (uint64_t)num_cus || (mt > 1 && tiles > (uint64_t)num_cus);
-        // wide weights, up to 32 rows: four, so that the activations cross the L2 half as often
-        const bool four = mt <= 2 && g_linear_form != 3 && w.batches == 1 && w.n_tiles >= 3 * (uint64_t)num_cus;
-        const dim3 grid(four ? (w.n_tiles + 3) / 4 : two ? (w.n_tiles + 1) / 2 : w.n_tiles, w.batches);
-#define FA_ROWS(MT_, NTW_)                                                                                             \
-    linear_rows_kernel<MT_, NTW_, 8, MODE><<<grid, 512, 0, s>>>(a, lda, a_batch, wt, (uint32_t)m, w.n, w.n_tiles, w.k_tiles, ep)
-        if (four) {
-            if (mt == 1) FA_ROWS(1, 4);
-            else FA_ROWS(2, 4);
-        } else if constexpr (GLU) {
-            if (mt == 1) FA_ROWS(1, 2);
-            else if (mt == 2) FA_ROWS(2, 2);
-            else FA_ROWS(4, 2);
-        } else {
-            if (mt == 1) two ? FA_ROWS(1, 2) : FA_ROWS(1, 1);
-            else if (mt == 2) two ? FA_ROWS(2, 2) : FA_ROWS(2, 1);
-            else two ? FA_ROWS(4, 2) : FA_ROWS(4, 1);
+        // Two tiles per block as soon as one tile each does not fit the device at once, so that the rows cross the L2 half as
+        // often (4096 -> 6144 with 4, 16, 32 rows 11.0, 12.6, 16.4 and 10.0, 11.0, 13.1 us; 2048 -> 4096, which fits, 4.7, 5.1, 6.2 and
+        // 5.5, 6.1, 7.5).  Four: behind two in nearly every shape (4096 -> 28672 with 32 rows 45.1 and 45.9).  Up to
+        // four rows are hardly in the way, and four rounds of single tiles end more evenly (4096 -> 28672 38.9 and 36.4).
+        const uint64_t tiles = (uint64_t)w.n_tiles * w.batches, cus = (uint64_t)num_cus;
+        const bool two = is_glu(MODE) || (tiles > cus && (m > 4 || tiles < 4 * cus));
+        if (m <= 16) {
+            if constexpr (!is_glu(MODE))
+                if (!two) return launch_rows<1, 1, MODE>(a, lda, a_batch, m, w, ep, s);
+            return launch_rows<1, 2, MODE>(a, lda, a_batch, m, w, ep, s);
         }
-#undef FA_ROWS
-        return;
+        if (m <= 32) {
+            if constexpr (!is_glu(MODE))
+                if (!two) return launch_rows<2, 1, MODE>(a, lda, a_batch, m, w, ep, s);
+            return launch_rows<2, 2, MODE>(a, lda, a_batch, m, w, ep, s);
+        }
+        if constexpr (!is_glu(MODE))
+            if (!two) return launch_rows<4, 1, MODE>(a, lda, a_batch, m, w, ep, s);
+        return launch_rows<4, 2, MODE>(a, lda, a_batch, m, w, ep, s);
     }
     if (MODE != LinearEpilogue::kHeadGate && g_linear_form != 2 && gemm_bf16_big_applies(lda, m, w)) return gemm_bf16_big(a, m, w, ep, num_cus, s);
     const dim3 grid((w.n_tiles + 7) / 8, (unsigned)((m + 127) / 128), w.batches);
@@ -369,18 +459,17 @@ void launch_grouped_bf16(const uint16_t *a, uint64_t lda, const LinearWeight &w,
     const int form = g_linear_form;
     if (form == 4 || (form != 5 && form != 6 && mean <= 10)) {
         const bool two = GLU || (uint64_t)w.n_tiles * std::min(rg.groups, rg.entries) >= 2 * (uint64_t)num_cus;
-        const dim3 grid(two ? (w.n_tiles + 1) / 2 : w.n_tiles, rg.groups);
-#define FA_ROWS(MT_, NTW_) linear_rows_grouped_kernel<MT_, NTW_, 8, MODE><<<grid, 512, 0, s>>>(a, lda, wt, w.n, w.n_tiles, w.k_tiles, rg, ep)
-        if constexpr (GLU) {
-            if (rg.most <= 16) FA_ROWS(1, 2);
-            else if (mean <= 8) FA_ROWS(2, 2);
-            else FA_ROWS(4, 2);
-        } else {
-            if (rg.most <= 16) two ? FA_ROWS(1, 2) : FA_ROWS(1, 1);
-            else if (mean <= 8) two ? FA_ROWS(2, 2) : FA_ROWS(2, 1);
-            else two ? FA_ROWS(4, 2) : FA_ROWS(4, 1);
-        }
-#undef FA_ROWS
+        const int mt = rg.most <= 16 ? 1 : mean <= 8 ? 2 : 4;
+        if constexpr (!GLU)
+            if (!two) {
+                if (mt == 1) launch_rows_grouped<1, 1, MODE>(a, lda, w, rg, ep, s);
+                else if (mt == 2) launch_rows_grouped<2, 1, MODE>(a, lda, w, rg, ep, s);
+                else launch_rows_grouped<4, 1, MODE>(a, lda, w, rg, ep, s);
+                return;
+            }
+        if (mt == 1) launch_rows_grouped<1, 2, MODE>(a, lda, w, rg, ep, s);
+        else if (mt == 2) launch_rows_grouped<2, 2, MODE>(a, lda, w, rg, ep, s);
+        else launch_rows_grouped<4, 2, MODE>(a, lda, w, rg, ep, s);
         return;
     }
     if (form == 6 || (form != 5 && mean >= 112 && lda == (uint64_t)w.k_tiles * 32 && w.n_tiles >= 14)) return gemm_bf16_big_grouped(a, w, rg, ep, num_cus, s);

@@ -11,7 +11,7 @@ using dev::sigmoid_f32;
 
 // The value the epilogue makes of y (and, for gate | up, of the up column's y).
 template <int MODE>
-__device__ __forceinline__ float epilogue_value(const LinearEpilogue &ep, uint32_t row, uint32_t batch, float y, float up) {
+__device__ __forceinline__ float epilogue_value(const LinearEpilogue &ep, float gate, float y, float up) {
     if constexpr (MODE == LinearEpilogue::kGlu) {
         const float g = fminf(y, ep.limit), u = fminf(fmaxf(up, -ep.limit), ep.limit);
         return g * sigmoid_f32(ep.alpha * g) * (u + 1.0f);
@@ -21,7 +21,7 @@ __device__ __forceinline__ float epilogue_value(const LinearEpilogue &ep, uint32
         y *= ep.factor;
         return ep.cap > 0.0f ? ep.cap * tanhf(y / ep.cap) : y;
     } else if constexpr (MODE == LinearEpilogue::kHeadGate) {
-        return y * ep.factor * sigmoid_f32(ep.gate[(uint64_t)row * ep.ld_gate + batch]);
+        return y * ep.factor * sigmoid_f32(gate);
     } else if constexpr (MODE == LinearEpilogue::kSquaredRelu) {
         const float r = fmaxf(y, 0.0f);
         return r * r;
@@ -38,8 +38,13 @@ __device__ __forceinline__ float epilogue_value(const LinearEpilogue &ep, uint32
 constexpr bool is_glu(int mode) { return mode == LinearEpilogue::kGlu || mode == LinearEpilogue::kSiluGlu; }
 
 template <int MODE>
+__device__ __forceinline__ float epilogue_gate(const LinearEpilogue &ep, uint32_t row, uint32_t batch) {
+    return MODE == LinearEpilogue::kHeadGate ? ep.gate[(uint64_t)row * ep.ld_gate + batch] : 0.0f;
+}
+
+template <int MODE>
 __device__ __forceinline__ void epilogue_store1(const LinearEpilogue &ep, uint32_t row, uint32_t col, uint32_t batch, float y, float up) {
-    float v = epilogue_value<MODE>(ep, row, batch, y, up);
+    float v = epilogue_value<MODE>(ep, epilogue_gate<MODE>(ep, row, batch), y, up);
     if (MODE == LinearEpilogue::kStore && ep.bias) v += ep.bias[col];
     if constexpr (MODE == LinearEpilogue::kResidual) {
         float *o = (float *)ep.out + (uint64_t)row * ep.ld_out + col;
@@ -55,12 +60,37 @@ __device__ __forceinline__ void epilogue_store1(const LinearEpilogue &ep, uint32
     else ((uint16_t *)ep.out)[o] = dev::f32_to_bf16(v);
 }
 
-// Columns col .. col + 3 of a row (those below n).
+// Whether columns col .. col + 3 go out as one store
 template <int MODE>
+__device__ __forceinline__ bool epilogue_whole(const LinearEpilogue &ep, uint32_t col, uint32_t n) {
+    return col + 4 <= n && ((ep.ld_out | ep.out_batch) & 3) == 0 && (MODE != LinearEpilogue::kStore || col + 4 <= ep.n_lo);
+}
+
+// What epilogue_store4 reads from memory for columns that go out as one store: the residual, its scale or the bias, the head's gate
+struct EpilogueAhead {
+    dev::v4f residual, factor;
+    float gate;
+};
+template <int MODE>
+__device__ __forceinline__ EpilogueAhead epilogue_ahead(const LinearEpilogue &ep, uint32_t row, uint32_t col, uint32_t n, uint32_t batch) {
+    EpilogueAhead p{};
+    if (!epilogue_whole<MODE>(ep, col, n)) return p;
+    if constexpr (MODE == LinearEpilogue::kStore) {
+        if (ep.bias) p.factor = *(const dev::v4f *)(ep.bias + col);
+    } else if constexpr (MODE == LinearEpilogue::kResidual) {
+        p.residual = *(const dev::v4f *)((const float *)ep.out + batch * ep.out_batch + (uint64_t)row * ep.ld_out + col);
+        p.factor = ep.scale ? *(const dev::v4f *)(ep.scale + col) : dev::v4f{1.0f, 1.0f, 1.0f, 1.0f};
+    }
+    p.gate = epilogue_gate<MODE>(ep, row, batch);
+    return p;
+}
+
+// Columns col .. col + 3 of a row (those below n).  AHEAD: what they need is there.
+template <int MODE, bool AHEAD = false>
 __device__ __forceinline__ void epilogue_store4(const LinearEpilogue &ep, uint32_t row, uint32_t col, uint32_t n, uint32_t batch,
-                                                dev::v4f y, dev::v4f up) {
+                                                dev::v4f y, dev::v4f up, const EpilogueAhead &ahead = EpilogueAhead{}) {
     const uint64_t o = batch * ep.out_batch + (uint64_t)row * ep.ld_out + col;
-    const bool whole = col + 4 <= n && ((ep.ld_out | ep.out_batch) & 3) == 0 && (MODE != LinearEpilogue::kStore || col + 4 <= ep.n_lo);
+    const bool whole = epilogue_whole<MODE>(ep, col, n);
     if (MODE == LinearEpilogue::kStore && col >= ep.n_lo && col + 4 <= n && ((ep.n_lo | ep.ld_hi) & 3) == 0 && !ep.bias) {
         *(dev::v4f *)(ep.out_hi + (uint64_t)row * ep.ld_hi + (col - ep.n_lo)) = y * ep.factor;
         return;
@@ -73,17 +103,17 @@ __device__ __forceinline__ void epilogue_store4(const LinearEpilogue &ep, uint32
     }
     float v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = epilogue_value<MODE>(ep, row, batch, y[e], up[e]);
+    for (int e = 0; e < 4; ++e) v[e] = epilogue_value<MODE>(ep, AHEAD ? ahead.gate : epilogue_gate<MODE>(ep, row, batch), y[e], up[e]);
     if constexpr (MODE == LinearEpilogue::kStore) {
         if (ep.bias) {
-            const dev::v4f b = *(const dev::v4f *)(ep.bias + col);
+            const dev::v4f b = AHEAD ? ahead.factor : *(const dev::v4f *)(ep.bias + col);
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] += b[e];
         }
     }
     if constexpr (MODE == LinearEpilogue::kResidual) {
         dev::v4f *p = (dev::v4f *)((float *)ep.out + o);
-        const dev::v4f r = *p, ls = ep.scale ? *(const dev::v4f *)(ep.scale + col) : dev::v4f{1.0f, 1.0f, 1.0f, 1.0f};
+        const dev::v4f r = AHEAD ? ahead.residual : *p, ls = AHEAD ? ahead.factor : ep.scale ? *(const dev::v4f *)(ep.scale + col) : dev::v4f{1.0f, 1.0f, 1.0f, 1.0f};
         *p = dev::v4f{r[0] + ls[0] * v[0], r[1] + ls[1] * v[1], r[2] + ls[2] * v[2], r[3] + ls[3] * v[3]};
     } else if (ep.out_f32) {
         *(dev::v4f *)((float *)ep.out + o) = dev::v4f{v[0], v[1], v[2], v[3]};
