@@ -4,6 +4,7 @@
 // per row of S.  Lightning attention is S <- g S + k v^T with constant g and q, k, v behind SiLU only.  The read-out is divided
 // by its root mean square (of a head or of all heads), weighted and gated.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "attention_tiles.hpp"
@@ -20,8 +21,7 @@ int g_delta_form = 0;        // tuning: 1 keeps the token-by-token kernel for pr
 namespace {
 
 __device__ __forceinline__ float log_decay(float a_log, float x) {
-    const float sp = x > 0.0f ? x + log1pf(expf(-x)) : log1pf(expf(x));
-    return -expf(a_log) * sp;
+    return -expf(a_log) * (fmaxf(x, 0.0f) + log1pf(expf(-fabsf(x))));
 }
 
 // x sigmoid(x) and exp(x) on the hardware's exponential and reciprocal (about one unit in the last place each)
@@ -58,19 +58,13 @@ __device__ __forceinline__ float conv_silu(const T *__restrict__ y, uint32_t ld,
 // ------------------------------------------------------------------ token by token
 // One block per (sequence, head), or per part of a wide state's columns (StepPlan); the state sits in registers (thread: four
 // neighbouring columns of up to RPT rows) from the first token of the pass to the last.  CG = column groups of four, a power of two.
-// FAST (single tokens, at most four taps, no more than NQ NT channels): the inputs of the convolution are requested ahead of
-// the state, so that the convolution runs while the state travels.
-// A single token of a few sequences is a chain of latencies: dependent loads, barriers, and the instructions themselves,
-// which come from memory at every launch (about half a microsecond per KiB of code that runs through once).  So a block is
-// a thousand threads with up to eight rows each where few blocks leave the CUs to them (StepPlan), every
-// wavefront forms the norms and k . q for itself, and the wavefronts meet three times: 4 sequences of 16 heads 128 x 128 13.4 us
-// on 256 threads with eight meetings, 11.5 so (32 sequences: 256 threads still, 35.5 us, 27 at the rate of a copy).
-constexpr int step_channels(int nt) { return nt == 1024 ? 1 : 2; }
-
-template <typename T, int NT, int RPT, bool FAST, Recurrence KIND>
+// A few tokens of a few sequences are a chain of latencies: dependent loads, barriers, and the instructions themselves.  So a block
+// is a thousand threads with up to eight rows each where few blocks leave the CUs to them (StepPlan), every
+// wavefront forms the norms and k . q for itself, and the wavefronts meet three times.  Single tokens: one_delta_step_kernel, unless
+// the convolution is longer or the head has more inputs than that takes.
+template <typename T, int NT, int RPT, Recurrence KIND>
 __global__ void __launch_bounds__(NT)
     delta_step_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, uint32_t cg_log2, int write_ring, uint32_t max_tokens) {
-    constexpr int NQ = step_channels(NT);
     // q [dim], k [dim], v [CG * 4], decays [dim] or shares of S^T k and S^T q [2][parts][CG * 4], their sums [2][CG * 4]
     extern __shared__ float lds[];
     constexpr bool CHANNEL = KIND == Recurrence::kChannelDelta, LIGHTNING = KIND == Recurrence::kLightning;
@@ -92,23 +86,6 @@ __global__ void __launch_bounds__(NT)
     const bool col_ok = col < vp;
     const uint32_t p0 = (uint32_t)rr.pos[row0];
     auto channel = [&](uint32_t i) { return i < dim ? hk * dim + i : i < 2 * dim ? (sh.kv_heads + hk) * dim + (i - dim) : 2 * sh.kv_heads * dim + h * vdim + col0 + (i - 2 * dim); };
-    float xin[NQ][4], win[NQ][4];
-    if constexpr (FAST) {
-#pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            const uint32_t i = threadIdx.x + q * NT;
-#pragma unroll
-            for (uint32_t back = 0; back < 4; ++back) {
-                xin[q][back] = win[q][back] = 0.0f;
-                if (i < 2 * dim + cols && (back < sh.taps || back == 0) && back <= p0) {
-                    const uint32_t c = channel(i);
-                    xin[q][back] = load_as_f32(back == 0 ? y + (uint64_t)row0 * io.ld_y + c : ring + (uint64_t)((p0 - back) % sh.taps) * channels + c);
-                    win[q][back] = sh.taps ? io.conv[(uint64_t)c * sh.taps + sh.taps - 1 - back] : 1.0f;
-                }
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
     // per-channel decays: thread d owns channel d (dim <= NT)
     static_assert(!CHANNEL || NT >= (int)kDeltaMaxDim, "a thread per channel");
     float decay_in = 0.0f, decay_bias = 0.0f;
@@ -129,21 +106,11 @@ __global__ void __launch_bounds__(NT)
         const uint64_t row = row0 + t;
         const uint32_t p = p0 + t;
         // q, k, v of this head behind the convolution
-#pragma unroll FAST ? NQ : 1
-        for (uint32_t q = 0; q < (FAST ? (uint32_t)NQ : 0x40000000u); ++q) {
-            const uint32_t i = threadIdx.x + q * NT;
-            if (i >= 2 * dim + CG * 4) break;
+        for (uint32_t i = threadIdx.x; i < 2 * dim + CG * 4; i += NT) {
             float v = 0.0f;
             if (i < 2 * dim + cols) {
                 const uint32_t c = channel(i);
-                if constexpr (FAST) {
-                    float acc = 0.0f;
-#pragma unroll
-                    for (int back = 3; back >= 0; --back) acc = fmaf(win[q][back], xin[q][back], acc);
-                    v = fast_silu(acc);
-                } else {
-                    v = conv_silu(y, io.ld_y, ring, io.conv, sh.taps, channels, c, row0, t, p);
-                }
+                v = conv_silu(y, io.ld_y, ring, io.conv, sh.taps, channels, c, row0, t, p);
                 if (write_ring && (i >= 2 * dim || (h % share == 0 && col0 == 0))) ring[(uint64_t)(p % sh.taps) * channels + c] = y[row * io.ld_y + c];
             }
             (i < dim ? lq[i] : i < 2 * dim ? lk[i - dim] : lv[i - 2 * dim]) = v;
@@ -243,6 +210,235 @@ __global__ void __launch_bounds__(NT)
         }
         if (t + 1 < n_tok) __syncthreads();          // q, k, v and the sums are overwritten by the next token
     }
+}
+
+// ------------------------------------------------------------------ single tokens
+// The same for passes of one token a sequence: at most four taps and 256 NQ inputs (q, k and the block's columns of v) to a head, on
+// 256 threads; thread (rg, cg) holds rows rg RPT .. + RPT - 1 of columns 4 cg .. + 3.  A block moves 64 KiB in and out, which is
+// a microsecond; the rest is the chain of dependent loads and the instructions of one wavefront (3 ns each where they depend on
+// each other), so everything that a load's address or size needs is one level of scalar loads away, the inputs, taps, gates and
+// norm weights are requested ahead of the state and without branches (a value converted inside one is waited for there), the sums run on q and k as they leave the convolution (their norms are factors
+// that are formed meanwhile), the ring's places take one remainder instead of one per tap, and the wavefronts meet twice.
+// 4 sequences of 16 heads 128 x 128: 7.4 us, 10.5 on a thousand threads of the kernel above; 32 sequences 14.5 and 35.5; 16 sequences
+// of 32 heads 16.8.
+// share_m, taps_m: 2^31 / n rounded up, whose product with the head and with the position, a number below 2^29, holds the quotient
+// by n (at most 4 taps) from bit 31 on.
+struct StepScalars {
+    uint32_t cg_log2, share, share_m, taps_m;
+    float rsqrt_dim;
+    int write_ring;
+};
+__device__ __forceinline__ uint32_t quotient(uint32_t x, uint32_t inverse) { return (uint32_t)((uint64_t)x * inverse >> 31); }
+// Element at a byte offset that 32 bits hold
+template <typename V>
+__device__ __forceinline__ V at_byte(const void *base, uint32_t offset) { return *(const V *)((const char *)base + offset); }
+// x^-1/2 with the hardware's estimate corrected by its remainder
+__device__ __forceinline__ float rsqrt_exact(float x) {
+    const float r = __builtin_amdgcn_rsqf(x);
+    return fmaf(fmaf(-x * r, r, 1.0f), 0.5f * r, r);
+}
+__device__ __forceinline__ v4f fma4(const v4f &a, float b, const v4f &c) {
+    return v4f{fmaf(a[0], b, c[0]), fmaf(a[1], b, c[1]), fmaf(a[2], b, c[2]), fmaf(a[3], b, c[3])};
+}
+
+template <typename T, int RPT, int NQ, Recurrence KIND>
+__global__ void __launch_bounds__(256) one_delta_step_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, StepScalars sc) {
+    constexpr bool CHANNEL = KIND == Recurrence::kChannelDelta, LIGHTNING = KIND == Recurrence::kLightning;
+    constexpr uint32_t NT = 256, STR = CHANNEL ? 4 : 2;
+    // [rows] k, q (decay, -), zeros behind dim; v [4 CG]; shares of S^T k and S^T q [4 wavefronts][2][4 CG]
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const uint32_t b = blockIdx.x, h = blockIdx.y;
+    // (a sequence without a token reads the pass's last row; it leaves ahead of the first store)
+    const uint32_t start = rr.row_start[b], end = rr.row_start[b + 1], slot = rr.state_slot[b], row = start < rr.rows ? start : rr.rows - 1;
+    const uint32_t dim = sh.dim, vdim = sh.vdim, vp = sh.vdim_p(), channels = sh.qkv(), taps = sh.taps;
+    const uint32_t CG = 1u << sc.cg_log2, RG = NT >> sc.cg_log2, cg = threadIdx.x & (CG - 1), rg = threadIdx.x >> sc.cg_log2, lane = threadIdx.x % 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), hk = quotient(h, sc.share_m), share = sc.share;
+    const uint32_t col0 = blockIdx.z * CG * 4, cols = vdim - col0 < CG * 4 ? vdim - col0 : CG * 4, col = col0 + cg * 4;
+    float *lv = lds + RPT * RG * STR, *part = lv + CG * 4;
+    const T *y = (const T *)io.y + (uint64_t)row * io.ld_y;
+    T *ring = (T *)io.ring + (uint64_t)slot * taps * channels;
+    // Inputs of the convolution: the new one and all places of the ring, so that their addresses do not wait for the position.  A
+    // thread without an input brings the last one; places that do not exist come from the first one, without a ring from y, and
+    // its taps from the norm weights, and none of it counts.
+    T x0[NQ], x[NQ][4];
+    float win[NQ][4];
+    uint32_t chan[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const uint32_t at = threadIdx.x + q * NT, i = at < 2 * dim + cols ? at : 2 * dim + cols - 1;
+        chan[q] = i + (i < dim ? hk * dim : i < 2 * dim ? (sh.kv_heads + hk - 1) * dim : 2 * (sh.kv_heads - 1) * dim + h * vdim + col0);
+        x0[q] = at_byte<T>(y, chan[q] * (uint32_t)sizeof(T));
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) x[q][j] = at_byte<T>(taps ? ring : y, ((j < taps ? j : 0) * channels + chan[q]) * (uint32_t)sizeof(T));
+#pragma unroll
+        for (uint32_t back = 0; back < 4; ++back)
+            win[q][back] = at_byte<float>(taps ? io.conv : io.norm, taps ? (chan[q] * taps + (back < taps ? taps - 1 - back : 0)) * 4 : 0);
+    }
+    // what the read-out needs (the first wavefront stores it)
+    T gate[4];
+    float weight[4];
+    const T *gates = sh.norm_all ? y : (const T *)io.gate + (uint64_t)row * io.ld_gate + h * vdim;
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+        const uint32_t c = sh.norm_all ? 0 : cg * 4 + e < vdim ? cg * 4 + e : vdim - 1;
+        gate[e] = at_byte<T>(gates, c * (uint32_t)sizeof(T));
+        weight[e] = at_byte<float>(io.norm, c * 4);
+    }
+    float decay_in = 0.0f, decay_bias = 0.0f;        // per channel: thread d owns channel d
+    if (CHANNEL && threadIdx.x < dim) {
+        decay_in = io.decay[(uint64_t)row * io.ld_decay + h * dim + threadIdx.x];
+        decay_bias = io.dt_bias[h * dim + threadIdx.x];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // the state; rows and columns behind it are loaded from its last ones, meet zeros and are not stored
+    const bool full = RPT * RG == dim && col0 + CG * 4 <= vp;
+    float *state = io.state + ((uint64_t)slot * sh.heads + h) * dim * vp;
+    const uint32_t mine = (rg * RPT * vp + col) * 4;
+    v4f S[RPT];
+    {
+        const uint32_t from = (col < vp ? col : vp - 4) * 4;
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            const uint32_t d = rg * RPT + i < dim ? rg * RPT + i : dim - 1;
+            S[i] = stream_load<true>((const v4f *)((const char *)state + (d * vp * 4 + from)));
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (start == end) return;
+    const uint32_t p = (uint32_t)rr.pos[row], place = p - quotient(p, sc.taps_m) * (taps ? taps : 1);          // p % taps
+    float beta = 1.0f, g = 1.0f;
+    const float a_log = LIGHTNING ? 0.0f : io.a_log[h];
+    if constexpr (LIGHTNING) {
+        g = io.decay[h];
+    } else {
+        beta = sigmoid_f32(io.beta[(uint64_t)row * io.ld_beta + h]);
+        if constexpr (!CHANNEL) g = expf(log_decay(a_log, io.decay[(uint64_t)row * io.ld_decay + h] + io.dt_bias[h]));
+    }
+    for (uint32_t d = dim + threadIdx.x; d < RPT * RG; d += NT)
+#pragma unroll
+        for (uint32_t e = 0; e < STR; ++e) lds[d * STR + e] = 0.0f;
+    if (CHANNEL && threadIdx.x < dim) lds[threadIdx.x * STR + 2] = expf(log_decay(a_log, decay_in + decay_bias));
+    uint32_t from[4];                                // the ring's place of the input that many tokens back; 4: none
+#pragma unroll
+    for (uint32_t back = 1; back < 4; ++back) {
+        const uint32_t there = place - back + (place < back ? taps : 0);
+        from[back] = (uint32_t)(back < taps) & (uint32_t)(back <= p) ? there : 4;
+    }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const uint32_t i = threadIdx.x + q * NT;
+        float acc = 0.0f;
+#pragma unroll
+        for (int back = 3; back > 0; --back) {
+            float u = 0.0f;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) u = from[back] == j ? load_as_f32(&x[q][j]) : u;
+            acc = fmaf(win[q][back], u, acc);
+        }
+        const float newest = load_as_f32(&x0[q]), v = fast_silu(taps ? fmaf(win[q][0], newest, acc) : newest);
+        if (i < 2 * dim + cols && sc.write_ring && (i >= 2 * dim || (h == hk * share && col0 == 0))) ring[place * channels + chan[q]] = x0[q];
+        if (i < 2 * dim + CG * 4) lds[i < dim ? i * STR + 1 : i < 2 * dim ? (i - dim) * STR : RPT * RG * STR + (i - 2 * dim)] = i < 2 * dim + cols ? v : 0.0f;
+    }
+    __syncthreads();
+    if (p == 0) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) S[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    }
+    float sq = 0.0f, sk = 0.0f, kq = 0.0f;           // the same in every wavefront
+    for (uint32_t d = lane; d < dim; d += 64) {
+        const v2f x = *(const v2f *)(lds + d * STR);
+        sq = fmaf(x[1], x[1], sq);
+        sk = fmaf(x[0], x[0], sk);
+        kq = fmaf(x[0], x[1], kq);
+    }
+    float rq = 1.0f, rk = 1.0f;
+    kq = wave_sum_dpp(kq);
+    if constexpr (!LIGHTNING) {
+        rq = rsqrt_exact(wave_sum_dpp(sq) + 1e-6f) * sc.rsqrt_dim;
+        rk = rsqrt_exact(wave_sum_dpp(sk) + 1e-6f);
+    }
+    v4f dk = v4f{0.f, 0.f, 0.f, 0.f}, dq = dk;
+    const float *rows = lds + rg * RPT * STR;
+    float kd[RPT];
+#pragma unroll
+    for (int i = 0; i < RPT; i += 2) {
+        float qd[2];
+        if constexpr (CHANNEL) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const v4f x = *(const v4f *)(rows + (i + e) * STR);
+                kd[i + e] = x[0];
+                qd[e] = x[1];
+                S[i + e] *= x[2];
+            }
+        } else {
+            const v4f x = *(const v4f *)(rows + i * STR);
+            kd[i] = x[0];
+            qd[0] = x[1];
+            kd[i + 1] = x[2];
+            qd[1] = x[3];
+        }
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            if constexpr (!LIGHTNING) dk = fma4(S[i + e], kd[i + e], dk);
+            dq = fma4(S[i + e], qd[e], dq);
+        }
+    }
+    for (uint32_t off = CG; off < 64; off <<= 1)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if constexpr (!LIGHTNING) dk[e] += __shfl_xor(dk[e], (int)off, 64);
+            dq[e] += __shfl_xor(dq[e], (int)off, 64);
+        }
+    if (lane < CG) {
+        if constexpr (!LIGHTNING) ((v4f *)part)[(wave * 2) * CG + cg] = dk;
+        ((v4f *)part)[(wave * 2 + 1) * CG + cg] = dq;
+    }
+    __syncthreads();
+    dk = dq = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (uint32_t w = 0; w < NT / 64; ++w) {
+        if constexpr (!LIGHTNING) dk += ((const v4f *)part)[(w * 2) * CG + cg];
+        dq += ((const v4f *)part)[(w * 2 + 1) * CG + cg];
+    }
+    const float gs = CHANNEL ? 1.0f : g;             // the decay that the sums do not hold yet
+    v4f u = *(const v4f *)(lv + cg * 4);
+    if constexpr (!LIGHTNING) u = fma4(dk, -gs * rk, u) * beta;
+    const v4f o = fma4(u, kq * (rq * rk), dq * (gs * rq)), uk = u * rk;
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+        if constexpr (!CHANNEL) S[i] *= g;
+        S[i] = fma4(uk, kd[i], S[i]);
+    }
+    if (full) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) __builtin_nontemporal_store(S[i], (v4f *)((char *)state + (mine + i * vp * 4)));
+    } else if (col < vp) {
+#pragma unroll
+        for (int i = 0; i < RPT; ++i)
+            if (rg * RPT + i < dim) __builtin_nontemporal_store(S[i], (v4f *)((char *)state + (mine + i * vp * 4)));
+    }
+    if (wave != 0) return;
+    if (sh.norm_all) {                               // the norm runs over more than this block's columns: another launch's
+        if (lane < CG) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (col + e < vdim) io.raw[((uint64_t)row * sh.heads + h) * vdim + col + e] = o[e];
+        }
+        return;
+    }
+    float so = 0.0f;                                 // (all column groups are lanes of this wavefront)
+    if (lane < CG) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (cg * 4 + e < vdim) so = fmaf(o[e], o[e], so);
+    }
+    const float ro = rsqrt_exact(wave_sum_dpp(so) / (float)vdim + sh.eps) * io.out_scale;
+    if (lane >= CG) return;
+    T *out = (T *)io.out + (uint64_t)row * io.ld_out + h * vdim + cg * 4;
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e)
+        if (cg * 4 + e < vdim) store_from_f32(out + e, o[e] * ro * weight[e] * output_gate(sh.gate_sigmoid, load_as_f32(&gate[e])));
 }
 
 // ------------------------------------------------------------------ chunk form
@@ -1250,15 +1446,12 @@ StepPlan step_plan(const DeltaShape &sh, uint32_t batch) {
 
 template <typename T, int NT, Recurrence KIND>
 void launch_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, const StepPlan &p, int write_ring, uint32_t max_tokens, hipStream_t s) {
-    const uint32_t CG = 1u << p.cg_log2, rg = NT >> p.cg_log2, rpt = (sh.dim + rg - 1) / rg, in = 2 * sh.dim + 4 * CG;
+    const uint32_t CG = 1u << p.cg_log2, rg = NT >> p.cg_log2, rpt = (sh.dim + rg - 1) / rg;
     const size_t lds = (3 * ((sh.dim + 3) / 4 * 4) + 4 * CG + 2 * (NT / 64 + 1) * 4 * CG) * 4;
     const dim3 grid(rr.batch, sh.heads, p.parts);
     DeltaShape part = sh;
     if (p.parts > 1) part.norm_all = 1;
-    const bool fast = max_tokens == 1 && sh.taps <= 4 && in <= step_channels(NT) * NT;
-#define FA_STEP(R_)                                                                                                           \
-    fast ? delta_step_kernel<T, NT, R_, true, KIND><<<grid, NT, lds, s>>>(part, io, rr, p.cg_log2, write_ring, max_tokens)       \
-         : delta_step_kernel<T, NT, R_, false, KIND><<<grid, NT, lds, s>>>(part, io, rr, p.cg_log2, write_ring, max_tokens)
+#define FA_STEP(R_) delta_step_kernel<T, NT, R_, KIND><<<grid, NT, lds, s>>>(part, io, rr, p.cg_log2, write_ring, max_tokens)
     if constexpr (NT == 1024) {                      // dim x columns <= 32 K: at most eight rows
         if (rpt <= 4) FA_STEP(4);
         else FA_STEP(8);
@@ -1270,6 +1463,32 @@ void launch_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, 
 #undef FA_STEP
 }
 
+// Single tokens on one_delta_step_kernel; false: not these.
+template <typename T, Recurrence KIND>
+bool launch_one_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, const StepPlan &p, int write_ring, hipStream_t s) {
+    const uint32_t CG = 1u << p.cg_log2, RG = 256 >> p.cg_log2, rpt = (sh.dim + RG - 1) / RG, in = 2 * sh.dim + 4 * CG;
+    if (sh.taps > 4 || in > 1024 || rpt > 32) return false;
+    auto inverse = [](uint32_t n) { return (uint32_t)(((1ull << 31) + n - 1) / n); };
+    const uint32_t share = sh.heads / sh.kv_heads;
+    const StepScalars sc{p.cg_log2, share, inverse(share), inverse(sh.taps ? sh.taps : 1), (float)(1.0 / std::sqrt((double)sh.dim)), write_ring};
+    DeltaShape part = sh;
+    if (p.parts > 1) part.norm_all = 1;
+    const dim3 grid(rr.batch, sh.heads, p.parts);
+    auto go = [&](auto rows, auto inputs) {
+        constexpr uint32_t R = decltype(rows)::value;
+        const size_t lds = ((KIND == Recurrence::kChannelDelta ? 4 : 2) * R * RG + 4 * CG + 4 * 2 * 4 * CG) * 4;
+        one_delta_step_kernel<T, R, decltype(inputs)::value, KIND><<<grid, 256, lds, s>>>(part, io, rr, sc);
+    };
+    auto with_rows = [&](auto inputs) {
+        if (rpt <= 4) go(std::integral_constant<int, 4>{}, inputs);
+        else if (rpt <= 16) go(std::integral_constant<int, 16>{}, inputs);
+        else go(std::integral_constant<int, 32>{}, inputs);
+    };
+    if (in <= 512) with_rows(std::integral_constant<int, 2>{});
+    else with_rows(std::integral_constant<int, 4>{});
+    return true;
+}
+
 template <typename T, Recurrence KIND>
 void mixer_kind(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, uint32_t max_new, hipStream_t s) {
     const StepPlan p = step_plan(sh, rr.batch);
@@ -1277,7 +1496,8 @@ void mixer_kind(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, u
     const bool chunks = max_new >= kChunkFrom && g_delta_form != 1;
     const uint32_t longest = chunks ? kChunkFrom - 1 : max_new;      // sequences of a pass go to one of the two forms by length
     if (!chunks || rr.batch > 1) {
-        if (p.small) launch_step<T, 256, KIND>(sh, io, rr, p, write_ring, longest, s);
+        if (longest == 1 && launch_one_step<T, KIND>(sh, io, rr, p, write_ring, s)) (void)0;
+        else if (p.small) launch_step<T, 256, KIND>(sh, io, rr, p, write_ring, longest, s);
         else launch_step<T, 1024, KIND>(sh, io, rr, p, write_ring, longest, s);
     }
     if (chunks) run_chunks<T, KIND>(sh, io, rr, p.parts > 1 ? 0 : kChunkFrom, s);
