@@ -14,7 +14,7 @@ namespace fa {
 namespace k {
 using namespace fa::dev;
 
-int g_linear_form = 0;        // tuning: 2 keeps the large-tile kernel out; grouped rows: 4 streamed
+int g_linear_form = 0;        // tuning: 2 keeps the large-tile kernel out, 3 norms in front of the linears; grouped rows: 4 streamed
                               // weights, 5 128 x 128 tiles, 6 large tiles whatever the rows
 
 namespace {
@@ -73,23 +73,88 @@ __device__ __forceinline__ void stage_read(v4i (&a)[4][2], const uint32_t (&at)[
                  : "memory");
 }
 
-template <int MT, int NTW, int MODE, typename RowOf>
+// Up to four rows that are still ahead of their norm: the block norms them itself, two wavefronts to a row, while its first weights
+// travel, and keeps them in LDS (pitch below), so that the norm needs no launch in front of this one.  V: four values per thread
+// and step of 512 columns.  4 rows, the norm's launch and this one against this one alone: 2048 -> 6176 9.4,
+// 8.1 us; 2048 -> 1360 7.2, 5.8; 2048 -> 16384 16.0, 14.5; 4096 -> 12352 22.6, 21.2.
+constexpr uint32_t kNormRows = 4;
+__host__ __device__ constexpr uint32_t normed_pitch(uint32_t k_pad) { return k_pad * 2 + 32; }     // rows in different banks
+template <int V>
+struct RowsAhead {
+    v4f x[V], w[V];
+};
+template <int V>
+__device__ __forceinline__ void norm_rows_load(const NormAhead &nm, uint32_t m, RowsAhead<V> &ra) {
+    const uint32_t row = __builtin_amdgcn_readfirstlane(threadIdx.x / 128);
+    if (row >= m) return;
+    const float *x = nm.x + (uint64_t)row * nm.hidden;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const uint32_t c = (threadIdx.x % 128) * 4 + i * 512, from = c < nm.hidden ? c : nm.hidden - 4;
+        ra.x[i] = *(const v4f *)(x + from);
+        ra.w[i] = *(const v4f *)(nm.w + from);
+    }
+}
+// The rows' sums meet in `meet` [2 x 8]; two barriers, the normed rows are not yet published.
+template <int V>
+__device__ __forceinline__ void norm_rows_store(const NormAhead &nm, uint32_t m, uint32_t k_pad, RowsAhead<V> &ra, float *meet, uint8_t *rows) {
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), row = wave / 2;
+    float sum = 0.0f, sq = 0.0f, mean = 0.0f;
+    if (row < m && !nm.rms) {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            if ((threadIdx.x % 128) * 4 + i * 512 < nm.hidden) sum += (ra.x[i][0] + ra.x[i][1]) + (ra.x[i][2] + ra.x[i][3]);
+        sum = wave_sum_dpp(sum);
+    }
+    if (threadIdx.x % 64 == 0) meet[wave] = sum;
+    __syncthreads();
+    if (row < m) {
+        mean = nm.rms ? 0.0f : (meet[row * 2] + meet[row * 2 + 1]) / (float)nm.hidden;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            if ((threadIdx.x % 128) * 4 + i * 512 >= nm.hidden) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                ra.x[i][e] -= mean;
+                sq = fmaf(ra.x[i][e], ra.x[i][e], sq);
+            }
+        }
+        sq = wave_sum_dpp(sq);
+    }
+    if (threadIdx.x % 64 == 0) meet[8 + wave] = sq;
+    __syncthreads();
+    if (row >= m) return;
+    const float rstd = 1.0f / sqrtf((meet[8 + row * 2] + meet[8 + row * 2 + 1]) / (float)nm.hidden + nm.eps);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const uint32_t c = (threadIdx.x % 128) * 4 + i * 512;
+        if (c >= k_pad) continue;
+        const v4f y = c < nm.hidden ? ra.x[i] * rstd * ra.w[i] : v4f{0.f, 0.f, 0.f, 0.f};
+        *(v2u *)(rows + row * normed_pitch(k_pad) + c * 2) = v2u{f32x2_to_bf16x2(y[0], y[1]), f32x2_to_bf16x2(y[2], y[3])};
+    }
+}
+
+// NORM: 0 rows of `a`, otherwise V of the rows that `nm` names
+template <int MT, int NTW, int MODE, int NORM, typename RowOf>
 __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint64_t lda, const uint8_t *__restrict__ w_batch, uint32_t m,
-                                            uint32_t n, uint32_t n_tiles, uint32_t k_tiles, uint32_t batch, const LinearEpilogue &ep, uint8_t *lds,
-                                            RowOf row_of) {
+                                            uint32_t n, uint32_t n_tiles, uint32_t k_tiles, uint32_t batch, const LinearEpilogue &ep, const NormAhead &nm,
+                                            uint8_t *lds, RowOf row_of) {
+    static_assert(NORM == 0 || MT == 1, "rows that the block norms are few");
     static_assert(!is_glu(MODE) || NTW % 2 == 0, "gate and up are neighbouring tiles");
-    constexpr int NT = MT * NTW, STEP = is_glu(MODE) ? 2 : 1, LOADS = 2 * (MT + NTW);
+    constexpr int NT = MT * NTW, STEP = is_glu(MODE) ? 2 : 1, LOADS = 2 * ((NORM ? 0 : MT) + NTW);
     static_assert(NT <= kRowWaves * STEP, "a wavefront finishes one tile, or one gate and its up");
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t nt0 = blockIdx.x * NTW, pairs = k_tiles / 2;
     const uint32_t cnt = pairs > (uint32_t)wave ? (pairs - wave + kRowWaves - 1) / kRowWaves : 0;
     // load x of a row tile: rows 8 x .. + 7, lane l brings piece (l % 8) ^ (l / 8) of row l / 8, so that the 16 lanes an LDS
     // read serves together (eight rows of two neighbouring k groups) find theirs in different banks
-    const uint8_t *a_src[MT][2];
+    [[maybe_unused]] const uint8_t *a_src[MT][2];
+    [[maybe_unused]] RowsAhead<NORM ? NORM : 1> ra;
+    if constexpr (NORM != 0) norm_rows_load(nm, m, ra);
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
+        for (int x = 0; x < (NORM ? 0 : 2); ++x) {
             const uint32_t r = i * 16 + x * 8 + lane / 8;
             a_src[i][x] = (const uint8_t *)(a + (uint64_t)row_of(r < m ? r : m - 1).x * lda) + ((lane % 8) ^ (lane / 8)) * 16;
         }
@@ -99,6 +164,9 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
     uint8_t *stage = lds + wave * (kRowPairs * row_stage_bytes(MT));
     const uint32_t r16 = lane % 16, at0 = (uint32_t)(uintptr_t)(lptr)stage + (r16 / 8) * 1024 + (r16 % 8) * 128;
     const uint32_t at[2] = {at0 + (((uint32_t)lane / 16) ^ (r16 % 8)) * 16, at0 + ((4 + (uint32_t)lane / 16) ^ (r16 % 8)) * 16};
+    // normed rows: k group lane / 16 of row lane % 16; rows at or past m read row 0 and are never stored
+    uint8_t *normed = lds + kRowWaves * NT * 1024;
+    [[maybe_unused]] const uint8_t *own_row = normed + (r16 < m ? r16 : 0) * normed_pitch(k_tiles * 32) + lane / 16 * 16;
     // the tile this wavefront finishes
     const uint32_t t = wave * STEP, row = t / NTW * 16 + r16, tile = nt0 + t % NTW;
     const bool own = t < (uint32_t)NT && row < m && tile < n_tiles;
@@ -121,13 +189,18 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int x = 0; x < 2; ++x)
+            for (int x = 0; x < (NORM ? 0 : 2); ++x)
                 __builtin_amdgcn_global_load_lds((gptr)(a_src[i][x] + (uint64_t)p * 128), (lptr)(stage + s * row_stage_bytes(MT) + i * 2048 + x * 1024), 16, 0, 0);
     };
-    auto mul = [&](auto sc) {
+    auto mul = [&](auto sc, uint32_t it) {
         constexpr int s = decltype(sc)::value;
         v4i av[MT][2];
-        stage_read<s * (int)row_stage_bytes(MT)>(av, at);
+        if constexpr (NORM != 0) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) av[0][h] = *(const v4i *)(own_row + (wave + it * kRowWaves) * 128 + h * 64);
+        } else {
+            stage_read<s * (int)row_stage_bytes(MT)>(av, at);
+        }
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -141,27 +214,34 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
     if (cnt != 0) {
         load(0, 0);
         load(1, 1);
+    }
+    if constexpr (NORM != 0) {
+        __builtin_amdgcn_sched_barrier(0);
+        norm_rows_store(nm, m, k_tiles * 32, ra, (float *)(normed + kNormRows * normed_pitch(k_tiles * 32)), normed);
+        __syncthreads();
+    }
+    if (cnt != 0) {
         uint32_t it = 0;
         for (; it + 2 < cnt; it += 2) {
             // the reads of a slot are complete (stage_read waits) before it is loaded again
             loads_wait<LOADS>();
-            mul(std::integral_constant<int, 0>{});
+            mul(std::integral_constant<int, 0>{}, it);
             __builtin_amdgcn_sched_barrier(0);
             load(0, it + 2);
             __builtin_amdgcn_sched_barrier(0);
             loads_wait<LOADS>();
-            mul(std::integral_constant<int, 1>{});
+            mul(std::integral_constant<int, 1>{}, it + 1);
             __builtin_amdgcn_sched_barrier(0);
             load(1, it + 3);
             __builtin_amdgcn_sched_barrier(0);
         }
         loads_wait<LOADS>();
-        mul(std::integral_constant<int, 0>{});
+        mul(std::integral_constant<int, 0>{}, it);
         loads_wait<0>();
-        if (it + 1 < cnt) mul(std::integral_constant<int, 1>{});
+        if (it + 1 < cnt) mul(std::integral_constant<int, 1>{}, it + 1);
     }
     v4f(*red)[NT][64] = (v4f(*)[NT][64])lds;
-    __syncthreads();                                 // nobody reads rows any more
+    if constexpr (NORM == 0) __syncthreads();        // nobody reads staged rows any more
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -184,8 +264,15 @@ __global__ void __launch_bounds__(kRowWaves * 64)
                        uint32_t n, uint32_t n_tiles, uint32_t k_tiles, LinearEpilogue ep) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const uint32_t batch = blockIdx.y;
-    linear_rows<MT, NTW, MODE>(a + batch * a_batch, lda, w + (uint64_t)batch * n_tiles * k_tiles * 1024, m, n, n_tiles, k_tiles, batch, ep, lds,
-                               [](uint32_t r) { return make_uint2(r, r); });
+    linear_rows<MT, NTW, MODE, 0>(a + batch * a_batch, lda, w + (uint64_t)batch * n_tiles * k_tiles * 1024, m, n, n_tiles, k_tiles, batch, ep,
+                                  NormAhead{}, lds, [](uint32_t r) { return make_uint2(r, r); });
+}
+
+template <int V, int NTW, int MODE>
+__global__ void __launch_bounds__(kRowWaves * 64)
+    linear_normed_rows_kernel(NormAhead nm, const uint8_t *__restrict__ w, uint32_t m, uint32_t n, uint32_t n_tiles, uint32_t k_tiles, LinearEpilogue ep) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    linear_rows<1, NTW, MODE, V>(nullptr, 0, w, m, n, n_tiles, k_tiles, 0, ep, nm, lds, [](uint32_t r) { return make_uint2(r, r); });
 }
 
 // The rows of a group, up to 16 MT at a time (its weights then come from the caches again); groups without rows cost a
@@ -207,9 +294,9 @@ __global__ void __launch_bounds__(kRowWaves * 64)
             return make_uint2(e / rg.a_div, e);
         };
         if (r0) __syncthreads();
-        if (MT == 1 || left <= 16) linear_rows<1, NTW, MODE>(a, lda, wg, left < 16 ? left : 16, n, n_tiles, k_tiles, 0, ep, lds, row_of);
-        else if (MT == 2 || left <= 32) linear_rows<(MT < 2 ? MT : 2), NTW, MODE>(a, lda, wg, left < 32 ? left : 32, n, n_tiles, k_tiles, 0, ep, lds, row_of);
-        else linear_rows<MT, NTW, MODE>(a, lda, wg, left < 16 * MT ? left : 16 * MT, n, n_tiles, k_tiles, 0, ep, lds, row_of);
+        if (MT == 1 || left <= 16) linear_rows<1, NTW, MODE, 0>(a, lda, wg, left < 16 ? left : 16, n, n_tiles, k_tiles, 0, ep, NormAhead{}, lds, row_of);
+        else if (MT == 2 || left <= 32) linear_rows<(MT < 2 ? MT : 2), NTW, MODE, 0>(a, lda, wg, left < 32 ? left : 32, n, n_tiles, k_tiles, 0, ep, NormAhead{}, lds, row_of);
+        else linear_rows<MT, NTW, MODE, 0>(a, lda, wg, left < 16 * MT ? left : 16 * MT, n, n_tiles, k_tiles, 0, ep, NormAhead{}, lds, row_of);
     }
 }
 
@@ -418,17 +505,35 @@ void launch_rows_grouped(const uint16_t *a, uint64_t lda, const LinearWeight &w,
         a, lda, (const uint8_t *)w.w, w.n, w.n_tiles, w.k_tiles, rg, ep);
 }
 
+// Two tiles per block as soon as one tile each does not fit the device at once, so that the rows cross the L2 half as
+// often (4096 -> 6144 with 4, 16, 32 rows 11.0, 12.6, 16.4 and 10.0, 11.0, 13.1 us; 2048 -> 4096, which fits, 4.7, 5.1, 6.2 and
+// 5.5, 6.1, 7.5).  Four: behind two in nearly every shape (4096 -> 28672 with 32 rows 45.1 and 45.9).  Up to
+// four rows are hardly in the way, and four rounds of single tiles end more evenly (4096 -> 28672 38.9 and 36.4).
+bool two_tiles(bool glu, const LinearWeight &w, uint64_t m, int num_cus) {
+    const uint64_t tiles = (uint64_t)w.n_tiles * w.batches, cus = (uint64_t)num_cus;
+    return glu || (tiles > cus && (m > 4 || tiles < 4 * cus));
+}
+
+template <int V, int NTW, int MODE>
+void launch_normed_rows(const NormAhead &nm, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, hipStream_t s) {
+    const uint32_t lds = kRowWaves * NTW * 1024 + kNormRows * normed_pitch(w.k_tiles * 32) + 64;
+    linear_normed_rows_kernel<V, NTW, MODE><<<(w.n_tiles + NTW - 1) / NTW, kRowWaves * 64, lds, s>>>(nm, (const uint8_t *)w.w, (uint32_t)m, w.n, w.n_tiles,
+                                                                                              w.k_tiles, ep);
+}
+template <int MODE>
+void launch_normed(const NormAhead &nm, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+    const bool two = two_tiles(is_glu(MODE), w, m, num_cus), wide = w.k_tiles * 32 > 2048;
+    if constexpr (!is_glu(MODE))
+        if (!two) return wide ? launch_normed_rows<8, 1, MODE>(nm, m, w, ep, s) : launch_normed_rows<4, 1, MODE>(nm, m, w, ep, s);
+    wide ? launch_normed_rows<8, 2, MODE>(nm, m, w, ep, s) : launch_normed_rows<4, 2, MODE>(nm, m, w, ep, s);
+}
+
 template <int MODE>
 void launch_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
                  int num_cus, hipStream_t s) {
     const uint8_t *wt = (const uint8_t *)w.w;
     if (m <= 64) {
-        // Two tiles per block as soon as one tile each does not fit the device at once, so that the rows cross the L2 half as
-        // often (4096 -> 6144 with 4, 16, 32 rows 11.0, 12.6, 16.4 and 10.0, 11.0, 13.1 us; 2048 -> 4096, which fits, 4.7, 5.1, 6.2 and
-        // 5.5, 6.1, 7.5).  Four: behind two in nearly every shape (4096 -> 28672 with 32 rows 45.1 and 45.9).  Up to
-        // four rows are hardly in the way, and four rounds of single tiles end more evenly (4096 -> 28672 38.9 and 36.4).
-        const uint64_t tiles = (uint64_t)w.n_tiles * w.batches, cus = (uint64_t)num_cus;
-        const bool two = is_glu(MODE) || (tiles > cus && (m > 4 || tiles < 4 * cus));
+        const bool two = two_tiles(is_glu(MODE), w, m, num_cus);
         if (m <= 16) {
             if constexpr (!is_glu(MODE))
                 if (!two) return launch_rows<1, 1, MODE>(a, lda, a_batch, m, w, ep, s);
@@ -502,6 +607,25 @@ void linear_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, 
         case LinearEpilogue::kHeadGate: return launch_bf16<LinearEpilogue::kHeadGate>(a, lda, a_batch, m, w, ep, num_cus, s);
         case LinearEpilogue::kXielu: return launch_bf16<LinearEpilogue::kXielu>(a, lda, a_batch, m, w, ep, num_cus, s);
         default: return launch_bf16<LinearEpilogue::kStore>(a, lda, a_batch, m, w, ep, num_cus, s);
+    }
+}
+
+// Up to what the LDS and a thread's registers hold of the rows, and while the blocks that norm the same rows again cost less than
+// the launch (4 rows, us, with the launch and without: 896 blocks at k of 4096 42.9 and 42.2, 2000 at 2048 25.4 and 24.7, 2000 at 4096
+// 44.6 and 46.3).
+bool linear_norms_rows(uint64_t m, uint64_t hidden, const LinearWeight &w, bool glu, int num_cus) {
+    const uint64_t k_pad = (uint64_t)w.k_tiles * 32, ntw = two_tiles(glu, w, m, num_cus) ? 2 : 1, blocks = (w.n_tiles + ntw - 1) / ntw;
+    return m <= kNormRows && hidden % 4 == 0 && hidden <= k_pad && k_pad <= 4096 && blocks * k_pad <= 5 << 20 && w.batches == 1 && g_linear_form != 3;
+}
+
+void linear_normed_bf16(const NormAhead &nm, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+    if (m == 0) return;
+    switch (ep.mode) {
+        case LinearEpilogue::kGlu: return launch_normed<LinearEpilogue::kGlu>(nm, m, w, ep, num_cus, s);
+        case LinearEpilogue::kSiluGlu: return launch_normed<LinearEpilogue::kSiluGlu>(nm, m, w, ep, num_cus, s);
+        case LinearEpilogue::kSoftcap: return launch_normed<LinearEpilogue::kSoftcap>(nm, m, w, ep, num_cus, s);
+        case LinearEpilogue::kXielu: return launch_normed<LinearEpilogue::kXielu>(nm, m, w, ep, num_cus, s);
+        default: return launch_normed<LinearEpilogue::kStore>(nm, m, w, ep, num_cus, s);
     }
 }
 

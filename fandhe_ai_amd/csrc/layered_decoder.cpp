@@ -266,6 +266,24 @@ void linear(fa_context *ctx, const LayeredState &L, const void *a, uint64_t lda,
     else k::linear_bf16((const uint16_t *)a, lda, a_batch, m, w, ep, ctx->props.multiProcessorCount, ctx->stream);
 }
 
+// A norm of the residual that the next linear may take into its own launch, or that goes out now, into a.hn
+struct Normed {
+    k::NormAhead ahead;
+    bool fused;
+};
+Normed norm_ahead(fa_context *ctx, const LayeredState &L, const Arena &a, const float *x, const float *w, int rms, uint32_t rows, const k::LinearWeight &next,
+                  bool glu = false) {
+    const uint32_t D = L.cfg.d_model, ld_hn = pad_to(D, 64);
+    const Normed nm{k::NormAhead{x, w, D, L.cfg.norm_eps, rms}, !L.is_f32 && k::linear_norms_rows(rows, D, next, glu, ctx->props.multiProcessorCount)};
+    if (!nm.fused) (rms ? k::rmsnorm_rows : k::layernorm_rows)(x, w, a.hn, L.is_f32, rows, D, ld_hn, L.cfg.norm_eps, ctx->stream);
+    return nm;
+}
+// ... and that linear, from the rows or from a.hn
+void linear_of(fa_context *ctx, const LayeredState &L, const Arena &a, const Normed *nm, uint32_t ld_hn, uint64_t m, const k::LinearWeight &w, const k::LinearEpilogue &ep) {
+    if (nm && nm->fused) k::linear_normed_bf16(nm->ahead, m, w, ep, ctx->props.multiProcessorCount, ctx->stream);
+    else linear(ctx, L, a.hn, ld_hn, 0, m, w, ep);
+}
+
 k::LinearEpilogue store_to(void *out, uint64_t ld, int out_f32) {
     k::LinearEpilogue e;
     e.out = out;
@@ -288,8 +306,8 @@ struct Portions {
 // Element `at` of an activation section in the activations' type
 void *element(const LayeredState &L, void *base, uint64_t at) { return (uint8_t *)base + at * L.esz; }
 
-// The layer's input a.hn -> what its mixers read, a.y and a.y32.
-void enqueue_in(fa_context *ctx, LayeredState &L, Arena &a, const Layer &l, uint32_t rows, uint32_t ld_hn) {
+// The layer's input (a.hn, or what nm says) -> what its mixers read, a.y and a.y32.
+void enqueue_in(fa_context *ctx, LayeredState &L, Arena &a, const Layer &l, uint32_t rows, uint32_t ld_hn, const Normed *nm) {
     k::LinearEpilogue e = l.lo ? store_to(a.y, l.lo, L.is_f32) : store_to(a.y32, pad_to(l.hi, 4), 1);
     if (l.lo) {
         e.n_lo = l.lo;
@@ -297,7 +315,7 @@ void enqueue_in(fa_context *ctx, LayeredState &L, Arena &a, const Layer &l, uint
         e.ld_hi = pad_to(l.hi, 4);
     }
     e.bias = l.in_bias;
-    linear(ctx, L, a.hn, ld_hn, 0, rows, l.in, e);
+    linear_of(ctx, L, a, nm, ld_hn, rows, l.in, e);
 }
 
 // The mixers: from a.y and a.y32 to their columns of a.o (pitch ld_o).
@@ -428,9 +446,9 @@ void enqueue_attention(fa_context *ctx, LayeredState &L, Arena &a, const Layer &
 }
 
 void enqueue_mixers(fa_context *ctx, fa_decoder *d, Arena &a, const Layer &l, const k::RaggedRows &rr, Portions n, uint32_t ld_hn, uint32_t ld_o,
-                    const ExpandPlan *expand) {
+                    const ExpandPlan *expand, const Normed *nm) {
     LayeredState &L = *d->layered;
-    enqueue_in(ctx, L, a, l, rr.rows, ld_hn);
+    enqueue_in(ctx, L, a, l, rr.rows, ld_hn, nm);
     for (const Mixer &m : l.mixers) {
         if (recurrent(m.cfg)) enqueue_recurrence(ctx, L, a, l, m, rr, n.max_new, ld_o);
         else if (m.cfg.mixer == FA_MIXER_MINGRU) enqueue_gated(ctx, L, a, l, m, rr, n.max_new, ld_o);
@@ -439,15 +457,16 @@ void enqueue_mixers(fa_context *ctx, fa_decoder *d, Arena &a, const Layer &l, co
     }
 }
 
-// Dense feed-forward: from a.hn to what `out` does with the down projection.
-void enqueue_dense(fa_context *ctx, LayeredState &L, Arena &a, const Layer &l, uint32_t M, uint32_t ld_hn, const k::LinearEpilogue &out) {
+// Dense feed-forward: from a.hn (or what nm says) to what `out` does with the down projection.
+void enqueue_dense(fa_context *ctx, LayeredState &L, Arena &a, const Layer &l, uint32_t M, uint32_t ld_hn, const k::LinearEpilogue &out,
+                   const Normed *nm = nullptr) {
     const uint32_t ld_act = pad_to(l.cfg.d_ffn, 64);
     k::LinearEpilogue g = store_to(a.act, ld_act, L.is_f32);
     g.mode = l.cfg.glu == FA_GLU_SILU ? k::LinearEpilogue::kSiluGlu : l.cfg.glu == FA_FFN_XIELU ? k::LinearEpilogue::kXielu : k::LinearEpilogue::kGlu;
     g.act = l.act;
     g.limit = l.cfg.ffn_limit;
     g.alpha = l.cfg.ffn_alpha;
-    linear(ctx, L, a.hn, ld_hn, 0, M, l.gate_up, g);
+    linear_of(ctx, L, a, nm, ld_hn, M, l.gate_up, g);
     linear(ctx, L, a.act, ld_act, 0, M, l.down, out);
 }
 
@@ -505,9 +524,10 @@ fa_status enqueue_layers(fa_context *ctx, fa_decoder *d, Arena &a, const k::Ragg
     }
     for (size_t li = 0; li < L.layers.size(); ++li) {
         const Layer &l = L.layers[li];
-        if (L.cfg.norm == FA_NORM_INPUT) k::layernorm_rows(a.x, l.norm1, a.hn, f32, M, D, ld_hn, eps, s);
+        Normed nm{};
+        if (L.cfg.norm == FA_NORM_INPUT) nm = norm_ahead(ctx, L, a, a.x, l.norm1, 0, M, l.in);
         const uint32_t ld_o = pad_to(l.o_width, 64);
-        enqueue_mixers(ctx, d, a, l, rr, n, ld_hn, ld_o, expand);
+        enqueue_mixers(ctx, d, a, l, rr, n, ld_hn, ld_o, expand, &nm);
         k::ResidualNorm rn;
         rn.y = a.y32;
         rn.eps = eps;
@@ -574,9 +594,9 @@ fa_status enqueue_layers(fa_context *ctx, fa_decoder *d, Arena &a, const k::Ragg
             r.scale = l.post1;
             linear(ctx, L, a.o, ld_o, 0, M, l.out, r);
             if (l.cfg.d_ffn) {
-                k::layernorm_rows(a.x, l.norm2, a.hn, f32, M, D, ld_hn, eps, s);
+                nm = norm_ahead(ctx, L, a, a.x, l.norm2, 0, M, l.gate_up, l.cfg.glu != FA_FFN_XIELU);
                 r.scale = l.post2;
-                enqueue_dense(ctx, L, a, l, M, ld_hn, r);
+                enqueue_dense(ctx, L, a, l, M, ld_hn, r, &nm);
             }
         }
         if (L.trace) {
@@ -600,13 +620,12 @@ void enqueue_embed(fa_context *ctx, const LayeredState &L, Arena &a, const int32
 // Final norm and head over rows of f32 residuals.
 void enqueue_head(fa_context *ctx, LayeredState &L, Arena &a, const float *x, uint32_t rows, float *logits) {
     const uint32_t ld_hn = pad_to(L.cfg.d_model, 64);
-    if (L.cfg.norm == FA_NORM_OUTPUT || L.cfg.norm == FA_NORM_INPUT_RMS) k::rmsnorm_rows(x, L.final_norm, a.hn, L.is_f32, rows, L.cfg.d_model, ld_hn, L.cfg.norm_eps, ctx->stream);
-    else k::layernorm_rows(x, L.final_norm, a.hn, L.is_f32, rows, L.cfg.d_model, ld_hn, L.cfg.norm_eps, ctx->stream);
+    const Normed nm = norm_ahead(ctx, L, a, x, L.final_norm, L.cfg.norm == FA_NORM_OUTPUT || L.cfg.norm == FA_NORM_INPUT_RMS, rows, L.head);
     k::LinearEpilogue e = store_to(logits, L.cfg.vocab, 1);
     e.mode = k::LinearEpilogue::kSoftcap;
     e.factor = L.cfg.logit_scale;
     e.cap = L.cfg.logit_softcap;
-    linear(ctx, L, a.hn, ld_hn, 0, rows, L.head, e);
+    linear_of(ctx, L, a, &nm, ld_hn, rows, L.head, e);
 }
 
 k::RaggedRows ragged(const fa_decoder *d, const Arena &a, const uint32_t *row_start, uint32_t rows) {

@@ -112,7 +112,7 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  * key 27: prompt passes whose q | k | v projection runs on the weight-stationary kernel: 0: RoPE, the bf16 rounding and
  *        the K / V append in that kernel's epilogue, 1: a pass of their own behind it;
  * layered decoders: key 28: rows per internal pass of a long prompt, from 64 up (smaller: the built-in 8192);
- * key 29: bf16 linears: 2: never the large-tile kernel; experts' linears: 4: weights streamed past the rows,
+ * key 29: bf16 linears: 2: never the large-tile kernel, 3: norms never inside them; experts' linears: 4: weights streamed past the rows,
  *        5: 128 x 128 tiles, 6: large tiles, whatever the number of rows;
  * key 30: latent attention: 1: the plain kernel, 2: the absorbed form for every pass, 3: the expanded form wherever it
  *        can run; key 31: gated delta rule: 1: token by token for prompts too, 2: a state's rows always

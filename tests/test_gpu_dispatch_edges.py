@@ -286,6 +286,26 @@ def test_bf16_rows(name, rows, tune):
     assert np.median(err) < 0.06 and err.max() < 0.12, (np.median(err), err.max())
 
 
+@pytest.mark.parametrize("width", [76, 2048, 2052, 4096])
+@pytest.mark.parametrize("rows", [1, 3, 4, 5])
+def test_norms_inside_the_linears(rows, width, tune):
+    """Up to four rows are normed by the linears that take them: widths around the pad of k and what a thread holds of a row, fewer rows
+    than four; the norm in a launch of its own beside it."""
+    cfg = lc.config([lc.delta(heads=2, kv_heads=1, dim=16, vdim=16, mlp=lc.glu(ff=96))], width=width, vocab=300)
+    w, toks = lc.weights(cfg, 5), lc.tokens(cfg, rows, 41)
+    dec = lc.make_decoder(ops(), cfg, w, "bfloat16", max_tokens=64, max_batch=1)
+    table = np.full((1, dec.cfg.max_blocks_per_seq), 0xFFFFFFFF, dtype=np.uint32)
+    table[0, 0] = 0
+    want = oracle.forward(cfg, w, toks)
+    err = {}
+    for form in (0, 3):
+        tune(29, form)
+        dec.set_sequences(table, [0])
+        err[form] = lc.error(dec.forward([toks], [list(range(rows))]), want)
+    dec.close()
+    assert max(err.values()) < 0.06 and abs(err[0] - err[3]) < 0.02, err
+
+
 @pytest.mark.parametrize("mtb,ntb,waves", [(8, 16, 4), (12, 14, 16), (16, 8, 4), (16, 14, 4), (16, 16, 16), (8, 8, 4)])
 @pytest.mark.parametrize("kind", ["int8", "e4m3"])
 def test_plan_names_the_wavefronts_that_are_launched(kind, mtb, ntb, waves, tune):
