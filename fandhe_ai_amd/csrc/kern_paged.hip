@@ -175,6 +175,8 @@ struct StreamParams {
     uint32_t shares = 1;
     float *one_part = nullptr, *one_part_ml = nullptr;
     uint32_t *one_counters = nullptr;
+    uint32_t items_inv = 0, kv_heads_inv = 0;               // ixm::inverse of batch * num_kv_heads and of num_kv_heads
+    uint32_t *xcc_seen = nullptr, *fault = nullptr;         // LOCAL: SplitKArea's
 };
 
 // The new tokens of sequence b: rows first .. first + n - 1 of the pass
@@ -222,7 +224,10 @@ __device__ __forceinline__ uint32_t range_pages(const StreamParams &p, uint32_t 
 // p.shares blocks while compute units are left: each leaves its sums, and the one that draws the last ticket adds them in the
 // order of the shares.  Eight kv heads of one sequence, 700 tokens: 18.9 us in 8 blocks, 13.4 in 24; the streamed form 9.6 and
 // 10.0 for its merge.  The arithmetic of both meetings is that of the merge kernels.
-template <int SP, int KD, int VD, int WPE, bool PF, int TT = 1, bool ONE = false>
+// LOCAL: the shares of a sequence and kv head run on one XCD and meet in its L2 (checked as in the split-k linears).  The launch is
+// a chain of latencies, so what a block needs to find its pages is 32-bit arithmetic without loops: with 64-bit divisions and a
+// meeting in memory a sequence of 700 tokens took 14.4 us, so 12.3, and 11.3 in groups of two pages instead of four.
+template <int SP, int KD, int VD, int WPE, bool PF, int TT = 1, bool ONE = false, bool LOCAL = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, WPE))) decode_stream_kernel(StreamParams p) {
     static_assert(PF || TT == 1, "several token tiles per wavefront exist only in the prefill form");
     static_assert(!ONE || !PF, "the one-block form is a decode form");
@@ -235,8 +240,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
     const int lane = threadIdx.x % 64;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int g = lane / 16, c = lane % 16;
-    const uint32_t item_id = ONE ? blockIdx.x % (p.batch * p.num_kv_heads) : blockIdx.x * 4 + wave;
-    const uint32_t kvh = item_id % p.num_kv_heads, r = item_id / p.num_kv_heads;   // ONE: r is the sequence
+    const uint32_t share = ONE ? ixm::quotient(blockIdx.x, p.items_inv) : 0;
+    const uint32_t item_id = ONE ? blockIdx.x - share * (p.batch * p.num_kv_heads) : blockIdx.x * 4 + wave;
+    const uint32_t r = ONE ? ixm::quotient(item_id, p.kv_heads_inv) : item_id / p.num_kv_heads;   // ONE: the sequence
+    const uint32_t kvh = item_id - r * p.num_kv_heads;
     if (r >= (ONE ? p.batch : p.n_ranges)) return;
     const uint32_t max_ctx = p.max_blocks_per_seq * kPage;
     const uint32_t nv = PF ? p.n_vseq : p.batch;
@@ -524,11 +531,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
         const uint32_t len_b = p.seq_lens[r];
         const uint32_t len_c = len_b > max_ctx ? max_ctx : len_b;
         const uint32_t npg = (len_c + kPage - 1) / kPage;
-        const uint32_t items = p.batch * p.num_kv_heads, share = blockIdx.x / items, fill = (npg + kOneSharePages - 1) / kOneSharePages;
+        const uint32_t fill = (npg + kOneSharePages - 1) / kOneSharePages;
         const uint32_t shares = fill < 2 ? 1 : fill < p.shares ? fill : p.shares;
         if (share >= shares) return;
-        const uint32_t part = share * 4 + wave, parts = shares * 4;
-        const uint32_t lo = (uint32_t)((uint64_t)npg * part / parts), hi = (uint32_t)((uint64_t)npg * (part + 1) / parts);
+        const uint32_t part = share * 4 + wave;
+        uint32_t lo, hi;
+        ixm::decode_one_pages(npg, part, shares, &lo, &hi);
         if (hi > lo) {
             segment(r, lo, hi, len_b);
         } else {                                                       // no pages for this wavefront: weight zero
@@ -560,27 +568,35 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
         }
         if (shares > 1) {
             const uint64_t first = (uint64_t)item_id * p.shares;
-            float *sums = p.one_part + first * 2048 + threadIdx.x * 8, *ml = p.one_part_ml + first * 32 + c;
+            // words of this thread in one_part, and of its column in one_part_ml
+            const uint32_t sums = (uint32_t)first * 2048 + threadIdx.x * 8, ml = (uint32_t)first * 32 + c;
             if ((uint32_t)c < p.group) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) meet_store<false>(sums + share * 2048 + e, acc[e]);
+                for (int e = 0; e < 8; e += 4)
+                    meet_store_b128<LOCAL>((int32_t *)p.one_part, sums + share * 2048 + e, __builtin_bit_cast(v4i, v4f{acc[e], acc[e + 1], acc[e + 2], acc[e + 3]}));
                 if (wave == 0 && g == 0) {
-                    meet_store<false>(ml + share * 32, mx);
-                    meet_store<false>(ml + share * 32 + 16, den);
+                    meet_store<LOCAL>(p.one_part_ml + ml + share * 32, mx);
+                    meet_store<LOCAL>(p.one_part_ml + ml + share * 32 + 16, den);
                 }
             }
-            if (meet_ticket<false>(p.one_counters + item_id, &one_ticket) != shares - 1) return;
-            if (threadIdx.x == 0) meet_store<false>(p.one_counters + item_id, 0u);
+            if (LOCAL && threadIdx.x == 0) meet_store<true>(p.xcc_seen + first + share, this_xcc() + 1u);
+            if (meet_ticket<LOCAL>(p.one_counters + item_id, &one_ticket) != shares - 1) return;
+            if (threadIdx.x == 0) meet_store<LOCAL>(p.one_counters + item_id, 0u);
+            if (LOCAL && wave == 3) {                                      // all shares on this XCD, or their sums went through two L2s
+                const uint32_t mine = this_xcc() + 1u, seen = (uint32_t)lane < shares ? meet_load<true>(p.xcc_seen + first + lane) : mine;
+                if (__ballot(seen != mine) != 0 && lane == 0) __hip_atomic_store(p.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
             // in the order of the shares, whoever came last; shares that are not there repeat the last with weight zero
-            float m[kOneShares], l[kOneShares], o[kOneShares][8];
+            float m[kOneShares], l[kOneShares];
+            v4f o[kOneShares][2];
             if ((uint32_t)c < p.group) {
 #pragma unroll
                 for (uint32_t t = 0; t < kOneShares; ++t) {
                     const uint32_t at = t < shares ? t : shares - 1;
-                    m[t] = meet_load<false>(ml + at * 32);
-                    l[t] = meet_load<false>(ml + at * 32 + 16);
+                    m[t] = meet_load<LOCAL>(p.one_part_ml + ml + at * 32);
+                    l[t] = meet_load<LOCAL>(p.one_part_ml + ml + at * 32 + 16);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) o[t][e] = meet_load<false>(sums + at * 2048 + e);
+                    for (int e = 0; e < 2; ++e) o[t][e] = __builtin_bit_cast(v4f, meet_load_b128<LOCAL>((const int32_t *)p.one_part, sums + at * 2048 + e * 4));
                 }
                 mx = -INFINITY;
 #pragma unroll
@@ -593,7 +609,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
                     const float wt = t < shares ? expf(m[t] - mx) : 0.0f;
                     den = __builtin_fmaf(wt, l[t], den);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(wt, o[t][e], acc[e]);
+                    for (int e = 0; e < 8; ++e) acc[e] = __builtin_fmaf(wt, o[t][e / 4][e % 4], acc[e]);
                 }
             }
         }
@@ -1547,7 +1563,16 @@ void paged_attention_decode_one_bf16(const uint16_t *q, const uint16_t *k_pool, 
         sp.one_part_ml = sp.one_part + items * shares * 2048;
         sp.one_counters = sk->counters;
     }
-    decode_stream_kernel<4, 4, 2, 2, false, 1, true><<<(unsigned)(items * shares), 256, 0, s>>>(sp);
+    sp.items_inv = ixm::inverse((uint32_t)items);
+    sp.kv_heads_inv = ixm::inverse(ps.num_kv_heads);
+    // the shares of an item are `items` blocks apart, and blocks go round the eight XCDs
+    if (shares > 1 && sk->xcd_local && items % 8 == 0 && sk->xcc_seen && sk->fault && items * shares <= sk->n_xcc_seen) {
+        sp.xcc_seen = sk->xcc_seen;
+        sp.fault = sk->fault;
+        decode_stream_kernel<2, 2, 2, 2, false, 1, true, true><<<(unsigned)(items * shares), 256, 0, s>>>(sp);
+    } else {
+        decode_stream_kernel<2, 2, 2, 2, false, 1, true><<<(unsigned)(items * shares), 256, 0, s>>>(sp);
+    }
 }
 
 // Prefill (l_new > 1) on the same streaming kernel: groups of kPrefillTT token tiles of 16 / group new tokens

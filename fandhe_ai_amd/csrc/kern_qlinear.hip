@@ -1187,34 +1187,6 @@ __global__ void __launch_bounds__(512)
 // are coherent between XCDs wherever the blocks run.  The ticket is relaxed; what orders it behind the stores is
 // the wait for their acknowledgement, not a fence (an agent-scope release writes back a whole L2).  (meet_store, meet_load,
 // meet_ticket: device_utils.hpp)
-// Four consecutive words of a partial tile set, with the cache policy of meet_load (a wider relaxed atomic load does not
-// exist; the words were written by one 16-byte store whose acknowledgement the writer awaited before its ticket).  A buffer
-// load, because its builtin takes the policy (1: sc0, 16: sc1) and leaves registers and waits to the compiler: as an
-// assembly statement whose wait stands elsewhere, nothing would keep the compiler from moving a register still in flight.
-// `word` counts from `base`; the resource has no bound of its own, so base + word must lie in the workspace (below 4 GiB).
-template <bool LOCAL>
-__device__ __forceinline__ v4i meet_load_b128(const int32_t *base, uint32_t word) {
-    const __amdgpu_buffer_rsrc_t area = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
-    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(area, word * 4, 0, LOCAL ? 1 : 16));
-}
-// LOCAL only: the members of a group must share an XCD, or the partial tiles above were exchanged through two
-// different L2s.  Every member notes the XCD it runs on before it takes its ticket; the last arriver compares and
-// reports a mismatch in host memory (the context then refuses further work: the launch's results are wrong).
-__device__ __forceinline__ uint32_t this_xcc() {
-    uint32_t id;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(id));
-    return id & 15u;
-}
-template <int S>
-__device__ __forceinline__ void meet_check_xcd(const uint32_t *xcc_seen, uint32_t group, uint32_t *fault) {
-    if (threadIdx.x != 0 || !xcc_seen) return;
-    const uint32_t mine = this_xcc();
-    bool same = true;
-#pragma unroll
-    for (int r = 0; r < S; ++r) same = same && meet_load<true>(xcc_seen + (uint64_t)group * S + r) == mine + 1u;
-    if (!same) __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 // block -> (group, member) of a split-k launch: see above
 template <int S>
 __device__ __forceinline__ void ksplit_ids(uint32_t *group, uint32_t *member) {
