@@ -36,10 +36,17 @@ FA_HD bool decode_attends_at_once(uint64_t share, uint64_t even, uint64_t shares
     return 8 * (share > even ? share - even : 0) + (shares == 2 ? 9 : 6) * share / 2 <= 6400;
 }
 
-// Quotients by a number of the launch: inverse(n) = 2^31 / n rounded up; exact for x < 2^31 / n (the product is off by less than
-// x n / 2^31 parts of one, and quotients are n-ths), and for any x below 2^31 where n is a power of two.
-FA_HD_CALL uint32_t inverse(uint32_t n) { return (uint32_t)(((1ull << 31) + n - 1) / n); }
-FA_HD_CALL uint32_t quotient(uint32_t x, uint32_t inverse_n) { return (uint32_t)((uint64_t)x * inverse_n >> 31); }
+// Quotients by a number of the launch without the device's division (20 to 30 instructions): m = 2^(31 + L) / n rounded up, 2^L >= n.
+// The product is off by less than x n / 2^(31 + L) <= x / 2^31 n-ths, so the quotient of any x below 2^31 is exact.
+struct Divider {
+    uint32_t m, shift;
+};
+FA_HD_CALL Divider divider(uint32_t n) {
+    uint32_t l = 0;
+    while ((1ull << l) < n) ++l;
+    return Divider{(uint32_t)(((1ull << (31 + l)) + n - 1) / n), 31 + l};
+}
+FA_HD_CALL uint32_t quotient(uint32_t x, const Divider &d) { return (uint32_t)((uint64_t)x * d.m >> d.shift); }
 // Pages lo .. hi - 1 of the npg pages of a sequence (below 2^26) for wavefront `part` of its 4 * shares (shares <= 8): an even split
 FA_HD_CALL void decode_one_pages(uint32_t npg, uint32_t part, uint32_t shares, uint32_t *lo, uint32_t *hi) {
     *lo = (npg * part >> 2) / shares;

@@ -222,9 +222,9 @@ __global__ void __launch_bounds__(NT)
 // that are formed meanwhile), the ring's places take one remainder instead of one per tap, and the wavefronts meet twice.
 // 4 sequences of 16 heads 128 x 128: 7.4 us, 10.5 on a thousand threads of the kernel above; 32 sequences 14.5 and 35.5; 16 sequences
 // of 32 heads 16.8.
-// share_m, taps_m: ixm::inverse (at most 4 taps, positions below 2^29).
 struct StepScalars {
-    uint32_t cg_log2, share, share_m, taps_m;
+    uint32_t cg_log2, share;
+    ixm::Divider by_share, by_taps;
     float rsqrt_dim;
     int write_ring;
 };
@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256) one_delta_step_kernel(DeltaShape sh, Delt
     const uint32_t start = rr.row_start[b], end = rr.row_start[b + 1], slot = rr.state_slot[b], row = start < rr.rows ? start : rr.rows - 1;
     const uint32_t dim = sh.dim, vdim = sh.vdim, vp = sh.vdim_p(), channels = sh.qkv(), taps = sh.taps;
     const uint32_t CG = 1u << sc.cg_log2, RG = NT >> sc.cg_log2, cg = threadIdx.x & (CG - 1), rg = threadIdx.x >> sc.cg_log2, lane = threadIdx.x % 64;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), hk = ixm::quotient(h, sc.share_m), share = sc.share;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), hk = ixm::quotient(h, sc.by_share), share = sc.share;
     const uint32_t col0 = blockIdx.z * CG * 4, cols = vdim - col0 < CG * 4 ? vdim - col0 : CG * 4, col = col0 + cg * 4;
     float *lv = lds + RPT * RG * STR, *part = lv + CG * 4;
     const T *y = (const T *)io.y + (uint64_t)row * io.ld_y;
@@ -304,7 +304,7 @@ __global__ void __launch_bounds__(256) one_delta_step_kernel(DeltaShape sh, Delt
     }
     __builtin_amdgcn_sched_barrier(0);
     if (start == end) return;
-    const uint32_t p = (uint32_t)rr.pos[row], place = p - ixm::quotient(p, sc.taps_m) * (taps ? taps : 1);          // p % taps
+    const uint32_t p = (uint32_t)rr.pos[row], place = p - ixm::quotient(p, sc.by_taps) * (taps ? taps : 1);          // p % taps
     float beta = 1.0f, g = 1.0f;
     const float a_log = LIGHTNING ? 0.0f : io.a_log[h];
     if constexpr (LIGHTNING) {
@@ -1468,7 +1468,7 @@ bool launch_one_step(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &
     const uint32_t CG = 1u << p.cg_log2, RG = 256 >> p.cg_log2, rpt = (sh.dim + RG - 1) / RG, in = 2 * sh.dim + 4 * CG;
     if (sh.taps > 4 || in > 1024 || rpt > 32) return false;
     const uint32_t share = sh.heads / sh.kv_heads;
-    const StepScalars sc{p.cg_log2, share, ixm::inverse(share), ixm::inverse(sh.taps ? sh.taps : 1), (float)(1.0 / std::sqrt((double)sh.dim)), write_ring};
+    const StepScalars sc{p.cg_log2, share, ixm::divider(share), ixm::divider(sh.taps ? sh.taps : 1), (float)(1.0 / std::sqrt((double)sh.dim)), write_ring};
     DeltaShape part = sh;
     if (p.parts > 1) part.norm_all = 1;
     const dim3 grid(rr.batch, sh.heads, p.parts);

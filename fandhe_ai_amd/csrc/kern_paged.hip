@@ -175,7 +175,7 @@ struct StreamParams {
     uint32_t shares = 1;
     float *one_part = nullptr, *one_part_ml = nullptr;
     uint32_t *one_counters = nullptr;
-    uint32_t items_inv = 0, kv_heads_inv = 0;               // ixm::inverse of batch * num_kv_heads and of num_kv_heads
+    ixm::Divider by_items{}, by_kv_heads{};                 // batch * num_kv_heads, num_kv_heads
     uint32_t *xcc_seen = nullptr, *fault = nullptr;         // LOCAL: SplitKArea's
 };
 
@@ -240,9 +240,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
     const int lane = threadIdx.x % 64;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int g = lane / 16, c = lane % 16;
-    const uint32_t share = ONE ? ixm::quotient(blockIdx.x, p.items_inv) : 0;
+    const uint32_t share = ONE ? ixm::quotient(blockIdx.x, p.by_items) : 0;
     const uint32_t item_id = ONE ? blockIdx.x - share * (p.batch * p.num_kv_heads) : blockIdx.x * 4 + wave;
-    const uint32_t r = ONE ? ixm::quotient(item_id, p.kv_heads_inv) : item_id / p.num_kv_heads;   // ONE: the sequence
+    const uint32_t r = ONE ? ixm::quotient(item_id, p.by_kv_heads) : item_id / p.num_kv_heads;   // ONE: the sequence
     const uint32_t kvh = item_id - r * p.num_kv_heads;
     if (r >= (ONE ? p.batch : p.n_ranges)) return;
     const uint32_t max_ctx = p.max_blocks_per_seq * kPage;
@@ -1563,8 +1563,8 @@ void paged_attention_decode_one_bf16(const uint16_t *q, const uint16_t *k_pool, 
         sp.one_part_ml = sp.one_part + items * shares * 2048;
         sp.one_counters = sk->counters;
     }
-    sp.items_inv = ixm::inverse((uint32_t)items);
-    sp.kv_heads_inv = ixm::inverse(ps.num_kv_heads);
+    sp.by_items = ixm::divider((uint32_t)items);
+    sp.by_kv_heads = ixm::divider(ps.num_kv_heads);
     // the shares of an item are `items` blocks apart, and blocks go round the eight XCDs
     if (shares > 1 && sk->xcd_local && items % 8 == 0 && sk->xcc_seen && sk->fault && items * shares <= sk->n_xcc_seen) {
         sp.xcc_seen = sk->xcc_seen;

@@ -435,10 +435,11 @@ static void decode_form_cases() {
 
 // Quotients by numbers of a launch, and the even split of a sequence's pages, against plain 64-bit arithmetic
 static void quotient_cases() {
-    for (uint32_t n = 1; n <= 2048; ++n)
-        for (uint32_t x : {0u, 1u, n - 1, n, n + 1, 7 * n - 1, 7 * n, 65535u, 1000000u}) CHECK(quotient(x, inverse(n)) == x / n);
-    for (uint32_t n = 1; n <= 4; ++n)
-        for (uint32_t x = (1u << 29) - 3000; x < (1u << 29); ++x) CHECK(quotient(x, inverse(n)) == x / n);
+    const uint32_t top = (1u << 31) - 1;
+    for (uint32_t n = 1; n <= 5000; ++n)
+        for (uint32_t x : {0u, 1u, n - 1, n, n + 1, 7 * n - 1, 7 * n, 65535u, 1000000u, top / n * n - 1, top / n * n, top}) CHECK(quotient(x, divider(n)) == x / n);
+    for (uint32_t n : {65535u, 65536u, 65537u, 1u << 30, top})
+        for (uint32_t x : {0u, 1u, n - 1, n, top / n * n - 1, top / n * n, top}) CHECK(quotient(x, divider(n)) == x / n);
     for (uint32_t shares = 1; shares <= 8; ++shares)
         for (uint32_t npg : {0u, 1u, 3u, 4u, 31u, 32u, 33u, 500u, 511u, 513u, 65537u, (1u << 26) - 1})
             for (uint32_t part = 0; part < 4 * shares; ++part) {
