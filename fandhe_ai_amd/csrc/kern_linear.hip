@@ -181,7 +181,7 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
         for (int j = 0; j < NTW; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
     v4i bv[kRowPairs][2][NTW];
     auto load = [&](int s, uint32_t it) {            // past the end: the wavefront's last pair again, so that the number under way is the same
-        const uint32_t p = wave + (it < cnt ? it : cnt - 1) * kRowWaves;
+        const uint32_t p = cnt ? wave + (it < cnt ? it : cnt - 1) * kRowWaves : 0;
 #pragma unroll
         for (int j = 0; j < NTW; ++j)
 #pragma unroll
@@ -211,10 +211,10 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
                                                                         acc[i][j], 0, 0, 0);
     };
     static_assert(kRowPairs == 2, "two slots are written out below");
-    if (cnt != 0) {
-        load(0, 0);
-        load(1, 1);
-    }
+    // (wavefronts without a pair load the first one, and nobody reads it: behind a branch nothing could count these loads, and the
+    // norm would wait for them instead of for its rows)
+    load(0, 0);
+    load(1, 1);
     if constexpr (NORM != 0) {
         __builtin_amdgcn_sched_barrier(0);
         norm_rows_store(nm, m, k_tiles * 32, ra, (float *)(normed + kNormRows * normed_pitch(k_tiles * 32)), normed);
@@ -240,6 +240,7 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
         loads_wait<0>();
         if (it + 1 < cnt) mul(std::integral_constant<int, 1>{}, it + 1);
     }
+    loads_wait<0>();                                 // (no load into LDS is under way any more)
     v4f(*red)[NT][64] = (v4f(*)[NT][64])lds;
     if constexpr (NORM == 0) __syncthreads();        // nobody reads staged rows any more
 #pragma unroll

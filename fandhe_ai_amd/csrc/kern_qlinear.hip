@@ -57,14 +57,13 @@ enum { kEpiPlain = 0, kEpiSwiglu = 1, kEpiRope = 2 };
 // a + head_dim/32 of one head, i.e. the two halves that the rotation pairs, rotates q and k heads by the
 // row's position (products rounded separately, no contraction), rounds once to bf16 and stores q rows
 // and the new K / V cache rows directly, so the f32 projection never reaches memory.
-// PRO != 0 (at most four rows, eight wavefronts): the block makes its own activation codes from `pro` behind its first
-// weight loads (row_prologue.hpp: 1 RMSNorm + quantizer, 2 quantizer from partial maxima) and reads the activation
-// operand from LDS; xq_tiled is not read.
+// PRO (Prologue; at most four rows, eight wavefronts): the block makes its own activation codes from `pro` behind its first
+// weight loads (row_prologue.hpp) and reads the activation operand from LDS; xq_tiled is not read.
 template <int MT, int NTW, int NWAVES, int MODE, int PRO = 0>
 __global__ void __launch_bounds__(NWAVES * 64)
     w8a8_skinny_kernel(const int8_t *__restrict__ xq_tiled, const int8_t *__restrict__ w_tiles, uint32_t m,
                        uint32_t n, uint32_t n_tiles, uint32_t k_tiles, EpiI8 ep, RowPrologue pro) {
-    constexpr bool SWIGLU = MODE == kEpiSwiglu, ROPE = MODE == kEpiRope;
+    constexpr bool SWIGLU = MODE == kEpiSwiglu, ROPE = MODE == kEpiRope, NORMS = prologue_norms(PRO);
     static_assert(MODE == kEpiPlain || NTW == 2, "the fused epilogues pair two tiles");
     static_assert(PRO == 0 || (MT == 1 && NWAVES * 64 == kPrologueThreads), "row prologues: one row tile, 512 threads");
     constexpr int NACC = MT * NTW * 4;
@@ -179,16 +178,15 @@ __global__ void __launch_bounds__(NWAVES * 64)
     };
     if constexpr (PRO != 0) {
         // the rows are requested first, the first weight tiles behind them: the row work runs while the tiles travel
-        typename std::conditional<PRO == 1, NormRows, PmaxRows>::type rows;
-        if constexpr (PRO == 1) prologue_norm_load(pro, m, k_tiles * 64, rows);
+        typename std::conditional<NORMS, NormRows<prologue_rows(PRO)>, PmaxRows<prologue_rows(PRO), prologue_vecs(PRO)>>::type rows;
+        if constexpr (NORMS) prologue_norm_load(pro, m, k_tiles * 64, rows);
         else prologue_pmax_load(pro, m, k_tiles * 64, rows);
         __builtin_amdgcn_sched_barrier(0);
-        if (cnt != 0) {
+        // (cnt >= 1: prologues are for at least as many k tiles as wavefronts)
 #pragma unroll
-            for (int s = 0; s < D; ++s) load_b(s, (uint32_t)s);
-        }
+        for (int s = 0; s < D; ++s) load_b(s, (uint32_t)s);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (PRO == 1) prologue_rmsnorm_quantize(pro, rows, m, k_tiles * 64, pro_codes, pro_sx, pro_d, pro_f);
+        if constexpr (NORMS) prologue_rmsnorm_quantize(pro, rows, m, k_tiles * 64, pro_codes, pro_sx, pro_d, pro_f);
         else prologue_quantize_from_pmax(pro, rows, m, k_tiles * 64, pro_codes, pro_sx, pro_f);
         prologue_publish(pro, m, k_tiles * 64, pro_codes, pro_sx);
 #pragma unroll
@@ -197,12 +195,10 @@ __global__ void __launch_bounds__(NWAVES * 64)
             const uint32_t row = (uint32_t)(4 * (lane / 16) + idx % 4);      // one row tile: element idx % 4 of the lane
             p_sx[q] = row < m ? pro_sx[row] : 0.0f;
         }
-        if (cnt != 0) {
 #pragma unroll
-            for (int s = 0; s < D; ++s) load_a(s, (uint32_t)s);
-        }
+        for (int s = 0; s < D; ++s) load_a(s, (uint32_t)s);
     }
-    if (cnt != 0) {
+    if (PRO != 0 || cnt != 0) {
         if constexpr (PRO == 0) {
 #pragma unroll
             for (int s = 0; s < D; ++s) load_slot(s, (uint32_t)s);
@@ -564,7 +560,7 @@ __global__ void __launch_bounds__(512)
 // meet in LDS (two buffers, one barrier per unit) and wavefront w finishes the rows
 // 4 (l / 16) + w % 4 of row tile w / 4 for both tiles of the unit, so SwiGLU has
 // gate and up of an element in the same lane.
-// PRO == 1 (at most four rows): the block makes its own activation codes (RMSNorm + quantizer of `pro`, see
+// PRO (a norm's form, at most four rows): the block makes its own activation codes (RMSNorm + quantizer of `pro`, see
 // row_prologue.hpp) behind the weight loads of its first unit and takes its activation registers from LDS.
 template <int MT, int KTW, int MODE, int PRO = 0>
 __global__ void __launch_bounds__(512)
@@ -572,7 +568,7 @@ __global__ void __launch_bounds__(512)
                       uint32_t n_tiles, uint32_t k_tiles, uint32_t n_units, EpiI8 ep, RowPrologue pro) {
     constexpr bool SWIGLU = MODE == kEpiSwiglu;
     constexpr int NW = 8, NACC = MT * 2 * 4;
-    static_assert(PRO == 0 || (PRO == 1 && MT == 1), "row prologue: norm + quantizer, one row tile");
+    static_assert(PRO == 0 || (prologue_norms(PRO) && MT == 1), "row prologue: norm + quantizer, one row tile");
     __shared__ int red[2][NW][NACC][64];
     extern __shared__ __attribute__((aligned(16))) int8_t pro_codes[];      // PRO: [m][k] activation codes
     __shared__ float pro_sx[PRO ? kPrologueMaxRows : 1], pro_f[PRO ? 16 : 1];
@@ -703,7 +699,7 @@ __global__ void __launch_bounds__(512)
     v4i b0[KTW][2], b1[KTW][2];
     UnitEpi ue0, ue1;
     uint32_t u = blockIdx.x;
-    NormRows rows;
+    [[maybe_unused]] NormRows<prologue_rows(PRO)> rows;
     if constexpr (PRO != 0) {
         // the rows are requested first, the first unit's weights behind them: the row work runs while they travel
         prologue_norm_load(pro, m, k_tiles * 64, rows);
@@ -1960,10 +1956,17 @@ WeightPrefetch prefetch_for_linear_w8a8_qkv_rope_skinny(const int8_t *w_tiles, u
 namespace {
 // bytes of LDS a block needs for its own activation codes
 inline size_t prologue_lds_bytes(uint64_t m, uint64_t k_pad) { return (size_t)((m * k_pad + 15) / 16 * 16); }
+template <typename F>
+void with_norm_rows(uint64_t m, F &&go) {
+    if (m == 1) go(std::integral_constant<int, kNorm1>{});
+    else if (m == 2) go(std::integral_constant<int, kNorm2>{});
+    else go(std::integral_constant<int, kNorm4>{});
+}
 inline bool norm_prologue_shape(uint64_t m, uint64_t k_pad) {
     // the stand-alone kernel whose f64 association the prologue reproduces is the 1024-thread, one-group-per-thread form
-    // by measurement one or two rows (whole steps of 1 / 2 / 3 / 4 rows through 32 layers, contexts 100-200: 2.10 / 2.22 / 2.35 /
-    // 2.47 ms with the row work in here against 2.30 / 2.34 / 2.29 / 2.30 ms with the row kernels); the kernels take four
+    // by measurement one or two rows (whole steps of 1 / 2 / 3 / 4 rows of 400 tokens through 8 layers of width 4096, us: 505 / 567 /
+    // 598 / 624 with the row work in here against 592 / 608 / 605 / 607 with the row kernels, of width 2048 378 / 404 / 416 from two rows
+    // on against 402 / 405 / 410); the kernels take four
     const uint64_t rows = g_row_fusion == 2 ? 4 : 2;
     return g_row_fusion != 1 && m >= 1 && m <= rows && k_pad > 1024 && k_pad <= 4096 && k_pad % 64 == 0;
 }
@@ -1974,9 +1977,8 @@ bool swiglu_fuses_norm(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus) 
     return norm_prologue_shape(m, k_pad) && astat_applies(n_pad / 32, k_pad / 64, num_cus);
 }
 bool plain_fuses_pmax_quantizer(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus) {
-    // by measurement one row (two rows: 2.22 ms a step without, 2.34 ms with); the kernel takes two
-    const uint64_t rows = g_row_fusion == 2 ? 2 : 1;
-    if (g_row_fusion == 1 || m == 0 || m > rows || k_pad % 64 != 0 || k_pad > 16384) return false;     // PmaxRows
+    // the kernel takes two rows (a step of two, norms fused: 567 us with the quantizers in here, 582 without; width 2048 378 and 390)
+    if (g_row_fusion == 1 || m == 0 || m > 2 || k_pad % 64 != 0 || k_pad > 16384 || k_pad < 512) return false;     // PmaxRows, a k tile per wavefront
     if (k_pad / 16 > 1024) return false;                     // partial maxima per row the prologue reads
     const uint64_t n_tiles = n_pad / 16, k_tiles = k_pad / 64;
     if (astat_applies((n_tiles + 1) / 2, k_tiles, num_cus)) return false;
@@ -1998,8 +2000,13 @@ void linear_w8a8_skinny(const int8_t *xq_tiled, const int8_t *w_tiles, uint64_t 
         e.acc_out = ep.acc_out;
         e.out = ep.out;
         e.out_bf16 = ep.out_bf16;
-        w8a8_skinny_kernel<1, 1, 8, kEpiPlain, 2><<<n_tiles, 512, prologue_lds_bytes(m, k_pad), s>>>(
-            nullptr, w_tiles, (uint32_t)m, (uint32_t)n, n_tiles, k_tiles, e, *pro);
+        auto go = [&](auto form) {
+            w8a8_skinny_kernel<1, 1, 8, kEpiPlain, decltype(form)::value><<<n_tiles, 512, prologue_lds_bytes(m, k_pad), s>>>(
+                nullptr, w_tiles, (uint32_t)m, (uint32_t)n, n_tiles, k_tiles, e, *pro);
+        };
+        if (m == 2) go(std::integral_constant<int, kPmaxWide2>{});
+        else if (k_pad <= 4096) go(std::integral_constant<int, kPmaxNarrow>{});
+        else go(std::integral_constant<int, kPmaxWide>{});
         return;
     }
     EpiI8 e{};
@@ -2207,8 +2214,10 @@ void linear_w8a8_swiglu_skinny(const int8_t *xq_tiled, const int8_t *w_tiles, co
     e.pmax = pmax;
     if (pro) {                                              // the caller asked swiglu_fuses_norm first
         unsigned blocks = (unsigned)std::min<uint64_t>(n_tiles / 2, (uint64_t)num_cus);
-        w8a8_astat_kernel<1, 8, kEpiSwiglu, 1><<<blocks, 512, prologue_lds_bytes(m, k_pad), s>>>(
-            nullptr, w_tiles, (uint32_t)m, (uint32_t)n, n_tiles, k_tiles, n_tiles / 2, e, *pro);
+        with_norm_rows(m, [&](auto form) {
+            w8a8_astat_kernel<1, 8, kEpiSwiglu, decltype(form)::value><<<blocks, 512, prologue_lds_bytes(m, k_pad), s>>>(
+                nullptr, w_tiles, (uint32_t)m, (uint32_t)n, n_tiles, k_tiles, n_tiles / 2, e, *pro);
+        });
         return;
     }
     if (m <= 32 && astat_applies(n_tiles / 2, k_tiles, num_cus)) {
@@ -2247,8 +2256,10 @@ void linear_w8a8_qkv_rope_skinny(const int8_t *xq_tiled, const int8_t *w_tiles, 
     e.pool_rows = t.pool_rows;
     unsigned grid = n / 32;                                  // one block per pair of 16-column tiles
     if (pro) {                                               // the caller asked qkv_rope_fuses_norm first
-        w8a8_skinny_kernel<1, 2, 8, kEpiRope, 1><<<grid, 512, prologue_lds_bytes(m, k_pad), s>>>(nullptr, w_tiles, (uint32_t)m, n, n_tiles,
-                                                                                              k_tiles, e, *pro);
+        with_norm_rows(m, [&](auto form) {
+            w8a8_skinny_kernel<1, 2, 8, kEpiRope, decltype(form)::value><<<grid, 512, prologue_lds_bytes(m, k_pad), s>>>(nullptr, w_tiles, (uint32_t)m, n,
+                                                                                                                      n_tiles, k_tiles, e, *pro);
+        });
         return;
     }
     int waves = g_skinny_waves ? g_skinny_waves : 8;

@@ -19,6 +19,15 @@ constexpr int kPrologueMaxRows = 4;
 
 using fa::k::RowPrologue;     // declared with the launchers (kernels.hpp)
 
+// The forms a linear is built in: how many rows, and of what width.  All loads are unconditional (rows and groups past the end repeat
+// the last one) and the weights' behind them too, so that the compiler can count what is under way and the row work waits for its
+// rows only.  (With loads behind branches it waited for the weights first: a step of one sequence of 700 tokens through eight layers of
+// width 4096 546 us, so 506.)
+enum Prologue { kNoPrologue = 0, kNorm1, kNorm2, kNorm4, kPmaxNarrow, kPmaxWide, kPmaxWide2 };
+constexpr bool prologue_norms(int p) { return p >= kNorm1 && p <= kNorm4; }
+constexpr int prologue_rows(int p) { return p == kNorm2 || p == kPmaxWide2 ? 2 : p == kNorm4 ? 4 : 1; }
+constexpr int prologue_vecs(int p) { return p == kPmaxNarrow ? 2 : 8; }      // pmax: four-element groups per thread and row
+
 // RMSNorm + per-token quantizer of rows 0 .. m - 1 (m <= 4, 1024 < k <= 4096, k a multiple of 64) by a block of 512
 // threads.  Thread t stands for threads t and t + 512 of the 1024-thread stand-alone kernel: it owns the
 // four-element groups t and t + 512, reduces each inside its own "virtual" wavefront (t / 64 and 8 + t / 64) with the
@@ -27,28 +36,33 @@ using fa::k::RowPrologue;     // declared with the launchers (kernels.hpp)
 // The rows and the norm weights as the thread's registers.  Issued before the block's first weight loads: loads return
 // in the order they were issued, so the row work can start while the weight tiles are still on their way (asked for
 // after them, it would wait for all of them first).
+template <int ROWS>
 struct NormRows {
-    v4f xv[kPrologueMaxRows][2], wv[2];
+    v4f xv[ROWS][2], wv[2];
 };
-__device__ __forceinline__ void prologue_norm_load(const RowPrologue &p, uint32_t m, uint32_t k, NormRows &t) {
+template <int ROWS>
+__device__ __forceinline__ void prologue_norm_load(const RowPrologue &p, uint32_t m, uint32_t k, NormRows<ROWS> &t) {
     const uint32_t tid = threadIdx.x, n_vec = k / 4;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        const uint32_t j = tid + h * kPrologueThreads;
-        t.wv[h] = j < n_vec ? *(const v4f *)(p.norm_w + j * 4) : v4f{0.f, 0.f, 0.f, 0.f};
+        const uint32_t at = tid + h * kPrologueThreads, j = at < n_vec ? at : n_vec - 1;
+        t.wv[h] = *(const v4f *)(p.norm_w + j * 4);
 #pragma unroll
-        for (int r = 0; r < kPrologueMaxRows; ++r)
-            t.xv[r][h] = ((uint32_t)r < m && j < n_vec) ? *(const v4f *)(p.x + (uint64_t)r * k + j * 4) : v4f{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < ROWS; ++r) t.xv[r][h] = *(const v4f *)(p.x + (uint64_t)((uint32_t)r < m ? r : 0) * k + j * 4);
     }
 }
-__device__ __forceinline__ void prologue_rmsnorm_quantize(const RowPrologue &p, NormRows &t, uint32_t m, uint32_t k, int8_t *codes,
+template <int ROWS>
+__device__ __forceinline__ void prologue_rmsnorm_quantize(const RowPrologue &p, NormRows<ROWS> &t, uint32_t m, uint32_t k, int8_t *codes,
                                                           float *sx, double *smem_d, float *smem_f) {
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, n_vec = k / 4;
-    v4f (&xv)[kPrologueMaxRows][2] = t.xv;
+    v4f (&xv)[ROWS][2] = t.xv;
     v4f (&wv)[2] = t.wv;
 #pragma unroll
-    for (int r = 0; r < kPrologueMaxRows; ++r) {
-        if ((uint32_t)r >= m) break;                    // uniform
+    for (int r = 0; r < ROWS; ++r) {
+        if (ROWS > 1 && (uint32_t)r >= m) break;        // uniform
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            if (tid + h * kPrologueThreads >= n_vec) xv[r][h] = v4f{0.f, 0.f, 0.f, 0.f};
         double part[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -105,33 +119,36 @@ __device__ __forceinline__ void prologue_rmsnorm_quantize(const RowPrologue &p, 
 // Per-token quantizer of rows whose absolute maximum is known as `parts` partial maxima (quantize_from_pmax_kernel):
 // at most two rows of at most 16384 elements (eight four-element groups per thread and row), any k that is a multiple
 // of 64, at most 1024 partial maxima per row.  The maximum is exact in any order.  Loads first, as above.
-constexpr int kPmaxRows = 2, kPmaxVecs = 8;
+template <int ROWS, int VECS>
 struct PmaxRows {
-    v4f xv[kPmaxRows][kPmaxVecs];
-    float pm[kPmaxRows][2];
+    v4f xv[ROWS][VECS];
+    float pm[ROWS][2];
 };
-__device__ __forceinline__ void prologue_pmax_load(const RowPrologue &p, uint32_t m, uint32_t k, PmaxRows &t) {
+template <int ROWS, int VECS>
+__device__ __forceinline__ void prologue_pmax_load(const RowPrologue &p, uint32_t m, uint32_t k, PmaxRows<ROWS, VECS> &t) {
     const uint32_t tid = threadIdx.x, n_vec = k / 4;
 #pragma unroll
-    for (int r = 0; r < kPmaxRows; ++r) {
+    for (int r = 0; r < ROWS; ++r) {
+        const uint64_t row = (uint32_t)r < m ? r : 0;
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < 2; ++u) {                   // (a maximum seen twice changes nothing)
             const uint32_t i = tid + u * kPrologueThreads;
-            t.pm[r][u] = ((uint32_t)r < m && i < p.parts) ? p.pmax[(uint64_t)r * p.parts + i] : 0.0f;
+            t.pm[r][u] = p.pmax[row * p.parts + (i < p.parts ? i : p.parts - 1)];
         }
 #pragma unroll
-        for (int u = 0; u < kPmaxVecs; ++u) {
+        for (int u = 0; u < VECS; ++u) {
             const uint32_t j = tid + u * kPrologueThreads;
-            t.xv[r][u] = ((uint32_t)r < m && j < n_vec) ? *(const v4f *)(p.x + (uint64_t)r * k + j * 4) : v4f{0.f, 0.f, 0.f, 0.f};
+            t.xv[r][u] = *(const v4f *)(p.x + row * k + (j < n_vec ? j : n_vec - 1) * 4);
         }
     }
 }
-__device__ __forceinline__ void prologue_quantize_from_pmax(const RowPrologue &p, PmaxRows &t, uint32_t m, uint32_t k, int8_t *codes,
+template <int ROWS, int VECS>
+__device__ __forceinline__ void prologue_quantize_from_pmax(const RowPrologue &p, PmaxRows<ROWS, VECS> &t, uint32_t m, uint32_t k, int8_t *codes,
                                                             float *sx, float *smem_f) {
     const uint32_t tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, n_vec = k / 4;
 #pragma unroll
-    for (int r = 0; r < kPmaxRows; ++r) {
-        if ((uint32_t)r >= m) break;                    // uniform
+    for (int r = 0; r < ROWS; ++r) {
+        if (ROWS > 1 && (uint32_t)r >= m) break;        // uniform
         float amax = wave_max_dpp(fmaxf(t.pm[r][0], t.pm[r][1]));
         if (lane == 0) smem_f[wave] = amax;
         __syncthreads();
@@ -141,7 +158,7 @@ __device__ __forceinline__ void prologue_quantize_from_pmax(const RowPrologue &p
         const float scale = __fdiv_rn(amax, 127.0f);
         if (tid == 0) sx[r] = scale;
 #pragma unroll
-        for (int u = 0; u < kPmaxVecs; u += 2) {
+        for (int u = 0; u < VECS; u += 2) {
             if ((uint32_t)u * kPrologueThreads >= n_vec) break;      // uniform
             const v4f pair[2] = {t.xv[r][u], t.xv[r][u + 1]};
             uint32_t words[2];
