@@ -335,12 +335,11 @@ __device__ __forceinline__ uint32_t this_xcc() {
 }
 template <int S>
 __device__ __forceinline__ void meet_check_xcd(const uint32_t *xcc_seen, uint32_t group, uint32_t *fault) {
-    if (threadIdx.x != 0 || !xcc_seen) return;
-    const uint32_t mine = this_xcc();
-    bool same = true;
-#pragma unroll
-    for (int r = 0; r < S; ++r) same = same && meet_load<true>(xcc_seen + (uint64_t)group * S + r) == mine + 1u;
-    if (!same) __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    // a lane per member, and not on the first wavefront, whose other work is the longest (one member behind the other: 1 us)
+    if (!xcc_seen || threadIdx.x / 64 != blockDim.x / 64 - 1) return;
+    const uint32_t lane = threadIdx.x % 64, mine = this_xcc() + 1u;
+    const uint32_t seen = lane < (uint32_t)S ? meet_load<true>(xcc_seen + (uint64_t)group * S + lane) : mine;
+    if (__ballot(seen != mine) != 0 && lane == 0) __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace dev

@@ -1223,16 +1223,15 @@ __global__ void __launch_bounds__(512)
     float p_sx[NE], p_sw[NE], p_bias[NE], p_res[NE];
 #pragma unroll
     for (int q = 0; q < NE; ++q) {
-        p_sx[q] = p_sw[q] = p_bias[q] = p_res[q] = 0.0f;
         const int idx = wave + q * NW;
         const int e = idx % 4, j = (idx / 4) % S, i = idx / (4 * S);
-        const uint32_t row = i * 16 + 4 * (lane / 16) + e, col = (nt0 + j) * 16 + lane % 16;
-        if (row < m && col < n) {
-            p_sx[q] = ep.sx[row];
-            p_sw[q] = ep.sw[col];
-            if (ep.bias) p_bias[q] = ep.bias[col];
-            if (ep.residual) p_res[q] = ep.residual[(uint64_t)row * n + col];
-        }
+        const uint32_t row0 = i * 16 + 4 * (lane / 16) + e, col0 = (nt0 + j) * 16 + lane % 16;
+        // without branches (what is not there is not used): behind them the compiler waits here for what it loaded
+        const uint32_t row = row0 < m ? row0 : m - 1, col = col0 < n ? col0 : n - 1;
+        p_sx[q] = ep.sx[row];
+        p_sw[q] = ep.sw[col];
+        p_bias[q] = (ep.bias ? ep.bias : ep.sw)[col];
+        p_res[q] = ep.residual ? ep.residual[(uint64_t)row * n + col] : 0.0f;
     }
     __builtin_amdgcn_sched_barrier(0);
 
