@@ -88,9 +88,13 @@ __global__ void __launch_bounds__(kArgmaxThreads)
         s_idx[threadIdx.x / 64] = best_i;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < kArgmaxThreads / 64; ++w) argmax_take(best, best_i, s_val[w], s_idx[w]);
-        out[blockIdx.x] = best_i == 0xffffffffu ? 0 : (int32_t)best_i;
+    if (threadIdx.x < 64) {                          // the wavefronts' results in the lanes of the first one
+        constexpr int NW = kArgmaxThreads / 64;
+        best = s_val[threadIdx.x % NW];
+        best_i = s_idx[threadIdx.x % NW];
+#pragma unroll
+        for (int off = NW / 2; off > 0; off >>= 1) argmax_take(best, best_i, __shfl_xor(best, off), (uint32_t)__shfl_xor((int)best_i, off));
+        if (threadIdx.x == 0) out[blockIdx.x] = best_i == 0xffffffffu ? 0 : (int32_t)best_i;
     }
 }
 

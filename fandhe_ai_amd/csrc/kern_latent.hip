@@ -32,6 +32,57 @@ __global__ void __launch_bounds__(256)
         for (uint32_t i = threadIdx.x; i < n; i += 256) acc = fmaf(v[i], v[i], acc);
         return 1.0f / sqrtf(block_sum<float, 4, true>(acc, smem) / (float)n + sh.eps);
     };
+    // Ranks of a few values per thread: all of the row is requested at once, without branches (past the end: the last value), and both
+    // norms meet in one go: 3.2 us instead of 5.3 for four rows of 768, 512 and 64.
+    constexpr uint32_t NQ = 6, NC = 2;
+    if (pool && sh.q_rank <= NQ * 256 && sh.kv_rank <= NC * 256 && sh.rot >= 2 && sh.rot <= 512) {
+        const uint32_t tid = threadIdx.x, half = sh.rot / 2, pair = tid < half ? tid : half - 1;
+        const float *c = row + sh.q_rank, *kr = c + sh.kv_rank, *cs = cos_sin + (uint64_t)r * sh.rot;
+        float vq[NQ], wq[NQ], vc[NC], wc[NC], sq = 0.0f, sc = 0.0f;
+#pragma unroll
+        for (uint32_t i = 0; i < NQ; ++i) {
+            const uint32_t at = tid + i * 256 < sh.q_rank ? tid + i * 256 : sh.q_rank - 1;
+            vq[i] = row[at];
+            wq[i] = q_norm[at];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < NC; ++i) {
+            const uint32_t at = tid + i * 256 < sh.kv_rank ? tid + i * 256 : sh.kv_rank - 1;
+            vc[i] = c[at];
+            wc[i] = kv_norm[at];
+        }
+        const uint2 at = rotation_pair(pair, half, sh.interleaved);
+        const float u = kr[at.x], v = kr[at.y], co = cs[pair], si = cs[half + pair];
+        const uint64_t slot = kv_slot[r];
+#pragma unroll
+        for (uint32_t i = 0; i < NQ; ++i) sq = tid + i * 256 < sh.q_rank ? fmaf(vq[i], vq[i], sq) : sq;
+#pragma unroll
+        for (uint32_t i = 0; i < NC; ++i) sc = tid + i * 256 < sh.kv_rank ? fmaf(vc[i], vc[i], sc) : sc;
+        __shared__ float both[2][4];
+        sq = wave_sum_dpp(sq);
+        sc = wave_sum_dpp(sc);
+        if (tid % 64 == 0) {
+            both[0][tid / 64] = sq;
+            both[1][tid / 64] = sc;
+        }
+        __syncthreads();
+        const float rq = 1.0f / sqrtf(((both[0][0] + both[0][1]) + (both[0][2] + both[0][3])) / (float)sh.q_rank + sh.eps);
+        const float rc = 1.0f / sqrtf(((both[1][0] + both[1][1]) + (both[1][2] + both[1][3])) / (float)sh.kv_rank + sh.eps);
+#pragma unroll
+        for (uint32_t i = 0; i < NQ; ++i)
+            if (tid + i * 256 < ld_cq) store_from_f32(cq + (uint64_t)r * ld_cq + tid + i * 256, tid + i * 256 < sh.q_rank ? vq[i] * rq * wq[i] : 0.0f);
+        for (uint32_t i = tid + NQ * 256; i < ld_cq; i += 256) store_from_f32(cq + (uint64_t)r * ld_cq + i, 0.0f);
+        if (slot >= sh.pool_rows) return;
+        T *dst = pool + slot * (sh.rank_p + sh.rot_p);
+#pragma unroll
+        for (uint32_t i = 0; i < NC; ++i)
+            if (tid + i * 256 < sh.kv_rank) store_from_f32(dst + tid + i * 256, vc[i] * rc * wc[i]);
+        if (tid < half) {
+            store_from_f32(dst + sh.rank_p + at.x, u * co - v * si);
+            store_from_f32(dst + sh.rank_p + at.y, v * co + u * si);
+        }
+        return;
+    }
     const float rq = rms(row, sh.q_rank);
     for (uint32_t i = threadIdx.x; i < ld_cq; i += 256)
         store_from_f32(cq + (uint64_t)r * ld_cq + i, i < sh.q_rank ? row[i] * rq * q_norm[i] : 0.0f);
