@@ -890,7 +890,10 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
             for (int j = 0; j < WNT; ++j) ahead[j] = *(const v4f *)(src + j * 16);
         };
-        if constexpr (has_residual) request(0);
+        // (with eight wavefronts only: the other counts have no registers left, spill 468 bytes a lane instead of 340, and 256 columns
+        // on four wavefronts, which hold every register the unit has, came out wrong in one accumulator's last column)
+        constexpr bool request_ahead = has_residual && WM == 4;
+        if constexpr (request_ahead) request(0);
 #pragma unroll
         for (int i = 0; i < AI; ++i) {
             const uint32_t row = m0 + row_l0 + i * 16;
@@ -899,13 +902,14 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
             const uint64_t o0 = (uint64_t)(row_ok ? row : m - 1) * n + nt0 * 16 + col_l0;
             uint8_t *orow = (uint8_t *)ep.out + o0 * (to_bf16 ? 2 : 4);
             v4f add[WNT];                             // the bias (read for every row: no room for it beside the scales) or the residual
-            if constexpr (has_residual) {
+            if constexpr (request_ahead) {
 #pragma unroll
                 for (int j = 0; j < WNT; ++j) add[j] = ahead[j];
                 if (i + 1 < AI) request(i + 1);
-            } else if constexpr (has_bias) {
+            } else if constexpr (has_bias || has_residual) {
+                const float *src = has_bias ? bias + col0 + 4 * g : residual + o0;
 #pragma unroll
-                for (int j = 0; j < WNT; ++j) add[j] = *(const v4f *)(bias + col0 + 4 * g + j * 16);
+                for (int j = 0; j < WNT; ++j) add[j] = *(const v4f *)(src + j * 16);
             }
             v2u pk[WNT];                              // bf16 output: the four columns of tile j, packed
 #pragma unroll
