@@ -120,16 +120,68 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
     return fmaxf(fmaxf(lane_value(v, 0), lane_value(v, 16)), fmaxf(lane_value(v, 32), lane_value(v, 48)));
 }
 
-// Block-wide reductions for blocks of NWAVES wavefronts; `smem` needs NWAVES slots.  DPP selects the wavefront
-// step above (a different association of the sum).  FRESH: nobody has read `smem` since the block's last barrier,
+// The same with the result in the last lane only: the rows meet by two more DPP steps (lane 15 of a row to the next, lane 31 to the
+// upper half) instead of eight reads of lanes.  Bit for bit the value above.
+constexpr int kDppRowBroadcast15 = 0x142, kDppRowBroadcast31 = 0x143;
+template <int CTRL, int ROWS, typename T>
+__device__ __forceinline__ T dpp_rows(T v, T other) {               // rows outside the mask take `other`
+    if constexpr (sizeof(T) == 4) {
+        return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, other), __builtin_bit_cast(int, v), CTRL, ROWS, 0xf, false));
+    } else {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v), o = __builtin_bit_cast(uint64_t, other);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)o, (int)(uint32_t)u, CTRL, ROWS, 0xf, false);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(uint32_t)(o >> 32), (int)(uint32_t)(u >> 32), CTRL, ROWS, 0xf, false);
+        return __builtin_bit_cast(T, (uint64_t)hi << 32 | lo);
+    }
+}
+template <typename T>
+__device__ __forceinline__ T wave_sum_last(T v) {
+    v = row16_sum(v);
+    v += dpp_rows<kDppRowBroadcast15, 0xa>(v, (T)0);
+    v += dpp_rows<kDppRowBroadcast31, 0xc>(v, (T)0);
+    return v;
+}
+__device__ __forceinline__ float wave_max_last(float v) {
+    v = row16_max(v);
+    v = fmaxf(v, dpp_rows<kDppRowBroadcast15, 0xa>(v, v));
+    v = fmaxf(v, dpp_rows<kDppRowBroadcast31, 0xc>(v, v));
+    return v;
+}
+// N values (a power of two up to 16) that lie behind each other in LDS, added or compared in every lane: lane l takes value l % N and
+// neighbours meet, pairs, quads, eights.  (Sixteen reads and fifteen dependent steps in every wavefront were 350 of the 1340 clocks of
+// a sum in 64 bits on sixteen wavefronts.)
+template <int N, typename T>
+__device__ __forceinline__ T lanes_sum(const T *smem) {
+    static_assert((N & (N - 1)) == 0 && N <= 16, "");
+    T v = smem[threadIdx.x % N];
+    if (N > 1) v += dpp_move<kDppXor1>(v);
+    if (N > 2) v += dpp_move<kDppXor2>(v);
+    if (N > 4) v += dpp_move<kDppHalfMirror>(v);
+    if (N > 8) v += dpp_move<kDppMirror>(v);
+    return v;
+}
+template <int N>
+__device__ __forceinline__ float lanes_max(const float *smem) {
+    static_assert((N & (N - 1)) == 0 && N <= 16, "");
+    float v = smem[threadIdx.x % N];
+    if (N > 1) v = fmaxf(v, dpp_move<kDppXor1>(v));
+    if (N > 2) v = fmaxf(v, dpp_move<kDppXor2>(v));
+    if (N > 4) v = fmaxf(v, dpp_move<kDppHalfMirror>(v));
+    if (N > 8) v = fmaxf(v, dpp_move<kDppMirror>(v));
+    return v;
+}
+
+// Block-wide reductions for blocks of NWAVES wavefronts; `smem` needs NWAVES slots.  DPP selects the steps
+// above (a different association of the sum).  FRESH: nobody has read `smem` since the block's last barrier,
 // so the barrier that protects earlier readers is left out.
 template <typename T, int NWAVES, bool DPP = false, bool FRESH = false>
 __device__ __forceinline__ T block_sum(T v, T *smem) {
-    v = DPP ? wave_sum_dpp(v) : wave_sum(v);
+    v = DPP ? wave_sum_last(v) : wave_sum(v);
     int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (!FRESH) __syncthreads();
-    if (lane == 0) smem[wave] = v;
+    if (lane == (DPP ? kWave - 1 : 0)) smem[wave] = v;
     __syncthreads();
+    if constexpr (DPP) return lanes_sum<NWAVES>(smem);
     T r = smem[0];
 #pragma unroll
     for (int i = 1; i < NWAVES; ++i) r += smem[i];
@@ -137,11 +189,12 @@ __device__ __forceinline__ T block_sum(T v, T *smem) {
 }
 template <int NWAVES, bool DPP = false, bool FRESH = false>
 __device__ __forceinline__ float block_max(float v, float *smem) {
-    v = DPP ? wave_max_dpp(v) : wave_max(v);
+    v = DPP ? wave_max_last(v) : wave_max(v);
     int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     if (!FRESH) __syncthreads();
-    if (lane == 0) smem[wave] = v;
+    if (lane == (DPP ? kWave - 1 : 0)) smem[wave] = v;
     __syncthreads();
+    if constexpr (DPP) return lanes_max<NWAVES>(smem);
     float r = smem[0];
 #pragma unroll
     for (int i = 1; i < NWAVES; ++i) r = fmaxf(r, smem[i]);

@@ -256,8 +256,9 @@ __global__ void __launch_bounds__(kBlock)
 
 // The same with neighbouring threads on neighbouring groups: for few rows (a decode step: 32 rows on 32 compute units), where
 // the kernel's time is its chain of dependent steps, and for many (wide_form): a block of THREADS threads per row, thread t owning the four-element groups
-// t, t + THREADS, ... (VPT of them), so that at 4096 columns a thread converts, squares, scales and divides four
-// elements instead of sixteen and the row's bytes are requested by sixteen wavefronts at once.  Same arithmetic
+// t, t + THREADS, ... (VPT of them), so that at 4096 columns a thread converts, squares, scales and divides eight
+// elements instead of sixteen and the row's bytes are requested by eight wavefronts at once.  (On sixteen, what every wavefront
+// computes for itself queued four deep on each SIMD: 3240 clocks from the loads' return to the codes, so 2280.)  Same arithmetic
 // per element; the f64 sum of squares is split over more threads (only its order differs, as above).
 template <int THREADS, int VPT, bool ROW>
 __global__ void __launch_bounds__(THREADS)
@@ -265,7 +266,7 @@ __global__ void __launch_bounds__(THREADS)
                                  float *__restrict__ out_f32, int8_t *__restrict__ xq, float *__restrict__ sx, uint64_t m,
                                  uint64_t hidden, uint32_t row_blocks, WeightPrefetch pull) {
     constexpr int NW = THREADS / kWave;
-    __shared__ double smem_d[NW];
+    __shared__ double smem_d[16];
     __shared__ float smem_f[NW];
     if (blockIdx.x >= row_blocks) {                      // appended blocks: weights of the linear that follows
         prefetch_weights(pull, blockIdx.x - row_blocks);
@@ -279,23 +280,46 @@ __global__ void __launch_bounds__(THREADS)
                 *(v4i *)(xq + tiled_chunk_offset(r, c, k_tiles)) = v4i{0, 0, 0, 0};
         return;
     }
+    // unconditional, the row before the weights of the norm (columns past the end repeat the last group): the sum waits for the row only
     const float *row = x + r * hidden;
     v4f xv[VPT], wv[VPT];
+    uint32_t at[VPT];
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-        const uint64_t j = threadIdx.x + (uint64_t)i * THREADS;
-        xv[i] = j < n_vec ? *(const v4f *)(row + j * 4) : v4f{0.f, 0.f, 0.f, 0.f};
-        wv[i] = j < n_vec ? *(const v4f *)(w + j * 4) : v4f{0.f, 0.f, 0.f, 0.f};
+        at[i] = threadIdx.x + i * THREADS < (uint32_t)n_vec ? threadIdx.x + i * THREADS : (uint32_t)n_vec - 1;
+        xv[i] = *(const v4f *)(row + at[i] * 4);
     }
-    double acc = 0.0;
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) wv[i] = *(const v4f *)(w + at[i] * 4);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < VPT; ++i)
+        if (threadIdx.x + i * THREADS >= (uint32_t)n_vec) xv[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    double acc = 0.0;
+    if constexpr (THREADS * VPT == 1024 && VPT == 2) {   // sums of 256 columns that meet as in the linears' own form (row_prologue.hpp)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const double d = (double)xv[i][e];
-            acc = fma(d, d, acc);
+        for (int i = 0; i < VPT; ++i) {
+            double part = 0.0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double d = (double)xv[i][e];
+                part = fma(d, d, part);
+            }
+            part = wave_sum_last(part);
+            if (threadIdx.x % kWave == kWave - 1) smem_d[i * NW + threadIdx.x / kWave] = part;
         }
-    acc = block_sum<double, NW, true, true>(acc, smem_d);
+        __syncthreads();
+        acc = lanes_sum<NW * VPT>(smem_d);
+    } else {
+#pragma unroll
+        for (int i = 0; i < VPT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const double d = (double)xv[i][e];
+                acc = fma(d, d, acc);
+            }
+        acc = block_sum<double, NW, true, true>(acc, smem_d);
+    }
     const float rstd = (float)(1.0 / sqrt(fma(acc, (double)inv_n, (double)eps)));
     float amax = 0.0f;
 #pragma unroll
@@ -506,8 +530,12 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
         for (int e = 0; e < 4; ++e) xv[0][e] = t[e];
     }
-    float amax = 0.0f;
-    for (uint32_t i = threadIdx.x; i < parts; i += kBlock) amax = fmaxf(amax, pmax[r * parts + i]);
+    float amax = 0.0f, pm[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) pm[u] = pmax[r * parts + min(threadIdx.x + u * kBlock, parts - 1)];    // (one seen twice changes nothing)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) amax = fmaxf(amax, pm[u]);
+    for (uint32_t i = threadIdx.x + 4 * kBlock; i < parts; i += kBlock) amax = fmaxf(amax, pmax[r * parts + i]);
     amax = block_max<kWaves, true, true>(amax, smem);
     const float scale = __fdiv_rn(amax, 127.0f);
     if (blockIdx.x == 0 && threadIdx.x == 0) sx[r] = scale;
@@ -614,7 +642,9 @@ void rmsnorm_f32(const float *x, const float *w, float *out, uint64_t rows, uint
 }
 
 // The row kernels that keep a row in registers: threads per row and four-element groups per thread.  Up to one block per compute
-// unit a row's chain is all there is: a thousand threads.  From there on rows queue, and what counts is how many are under way
+// unit a row's chain is all there is: 512 threads, a thousand for rows of more than 4096 (a decode step of 32 rows of 4096 through
+// eight layers, whose 17 norms and 8 meetings of the attention are such kernels, 1417 -> 1402 us with both on 512, of 40 rows of 2048
+// 672 -> 662, of six 404 -> 396).  From there on rows queue, and what counts is how many are under way
 // and that every load is a whole line: 256 threads (RMSNorm and quantizer of 8192 x 4096, us: 128 threads 31.9, 256 29.4, 512
 // 36.2, 1024 66; with sixteen neighbouring elements per thread 39.9; of 2545 x 2048 8.8, 8.6, 10.4, 17.9; 11.4), up to two
 // blocks per unit 512 (300 x 4096: 256 threads 6.3, 512 5.6, 1024 6.2; sixteen neighbours 6.5; all with codes that were divided
@@ -626,7 +656,8 @@ static bool wide_form(uint64_t rows, uint64_t width, F &&go) {
     if (g_rows_wide == 1 || width > 16384) return false;
     const uint64_t cus = compute_units();
     if (rows <= cus && width > 1024) {
-        if (width <= 4096) go(integral_constant<int, 1024>{}, integral_constant<int, 1>{});
+        if (width <= 2048) go(integral_constant<int, 512>{}, integral_constant<int, 1>{});
+        else if (width <= 4096) go(integral_constant<int, 512>{}, integral_constant<int, 2>{});
         else if (width <= 8192) go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
         else go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
     } else if (rows > 2 * cus ? width > 8192 : width > 1024) {

@@ -175,7 +175,7 @@ struct StreamParams {
     uint32_t shares = 1;
     float *one_part = nullptr, *one_part_ml = nullptr;
     uint32_t *one_counters = nullptr;
-    ixm::Divider by_items{}, by_kv_heads{};                 // batch * num_kv_heads, num_kv_heads
+    ixm::Divider by_items{}, by_kv_heads{}, by_group{};     // batch * num_kv_heads, num_kv_heads, group
     uint32_t *xcc_seen = nullptr, *fault = nullptr;         // LOCAL: SplitKArea's
 };
 
@@ -829,25 +829,63 @@ __global__ void __launch_bounds__(kPrefillMergeThreads)
 }
 
 // The merge above for a whole sequence per block, followed by the per-token int8 quantizer of the
-// projection that consumes the attention output: thread (head, 4 dims) merges its partial results,
+// projection that consumes the attention output: thread (head, 8 dims) merges its partial results,
 // rounds once to bf16 (the attention output's type), the block takes the row's absmax, and the row
 // leaves as int8 activation tiles plus its scale.  Rows at or past the batch are written as zeros.
 // QUANT = false: the same merge without the quantizer, the row stored as the operator's output (bf16 or
 // f32) with, when asked, the absmax of every head's slice; used whenever the heads fit one block.
+// One compute unit works on a row, so the kernel is a chain: a load of the lengths, one of the partial results, and what
+// every wavefront computes for itself, which on sixteen wavefronts (four dims a thread) queued four deep.  Every wavefront adds the
+// lengths up by itself, without a meeting; partial results are requested for up to four ranges, or for up to eight.  32 sequences of 1024
+// to 8192 tokens, 32 heads: 8.6 us, so 7.8; 40 of 300 to 3000, 16 heads: 7.0, so 6.8.
+struct MergedDims {
+    v4f o[2];
+    float den;
+};
+template <int N>
+__device__ __forceinline__ MergedDims merge_ranges(const float *ml, const float *po, uint64_t ml_step, uint64_t po_step, uint32_t g_pad, uint32_t r_lo,
+                                                   uint32_t count) {
+    // everything is requested at once and the maximum is taken from registers; ranges past the last repeat it, with weight zero
+    float m[N], l[N];
+    v4f o[N][2];
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) {
+        const uint64_t r = r_lo + (u < count ? u : count - 1);
+        m[u] = ml[r * ml_step];
+        l[u] = ml[r * ml_step + g_pad];
+        o[u][0] = *(const v4f *)(po + r * po_step);
+        o[u][1] = *(const v4f *)(po + r * po_step + 4);
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < N; ++u) mx = (m[u] != m[u] || mx != mx) ? __uint_as_float(0x7fc00000u) : fmaxf(mx, m[u]);   // NaN marks a violation
+    MergedDims t{{v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}}, 0.0f};
+#pragma unroll
+    for (uint32_t u = 0; u < N; ++u) {
+        if (u >= count) break;                            // uniform
+        const float w = expf(m[u] - mx);
+        t.den = __builtin_fmaf(w, l[u], t.den);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t.o[e / 4][e % 4] = __builtin_fmaf(w, o[u][e / 4][e % 4], t.o[e / 4][e % 4]);
+    }
+    return t;
+}
+
+constexpr uint32_t kMergeHeads = 32;                       // heads of the widest row; a block has 16 threads a head, in whole wavefronts
+constexpr uint32_t merge_threads(uint32_t heads) { return (heads * 16 + 63) / 64 * 64; }
 template <bool QUANT>
-__global__ void __launch_bounds__(1024) decode_stream_merge_quantize_kernel(StreamParams p, int8_t *__restrict__ xq_tiled,
+__global__ void __launch_bounds__(kMergeHeads * 16) decode_stream_merge_quantize_kernel(StreamParams p, int8_t *__restrict__ xq_tiled,
                                                                            float *__restrict__ sx, void *__restrict__ out,
                                                                            int out_bf16, float *__restrict__ pmax,
                                                                            uint32_t row_blocks, WeightPrefetch pull) {
-    __shared__ uint32_t s_tot[16], s_pre[16];
-    __shared__ float s_max[16];
+    __shared__ float s_max[8];
     if (blockIdx.x >= row_blocks) {                      // appended blocks: weights of the linear that follows
         prefetch_weights(pull, blockIdx.x - row_blocks);
         return;
     }
     const uint32_t b = blockIdx.x;
-    const uint32_t e_q = p.num_heads * kDh, k_tiles = e_q / 64;
-    const int wave = threadIdx.x / 64, n_waves = blockDim.x / 64;
+    const uint32_t e_q = p.num_heads * kDh, k_tiles = e_q / 64, lane = threadIdx.x % 64;
+    const int wave = threadIdx.x / 64;
     if (b >= p.batch) {
         if constexpr (QUANT)
             for (uint32_t c = threadIdx.x; c < e_q / 16; c += blockDim.x)
@@ -855,136 +893,106 @@ __global__ void __launch_bounds__(1024) decode_stream_merge_quantize_kernel(Stre
         return;
     }
     const uint32_t max_ctx = p.max_blocks_per_seq * kPage;
-    uint32_t tot = 0, pre = 0;
-    for (uint32_t bb = threadIdx.x; bb < p.batch; bb += blockDim.x) {
-        uint32_t v = seq_pages<false>(p, bb, max_ctx);
+    uint32_t tot = 0, pre = 0, npg = 0;
+    for (uint32_t b0 = 0; b0 < p.batch; b0 += 64) {
+        const uint32_t bb = b0 + lane, v = bb < p.batch ? seq_pages<false>(p, bb, max_ctx) : 0;
         tot += v;
         if (bb < b) pre += v;
+        if (b / 64 * 64 == b0) npg = lane_value(v, (int)(b % 64));
     }
-    tot = wave_sum_dpp<uint32_t>(tot);
-    pre = wave_sum_dpp<uint32_t>(pre);
-    if (threadIdx.x % 64 == 0) {
-        s_tot[wave] = tot;
-        s_pre[wave] = pre;
-    }
-    __syncthreads();
-    tot = 0;
-    pre = 0;
-    for (int w = 0; w < n_waves; ++w) {
-        tot += s_tot[w];
-        pre += s_pre[w];
-    }
-    const uint32_t npg = seq_pages<false>(p, b, max_ctx);
+    tot = __builtin_amdgcn_readfirstlane(wave_sum_dpp<uint32_t>(tot));
+    pre = __builtin_amdgcn_readfirstlane(wave_sum_dpp<uint32_t>(pre));
     const uint32_t per = range_pages(p, tot);
     uint32_t r_lo, r_hi;
     ixm::stream_merge_ranges(pre, npg, per, &r_lo, &r_hi);   // empty sequence: no partials
+    r_lo = __builtin_amdgcn_readfirstlane(r_lo);
+    r_hi = __builtin_amdgcn_readfirstlane(r_hi);
 
-    // blockDim.x == num_heads * 32: thread (h, q) owns dims 4 q .. 4 q + 3 of head h
-    const uint32_t h = threadIdx.x / 32, d4 = (threadIdx.x % 32) * 4;
-    const uint32_t kvh = h / p.group, hg = h % p.group;
-    // partial results four at a time, all loads of a batch issued before the first use (the loop is a
-    // chain of L2 round trips otherwise); slots past r_hi repeat the last one with weight zero
+    // thread (h, q) owns dims 8 q .. 8 q + 7 of head h; threads past the last head repeat it and store nothing
+    const bool mine = threadIdx.x / 16 < p.num_heads;
+    const uint32_t h = mine ? threadIdx.x / 16 : p.num_heads - 1, d8 = (threadIdx.x % 16) * 8;
+    const uint32_t kvh = ixm::quotient(h, p.by_group), hg = h - kvh * p.group;
     const float *ml = p.part_ml + ((uint64_t)b * p.num_kv_heads + kvh) * (2 * p.g_pad) + hg;
-    const float *po = p.part_o + (((uint64_t)b * p.num_kv_heads + kvh) * p.g_pad + hg) * kDh + d4;
+    const float *po = p.part_o + (((uint64_t)b * p.num_kv_heads + kvh) * p.g_pad + hg) * kDh + d8;
     const uint64_t ml_step = (uint64_t)p.num_kv_heads * (2 * p.g_pad), po_step = (uint64_t)p.num_kv_heads * p.g_pad * kDh;
-    float mx = -INFINITY;
-    v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
-    float den = 0.0f;
-    constexpr int kOneTrip = 8;
-    const bool one_trip = npg == 0 || r_hi - r_lo < (uint32_t)kOneTrip;
-    if (one_trip) {
-        // up to eight partial results: everything is requested at once and the maximum is taken from registers,
-        // one memory round trip instead of two; the arithmetic and its order are those of the loops below
-        float m[kOneTrip], l[kOneTrip];
-        v4f o[kOneTrip];
+    const uint32_t count = npg == 0 ? 0 : r_hi - r_lo + 1;
+    MergedDims t{{v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}}, 0.0f};
+    if (count == 0) {
+    } else if (count <= 4) {
+        t = merge_ranges<4>(ml, po, ml_step, po_step, p.g_pad, r_lo, count);
+    } else if (count <= 8) {
+        t = merge_ranges<8>(ml, po, ml_step, po_step, p.g_pad, r_lo, count);
+    } else {                                              // the maximum first, then the sums, four ranges at a time: two chains of trips
+        float mx = -INFINITY;
+        for (uint32_t r0 = r_lo; r0 <= r_hi; r0 += 4) {
+            float m[4];
 #pragma unroll
-        for (int u = 0; u < kOneTrip; ++u) {
-            const uint64_t r = r_lo + u <= r_hi ? r_lo + u : r_hi;
-            m[u] = ml[r * ml_step];
-            l[u] = ml[r * ml_step + p.g_pad];
-            o[u] = *(const v4f *)(po + r * po_step);
+            for (int u = 0; u < 4; ++u) m[u] = ml[(uint64_t)(r0 + u <= r_hi ? r0 + u : r_hi) * ml_step];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) mx = (m[u] != m[u] || mx != mx) ? __uint_as_float(0x7fc00000u) : fmaxf(mx, m[u]);
         }
+        for (uint32_t r0 = r_lo; r0 <= r_hi; r0 += 4) {
+            float m[4], l[4];
+            v4f o[4][2];
 #pragma unroll
-        for (int u = 0; u < kOneTrip; ++u)
-            if (r_lo + u <= r_hi) mx = (m[u] != m[u] || mx != mx) ? __uint_as_float(0x7fc00000u) : fmaxf(mx, m[u]);
+            for (int u = 0; u < 4; ++u) {
+                const uint64_t r = r0 + u <= r_hi ? r0 + u : r_hi;
+                m[u] = ml[r * ml_step];
+                l[u] = ml[r * ml_step + p.g_pad];
+                o[u][0] = *(const v4f *)(po + r * po_step);
+                o[u][1] = *(const v4f *)(po + r * po_step + 4);
+            }
 #pragma unroll
-        for (int u = 0; u < kOneTrip; ++u) {
-            if (r_lo + u <= r_hi) {
-                const float w = expf(m[u] - mx);
-                den = __builtin_fmaf(w, l[u], den);
+            for (int u = 0; u < 4; ++u) {
+                const float w = r0 + u <= r_hi ? expf(m[u] - mx) : 0.0f;
+                t.den = __builtin_fmaf(w, l[u], t.den);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w, o[u][e], acc[e]);
+                for (int e = 0; e < 8; ++e) t.o[e / 4][e % 4] = __builtin_fmaf(w, o[u][e / 4][e % 4], t.o[e / 4][e % 4]);
             }
         }
     }
-    for (uint32_t r0 = r_lo; !one_trip && r0 <= r_hi; r0 += 4) {
-        float m[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) m[u] = ml[(uint64_t)(r0 + u <= r_hi ? r0 + u : r_hi) * ml_step];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            mx = (m[u] != m[u] || mx != mx) ? __uint_as_float(0x7fc00000u) : fmaxf(mx, m[u]);   // NaN marks a violation
-    }
-    for (uint32_t r0 = r_lo; !one_trip && r0 <= r_hi; r0 += 4) {
-        float m[4], l[4];
-        v4f o[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const uint64_t r = r0 + u <= r_hi ? r0 + u : r_hi;
-            m[u] = ml[r * ml_step];
-            l[u] = ml[r * ml_step + p.g_pad];
-            o[u] = *(const v4f *)(po + r * po_step);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            float w = r0 + u <= r_hi ? expf(m[u] - mx) : 0.0f;
-            den = __builtin_fmaf(w, l[u], den);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w, o[u][e], acc[e]);
-        }
-    }
-    float v[4], amax = 0.0f;
+    v4f v[2];
+    float amax = 0.0f;
     if constexpr (!QUANT) {
-        const uint64_t oi = ((uint64_t)b * p.num_heads + h) * kDh + d4;
+        const uint64_t oi = ((uint64_t)b * p.num_heads + h) * kDh + d8;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float res = npg == 0 ? 0.0f : __fdiv_rn(acc[e], den);
+        for (int e = 0; e < 8; ++e) {
+            float res = npg == 0 ? 0.0f : __fdiv_rn(t.o[e / 4][e % 4], t.den);
             if (out_bf16) res = bf16_to_f32(f32_to_bf16(res));
-            v[e] = res;
+            v[e / 4][e % 4] = res;
             amax = fmaxf(amax, fabsf(res));
         }
-        if (out_bf16) {
-            const uint32_t lo = (uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16);
-            const uint32_t hi = (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16);
-            *(v2u *)((uint16_t *)out + oi) = v2u{lo, hi};
-        } else {
-            *(v4f *)((float *)out + oi) = v4f{v[0], v[1], v[2], v[3]};
-        }
-        if (pmax) {                                    // absmax of the stored head slice: the 32 threads of a head
+        if (mine && out_bf16) {
+            uint32_t w[4];
 #pragma unroll
-            for (int off = 1; off < 32; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-            if (threadIdx.x % 32 == 0) pmax[(uint64_t)b * p.num_heads + h] = amax;
+            for (int e = 0; e < 4; ++e) w[e] = (uint32_t)f32_to_bf16(v[e / 2][e % 2 * 2]) | ((uint32_t)f32_to_bf16(v[e / 2][e % 2 * 2 + 1]) << 16);
+            *(v4u *)((uint16_t *)out + oi) = v4u{w[0], w[1], w[2], w[3]};
+        } else if (mine) {
+            *(v4f *)((float *)out + oi) = v[0];
+            *(v4f *)((float *)out + oi + 4) = v[1];
+        }
+        if (pmax) {                                    // absmax of the stored head slice: the 16 threads of a head
+            amax = row16_max(amax);
+            if (mine && threadIdx.x % 16 == 0) pmax[(uint64_t)b * p.num_heads + h] = amax;
         }
         return;
     }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        float res = npg == 0 ? 0.0f : __fdiv_rn(acc[e], den);
-        v[e] = bf16_to_f32(f32_to_bf16(res));         // the attention output is bf16: round once, then quantize
-        amax = fmaxf(amax, fabsf(v[e]));
+    for (int e = 0; e < 8; ++e) {
+        const float res = npg == 0 ? 0.0f : __fdiv_rn(t.o[e / 4][e % 4], t.den);
+        v[e / 4][e % 4] = bf16_to_f32(f32_to_bf16(res));   // the attention output is bf16: round once, then quantize
+        amax = fmaxf(amax, fabsf(v[e / 4][e % 4]));
     }
-    amax = wave_max_dpp(amax);
-    if (threadIdx.x % 64 == 0) s_max[wave] = amax;
+    amax = wave_max_last(amax);
+    if (lane == 63) s_max[wave] = amax;
+    if (threadIdx.x < 8 && threadIdx.x >= blockDim.x / 64) s_max[threadIdx.x] = 0.0f;   // wavefronts a narrower row does not have
     __syncthreads();
-    amax = 0.0f;
-    for (int w = 0; w < n_waves; ++w) amax = fmaxf(amax, s_max[w]);
-    const float scale = __fdiv_rn(amax, 127.0f);
+    const float scale = __fdiv_rn(lanes_max<8>(s_max), 127.0f);
     if (threadIdx.x == 0) sx[b] = scale;
-    uint32_t word = 0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) word |= ((uint32_t)quant_i8(v[e], scale) & 0xffu) << (8 * e);
-    const uint32_t col = h * kDh + d4;
-    *(uint32_t *)(xq_tiled + tiled_chunk_offset(b, col / 16, k_tiles) + col % 16) = word;
+    uint32_t word[2];
+    quant_i8_words(v, scale, word);
+    const uint32_t col = h * kDh + d8;
+    if (mine) *(v2u *)(xq_tiled + tiled_chunk_offset(b, col / 16, k_tiles) + col % 16) = v2u{word[0], word[1]};
 }
 
 // ------------------------------------------------------- prefill, block form
@@ -1492,6 +1500,7 @@ void paged_attention_decode_bf16(const uint16_t *q, const uint16_t *k_pool, cons
     sp.num_kv_heads = ps.num_kv_heads;
     sp.group = ps.num_heads / ps.num_kv_heads;
     sp.g_pad = (uint32_t)group_pad(sp.group);
+    sp.by_group = ixm::divider(sp.group);
     sp.max_blocks_per_seq = ps.max_blocks_per_seq;
     sp.n_ranges = stream_ranges(ps, waves_per_cu);
     sp.min_pages = 4;
@@ -1505,15 +1514,15 @@ void paged_attention_decode_bf16(const uint16_t *q, const uint16_t *k_pool, cons
     uint64_t waves = (uint64_t)sp.n_ranges * ps.num_kv_heads;
     decode_stream_kernel<4, 4, 2, 2, false><<<(unsigned)((waves + 3) / 4), 256, 0, s>>>(sp);
     if (g_decode_partials_only) return;
-    if (xq_tiled != nullptr && ps.num_heads <= 32) {
+    if (xq_tiled != nullptr && ps.num_heads <= kMergeHeads) {
         // fused merge + per-token quantizer (the bf16 output itself is not written)
         const WeightPrefetch pf = (pull.w && m_pad % 8 == 0) ? pull : WeightPrefetch{};
-        decode_stream_merge_quantize_kernel<true><<<m_pad + pf.blocks, ps.num_heads * 32, 0, s>>>(sp, xq_tiled, sx, nullptr, 0, nullptr,
+        decode_stream_merge_quantize_kernel<true><<<m_pad + pf.blocks, merge_threads(ps.num_heads), 0, s>>>(sp, xq_tiled, sx, nullptr, 0, nullptr,
                                                                                                  m_pad, pf);
         return;
     }
-    if (ps.num_heads <= 32 && ps.num_heads % 2 == 0) {    // a row per block (whole wavefronts): one launch of batch blocks
-        decode_stream_merge_quantize_kernel<false><<<ps.batch, ps.num_heads * 32, 0, s>>>(sp, nullptr, nullptr, out, out_bf16, pmax, ps.batch,
+    if (ps.num_heads <= kMergeHeads && ps.num_heads % 2 == 0) {    // a row per block: one launch of batch blocks
+        decode_stream_merge_quantize_kernel<false><<<ps.batch, merge_threads(ps.num_heads), 0, s>>>(sp, nullptr, nullptr, out, out_bf16, pmax, ps.batch,
                                                                                          WeightPrefetch{});
         return;
     }

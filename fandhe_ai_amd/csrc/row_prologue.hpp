@@ -4,7 +4,7 @@
 // block of the linear redoes that row work for itself (4096 elements per row: eight per thread) behind its first
 // weight loads, which are already in flight, and keeps the codes in LDS, where the matrix instruction's activation
 // operand is read from.  The arithmetic, including the association of the f64 sum of squares, is that of the
-// stand-alone kernels (kern_norm_quant.hip: rmsnorm_quantize_wide_kernel<1024, 1>, quantize_from_pmax_kernel), so a
+// stand-alone kernels (kern_norm_quant.hip: rmsnorm_quantize_wide_kernel<512, 2>, quantize_from_pmax_kernel), so a
 // sequence decodes to the same bits alone and in a batch of 32.
 #pragma once
 
@@ -29,9 +29,8 @@ constexpr int prologue_rows(int p) { return p == kNorm2 || p == kPmaxWide2 ? 2 :
 constexpr int prologue_vecs(int p) { return p == kPmaxNarrow ? 2 : 8; }      // pmax: four-element groups per thread and row
 
 // RMSNorm + per-token quantizer of rows 0 .. m - 1 (m <= 4, 1024 < k <= 4096, k a multiple of 64) by a block of 512
-// threads.  Thread t stands for threads t and t + 512 of the 1024-thread stand-alone kernel: it owns the
-// four-element groups t and t + 512, reduces each inside its own "virtual" wavefront (t / 64 and 8 + t / 64) with the
-// same DPP steps, and the sixteen wavefront sums are added in index order, exactly as block_sum does there.
+// threads, as the stand-alone kernel does it: thread t owns the four-element groups t and t + 512, reduces each inside its
+// wavefront by itself (sums t / 64 and 8 + t / 64) with the same DPP steps, and the sixteen sums meet by lanes.
 // codes: LDS, row-major [m][k]; sx: LDS [m]; smem_d / smem_f: 16 slots each.  Ends with a barrier.
 // The rows and the norm weights as the thread's registers.  Issued before the block's first weight loads: loads return
 // in the order they were issued, so the row work can start while the weight tiles are still on their way (asked for
@@ -72,16 +71,14 @@ __device__ __forceinline__ void prologue_rmsnorm_quantize(const RowPrologue &p, 
                 const double d = (double)xv[r][h][e];
                 acc = fma(d, d, acc);
             }
-            part[h] = wave_sum_dpp(acc);
+            part[h] = wave_sum_last(acc);
         }
-        if (lane == 0) {
+        if (lane == kWave - 1) {
             smem_d[wave] = part[0];
             smem_d[8 + wave] = part[1];
         }
         __syncthreads();
-        double total = smem_d[0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) total += smem_d[i];
+        const double total = lanes_sum<16>(smem_d);
         const float rstd = (float)(1.0 / sqrt(fma(total, (double)p.inv_n, (double)p.eps)));
         float am[2];
 #pragma unroll
@@ -93,16 +90,14 @@ __device__ __forceinline__ void prologue_rmsnorm_quantize(const RowPrologue &p, 
                 xv[r][h][e] = y;
                 amax = fmaxf(amax, fabsf(y));
             }
-            am[h] = wave_max_dpp(amax);
+            am[h] = wave_max_last(amax);
         }
-        if (lane == 0) {
+        if (lane == kWave - 1) {
             smem_f[wave] = am[0];
             smem_f[8 + wave] = am[1];
         }
         __syncthreads();                                // also: everybody has read smem_d before the next row writes it
-        float amax = smem_f[0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) amax = fmaxf(amax, smem_f[i]);
+        const float amax = lanes_max<16>(smem_f);
         const float scale = __fdiv_rn(amax, 127.0f);
         if (tid == 0) sx[r] = scale;
         uint32_t words[2];
@@ -149,12 +144,10 @@ __device__ __forceinline__ void prologue_quantize_from_pmax(const RowPrologue &p
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) {
         if (ROWS > 1 && (uint32_t)r >= m) break;        // uniform
-        float amax = wave_max_dpp(fmaxf(t.pm[r][0], t.pm[r][1]));
-        if (lane == 0) smem_f[wave] = amax;
+        float amax = wave_max_last(fmaxf(t.pm[r][0], t.pm[r][1]));
+        if (lane == kWave - 1) smem_f[wave] = amax;
         __syncthreads();
-        amax = smem_f[0];
-#pragma unroll
-        for (int i = 1; i < kPrologueThreads / kWave; ++i) amax = fmaxf(amax, smem_f[i]);
+        amax = lanes_max<kPrologueThreads / kWave>(smem_f);
         const float scale = __fdiv_rn(amax, 127.0f);
         if (tid == 0) sx[r] = scale;
 #pragma unroll

@@ -473,6 +473,33 @@ def test_attention_shares_of_one_launch(ctxs, tune):
     assert np.abs(ca - cb).max() <= 1 and (ca != cb).mean() < 2e-3 and np.any(ca != 0)
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(1, 1), (2, 1), (6, 2), (10, 10), (12, 4), (30, 6), (32, 32)])
+def test_merged_rows(heads, kv_heads):
+    """The merge of a whole row per block: heads that do not fill its wavefronts, more sequences than a wavefront has lanes, and
+    sequences on one range, up to four, up to eight and more (ranges are of four pages here)."""
+    import test_gpu_paged as tp
+    import oracle_lib as o
+    import fandhe_ai_amd as fa
+    from gpu_common import assert_bf16_rounding_of, assert_parity
+    be = ops()
+    rng = o.Rng(7000 + heads * 10 + kv_heads)
+    ctxs = [1 + 5 * i % 60 for i in range(66)] + [257, 500, 129, 1100]
+    batch, num_blocks = len(ctxs), sum(c // 16 + 1 for c in ctxs)
+    tables, lens, max_blocks, e_kv, e_q = tp._decode_case(rng, batch, heads, kv_heads, ctxs, num_blocks)
+    kp, vp = o.to_bf16(rng.randn((num_blocks, 16, e_kv))), o.to_bf16(rng.randn((num_blocks, 16, e_kv)))
+    q = o.to_bf16(rng.randn((batch, 1, e_q)))
+    layout = fa.PagedKvLayout.new(num_blocks, 16, e_kv)
+    args = fa.PagedAttentionArgs(layout, batch, 1, heads, max_blocks, fa.default_scale(128), kv_heads)
+    o.set_threads(8)
+    rc, want = o.paged_attention_bf16(q, kp, vp, tables, lens, o.paged_args(num_blocks, 16, e_kv, batch, 1, heads, max_blocks, args.scale, kv_heads))
+    o.set_threads(1)
+    assert rc == 0
+    dq, dk, dv = be.upload(q), be.upload(kp), be.upload(vp)
+    got = be.download_owned(be.paged_attention_forward(dq, dk, dv, tables, lens, args, out_dtype=fa.capi.F32))
+    assert_parity("PAGED_DECODE_PARITY", f"merged rows H{heads}/{kv_heads}", got, want)
+    assert_bf16_rounding_of("merged rows bf16", be.download_owned(be.paged_attention_forward(dq, dk, dv, tables, lens, args)), got)
+
+
 @pytest.mark.parametrize("rows,k", [(256, 1088), (257, 1024), (257, 2112), (512, 4160), (513, 1024), (513, 2112), (600, 4096), (600, 8256),
                                     (300, 16384), (513, 16384), (300, 16448)])
 @pytest.mark.parametrize("bf16", [False, True])
