@@ -838,46 +838,52 @@ __global__ void __launch_bounds__(kPrefillMergeThreads)
 // every wavefront computes for itself, which on sixteen wavefronts (four dims a thread) queued four deep.  Every wavefront adds the
 // lengths up by itself, without a meeting; partial results are requested for up to four ranges, or for up to eight.  32 sequences of 1024
 // to 8192 tokens, 32 heads: 8.6 us, so 7.8; 40 of 300 to 3000, 16 heads: 7.0, so 6.8.
+template <int V>
 struct MergedDims {
-    v4f o[2];
+    v4f o[V];
     float den;
 };
-template <int N>
-__device__ __forceinline__ MergedDims merge_ranges(const float *ml, const float *po, uint64_t ml_step, uint64_t po_step, uint32_t g_pad, uint32_t r_lo,
-                                                   uint32_t count) {
+template <int N, int V>
+__device__ __forceinline__ MergedDims<V> merge_ranges(const float *ml, const float *po, uint64_t ml_step, uint64_t po_step, uint32_t g_pad, uint32_t r_lo,
+                                                      uint32_t count) {
     // everything is requested at once and the maximum is taken from registers; ranges past the last repeat it, with weight zero
     float m[N], l[N];
-    v4f o[N][2];
+    v4f o[N][V];
 #pragma unroll
     for (uint32_t u = 0; u < N; ++u) {
         const uint64_t r = r_lo + (u < count ? u : count - 1);
         m[u] = ml[r * ml_step];
         l[u] = ml[r * ml_step + g_pad];
         o[u][0] = *(const v4f *)(po + r * po_step);
-        o[u][1] = *(const v4f *)(po + r * po_step + 4);
+        if constexpr (V == 2) o[u][1] = *(const v4f *)(po + r * po_step + 4);
     }
     float mx = -INFINITY;
 #pragma unroll
     for (int u = 0; u < N; ++u) mx = (m[u] != m[u] || mx != mx) ? __uint_as_float(0x7fc00000u) : fmaxf(mx, m[u]);   // NaN marks a violation
-    MergedDims t{{v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}}, 0.0f};
+    MergedDims<V> t{};
 #pragma unroll
     for (uint32_t u = 0; u < N; ++u) {
         if (u >= count) break;                            // uniform
         const float w = expf(m[u] - mx);
         t.den = __builtin_fmaf(w, l[u], t.den);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) t.o[e / 4][e % 4] = __builtin_fmaf(w, o[u][e / 4][e % 4], t.o[e / 4][e % 4]);
+        for (int e = 0; e < 4 * V; ++e) t.o[e / 4][e % 4] = __builtin_fmaf(w, o[u][e / 4][e % 4], t.o[e / 4][e % 4]);
     }
     return t;
 }
 
 constexpr uint32_t kMergeHeads = 32;                       // heads of the widest row; a block has 16 threads a head, in whole wavefronts
 constexpr uint32_t merge_threads(uint32_t heads) { return (heads * 16 + 63) / 64 * 64; }
-template <bool QUANT>
+// V: vectors of four dims a thread.  One, without the quantizer, for rows whose threads are eight wavefronts even so (up to half of
+// kMergeHeads): half the chain to a thread and nothing queued.  16 heads, 29 sequences of 280 to 3525 tokens 6.2 us with two, 5.7 so; 12
+// of 64 to 900 6.5, 6.1; 48 of 200 to 700 4.6, 4.4.
+template <bool QUANT, int V = 2>
 __global__ void __launch_bounds__(kMergeHeads * 16) decode_stream_merge_quantize_kernel(StreamParams p, int8_t *__restrict__ xq_tiled,
                                                                            float *__restrict__ sx, void *__restrict__ out,
                                                                            int out_bf16, float *__restrict__ pmax,
                                                                            uint32_t row_blocks, WeightPrefetch pull) {
+    static_assert(V == 2 || !QUANT, "the quantizer stores eight codes a thread");
+    constexpr uint32_t TH = 32 / V;                      // threads a head
     __shared__ float s_max[8];
     if (blockIdx.x >= row_blocks) {                      // appended blocks: weights of the linear that follows
         prefetch_weights(pull, blockIdx.x - row_blocks);
@@ -908,20 +914,20 @@ __global__ void __launch_bounds__(kMergeHeads * 16) decode_stream_merge_quantize
     r_lo = __builtin_amdgcn_readfirstlane(r_lo);
     r_hi = __builtin_amdgcn_readfirstlane(r_hi);
 
-    // thread (h, q) owns dims 8 q .. 8 q + 7 of head h; threads past the last head repeat it and store nothing
-    const bool mine = threadIdx.x / 16 < p.num_heads;
-    const uint32_t h = mine ? threadIdx.x / 16 : p.num_heads - 1, d8 = (threadIdx.x % 16) * 8;
+    // thread (h, q) owns dims 4 V q .. + 4 V - 1 of head h; threads past the last head repeat it and store nothing
+    const bool mine = threadIdx.x / TH < p.num_heads;
+    const uint32_t h = mine ? threadIdx.x / TH : p.num_heads - 1, d0 = threadIdx.x % TH * (4 * V);
     const uint32_t kvh = ixm::quotient(h, p.by_group), hg = h - kvh * p.group;
     const float *ml = p.part_ml + ((uint64_t)b * p.num_kv_heads + kvh) * (2 * p.g_pad) + hg;
-    const float *po = p.part_o + (((uint64_t)b * p.num_kv_heads + kvh) * p.g_pad + hg) * kDh + d8;
+    const float *po = p.part_o + (((uint64_t)b * p.num_kv_heads + kvh) * p.g_pad + hg) * kDh + d0;
     const uint64_t ml_step = (uint64_t)p.num_kv_heads * (2 * p.g_pad), po_step = (uint64_t)p.num_kv_heads * p.g_pad * kDh;
     const uint32_t count = npg == 0 ? 0 : r_hi - r_lo + 1;
-    MergedDims t{{v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}}, 0.0f};
+    MergedDims<V> t{};
     if (count == 0) {
     } else if (count <= 4) {
-        t = merge_ranges<4>(ml, po, ml_step, po_step, p.g_pad, r_lo, count);
+        t = merge_ranges<4, V>(ml, po, ml_step, po_step, p.g_pad, r_lo, count);
     } else if (count <= 8) {
-        t = merge_ranges<8>(ml, po, ml_step, po_step, p.g_pad, r_lo, count);
+        t = merge_ranges<8, V>(ml, po, ml_step, po_step, p.g_pad, r_lo, count);
     } else {                                              // the maximum first, then the sums, four ranges at a time: two chains of trips
         float mx = -INFINITY;
         for (uint32_t r0 = r_lo; r0 <= r_hi; r0 += 4) {
@@ -933,66 +939,70 @@ __global__ void __launch_bounds__(kMergeHeads * 16) decode_stream_merge_quantize
         }
         for (uint32_t r0 = r_lo; r0 <= r_hi; r0 += 4) {
             float m[4], l[4];
-            v4f o[4][2];
+            v4f o[4][V];
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const uint64_t r = r0 + u <= r_hi ? r0 + u : r_hi;
                 m[u] = ml[r * ml_step];
                 l[u] = ml[r * ml_step + p.g_pad];
                 o[u][0] = *(const v4f *)(po + r * po_step);
-                o[u][1] = *(const v4f *)(po + r * po_step + 4);
+                if constexpr (V == 2) o[u][1] = *(const v4f *)(po + r * po_step + 4);
             }
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const float w = r0 + u <= r_hi ? expf(m[u] - mx) : 0.0f;
                 t.den = __builtin_fmaf(w, l[u], t.den);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) t.o[e / 4][e % 4] = __builtin_fmaf(w, o[u][e / 4][e % 4], t.o[e / 4][e % 4]);
+                for (int e = 0; e < 4 * V; ++e) t.o[e / 4][e % 4] = __builtin_fmaf(w, o[u][e / 4][e % 4], t.o[e / 4][e % 4]);
             }
         }
     }
-    v4f v[2];
+    v4f v[V];
     float amax = 0.0f;
     if constexpr (!QUANT) {
-        const uint64_t oi = ((uint64_t)b * p.num_heads + h) * kDh + d8;
+        const uint64_t oi = ((uint64_t)b * p.num_heads + h) * kDh + d0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < 4 * V; ++e) {
             float res = npg == 0 ? 0.0f : __fdiv_rn(t.o[e / 4][e % 4], t.den);
             if (out_bf16) res = bf16_to_f32(f32_to_bf16(res));
             v[e / 4][e % 4] = res;
             amax = fmaxf(amax, fabsf(res));
         }
         if (mine && out_bf16) {
-            uint32_t w[4];
+            uint32_t w[2 * V];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) w[e] = (uint32_t)f32_to_bf16(v[e / 2][e % 2 * 2]) | ((uint32_t)f32_to_bf16(v[e / 2][e % 2 * 2 + 1]) << 16);
-            *(v4u *)((uint16_t *)out + oi) = v4u{w[0], w[1], w[2], w[3]};
+            for (int e = 0; e < 2 * V; ++e) w[e] = (uint32_t)f32_to_bf16(v[e / 2][e % 2 * 2]) | ((uint32_t)f32_to_bf16(v[e / 2][e % 2 * 2 + 1]) << 16);
+            if constexpr (V == 2) *(v4u *)((uint16_t *)out + oi) = v4u{w[0], w[1], w[2], w[3]};
+            else *(v2u *)((uint16_t *)out + oi) = v2u{w[0], w[1]};
         } else if (mine) {
-            *(v4f *)((float *)out + oi) = v[0];
-            *(v4f *)((float *)out + oi + 4) = v[1];
+#pragma unroll
+            for (int i = 0; i < V; ++i) *(v4f *)((float *)out + oi + 4 * i) = v[i];
         }
-        if (pmax) {                                    // absmax of the stored head slice: the 16 threads of a head
+        if (pmax) {                                    // absmax of the stored head slice: the threads of a head
             amax = row16_max(amax);
-            if (mine && threadIdx.x % 16 == 0) pmax[(uint64_t)b * p.num_heads + h] = amax;
+            if constexpr (V == 1) amax = fmaxf(amax, __shfl_xor(amax, 16));
+            if (mine && threadIdx.x % TH == 0) pmax[(uint64_t)b * p.num_heads + h] = amax;
         }
         return;
     }
+    if constexpr (QUANT) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const float res = npg == 0 ? 0.0f : __fdiv_rn(t.o[e / 4][e % 4], t.den);
-        v[e / 4][e % 4] = bf16_to_f32(f32_to_bf16(res));   // the attention output is bf16: round once, then quantize
-        amax = fmaxf(amax, fabsf(v[e / 4][e % 4]));
+        for (int e = 0; e < 4 * V; ++e) {
+            const float res = npg == 0 ? 0.0f : __fdiv_rn(t.o[e / 4][e % 4], t.den);
+            v[e / 4][e % 4] = bf16_to_f32(f32_to_bf16(res));   // the attention output is bf16: round once, then quantize
+            amax = fmaxf(amax, fabsf(v[e / 4][e % 4]));
+        }
+        amax = wave_max_last(amax);
+        if (lane == 63) s_max[wave] = amax;
+        if (threadIdx.x < 8 && threadIdx.x >= blockDim.x / 64) s_max[threadIdx.x] = 0.0f;   // wavefronts a narrower row does not have
+        __syncthreads();
+        const float scale = __fdiv_rn(lanes_max<8>(s_max), 127.0f);
+        if (threadIdx.x == 0) sx[b] = scale;
+        uint32_t word[2];
+        quant_i8_words(v, scale, word);
+        const uint32_t col = h * kDh + d0;
+        if (mine) *(v2u *)(xq_tiled + tiled_chunk_offset(b, col / 16, k_tiles) + col % 16) = v2u{word[0], word[1]};
     }
-    amax = wave_max_last(amax);
-    if (lane == 63) s_max[wave] = amax;
-    if (threadIdx.x < 8 && threadIdx.x >= blockDim.x / 64) s_max[threadIdx.x] = 0.0f;   // wavefronts a narrower row does not have
-    __syncthreads();
-    const float scale = __fdiv_rn(lanes_max<8>(s_max), 127.0f);
-    if (threadIdx.x == 0) sx[b] = scale;
-    uint32_t word[2];
-    quant_i8_words(v, scale, word);
-    const uint32_t col = h * kDh + d8;
-    if (mine) *(v2u *)(xq_tiled + tiled_chunk_offset(b, col / 16, k_tiles) + col % 16) = v2u{word[0], word[1]};
 }
 
 // ------------------------------------------------------- prefill, block form
@@ -1522,8 +1532,12 @@ void paged_attention_decode_bf16(const uint16_t *q, const uint16_t *k_pool, cons
         return;
     }
     if (ps.num_heads <= kMergeHeads && ps.num_heads % 2 == 0) {    // a row per block: one launch of batch blocks
-        decode_stream_merge_quantize_kernel<false><<<ps.batch, merge_threads(ps.num_heads), 0, s>>>(sp, nullptr, nullptr, out, out_bf16, pmax, ps.batch,
-                                                                                         WeightPrefetch{});
+        if (2 * ps.num_heads <= kMergeHeads)
+            decode_stream_merge_quantize_kernel<false, 1><<<ps.batch, merge_threads(2 * ps.num_heads), 0, s>>>(sp, nullptr, nullptr, out, out_bf16, pmax,
+                                                                                                               ps.batch, WeightPrefetch{});
+        else
+            decode_stream_merge_quantize_kernel<false><<<ps.batch, merge_threads(ps.num_heads), 0, s>>>(sp, nullptr, nullptr, out, out_bf16, pmax,
+                                                                                                        ps.batch, WeightPrefetch{});
         return;
     }
     dim3 grid2(ps.num_heads, ps.batch);
