@@ -21,16 +21,19 @@ namespace {
 
 // ------------------------------------------------------------------ up to 64 rows
 // A block owns NTW column tiles.  Its eight wavefronts take every eighth pair of k tiles, two pairs at a time under way: the weight
-// tiles in registers, the activation rows' 128 bytes of a pair in LDS, eight neighbouring lanes to a row (global_load_lds).  The
+// tiles in registers, the activation rows' 128 bytes of a pair in LDS, eight neighbouring lanes to a row.  The
 // sums meet in LDS in a fixed order.  row_of(i): the activation row behind row i of the block's rows (i < m; others repeat the last
 // one and are never stored) and the output row.
 // What bounds it is the weights' way from memory, as long as the rows do not stand in it: the matrix instruction wants a lane to
 // hold 16 bytes of its own row, and loaded that way into registers four neighbouring lanes touch four cache lines, which the
 // address unit serves one per cycle (64 cycles an instruction instead of 16).  In microseconds, loaded so and staged, with 4, 16
 // and 32 rows: 2048 -> 2048 4.6, 6.0, 8.0 and 4.1, 4.7, 5.7; 2048 -> 6176 6.7, 9.3, 9.5 and 6.1, 6.6, 8.1; 8192 -> 2048 10.0,
-// 15.1, 21.1 and 9.1, 11.5, 15.3; 4096 -> 32000 47, 45, 50 and 42, 42, 47 (6.3 TB/s).  Three and four pairs under way: slower
-// (longer code, fewer blocks to a compute unit) in nearly all shapes.  What the epilogue reads from memory is requested ahead of
-// the weights (0.7 us of the residual form at 4.5).
+// 15.1, 21.1 and 9.1, 11.5, 15.3; 4096 -> 32000 47, 45, 50 and 42, 42, 47 (6.3 TB/s).  33 to 64 rows, whole prompts of 33, 48 and
+// 64 rows through four layers of width 2048 373, 397, 421 and 335, 343, 353, of 4096 574, 620, 670 and 504, 524, 548.  What the
+// epilogue reads from memory is requested ahead of the weights (0.7 us of the residual form at 4.5).
+// Loads of rows are buffer loads: behind a global load into LDS, which the compiler takes for one that LDS answers, it waits for
+// everything instead of counting.  (Level so far: drained at every second pair, the block's other wavefronts still had theirs
+// under way; prompts of 1 to 64 rows within 1 % either way.)
 constexpr int kRowWaves = 8, kRowPairs = 2;          // wavefronts of a block; pairs of k tiles under way in each
 constexpr uint32_t row_stage_bytes(int mt) { return mt * 2048; }     // rows of one pair
 constexpr uint32_t row_lds_bytes(int mt, int ntw) {
@@ -40,7 +43,9 @@ constexpr uint32_t row_lds_bytes(int mt, int ntw) {
 typedef __attribute__((address_space(1))) const void *gptr;
 typedef __attribute__((address_space(3))) void *lptr;
 
-// This wavefront's loads but the N youngest have landed, those into LDS too.
+// No load moves across this one (in the program; it is no instruction).
+__device__ __forceinline__ void loads_stay() { asm volatile("" ::: "memory"); }
+// This wavefront's loads but the N youngest have landed, those into LDS too.  N counts what was issued since: loads_stay keeps it there.
 template <int N>
 __device__ __forceinline__ void loads_wait() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
@@ -148,7 +153,8 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
     const uint32_t cnt = pairs > (uint32_t)wave ? (pairs - wave + kRowWaves - 1) / kRowWaves : 0;
     // load x of a row tile: rows 8 x .. + 7, lane l brings piece (l % 8) ^ (l / 8) of row l / 8, so that the 16 lanes an LDS
     // read serves together (eight rows of two neighbouring k groups) find theirs in different banks
-    [[maybe_unused]] const uint8_t *a_src[MT][2];
+    [[maybe_unused]] uint32_t a_at[MT][2];
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t a_all = __builtin_amdgcn_make_buffer_rsrc((void *)a, 0, -1, 0x00020000);
     [[maybe_unused]] RowsAhead<NORM ? NORM : 1> ra;
     if constexpr (NORM != 0) norm_rows_load(nm, m, ra);
 #pragma unroll
@@ -156,11 +162,13 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
 #pragma unroll
         for (int x = 0; x < (NORM ? 0 : 2); ++x) {
             const uint32_t r = i * 16 + x * 8 + lane / 8;
-            a_src[i][x] = (const uint8_t *)(a + (uint64_t)row_of(r < m ? r : m - 1).x * lda) + ((lane % 8) ^ (lane / 8)) * 16;
+            a_at[i][x] = row_of(r < m ? r : m - 1).x * (uint32_t)lda * 2 + ((lane % 8) ^ (lane / 8)) * 16;
         }
+    gptr w_all = (gptr)w_batch;
+    asm volatile("" : "+s"(w_all));                  // (of a pointer that nothing else names, loads could pass loads_stay)
     const uint8_t *w_src[NTW];
 #pragma unroll
-    for (int j = 0; j < NTW; ++j) w_src[j] = w_batch + (uint64_t)(nt0 + j < n_tiles ? nt0 + j : n_tiles - 1) * k_tiles * 1024 + lane * 16;
+    for (int j = 0; j < NTW; ++j) w_src[j] = (const uint8_t *)w_all + (uint64_t)(nt0 + j < n_tiles ? nt0 + j : n_tiles - 1) * k_tiles * 1024 + lane * 16;
     uint8_t *stage = lds + wave * (kRowPairs * row_stage_bytes(MT));
     const uint32_t r16 = lane % 16, at0 = (uint32_t)(uintptr_t)(lptr)stage + (r16 / 8) * 1024 + (r16 % 8) * 128;
     const uint32_t at[2] = {at0 + (((uint32_t)lane / 16) ^ (r16 % 8)) * 16, at0 + ((4 + (uint32_t)lane / 16) ^ (r16 % 8)) * 16};
@@ -186,11 +194,13 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
         for (int j = 0; j < NTW; ++j)
 #pragma unroll
             for (int h = 0; h < 2; ++h) bv[s][h][j] = stream_load<true>((const v4i *)(w_src[j] + (uint64_t)p * 2048 + h * 1024));
+        loads_stay();
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int x = 0; x < (NORM ? 0 : 2); ++x)
-                __builtin_amdgcn_global_load_lds((gptr)(a_src[i][x] + (uint64_t)p * 128), (lptr)(stage + s * row_stage_bytes(MT) + i * 2048 + x * 1024), 16, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(a_all, (lptr)(stage + s * row_stage_bytes(MT) + i * 2048 + x * 1024), 16, a_at[i][x], p * 128, 0, 0);
+        loads_stay();
     };
     auto mul = [&](auto sc, uint32_t it) {
         constexpr int s = decltype(sc)::value;
@@ -212,7 +222,7 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
     };
     static_assert(kRowPairs == 2, "two slots are written out below");
     // (wavefronts without a pair load the first one, and nobody reads it: behind a branch nothing could count these loads, and the
-    // norm would wait for them instead of for its rows)
+    // norm would wait for them instead of for its rows.  loads_stay keeps the weights ahead of that branch, too.)
     load(0, 0);
     load(1, 1);
     if constexpr (NORM != 0) {
@@ -489,6 +499,8 @@ template <typename K>
 void allow_lds(K kernel, uint32_t bytes) {
     if (bytes > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
+// The rows are addressed by 32-bit byte offsets
+bool rows_reach(uint64_t rows, uint64_t lda) { return rows * lda * 2 <= 1ull << 32; }
 template <int MT, int NTW, int MODE>
 void launch_rows(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, hipStream_t s) {
     constexpr uint32_t lds = row_lds_bytes(MT, NTW);
@@ -533,7 +545,7 @@ template <int MODE>
 void launch_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
                  int num_cus, hipStream_t s) {
     const uint8_t *wt = (const uint8_t *)w.w;
-    if (m <= 64) {
+    if (m <= 64 && rows_reach(m, lda)) {
         const bool two = two_tiles(is_glu(MODE), w, m, num_cus);
         if (m <= 16) {
             if constexpr (!is_glu(MODE))
@@ -563,7 +575,7 @@ void launch_grouped_bf16(const uint16_t *a, uint64_t lda, const LinearWeight &w,
     constexpr bool GLU = is_glu(MODE);
     const uint64_t mean = (rg.likely ? rg.likely : rg.entries) / rg.groups;
     const int form = g_linear_form;
-    if (form == 4 || (form != 5 && form != 6 && mean <= 10)) {
+    if ((form == 4 || (form != 5 && form != 6 && mean <= 10)) && rows_reach((rg.entries + rg.a_div - 1) / rg.a_div, lda)) {
         const bool two = GLU || (uint64_t)w.n_tiles * std::min(rg.groups, rg.entries) >= 2 * (uint64_t)num_cus;
         const int mt = rg.most <= 16 ? 1 : mean <= 8 ? 2 : 4;
         if constexpr (!GLU)
