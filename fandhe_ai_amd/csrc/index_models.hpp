@@ -18,6 +18,11 @@
 namespace fa {
 namespace ixm {
 
+// ------------------------------------------------------------------ blocks that meet
+// Whether the blocks of a group leave their partial results to each other in the L2 of their XCD or in memory: by what was `probed`
+// (workgroups b and b + 8 run on one XCD), unless the tuning key of the split-k linears says memory (2, 4) or the L2 (3).
+FA_HD bool meets_in_l2(int key, int probed) { return key == 3 || (key != 2 && key != 4 && probed != 0); }
+
 // ------------------------------------------------------------------ decode attention
 // Whether a decode step's attention runs as one launch: a block per sequence and kv head, or up to `shares` where compute units are
 // left, `share` tokens in the longest; `even`: what an even division over the units would give each.  That form saves the partial

@@ -21,7 +21,6 @@ namespace k {
 using namespace fa::dev;
 
 int g_gemm_small_tiles = 0;   // tuning: nonzero keeps the 128 x 128 kernel for every shape
-extern int g_skinny_ksplit;   // kern_qlinear.hip
 int g_gemm_pair = 0;          // tuning, tiles of 128 columns of the large-tile kernel: 1 keeps one block per tile
 int g_gemm_swiglu = 0;        // tuning, prompt passes: bit 0 keeps SwiGLU out of the gate | up GEMM's epilogue, bit 1 RoPE
                               // and the K / V append out of the q | k | v GEMM's
@@ -1187,7 +1186,7 @@ void gemm_w8a8_mfma(const int8_t *aq, const int8_t *w_tiles, uint64_t m, uint64_
         const uint64_t tiles = big_tiles(p.tile, m, n_pad);
         if (workspace && workspace_bytes >= share_bytes(p.tile, m, n_pad)) {
             // (the scope knob of the split-k decode linears forces either form here as well: 2 agent scope, 3 the XCD's L2)
-            const EpiI8Split es{e, (int32_t *)workspace, sk->counters, g_skinny_ksplit == 2 ? 0 : g_skinny_ksplit == 3 ? 1 : sk->xcd_local, p.tile.share};
+            const EpiI8Split es{e, (int32_t *)workspace, sk->counters, meets_in_l2(sk), p.tile.share};
             const unsigned grid = 8u * p.tile.share * (unsigned)((tiles + 7) / 8);   // whole groups on every XCD; surplus groups return at once
             launch_big<false, kWide8>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, es, s, grid);
             return;

@@ -1589,7 +1589,7 @@ void paged_attention_decode_one_bf16(const uint16_t *q, const uint16_t *k_pool, 
     sp.by_items = ixm::divider((uint32_t)items);
     sp.by_kv_heads = ixm::divider(ps.num_kv_heads);
     // the shares of an item are `items` blocks apart, and blocks go round the eight XCDs
-    if (shares > 1 && sk->xcd_local && items % 8 == 0 && sk->xcc_seen && sk->fault && items * shares <= sk->n_xcc_seen) {
+    if (shares > 1 && meets_in_l2(sk) && items % 8 == 0 && sk->xcc_seen && sk->fault && items * shares <= sk->n_xcc_seen) {
         sp.xcc_seen = sk->xcc_seen;
         sp.fault = sk->fault;
         decode_stream_kernel<2, 2, 2, 2, false, 1, true, true><<<(unsigned)(items * shares), 256, 0, s>>>(sp);

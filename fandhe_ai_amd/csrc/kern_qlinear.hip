@@ -28,6 +28,8 @@ int g_skinny_ksplit = 0;    // split k over the blocks of an XCD: 0 by shape, 1 
 int g_skinny_ksplit_s = 0;  // members per group of the split (0 by shape, 2 or 4)
 int g_row_fusion = 0;       // row work inside the linears: 0 where it measured faster (norm: two rows, quantizer: one), 1 never, 2 up to the kernels' four / two rows
 
+bool meets_in_l2(const SplitKArea *sk) { return ixm::meets_in_l2(g_skinny_ksplit, sk->xcd_local); }
+
 namespace {
 
 struct EpiI8 {
@@ -1837,7 +1839,7 @@ inline bool ksplit_plan(uint64_t m, uint32_t n_tiles, uint32_t k_tiles, int num_
     if (n_groups > sk->n_counters || bytes > sk->partial_bytes) return false;
     p->s = s;
     p->d = k_tiles / (uint32_t)s >= 32 ? 4 : 2;
-    p->local = g_skinny_ksplit == 3 || ((g_skinny_ksplit == 0) && sk->xcd_local);
+    p->local = meets_in_l2(sk);
     p->n_groups = n_groups;
     p->blocks = 8u * (uint32_t)s * ((n_groups + 7) / 8);       // whole groups on every XCD; surplus groups return at once
     return true;
@@ -2090,7 +2092,7 @@ inline bool rows_ksplit_plan(uint64_t m, uint32_t n_tiles, uint32_t k_tiles, int
     p->row_groups = (uint32_t)((m + 31) / 32);
     p->workspace_bytes = (uint64_t)n_groups * 4 * p->row_groups * (2 * 4 * 4 * 64 * 4);
     if (p->workspace_bytes >> 32) return false;                // the partial sets are read by 32-bit byte offsets
-    p->local = g_skinny_ksplit == 3 || ((g_skinny_ksplit == 0) && sk->xcd_local);
+    p->local = meets_in_l2(sk);
     return true;
 }
 }  // namespace

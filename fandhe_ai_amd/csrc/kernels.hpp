@@ -154,6 +154,9 @@ struct SplitKArea {
     uint32_t n_xcc_seen = 0;
     uint32_t *fault = nullptr;
 };
+// Whether the blocks of a launch that leave partial results to each other may do so in the XCD's L2 (ixm::meets_in_l2): asked by
+// every kernel whose blocks meet.
+bool meets_in_l2(const SplitKArea *sk);
 // out[b] = hardware id of the XCD workgroup b of the probe launch ran on (b < blocks)
 void xcc_id_probe(uint32_t *out, uint32_t blocks, hipStream_t s);
 // Row work that a decode-shape linear of at most four rows does for itself (row_prologue.hpp) instead of reading

@@ -131,11 +131,11 @@ fa_pool_stats SizeClassPool::stats() {
 fa_status check_ctx(const fa_context *ctx) {
     if (!ctx || ctx->magic != kCtxMagic) return fail(FA_ERR_INVALID_ARGUMENT, "context: null or not a context");
     if (ctx->poisoned) return fail(FA_ERR_CONTEXT_POISONED, "context: poisoned by an earlier device failure");
-    // a split-k linear found the blocks of a group on different XCDs although the probe at creation said they share
-    // one: its partial tiles met through two L2s and what it wrote cannot be trusted
+    // a launch found the blocks of a group on different XCDs although the probe at creation said they share one: their
+    // partial results met through two L2s and what it wrote cannot be trusted
     if (ctx->splitk.fault && *(volatile uint32_t *)ctx->splitk.fault != 0)
-        return fail(FA_ERR_CONTEXT_POISONED, "context: a split-k linear ran its groups across XCDs (results invalid); "
-                                             "recreate the context, or set tuning key 16 to 4 to let partial tiles meet in memory");
+        return fail(FA_ERR_CONTEXT_POISONED, "context: blocks that meet in an L2 ran on different XCDs (results invalid); "
+                                             "recreate the context, with tuning key 16 set to 4 they meet in memory");
     return FA_OK;
 }
 fa_status check_buf(const fa_context *ctx, const fa_buffer *b, const char *what) {

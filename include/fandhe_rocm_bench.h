@@ -81,7 +81,8 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  * key 16: split-k form of the decode-shape linears (groups of blocks that share an XCD divide k and add their
  *        partial tiles through a workspace): 0 by shape, 1 never, 2 whenever the shape allows it with the partial
  *        tiles meeting in memory (agent-scope accesses), 3 whenever the shape allows it with the partial tiles
- *        meeting in the XCD's L2, 4 by shape but meeting in memory;
+ *        meeting in the XCD's L2, 4 by shape but meeting in memory; where they meet (2, 4 memory, 3 the L2) holds for
+ *        the shared tiles of the prompt GEMM and the shares of the decode attention as well;
  * key 17: blocks per group of that form: 0 by shape, 2 or 4;
  * key 18: 1 keeps the row kernels (norm, quantizer, norm + quantizer) of sixteen neighbouring elements per thread for every
  *        row count and width;

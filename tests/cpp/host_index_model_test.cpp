@@ -5,6 +5,7 @@
 //   large-tile GEMM   : e4m3 / int8 (bf16 moves the same bytes) x 8 / 14 / 16 column tiles x 8 / 12 / 16 row tiles x 4 / 8 / 16 wavefronts
 //   streamed attention: ranges, segments and partial-result slots against the merge's expectation, ragged lengths
 //   split-k linears   : groups on one XCD, k ranges, workspace offsets
+//   blocks that meet  : where, by the probe and the tuning key
 //   decode attention  : which form a step takes
 //   row quantizer     : codes at the middles of two codes
 #include <cmath>
@@ -449,7 +450,16 @@ static void quotient_cases() {
             }
 }
 
+// Where blocks that share work meet: by the probe, unless the key says memory or the L2
+static void meeting_cases() {
+    for (int probed : {0, 1}) {
+        CHECK(meets_in_l2(0, probed) == (probed == 1) && meets_in_l2(1, probed) == (probed == 1));
+        CHECK(!meets_in_l2(2, probed) && meets_in_l2(3, probed) && !meets_in_l2(4, probed));
+    }
+}
+
 int main(int argc, char **) {
+    meeting_cases();
     quotient_cases();
     decode_form_cases();
     quantizer_case(argc > 1 ? 1 : 64);

@@ -473,6 +473,35 @@ def test_attention_shares_of_one_launch(ctxs, tune):
     assert np.abs(ca - cb).max() <= 1 and (ca != cb).mean() < 2e-3 and np.any(ca != 0)
 
 
+@pytest.mark.parametrize("ctxs", [[513, 1792], [2047, 2500], [300, 3999, 16, 1]], ids=str)
+def test_attention_shares_meet_in_the_l2_or_in_memory(ctxs, tune):
+    """The shares of a sequence meet in the L2 of their XCD, or, as the tuning key of the split linears has it, in memory: the same sums
+    in the same order, to the last bit, also when a launch of the one kind follows one of the other."""
+    import ctypes as C
+    import test_gpu_decoder as td
+    import fandhe_ai_amd as fa
+    be, lib = ops(), fa.capi.lib
+    m = td.build_model(seed=90 + sum(ctxs), steps=5, batch=len(ctxs), ctxs=ctxs, n_layers=2, d_model=2048, n_heads=16, n_kv_heads=4, d_ffn=3072, vocab=3000)
+    dec = td.GpuDecoder(be, m)
+    tune(20, 3)
+    got = []
+    for key in (0, 4, 0, 2, 3):
+        tune(16, key)
+        dec.set_state(m.seq_lens, m.tokens)
+        fa.check(lib.fa_decoder_debug_step_until(be._ctx, dec.h, 4))
+        xq, sx = C.c_void_p(), C.c_void_p()
+        fa.check(lib.fa_decoder_debug_buffer(dec.h, 1, C.byref(xq)))
+        fa.check(lib.fa_decoder_debug_buffer(dec.h, 2, C.byref(sx)))
+        codes, scales = np.empty(16 * 2048, np.int8), np.empty(len(ctxs), np.float32)
+        fa.check(lib.fa_download(be._ctx, xq, 0, codes.ctypes.data, codes.size))
+        fa.check(lib.fa_download(be._ctx, sx, 0, scales.ctypes.data, len(ctxs)))
+        got.append((codes, scales))
+    dec.close()
+    assert np.any(got[0][0] != 0) and np.all(got[0][1] > 0)
+    for codes, scales in got[1:]:
+        assert np.array_equal(codes, got[0][0]) and np.array_equal(scales, got[0][1])
+
+
 @pytest.mark.parametrize("heads,kv_heads", [(1, 1), (2, 1), (6, 2), (10, 10), (12, 4), (30, 6), (32, 32)])
 def test_merged_rows(heads, kv_heads):
     """The merge of a whole row per block: heads that do not fill its wavefronts, more sequences than a wavefront has lanes, and
