@@ -386,12 +386,14 @@ __device__ __forceinline__ uint32_t this_xcc() {
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(id));
     return id & 15u;
 }
-template <int S>
-__device__ __forceinline__ void meet_check_xcd(const uint32_t *xcc_seen, uint32_t group, uint32_t *fault) {
+__device__ __forceinline__ void meet_note_xcd(uint32_t *xcc_seen, uint32_t group, uint32_t member) {
+    if (xcc_seen && threadIdx.x == 0) meet_store<true>(xcc_seen + ixm::xcc_note(group, member), this_xcc() + 1u);
+}
+__device__ __forceinline__ void meet_check_xcd(const uint32_t *xcc_seen, uint32_t group, uint32_t members, uint32_t *fault) {
     // a lane per member, and not on the first wavefront, whose other work is the longest (one member behind the other: 1 us)
     if (!xcc_seen || threadIdx.x / 64 != blockDim.x / 64 - 1) return;
     const uint32_t lane = threadIdx.x % 64, mine = this_xcc() + 1u;
-    const uint32_t seen = lane < (uint32_t)S ? meet_load<true>(xcc_seen + (uint64_t)group * S + lane) : mine;
+    const uint32_t seen = lane < members ? meet_load<true>(xcc_seen + ixm::xcc_note(group, lane)) : mine;
     if (__ballot(seen != mine) != 0 && lane == 0) __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 

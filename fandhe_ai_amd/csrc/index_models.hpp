@@ -22,6 +22,11 @@ namespace ixm {
 // Whether the blocks of a group leave their partial results to each other in the L2 of their XCD or in memory: by what was `probed`
 // (workgroups b and b + 8 run on one XCD), unless the tuning key of the split-k linears says memory (2, 4) or the L2 (3).
 FA_HD bool meets_in_l2(int key, int probed) { return key == 3 || (key != 2 && key != 4 && probed != 0); }
+// Word of the note that member `member` of group `group` leaves of the XCD it runs on.  A cache line to a group: the last one to
+// arrive reads the notes through its unit's L1, and a line that it read before, for another group of the launch, would still hold the
+// words from before this group's members wrote theirs.
+constexpr uint32_t kNoteWords = 32;                        // 128 bytes
+FA_HD uint64_t xcc_note(uint32_t group, uint32_t member) { return (uint64_t)group * kNoteWords + member; }
 
 // ------------------------------------------------------------------ decode attention
 // Whether a decode step's attention runs as one launch: a block per sequence and kv head, or up to `shares` where compute units are

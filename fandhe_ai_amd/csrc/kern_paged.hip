@@ -579,13 +579,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WPE, W
                     meet_store<LOCAL>(p.one_part_ml + ml + share * 32 + 16, den);
                 }
             }
-            if (LOCAL && threadIdx.x == 0) meet_store<true>(p.xcc_seen + first + share, this_xcc() + 1u);
+            if constexpr (LOCAL) meet_note_xcd(p.xcc_seen, item_id, share);
             if (meet_ticket<LOCAL>(p.one_counters + item_id, &one_ticket) != shares - 1) return;
             if (threadIdx.x == 0) meet_store<LOCAL>(p.one_counters + item_id, 0u);
-            if (LOCAL && wave == 3) {                                      // all shares on this XCD, or their sums went through two L2s
-                const uint32_t mine = this_xcc() + 1u, seen = (uint32_t)lane < shares ? meet_load<true>(p.xcc_seen + first + lane) : mine;
-                if (__ballot(seen != mine) != 0 && lane == 0) __hip_atomic_store(p.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
+            if constexpr (LOCAL) meet_check_xcd(p.xcc_seen, item_id, shares, p.fault);
             // in the order of the shares, whoever came last; shares that are not there repeat the last with weight zero
             float m[kOneShares], l[kOneShares];
             v4f o[kOneShares][2];
@@ -1589,7 +1586,7 @@ void paged_attention_decode_one_bf16(const uint16_t *q, const uint16_t *k_pool, 
     sp.by_items = ixm::divider((uint32_t)items);
     sp.by_kv_heads = ixm::divider(ps.num_kv_heads);
     // the shares of an item are `items` blocks apart, and blocks go round the eight XCDs
-    if (shares > 1 && meets_in_l2(sk) && items % 8 == 0 && sk->xcc_seen && sk->fault && items * shares <= sk->n_xcc_seen) {
+    if (shares > 1 && meets_in_l2(sk) && items % 8 == 0 && sk->xcc_seen && sk->fault && items <= sk->n_xcc_groups) {
         sp.xcc_seen = sk->xcc_seen;
         sp.fault = sk->fault;
         decode_stream_kernel<2, 2, 2, 2, false, 1, true, true><<<(unsigned)(items * shares), 256, 0, s>>>(sp);

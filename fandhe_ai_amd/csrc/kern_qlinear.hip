@@ -1292,11 +1292,11 @@ __global__ void __launch_bounds__(512)
         own[q] = sum;
         meet_store<LOCAL>(mine + idx * 64 + lane, sum);
     }
-    if (LOCAL && xcc_seen && threadIdx.x == 0) meet_store<true>(xcc_seen + (uint64_t)group * S + member, this_xcc() + 1u);
+    if constexpr (LOCAL) meet_note_xcd(xcc_seen, group, member);
     const uint32_t ticket = meet_ticket<LOCAL>(counters + group, (uint32_t *)&red[0][0][0]);
     if (ticket != S - 1) return;
     if (threadIdx.x == 0) meet_store<LOCAL>(counters + group, 0u);      // for the next launch
-    if constexpr (LOCAL) meet_check_xcd<S>(xcc_seen, group, fault);
+    if constexpr (LOCAL) meet_check_xcd(xcc_seen, group, S, fault);
     int other[NE][S];
 #pragma unroll
     for (int q = 0; q < NE; ++q)
@@ -1416,11 +1416,11 @@ __global__ void __launch_bounds__(512)
         int32_t *mine = partial + ixm::rows_ksplit_partial_base(group, member, S, row_groups, g, NACC);
         store_unseen_b128<LOCAL ? 1 : 2>(mine + (wave * 64 + lane) * 4, sum);       // the policy meet_store uses
     }
-    if (LOCAL && xcc_seen && threadIdx.x == 0) meet_store<true>(xcc_seen + (uint64_t)group * S + member, this_xcc() + 1u);
+    if constexpr (LOCAL) meet_note_xcd(xcc_seen, group, member);
     const uint32_t ticket = meet_ticket<LOCAL>(counters + group, (uint32_t *)&red[0][0][0][0]);
     if (ticket != S - 1) return;
     if (threadIdx.x == 0) meet_store<LOCAL>(counters + group, 0u);      // for the next launch
-    if constexpr (LOCAL) meet_check_xcd<S>(xcc_seen, group, fault);
+    if constexpr (LOCAL) meet_check_xcd(xcc_seen, group, S, fault);
     // this wavefront's tile of every row group: rows 4 (lane / 16) + e of row tile wave / S, column lane % 16 of
     // column tile wave % S; the four members' sums are added in member order (int32: exact in any order)
     const int ti = wave / S, tj = wave % S;
@@ -1576,11 +1576,11 @@ __global__ void __launch_bounds__(512)
         own[q] = sum;
         meet_store<LOCAL>(mine + idx * 64 + lane, sum);
     }
-    if (LOCAL && xcc_seen && threadIdx.x == 0) meet_store<true>(xcc_seen + (uint64_t)group * S + member, this_xcc() + 1u);
+    if constexpr (LOCAL) meet_note_xcd(xcc_seen, group, member);
     const uint32_t ticket = meet_ticket<LOCAL>(counters + group, (uint32_t *)&red[0][0][0]);
     if (ticket != S - 1) return;
     if (threadIdx.x == 0) meet_store<LOCAL>(counters + group, 0u);
-    if constexpr (LOCAL) meet_check_xcd<S>(xcc_seen, group, fault);
+    if constexpr (LOCAL) meet_check_xcd(xcc_seen, group, S, fault);
     float other[NE][S];
 #pragma unroll
     for (int q = 0; q < NE; ++q)
@@ -1845,9 +1845,9 @@ inline bool ksplit_plan(uint64_t m, uint32_t n_tiles, uint32_t k_tiles, int num_
     return true;
 }
 
-// the XCD notes of a launch, when the area has room for one word per block and a place to report to
+// the XCD notes of a launch, when the area has room for its groups' and a place to report to
 inline uint32_t *xcc_seen_for(const SplitKArea *sk, const KsplitPlan &p) {
-    return (sk->xcc_seen && sk->fault && (uint64_t)p.n_groups * p.s <= sk->n_xcc_seen) ? sk->xcc_seen : nullptr;
+    return (sk->xcc_seen && sk->fault && p.n_groups <= sk->n_xcc_groups) ? sk->xcc_seen : nullptr;
 }
 
 // Calls go(MT, S, D, LOCAL) with the plan's values as integral constants.

@@ -1,5 +1,6 @@
 // Context, stream, memory pool, transfers, graph capture and timers.
 #include "runtime.hpp"
+#include "index_models.hpp"
 
 #include <algorithm>
 #include <cstdio>
@@ -480,9 +481,9 @@ fa_status fa_context_create(int32_t ordinal, fa_context **out) {
     // workgroups report the XCD they run on.  Without that property the partial tiles meet in memory instead.
     {
         constexpr uint64_t kPartial = 16ull << 20;
-        constexpr uint32_t kCounters = 4096, kProbe = 2048, kXccSeen = 16384;
+        constexpr uint32_t kCounters = 4096, kProbe = 2048, kNotes = kCounters * fa::ixm::kNoteWords;
         void *area = nullptr;
-        if (hipMalloc(&area, kPartial + (kCounters + kXccSeen) * 4) == hipSuccess) {
+        if (hipMalloc(&area, kPartial + (kCounters + kNotes) * 4) == hipSuccess) {
             uint32_t *counters = (uint32_t *)((uint8_t *)area + kPartial);
             std::vector<uint32_t> ids(kProbe, 0xffu);
             fa::k::xcc_id_probe(counters, kProbe, ctx->stream);
@@ -498,7 +499,7 @@ fa_status fa_context_create(int32_t ordinal, fa_context **out) {
                 for (uint32_t b = 0; b < kProbe; ++b) seen[ids[b] & 15u] = true;
                 for (bool x : seen) ctx->xcd_count += x ? 1 : 0;
             }
-            ok = ok && hipMemsetAsync(area, 0, kPartial + (kCounters + kXccSeen) * 4, ctx->stream) == hipSuccess &&
+            ok = ok && hipMemsetAsync(area, 0, kPartial + (kCounters + kNotes) * 4, ctx->stream) == hipSuccess &&
                  hipStreamSynchronize(ctx->stream) == hipSuccess;
             if (ok) {
                 ctx->splitk.partial = area;
@@ -506,10 +507,10 @@ fa_status fa_context_create(int32_t ordinal, fa_context **out) {
                 ctx->splitk.counters = counters;
                 ctx->splitk.n_counters = kCounters;
                 ctx->splitk.xcd_local = round_robin ? 1 : 0;
-                // one word per block of a launch (the groups' XCD notes) behind the counters, and the word of pinned
-                // host memory a launch reports a split group to
+                // the groups' XCD notes behind the counters, and the word of pinned host memory a launch reports a
+                // split group to
                 ctx->splitk.xcc_seen = counters + kCounters;
-                ctx->splitk.n_xcc_seen = kXccSeen;
+                ctx->splitk.n_xcc_groups = kCounters;
                 void *flag = nullptr;
                 if (hipHostMalloc(&flag, 64, hipHostMallocMapped) == hipSuccess) {
                     *(volatile uint32_t *)flag = 0;

@@ -456,6 +456,9 @@ static void meeting_cases() {
         CHECK(meets_in_l2(0, probed) == (probed == 1) && meets_in_l2(1, probed) == (probed == 1));
         CHECK(!meets_in_l2(2, probed) && meets_in_l2(3, probed) && !meets_in_l2(4, probed));
     }
+    // notes of two groups are never in one line of 128 bytes, those of a group (eight members at most) always
+    for (uint32_t group = 0; group < 4096; ++group)
+        for (uint32_t member = 0; member < 8; ++member) CHECK(xcc_note(group, member) / 32 == group && xcc_note(group, member) % 32 == member);
 }
 
 int main(int argc, char **) {
