@@ -231,10 +231,13 @@ struct StepScalars {
 // Element at a byte offset that 32 bits hold
 template <typename V>
 __device__ __forceinline__ V at_byte(const void *base, uint32_t offset) { return *(const V *)((const char *)base + offset); }
-// x^-1/2 with the hardware's estimate corrected by its remainder
+// x^-1/2 of a normal x with the hardware's estimate corrected by its remainder
 __device__ __forceinline__ float rsqrt_exact(float x) {
     const float r = __builtin_amdgcn_rsqf(x);
     return fmaf(fmaf(-x * r, r, 1.0f), 0.5f * r, r);
+}
+__device__ __forceinline__ float rsqrt_any(float x) {
+    return __builtin_expect(x >= 0x1p-126f && x < INFINITY, 1) ? rsqrt_exact(x) : 1.0f / sqrtf(x);
 }
 __device__ __forceinline__ v4f fma4(const v4f &a, float b, const v4f &c) {
     return v4f{fmaf(a[0], b, c[0]), fmaf(a[1], b, c[1]), fmaf(a[2], b, c[2]), fmaf(a[3], b, c[3])};
@@ -343,18 +346,38 @@ __global__ void __launch_bounds__(256) one_delta_step_kernel(DeltaShape sh, Delt
 #pragma unroll
         for (int i = 0; i < RPT; ++i) S[i] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    float sq = 0.0f, sk = 0.0f, kq = 0.0f;           // the same in every wavefront
-    for (uint32_t d = lane; d < dim; d += 64) {
-        const v2f x = *(const v2f *)(lds + d * STR);
-        sq = fmaf(x[1], x[1], sq);
-        sk = fmaf(x[0], x[0], sk);
-        kq = fmaf(x[0], x[1], kq);
-    }
+    float sq, sk, kq;                                // the same in every wavefront
+    auto lengths = [&] {
+        sq = sk = kq = 0.0f;
+        for (uint32_t d = lane; d < dim; d += 64) {
+            const v2f x = *(const v2f *)(lds + d * STR);
+            sq = fmaf(x[1], x[1], sq);
+            sk = fmaf(x[0], x[0], sk);
+            kq = fmaf(x[0], x[1], kq);
+        }
+        sq = wave_sum_dpp(sq);
+        sk = wave_sum_dpp(sk);
+        kq = wave_sum_dpp(kq);
+    };
+    lengths();
     float rq = 1.0f, rk = 1.0f;
-    kq = wave_sum_dpp(kq);
     if constexpr (!LIGHTNING) {
-        rq = rsqrt_exact(wave_sum_dpp(sq) + 1e-6f) * sc.rsqrt_dim;
-        rk = rsqrt_exact(wave_sum_dpp(sk) + 1e-6f);
+        // Vectors of more than 2^16, whose sums with the state could leave the range although those of unit vectors do not (or
+        // whose lengths did, and count as infinite), are brought to unit length ahead of the sums.
+        if (__builtin_expect(!(sq < 0x1p32f && sk < 0x1p32f), 0)) {
+            const float fq = rsqrt_any(sq + 1e-6f), fk = rsqrt_any(sk + 1e-6f);
+            __syncthreads();
+            for (uint32_t d = threadIdx.x; d < dim; d += NT) {
+                lds[d * STR] *= fk;
+                lds[d * STR + 1] *= fq;
+            }
+            __syncthreads();
+            lengths();
+            rq = sc.rsqrt_dim;
+        } else {
+            rq = rsqrt_exact(sq + 1e-6f) * sc.rsqrt_dim;
+            rk = rsqrt_exact(sk + 1e-6f);
+        }
     }
     v4f dk = v4f{0.f, 0.f, 0.f, 0.f}, dq = dk;
     const float *rows = lds + rg * RPT * STR;
@@ -432,7 +455,7 @@ __global__ void __launch_bounds__(256) one_delta_step_kernel(DeltaShape sh, Delt
         for (int e = 0; e < 4; ++e)
             if (cg * 4 + e < vdim) so = fmaf(o[e], o[e], so);
     }
-    const float ro = rsqrt_exact(wave_sum_dpp(so) / (float)vdim + sh.eps) * io.out_scale;
+    const float ro = rsqrt_any(wave_sum_dpp(so) / (float)vdim + sh.eps) * io.out_scale;
     if (lane >= CG) return;
     T *out = (T *)io.out + (uint64_t)row * io.ld_out + h * vdim + cg * 4;
 #pragma unroll

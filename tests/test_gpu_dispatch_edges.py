@@ -264,6 +264,31 @@ def test_bf16_linears_on_every_tile(name, tune):
     assert near(got[TILES[0]]) < 0.06 and abs(near(other) - near(got[TILES[0]])) < 0.02, (near(got[TILES[0]]), near(other))
 
 
+@pytest.mark.parametrize("q,k,v", [(1, 1, 1), (1e4, 1, 1), (1e6, 1e6, 1), (1e25, 1, 1), (1, 1e25, 1), (1e25, 1, 1e14), (1, 1, 1e25), (1e12, 1e12, 1e25)])
+@pytest.mark.parametrize("kind", ["delta", "channel"])
+def test_single_tokens_of_long_vectors(kind, q, k, v):
+    """Tokens one by one against pairs of them on the general kernel: queries, keys and values up to lengths whose squares, or whose
+    products with the state, leave the range of 32 bits, which make the read-out zero and never a NaN."""
+    layers = [lc.delta(heads=4, kv_heads=2, dim=24, vdim=20)] if kind == "delta" else [lc.parallel_2(right=lc.channel_right(4, 2, 20, 12))]
+    cfg = lc.config(layers) if kind == "delta" else lc.bubetar(layers)
+    w = lc.weights(cfg, 11)
+    for leaf, scale in (("q", q), ("k", k), ("v", v)):
+        name = [n for n in w if n.endswith("." + leaf) and (kind == "delta" or ".right." in n)]
+        assert len(name) == 1, (leaf, sorted(w))
+        w[name[0]] = lc.bf16_round(w[name[0]] * np.float32(scale))
+    toks = lc.tokens(cfg, 8, 41)
+    dec = lc.make_decoder(ops(), cfg, w, "float32", max_tokens=64, max_batch=1)
+    table = np.full((1, dec.cfg.max_blocks_per_seq), 0xFFFFFFFF, dtype=np.uint32)
+    table[0, 0] = 0
+    got = []
+    for n in (1, 2):
+        dec.set_sequences(table, [0])
+        got.append(np.concatenate([dec.forward([toks[i:i + n]], [list(range(n))]) for i in range(0, len(toks), n)]))
+    dec.close()
+    assert np.isfinite(got[1]).all() and np.isfinite(got[0]).all()
+    assert lc.error(got[0], got[1]) < 5e-5
+
+
 @pytest.mark.parametrize("rows", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("name", ["nugelix", "zoferax"])
 def test_bf16_rows(name, rows, tune):
