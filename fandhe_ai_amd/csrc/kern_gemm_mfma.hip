@@ -889,8 +889,10 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
             for (int j = 0; j < WNT; ++j) ahead[j] = *(const v4f *)(src + j * 16);
         };
-        // (with eight wavefronts only: the other counts have no registers left, spill 468 bytes a lane instead of 340, and 256 columns
-        // on four wavefronts, which hold every register the unit has, came out wrong in one accumulator's last column)
+        // (with eight wavefronts only: the other counts have no registers left and spill 468 bytes a lane instead of 340.  In 256 columns
+        // on four wavefronts, which hold every register the unit has, the compiler then spilled the last accumulator in part, a[252:254]
+        // to scratch and a255 to a vector register, and reloaded three words where four are read: one column of four was wrong.
+        // tests/test_gemm_codegen_cpu.py looks for such spills.)
         constexpr bool request_ahead = has_residual && WM == 4;
         if constexpr (request_ahead) request(0);
 #pragma unroll

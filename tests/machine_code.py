@@ -1,0 +1,39 @@
+"""The machine code of the built library's kernels, for checks of what the compiler made of them."""
+import os
+import re
+import shutil
+import subprocess
+
+LLVM = "/opt/rocm/llvm/bin"
+HAVE_TOOLS = os.path.exists(os.path.join(LLVM, "llvm-objdump"))
+
+
+def disassemble(tmp_path, pattern):
+    """Kernels whose names match: {name: ([instruction], [(a branch's index, its target's index)])}."""
+    from fandhe_ai_amd import capi
+    objdump = os.path.join(LLVM, "llvm-objdump")
+    lib = shutil.copy(capi.LIB_PATH, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", lib], check=True, capture_output=True, cwd=tmp_path)
+    out = {}
+    for f in sorted(tmp_path.iterdir()):
+        if "gfx950" not in f.name:
+            continue
+        names = subprocess.run([objdump, "-t", str(f)], check=True, capture_output=True, text=True).stdout
+        names = sorted(set(re.findall(r" F .*?(\S*" + pattern + r"\S*)$", names, flags=re.M)))
+        if not names:
+            continue
+        text = subprocess.run([objdump, "-d", "--disassemble-symbols=" + ",".join(names), str(f)], check=True, capture_output=True, text=True).stdout
+        for name, body in re.findall(r"^[0-9a-f]+ <(\S+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", text, flags=re.S | re.M):
+            base, lines, at, jumps = None, [], {}, []
+            for l in body.split("\n"):
+                m = re.match(r"\s*(\S.*?)\s*//\s*([0-9A-F]+):", l)
+                if not m:
+                    continue
+                base = int(m.group(2), 16) if base is None else base
+                at[int(m.group(2), 16)] = len(lines)
+                lines.append(m.group(1))
+                j = re.search(r"<\S+\+0x([0-9a-f]+)>\s*$", l)
+                if j and m.group(1).startswith(("s_cbranch", "s_branch")):
+                    jumps.append((len(lines) - 1, base + int(j.group(1), 16)))
+            out[name] = (lines, [(i, at[to]) for i, to in jumps if to in at])
+    return out

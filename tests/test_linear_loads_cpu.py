@@ -5,47 +5,14 @@ The count is right only as long as the compiler leaves the loads where the sourc
 instance is walked: no row tile is read with one of its own loads under way, none is loaded again with a read of it under way,
 and no wait inside the loop asks for the pair that was requested last.
 """
-import os
 import re
-import shutil
-import subprocess
 
 import pytest
 
-LLVM = "/opt/rocm/llvm/bin"
+from machine_code import HAVE_TOOLS, disassemble
+
 LDS_LOAD = re.compile(r"(buffer|global)_load_dwordx4 .* lds$|global_load_lds")
 VMEM = re.compile(r"(buffer|global|flat|scratch)_(load|store|atomic)")
-
-
-def disassemble(tmp_path, pattern):
-    """Bodies of the library's kernels whose names match: {name: ([instruction], [(branch's index, target's index)])}."""
-    from fandhe_ai_amd import capi
-    objdump = os.path.join(LLVM, "llvm-objdump")
-    lib = shutil.copy(capi.LIB_PATH, tmp_path / "lib.so")
-    subprocess.run([objdump, "--offloading", lib], check=True, capture_output=True, cwd=tmp_path)
-    out = {}
-    for f in sorted(tmp_path.iterdir()):
-        if "gfx950" not in f.name:
-            continue
-        names = subprocess.run([objdump, "-t", str(f)], check=True, capture_output=True, text=True).stdout
-        names = sorted(set(re.findall(r" F .*?(\S*" + pattern + r"\S*)$", names, flags=re.M)))
-        if not names:
-            continue
-        text = subprocess.run([objdump, "-d", "--disassemble-symbols=" + ",".join(names), str(f)], check=True, capture_output=True, text=True).stdout
-        for name, body in re.findall(r"^[0-9a-f]+ <(\S+)>:\n(.*?)(?=^[0-9a-f]+ <|\Z)", text, flags=re.S | re.M):
-            base, lines, at, jumps = None, [], {}, []
-            for l in body.split("\n"):
-                m = re.match(r"\s*(\S.*?)\s*//\s*([0-9A-F]+):", l)
-                if not m:
-                    continue
-                base = int(m.group(2), 16) if base is None else base
-                at[int(m.group(2), 16)] = len(lines)
-                lines.append(m.group(1))
-                j = re.search(r"<\S+\+0x([0-9a-f]+)>\s*$", l)
-                if j and m.group(1).startswith(("s_cbranch", "s_branch")):
-                    jumps.append((len(lines) - 1, base + int(j.group(1), 16)))
-            out[name] = (lines, [(i, at[to]) for i, to in jumps if to in at])
-    return out
 
 
 def faults(lines, row_tiles, jumps=(), start=0, wait_at_least=0):
@@ -103,7 +70,7 @@ def test_faults_are_found():
     assert faults(jump, 1) == [] and faults(jump, 1, [(8, 10)])
 
 
-@pytest.mark.skipif(not os.path.exists(os.path.join(LLVM, "llvm-objdump")), reason="no LLVM tools")
+@pytest.mark.skipif(not HAVE_TOOLS, reason="no LLVM tools")
 def test_rows_are_read_behind_their_loads(tmp_path):
     walked = 0
     for name, (lines, jumps) in disassemble(tmp_path, "linear_rows(?:_grouped)?_kernel").items():
