@@ -100,7 +100,7 @@ void free_all(fa_context *ctx, fa_decoder *d) {
 // Whether the attention of the step about to be enqueued (the host lengths already count its token) finishes in one launch
 // (ixm::decode_attends_at_once); the recorded graphs of the two kinds are kept apart.
 bool step_attends_at_once(const fa_decoder *d) {
-    if (k::g_decode_one == 1) return false;
+    if (k::g_decode_one == 1 || !ixm::decode_one_holds(d->cfg.max_blocks_per_seq)) return false;
     uint64_t longest = 0, all = 0;
     for (uint32_t b = 0; b < d->batch && b < d->host_lens.size(); ++b) {
         longest = std::max<uint64_t>(longest, d->host_lens[b]);

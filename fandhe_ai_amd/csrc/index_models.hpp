@@ -57,7 +57,9 @@ FA_HD_CALL Divider divider(uint32_t n) {
     return Divider{(uint32_t)(((1ull << (31 + l)) + n - 1) / n), 31 + l};
 }
 FA_HD_CALL uint32_t quotient(uint32_t x, const Divider &d) { return (uint32_t)((uint64_t)x * d.m >> d.shift); }
-// Pages lo .. hi - 1 of the npg pages of a sequence (below 2^26) for wavefront `part` of its 4 * shares (shares <= 8): an even split
+// Pages lo .. hi - 1 of the npg pages of a sequence for wavefront `part` of its 4 * shares (shares <= 8): an even split, exact in 32
+// bits for tables that decode_one_holds.
+FA_HD bool decode_one_holds(uint64_t max_blocks_per_seq) { return max_blocks_per_seq < 1u << 26; }
 FA_HD_CALL void decode_one_pages(uint32_t npg, uint32_t part, uint32_t shares, uint32_t *lo, uint32_t *hi) {
     *lo = (npg * part >> 2) / shares;
     *hi = (npg * (part + 1) >> 2) / shares;

@@ -448,6 +448,10 @@ static void quotient_cases() {
                 decode_one_pages(npg, part, shares, &lo, &hi);
                 CHECK(lo == (uint64_t)npg * part / (4 * shares) && hi == (uint64_t)npg * (part + 1) / (4 * shares));
             }
+    uint32_t lo, hi;
+    decode_one_pages(1u << 27, 31, 8, &lo, &hi);             // the last wavefront of a sequence that the split does not hold
+    CHECK(hi != 1u << 27);
+    for (uint64_t blocks : {1ull, (1ull << 26) - 1, 1ull << 26, 1ull << 27, (1ull << 32) - 1}) CHECK(decode_one_holds(blocks) == (blocks < 1ull << 26));
 }
 
 // Where blocks that share work meet: by the probe, unless the key says memory or the L2
