@@ -626,9 +626,9 @@ void linear_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, 
 // Up to what the LDS and a thread's registers hold of the rows, and while the blocks that norm the same rows again cost less than
 // the launch (4 rows, us, with the launch and without: 896 blocks at k of 4096 42.9 and 42.2, 2000 at 2048 25.4 and 24.7, 2000 at 4096
 // 44.6 and 46.3).
-bool linear_norms_rows(uint64_t m, uint64_t hidden, const LinearWeight &w, bool glu, int num_cus) {
-    const uint64_t k_pad = (uint64_t)w.k_tiles * 32, ntw = two_tiles(glu, w, m, num_cus) ? 2 : 1, blocks = (w.n_tiles + ntw - 1) / ntw;
-    return m <= kNormRows && hidden % 4 == 0 && hidden <= k_pad && k_pad <= 4096 && blocks * k_pad <= 5 << 20 && w.batches == 1 && g_linear_form != 3;
+bool linear_norms_rows(uint64_t m, uint64_t hidden, const LinearWeight &w, int mode, int num_cus) {
+    const uint64_t k_pad = (uint64_t)w.k_tiles * 32, ntw = two_tiles(is_glu(mode), w, m, num_cus) ? 2 : 1, blocks = (w.n_tiles + ntw - 1) / ntw;
+    return linear_norms_mode(mode) && m <= kNormRows && hidden % 4 == 0 && hidden <= k_pad && k_pad <= 4096 && blocks * k_pad <= 5 << 20 && w.batches == 1 && g_linear_form != 3;
 }
 
 void linear_normed_bf16(const NormAhead &nm, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
@@ -638,7 +638,9 @@ void linear_normed_bf16(const NormAhead &nm, uint64_t m, const LinearWeight &w, 
         case LinearEpilogue::kSiluGlu: return launch_normed<LinearEpilogue::kSiluGlu>(nm, m, w, ep, num_cus, s);
         case LinearEpilogue::kSoftcap: return launch_normed<LinearEpilogue::kSoftcap>(nm, m, w, ep, num_cus, s);
         case LinearEpilogue::kXielu: return launch_normed<LinearEpilogue::kXielu>(nm, m, w, ep, num_cus, s);
-        default: return launch_normed<LinearEpilogue::kStore>(nm, m, w, ep, num_cus, s);
+        case LinearEpilogue::kStore: return launch_normed<LinearEpilogue::kStore>(nm, m, w, ep, num_cus, s);
+        default: static_assert(!linear_norms_mode(LinearEpilogue::kResidual) && !linear_norms_mode(LinearEpilogue::kHeadGate) &&
+                               !linear_norms_mode(LinearEpilogue::kSquaredRelu), "the modes above are those of the predicate");
     }
 }
 

@@ -375,14 +375,18 @@ void linear_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, 
 void linear_f32(const float *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
                 hipStream_t s);
 // The same on rows ahead of their norm, a = (x - mean) / sqrt(mean((x - mean)^2) + eps) * w (rms: without the mean), x [m, hidden] f32,
-// rounded to bf16: linears whose predicate holds, modes kStore, kGlu, kSiluGlu, kSoftcap, kXielu.
+// rounded to bf16: linears whose predicate holds, with an epilogue of that mode.
 struct NormAhead {
     const float *x = nullptr, *w = nullptr;
     uint32_t hidden = 0;
     float eps = 0.0f;
     int rms = 0;
 };
-bool linear_norms_rows(uint64_t m, uint64_t hidden, const LinearWeight &w, bool glu, int num_cus);
+constexpr bool linear_norms_mode(int mode) {
+    return mode == LinearEpilogue::kStore || mode == LinearEpilogue::kGlu || mode == LinearEpilogue::kSiluGlu || mode == LinearEpilogue::kSoftcap ||
+           mode == LinearEpilogue::kXielu;
+}
+bool linear_norms_rows(uint64_t m, uint64_t hidden, const LinearWeight &w, int mode, int num_cus);
 void linear_normed_bf16(const NormAhead &nm, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s);
 // Rows chosen on the device per batch entry of a weight (the experts of a sparse feed-forward): entry list[g * pitch + i],
 // i < count[g], of group g takes row entry / a_div of the activations and is row `entry` of the output.  Entries are below

@@ -266,15 +266,15 @@ void linear(fa_context *ctx, const LayeredState &L, const void *a, uint64_t lda,
     else k::linear_bf16((const uint16_t *)a, lda, a_batch, m, w, ep, ctx->props.multiProcessorCount, ctx->stream);
 }
 
-// A norm of the residual that the next linear may take into its own launch, or that goes out now, into a.hn
+// A norm of the residual that the next linear, with an epilogue of `mode`, may take into its own launch, or that goes out now, into a.hn
 struct Normed {
     k::NormAhead ahead;
     bool fused;
 };
 Normed norm_ahead(fa_context *ctx, const LayeredState &L, const Arena &a, const float *x, const float *w, int rms, uint32_t rows, const k::LinearWeight &next,
-                  bool glu = false) {
+                  int mode) {
     const uint32_t D = L.cfg.d_model, ld_hn = pad_to(D, 64);
-    const Normed nm{k::NormAhead{x, w, D, L.cfg.norm_eps, rms}, !L.is_f32 && k::linear_norms_rows(rows, D, next, glu, ctx->props.multiProcessorCount)};
+    const Normed nm{k::NormAhead{x, w, D, L.cfg.norm_eps, rms}, !L.is_f32 && k::linear_norms_rows(rows, D, next, mode, ctx->props.multiProcessorCount)};
     if (!nm.fused) (rms ? k::rmsnorm_rows : k::layernorm_rows)(x, w, a.hn, L.is_f32, rows, D, ld_hn, L.cfg.norm_eps, ctx->stream);
     return nm;
 }
@@ -457,12 +457,15 @@ void enqueue_mixers(fa_context *ctx, fa_decoder *d, Arena &a, const Layer &l, co
     }
 }
 
+int dense_mode(const Layer &l) {
+    return l.cfg.glu == FA_GLU_SILU ? k::LinearEpilogue::kSiluGlu : l.cfg.glu == FA_FFN_XIELU ? k::LinearEpilogue::kXielu : k::LinearEpilogue::kGlu;
+}
 // Dense feed-forward: from a.hn (or what nm says) to what `out` does with the down projection.
 void enqueue_dense(fa_context *ctx, LayeredState &L, Arena &a, const Layer &l, uint32_t M, uint32_t ld_hn, const k::LinearEpilogue &out,
                    const Normed *nm = nullptr) {
     const uint32_t ld_act = pad_to(l.cfg.d_ffn, 64);
     k::LinearEpilogue g = store_to(a.act, ld_act, L.is_f32);
-    g.mode = l.cfg.glu == FA_GLU_SILU ? k::LinearEpilogue::kSiluGlu : l.cfg.glu == FA_FFN_XIELU ? k::LinearEpilogue::kXielu : k::LinearEpilogue::kGlu;
+    g.mode = dense_mode(l);
     g.act = l.act;
     g.limit = l.cfg.ffn_limit;
     g.alpha = l.cfg.ffn_alpha;
@@ -525,7 +528,7 @@ fa_status enqueue_layers(fa_context *ctx, fa_decoder *d, Arena &a, const k::Ragg
     for (size_t li = 0; li < L.layers.size(); ++li) {
         const Layer &l = L.layers[li];
         Normed nm{};
-        if (L.cfg.norm == FA_NORM_INPUT) nm = norm_ahead(ctx, L, a, a.x, l.norm1, 0, M, l.in);
+        if (L.cfg.norm == FA_NORM_INPUT) nm = norm_ahead(ctx, L, a, a.x, l.norm1, 0, M, l.in, k::LinearEpilogue::kStore);
         const uint32_t ld_o = pad_to(l.o_width, 64);
         enqueue_mixers(ctx, d, a, l, rr, n, ld_hn, ld_o, expand, &nm);
         k::ResidualNorm rn;
@@ -594,7 +597,7 @@ fa_status enqueue_layers(fa_context *ctx, fa_decoder *d, Arena &a, const k::Ragg
             r.scale = l.post1;
             linear(ctx, L, a.o, ld_o, 0, M, l.out, r);
             if (l.cfg.d_ffn) {
-                nm = norm_ahead(ctx, L, a, a.x, l.norm2, 0, M, l.gate_up, l.cfg.glu != FA_FFN_XIELU);
+                nm = norm_ahead(ctx, L, a, a.x, l.norm2, 0, M, l.gate_up, dense_mode(l));
                 r.scale = l.post2;
                 enqueue_dense(ctx, L, a, l, M, ld_hn, r, &nm);
             }
@@ -620,7 +623,8 @@ void enqueue_embed(fa_context *ctx, const LayeredState &L, Arena &a, const int32
 // Final norm and head over rows of f32 residuals.
 void enqueue_head(fa_context *ctx, LayeredState &L, Arena &a, const float *x, uint32_t rows, float *logits) {
     const uint32_t ld_hn = pad_to(L.cfg.d_model, 64);
-    const Normed nm = norm_ahead(ctx, L, a, x, L.final_norm, L.cfg.norm == FA_NORM_OUTPUT || L.cfg.norm == FA_NORM_INPUT_RMS, rows, L.head);
+    const Normed nm = norm_ahead(ctx, L, a, x, L.final_norm, L.cfg.norm == FA_NORM_OUTPUT || L.cfg.norm == FA_NORM_INPUT_RMS, rows, L.head,
+                                 k::LinearEpilogue::kSoftcap);
     k::LinearEpilogue e = store_to(logits, L.cfg.vocab, 1);
     e.mode = k::LinearEpilogue::kSoftcap;
     e.factor = L.cfg.logit_scale;
