@@ -723,6 +723,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
         constexpr int MODE = IsBf16<Epi>::mode, STEP = is_glu(MODE) ? 2 : 1;      // gate, up: neighbouring tiles
         static_assert(STEP == 1 || WNT % 2 == 0, "a gate tile and its up tile belong to one wavefront");
         if constexpr (MODE == LinearEpilogue::kResidual) {
+            static_assert(!GROUPED, "rows of a group go to where its list says");
             // The stream is read and written in place, so the compiler keeps every read behind the writes before it: a memory round
             // trip per tile.  Here four tiles are requested while the four before them are added.
             const uint32_t col0 = (nt0 + wn * WNT) * 16;
