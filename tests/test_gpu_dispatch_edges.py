@@ -307,8 +307,12 @@ def test_bf16_rows(name, rows, tune):
     dec.close()
     want = oracle.forward(cfg, w, toks)
     # the bf16 tests' bar for the worst row is 0.12; half of it for the middle one
-    err = np.sqrt(np.mean((got - want) ** 2, axis=1)) / np.sqrt(np.mean(want ** 2))
+    size = np.sqrt(np.mean(want ** 2))
+    err = np.sqrt(np.mean((got - want) ** 2, axis=1)) / size
     assert np.median(err) < 0.06 and err.max() < 0.12, (np.median(err), err.max())
+    # every column tile by itself: a row's error hardly shows one of 263 that is missing (0.044 for the last one's eight columns)
+    tiles = np.add.reduceat((got - want) ** 2, np.arange(0, 4200, 16), axis=1).sum(axis=0) / (rows * np.minimum(16, 4200 - np.arange(0, 4200, 16)))
+    assert np.sqrt(np.mean(want[:, -8:] ** 2)) > 0.24 * size and np.sqrt(tiles.max()) < 0.12 * size, (np.sqrt(tiles.max()) / size, tiles.argmax())
 
 
 @pytest.mark.parametrize("width", [76, 2048, 2052, 4096])
