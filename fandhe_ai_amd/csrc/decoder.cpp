@@ -858,9 +858,6 @@ static fa_status prefill_impl(fa_context *ctx, fa_decoder *d, const int32_t *tok
     for (uint32_t b = 0; b < B; ++b) {
         if (padded && (row_lens[b] == 0 || row_lens[b] > l_new))
             return fail(FA_ERR_INVALID_ARGUMENT, "decoder_prefill: row " + std::to_string(b) + " has a length outside 1..=l_max");
-        // the padding needs no pages, but its positions must stay inside the row of the block table
-        if ((uint64_t)d->host_lens[b] + l_new > (uint64_t)c.max_blocks_per_seq * c.block_size)
-            return fail(FA_ERR_INVALID_ARGUMENT, "paged_kv: row " + std::to_string(b) + " has no room for the prompt");
         const uint64_t end = (uint64_t)d->host_lens[b] + (padded ? row_lens[b] : l_new);
         const uint64_t need = (end + c.block_size - 1) / c.block_size;
         if (need > c.max_blocks_per_seq)

@@ -437,6 +437,32 @@ def test_padded_prompt_pass_leaves_every_row_as_its_own_prompt_pass_would():
     dec.close()
 
 
+def test_a_short_prompt_on_a_nearly_full_row_beside_a_long_one():
+    """What a row needs room for are its own tokens: the rest of its neighbour's length is never placed."""
+    import fandhe_ai_amd as fa
+    dec = _decoder(max_blocks_per_seq=4, num_blocks=8, max_batch=2)
+    rng = np.random.default_rng(9)
+    before, prompts = rng.integers(0, VOCAB, (1, 60)).astype(np.int32), [rng.integers(0, VOCAB, n).astype(np.int32) for n in (4, 45)]
+    tables = np.arange(8, dtype=np.uint32).reshape(2, 4)
+
+    def row_0():
+        dec.set_sequences(tables[:1], np.zeros(1, np.uint32))
+        dec.prefill(before)
+
+    row_0()
+    dec.prefill(prompts[0][None])
+    alone = dec.logits()[0].copy()
+    row_0()
+    dec.set_sequences(tables, np.array([60, 0], np.uint32))
+    with pytest.raises(fa.InvalidArgument):
+        dec.prefill_padded([np.zeros(5, np.int32), prompts[1]])
+    dec.prefill_padded(prompts)
+    assert dec.seq_lens().tolist() == [64, 45]
+    err = np.abs(dec.logits()[0] - alone) / float(alone.max() - alone.min())
+    assert err.mean() < 2e-4 and err.max() < 2e-2, (err.mean(), err.max())
+    dec.close()
+
+
 @pytest.mark.parametrize("form", [{10: 2, 23: 1}, {10: 2, 23: 2}, {10: 2, 12: 4}, {10: 1}], ids=["narrow", "wide", "split", "streamed"])
 @pytest.mark.parametrize("cached,lens", [(0, (1, 33, 16, 32)), (16, (17, 1, 40)), (150, (2, 31, 5))])
 def test_padded_pass_without_its_padding(cached, lens, form):
