@@ -495,7 +495,7 @@ class BatchScheduler:
         self._pages = PageAllocator(cfg.num_blocks)
         self._slots = PageAllocator(slots) if slots else None
         self._resident = None                              # ids whose decode state is installed on the device, in row order
-        # what the device was asked to do so far: prompt passes, their rows incl. padding, decode steps and their rows
+        # what the device was asked to do so far: prompt passes, their rows, decode steps and their rows
         self.stats = {"prompt_passes": 0, "prompt_rows": 0, "decode_steps": 0, "decode_rows": 0}
 
     def queued_len(self):
@@ -670,8 +670,9 @@ class BatchScheduler:
 
     def _prompt_groups(self, fresh):
         """Requests that join in the same iteration share prompt passes: sorted by prompt length and cut into
-        groups whose padded size stays within one pass and whose longest prompt is at most twice the
-        shortest (the padding is computed and thrown away)."""
+        groups whose padded size stays within what one pass takes and whose longest prompt is at most twice the
+        shortest.  (The pass leaves the padding out; the factor is from when it was computed, and wider groups have
+        not been measured since.)"""
         groups, cur = [], []
         for a in sorted(fresh, key=lambda a: (len(a.tokens), a.id)):
             n = len(a.tokens)
@@ -689,7 +690,7 @@ class BatchScheduler:
         self._place(group, [0] * len(group))
         self._dec.set_row_sampling(self._policy_rows(group))
         self.stats["prompt_passes"] += 1
-        self.stats["prompt_rows"] += len(group) * max(len(a.tokens) for a in group)
+        self.stats["prompt_rows"] += sum(len(a.tokens) for a in group)
         if len(group) == 1:
             self._dec.prefill(np.array([group[0].tokens], dtype=np.int32))
         else:

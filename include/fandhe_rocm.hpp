@@ -812,7 +812,7 @@ class PageAllocator {
     std::vector<uint32_t> returned_;
 };
 
-// What the device was asked to do so far: prompt passes, their rows including padding, decode steps, their rows.
+// What the device was asked to do so far: prompt passes, their rows, decode steps, their rows.
 struct SchedulerStats {
     uint64_t prompt_passes = 0, prompt_rows = 0, decode_steps = 0, decode_rows = 0;
 };
@@ -1004,7 +1004,8 @@ template <typename DecoderT> class BatchScheduler {
         resident_.reset();
     }
     // requests that join in the same iteration share prompt passes: sorted by prompt length and cut into groups
-    // whose padded size stays within one pass and whose longest prompt is at most twice the shortest
+    // whose padded size stays within what one pass takes and whose longest prompt is at most twice the shortest (the pass
+    // leaves the padding out; the factor is from when it was computed, and wider groups have not been measured since)
     std::vector<std::vector<Active *>> prompt_groups(std::vector<Active *> fresh) const {
         std::sort(fresh.begin(), fresh.end(), [](const Active *x, const Active *y) {
             return x->tokens.size() != y->tokens.size() ? x->tokens.size() < y->tokens.size() : x->id < y->id;
@@ -1029,10 +1030,8 @@ template <typename DecoderT> class BatchScheduler {
         table_rows(group, tables);
         dec_.set_sequences(tables, std::vector<uint32_t>(group.size(), 0));
         dec_.set_row_sampling(policy_rows(group));
-        uint64_t l_max = 0;
-        for (const Active *a : group) l_max = std::max<uint64_t>(l_max, a->tokens.size());
         stats_.prompt_passes += 1;
-        stats_.prompt_rows += group.size() * l_max;
+        for (const Active *a : group) stats_.prompt_rows += a->tokens.size();
         if (group.size() == 1) {
             dec_.prefill(group[0]->tokens, (uint32_t)group[0]->tokens.size());
         } else {

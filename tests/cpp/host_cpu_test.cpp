@@ -228,7 +228,7 @@ int main() {
         ToyDecoder d(tc);
         BatchScheduler<ToyDecoder> s(d, SchedulerLimits(4, 64, 64));
         std::map<uint64_t, std::vector<int32_t>> want;
-        uint64_t rng = 12345, decode_rows = 0, submitted = 0, prompt_only = 0;
+        uint64_t rng = 12345, decode_rows = 0, prompt_rows = 0, submitted = 0, prompt_only = 0;
         std::map<uint64_t, std::vector<int32_t>> got;
         std::vector<uint64_t> order;
         auto drain = [&] {
@@ -254,6 +254,7 @@ int main() {
                 const uint64_t id = s.submit(prompt, c);
                 want[id] = alone(prompt, c, tc.vocab);
                 decode_rows += extra > 1 ? extra - 1 : 0;
+                prompt_rows += extra > 0 ? plen : 0;
                 prompt_only += extra == 0;
                 ++submitted;
             }
@@ -272,7 +273,7 @@ int main() {
         CHECK(got.size() == submitted);
         for (auto &kv : want) CHECK(got[kv.first] == kv.second);
         CHECK(s.free_pages() == tc.num_blocks);
-        CHECK(s.stats().decode_rows == decode_rows);
+        CHECK(s.stats().decode_rows == decode_rows && s.stats().prompt_rows == prompt_rows);
         CHECK(s.stats().prompt_passes >= 1 && s.stats().prompt_passes <= submitted - prompt_only);
     }
     // ---- failures stay with their request

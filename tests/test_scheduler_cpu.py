@@ -260,6 +260,7 @@ def test_interleaved_requests_match_single_generate():
         assert done[rid].shape == want.shape and done[rid].tolist() == want.tolist()
     assert m.calls["step_rows"] > m.calls["step"]          # decode steps really ran several requests at once
     assert m.calls.get("padded_rows", 0) >= 2              # and requests that joined together shared a prompt pass
+    assert s.stats["prompt_rows"] == sum(np.size(i) for i, _ in reqs)      # whose rows are the prompts' own
     assert s.free_pages() == 6                             # every page came back
 
 
