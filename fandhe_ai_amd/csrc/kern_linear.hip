@@ -146,7 +146,7 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
                                             uint8_t *lds, RowOf row_of) {
     static_assert(NORM == 0 || MT == 1, "rows that the block norms are few");
     static_assert(!is_glu(MODE) || NTW % 2 == 0, "gate and up are neighbouring tiles");
-    constexpr int NT = MT * NTW, STEP = is_glu(MODE) ? 2 : 1, LOADS = 2 * ((NORM ? 0 : MT) + NTW);
+    constexpr int NT = MT * NTW, STEP = is_glu(MODE) ? 2 : 1, SINCE = 2 * (NORM ? 0 : MT) + 4 * NTW;      // issued since a slot's rows
     static_assert(NT <= kRowWaves * STEP, "a wavefront finishes one tile, or one gate and its up");
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const uint32_t nt0 = blockIdx.x * NTW, pairs = k_tiles / 2;
@@ -191,15 +191,15 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
     auto load = [&](int s, uint32_t it) {            // past the end: the wavefront's last pair again, so that the number under way is the same
         const uint32_t p = cnt ? wave + (it < cnt ? it : cnt - 1) * kRowWaves : 0;
 #pragma unroll
-        for (int j = 0; j < NTW; ++j)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) bv[s][h][j] = stream_load<true>((const v4i *)(w_src[j] + (uint64_t)p * 2048 + h * 1024));
-        loads_stay();
-#pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int x = 0; x < (NORM ? 0 : 2); ++x)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(a_all, (lptr)(stage + s * row_stage_bytes(MT) + i * 2048 + x * 1024), 16, a_at[i][x], p * 128, 0, 0);
+        loads_stay();
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) bv[s][h][j] = stream_load<true>((const v4i *)(w_src[j] + (uint64_t)p * 2048 + h * 1024));
         loads_stay();
     };
     auto mul = [&](auto sc, uint32_t it) {
@@ -221,10 +221,12 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
                                                                         acc[i][j], 0, 0, 0);
     };
     static_assert(kRowPairs == 2, "two slots are written out below");
-    // (wavefronts without a pair load the first one, and nobody reads it: behind a branch nothing could count these loads, and the
-    // norm would wait for them instead of for its rows.  loads_stay keeps the weights ahead of that branch, too.)
-    load(0, 0);
-    load(1, 1);
+    // (ahead of a norm also in wavefronts without a pair, who load the first one, and nobody reads it: behind a branch nothing could
+    // count these loads, and the norm would wait for them instead of for its rows)
+    if (NORM != 0 || cnt != 0) {
+        load(0, 0);
+        load(1, 1);
+    }
     if constexpr (NORM != 0) {
         __builtin_amdgcn_sched_barrier(0);
         norm_rows_store(nm, m, k_tiles * 32, ra, (float *)(normed + kNormRows * normed_pitch(k_tiles * 32)), normed);
@@ -234,18 +236,18 @@ __device__ __forceinline__ void linear_rows(const uint16_t *__restrict__ a, uint
         uint32_t it = 0;
         for (; it + 2 < cnt; it += 2) {
             // the reads of a slot are complete (stage_read waits) before it is loaded again
-            loads_wait<LOADS>();
+            loads_wait<SINCE>();
             mul(std::integral_constant<int, 0>{}, it);
             __builtin_amdgcn_sched_barrier(0);
             load(0, it + 2);
             __builtin_amdgcn_sched_barrier(0);
-            loads_wait<LOADS>();
+            loads_wait<SINCE>();
             mul(std::integral_constant<int, 1>{}, it + 1);
             __builtin_amdgcn_sched_barrier(0);
             load(1, it + 3);
             __builtin_amdgcn_sched_barrier(0);
         }
-        loads_wait<LOADS>();
+        loads_wait<SINCE>();
         mul(std::integral_constant<int, 0>{}, it);
         loads_wait<0>();
         if (it + 1 < cnt) mul(std::integral_constant<int, 1>{}, it + 1);
