@@ -346,38 +346,36 @@ __global__ void __launch_bounds__(256) one_delta_step_kernel(DeltaShape sh, Delt
 #pragma unroll
         for (int i = 0; i < RPT; ++i) S[i] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    float sq, sk, kq;                                // the same in every wavefront
+    float sq, sk, kq, most;                          // the same in every wavefront
     auto lengths = [&] {
-        sq = sk = kq = 0.0f;
+        sq = sk = kq = most = 0.0f;
         for (uint32_t d = lane; d < dim; d += 64) {
             const v2f x = *(const v2f *)(lds + d * STR);
             sq = fmaf(x[1], x[1], sq);
             sk = fmaf(x[0], x[0], sk);
             kq = fmaf(x[0], x[1], kq);
+            most = fmaxf(most, fmaxf(fabsf(x[0]), fabsf(x[1])));
         }
-        sq = wave_sum_dpp(sq);
-        sk = wave_sum_dpp(sk);
-        kq = wave_sum_dpp(kq);
     };
     lengths();
-    float rq = 1.0f, rk = 1.0f;
-    if constexpr (!LIGHTNING) {
-        // Vectors of more than 2^16, whose sums with the state could leave the range although those of unit vectors do not (or
-        // whose lengths did, and count as infinite), are brought to unit length ahead of the sums.
-        if (__builtin_expect(!(sq < 0x1p32f && sk < 0x1p32f), 0)) {
-            const float fq = rsqrt_any(sq + 1e-6f), fk = rsqrt_any(sk + 1e-6f);
-            __syncthreads();
-            for (uint32_t d = threadIdx.x; d < dim; d += NT) {
-                lds[d * STR] *= fk;
-                lds[d * STR + 1] *= fq;
-            }
-            __syncthreads();
-            lengths();
-            rq = sc.rsqrt_dim;
-        } else {
-            rq = rsqrt_exact(sq + 1e-6f) * sc.rsqrt_dim;
-            rk = rsqrt_exact(sk + 1e-6f);
+    // Vectors of more than 2^14, whose sums with the state could leave the range although those of unit vectors do not (or whose
+    // lengths do, and count as infinite), are brought to unit length ahead of the sums.
+    const bool long_ones = !LIGHTNING && __ballot(most > 0x1p14f) != 0;
+    if (__builtin_expect(long_ones, 0)) {
+        const float fq = rsqrt_any(wave_sum_dpp(sq) + 1e-6f), fk = rsqrt_any(wave_sum_dpp(sk) + 1e-6f);
+        __syncthreads();
+        for (uint32_t d = threadIdx.x; d < dim; d += NT) {
+            lds[d * STR] *= fk;
+            lds[d * STR + 1] *= fq;
         }
+        __syncthreads();
+        lengths();
+    }
+    float rq = 1.0f, rk = 1.0f;
+    kq = wave_sum_dpp(kq);
+    if constexpr (!LIGHTNING) {
+        rq = (long_ones ? 1.0f : rsqrt_exact(wave_sum_dpp(sq) + 1e-6f)) * sc.rsqrt_dim;
+        rk = long_ones ? 1.0f : rsqrt_exact(wave_sum_dpp(sk) + 1e-6f);
     }
     v4f dk = v4f{0.f, 0.f, 0.f, 0.f}, dq = dk;
     const float *rows = lds + rg * RPT * STR;
