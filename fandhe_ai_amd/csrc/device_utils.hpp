@@ -240,8 +240,9 @@ __device__ __forceinline__ void quant_i8_words(const V (&x)[N], float scale, uin
     }
 }
 
-// e^-|x|, about one unit in the last place down to the subnormal range: 2^r 2^f with the product by log2(e) kept in two parts.  Needs
-// none of expf's selects for large arguments.
+// e^-|x|, about one unit in the last place down to the subnormal range: Cody and Waite's argument reduction, for base 2.  The product by
+// log2(e) is kept in two parts, r of it rounded goes to the exponent and what is left through 2^f.  Needs none of expf's selects for
+// large arguments.
 __device__ __forceinline__ float exp_minus_abs(float x) {
     constexpr float kHi = 1.44269502f, kLo = 1.92596303e-8f;          // log2(e)
     const float a = __builtin_elementwise_maximum(-fabsf(x), -256.0f);    // 2^-369 is zero; a NaN stays one

@@ -33,14 +33,15 @@ FA_HD uint64_t xcc_note(uint32_t group, uint32_t member) { return (uint64_t)grou
 // left, `share` tokens in the longest; `even`: what an even division over the units would give each.  That form saves the partial
 // results and the merge, and its time is the longest share; the streamed form cuts all pages into equal ranges, whatever the lengths.
 // So what counts is how far the longest share exceeds an even one, and how long it is (a block alone keeps a unit's loads less busy
-// than the streamed form's wavefronts).  Step through 4 layers, streamed and one launch, us:
-//   32 / 8 heads, equal lengths, 16 sequences (two shares) of 3000 475 and 474, 6000 572 and 606; 24 (one) of 1000 445 and 429, 2000 501
-//   and 507; 32 of 1000 471 and 445, 2000 548 and 535, 3000 601 and 623, 4096 703 and 723;
-//   16 / 4 heads, 24 (two shares) of 2000 332 and 332, 4096 391 and 418; 32 of 2000 355 and 347, 3000 381 and 391, 4096 434 and 445; 48 of
-//   1500 368 and 377; 16 (four shares) of 4096 338 and 333, 8000 416 and 412;
-//   lengths apart, 32 / 8 heads: 16 of 100 .. 1000 395 and 379, 2000 .. 4096 487 and 510; 8 (four shares) of 1000 .. 4000 419 and 408.
-// (Two blocks to a sequence fill the units no better than one does, and have to meet.)  With so few sequences that units are left
-// over at `most` shares, the streamed form's many small ranges cost it more: one of 8000 465 and 360, four of 500 .. 8000 449 and 400.
+// than the streamed form's wavefronts).  Step through 4 layers, streamed and one launch (groups of two pages), us:
+//   32 / 8 heads, equal lengths, 16 sequences (two shares) of 3000 458 and 465, 6000 580 and 605; 24 (one) of 1000 436 and 419, 2000 494
+//   and 502; 32 of 1000 463 and 438, 2000 542 and 531, 3000 602 and 624, 4096 708 and 720;
+//   16 / 4 heads, 24 (two shares) of 2000 320 and 306, 4096 378 and 388; 32 of 2000 342 and 325, 3000 369 and 366, 4096 422 and 418; 48 of
+//   1500 357 and 358; 16 (four shares) of 4096 327 and 305, 8000 408 and 392;
+//   lengths apart, 32 / 8 heads: 16 of 100 .. 1000 383 and 360, 2000 .. 4096 475 and 495; 8 (four shares) of 1000 .. 4000 415 and 383.
+// (Two blocks to a sequence fill the units no better than one does, and have to meet.)  The line was set with groups of four pages; with
+// two it is on the worse side by 1.5 % at 16 of 3000 and by 4.5 % at 24 of 2000 with 16 / 4 heads.  With so few sequences that units are
+// left over at `most` shares, the streamed form's many small ranges cost it more: one of 8000 430 and 326, four of 500 .. 8000 433 and 381.
 FA_HD bool decode_attends_at_once(uint64_t share, uint64_t even, uint64_t shares, uint64_t most) {
     if (shares == most) return share <= even + 1024;
     return 8 * (share > even ? share - even : 0) + (shares == 2 ? 9 : 6) * share / 2 <= 6400;

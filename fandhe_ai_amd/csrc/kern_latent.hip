@@ -33,7 +33,8 @@ __global__ void __launch_bounds__(256)
         return 1.0f / sqrtf(block_sum<float, 4, true>(acc, smem) / (float)n + sh.eps);
     };
     // Ranks of a few values per thread: all of the row is requested at once, without branches (past the end: the last value), and both
-    // norms meet in one go: 3.2 us instead of 5.3 for four rows of 768, 512 and 64.
+    // norms meet in one go: 3.2 us instead of 5.3 for four rows of 768, 512 and 64.  (Six and two values a thread are the widest ranks
+    // of the stacks here, 1536 and 512; wider ones go through the loops below, and longer rows of registers were not measured.)
     constexpr uint32_t NQ = 6, NC = 2;
     if (pool && sh.q_rank <= NQ * 256 && sh.kv_rank <= NC * 256 && sh.rot >= 2 && sh.rot <= 512) {
         const uint32_t tid = threadIdx.x, half = sh.rot / 2, pair = tid < half ? tid : half - 1;

@@ -32,8 +32,9 @@ namespace {
 // 64 rows through four layers of width 2048 373, 397, 421 and 335, 343, 353, of 4096 574, 620, 670 and 504, 524, 548.  What the
 // epilogue reads from memory is requested ahead of the weights (0.7 us of the residual form at 4.5).
 // Loads of rows are buffer loads: behind a global load into LDS, which the compiler takes for one that LDS answers, it waits for
-// everything instead of counting.  (Level so far: drained at every second pair, the block's other wavefronts still had theirs
-// under way; prompts of 1 to 64 rows within 1 % either way.)
+// everything instead of counting.  (Worth up to 2 %, and that with 33 to 48 rows of width 4096: while one wavefront waited for both
+// pairs, the block's other seven had theirs under way.)  A pair's rows are requested ahead of its weights, so that they are read back
+// while those travel.
 constexpr int kRowWaves = 8, kRowPairs = 2;          // wavefronts of a block; pairs of k tiles under way in each
 constexpr uint32_t row_stage_bytes(int mt) { return mt * 2048; }     // rows of one pair
 constexpr uint32_t row_lds_bytes(int mt, int ntw) {

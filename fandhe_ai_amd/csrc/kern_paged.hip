@@ -834,7 +834,7 @@ __global__ void __launch_bounds__(kPrefillMergeThreads)
 // One compute unit works on a row, so the kernel is a chain: a load of the lengths, one of the partial results, and what
 // every wavefront computes for itself, which on sixteen wavefronts (four dims a thread) queued four deep.  Every wavefront adds the
 // lengths up by itself, without a meeting; partial results are requested for up to four ranges, or for up to eight.  32 sequences of 1024
-// to 8192 tokens, 32 heads: 8.6 us, so 7.8; 40 of 300 to 3000, 16 heads: 7.0, so 6.8.
+// to 8192 tokens, 32 heads: 8.6 us, so 7.5 to 7.8; 40 of 300 to 3000, 16 heads: 7.0, so 6.8.
 template <int V>
 struct MergedDims {
     v4f o[V];

@@ -26,7 +26,7 @@ int g_skinny_astat = 0;     // activation-stationary kernel: 0 by shape, 1 never
 int g_skinny_ksplit = 0;    // split k over the blocks of an XCD: 0 by shape, 1 never, 2 whenever it can run (agent-scope
                             // meeting), 3 whenever it can run (meeting in the XCD's L2), 4 by shape but agent scope
 int g_skinny_ksplit_s = 0;  // members per group of the split (0 by shape, 2 or 4)
-int g_row_fusion = 0;       // row work inside the linears: 0 where it measured faster (norm: two rows, quantizer: one), 1 never, 2 up to the kernels' four / two rows
+int g_row_fusion = 0;       // row work inside the linears: 0 where it measured faster (up to two rows), 1 never, 2 up to the kernels' four / two rows
 
 bool meets_in_l2(const SplitKArea *sk) { return ixm::meets_in_l2(g_skinny_ksplit, sk->xcd_local); }
 
@@ -1964,7 +1964,7 @@ void with_norm_rows(uint64_t m, F &&go) {
     else go(std::integral_constant<int, kNorm4>{});
 }
 inline bool norm_prologue_shape(uint64_t m, uint64_t k_pad) {
-    // the stand-alone kernel whose f64 association the prologue reproduces is the 1024-thread, one-group-per-thread form
+    // the stand-alone kernel whose f64 association the prologue reproduces is that of up to 4096 columns (512 threads, two groups each);
     // by measurement one or two rows (whole steps of 1 / 2 / 3 / 4 rows of 400 tokens through 8 layers of width 4096, us: 505 / 567 /
     // 598 / 624 with the row work in here against 592 / 608 / 605 / 607 with the row kernels, of width 2048 378 / 404 / 416 from two rows
     // on against 402 / 405 / 410); the kernels take four

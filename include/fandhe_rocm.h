@@ -527,7 +527,8 @@ fa_status fa_decoder_read_row_sampling(fa_context *ctx, fa_decoder *dec, fa_row_
 fa_status fa_decoder_prefill(fa_context *ctx, fa_decoder *dec, const int32_t *tokens, uint32_t l_new);
 /* Prompts of different lengths in one pass: tokens [batch, l_max] holds row b's
  * row_lens[b] prompt tokens followed by padding (any valid token id), row_lens
- * [batch] is a host array with 1 <= row_lens[b] <= l_max, batch * l_max <= 4096.
+ * [batch] is a host array with 1 <= row_lens[b] <= l_max, batch * l_max <= 4096;
+ * row b has pages for row_lens[b] tokens.
  * Every row ends as if it had been ingested alone with fa_decoder_prefill: its
  * length advances by row_lens[b], the logits and the next token are those of
  * its own last prompt token.  The padding is left out: nothing is computed for
