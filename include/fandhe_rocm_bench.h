@@ -87,8 +87,7 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  * key 18: 1 keeps the row kernels (norm, quantizer, norm + quantizer) of sixteen neighbouring elements per thread for every
  *        row count and width;
  * key 19: 1 keeps the norm + quantizer and quantizer kernels of a decode step as launches of their own for every batch
- *        size; 0: the linears that follow do that row work themselves where that measured faster (norm + quantizer: one
- *        or two rows, quantizer from partial maxima: one row); 2: wherever the kernels can (four / two rows); takes
+ *        size; 0: the linears that follow do that row work themselves where that measured faster (up to two rows); 2: wherever the kernels can (four / two rows); takes
  *        effect when a step is recorded;
  * key 20: 1 keeps the streamed attention with its merge launch for every decode step; 0: the attention runs as one
  *        launch while there is at most one (sequence, kv head) per compute unit and no share of a sequence is much longer
