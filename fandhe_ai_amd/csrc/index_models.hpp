@@ -94,6 +94,21 @@ struct BigLds {
     static constexpr int bytes = b_base + stages_b * b_stage;
 };
 
+// Tiles with room for five stages but not six, of which the weights take three and the rows two: the weights are what comes from
+// memory (a block's rows are read by every other column block and lie in the L2), so theirs are the requests to make earlier.  us on
+// 192 x 256, rows and weights ahead: int8 300 x 4096 -> 28672 50.2 and 45.6, bf16 experts' 3072 -> 2048 of 525 rows each 152 and
+// 137; 256 x 224, e4m3 2048 x 4096 -> 14336 99.0 and 96.6.  Tiles of 256 x 256 have so many rows to them that the rows come from
+// memory too: int8 8192 x 14336 -> 4096 360 and 375, so they keep three stages of rows.
+FA_HD bool big_b_ahead(int mtb, int ntb) { return big_stages_b(mtb, ntb) == kBigStagesB && mtb + ntb < 32; }
+template <int NTB, int MTB>
+struct BigSlots {
+    static constexpr bool b_ahead = big_b_ahead(MTB, NTB);
+    static constexpr int a = b_ahead ? 2 : kBigStagesA, b = b_ahead ? 3 : BigLds<NTB, MTB>::stages_b;
+    static constexpr int b_base = a * MTB * kBigTile, bytes = b_base + b * NTB * kBigTile;
+};
+template <int NTB, int MTB>
+FA_HD int big_b_slot_slice(int slot, int tile, int h) { return BigSlots<NTB, MTB>::b_base + slot * NTB * kBigTile + tile * kBigTile + h * 1024; }
+
 // Blocks of one XCD (the hardware deals consecutive ids round-robin over 8 XCDs) take consecutive tiles, m fastest.
 // With eight or more row blocks and a whole number of column blocks per XCD, an XCD walks its column blocks for eight
 // row blocks at a time: the 32 tiles its compute units hold together are then 8 x 4 (12 operand panels per k step)

@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     constexpr int TPWB = (NTB + NWAVES - 1) / NWAVES;        // weight tiles each wavefront moves per stage
     static_assert(MTB % WM == 0 && 2 * MTB % NWAVES == 0, "whole row tiles per wavefront, whole load instructions");
     constexpr int A_STAGE = MTB * TILE, B_STAGE = NTB * TILE;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [3][A_STAGE] then [2 or 3][B_STAGE]
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [2 or 3][A_STAGE] then [2 or 3][B_STAGE]
 
     constexpr bool SWI = std::is_same<Epi, EpiI8Swiglu>::value, ROPE = std::is_same<Epi, EpiI8QkvRope>::value;
     constexpr bool BF16 = IsBf16<Epi>::value;
@@ -504,8 +504,10 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     // LDS holds three stages of A and, on the wide tiles, two of B: A runs two stages ahead of the multiplies, B one, so
     // that requests stay in flight across the wait at the top of a stage (with both operands one stage ahead the path from
     // L2 runs dry there; a third stage of both does not fit).  The small tiles' stages are shorter than the way from L2
-    // (about 1900 cycles under load, which their stages took with B one stage ahead): there B has three too.
-    constexpr int NSA = 3, NSB = ixm::big_stages_b(MTB, NTB);
+    // (about 1900 cycles under load, which their stages took with B one stage ahead): there B has three too.  Tiles in between
+    // turn it round: B runs two stages ahead and A one (ixm::big_b_ahead).
+    using Slots = ixm::BigSlots<NTB, MTB>;
+    constexpr int NSA = Slots::a, NSB = Slots::b, DA = NSA - 1, DB = NSB - 1;      // stages ahead
     // Load instruction `idx` of a stage: tile wave + NWAVES (idx / 2), slice idx % 2.  They are spread over
     // the multiply groups of the stage before, which keeps a steady stream of requests going to the L2
     // instead of one burst per stage.
@@ -519,7 +521,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     auto issue_b = [&](uint32_t ks, int slot, int idx) {
         const int i = idx / 2, h = idx % 2;
         __builtin_amdgcn_global_load_lds((gptr)(b_src[i] + (uint64_t)ks * TILE + h * B_H),
-                                         (lptr)(lds + ixm::big_b_lds_slice<NTB, MTB>(slot, ixm::big_b_tile<NTB, NWAVES>(wave, i), h)), 16, 0, 0);
+                                         (lptr)(lds + ixm::big_b_slot_slice<NTB, MTB>(slot, ixm::big_b_tile<NTB, NWAVES>(wave, i), h)), 16, 0, 0);
     };
 
     typedef typename std::conditional<FP8 || BF16, v4f, v4i>::type acc_t;
@@ -538,33 +540,32 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
         if (ep.sx == nullptr) fscale = __fmul_rn(*ep.a_scale, *ep.w_scale);
     }
 
-    // Per stage a wavefront issues its B loads of stage ks + 1 first and its A loads of stage ks + 2 after
-    // them, so the wait at the top of stage ks + 1 can leave exactly those NLDA loads outstanding (three stages of B: both
+    // Per stage a wavefront issues the loads of the operand that runs one stage ahead first and those of stage ks + 2 after
+    // them, so the wait at the top of stage ks + 1 can leave exactly the latter outstanding (three stages of both: both
     // operands' loads of stage ks + 2).  Past
     // the end the loads are repeated from the last stage into slots nobody reads again, which keeps the
     // count of outstanding loads the same in every pass.
     const uint32_t last = ks_n - 1;                  // stages are counted from the block's first one
 #pragma unroll
-    for (int idx = 0; idx < NLDA; ++idx) issue_a(0, 0, idx);
+    for (int d = 0; d < 2; ++d) {
+        const uint32_t st = (uint32_t)d < last ? d : last;
 #pragma unroll
-    for (int idx = 0; idx < NLDB; ++idx) issue_b(0, 0, idx);
+        for (int idx = 0; idx < (d < DA ? NLDA : 0); ++idx) issue_a(st, d, idx);
 #pragma unroll
-    for (int idx = 0; idx < NLDA; ++idx) issue_a(last < 1 ? last : 1, 1, idx);
-    if constexpr (NSB == 3) {
-#pragma unroll
-        for (int idx = 0; idx < NLDB; ++idx) issue_b(last < 1 ? last : 1, 1, idx);
+        for (int idx = 0; idx < (d < DB ? NLDB : 0); ++idx) issue_b(st, d, idx);
     }
-    constexpr int AHEAD = NSB == 3 ? NLDA + NLDB : NLDA;      // loads of the stage after next that a wait leaves in flight
+    constexpr int AHEAD = (DA == 2 ? NLDA : 0) + (DB == 2 ? NLDB : 0);      // loads of the stage after next that a wait leaves in flight
+    static_assert((DA == 2 || DB == 2) && AHEAD <= 15, "four bits of the wait's immediate");
     // The barrier that opens stage ks + 1 sits before the last multiply group of stage ks, and the first
     // fragments of stage ks + 1 (all of A, the first of B) are read under that group: with the barrier
     // at the top of a stage every wavefront of the block would wait there for its first fragments at
     // the same time, with the matrix cores idle.  Per stage:
-    //   groups 0 .. WNT - 2: loads of B (stage ks + 1, or + 2) and A (stage ks + 2), B fragment j + 1, multiplies j
+    //   groups 0 .. WNT - 2: loads of A and B (stage ks + 1 or + 2), B fragment j + 1, multiplies j
     //   group WNT - 1: own reads of stage ks complete and own loads of stage ks + 1 landed, barrier,
     //                  multiplies interleaved with the A fragment reads of stage ks + 1, then its first B
     // The loads overwrite the buffers of stage ks - 1; they are issued after the barrier that opened
     // stage ks, which a wavefront reaches only after all its reads of stage ks - 1 have completed.
-    int slot_a = 0;
+    int slot_a = 0, slot_b = 0;
     // Fragment reads are written as assembly with their own lgkmcnt waits (lds_read16 / lds_wait above): left to
     // the compiler, every wait for a fragment becomes lgkmcnt(0), which also waits for the fragment of the NEXT
     // group that was issued a moment earlier, and the read-ahead is lost.  Addresses are LDS byte offsets.
@@ -591,19 +592,23 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     lds_read16<1024>(b[2][1], lb);
     uint32_t ks = 0;
     do {                                              // ks_n >= 1: the launcher sees to it
-        const int buf = ks % 2;
-        const uint32_t ks_b = ks + 1 < last ? ks + 1 : last, ks_a = ks + 2 < last ? ks + 2 : last;
-        const int slot_a2 = slot_a == 0 ? 2 : slot_a - 1;             // (slot_a + 2) % 3
+        const uint32_t ks_a = ks + DA < last ? ks + DA : last, ks_b = ks + DB < last ? ks + DB : last;
+        const int to_a = slot_a == 0 ? DA : slot_a - 1, to_b = slot_b == 0 ? DB : slot_b - 1;      // (slot_a + DA) % NSA, ...
         static_for<WNT>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
             {
-                // the load instructions over the first multiply groups, B before A
+                // the load instructions over the first multiply groups, those one stage ahead before those two ahead
                 constexpr int PER = (NLDA + NLDB + WNT - 3) / (WNT - 2);
 #pragma unroll
                 for (int q = 0; q < PER; ++q) {
                     const int idx = j * PER + q;
-                    if (idx < NLDB) issue_b(NSB == 3 ? ks_a : ks_b, NSB == 3 ? slot_a2 : buf ^ 1, idx);
-                    else if (idx < NLDB + NLDA) issue_a(ks_a, slot_a2, idx - NLDB);
+                    if (Slots::b_ahead) {
+                        if (idx < NLDA) issue_a(ks_a, to_a, idx);
+                        else if (idx < NLDA + NLDB) issue_b(ks_b, to_b, idx - NLDA);
+                    } else {
+                        if (idx < NLDB) issue_b(ks_b, to_b, idx);
+                        else if (idx < NLDB + NLDA) issue_a(ks_a, to_a, idx - NLDB);
+                    }
                 }
             }
             constexpr int cur = j == 0 ? 2 : (j - 1) % 2, nxt = j % 2;   // sets of group j and of group j + 1
@@ -619,10 +624,11 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
                 __builtin_amdgcn_s_waitcnt(0x0070 | AHEAD);
                 lds_wait<0>(b[cur][0], b[cur][1]);    // no instruction: ties the fragment to the wait above
                 __builtin_amdgcn_s_barrier();         // stage ks + 1 visible to all; stage ks no longer read
-                slot_a = slot_a == 2 ? 0 : slot_a + 1;
+                slot_a = slot_a == DA ? 0 : slot_a + 1;
+                slot_b = slot_b == DB ? 0 : slot_b + 1;
                 la[0] = la_lane[0] + slot_a * A_STAGE;
                 la[1] = la_lane[1] + slot_a * A_STAGE;
-                lb = lb_lane + (NSB == 3 ? slot_a : buf ^ 1) * B_STAGE;
+                lb = lb_lane + slot_b * B_STAGE;
                 lds_read16<0>(b[2][0], lb);           // fragment 0 of the next stage (set 2 was last used by group 0)
                 lds_read16<1024>(b[2][1], lb);
             }
@@ -1075,7 +1081,7 @@ void allow_lds(F f, size_t bytes) {
 template <bool FP8, int NTB, int WM, int MTB, typename Epi>
 void launch_big_tile(const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, uint32_t n_blocks,
                      unsigned grid, const Epi &e, hipStream_t s) {
-    constexpr size_t smem = ixm::BigLds<NTB, MTB>::bytes;
+    constexpr size_t smem = ixm::BigSlots<NTB, MTB>::bytes;
     static bool configured = false;
     if (!configured) allow_lds(&gemm_mfma_big_kernel<FP8, NTB, WM, Epi, MTB>, smem);
     configured = true;

@@ -382,6 +382,40 @@ static void stage_ring_case(int nsb) {
     }
 }
 
+// Where the stages of A and B lie, and that a stage's loads meet no slot that is still read: a block's passes over ks_n stages, with
+// what has landed when a wait leaves the loads of the operand two stages ahead (the kernel's order: one stage ahead first).
+template <int NTB, int MTB>
+static void slots_case() {
+    using S = BigSlots<NTB, MTB>;
+    using L = BigLds<NTB, MTB>;
+    static_assert(S::bytes <= 160 * 1024 && S::b_base == S::a * L::a_stage && S::bytes == S::b_base + S::b * L::b_stage, "one behind the other");
+    for (int slot = 0; slot < S::b; ++slot)
+        for (int tile = 0; tile < NTB; ++tile)
+            for (int h = 0; h < 2; ++h) {
+                const int at = big_b_slot_slice<NTB, MTB>(slot, tile, h);
+                CHECK(at == S::b_base + slot * L::b_stage + tile * kBigTile + h * 1024);
+                CHECK(at + 1024 <= S::bytes);
+                if (!S::b_ahead) CHECK((at == big_b_lds_slice<NTB, MTB>(slot, tile, h)));
+            }
+    constexpr int DA = S::a - 1, DB = S::b - 1;
+    for (int ks_n = 1; ks_n <= 9; ++ks_n) {
+        const int last = ks_n - 1;
+        std::vector<int> a(S::a, -1), b(S::b, -1);
+        for (int d = 0; d < DA; ++d) a[d] = d < last ? d : last;
+        for (int d = 0; d < DB; ++d) b[d] = d < last ? d : last;
+        int sa = 0, sb = 0;
+        for (int ks = 0; ks < ks_n; ++ks) {
+            CHECK(a[sa] == ks && b[sb] == ks);
+            const int to_a = sa == 0 ? DA : sa - 1, to_b = sb == 0 ? DB : sb - 1;
+            CHECK(to_a == (sa + DA) % S::a && to_b == (sb + DB) % S::b && to_a != sa && to_b != sb);
+            a[to_a] = ks + DA < last ? ks + DA : last;
+            b[to_b] = ks + DB < last ? ks + DB : last;
+            sa = sa == DA ? 0 : sa + 1;
+            sb = sb == DB ? 0 : sb + 1;
+        }
+    }
+}
+
 template <bool FP8>
 static void gemm_cases() {
     gemm_case<FP8, 16, 4, 16>();
@@ -396,6 +430,15 @@ static void gemm_cases() {
     gemm_case<FP8, 16, 2>();
     gemm_case<FP8, 14, 8>();
     gemm_case<FP8, 16, 8>();
+    slots_case<16, 16>();
+    slots_case<16, 12>();
+    slots_case<16, 8>();
+    slots_case<14, 16>();
+    slots_case<14, 12>();
+    slots_case<8, 16>();
+    slots_case<8, 12>();
+    slots_case<8, 8>();
+    static_assert(BigSlots<16, 12>::b_ahead && BigSlots<14, 16>::b_ahead && !BigSlots<16, 16>::b_ahead && !BigSlots<14, 12>::b_ahead, "the tiles in between");
 }
 
 // Row quantizer: codes around every middle of two codes are those of the division, for every 64th mantissa of the scale (with an
