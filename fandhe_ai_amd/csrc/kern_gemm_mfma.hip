@@ -556,6 +556,38 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     }
     constexpr int AHEAD = (DA == 2 ? NLDA : 0) + (DB == 2 ? NLDB : 0);      // loads of the stage after next that a wait leaves in flight
     static_assert((DA == 2 || DB == 2) && AHEAD <= 15, "four bits of the wait's immediate");
+    // Wavefronts whose rows all lie at or past m move their share of the tiles and multiply nothing.  (The last row block of a
+    // matrix or of a group; the part runs these kernels at its power limit, so what they multiplied cost the other blocks too.)
+    const bool idle = m0 + wm * AI * 16 >= m;
+    constexpr int PER = (NLDA + NLDB + WNT - 3) / (WNT - 2);      // load instructions per multiply group, over the first groups
+    // load instruction idx of a pass, those one stage ahead before those two ahead
+    auto issue = [&](uint32_t ks_a, uint32_t ks_b, int to_a, int to_b, int idx) {
+        if (Slots::b_ahead) {
+            if (idx < NLDA) issue_a(ks_a, to_a, idx);
+            else if (idx < NLDA + NLDB) issue_b(ks_b, to_b, idx - NLDA);
+        } else {
+            if (idx < NLDB) issue_b(ks_b, to_b, idx);
+            else if (idx < NLDB + NLDA) issue_a(ks_a, to_a, idx - NLDB);
+        }
+    };
+    int slot_a = 0, slot_b = 0;
+    uint32_t ks = 0;
+    if (idle) {
+        __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);
+        __builtin_amdgcn_s_barrier();
+        do {
+            const uint32_t ks_a = ks + DA < last ? ks + DA : last, ks_b = ks + DB < last ? ks + DB : last;
+            const int to_a = slot_a == 0 ? DA : slot_a - 1, to_b = slot_b == 0 ? DB : slot_b - 1;
+#pragma unroll
+            for (int idx = 0; idx < NLDA + NLDB; ++idx) issue(ks_a, ks_b, to_a, to_b, idx);
+            __builtin_amdgcn_s_waitcnt(0x0F70 | AHEAD);
+            __builtin_amdgcn_s_barrier();
+            slot_a = slot_a == DA ? 0 : slot_a + 1;
+            slot_b = slot_b == DB ? 0 : slot_b + 1;
+        } while (++ks < ks_n);
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        if constexpr (!SPLIT) return;
+    } else {
     // The barrier that opens stage ks + 1 sits before the last multiply group of stage ks, and the first
     // fragments of stage ks + 1 (all of A, the first of B) are read under that group: with the barrier
     // at the top of a stage every wavefront of the block would wait there for its first fragments at
@@ -565,7 +597,6 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     //                  multiplies interleaved with the A fragment reads of stage ks + 1, then its first B
     // The loads overwrite the buffers of stage ks - 1; they are issued after the barrier that opened
     // stage ks, which a wavefront reaches only after all its reads of stage ks - 1 have completed.
-    int slot_a = 0, slot_b = 0;
     // Fragment reads are written as assembly with their own lgkmcnt waits (lds_read16 / lds_wait above): left to
     // the compiler, every wait for a fragment becomes lgkmcnt(0), which also waits for the fragment of the NEXT
     // group that was issued a moment earlier, and the read-ahead is lost.  Addresses are LDS byte offsets.
@@ -590,26 +621,14 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     });
     lds_read16<0>(b[2][0], lb);
     lds_read16<1024>(b[2][1], lb);
-    uint32_t ks = 0;
     do {                                              // ks_n >= 1: the launcher sees to it
         const uint32_t ks_a = ks + DA < last ? ks + DA : last, ks_b = ks + DB < last ? ks + DB : last;
         const int to_a = slot_a == 0 ? DA : slot_a - 1, to_b = slot_b == 0 ? DB : slot_b - 1;      // (slot_a + DA) % NSA, ...
         static_for<WNT>([&](auto jc) {
             constexpr int j = decltype(jc)::value;
             {
-                // the load instructions over the first multiply groups, those one stage ahead before those two ahead
-                constexpr int PER = (NLDA + NLDB + WNT - 3) / (WNT - 2);
 #pragma unroll
-                for (int q = 0; q < PER; ++q) {
-                    const int idx = j * PER + q;
-                    if (Slots::b_ahead) {
-                        if (idx < NLDA) issue_a(ks_a, to_a, idx);
-                        else if (idx < NLDA + NLDB) issue_b(ks_b, to_b, idx - NLDA);
-                    } else {
-                        if (idx < NLDB) issue_b(ks_b, to_b, idx);
-                        else if (idx < NLDB + NLDA) issue_a(ks_a, to_a, idx - NLDB);
-                    }
-                }
+                for (int q = 0; q < PER; ++q) issue(ks_a, ks_b, to_a, to_b, j * PER + q);
             }
             constexpr int cur = j == 0 ? 2 : (j - 1) % 2, nxt = j % 2;   // sets of group j and of group j + 1
             constexpr bool tail = j + 1 == WNT;
@@ -669,6 +688,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
     for (int i = 0; i < AI; ++i) drain_row(acc[i]);
     __builtin_amdgcn_s_waitcnt(0x0F70);               // the repeated loads of the tail have landed too
+    }
 
     if constexpr (SPLIT) {
         // raw sums of this half of k: word (i, j, e) of thread t at [(i * WNT + j) * 4 + e][t], 2 KiB per store
@@ -676,6 +696,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
         const uint32_t S = ep.split_s;
         int32_t *mine = ep.split_partial + ((uint64_t)tile_id * S + half) * ((uint64_t)WORDS * 128 * WM);
         const bool local = ep.split_local != 0;
+        if (!idle) {
 #pragma unroll
         for (int i = 0; i < AI; ++i)
 #pragma unroll
@@ -686,6 +707,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
                     if (local) __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     else __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
+        }
         __builtin_amdgcn_s_waitcnt(0);            // this thread's stores are acknowledged
         __syncthreads();                          // ... and everybody's; nobody reads the stages any more
         uint32_t *slot = (uint32_t *)lds;
@@ -700,7 +722,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
             *slot = t;
         }
         __syncthreads();
-        if (*slot != S - 1) return;               // a partner finishes the tile
+        if (*slot != S - 1 || idle) return;       // a partner finishes the tile
         for (uint32_t r = 0; r < S; ++r) {
             if (r == half) continue;
             const int32_t *other = ep.split_partial + ((uint64_t)tile_id * S + r) * ((uint64_t)WORDS * 128 * WM);
