@@ -510,16 +510,17 @@ __device__ __forceinline__ v4f mfma4(const v4f &a, const v4f &b, v4f c) {
 }
 
 // silu(convolution) of `cols` channels from c0 on for the chunk's tokens t0 .. into dst [32][pitch]; zeros for tokens past
-// the end and columns up to cols_p.  A thread takes TG tokens of two neighbouring channels (one where they are not aligned).
+// the end and columns up to cols_p.  A thread takes TG tokens of two neighbouring channels (one where they are not aligned); threads
+// `first` .. first + NT - 1 of the block.
 template <typename T, int MAXTAPS, int TG, int NT = 256>
 __device__ __forceinline__ void conv_chunk(float *dst, uint32_t pitch, const T *__restrict__ y, uint32_t ld, const T *__restrict__ ring,
                                            const float *__restrict__ conv, uint32_t taps, uint32_t channels, uint32_t c0, uint32_t cols,
-                                           uint32_t cols_p, uint64_t row0, uint32_t t0, uint32_t n, uint32_t p0) {
+                                           uint32_t cols_p, uint64_t row0, uint32_t t0, uint32_t n, uint32_t p0, uint32_t first = 0) {
     constexpr uint32_t NG = kChunk / TG;
     if (MAXTAPS != 0 && ((ld | channels | c0 | cols) & 1) == 0) {
         constexpr int NX = TG + (MAXTAPS ? MAXTAPS : 1) - 1, MT = MAXTAPS ? MAXTAPS : 1;
         const uint32_t pairs = cols_p / 2;
-        for (uint32_t item = threadIdx.x; item < pairs * NG; item += NT) {
+        for (uint32_t item = threadIdx.x - first; item < pairs * NG; item += NT) {
             const uint32_t col = item % pairs * 2, tg = item / pairs * TG;
             const uint32_t c = c0 + (col < cols ? col : 0);
             v2f w[MT], x[NX];
@@ -557,7 +558,7 @@ __device__ __forceinline__ void conv_chunk(float *dst, uint32_t pitch, const T *
         }
         return;
     }
-    for (uint32_t item = threadIdx.x; item < cols_p * NG; item += NT) {
+    for (uint32_t item = threadIdx.x - first; item < cols_p * NG; item += NT) {
         const uint32_t col = item % cols_p, tg = item / cols_p * TG;
         for (uint32_t j = 0; j < TG; ++j) {
             const uint32_t t = t0 + tg + j;
@@ -567,7 +568,7 @@ __device__ __forceinline__ void conv_chunk(float *dst, uint32_t pitch, const T *
 }
 
 // lt = T = (I + A)^-1 for the strictly lower A in la (pitch 36), by one wavefront: the diagonal blocks column by column (lanes
-// 0 - 15, 16 - 31), then T10 = -T11 A10 T00.
+// 0 - 15, 16 - 31), then T10 = -T11 A10 T00.  lt may be la: a row of A is read in front of T's, and not again.
 __device__ __forceinline__ void invert_unit_lower(const float *la, float *lt, int lane) {
     const int lr = lane % 16, g = lane / 16;
     if (lane < 32) {
@@ -620,15 +621,24 @@ __device__ __forceinline__ v4f value_tile(const v4f (&tf)[2][2], const float *lv
     return acc;
 }
 
+// Columns of V that a block of delta_chunk_kernel takes at a time, in the place of Q, and its LDS.
+constexpr int chunk_v_cols(int kt) { return kt < 4 ? 64 : kt * 16; }
+constexpr size_t chunk_lds_bytes(int kt) { return (32 * (kt * 16 + 4) + 32 * (chunk_v_cols(kt) + 4) + 32 * 36) * 4; }
+
 // One block per (chunk, q / k head); the heads that share it are taken one after the other.
+// A block is a chain (convolutions, norms and products, decays, A, its inverse, W and T V), so the time is the chain's and the number of blocks that
+// run beside each other: V takes the place of Q, the inverse that of A, so that heads of 128 leave four to a compute unit, and one wavefront
+// inverts while the other three bring V.  2048 tokens, 32 heads of 128 x 128, 16 of q and k (a floor of 27 us for the fragments it writes):
+// 96 us with three blocks to a unit, V in a place of its own 64 columns at a time and the heads' steps one by one, 71 so.
 template <typename T, int KT, int MAXTAPS>
 __global__ void __launch_bounds__(256)
     delta_chunk_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, float *__restrict__ frags, float *__restrict__ chunk_decay, uint32_t n_frags) {
-    constexpr uint32_t DP = KT * 16, PITCH = DP + 4, VS = 64, VPITCH = VS + 4;
+    constexpr uint32_t DP = KT * 16, PITCH = DP + 4, VS = chunk_v_cols(KT), VPITCH = VS + 4;
+    static_assert(VPITCH >= PITCH, "Q and V share their place");
     extern __shared__ __attribute__((aligned(16))) float lds[];
-    float *lk = lds, *lq = lk + 32 * PITCH, *lv = lq + 32 * PITCH;          // K, Q, 64 columns of V
-    float *la = lv + 32 * VPITCH, *lt = la + 32 * 36;                       // A and T, pitch 36
-    __shared__ float rq[32], rk[32], beta[32], G[32], qs[32], ks[32], ke[32];   // qs = rq exp(G), ks = rk exp(G), ke = rk exp(G_C - G)
+    float *lk = lds, *lq = lk + 32 * PITCH, *lv = lq, *la = lv + 32 * VPITCH;      // K, Q, then columns of V, A, then T (pitch 36)
+    __shared__ float rq[32], rk[32];
+    __shared__ float beta[2][32], G[2][32], qs[2][32], ks[2][32], ke[2][32];        // of two heads: qs = rq exp(G), ks = rk exp(G), ke = rk exp(G_C - G)
     // the slot's sequence and chunk
     uint32_t lo = 0, hi = rr.batch;
     while (hi - lo > 1) {
@@ -645,6 +655,33 @@ __global__ void __launch_bounds__(256)
 
     conv_chunk<T, MAXTAPS, 8>(lq, PITCH, y, io.ld_y, ring, io.conv, sh.taps, channels, hk * dim, dim, DP, row0, t0, n, p0);
     conv_chunk<T, MAXTAPS, 8>(lk, PITCH, y, io.ld_y, ring, io.conv, sh.taps, channels, (sh.kv_heads + hk) * dim, dim, DP, row0, t0, n, p0);
+    // decays and beta of heads h0, h0 + 1 (a lane to a token, half a wavefront to a head)
+    float lg = 0.0f, be = 0.0f;
+    auto request = [&](uint32_t h0) {
+        const uint32_t t = t0 + lane % 32, h = h0 + lane / 32;
+        lg = be = 0.0f;
+        if (tid < 64 && t < n && h < (hk + 1) * share) {
+            be = sigmoid_f32(io.beta[(uint64_t)(row0 + t) * io.ld_beta + h]);
+            lg = log_decay(io.a_log[h], io.decay[(uint64_t)(row0 + t) * io.ld_decay + h] + io.dt_bias[h]);
+        }
+    };
+    auto scalars = [&](uint32_t h0) {
+        if (tid >= 64) return;
+        const int t = lane % 32, x = lane / 32;
+#pragma unroll
+        for (int off = 1; off < 32; off <<= 1) {
+            const float o = __shfl_up(lg, off, 32);
+            if (t >= off) lg += o;
+        }
+        const float last = __shfl(lg, 31, 32);
+        beta[x][t] = be;
+        G[x][t] = lg;
+        qs[x][t] = rq[t] * expf(lg);
+        ks[x][t] = rk[t] * expf(lg);
+        ke[x][t] = rk[t] * expf(last - lg);
+        if (t == 31 && h0 + x < (hk + 1) * share) chunk_decay[(uint64_t)blockIdx.x * sh.heads + h0 + x] = expf(lg);
+    };
+    request(hk * share);
     __syncthreads();
     {   // four threads per row of Q and of K
         const float *row = (tid < 128 ? lq : lk) + ((tid % 128) / 4) * PITCH;
@@ -672,76 +709,69 @@ __global__ void __launch_bounds__(256)
     v4f kk = v4f{0.f, 0.f, 0.f, 0.f}, qk = kk;
     if (wave != 2) kk = dot_tile(lk + tj * 16 * PITCH, lk + ti * 16 * PITCH);
     if (wave != 1) qk = dot_tile(lk + tj * 16 * PITCH, lq + ti * 16 * PITCH);
+    auto place = [&](uint32_t h) { return (v4f *)(frags + ((uint64_t)blockIdx.x * sh.heads + h) * n_frags * 256) + lane; };
 
-    for (uint32_t h = hk * share; h < (hk + 1) * share; ++h) {
-        v4f *out = (v4f *)(frags + ((uint64_t)blockIdx.x * sh.heads + h) * n_frags * 256) + lane;
-        auto put = [&](uint32_t f, const v4f &v) { out[f * 64] = v; };
-        __syncthreads();                             // norms are there; the previous head's scalars and A, T, V are read
-        if (tid < 64) {                              // lanes past 31 only keep the scan whole
-            const uint32_t t = t0 + lane;
-            float lg = 0.0f, be = 0.0f;
-            if (lane < 32 && t < n) {
-                be = sigmoid_f32(io.beta[(uint64_t)(row0 + t) * io.ld_beta + h]);
-                lg = log_decay(io.a_log[h], io.decay[(uint64_t)(row0 + t) * io.ld_decay + h] + io.dt_bias[h]);
-            }
+    // what needs Q, for all heads: P, exp(G) Q; and the decayed K^T
+    for (uint32_t h0 = hk * share; h0 < (hk + 1) * share; h0 += 2) {
+        if (h0 != hk * share) request(h0);
+        __syncthreads();                             // norms are there; the scalars before are read
+        scalars(h0);
+        __syncthreads();
+        for (uint32_t x = 0; x < 2 && h0 + x < (hk + 1) * share; ++x) {
+            v4f *out = place(h0 + x);
+            if (wave != 1) {
+                v4f d;
 #pragma unroll
-            for (int off = 1; off < 32; off <<= 1) {
-                const float o = __shfl_up(lg, off, 64);
-                if (lane >= off) lg += o;
+                for (int e = 0; e < 4; ++e) {
+                    const int j = tj * 16 + 4 * g + e;
+                    d[e] = j <= i_ ? fast_exp(G[x][i_] - G[x][j]) * rq[i_] * rk[j] * qk[e] : 0.0f;
+                }
+                out[(6 * KT + ti + tj) * 64] = d;
             }
-            const float last = __shfl(lg, 31, 64);
-            if (lane < 32) {
-                beta[lane] = be;
-                G[lane] = lg;
-                qs[lane] = rq[lane] * expf(lg);
-                ks[lane] = rk[lane] * expf(lg);
-                ke[lane] = rk[lane] * expf(last - lg);
+            for (uint32_t f = wave; f < 2 * KT; f += 4) {
+                const uint32_t rt = f / KT, kt = f % KT, i = rt * 16 + lr;
+                out[(2 * KT + f) * 64] = *(const v4f *)(lq + i * PITCH + kt * 16 + 4 * g) * qs[x][i];
+                const uint32_t dt = f / 2, ct = f % 2;
+                v4f v;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t j = ct * 16 + 4 * g + e;
+                    v[e] = lk[j * PITCH + dt * 16 + lr] * ke[x][j];
+                }
+                out[(4 * KT + f) * 64] = v;
             }
         }
-        __syncthreads();
+    }
+    for (uint32_t h = hk * share; h < (hk + 1) * share; ++h) {
+        const uint32_t x = (h - hk * share) % 2;
+        if (share > 2 && x == 0) {                   // the scalars are the last two heads'
+            request(h);
+            __syncthreads();
+            scalars(h);
+            __syncthreads();
+        }
+        v4f *out = place(h);
+        // A: its place and that of V are free behind the barriers that close a head and, for the first one, the loop above
         if (wave != 2) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int j = tj * 16 + 4 * g + e;
-                la[i_ * 36 + j] = j < i_ ? beta[i_] * fast_exp(G[i_] - G[j]) * rk[i_] * rk[j] * kk[e] : 0.0f;
+                la[i_ * 36 + j] = j < i_ ? beta[x][i_] * fast_exp(G[x][i_] - G[x][j]) * rk[i_] * rk[j] * kk[e] : 0.0f;
             }
         }
-        if (wave != 1) {
-            v4f d;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int j = tj * 16 + 4 * g + e;
-                d[e] = j <= i_ ? fast_exp(G[i_] - G[j]) * rq[i_] * rk[j] * qk[e] : 0.0f;
-            }
-            put(6 * KT + ti + tj, d);
-        }
-        // exp(G) Q and the decayed K^T
-        for (uint32_t f = wave; f < 2 * KT; f += 4) {
-            const uint32_t rt = f / KT, kt = f % KT, i = rt * 16 + lr;
-            put(2 * KT + f, *(const v4f *)(lq + i * PITCH + kt * 16 + 4 * g) * qs[i]);
-            const uint32_t dt = f / 2, ct = f % 2;
-            v4f v;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t j = ct * 16 + 4 * g + e;
-                v[e] = lk[j * PITCH + dt * 16 + lr] * ke[j];
-            }
-            put(4 * KT + f, v);
-        }
-        if (tid == 0) chunk_decay[(uint64_t)blockIdx.x * sh.heads + h] = expf(G[31]);
-        // the first columns of V, whose loads travel under the inversion
         const uint32_t vc0 = 2 * sh.kv_heads * dim + h * vdim;
-        auto conv_v = [&](uint32_t v0) {
+        auto conv_v = [&](uint32_t v0, auto nt) {
+            constexpr int NT = decltype(nt)::value;
             const uint32_t cols = vdim - v0 < VS ? vdim - v0 : VS;
-            conv_chunk<T, MAXTAPS, 4>(lv, VPITCH, y, io.ld_y, ring, io.conv, sh.taps, channels, vc0 + v0, cols, (cols + 15) / 16 * 16, row0, t0, n, p0);
+            conv_chunk<T, MAXTAPS, 4, NT>(lv, VPITCH, y, io.ld_y, ring, io.conv, sh.taps, channels, vc0 + v0, cols, (cols + 15) / 16 * 16, row0, t0, n, p0, 256 - NT);
         };
-        conv_v(0);
         __syncthreads();
-        if (wave == 0) invert_unit_lower(la, lt, lane);
+        if (wave == 0) invert_unit_lower(la, la, lane);
+        else conv_v(0, std::integral_constant<int, 192>{});
         __syncthreads();
         // -W^T = -K'^T T^T, K' = diag(beta exp(G) rk) K: the columns of the result are tokens, so its D order is W's A order
         v4f tf[2][2];
-        load_scaled_inverse(tf, lt, beta, lr, g);
+        load_scaled_inverse(tf, la, beta[x], lr, g);
         for (uint32_t f = wave; f < 2 * KT; f += 4) {
             const uint32_t rt = f / KT, kt = f % KT;
             v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
@@ -750,25 +780,26 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const uint32_t j = ct * 16 + 4 * g + e;
-                    kf[e] = -lk[j * PITCH + kt * 16 + lr] * ks[j];
+                    kf[e] = -lk[j * PITCH + kt * 16 + lr] * ks[x][j];
                 }
                 acc = mfma4(kf, rt == 0 ? tf[0][0] : ct == 0 ? tf[1][0] : tf[1][1], acc);
             }
-            put(f, acc);
+            out[f * 64] = acc;
         }
         // T diag(beta) V
         for (uint32_t v0 = 0; v0 < vdim; v0 += VS) {
             if (v0) {
                 __syncthreads();
-                conv_v(v0);
+                conv_v(v0, std::integral_constant<int, 256>{});
                 __syncthreads();
             }
             const uint32_t tiles = ((vdim - v0 < VS ? vdim - v0 : VS) + 15) / 16;
             for (uint32_t f = wave; f < 2 * tiles; f += 4) {
                 const uint32_t rt = f % 2, nt = f / 2;
-                put(6 * KT + 3 + (v0 / 16 + nt) * 2 + rt, value_tile(tf, lv, VPITCH, rt, nt, lr, g));
+                out[(6 * KT + 3 + (v0 / 16 + nt) * 2 + rt) * 64] = value_tile(tf, lv, VPITCH, rt, nt, lr, g);
             }
         }
+        __syncthreads();                             // T and V are read
     }
 }
 
@@ -1163,6 +1194,20 @@ __global__ void __launch_bounds__(512)
         }
 }
 
+// Loads and stores at base + scalar + lane_at bytes: nothing of an address is formed anew in vector registers
+__device__ __forceinline__ v4f load_fragment(const float *base, uint32_t lane_at, uint32_t scalar) {
+    const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
+    return __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(all, lane_at, scalar, 0));
+}
+__device__ __forceinline__ float load_word(const float *base, uint32_t lane_at, uint32_t scalar) {
+    const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(all, lane_at, scalar, 0));
+}
+__device__ __forceinline__ void store_word(float *base, uint32_t lane_at, float v) {
+    const __amdgpu_buffer_rsrc_t all = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), all, lane_at, 0, 0);
+}
+
 // Wavefronts that share the rows of a state's 16 columns in delta_scan_split_kernel.
 constexpr int scan_waves(int kt) { return kt >= 16 ? 8 : kt >= 4 ? 4 : kt; }
 
@@ -1171,8 +1216,11 @@ constexpr int scan_waves(int kt) { return kt >= 16 ? 8 : kt >= 4 ? 4 : kt; }
 // KT / waves row tiles of the state each.  A chunk is: every wavefront's share of W S_0 and exp(G) Q S_0 over its own rows, the
 // shares exchanged through LDS (one barrier), the writes U whole in every wavefront, every wavefront's own rows of the state; the
 // first two also form a half of the read-outs each.  A wavefront alone reads its rows' fragments: they go from memory to
-// registers, a chunk ahead.  Measured, 32 heads 128 x 128: 2048 tokens of one sequence 330 -> 130 us (of two 335 -> 270); with
-// four sequences (1024 tiles, four per compute unit) the exchanges cost more than the idle cores: 10 % slower than the form above.
+// registers, a chunk ahead, by loads whose addresses take no vector instruction (with 64-bit ones formed for each, and decays by scalar
+// loads, which LDS reads are waited for with, 113 us where it is 106 now).  Measured, 32 heads 128 x 128: 2048 tokens of one sequence 330 us in the
+// form above and 106 here (of two 335 and 270); with four sequences (1024 tiles, four per compute unit) the exchanges cost more than the
+// idle cores: 10 % slower than the form above.  Of a chunk's 1.65 us the 48 to 56 multiplies are 0.7, the LDS reads of the shares 0.3, fragments 0.15, the
+// stores of the read-outs 0.15; read-outs in wavefronts of their own (eight to a block, the state through LDS) made it 124 us.
 template <int KT, Recurrence KIND>
 __global__ void __launch_bounds__(scan_waves(KT) * 64)
     delta_scan_split_kernel(DeltaShape sh, DeltaIo io, RaggedRows rr, const float *__restrict__ frags, const float *__restrict__ chunk_decay,
@@ -1186,8 +1234,41 @@ __global__ void __launch_bounds__(scan_waves(KT) * 64)
     const uint32_t row0 = rr.row_start[b], n = rr.row_start[b + 1] - row0;
     if (n < kChunkFrom || h >= sh.heads) return;
     const uint32_t dim = sh.dim, vp = sh.vdim_p(), col = nt * 16 + lr, slot0 = slot_base(rr, b), vdim = sh.vdim;
+    const uint32_t chunks = (n + kChunk - 1) / kChunk, lane16 = lane * 16;
     float *state = io.state + ((uint64_t)rr.state_slot[b] * sh.heads + h) * dim * vp;
     const bool fresh = rr.pos[row0] == 0;
+    struct Fragments {
+        v4f w[KW][2], q[KW][2], k[KW][2], d[KW], p[3], v[2];
+        float decay;
+    };
+    const bool first = wave == 0, second = NW == 1 || wave == 1;     // read-outs of the chunk's first, second 16 tokens
+    auto read = [&](uint32_t c, Fragments &f) {
+        c = slot0 + (c < chunks ? c : chunks - 1);
+        const float *src = frags + ((uint64_t)c * sh.heads + h) * n_frags * 256;
+#pragma unroll
+        for (int kt = 0; kt < KW; ++kt)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if constexpr (!LIGHTNING) f.w[kt][t] = load_fragment(src, lane16, (t * KT + wave * KW + kt) * 1024);
+                f.q[kt][t] = load_fragment(src, lane16, (FQ + t * KT + wave * KW + kt) * 1024);
+            }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) f.v[t] = load_fragment(src, lane16, (SHARED + nt * 2 + t) * 1024);
+        if constexpr (!CHANNEL) f.decay = load_word(chunk_decay + (uint64_t)c * sh.heads, 0, h * 4);
+#pragma unroll
+        for (int kt = 0; kt < KW; ++kt) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) f.k[kt][t] = load_fragment(src, lane16, (FK + (wave * KW + kt) * 2 + t) * 1024);
+            if constexpr (CHANNEL) f.d[kt] = load_fragment(src, g * 16, (FP + 3) * 1024 + (wave * KW + kt) * 64);
+        }
+        if (first) f.p[0] = load_fragment(src, lane16, FP * 1024);
+        if (second) {
+            f.p[1] = load_fragment(src, lane16, (FP + 1) * 1024);
+            f.p[2] = load_fragment(src, lane16, (FP + 2) * 1024);
+        }
+    };
+    Fragments even, odd;
+    read(0, even);
     v4f S[KW];
 #pragma unroll
     for (int kt = 0; kt < KW; ++kt)
@@ -1196,39 +1277,10 @@ __global__ void __launch_bounds__(scan_waves(KT) * 64)
             const uint32_t d = (wave * KW + kt) * 16 + 4 * g + e;
             S[kt][e] = !fresh && d < dim && col < vdim ? state[(uint64_t)d * vp + col] : 0.0f;
         }
-    struct Fragments {
-        v4f w[KW][2], q[KW][2], k[KW][2], d[KW], p[3], v[2];
-        float decay;
-    };
-    const bool first = wave == 0, second = NW == 1 || wave == 1;     // read-outs of the chunk's first, second 16 tokens
-    auto read = [&](uint32_t c, Fragments &f) {
-        const v4f *src = (const v4f *)(frags + ((uint64_t)(slot0 + c) * sh.heads + h) * n_frags * 256) + lane;
-#pragma unroll
-        for (int kt = 0; kt < KW; ++kt)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                if constexpr (!LIGHTNING) f.w[kt][t] = src[(t * KT + wave * KW + kt) * 64];
-                f.q[kt][t] = src[(FQ + t * KT + wave * KW + kt) * 64];
-            }
-        f.v[0] = src[(SHARED + nt * 2) * 64];
-        f.v[1] = src[(SHARED + nt * 2 + 1) * 64];
-#pragma unroll
-        for (int kt = 0; kt < KW; ++kt) {
-            f.k[kt][0] = src[(FK + (wave * KW + kt) * 2) * 64];
-            f.k[kt][1] = src[(FK + (wave * KW + kt) * 2 + 1) * 64];
-            if constexpr (CHANNEL) f.d[kt] = (src - lane + (FP + 3) * 64)[(wave * KW + kt) * 4 + g];
-        }
-        if constexpr (!CHANNEL) f.decay = chunk_decay[(uint64_t)(slot0 + c) * sh.heads + h];
-        if (first) f.p[0] = src[FP * 64];
-        if (second) {
-            f.p[1] = src[(FP + 1) * 64];
-            f.p[2] = src[(FP + 2) * 64];
-        }
-    };
-    const uint32_t chunks = (n + kChunk - 1) / kChunk;
     const v4f zero = v4f{0.f, 0.f, 0.f, 0.f};
+    const uint32_t own_row = (4 * g * sh.heads * vdim + col) * 4;
     auto chunk = [&](uint32_t c, const Fragments &f, Fragments &next) {
-        read(c + 1 < chunks ? c + 1 : c, next);
+        read(c + 1, next);
         __builtin_amdgcn_sched_barrier(0);           // asked for ahead of everything else
         v4f x[4] = {zero, zero, zero, zero};
 #pragma unroll
@@ -1262,17 +1314,15 @@ __global__ void __launch_bounds__(scan_waves(KT) * 64)
 #pragma unroll
                 for (int kt = 0; kt < KW; ++kt) S[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.k[kt][t][e], u[t][e], S[kt], 0, 0, 0);
         auto store = [&](int t, const v4f &r) {
+            float *dst = o + ((uint64_t)(row0 + c * kChunk + t * 16) * sh.heads + h) * vdim;
+            const int32_t left = (int32_t)(n - c * kChunk) - t * 16;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t at = c * kChunk + t * 16 + 4 * g + e;
-                if (at < n && col < vdim) o[((uint64_t)(row0 + at) * sh.heads + h) * vdim + col] = r[e];
-            }
+            for (int e = 0; e < 4; ++e)
+                if (left > 4 * g + e && col < vdim) store_word(dst, own_row + e * sh.heads * vdim * 4, r[e]);
         };
         if (first) store(0, mfma4(f.p[0], u[0], sum(2, zero)));
         if (second) store(1, mfma4(f.p[2], u[1], mfma4(f.p[1], u[0], sum(3, zero))));
     };
-    Fragments even, odd;
-    read(0, even);
     for (uint32_t c = 0; c < chunks; c += 2) {
         chunk(c, even, odd);
         if (c + 1 < chunks) chunk(c + 1, odd, even);
@@ -1379,7 +1429,8 @@ void allow_lds(F f, size_t bytes) {
 template <typename T, int KT, Recurrence KIND>
 void launch_chunks(const DeltaShape &sh, const DeltaIo &io, const RaggedRows &rr, const ChunkPlan &p, uint32_t gate_from, hipStream_t s) {
     float *frags = io.scratch, *decay = frags + (uint64_t)p.slots * sh.heads * p.frags * 256;
-    constexpr size_t rows = 32 * (KT * 16 + 4), lds = (rows * (KIND == Recurrence::kChannelDelta ? 3 : 2) + 32 * 68 + 2 * 32 * 36) * 4;
+    constexpr size_t rows = 32 * (KT * 16 + 4);
+    constexpr size_t lds = KIND == Recurrence::kDelta ? chunk_lds_bytes(KT) : (rows * (KIND == Recurrence::kChannelDelta ? 3 : 2) + 32 * 68 + 2 * 32 * 36) * 4;
     static bool configured = false;
     auto configure = [&](auto... kernels) {
         if (lds > 65536 && !configured) (allow_lds(kernels, lds), ...);

@@ -67,6 +67,25 @@ def test_scan_forms(kind, dim, vdim, form, tune):
     dec.close()
 
 
+@pytest.mark.parametrize("heads,kv", [(2, 2), (4, 2), (5, 1)], ids=["one", "a pair", "two pairs and one"])
+@pytest.mark.parametrize("dim,vdim", [(20, 150), (128, 200)])
+def test_heads_that_share_a_chunk(heads, kv, dim, vdim):
+    """The heads of one q / k head in the chunk kernel: their decays come in pairs, V in the place of Q in one piece and more."""
+    cfg = lc.config([lc.delta(heads=heads, kv_heads=kv, dim=dim, vdim=vdim)])
+    w = lc.weights(cfg, 6)
+    lens = [40, 12, 65]
+    toks = [lc.tokens(cfg, n, 50 + n) for n in lens]
+    dec = lc.make_decoder(ops(), cfg, w, max_tokens=1024, max_batch=len(lens))
+    table = np.full((len(lens), dec.cfg.max_blocks_per_seq), 0xFFFFFFFF, dtype=np.uint32)
+    table[:, :8] = np.arange(8 * len(lens)).reshape(8, len(lens)).T
+    dec.set_sequences(table, [0] * len(lens))
+    got, at = dec.forward(toks, [list(range(n)) for n in lens]), 0
+    for b, n in enumerate(lens):
+        assert lc.error(got[at:at + n], oracle.forward(cfg, w, toks[b])) < F32_TOL, b
+        at += n
+    dec.close()
+
+
 _FAULTED = pytest.mark.skip(reason="a variant of the form that this size took, 32 rows per thread with a scratch of 900 bytes, ended here in a "
                                    "memory fault whose cause was not shown; the form is gone, the case is not run again")
 
