@@ -12,7 +12,7 @@ namespace fa {
 namespace k {
 using namespace fa::dev;
 
-int g_attention_form = 0;     // tuning: 1 the plain kernel, 2 the few-rows kernel for every sequence, 3 the many-rows kernel for every one
+int g_attention_form = 0;     // tuning: 1 the plain kernel, 2 the few-rows kernel for every sequence, 3 the many-rows kernel for every one, 4 on 128 columns a block
 int g_attention_blocks = 0;   // tuning: blocks per compute unit the key split aims at
 
 namespace {
@@ -537,7 +537,8 @@ __global__ void __launch_bounds__(64) attention_merge_kernel(StreamParams p, Att
 
 // ------------------------------------------------------------------ many query rows
 // A block of four wavefronts takes 64 NQ columns of one (sequence, key head), every wavefront 16 NQ of them, and walks the keys
-// they see 32 at a time; K and V of a step are staged in LDS, two stages.
+// they see 32 at a time; K and V of a step are staged in LDS, two stages.  Rows are requested two steps ahead (one step is shorter than
+// the way from memory where the walks are few: 3 x 700 tokens of 16 / 4 heads of 128 / 64 31.4 -> 29.0 us) in two sets of registers.
 template <int D, int V, int NQ, bool SIGMOID>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
     attention_flash_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_pool, const uint16_t *__restrict__ v_pool,
@@ -581,28 +582,30 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
     // staging: eight threads per key, 16 bytes each at a time; keys past the walk repeat its last one (masked)
     const int key = tid / 8, part = tid % 8;
     const uint64_t kw = (uint64_t)G * (D * 32), vw = (uint64_t)G * (V * 32);
-    v4u sk[PK], sv[PV];
+    struct Rows {
+        v4u k[PK], v[PV];
+    };
     auto page_of = [&](int32_t j) -> uint32_t {
         j = j < k_hi ? j : k_hi - 1;
         const uint32_t blk = (uint32_t)j / rr.block_size;
         return blk < rr.max_blocks ? table[blk] : 0xffffffffu;
     };
-    auto fetch = [&](int32_t j, uint32_t id) {
+    auto fetch = [&](int32_t j, uint32_t id, Rows &r) {
         j = j < k_hi ? j : k_hi - 1;
         const bool ok = id < rr.num_blocks;
         const uint64_t slot = (uint64_t)(ok ? id : 0) * rr.block_size + (uint32_t)j % rr.block_size;
         const uint16_t *kr = k_pool + slot * kw + kh * (D * 32) + part * 8, *vr = v_pool + slot * vw + kh * (V * 32) + part * 8;
 #pragma unroll
-        for (int i = 0; i < PK; ++i) sk[i] = *(const v4u *)(kr + i * 64);
+        for (int i = 0; i < PK; ++i) r.k[i] = *(const v4u *)(kr + i * 64);
 #pragma unroll
-        for (int i = 0; i < PV; ++i) sv[i] = *(const v4u *)(vr + i * 64);
-        if (!ok) sk[0] = v4u{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};      // no page: NaN, never a silent zero
+        for (int i = 0; i < PV; ++i) r.v[i] = *(const v4u *)(vr + i * 64);
     };
-    auto put = [&](int buf) {
+    auto put = [&](int buf, Rows &r, bool ok) {
+        if (!ok) r.k[0] = v4u{0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};     // no page: NaN, never a silent zero
 #pragma unroll
-        for (int i = 0; i < PK; ++i) *(v4u *)(ks + (buf * kKeys + key) * KP + (part + 8 * i) * 8) = sk[i];
+        for (int i = 0; i < PK; ++i) *(v4u *)(ks + (buf * kKeys + key) * KP + (part + 8 * i) * 8) = r.k[i];
 #pragma unroll
-        for (int i = 0; i < PV; ++i) *(v4u *)(vs + (buf * kKeys + key) * VP + (part + 8 * i) * 8) = sv[i];
+        for (int i = 0; i < PV; ++i) *(v4u *)(vs + (buf * kKeys + key) * VP + (part + 8 * i) * 8) = r.v[i];
     };
     const float factor = sh.scale * kLog2e;
     float m[NQ], l[NQ];
@@ -614,17 +617,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 #pragma unroll
         for (int t = 0; t < VT; ++t) o[qi][t] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    uint32_t id = page_of(k_lo + key);
-    fetch(k_lo + key, id);
-    id = page_of(k_lo + kKeys + key);
-    put(0);
+    // page ids three steps ahead
+    Rows even, odd;
+    uint32_t id = page_of(k_lo + key), id1 = page_of(k_lo + kKeys + key);
+    bool ok = id < rr.num_blocks, ok1 = id1 < rr.num_blocks;
+    fetch(k_lo + key, id, even);
+    fetch(k_lo + kKeys + key, id1, odd);
+    id = page_of(k_lo + 2 * kKeys + key);
+    put(0, even, ok);
     __syncthreads();
-    int buf = 0;
-    for (int32_t k0 = k_lo; k0 < k_hi; k0 += kKeys, buf ^= 1) {
+    // cur: the step's rows, in LDS already; next: those of the step behind it, under way
+    auto step = [&](int32_t k0, int buf, Rows &cur, Rows &next) {
         const bool more = k0 + kKeys < k_hi;
+        const bool ok_next = ok1;
         if (more) {
-            fetch(k0 + kKeys + key, id);
-            id = page_of(k0 + 2 * kKeys + key);
+            ok1 = id < rr.num_blocks;
+            fetch(k0 + 2 * kKeys + key, id, cur);
+            id = page_of(k0 + 3 * kKeys + key);
+            __builtin_amdgcn_sched_barrier(0);
         }
         if (k0 <= w_hi_pos && k0 + kKeys > w_lo_pos - W + 1) {       // some column of this wavefront sees some key of the step
             const bool inside = k0 + kKeys - 1 <= w_lo_pos && k0 > w_hi_pos - W;       // every column sees every key
@@ -674,8 +684,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
                 }
             }
         }
-        if (more) put(buf ^ 1);
+        if (more) put(buf ^ 1, next, ok_next);
         __syncthreads();
+    };
+    for (int32_t k0 = k_lo; k0 < k_hi; k0 += 2 * kKeys) {
+        step(k0, 0, even, odd);
+        if (k0 + kKeys < k_hi) step(k0 + kKeys, 1, odd, even);
     }
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
@@ -708,7 +722,7 @@ AttentionPlan attention_plan(const AttentionShape &sh, const AttentionOutput &ao
         return p;
     }
     const uint32_t S = sh.share();
-    p.max_cols = g_attention_form == 2 ? 0x7fffffffu : g_attention_form == 3 ? 0 : 64;
+    p.max_cols = g_attention_form == 2 ? 0x7fffffffu : g_attention_form >= 3 ? 0 : 64;
     p.stream = (uint64_t)min_new * S <= p.max_cols || (min_new <= 1 && p.max_cols);
     p.flash = (uint64_t)max_new * S > p.max_cols && (max_new > 1 || !p.max_cols);
     if (!p.stream) return p;
@@ -742,36 +756,51 @@ void launch_stream(const StreamParams &p, const AttentionShape &sh, const Ragged
     if (p.splits > 1) attention_merge_kernel<<<dim3(rr.batch * p.tiles, sh.kv_heads, 16 * NQ), 64, 0, s>>>(p, sh, rr, 16 * NQ);
 }
 
+// 128 columns to a block of attention_flash_kernel from eight such blocks a compute unit on, 64 below: a block's time is its longest walk, a
+// chain of staged steps, and more blocks on a unit fill each other's waits.  Prompts through layers of 16 / 4 heads of 128 / 64,
+// 128 and 64 columns, us: four layers, 3 x 700 tokens 1697 and 1664 (the kernel 40.6 and 31.4), 1 x 300 780 and 759, 1 x 2000 1815 and
+// 1717, 8 x 500 2724 and 2703; two layers, 4 x 2048 2708 and 2686, 8 x 2048 (eight a unit) 5306 and 5310; 32 / 8 heads of 128 / 128,
+// one layer, 1 x 1024 819 and 805, 4 x 2048 (eight a unit) 3852 and 3882.
+bool flash_is_wide(uint64_t rows, uint32_t share, uint32_t kv_heads, int num_cus) {
+    return g_attention_form == 4 || rows * share / 128 * kv_heads >= 8 * (uint64_t)num_cus;
+}
+
 template <int D, int V, bool SIGMOID>
-void launch_matrix_kind(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, hipStream_t s) {
+void launch_matrix_kind(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, int num_cus, hipStream_t s) {
     if (plan.stream) {
         if (plan.nq == 1) launch_stream<D, V, 1, SIGMOID>(p, sh, rr, s);
         else launch_stream<D, V, 2, SIGMOID>(p, sh, rr, s);
     }
     if (plan.flash) {
-        constexpr int NQ = D == 8 || V == 8 ? 1 : 2;
-        constexpr size_t lds = 2ull * kKeys * (D * 32 + 8 + V * 32 + 8) * 2;
-        if constexpr (lds > 65536) {
-            static bool configured = false;
-            if (!configured) {
-                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_flash_kernel<D, V, NQ, SIGMOID>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                configured = true;
+        auto flash = [&](auto nq) {
+            constexpr int NQ = decltype(nq)::value;
+            constexpr size_t lds = 2ull * kKeys * (D * 32 + 8 + V * 32 + 8) * 2;
+            if constexpr (lds > 65536) {
+                static bool configured = false;
+                if (!configured) {
+                    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_flash_kernel<D, V, NQ, SIGMOID>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                    configured = true;
+                }
             }
+            const dim3 grid((uint32_t)((uint64_t)rr.rows * sh.share() / (64 * NQ)) + rr.batch, sh.kv_heads);
+            attention_flash_kernel<D, V, NQ, SIGMOID><<<grid, 256, lds, s>>>(p.q, p.k_pool, p.v_pool, p.out, p.ld_out, p.ao, plan.max_cols, sh, rr);
+        };
+        if constexpr (D < 8 && V < 8) {
+            if (flash_is_wide(rr.rows, sh.share(), sh.kv_heads, num_cus)) return flash(std::integral_constant<int, 2>{});
         }
-        const dim3 grid((uint32_t)((uint64_t)rr.rows * sh.share() / (64 * NQ)) + rr.batch, sh.kv_heads);
-        attention_flash_kernel<D, V, NQ, SIGMOID><<<grid, 256, lds, s>>>(p.q, p.k_pool, p.v_pool, p.out, p.ld_out, p.ao, plan.max_cols, sh, rr);
+        flash(std::integral_constant<int, 1>{});
     }
 }
 template <int D, int V>
-void launch_matrix(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, hipStream_t s) {
-    if (p.ao.sigmoid) launch_matrix_kind<D, V, true>(plan, p, sh, rr, s);
-    else launch_matrix_kind<D, V, false>(plan, p, sh, rr, s);
+void launch_matrix(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, int num_cus, hipStream_t s) {
+    if (p.ao.sigmoid) launch_matrix_kind<D, V, true>(plan, p, sh, rr, num_cus, s);
+    else launch_matrix_kind<D, V, false>(plan, p, sh, rr, num_cus, s);
 }
 template <int D>
-void launch_matrix_v(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, hipStream_t s) {
-    if (sh.v_p == 64) launch_matrix<D, 2>(plan, p, sh, rr, s);
-    else if (sh.v_p == 128) launch_matrix<D, 4>(plan, p, sh, rr, s);
-    else launch_matrix<D, 8>(plan, p, sh, rr, s);
+void launch_matrix_v(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, int num_cus, hipStream_t s) {
+    if (sh.v_p == 64) launch_matrix<D, 2>(plan, p, sh, rr, num_cus, s);
+    else if (sh.v_p == 128) launch_matrix<D, 4>(plan, p, sh, rr, num_cus, s);
+    else launch_matrix<D, 8>(plan, p, sh, rr, num_cus, s);
 }
 
 }  // namespace
@@ -844,9 +873,9 @@ void attention(const void *q, const void *k_pool, const void *v_pool, void *out,
     StreamParams p{(const uint16_t *)q, (const uint16_t *)k_pool, (const uint16_t *)v_pool, (uint16_t *)out, ld_out, ao, (float *)workspace, nullptr, plan.splits,
                    plan.tiles, plan.max_cols};
     if (p.splits > 1) p.part_ml = p.part_o + (uint64_t)rr.batch * plan.tiles * sh.kv_heads * plan.splits * 16 * plan.nq * sh.v_p;
-    if (sh.dim_p == 64) launch_matrix_v<2>(plan, p, sh, rr, s);
-    else if (sh.dim_p == 128) launch_matrix_v<4>(plan, p, sh, rr, s);
-    else launch_matrix_v<8>(plan, p, sh, rr, s);
+    if (sh.dim_p == 64) launch_matrix_v<2>(plan, p, sh, rr, num_cus, s);
+    else if (sh.dim_p == 128) launch_matrix_v<4>(plan, p, sh, rr, num_cus, s);
+    else launch_matrix_v<8>(plan, p, sh, rr, num_cus, s);
 }
 
 }  // namespace k

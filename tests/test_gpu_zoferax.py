@@ -297,6 +297,28 @@ def test_a_key_that_stands_out(dtype, case, form, tune):
     dec.close()
 
 
+@pytest.mark.parametrize("form", [3, 4], ids=["64 columns", "128 columns"])
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 64), (4, 1, 128, 40), (6, 2, 100, 128), (3, 3, 64, 128)])
+def test_columns_of_a_block(heads, kv, dim, vdim, form, tune):
+    """The many-rows kernel on both widths: one key, walks of one to four steps of 32 keys and a key more, tiles that end inside a sequence, and more
+    tokens behind them."""
+    tune(33, form)
+    cfg = lc.zoferax([lc.attention(heads=heads, kv_heads=kv, dim=dim, vdim=vdim), lc.attention(heads=heads, kv_heads=kv, dim=dim, vdim=vdim)])
+    w = lc.weights(cfg, 21)
+    lens, more = [1, 32, 33, 64, 65, 97, 129], 33
+    toks = [lc.tokens(cfg, n + more, 60 + n) for n in lens]
+    dec = lc.make_decoder(ops(), cfg, w, "bfloat16", max_tokens=2048, max_batch=len(lens))
+    dec.set_sequences(tables_of(dec, len(lens)), [0] * len(lens))
+    first = dec.forward([t[:n] for t, n in zip(toks, lens)], [list(range(n)) for n in lens])
+    second = dec.forward([t[n:] for t, n in zip(toks, lens)], [list(range(more))] * len(lens))
+    at = 0
+    for b, n in enumerate(lens):
+        got = np.concatenate([first[at:at + n], second[b * more:(b + 1) * more]])
+        assert lc.error(got, oracle.forward(cfg, w, toks[b])) < BF16_TOL, n
+        at += n
+    dec.close()
+
+
 def test_first_tokens():
     cfg = lc.zoferax(MECHANISMS["all"])
     w = lc.weights(cfg, 14)
