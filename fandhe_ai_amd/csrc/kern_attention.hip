@@ -12,7 +12,7 @@ namespace fa {
 namespace k {
 using namespace fa::dev;
 
-int g_attention_form = 0;     // tuning: 1 the plain kernel, 2 the few-rows kernel for every sequence, 3 the many-rows kernel for every one, 4 on 128 columns a block
+int g_attention_form = 0;     // tuning: 1 the plain kernel, 2 the few-rows kernel for every sequence, 3 the many-rows kernel for every one
 int g_attention_blocks = 0;   // tuning: blocks per compute unit the key split aims at
 
 namespace {
@@ -536,20 +536,24 @@ __global__ void __launch_bounds__(64) attention_merge_kernel(StreamParams p, Att
 }
 
 // ------------------------------------------------------------------ many query rows
-// A block of four wavefronts takes 64 NQ columns of one (sequence, key head), every wavefront 16 NQ of them, and walks the keys
-// they see 32 at a time; K and V of a step are staged in LDS, two stages.  Rows are requested two steps ahead (one step is shorter than
-// the way from memory where the walks are few: 3 x 700 tokens of 16 / 4 heads of 128 / 64 31.4 -> 29.0 us) in two sets of registers.
-template <int D, int V, int NQ, bool SIGMOID>
+// A block of four wavefronts takes 64 columns of one (sequence, key head), every wavefront 16 of them, and walks the keys
+// they see 32 at a time; K and V of a step are staged in LDS, two stages, their rows requested two steps ahead in two sets of registers.
+// Key heads go round the block ids, so that an XCD has few heads' tiles and their rows in its L2.
+// A block's time is its walk, a chain of staged steps, so several blocks on a unit fill each other's waits.  Layers of 16 / 4 heads of
+// 128 / 64, us, 128 columns a block and rows one step ahead against this: 3 x 700 tokens 40.6 and 28.5 the kernel; passes through four such layers,
+// 1 x 300 780 and 749, 1 x 2000 1815 and 1665; through two, 4 x 2048 2666 and 2640, 8 x 2048 5264 and 5240; one of 32 / 8 heads of 128 / 128,
+// 4 x 2048 3940 and 3946.
+template <int D, int V, bool SIGMOID>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
     attention_flash_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ k_pool, const uint16_t *__restrict__ v_pool,
                            uint16_t *__restrict__ out, uint32_t ld_out, AttentionOutput ao, uint32_t max_cols, AttentionShape sh, RaggedRows rr) {
-    constexpr int VT = 2 * V, KP = D * 32 + 8, VP = V * 32 + 8, PK = D / 2, PV = V / 2, BC = 64 * NQ;
+    constexpr int VT = 2 * V, KP = D * 32 + 8, VP = V * 32 + 8, PK = D / 2, PV = V / 2, NQ = 1, BC = 64 * NQ;
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     uint16_t *ks = lds, *vs = lds + 2 * kKeys * KP;  // [2][32][KP], [2][32][VP]
-    const uint32_t S = sh.share(), G = sh.kv_heads, kh = blockIdx.y;
+    const uint32_t S = sh.share(), G = sh.kv_heads, kh = blockIdx.x % G;      // one XCD has few key heads' tiles, and their rows in its L2
     // longest walks first: the last tiles of a sequence
     uint32_t lo = 0, hi = rr.batch;
-    const uint32_t slot = gridDim.x - 1 - blockIdx.x;
+    const uint32_t slot = gridDim.x / G - 1 - blockIdx.x / G;
     auto base = [&](uint32_t b) { return (uint32_t)((uint64_t)rr.row_start[b] * S / BC) + b; };
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) / 2;
@@ -722,7 +726,7 @@ AttentionPlan attention_plan(const AttentionShape &sh, const AttentionOutput &ao
         return p;
     }
     const uint32_t S = sh.share();
-    p.max_cols = g_attention_form == 2 ? 0x7fffffffu : g_attention_form >= 3 ? 0 : 64;
+    p.max_cols = g_attention_form == 2 ? 0x7fffffffu : g_attention_form == 3 ? 0 : 64;
     p.stream = (uint64_t)min_new * S <= p.max_cols || (min_new <= 1 && p.max_cols);
     p.flash = (uint64_t)max_new * S > p.max_cols && (max_new > 1 || !p.max_cols);
     if (!p.stream) return p;
@@ -756,51 +760,35 @@ void launch_stream(const StreamParams &p, const AttentionShape &sh, const Ragged
     if (p.splits > 1) attention_merge_kernel<<<dim3(rr.batch * p.tiles, sh.kv_heads, 16 * NQ), 64, 0, s>>>(p, sh, rr, 16 * NQ);
 }
 
-// 128 columns to a block of attention_flash_kernel from eight such blocks a compute unit on, 64 below: a block's time is its longest walk, a
-// chain of staged steps, and more blocks on a unit fill each other's waits.  Prompts through layers of 16 / 4 heads of 128 / 64,
-// 128 and 64 columns, us: four layers, 3 x 700 tokens 1697 and 1664 (the kernel 40.6 and 31.4), 1 x 300 780 and 759, 1 x 2000 1815 and
-// 1717, 8 x 500 2724 and 2703; two layers, 4 x 2048 2708 and 2686, 8 x 2048 (eight a unit) 5306 and 5310; 32 / 8 heads of 128 / 128,
-// one layer, 1 x 1024 819 and 805, 4 x 2048 (eight a unit) 3852 and 3882.
-bool flash_is_wide(uint64_t rows, uint32_t share, uint32_t kv_heads, int num_cus) {
-    return g_attention_form == 4 || rows * share / 128 * kv_heads >= 8 * (uint64_t)num_cus;
-}
-
 template <int D, int V, bool SIGMOID>
-void launch_matrix_kind(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, int num_cus, hipStream_t s) {
+void launch_matrix_kind(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, hipStream_t s) {
     if (plan.stream) {
         if (plan.nq == 1) launch_stream<D, V, 1, SIGMOID>(p, sh, rr, s);
         else launch_stream<D, V, 2, SIGMOID>(p, sh, rr, s);
     }
     if (plan.flash) {
-        auto flash = [&](auto nq) {
-            constexpr int NQ = decltype(nq)::value;
-            constexpr size_t lds = 2ull * kKeys * (D * 32 + 8 + V * 32 + 8) * 2;
-            if constexpr (lds > 65536) {
-                static bool configured = false;
-                if (!configured) {
-                    (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_flash_kernel<D, V, NQ, SIGMOID>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-                    configured = true;
-                }
+        constexpr size_t lds = 2ull * kKeys * (D * 32 + 8 + V * 32 + 8) * 2;
+        if constexpr (lds > 65536) {
+            static bool configured = false;
+            if (!configured) {
+                (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&attention_flash_kernel<D, V, SIGMOID>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+                configured = true;
             }
-            const dim3 grid((uint32_t)((uint64_t)rr.rows * sh.share() / (64 * NQ)) + rr.batch, sh.kv_heads);
-            attention_flash_kernel<D, V, NQ, SIGMOID><<<grid, 256, lds, s>>>(p.q, p.k_pool, p.v_pool, p.out, p.ld_out, p.ao, plan.max_cols, sh, rr);
-        };
-        if constexpr (D < 8 && V < 8) {
-            if (flash_is_wide(rr.rows, sh.share(), sh.kv_heads, num_cus)) return flash(std::integral_constant<int, 2>{});
         }
-        flash(std::integral_constant<int, 1>{});
+        const uint32_t grid = ((uint32_t)((uint64_t)rr.rows * sh.share() / 64) + rr.batch) * sh.kv_heads;
+        attention_flash_kernel<D, V, SIGMOID><<<grid, 256, lds, s>>>(p.q, p.k_pool, p.v_pool, p.out, p.ld_out, p.ao, plan.max_cols, sh, rr);
     }
 }
 template <int D, int V>
-void launch_matrix(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, int num_cus, hipStream_t s) {
-    if (p.ao.sigmoid) launch_matrix_kind<D, V, true>(plan, p, sh, rr, num_cus, s);
-    else launch_matrix_kind<D, V, false>(plan, p, sh, rr, num_cus, s);
+void launch_matrix(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, hipStream_t s) {
+    if (p.ao.sigmoid) launch_matrix_kind<D, V, true>(plan, p, sh, rr, s);
+    else launch_matrix_kind<D, V, false>(plan, p, sh, rr, s);
 }
 template <int D>
-void launch_matrix_v(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, int num_cus, hipStream_t s) {
-    if (sh.v_p == 64) launch_matrix<D, 2>(plan, p, sh, rr, num_cus, s);
-    else if (sh.v_p == 128) launch_matrix<D, 4>(plan, p, sh, rr, num_cus, s);
-    else launch_matrix<D, 8>(plan, p, sh, rr, num_cus, s);
+void launch_matrix_v(const AttentionPlan &plan, const StreamParams &p, const AttentionShape &sh, const RaggedRows &rr, hipStream_t s) {
+    if (sh.v_p == 64) launch_matrix<D, 2>(plan, p, sh, rr, s);
+    else if (sh.v_p == 128) launch_matrix<D, 4>(plan, p, sh, rr, s);
+    else launch_matrix<D, 8>(plan, p, sh, rr, s);
 }
 
 }  // namespace
@@ -873,9 +861,9 @@ void attention(const void *q, const void *k_pool, const void *v_pool, void *out,
     StreamParams p{(const uint16_t *)q, (const uint16_t *)k_pool, (const uint16_t *)v_pool, (uint16_t *)out, ld_out, ao, (float *)workspace, nullptr, plan.splits,
                    plan.tiles, plan.max_cols};
     if (p.splits > 1) p.part_ml = p.part_o + (uint64_t)rr.batch * plan.tiles * sh.kv_heads * plan.splits * 16 * plan.nq * sh.v_p;
-    if (sh.dim_p == 64) launch_matrix_v<2>(plan, p, sh, rr, num_cus, s);
-    else if (sh.dim_p == 128) launch_matrix_v<4>(plan, p, sh, rr, num_cus, s);
-    else launch_matrix_v<8>(plan, p, sh, rr, num_cus, s);
+    if (sh.dim_p == 64) launch_matrix_v<2>(plan, p, sh, rr, s);
+    else if (sh.dim_p == 128) launch_matrix_v<4>(plan, p, sh, rr, s);
+    else launch_matrix_v<8>(plan, p, sh, rr, s);
 }
 
 }  // namespace k

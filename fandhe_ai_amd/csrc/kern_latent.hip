@@ -519,32 +519,36 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// A block of four wavefronts takes 128 tokens of one (sequence, head), every wavefront 32 columns of S^T = K Q^T, and walks
-// the keys they see 32 at a time; K (unrotated | rotated) and V of a step are staged in LDS, two stages.  D, RO:
-// dim_p = v_p and rot_p in units of 32.
+// A block of four wavefronts takes 64 tokens of one (sequence, head), every wavefront 16 columns of S^T = K Q^T, and walks
+// the keys they see 32 at a time; K (unrotated | rotated) and V of a step are staged in LDS, two stages, their rows requested two
+// steps ahead.  Heads go round the block ids, so that with a multiple of eight an XCD has the tiles of the same heads, whose expanded rows
+// then come out of its L2.  D, RO: dim_p = v_p and rot_p in units of 32.
+// A block is a chain of steps, and three of them fill each other's waits on a unit; 128 tokens a block left two: 32 heads of
+// 128 + 64, 300 tokens 22 -> 14.5 us, 1000 67 -> 58; a pass with 2 x 2048 tokens through one such layer 1800 us with 128 tokens a block, 1783 with 64,
+// 1735 with the heads dealt to the XCDs as well.
 template <int D, int RO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
     latent_flash_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kv, const uint16_t *__restrict__ kr,
                         const float *__restrict__ gate, uint32_t ld_gate, float out_scale, uint16_t *__restrict__ out, uint32_t ld_out,
                         LatentShape sh, RaggedRows rr, LatentExpand ex) {
-    constexpr int KS = D + RO, VT = 2 * D, KP = KS * 32 + 8, VP = D * 32 + 8, NQ = 2;
+    constexpr int KS = D + RO, VT = 2 * D, KP = KS * 32 + 8, VP = D * 32 + 8, NQ = 1, BC = 64 * NQ;
     constexpr int PKR = (KS * 4 + 7) / 8, PV = D * 4 / 8;        // 16-byte pieces per thread and step, eight threads per key
     __shared__ __attribute__((aligned(16))) uint16_t ks[2][kKeys * KP], vs[2][kKeys * VP];
     // longest walks first: the last tiles of a sequence
     uint32_t lo = 0, hi = rr.batch;
-    const uint32_t slots = gridDim.x, slot = slots - 1 - blockIdx.x;
+    const uint32_t H = sh.heads, h = blockIdx.x % H, slot = gridDim.x / H - 1 - blockIdx.x / H;
     while (hi - lo > 1) {
         const uint32_t mid = (lo + hi) / 2;
-        if (rr.row_start[mid] / 128 + mid <= slot) lo = mid;
+        if (rr.row_start[mid] / BC + mid <= slot) lo = mid;
         else hi = mid;
     }
-    const uint32_t b = lo, row0 = rr.row_start[b], n = rr.row_start[b + 1] - row0, t0 = (slot - (row0 / 128 + b)) * 128;
+    const uint32_t b = lo, row0 = rr.row_start[b], n = rr.row_start[b + 1] - row0, t0 = (slot - (row0 / BC + b)) * BC;
     if (t0 >= n) return;
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), g = lane / 16, c = lane % 16;
-    const uint32_t h = blockIdx.y, H = sh.heads, qw = KS * 32;
+    const uint32_t qw = KS * 32;
     constexpr uint32_t hw = 2 * D * 32;              // one head of an expanded row
     const int32_t p0 = rr.pos[row0], W = (int32_t)sh.window, first = (int32_t)ex.first[b];
-    const uint32_t t_last = t0 + 127 < n ? t0 + 127 : n - 1;
+    const uint32_t t_last = t0 + BC - 1 < n ? t0 + BC - 1 : n - 1;
     int32_t k_lo = p0 + (int32_t)t0 - W + 1, k_hi = p0 + (int32_t)t_last + 1;
     k_lo = k_lo > first ? k_lo : first;
     const uint64_t e0 = (uint64_t)ex.start[b] - (uint64_t)first;     // expanded row of key j: e0 + j
@@ -553,7 +557,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     int32_t pos[NQ];
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
-        uint32_t t = t0 + wave * 32 + qi * 16 + c;
+        uint32_t t = t0 + wave * 16 * NQ + qi * 16 + c;
         t = t < n ? t : n - 1;
         pos[qi] = p0 + (int32_t)t;
         const uint16_t *src = q + ((uint64_t)(row0 + t) * H + h) * qw + 8 * g;
@@ -564,12 +568,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) hold(qf[qi]);
-    const int32_t w_lo_pos = p0 + (int32_t)(t0 + wave * 32 < n ? t0 + wave * 32 : n - 1);
-    const int32_t w_hi_pos = p0 + (int32_t)(t0 + wave * 32 + 31 < n ? t0 + wave * 32 + 31 : n - 1);
+    const int32_t w_lo_pos = p0 + (int32_t)(t0 + wave * 16 * NQ < n ? t0 + wave * 16 * NQ : n - 1);
+    const int32_t w_hi_pos = p0 + (int32_t)(t0 + (wave + 1) * 16 * NQ - 1 < n ? t0 + (wave + 1) * 16 * NQ - 1 : n - 1);
 
     const int key = tid / 8, part = tid % 8;
-    v4u sk[PKR], sv[PV];
-    auto fetch = [&](int32_t k0) {
+    struct Rows {
+        v4u k[PKR], v[PV];
+    };
+    auto fetch = [&](int32_t k0, Rows &r) {
         const int32_t j = k0 + key;
         const bool ok = j < k_hi;
         const uint64_t e = e0 + (uint64_t)(ok ? j : k_hi - 1);
@@ -577,17 +583,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int i = 0; i < PKR; ++i) {
             const int pc = part + 8 * i;
-            if (pc < KS * 4) sk[i] = *(const v4u *)(pc < D * 4 ? row + pc * 8 : rot + (pc - D * 4) * 8);
+            if (pc < KS * 4) r.k[i] = *(const v4u *)(pc < D * 4 ? row + pc * 8 : rot + (pc - D * 4) * 8);
         }
 #pragma unroll
-        for (int i = 0; i < PV; ++i) sv[i] = *(const v4u *)(row + D * 32 + (part + 8 * i) * 8);
+        for (int i = 0; i < PV; ++i) r.v[i] = *(const v4u *)(row + D * 32 + (part + 8 * i) * 8);
     };
-    auto put = [&](int buf) {
+    auto put = [&](int buf, const Rows &r) {
 #pragma unroll
         for (int i = 0; i < PKR; ++i)
-            if (part + 8 * i < KS * 4) *(v4u *)&ks[buf][key * KP + (part + 8 * i) * 8] = sk[i];
+            if (part + 8 * i < KS * 4) *(v4u *)&ks[buf][key * KP + (part + 8 * i) * 8] = r.k[i];
 #pragma unroll
-        for (int i = 0; i < PV; ++i) *(v4u *)&vs[buf][key * VP + (part + 8 * i) * 8] = sv[i];
+        for (int i = 0; i < PV; ++i) *(v4u *)&vs[buf][key * VP + (part + 8 * i) * 8] = r.v[i];
     };
     float m[NQ], l[NQ];
     v4f o[NQ][VT];
@@ -598,13 +604,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
         for (int t = 0; t < VT; ++t) o[qi][t] = v4f{0.f, 0.f, 0.f, 0.f};
     }
-    fetch(k_lo);
-    put(0);
+    // rows are requested two steps ahead of the step that multiplies them
+    Rows even, odd;
+    fetch(k_lo, even);
+    fetch(k_lo + kKeys, odd);
+    put(0, even);
     __syncthreads();
-    int buf = 0;
-    for (int32_t k0 = k_lo; k0 < k_hi; k0 += kKeys, buf ^= 1) {
+    // cur: the step's rows, in LDS already; next: those of the step behind it, under way
+    auto step = [&](int32_t k0, int buf, Rows &cur, const Rows &next) {
         const bool more = k0 + kKeys < k_hi;
-        if (more) fetch(k0 + kKeys);
+        if (more) {
+            fetch(k0 + 2 * kKeys, cur);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         if (k0 <= w_hi_pos && k0 + kKeys > w_lo_pos - W + 1) {       // some column of this wavefront sees some key of the step
             const bool inside = k0 + kKeys - 1 <= w_lo_pos && k0 > w_hi_pos - W;       // every column sees every key
             float sc[NQ][8];
@@ -650,15 +662,19 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
                 }
             }
         }
-        if (more) put(buf ^ 1);
+        if (more) put(buf ^ 1, next);
         __syncthreads();
+    };
+    for (int32_t k0 = k_lo; k0 < k_hi; k0 += 2 * kKeys) {
+        step(k0, 0, even, odd);
+        if (k0 + kKeys < k_hi) step(k0 + kKeys, 1, odd, even);
     }
 #pragma unroll
     for (int qi = 0; qi < NQ; ++qi) {
         float sum = l[qi];
         sum += __shfl_xor(sum, 16, 64);
         sum += __shfl_xor(sum, 32, 64);
-        const uint32_t t = t0 + wave * 32 + qi * 16 + c;
+        const uint32_t t = t0 + wave * 16 * NQ + qi * 16 + c;
         if (t >= n) continue;
         const float f = gate ? out_scale / (1.0f + expf(-gate[(uint64_t)(row0 + t) * ld_gate + h])) / sum : out_scale / sum;
         uint16_t *dst = out + (uint64_t)(row0 + t) * ld_out + h * sh.vdim;
@@ -751,8 +767,8 @@ void latent_gather(const void *pool, void *c, uint32_t ld_c, void *kr, const Lat
 
 void latent_attention_expanded(const void *q, const void *kv, const void *kr, const float *gate, uint32_t ld_gate, float out_scale, void *out,
                                uint32_t ld_out, const LatentShape &sh, const RaggedRows &rr, const LatentExpand &ex, hipStream_t s) {
-    const dim3 grid(rr.rows / 128 + rr.batch + 1, sh.heads);
     const bool wide = sh.v_p > 64, rot2 = sh.rot_p > 32;
+    const uint32_t grid = (uint32_t)(rr.rows / 64 + rr.batch) * sh.heads;
 #define FA_FLASH(D_, RO_)                                                                                                                    \
     latent_flash_kernel<D_, RO_><<<grid, 256, 0, s>>>((const uint16_t *)q, (const uint16_t *)kv, (const uint16_t *)kr, gate, ld_gate, out_scale, \
                                                       (uint16_t *)out, ld_out, sh, rr, ex)

@@ -119,7 +119,7 @@ fa_status fa_probe_l2_path(fa_context *ctx, const fa_buffer *cold, uint64_t cold
  *        over a block's wavefronts, 3: never;
  * key 32: blocks per compute unit the key split of the absorbed form aims at;
  * key 33: grouped-query attention: 1: the plain kernel, 2: the few-rows kernel for every sequence, 3: the many-rows kernel
- *        for every sequence, 4: the same on 128 columns a block; key 34: blocks per compute unit its key split aims at;
+ *        for every sequence; key 34: blocks per compute unit its key split aims at;
  * key 35: routing of experts: 1: always in the residual update's launch, 2: always in a launch of its own.
  * key 36: minimal gated recurrence: threads across the channels of a block of the scan, 8 or 16;
  * key 37: row tiles of 16 per block of the large-tile prefill GEMMs (8, 12 or 16; with key 7). */

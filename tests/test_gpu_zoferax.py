@@ -297,12 +297,11 @@ def test_a_key_that_stands_out(dtype, case, form, tune):
     dec.close()
 
 
-@pytest.mark.parametrize("form", [3, 4], ids=["64 columns", "128 columns"])
 @pytest.mark.parametrize("heads,kv,dim,vdim", [(8, 2, 64, 64), (4, 1, 128, 40), (6, 2, 100, 128), (3, 3, 64, 128)])
-def test_columns_of_a_block(heads, kv, dim, vdim, form, tune):
-    """The many-rows kernel on both widths: one key, walks of one to four steps of 32 keys and a key more, tiles that end inside a sequence, and more
+def test_columns_of_a_block(heads, kv, dim, vdim, tune):
+    """The many-rows kernel: one key, walks of one to four steps of 32 keys and a key more, tiles that end inside a sequence, and more
     tokens behind them."""
-    tune(33, form)
+    tune(33, 3)
     cfg = lc.zoferax([lc.attention(heads=heads, kv_heads=kv, dim=dim, vdim=vdim), lc.attention(heads=heads, kv_heads=kv, dim=dim, vdim=vdim)])
     w = lc.weights(cfg, 21)
     lens, more = [1, 32, 33, 64, 65, 97, 129], 33
