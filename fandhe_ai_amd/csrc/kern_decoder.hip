@@ -158,6 +158,55 @@ __global__ void __launch_bounds__(256)
     if (r + 1 == row_start[lo + 1]) last_rows[lo] = (int32_t)r;
 }
 
+// Block (b, 0): row b and its tables; blocks (b, 1 ..): the embedding of token b, four columns a thread.  A step's chain begins here, and each of
+// the launches that this was waited for the one before (lengths and slots 1.6 us, advanced lengths 1.4, tables 1.8, embeddings 2.8): turns of 16
+// steps of four sequences on recurrent states 5376 -> 5295 us, of one 2659 -> 2574, a step of 32 on sparse experts 505 -> 502.3.
+template <typename T>
+__global__ void __launch_bounds__(256) step_rows_kernel(StepRows st) {
+    const uint32_t b = blockIdx.x;
+    if (blockIdx.y > 0) {
+        typedef T vt __attribute__((ext_vector_type(4)));
+        const int64_t src = st.tokens[b];
+        const bool ok = src >= 0 && (uint64_t)src < st.table_rows;
+        const uint32_t c = ((blockIdx.y - 1) * 256 + threadIdx.x) * 4;
+        if (c >= st.cols) return;
+        const float nanv = __uint_as_float(0x7fc00000u);
+        v4f v = v4f{nanv, nanv, nanv, nanv};
+        if (ok) {
+            const vt t = *(const vt *)((const T *)st.table + src * st.cols + c);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (sizeof(T) == 4) v[e] = t[e];
+                else v[e] = bf16_to_f32(t[e]);
+            }
+        }
+        *(v4f *)(st.out + (uint64_t)b * st.cols + c) = v;
+        return;
+    }
+    uint32_t p = st.seq_lens[b];
+    asm volatile("" : "+v"(p));                      // read by every wavefront ahead of the barrier; one writes it behind
+    __syncthreads();
+    for (int i = 0; i < st.rotations; ++i) {
+        const uint32_t dims = st.rotation[i].dims, half = dims / 2;
+        for (uint32_t t = threadIdx.x; t < half; t += 256) {
+            const double ang = (double)(int32_t)p * st.rotation[i].freq[t];
+            st.rotation[i].cos_sin[(uint64_t)b * dims + t] = (float)cos(ang);
+            st.rotation[i].cos_sin[(uint64_t)b * dims + half + t] = (float)sin(ang);
+        }
+    }
+    if (threadIdx.x != 255) return;                  // not of the wavefront that has the angles
+    uint32_t slot = 0xffffffffu;
+    if (p / st.block_size < st.max_blocks) {
+        const uint32_t id = st.tables[(uint64_t)b * st.max_blocks + p / st.block_size];
+        if (id < st.num_blocks) slot = id * st.block_size + p % st.block_size;
+    }
+    st.row_seq[b] = b;
+    st.pos[b] = (int32_t)p;
+    st.kv_slot[b] = slot;
+    st.last_rows[b] = (int32_t)b;
+    st.seq_lens[b] = p + 1;
+}
+
 __global__ void ragged_advance_kernel(const uint32_t *__restrict__ row_start, uint32_t *__restrict__ seq_lens, uint32_t batch) {
     const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b < batch) seq_lens[b] += row_start[b + 1] - row_start[b];
@@ -185,6 +234,16 @@ void ragged_prepare(const uint32_t *row_start, const uint32_t *tables, const uin
 
 void ragged_advance(const uint32_t *row_start, uint32_t *seq_lens, uint32_t batch, hipStream_t s) {
     ragged_advance_kernel<<<(batch + 63) / 64, 64, 0, s>>>(row_start, seq_lens, batch);
+}
+
+bool step_rows_embeds(const void *table, int table_f32, uint64_t cols, const float *out) {
+    return cols % 4 == 0 && cols < 1ull << 32 && (uintptr_t)table % (table_f32 ? 16 : 8) == 0 && (uintptr_t)out % 16 == 0;
+}
+void step_rows(const StepRows &st, int table_f32, hipStream_t s) {
+    if (st.batch == 0) return;
+    const dim3 grid(st.batch, 1 + (st.table ? (st.cols + 1023) / 1024 : 0));
+    if (table_f32) step_rows_kernel<float><<<grid, 256, 0, s>>>(st);
+    else step_rows_kernel<uint16_t><<<grid, 256, 0, s>>>(st);
 }
 
 void rotation_table(const int32_t *pos, float *cos_sin, uint32_t rows, uint32_t dims, const double *freq, hipStream_t s) {

@@ -427,6 +427,30 @@ void ragged_prepare(const uint32_t *row_start, const uint32_t *tables, const uin
                     uint32_t *kv_slot, int32_t *last_rows, uint32_t batch, uint32_t rows, uint32_t block_size, uint32_t max_blocks,
                     uint32_t num_blocks, hipStream_t s);
 void ragged_advance(const uint32_t *row_start, uint32_t *seq_lens, uint32_t batch, hipStream_t s);
+// Both for a step, row b the one new token of sequence b, with the rotation tables (rotation_table) of its positions and the rows' embeddings
+// (gather_rows_any; table null: none) in one launch.
+struct StepRows {
+    static constexpr int kRotations = 4;
+    const uint32_t *tables;
+    uint32_t *seq_lens, *row_seq;
+    int32_t *pos;
+    uint32_t *kv_slot;
+    int32_t *last_rows;
+    uint32_t batch, block_size, max_blocks, num_blocks;
+    struct {
+        float *cos_sin;
+        const double *freq;
+        uint32_t dims;
+    } rotation[kRotations];
+    int rotations;
+    const void *table;
+    uint64_t table_rows;
+    uint32_t cols;
+    const int32_t *tokens;
+    float *out;
+};
+bool step_rows_embeds(const void *table, int table_f32, uint64_t cols, const float *out);
+void step_rows(const StepRows &st, int table_f32, hipStream_t s);
 // cos_sin [rows, dims] of the rows' positions (cos in the first half, sin in the second) for the frequencies freq [dims / 2],
 // angles formed in double
 void rotation_table(const int32_t *pos, float *cos_sin, uint32_t rows, uint32_t dims, const double *freq, hipStream_t s);

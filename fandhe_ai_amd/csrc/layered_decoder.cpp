@@ -510,13 +510,13 @@ void add_experts(k::ResidualNorm &rn, const Arena &a, const Layer &l) {
 
 // All layers over the rows of a pass whose embeddings are in a.x (and, with norms at the output, in a.hn).
 fa_status enqueue_layers(fa_context *ctx, fa_decoder *d, Arena &a, const k::RaggedRows &rr, Portions n, uint64_t trace_row0,
-                         const ExpandPlan *expand = nullptr) {
+                         const ExpandPlan *expand = nullptr, bool rotations = true) {
     LayeredState &L = *d->layered;
     hipStream_t s = ctx->stream;
     const uint32_t M = rr.rows, D = L.cfg.d_model, ld_hn = pad_to(D, 64);
     const float eps = L.cfg.norm_eps;
     const int f32 = L.is_f32;
-    for (size_t i = 0; i < L.rotations.size(); ++i) k::rotation_table(rr.pos, a.cos_sin[i], M, L.rotations[i].dims, L.rotation_freq[i], s);
+    for (size_t i = 0; rotations && i < L.rotations.size(); ++i) k::rotation_table(rr.pos, a.cos_sin[i], M, L.rotations[i].dims, L.rotation_freq[i], s);
     if (L.cfg.norm == FA_NORM_BOTH) k::layernorm_rows(a.x, L.layers[0].norm1, a.hn, f32, M, D, ld_hn, eps, s);
     if (L.cfg.norm == FA_NORM_INPUT_RMS) {
         k::ResidualNorm rn;
@@ -611,9 +611,11 @@ fa_status enqueue_layers(fa_context *ctx, fa_decoder *d, Arena &a, const k::Ragg
     return FA_OK;
 }
 
+// Whether embeddings are rows of the table as they are
+bool plain_embedding(const LayeredState &L) { return L.cfg.norm != FA_NORM_OUTPUT && L.cfg.norm != FA_NORM_INPUT_RMS; }
 // Embeddings of the pass's tokens.
 void enqueue_embed(fa_context *ctx, const LayeredState &L, Arena &a, const int32_t *tokens, const k::RaggedRows &rr) {
-    if (L.cfg.norm == FA_NORM_OUTPUT || L.cfg.norm == FA_NORM_INPUT_RMS)
+    if (!plain_embedding(L))
         k::embed_rows(L.embed, L.is_f32, L.cfg.vocab, L.cfg.d_model, tokens, rr.pos, L.position_freq, L.cfg.embed_scale, a.x,
                       L.cfg.norm == FA_NORM_OUTPUT ? a.hn : nullptr, pad_to(L.cfg.d_model, 64), rr.rows, ctx->stream);
     else
@@ -742,10 +744,44 @@ fa_status layered_enqueue_step(fa_context *ctx, fa_decoder *d) {
     Arena &a = L.step;
     const uint32_t B = d->batch;
     const uint32_t *starts = (const uint32_t *)L.unit_starts->ptr;
-    prepare_rows(ctx, d, a, starts, B);
     const k::RaggedRows rr = ragged(d, a, starts, B);
-    enqueue_embed(ctx, L, a, (const int32_t *)d->tokens->ptr, rr);
-    if (fa_status s = enqueue_layers(ctx, d, a, rr, Portions{1, 1}, 0)) return s;
+    const int32_t *tokens = (const int32_t *)d->tokens->ptr;
+    // rotations of more than a few kinds, and embeddings that take the position, keep their launches
+    const bool together = L.rotations.size() <= k::StepRows::kRotations;
+    if (together) {
+        const fa_decoder_config &c = d->cfg;
+        k::StepRows st{};
+        st.tables = (const uint32_t *)d->tables->ptr;
+        st.seq_lens = (uint32_t *)d->seq_lens->ptr;
+        st.row_seq = a.row_seq;
+        st.pos = a.pos;
+        st.kv_slot = a.kv_slot;
+        st.last_rows = (int32_t *)L.last_rows->ptr;
+        st.batch = B;
+        st.block_size = c.block_size;
+        st.max_blocks = c.max_blocks_per_seq;
+        st.num_blocks = c.num_blocks;
+        st.rotations = (int)L.rotations.size();
+        for (int i = 0; i < st.rotations; ++i) {
+            st.rotation[i].cos_sin = a.cos_sin[i];
+            st.rotation[i].freq = L.rotation_freq[i];
+            st.rotation[i].dims = L.rotations[i].dims;
+        }
+        const bool embeds = plain_embedding(L) && k::step_rows_embeds(L.embed, L.is_f32, L.cfg.d_model, a.x);
+        if (embeds) {
+            st.table = L.embed;
+            st.table_rows = L.cfg.vocab;
+            st.cols = L.cfg.d_model;
+            st.tokens = tokens;
+            st.out = a.x;
+        }
+        k::step_rows(st, L.is_f32, ctx->stream);
+        if (!embeds) enqueue_embed(ctx, L, a, tokens, rr);
+    } else {
+        prepare_rows(ctx, d, a, starts, B);
+        enqueue_embed(ctx, L, a, tokens, rr);
+    }
+    if (fa_status s = enqueue_layers(ctx, d, a, rr, Portions{1, 1}, 0, nullptr, !together)) return s;
     enqueue_head(ctx, L, a, a.x, B, (float *)d->logits->ptr);
     enqueue_pick(d, ctx->stream);
     return after_launch(ctx, "layered decoder step");

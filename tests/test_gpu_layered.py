@@ -145,6 +145,31 @@ def step_logits(dec, toks, start, use_graph):
 
 
 @pytest.mark.parametrize("use_graph", [False, True])
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("rotations,width", [(1, 76), (4, 78), (5, 76), (0, 1028), (2, 1030)])
+def test_rows_of_a_step(rotations, width, batch, use_graph):
+    """What begins a step in one launch (rows, lengths, rotations of up to four kinds, embeddings of whole groups of four columns) and in several,
+    over page borders and behind a rewind: whole passes are the reference."""
+    layers = [lc.latent(base=1000.0 * (i + 1)) for i in range(rotations)] or [lc.delta()]
+    cfg = lc.config(layers, width=width)
+    w = lc.weights(cfg, 9)
+    toks = [lc.tokens(cfg, 20, 70 + b) for b in range(batch)]
+    dec = lc.make_decoder(ops(), cfg, w, max_batch=batch)
+    dec.set_sequences(tables_of(dec, batch), [0] * batch)
+    dec.prefill([t[:14] for t in toks])
+    want = [oracle.forward(cfg, w, t) for t in toks]
+    for at in list(range(14, 20)) + ([17, 18] if rotations else []):          # (states do not go back)
+        if at == 17 and rotations:
+            dec.rewind([17] * batch)
+        dec.set_tokens([int(t[at]) for t in toks])
+        dec.step(use_graph)
+        got = dec.logits()
+        for b in range(batch):
+            assert lc.error(got[b:b + 1], want[b][at:at + 1]) < F32_TOL, (at, b)
+    dec.close()
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
 def test_steps_continue_a_prompt_pass(use_graph):
     """fa_decoder_prefill and fa_decoder_step (eager, and replayed from a graph) against one whole pass."""
     cfg = lc.config(MECHANISMS["all"])
