@@ -199,6 +199,9 @@ struct StreamParams {
     float *part_o, *part_ml;                         // [slot][split][16 NQ][rank_p], [slot][split][16 NQ][2]: maximum, sum
     uint32_t splits;
     int direct;                                      // one token per sequence, its heads in one block: block b is sequence b
+    const uint16_t *q = nullptr;                     // where the rotated parts are still to be turned: [rows, heads, q_pitch], theirs from q_rot on
+    const float *cos_sin = nullptr;                  // [rows, 64]
+    uint32_t q_pitch = 0, q_rot = 0;
 };
 
 template <int NQ>
@@ -294,7 +297,40 @@ __global__ void __launch_bounds__(NQ * DH * GR * 64) __attribute__((amdgpu_waves
     const uint16_t *q = p.qa + ((uint64_t)row0 * H + qr) * WIDTH + 8 * g;
     v8bf qf[KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[s] = *(const v8bf *)(q + s * 32);
+    for (int s = 0; s < (RO == 2 ? RK : KS); ++s) qf[s] = *(const v8bf *)(q + s * 32);
+    if constexpr (RO == 2) {
+        if (p.q) {
+            // dims d and d + 32 of the rotated part sit in one lane: latent_rotate_query_kernel's expressions and rounding
+            const uint16_t *src = p.q + ((uint64_t)row0 * H + qr) * p.q_pitch + p.q_rot + 8 * g;
+            const float *cs = p.cos_sin + (uint64_t)(row0 + qr / H) * 64 + 8 * g;
+            const v4u u4 = *(const v4u *)src, v4 = *(const v4u *)(src + 32);
+            v4f co[2], si[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                co[i] = *(const v4f *)(cs + 4 * i);
+                si[i] = *(const v4f *)(cs + 32 + 4 * i);
+            }
+            v4u lo, hi;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float u[2] = {bf16_lo(u4[i]), bf16_hi(u4[i])}, v[2] = {bf16_lo(v4[i]), bf16_hi(v4[i])};
+                float x[2], y[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const float c1 = co[i / 2][i % 2 * 2 + e], s1 = si[i / 2][i % 2 * 2 + e];
+                    x[e] = u[e] * c1 - v[e] * s1;
+                    y[e] = v[e] * c1 + u[e] * s1;
+                }
+                lo[i] = f32x2_to_bf16x2(x[0], x[1]);
+                hi[i] = f32x2_to_bf16x2(y[0], y[1]);
+            }
+            qf[RK] = __builtin_bit_cast(v8bf, lo);
+            qf[RK + 1] = __builtin_bit_cast(v8bf, hi);
+        } else {
+            qf[RK] = *(const v8bf *)(q + RK * 32);
+            qf[RK + 1] = *(const v8bf *)(q + (RK + 1) * 32);
+        }
+    }
     hold(qf);
     const float factor = sh.scale * kLog2e;
     float m = -INFINITY, l = 0.0f;
@@ -732,14 +768,21 @@ uint64_t latent_attention_workspace_bytes(const LatentShape &sh, int is_f32, uin
     return p.splits > 1 ? (uint64_t)p.slots * p.splits * 16 * p.nq * (sh.rank_p + 2) * 4 : 0;
 }
 
+bool latent_attention_rotates(const LatentShape &sh, int is_f32, const RaggedRows &rr, uint32_t max_new, int num_cus) {
+    return !is_f32 && sh.rot == 64 && !sh.interleaved && stream_plan(sh, rr.rows, rr.batch, max_new, num_cus).nq != 0;
+}
 void latent_attention(const void *qa, const void *pool, void *out, int is_f32, const LatentShape &sh, const RaggedRows &rr,
-                      uint32_t max_new, void *workspace, int num_cus, hipStream_t s) {
+                      uint32_t max_new, void *workspace, int num_cus, hipStream_t s, const void *q, const float *cos_sin) {
     if (rr.rows == 0) return;
     if (!is_f32) {
         const StreamPlan plan = stream_plan(sh, rr.rows, rr.batch, max_new, num_cus);
         if (plan.nq) {
             StreamParams p{(const uint16_t *)qa, (const uint16_t *)pool, (uint16_t *)out, (float *)workspace, nullptr, plan.splits, plan.direct};
             if (p.splits > 1) p.part_ml = p.part_o + (uint64_t)plan.slots * plan.splits * 16 * plan.nq * sh.rank_p;
+            p.q = (const uint16_t *)q;
+            p.cos_sin = cos_sin;
+            p.q_pitch = sh.dim_p + sh.rot_p;
+            p.q_rot = sh.dim_p;
             if (sh.rank_p <= 64) launch_stream_ro<2>(p, sh, rr, plan, s);
             else if (sh.rank_p <= 128) launch_stream_ro<4>(p, sh, rr, plan, s);
             else if (sh.rank_p <= 256) launch_stream_ro<8>(p, sh, rr, plan, s);

@@ -579,8 +579,11 @@ void latent_rotate_query(const void *q, const float *cos_sin, void *dst, uint32_
 // latents.  bf16 with kv_rank <= 512 and rot <= 64: the matrix-core kernel (workspace for the key splits); otherwise a
 // plain one.  max_new: most new tokens of any sequence.
 uint64_t latent_attention_workspace_bytes(const LatentShape &sh, int is_f32, uint32_t rows, uint32_t batch, uint32_t max_new, int num_cus);
+// q != null (where latent_attention_rotates): the rotated parts of the queries are those of q [rows, heads, dim_p + rot_p], not turned yet, and
+// latent_rotate_query does not run.
+bool latent_attention_rotates(const LatentShape &sh, int is_f32, const RaggedRows &rr, uint32_t max_new, int num_cus);
 void latent_attention(const void *qa, const void *pool, void *out, int is_f32, const LatentShape &sh, const RaggedRows &rr,
-                      uint32_t max_new, void *workspace, int num_cus, hipStream_t s);
+                      uint32_t max_new, void *workspace, int num_cus, hipStream_t s, const void *q = nullptr, const float *cos_sin = nullptr);
 // The form for prompts (bf16, dim, vdim <= 128, rot <= 64): the keys first[b] .. of every sequence are gathered as rows
 // start[b] .. start[b + 1] - 1 (latents c [rows, ld_c], rotated parts kr [rows, rot_p]), a linear turns the latents into
 // kv [rows, heads, dim_p + v_p], and attention runs per head on those; q is [rows, heads, dim_p + rot_p] with its

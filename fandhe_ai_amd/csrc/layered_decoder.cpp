@@ -383,8 +383,9 @@ void enqueue_latent(fa_context *ctx, const fa_decoder *d, Arena &a, const Layer 
         k::LinearEpilogue e = store_to(a.qa, (uint64_t)sh.heads * kw, f32);
         e.out_batch = kw;
         linear(ctx, L, a.q, (uint64_t)sh.heads * qw, qw, M, m.uk, e);
-        k::latent_rotate_query(a.q, cs, a.qa, kw, sh.rank_p, f32, sh, M, s);
-        k::latent_attention(a.qa, pool, a.olat, f32, sh, rr, max_new, ctx->workspace, ctx->props.multiProcessorCount, s);
+        const bool rotates = k::latent_attention_rotates(sh, f32, rr, max_new, ctx->props.multiProcessorCount);
+        if (!rotates) k::latent_rotate_query(a.q, cs, a.qa, kw, sh.rank_p, f32, sh, M, s);
+        k::latent_attention(a.qa, pool, a.olat, f32, sh, rr, max_new, ctx->workspace, ctx->props.multiProcessorCount, s, rotates ? a.q : nullptr, cs);
         e = store_to(o, ld_o, f32);
         if (gate) e.mode = k::LinearEpilogue::kHeadGate;
         e.factor = m.out_scale;

@@ -144,6 +144,35 @@ def step_logits(dec, toks, start, use_graph):
     return np.array(out)
 
 
+@pytest.mark.parametrize("heads,kv_rank", [(3, 64), (20, 128), (16, 256), (33, 512)])
+def test_queries_turned_where_they_are_read(heads, kv_rank):
+    """The absorbed kernel on rotated parts of 64 dims turns the queries itself: prompts and single tokens, one and several tokens of a sequence in a
+    column tile, key splits, against the plain kernel, which reads what a launch of its own has turned."""
+    from fandhe_ai_amd.capi import lib
+    cfg = lc.config([lc.latent(heads=heads, dim=64, rot=64, vdim=64, q_rank=64, kv_rank=kv_rank, window=600, base=100.0)])
+    w = lc.weights(cfg, 11)
+    toks = [lc.tokens(cfg, n, 80 + n) for n in (560, 37)]
+    got = []
+    for form in (1, 2):
+        lib.fa_set_tuning(30, form)
+        try:
+            dec = lc.make_decoder(ops(), cfg, w, "bfloat16", max_tokens=2048, max_batch=2)
+            dec.set_sequences(tables_of(dec, 2), [0, 0])
+            out = [dec.forward([t[:-5] for t in toks], [list(range(len(t) - 5)) for t in toks])]
+            out.append(dec.forward([t[-5:-2] for t in toks], [[0, 1, 2]] * 2))
+            for i in (-2, -1):
+                dec.set_tokens([int(t[i]) for t in toks])
+                dec.step(False)
+                out.append(np.array(dec.logits()))
+            dec.close()
+        finally:
+            lib.fa_set_tuning(30, 0)
+        got.append(np.concatenate(out))
+    # both round the same operands to bf16; what differs are sums in another order and the weights' two terms of bf16
+    assert lc.error(got[1], got[0]) < 0.02
+    assert lc.error(got[0][-2:], np.stack([oracle.forward(cfg, w, t)[-1] for t in toks])) < 0.1
+
+
 @pytest.mark.parametrize("use_graph", [False, True])
 @pytest.mark.parametrize("batch", [1, 3])
 @pytest.mark.parametrize("rotations,width", [(1, 76), (4, 78), (5, 76), (0, 1028), (2, 1030)])
