@@ -461,7 +461,7 @@ fa_status fa_gemm_e4m3(fa_context *ctx, const fa_buffer *aq, const fa_buffer *a_
     if (m > (1ull << 22)) return fail(FA_ERR_INVALID_ARGUMENT, "gemm_e4m3: m too large for one launch");
     k::gemm_e4m3_mfma((const uint8_t *)aq->ptr, (const uint8_t *)qw->codes->ptr, (const float *)a_scale->ptr,
                       (const float *)qw->scales->ptr, m, qw->n, qw->n_pad, qw->k_pad, out->ptr, out->dtype == FA_BF16,
-                      ctx->props.multiProcessorCount, ctx->stream);
+                      ctx->props.multiProcessorCount, ctx->stream, &ctx->splitk);
     return after_launch(ctx, "gemm_e4m3_mfma");
 }
 
@@ -491,7 +491,7 @@ static fa_status launch_e4m3_rows(fa_context *ctx, const uint8_t *aq, const floa
     else
         k::gemm_e4m3_rows_mfma(aq, (const uint8_t *)qw->codes->ptr, sx, (const float *)qw->scales->ptr, bp, m, qw->n,
                                qw->n_pad, qw->k_pad, out->ptr, out->dtype == FA_BF16, ctx->props.multiProcessorCount,
-                               ctx->stream);
+                               ctx->stream, &ctx->splitk);
     return after_launch(ctx, "linear_e4m3");
 }
 

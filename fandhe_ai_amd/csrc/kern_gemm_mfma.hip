@@ -21,7 +21,7 @@ namespace k {
 using namespace fa::dev;
 
 int g_gemm_small_tiles = 0;   // tuning: nonzero keeps the 128 x 128 kernel for every shape
-int g_gemm_pair = 0;          // tuning, tiles of 128 columns of the large-tile kernel: 1 keeps one block per tile
+int g_gemm_pair = 0;          // tuning, tiles of 128 columns of the large-tile kernel: 1 keeps one block per tile; 2, 4: that many, f32 sums
 int g_gemm_swiglu = 0;        // tuning, prompt passes: bit 0 keeps SwiGLU out of the gate | up GEMM's epilogue, bit 1 RoPE
                               // and the K / V append out of the q | k | v GEMM's
 int g_gemm_waves = 0;         // tuning: 4 = four wavefronts per large-tile block instead of eight, 16 = sixteen
@@ -39,15 +39,20 @@ struct EpiI8 {
 };
 // Large-tile kernel on tiles of 128 columns, k split over split_s = 2 or 4 blocks: blocks b, b + 8, ... of a launch (one XCD) own
 // one output tile and a share of k each; all leave their raw sums in split_partial, wait for their stores and take a ticket from
-// the tile's counter, and the one that draws the last ticket adds the others' sums (int32: exact in any order) and runs the
-// epilogue.  split_local: the exchange stays in the XCD's L2.  (A type of its own: the sums added to the accumulators make the
-// compiler spill on the wide tiles.)
-struct EpiI8Split : EpiI8 {
-    int32_t *split_partial;
+// the tile's counter, and the one that draws the last ticket adds the others' sums (int32: exact in any order; f32: in the order of
+// the shares, whoever came last, so that a call's bits do not depend on it) and runs the epilogue.  split_local: the exchange stays
+// in the XCD's L2.  (A type of its own: the sums added to the accumulators make the compiler spill on the wide tiles.)
+template <typename Base>
+struct EpiSplit : Base {
+    int32_t *split_partial;          // the sums' bits
     uint32_t *split_counters;
     int split_local;
     uint32_t split_s;
 };
+template <typename Epi>
+struct IsSplit : std::false_type {};
+template <typename Base>
+struct IsSplit<EpiSplit<Base>> : std::true_type {};
 // int8, large-tile kernel only: the weight is gate | up (f columns each) and the kernel leaves silu(gate) * up, f32 [m, f]
 struct EpiI8Swiglu {
     const float *sx, *sw;
@@ -96,6 +101,8 @@ struct IsBf16<EpiBf16Grouped<MODE>> : std::true_type {
     static constexpr int mode = MODE;
     static constexpr bool grouped = true;
 };
+template <typename Base>
+struct IsBf16<EpiSplit<Base>> : IsBf16<Base> {};
 
 constexpr int BM = 128, BN = 128;      // block tile; 4 wavefronts in 2 x 2, 64 x 64 each
 constexpr int MT = BM / 16, NT = BN / 16;
@@ -430,7 +437,7 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     const int wm = wave / 2, wn = wave % 2;
     uint32_t mb, nb;
     uint32_t tile_id = blockIdx.x, half = 0, ks_lo = 0, ks_n = k_steps;
-    constexpr bool SPLIT = std::is_same<Epi, EpiI8Split>::value;
+    constexpr bool SPLIT = IsSplit<Epi>::value;
     if constexpr (SPLIT) {
         ixm::ksplit_block(blockIdx.x, ep.split_s, &tile_id, &half);          // partners b, b + 8, ...: one XCD
         if (tile_id >= m_blocks * n_blocks) return;                   // the same for all partners
@@ -691,11 +698,13 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
     }
 
     if constexpr (SPLIT) {
-        // raw sums of this half of k: word (i, j, e) of thread t at [(i * WNT + j) * 4 + e][t], 2 KiB per store
+        // raw sums of this share of k: word (i, j, e) of thread t at [(i * WNT + j) * 4 + e][t], 2 KiB per store
         constexpr int WORDS = AI * WNT * 4;
         const uint32_t S = ep.split_s;
         int32_t *mine = ep.split_partial + ((uint64_t)tile_id * S + half) * ((uint64_t)WORDS * 128 * WM);
         const bool local = ep.split_local != 0;
+        constexpr bool EXACT = !FP8 && !BF16;                          // int32 sums
+        auto bits = [](auto x) { return __builtin_bit_cast(int32_t, x); };
         if (!idle) {
 #pragma unroll
         for (int i = 0; i < AI; ++i)
@@ -704,8 +713,8 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     int32_t *p = mine + ((i * WNT + j) * 4 + e) * (128 * WM) + tid;
-                    if (local) __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    else __hip_atomic_store(p, (int32_t)acc[i][j][e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (local) __hip_atomic_store(p, bits(acc[i][j][e]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    else __hip_atomic_store(p, bits(acc[i][j][e]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
         }
         __builtin_amdgcn_s_waitcnt(0);            // this thread's stores are acknowledged
@@ -723,8 +732,15 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
         }
         __syncthreads();
         if (*slot != S - 1 || idle) return;       // a partner finishes the tile
+        const bool in_order = !EXACT && S > 2;        // f32: from the first share on, this block's own read back too (two commute)
+        if (in_order) {
+#pragma unroll
+            for (int i = 0; i < AI; ++i)
+#pragma unroll
+                for (int j = 0; j < WNT; ++j) acc[i][j] = acc_t{};
+        }
         for (uint32_t r = 0; r < S; ++r) {
-            if (r == half) continue;
+            if (r == half && !in_order) continue;
             const int32_t *other = ep.split_partial + ((uint64_t)tile_id * S + r) * ((uint64_t)WORDS * 128 * WM);
 #pragma unroll
             for (int i = 0; i < AI; ++i)
@@ -733,8 +749,10 @@ __global__ void __launch_bounds__(128 * WM) __attribute__((amdgpu_waves_per_eu(W
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const int32_t *p = other + ((i * WNT + j) * 4 + e) * (128 * WM) + tid;
-                        acc[i][j][e] += local ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
-                                              : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        const int32_t v = local ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)
+                                                : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        if constexpr (EXACT) acc[i][j][e] += v;
+                        else acc[i][j][e] += __builtin_bit_cast(float, v);
                     }
         }
     }
@@ -1063,15 +1081,21 @@ struct BigShape {
     double fixed, per_2k;
 };
 constexpr double kShareCost = 1.5;           // us per sharing block of 128 x 128: partial sums left and added
+constexpr double kShareF8 = 0.0, kShareBf16 = 4.0;      // ... and besides, where the sums are f32 (pick_big_f32)
 constexpr BigShape kBigShapes[] = {{16, 16, 14.5, 23.7}, {16, 14, 12.3, 21.6}, {12, 16, 10.4, 18.6}, {12, 14, 10.3, 16.6},
                                    {16, 8, 9.5, 13.4},   {8, 16, 9.8, 13.1},   {12, 8, 7.6, 10.6},   {8, 8, 6.0, 7.5}};
 
+// Blocks that may share a tile of 128 columns, a part of k each: how many, the stages of a part, what sharing costs besides
+struct ShareRule {
+    uint32_t most = 1, least = 1, stages = 8;
+    double extra = 0;
+};
+
 // The tile with the lowest cost: whole rounds over the compute units, and a last one that costs less the emptier it is (0.6 of a
 // full one at the least: measured 0.65 at 0.3, 0.8 at 0.6: the blocks in it have the L2s, and the power, to themselves).
-// tiles_of(rows): row blocks of that many rows.  max_share: blocks that may share a tile of 128 columns, a part of k each (8 stages
-// at the least).  low: what tiles of fewer than 256 rows cost more than the table says.
+// tiles_of(rows): row blocks of that many rows.  low: what tiles of fewer than 256 rows cost more than the table says.
 template <typename F>
-BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, uint32_t max_share, double low = 1.0) {
+BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, const ShareRule &rule, double low = 1.0) {
     BigTile best;
     auto has = [&](const BigShape &b) { return (widths & (b.ntb == 16 ? kWide16 : b.ntb == 14 ? kWide14 : kWide8)) != 0; };
     auto wanted = [](const BigShape &b) { return (!g_gemm_ntb || g_gemm_ntb == b.ntb) && (!g_gemm_mtb || g_gemm_mtb == b.mtb); };
@@ -1080,18 +1104,18 @@ BigTile pick_big_rows(F &&tiles_of, uint64_t n_tiles, uint64_t k_steps, int num_
     for (const BigShape &b : kBigShapes) {
         if (!has(b) || (knobs && !wanted(b))) continue;
         const double tiles = (double)tiles_of(b.mtb * 16) * (double)((n_tiles + b.ntb - 1) / b.ntb);
-        for (uint32_t share = 1; share <= max_share; share *= 2) {
-            if (share > 1 && (b.ntb != 8 || k_steps / share < 8)) break;
+        for (uint32_t share = rule.least; share <= rule.most; share *= 2) {
+            if (share > 1 && (b.ntb != 8 || k_steps / share < rule.stages)) break;
             const double blocks = tiles * share, rounds = std::floor(blocks / num_cus), rest = blocks / num_cus - rounds;
-            const double one = b.fixed + b.per_2k * (double)((k_steps + share - 1) / share) / 16.0 + (share > 1 ? kShareCost * share * b.mtb * b.ntb / 64.0 : 0.0);
+            const double one = b.fixed + b.per_2k * (double)((k_steps + share - 1) / share) / 16.0 + (share > 1 ? kShareCost * share * b.mtb * b.ntb / 64.0 + rule.extra : 0.0);
             const double cost = one * (rounds + (rest > 0 ? 0.6 + 0.4 * rest : 0.0)) * (b.mtb < 16 ? low : 1.0);
             if (best.ntb == 0 || cost < best.cost) best = BigTile{b.mtb, b.ntb, share, cost};
         }
     }
     return best;
 }
-BigTile pick_big(uint64_t m, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, uint32_t max_share = 1) {
-    return pick_big_rows([m](int rows) { return (m + rows - 1) / rows; }, n_tiles, k_steps, num_cus, widths, max_share);
+BigTile pick_big(uint64_t m, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, const ShareRule &rule = {}) {
+    return pick_big_rows([m](int rows) { return (m + rows - 1) / rows; }, n_tiles, k_steps, num_cus, widths, rule);
 }
 
 // One of a kernel's forms with its LDS (above the default limit)
@@ -1167,7 +1191,7 @@ struct W8a8Plan {
 static W8a8Plan plan_w8a8(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, bool may_share = true) {
     const uint64_t n_tiles = n_pad / 16;
     if (big_applies(n_tiles, k_pad))
-        return {pick_big(m, n_tiles, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8, may_share && g_gemm_pair != 1 ? 4 : 1), 1};
+        return {pick_big(m, n_tiles, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8, ShareRule{may_share && g_gemm_pair != 1 ? 4u : 1u}), 1};
     const uint64_t fill = (uint64_t)num_cus * (g_gemm_split_fill > 0 ? g_gemm_split_fill : 2);
     const uint64_t blocks = ((n_tiles + NT - 1) / NT) * ((m + BM - 1) / BM);
     if (blocks == 0 || blocks * 2 > fill) return {};
@@ -1177,6 +1201,34 @@ static W8a8Plan plan_w8a8(uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cu
 static uint64_t big_tiles(const BigTile &t, uint64_t m, uint64_t n_pad) { return (m + t.mtb * 16 - 1) / (t.mtb * 16) * ((n_pad / 16 + t.ntb - 1) / t.ntb); }
 static uint64_t share_bytes(const BigTile &t, uint64_t m, uint64_t n_pad) {
     return t.share > 1 ? big_tiles(t, m, n_pad) * t.share * ((uint64_t)t.mtb * t.ntb * 256 * 4) : 0;
+}
+// The tile of a GEMM whose sums are f32, whose blocks may share one where the context's area holds their partial sums (it holds those
+// of 256 blocks of 128 x 128; no more than that share where units would idle) and the tuning keys name no tile (the tiles they name
+// are to give the same bits).  A part of k has twelve stages at the least.  e4m3, us, one block a tile / two / four:
+//   rows -> columns    16 stages of k   24                32                   48                   64                   112
+//   130 -> 2048        8.9 10.0 -       11.4 11.6 -       15.8 13.5 14.1       22.5 16.9 15.8       27.6 19.6 17.4       47.2 29.7 23.1
+//   500 -> 2048        10.1 11.1 -      13.5 13.2 -       16.3 14.8 17.6       23.0 18.4 19.5       28.5 21.3 21.0       48.3 31.6 26.2
+//   1000 -> 2048       10.6 13.2 -      14.2 15.5 -       17.2 16.8 -          23.8 20.4 -          29.7 23.8 -          50.2 35.1 -
+// The bf16 linears of a pass alternate with each other and find their code cold, and both kinds are then in use: another 4 us (a pass
+// through four layers, none shared, with no such cost, with 3 and with 4: grouped-query attention of width 2048, 70 rows 667, 675, 677 and
+// 666, 130 rows 687, 694, 686 and 683; latent and delta layers of width 2048, 130 rows 470, 446, 438 and 446, of 4096, 70 rows 773, 618
+// with none, 300 rows 874, 792, 783 and 788).  The form with the sums for every tile of 128 columns, so that one code serves both: the
+// tiles of one block 1 us slower, the passes that share the same.
+static BigTile pick_big_f32(uint64_t m, uint64_t n_tiles, uint64_t k_steps, int num_cus, int widths, const SplitKArea *sk, double extra) {
+    const bool may = sk && sk->partial && sk->counters && g_gemm_pair != 1 && !g_gemm_ntb && !g_gemm_mtb && g_gemm_waves != 4 && g_gemm_waves != 16;
+    const uint32_t named = may && (g_gemm_pair == 2 || g_gemm_pair == 4) ? g_gemm_pair : 0;
+    for (uint32_t most = named ? named : may ? 4 : 1;; most /= 2) {
+        const BigTile t = pick_big(m, n_tiles, k_steps, num_cus, widths, {most, named == most ? named : 1, named ? 8u : 12u, extra});
+        if (t.ntb == 0) continue;                     // too little k for the share that was named
+        if (t.share == 1 || (big_tiles(t, m, n_tiles * 16) <= sk->n_counters && share_bytes(t, m, n_tiles * 16) <= sk->partial_bytes)) return t;
+    }
+}
+// Tiles of 128 columns, share blocks each: whole groups on every XCD, surplus groups return at once
+template <bool FP8, typename Epi>
+static void launch_shared(const BigTile &t, const uint8_t *aq, const uint8_t *w_tiles, uint64_t m, uint64_t n, uint64_t n_tiles, uint64_t k_steps, const Epi &e, void *partial,
+                          const SplitKArea *sk, hipStream_t s) {
+    const EpiSplit<Epi> es{e, (int32_t *)partial, sk->counters, meets_in_l2(sk), t.share};      // scope: as in the split-k decode linears
+    launch_big<FP8, kWide8>(t, aq, w_tiles, m, n, n_tiles, k_steps, es, s, 8u * t.share * (unsigned)((big_tiles(t, m, n_tiles * 16) + 7) / 8));
 }
 
 // ... with what the context has for blocks that share a tile (they come with eight wavefronts only)
@@ -1190,7 +1242,7 @@ GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num
     GemmPlan out{0, 4, 1, 0, 1};
     W8a8Plan p;
     if (!fp8) p = plan_w8a8(m, n_pad, k_pad, num_cus, sk);
-    else if (big_applies(n_pad / 16, k_pad)) p.tile = pick_big(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8);
+    else if (big_applies(n_pad / 16, k_pad)) p.tile = pick_big_f32(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8, sk, kShareF8);
     out.splits = p.splits;
     if (p.tile.ntb) {
         out.big_ntb = p.tile.ntb;
@@ -1214,14 +1266,8 @@ void gemm_w8a8_mfma(const int8_t *aq, const int8_t *w_tiles, uint64_t m, uint64_
     const EpiI8 e{ep.sx, ep.sw, ep.bias, ep.residual, ep.acc_out, ep.out, ep.out_bf16};
     W8a8Plan p = plan_w8a8(m, n_pad, k_pad, num_cus, sk);
     if (p.tile.share > 1) {
-        const uint64_t tiles = big_tiles(p.tile, m, n_pad);
-        if (workspace && workspace_bytes >= share_bytes(p.tile, m, n_pad)) {
-            // (the scope knob of the split-k decode linears forces either form here as well: 2 agent scope, 3 the XCD's L2)
-            const EpiI8Split es{e, (int32_t *)workspace, sk->counters, meets_in_l2(sk), p.tile.share};
-            const unsigned grid = 8u * p.tile.share * (unsigned)((tiles + 7) / 8);   // whole groups on every XCD; surplus groups return at once
-            launch_big<false, kWide8>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, es, s, grid);
-            return;
-        }
+        if (workspace && workspace_bytes >= share_bytes(p.tile, m, n_pad))
+            return launch_shared<false>(p.tile, (const uint8_t *)aq, (const uint8_t *)w_tiles, m, n, n_pad / 16, k_pad / 128, e, workspace, sk, s);
         p = plan_w8a8(m, n_pad, k_pad, num_cus, false);      // no room: the plan without shared tiles
     }
     if (p.splits > 1 && (!workspace || workspace_bytes < (uint64_t)p.splits * m * n * 4))
@@ -1280,26 +1326,27 @@ void gemm_w8a8_qkv_rope_mfma(const int8_t *aq, const int8_t *w_tiles, const floa
 }
 
 static void launch_e4m3(const uint8_t *aq, const uint8_t *w_tiles, const EpiF8 &e, uint64_t m, uint64_t n, uint64_t n_pad,
-                        uint64_t k_pad, int num_cus, hipStream_t s);
+                        uint64_t k_pad, int num_cus, hipStream_t s, const SplitKArea *sk);
 
 void gemm_e4m3_mfma(const uint8_t *aq, const uint8_t *w_tiles, const float *a_scale, const float *w_scale, uint64_t m,
-                    uint64_t n, uint64_t n_pad, uint64_t k_pad, void *out, int out_bf16, int num_cus, hipStream_t s) {
+                    uint64_t n, uint64_t n_pad, uint64_t k_pad, void *out, int out_bf16, int num_cus, hipStream_t s, const SplitKArea *sk) {
     if (m == 0 || n == 0) return;
-    launch_e4m3(aq, w_tiles, EpiF8{a_scale, w_scale, out, out_bf16, nullptr, nullptr, nullptr}, m, n, n_pad, k_pad, num_cus, s);
+    launch_e4m3(aq, w_tiles, EpiF8{a_scale, w_scale, out, out_bf16, nullptr, nullptr, nullptr}, m, n, n_pad, k_pad, num_cus, s, sk);
 }
 
 void gemm_e4m3_rows_mfma(const uint8_t *aq, const uint8_t *w_tiles, const float *sx, const float *sw, const float *bias,
                          uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad, void *out, int out_bf16, int num_cus,
-                         hipStream_t s) {
+                         hipStream_t s, const SplitKArea *sk) {
     if (m == 0 || n == 0) return;
-    launch_e4m3(aq, w_tiles, EpiF8{nullptr, nullptr, out, out_bf16, sx, sw, bias}, m, n, n_pad, k_pad, num_cus, s);
+    launch_e4m3(aq, w_tiles, EpiF8{nullptr, nullptr, out, out_bf16, sx, sw, bias}, m, n, n_pad, k_pad, num_cus, s, sk);
 }
 
 static void launch_e4m3(const uint8_t *aq, const uint8_t *w_tiles, const EpiF8 &e, uint64_t m, uint64_t n, uint64_t n_pad,
-                        uint64_t k_pad, int num_cus, hipStream_t s) {
+                        uint64_t k_pad, int num_cus, hipStream_t s, const SplitKArea *sk) {
     if (big_applies(n_pad / 16, k_pad)) {
-        const BigTile t = pick_big(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8);
-        if (!launch_big_waves<true>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s)) launch_big<true, kWide16 | kWide14 | kWide8>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
+        const BigTile t = pick_big_f32(m, n_pad / 16, k_pad / 128, num_cus, kWide16 | kWide14 | kWide8, sk, kShareF8);
+        if (t.share > 1) launch_shared<true>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, sk->partial, sk, s);
+        else if (!launch_big_waves<true>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s)) launch_big<true, kWide16 | kWide14 | kWide8>(t, aq, w_tiles, m, n, n_pad / 16, k_pad / 128, e, s);
         return;
     }
     dim3 grid((unsigned)((n_pad / 16 + NT - 1) / NT), (unsigned)((m + BM - 1) / BM));
@@ -1309,10 +1356,12 @@ static void launch_e4m3(const uint8_t *aq, const uint8_t *w_tiles, const EpiF8 &
 
 namespace {
 template <int MODE>
-void launch_big_bf16(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+void launch_big_bf16(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s, const SplitKArea *sk) {
     constexpr int WIDTHS = is_glu(MODE) ? kWide16 | kWide8 : kWide16 | kWide14 | kWide8;
-    launch_big<false, WIDTHS>(pick_big(m, w.n_tiles, w.k_tiles / 2, num_cus, WIDTHS), (const uint8_t *)a, (const uint8_t *)w.w, m, w.n, w.n_tiles,
-                              w.k_tiles / 2, EpiBf16<MODE>{ep}, s);
+    const BigTile t = pick_big_f32(m, w.n_tiles, w.k_tiles / 2, num_cus, WIDTHS, sk, kShareBf16);
+    if (t.share > 1)
+        return launch_shared<false>(t, (const uint8_t *)a, (const uint8_t *)w.w, m, w.n, w.n_tiles, w.k_tiles / 2, EpiBf16<MODE>{ep}, sk->partial, sk, s);
+    launch_big<false, WIDTHS>(t, (const uint8_t *)a, (const uint8_t *)w.w, m, w.n, w.n_tiles, w.k_tiles / 2, EpiBf16<MODE>{ep}, s);
 }
 }  // namespace
 
@@ -1320,14 +1369,14 @@ bool gemm_bf16_big_applies(uint64_t lda, uint64_t m, const LinearWeight &w) {
     return w.batches == 1 && lda == (uint64_t)w.k_tiles * 32 && w.k_tiles % 2 == 0 && m > 64;
 }
 
-void gemm_bf16_big(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s) {
+void gemm_bf16_big(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s, const SplitKArea *sk) {
     switch (ep.mode) {
-        case LinearEpilogue::kResidual: return launch_big_bf16<LinearEpilogue::kResidual>(a, m, w, ep, num_cus, s);
-        case LinearEpilogue::kGlu: return launch_big_bf16<LinearEpilogue::kGlu>(a, m, w, ep, num_cus, s);
-        case LinearEpilogue::kSiluGlu: return launch_big_bf16<LinearEpilogue::kSiluGlu>(a, m, w, ep, num_cus, s);
-        case LinearEpilogue::kXielu: return launch_big_bf16<LinearEpilogue::kXielu>(a, m, w, ep, num_cus, s);
-        case LinearEpilogue::kSoftcap: return launch_big_bf16<LinearEpilogue::kSoftcap>(a, m, w, ep, num_cus, s);
-        default: return launch_big_bf16<LinearEpilogue::kStore>(a, m, w, ep, num_cus, s);
+        case LinearEpilogue::kResidual: return launch_big_bf16<LinearEpilogue::kResidual>(a, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kGlu: return launch_big_bf16<LinearEpilogue::kGlu>(a, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kSiluGlu: return launch_big_bf16<LinearEpilogue::kSiluGlu>(a, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kXielu: return launch_big_bf16<LinearEpilogue::kXielu>(a, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kSoftcap: return launch_big_bf16<LinearEpilogue::kSoftcap>(a, m, w, ep, num_cus, s, sk);
+        default: return launch_big_bf16<LinearEpilogue::kStore>(a, m, w, ep, num_cus, s, sk);
     }
 }
 
@@ -1351,7 +1400,7 @@ void launch_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroup
         for (int d = -3; d <= 3; ++d) sum += std::ceil(mean * (1.0 + 0.05 * d) / r);
         return sum / 7.0 * rg.groups;
     };
-    const BigTile t = pick_big_rows(tiles, w.n_tiles, w.k_tiles / 2, num_cus, kWide16, 1, rg.a_div > 1 ? 1.1 : 1.18);
+    const BigTile t = pick_big_rows(tiles, w.n_tiles, w.k_tiles / 2, num_cus, kWide16, ShareRule{}, rg.a_div > 1 ? 1.1 : 1.18);
     if (t.mtb == 8) rows(std::integral_constant<int, 8>{});
     else if (t.mtb == 12) rows(std::integral_constant<int, 12>{});
     else rows(std::integral_constant<int, 16>{});

@@ -546,7 +546,7 @@ void launch_normed(const NormAhead &nm, uint64_t m, const LinearWeight &w, const
 
 template <int MODE>
 void launch_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
-                 int num_cus, hipStream_t s) {
+                 int num_cus, hipStream_t s, const SplitKArea *sk) {
     const uint8_t *wt = (const uint8_t *)w.w;
     if (m <= 64 && rows_reach(m, lda)) {
         const bool two = two_tiles(is_glu(MODE), w, m, num_cus);
@@ -564,7 +564,7 @@ void launch_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, 
             if (!two) return launch_rows<4, 1, MODE>(a, lda, a_batch, m, w, ep, s);
         return launch_rows<4, 2, MODE>(a, lda, a_batch, m, w, ep, s);
     }
-    if (MODE != LinearEpilogue::kHeadGate && g_linear_form != 2 && gemm_bf16_big_applies(lda, m, w)) return gemm_bf16_big(a, m, w, ep, num_cus, s);
+    if (MODE != LinearEpilogue::kHeadGate && g_linear_form != 2 && gemm_bf16_big_applies(lda, m, w)) return gemm_bf16_big(a, m, w, ep, num_cus, s, sk);
     const dim3 grid((w.n_tiles + 7) / 8, (unsigned)((m + 127) / 128), w.batches);
     linear_tile_kernel<MODE><<<grid, 256, 0, s>>>(a, lda, a_batch, wt, (uint32_t)m, w.n, w.n_tiles, w.k_tiles, ep, RowGroups{});
 }
@@ -613,16 +613,16 @@ void launch_f32(const float *a, uint64_t lda, uint64_t a_batch, uint64_t m, cons
 }  // namespace
 
 void linear_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
-                 int num_cus, hipStream_t s) {
+                 int num_cus, hipStream_t s, const SplitKArea *sk) {
     if (m == 0) return;
     switch (ep.mode) {
-        case LinearEpilogue::kResidual: return launch_bf16<LinearEpilogue::kResidual>(a, lda, a_batch, m, w, ep, num_cus, s);
-        case LinearEpilogue::kGlu: return launch_bf16<LinearEpilogue::kGlu>(a, lda, a_batch, m, w, ep, num_cus, s);
-        case LinearEpilogue::kSiluGlu: return launch_bf16<LinearEpilogue::kSiluGlu>(a, lda, a_batch, m, w, ep, num_cus, s);
-        case LinearEpilogue::kSoftcap: return launch_bf16<LinearEpilogue::kSoftcap>(a, lda, a_batch, m, w, ep, num_cus, s);
-        case LinearEpilogue::kHeadGate: return launch_bf16<LinearEpilogue::kHeadGate>(a, lda, a_batch, m, w, ep, num_cus, s);
-        case LinearEpilogue::kXielu: return launch_bf16<LinearEpilogue::kXielu>(a, lda, a_batch, m, w, ep, num_cus, s);
-        default: return launch_bf16<LinearEpilogue::kStore>(a, lda, a_batch, m, w, ep, num_cus, s);
+        case LinearEpilogue::kResidual: return launch_bf16<LinearEpilogue::kResidual>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kGlu: return launch_bf16<LinearEpilogue::kGlu>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kSiluGlu: return launch_bf16<LinearEpilogue::kSiluGlu>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kSoftcap: return launch_bf16<LinearEpilogue::kSoftcap>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kHeadGate: return launch_bf16<LinearEpilogue::kHeadGate>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
+        case LinearEpilogue::kXielu: return launch_bf16<LinearEpilogue::kXielu>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
+        default: return launch_bf16<LinearEpilogue::kStore>(a, lda, a_batch, m, w, ep, num_cus, s, sk);
     }
 }
 

@@ -264,15 +264,16 @@ struct GemmPlan {
     uint32_t share;
 };
 GemmPlan gemm_plan(bool fp8, uint64_t m, uint64_t n_pad, uint64_t k_pad, int num_cus, const SplitKArea *sk);
-// aq: e4m3 [m, k_pad] row-major; scales are device scalars.
+// aq: e4m3 [m, k_pad] row-major; scales are device scalars.  sk (optional): blocks may share a tile as above; they meet in sk's own
+// area and their f32 sums are added in a fixed order (not on a tile that the tuning keys name: those are all the same bits).
 void gemm_e4m3_mfma(const uint8_t *aq, const uint8_t *w_tiles, const float *a_scale,
                     const float *w_scale, uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad,
-                    void *out, int out_bf16, int num_cus, hipStream_t s);
+                    void *out, int out_bf16, int num_cus, hipStream_t s, const SplitKArea *sk = nullptr);
 // The same with one scale per row of aq (sx[m]) and one per output column (sw[n_pad]):
 // out = acc * (sx[row] * sw[col]) (+ bias[col]).
 void gemm_e4m3_rows_mfma(const uint8_t *aq, const uint8_t *w_tiles, const float *sx, const float *sw, const float *bias,
                          uint64_t m, uint64_t n, uint64_t n_pad, uint64_t k_pad, void *out, int out_bf16, int num_cus,
-                         hipStream_t s);
+                         hipStream_t s, const SplitKArea *sk = nullptr);
 // Decode shape (m <= 64) of the same operator: a weight-streaming kernel, one block per 16-column tile, k split
 // over the block's wavefronts.
 void linear_e4m3_skinny(const uint8_t *aq, const uint8_t *w_tiles, const float *sx, const float *sw, const float *bias,
@@ -370,9 +371,10 @@ struct LinearEpilogue {
     uint32_t ld_gate = 0;
 };
 // a [m, lda] (batch entry i starts i * a_batch elements further on) with 32 * k_tiles readable, finite elements per row;
-// what lies past the weight's own k meets zero weights.
+// what lies past the weight's own k meets zero weights.  sk (optional): more than 64 rows that leave units idle may have k divided
+// over blocks that meet there.
 void linear_bf16(const uint16_t *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
-                 int num_cus, hipStream_t s);
+                 int num_cus, hipStream_t s, const SplitKArea *sk = nullptr);
 void linear_f32(const float *a, uint64_t lda, uint64_t a_batch, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep,
                 hipStream_t s);
 // The same on rows ahead of their norm, a = (x - mean) / sqrt(mean((x - mean)^2) + eps) * w (rms: without the mean), x [m, hidden] f32,
@@ -404,7 +406,7 @@ void linear_grouped_f32(const float *a, uint64_t lda, const LinearWeight &w, con
 void gemm_bf16_big_grouped(const uint16_t *a, const LinearWeight &w, const RowGroups &rg, const LinearEpilogue &ep, int num_cus, hipStream_t s);
 // The large-tile form (kern_gemm_mfma.hip): m > 64, one batch entry, lda == 32 * k_tiles.
 bool gemm_bf16_big_applies(uint64_t lda, uint64_t m, const LinearWeight &w);
-void gemm_bf16_big(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s);
+void gemm_bf16_big(const uint16_t *a, uint64_t m, const LinearWeight &w, const LinearEpilogue &ep, int num_cus, hipStream_t s, const SplitKArea *sk);
 // Packs `rows` source rows of `cols` values (bf16 bits or f32; element (r, c) at src[r * row_stride + c * col_stride]) into
 // columns dst_row(r) of a weight: dst_row(r) = n0 + (r / group) * pitch + r % group, from its input k0 on.
 void pack_linear(const void *src, int src_f32, uint64_t row_stride, uint64_t col_stride, uint32_t rows, uint32_t cols, void *dst,

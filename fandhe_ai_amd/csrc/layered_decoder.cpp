@@ -263,7 +263,7 @@ fa_status arena_reserve(fa_context *ctx, LayeredState &L, Arena &a, uint32_t row
 void linear(fa_context *ctx, const LayeredState &L, const void *a, uint64_t lda, uint64_t a_batch, uint64_t m, const k::LinearWeight &w,
             k::LinearEpilogue ep) {
     if (L.is_f32) k::linear_f32((const float *)a, lda, a_batch, m, w, ep, ctx->stream);
-    else k::linear_bf16((const uint16_t *)a, lda, a_batch, m, w, ep, ctx->props.multiProcessorCount, ctx->stream);
+    else k::linear_bf16((const uint16_t *)a, lda, a_batch, m, w, ep, ctx->props.multiProcessorCount, ctx->stream, &ctx->splitk);
 }
 
 // A norm of the residual that the next linear, with an epilogue of `mode`, may take into its own launch, or that goes out now, into a.hn

@@ -432,6 +432,49 @@ def test_narrow_weights_on_large_tiles(m, k, n, kind):
     assert np.all(np.abs(got[rows] - a64 @ w64 * scale) <= bound)
 
 
+@pytest.mark.parametrize("m,k,n", [(65, 4096, 16), (193, 4224, 100), (300, 4352, 520), (700, 4096, 1000), (129, 8192, 2047)])
+@pytest.mark.parametrize("share,scope", [(2, 0), (4, 0), (4, 2), (0, 0)])
+def test_e4m3_tiles_shared_by_blocks(m, k, n, share, scope, tune):
+    """k over two and four blocks that meet in the XCD's L2 or in memory: parts of different length, tiles that the last row and
+    column cut, fewer tiles than XCDs.  Every sum within k roundings of the exact one, the same bits from call to call."""
+    import fandhe_ai_amd as fa
+    import oracle_lib as o
+    import test_gpu_quantized as tq
+    be = ops()
+    rng = np.random.default_rng(m + n)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    aq, sa = be.quantize_tensor_e4m3(be.upload(x))
+    qw = be.quantize_weight(fa.DeviceBufferView(be.upload(w), 0, (k, n)), fa.capi.QW_E4M3_TENSOR)
+    tune(24, share)
+    tune(16, scope)
+    assert share == 0 or tq._gemm_plan(fa, be, m, qw).share == share
+    got = [be.download_owned(be.gemm_e4m3(aq, sa, qw, fa.capi.F32)) for _ in range(4)]
+    assert all(np.array_equal(got[0], g) for g in got[1:])
+    codes, sw = qw.export()
+    a64, w64 = o.from_e4m3(be.download(aq)).astype(np.float64), o.from_e4m3(codes).astype(np.float64)
+    scale = float(be.download(sa)[0]) * float(sw[0])
+    assert np.all(np.abs(got[0] - a64 @ w64 * scale) <= (np.abs(a64) @ np.abs(w64)) * scale * (k + 2) * 2.0 ** -24)
+
+
+@pytest.mark.parametrize("rows", [65, 130, 300])
+def test_bf16_tiles_shared_by_blocks(rows, tune):
+    """The epilogues of the unquantized linears behind sums that two and four blocks share, by key and by the plan's own choice."""
+    cfg = lc.config([lc.delta(heads=4, kv_heads=2, dim=128, vdim=128, mlp=lc.glu(ff=2112)),
+                     lc.latent(heads=4, dim=128, rot=64, vdim=128, q_rank=64, kv_rank=512)], width=2112, vocab=300)
+    w, toks = lc.weights(cfg, 5), lc.tokens(cfg, rows, 41)
+    dec = lc.make_decoder(ops(), cfg, w, "bfloat16", max_tokens=512, max_batch=1)
+    table = np.full((1, dec.cfg.max_blocks_per_seq), 0xFFFFFFFF, dtype=np.uint32)
+    table[0, :-(-rows // 16)] = np.arange(-(-rows // 16))
+    want = oracle.forward(cfg, w, toks)
+    err = {}
+    for share in (1, 2, 4, 0):
+        tune(24, share)
+        dec.set_sequences(table, [0])
+        err[share] = lc.error(dec.forward([toks], [list(range(rows))]), want)
+    dec.close()
+    assert max(err.values()) < 0.06 and max(abs(err[s] - err[1]) for s in err) < 0.01, err
+
+
 @pytest.mark.parametrize("scale", [-0.25, 0.0, 0.0883883476, 3.0])
 @pytest.mark.parametrize("split,cols", [(1, 2), (1, 1), (2, 2)])
 @pytest.mark.parametrize("l_new,lens", [(70, [70, 101, 400]), (33, [33, 64, 65])])
